@@ -393,6 +393,20 @@ int vla_seq_delta_rule_scan(void* out, int64_t out_stride, int out_dtype, const 
                             const int* context_lens, const int* state_slots, int num_tokens,
                             int num_seqs, int max_query_len, int num_slots, int heads, int kv_heads,
                             int dim, int vdim, float eps, float* scratch, void* stream);
+/* The same with scratch for runs that go in blocks of 32 rows (longer runs of heads up to 256 x vdim):
+ * scratch_floats values, 16-byte aligned, at least what vla_seq_delta_rule_block_scratch_floats says for
+ * the same numbers and kernel choice.  max_query_len 0 (unknown) never takes blocks. */
+int64_t vla_seq_delta_rule_block_scratch_floats(int num_tokens, int num_seqs, int max_query_len, int heads,
+                                                int dim, int vdim);
+int vla_seq_delta_rule_scan_blocks(void* out, int64_t out_stride, int out_dtype, const void* q,
+                                   int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                                   int64_t v_stride, const void* gate, int64_t gate_stride,
+                                   const void* beta, int64_t beta_stride, const void* dt, int64_t dt_stride,
+                                   int in_dtype, const float* a_log, const float* dt_bias,
+                                   const float* norm_weight, float* state, const int* query_start_loc,
+                                   const int* context_lens, const int* state_slots, int num_tokens,
+                                   int num_seqs, int max_query_len, int num_slots, int heads, int kv_heads,
+                                   int dim, int vdim, float eps, float* scratch, int64_t scratch_floats, void* stream);
 
 /* The delta rule with a decay per key channel: per head, on a state S fp32 [dim, vdim] (stored
  * [num_slots, heads, vdim, dim]):

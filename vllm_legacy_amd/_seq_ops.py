@@ -753,16 +753,17 @@ def delta_rule_scan(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torc
         assert t.dtype == torch.int32 and t.is_contiguous()
     assert query_start_loc.numel() == B + 1 and state_slots.numel() == B
     T = q.shape[0]
-    scratch = torch.empty(_lib.seq_lib().vla_seq_delta_rule_scratch_floats(T, H, V), dtype=torch.float32, device=q.device)
+    L = _lib.seq_lib()
+    need = L.vla_seq_delta_rule_block_scratch_floats(T, B, int(max_query_len), H, D, V)
+    scratch = torch.empty(need, dtype=torch.float32, device=q.device)
     with torch.cuda.device(q.device):
-        seq_check(_lib.seq_lib().vla_seq_delta_rule_scan(
+        seq_check(L.vla_seq_delta_rule_scan_blocks(
             out.data_ptr(), _rows(out, H * V), _dt(out.dtype), q.data_ptr(), _rows(q, kv_heads * D), k.data_ptr(),
             _rows(k, kv_heads * D), v.data_ptr(), _rows(v, H * V), gate.data_ptr(), _rows(gate, H * V),
             beta.data_ptr(), _rows(beta, H), dt.data_ptr(), _rows(dt, H), _lib.F32, a_log.data_ptr(),
             dt_bias.data_ptr(), norm_weight.data_ptr(), state.data_ptr(), query_start_loc.data_ptr(),
             context_lens.data_ptr(), state_slots.data_ptr(), T, B, int(max_query_len), slots, H, int(kv_heads), D, V,
-            float(eps),
-            scratch.data_ptr(), _stream(q.device)), "delta_rule_scan")
+            float(eps), scratch.data_ptr(), need, _stream(q.device)), "delta_rule_scan")
 
 
 def set_delta_kernel(mode: int) -> None:

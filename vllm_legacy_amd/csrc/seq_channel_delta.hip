@@ -43,10 +43,6 @@ constexpr int kMaxSplit = 16;
 constexpr int kTri = 20;            // floats per row of a 16 x 16 matrix in LDS
 std::atomic<int> g_channel_delta_kernel{0};
 
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 struct ChannelDelta {
   float* o;                   // [T][heads * vdim]
   const void* q;
@@ -69,27 +65,6 @@ struct ChannelDelta {
   int num_seqs, heads, kv_heads, dim, vdim, mode;
   bool vec_qk, vec_z, vec_state;
 };
-
-// four values d .. d + 3 of a row of `dim`, zeros behind its end
-template <class S>
-__device__ __forceinline__ f32x4 load4(const typename S::T* row, int d, int dim, bool vec) {
-  f32x4 r = {0.f, 0.f, 0.f, 0.f};
-  if (vec) {
-    if (d < dim) {
-      if constexpr (sizeof(typename S::T) == 2) {
-        const u32x2 x = *reinterpret_cast<const u32x2*>(row + d);
-        r = f32x4{lo16<S>(x[0]), hi16<S>(x[0]), lo16<S>(x[1]), hi16<S>(x[1])};
-      } else {
-        r = *reinterpret_cast<const f32x4*>(row + d);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (d + e < dim) r[e] = S::to_f32(row[d + e]);
-  }
-  return r;
-}
 
 __device__ __forceinline__ float channel_decay(float rate, float z) { return expf(-rate * softplusf(z)); }
 

@@ -93,6 +93,33 @@ __device__ __forceinline__ void group_sums(float& a, float& b, int split) {
   }
 }
 
+// one 16x16x4 fp32 matrix-core step.  lane = (g, c) = (lane >> 4, lane & 15): A operand row c,
+// contraction index g; B operand column c, contraction index g; result column c, rows 4 g .. 4 g + 3
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// four values d .. d + 3 of a row of `dim`, zeros behind its end
+template <class S>
+__device__ __forceinline__ f32x4 load4(const typename S::T* row, int d, int dim, bool vec) {
+  f32x4 r = {0.f, 0.f, 0.f, 0.f};
+  if (vec) {
+    if (d < dim) {
+      if constexpr (sizeof(typename S::T) == 2) {
+        const u32x2 x = *reinterpret_cast<const u32x2*>(row + d);
+        r = f32x4{lo16<S>(x[0]), hi16<S>(x[0]), lo16<S>(x[1]), hi16<S>(x[1])};
+      } else {
+        r = *reinterpret_cast<const f32x4*>(row + d);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (d + e < dim) r[e] = S::to_f32(row[d + e]);
+  }
+  return r;
+}
+
 __device__ __forceinline__ float softplusf(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 
 }  // namespace seq

@@ -226,10 +226,6 @@ __device__ __forceinline__ void land_piece(float* dst, const Piece<W16>& p, int 
   *reinterpret_cast<f32x4*>(dst + 4) = hi;
 }
 
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 // Which sequence and piece a piece slot is: sequence b's pieces are slots start_b / R + b + 0, 1, ...
 // (enough for ceil(n / R) of them; slots behind a sequence's last piece stay empty).
 __device__ __forceinline__ bool find_piece(const DecayScan& a, int z, int& b, int& piece) {

@@ -19,6 +19,19 @@
 // key themselves and the unit norms are lane sums.  The walk leaves o in fp32; a
 // second launch norms each head's o over vdim, weighs and gates it.  The state is stored
 // [slot, head, vdim, dim], so a thread's rows are contiguous.  Everything is fp32.
+//
+// Longer runs (heads of at most 256 rows) go in blocks of 32 rows.  With L_ij the product of g over
+// rows j + 1 .. i of a block (formed as that product: decays that underflow beside decays of 1 are
+// exact) and G_i the one over rows 0 .. i:
+//   B_ij = beta_i (k_i . k_j) L_ij  (j < i),   A_ij = (q_i . k_j) L_ij  (j <= i)
+//   T = (I + B)^-1 diag(beta)                                            (32 x 32, lower triangular)
+//   U = T V - W S,   O = A U + Q~ S      W = T (G k),   Q~ = G q
+//   S <- G_31 S + K^^T U                 K^_j = L_31,j k_j
+// Everything but the last two lines' products with S and U depends on the block alone:
+// delta_block_prepare_kernel forms it for all blocks at once, one workgroup per block and head, and
+// leaves W, Q~, K^, G_31, A and T V in scratch; delta_block_walk_kernel goes over a run's blocks in
+// order, a workgroup per 16 columns of S, whose rows its four waves share and keep in registers.  All
+// products run on 16x16x4 fp32 matrix cores.
 #include <algorithm>
 #include <atomic>
 
@@ -255,7 +268,7 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(
     const float* __restrict__ dt_bias, float* __restrict__ state,
     const int* __restrict__ query_start_loc, const int* __restrict__ context_lens,
     const int* __restrict__ state_slots, int heads, int kv_heads, int dim, int vdim, int split,
-    int cols) {
+    int cols, int longest) {
   const int h = blockIdx.y, b = blockIdx.z, j0 = blockIdx.x * cols;
   const int g_head = h / (heads / kv_heads);
   const int tid = threadIdx.x;
@@ -263,6 +276,7 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(
   const int j = j0 + jl;
   const bool col = jl < cols && j < vdim;
   const int start = query_start_loc[b], end = query_start_loc[b + 1];
+  if (longest > 0 && end - start > longest) return;        // the block kernels'
   float* st = state + (((int64_t)state_slots[b] * heads + h) * vdim + (col ? j : 0)) * dim;
   const bool whole = dim == split * R && (dim & 3) == 0;
   const bool vec = whole && (in.q_stride & 3) == 0 && (in.k_stride & 3) == 0 &&
@@ -350,6 +364,550 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Blocks of 32 rows
+constexpr int kRows = 32;
+constexpr int kStepRows = 4;        // runs of at most this many rows go token by token beside blocks
+constexpr int kMaxBlockDim = 256;
+constexpr int kMat = 36;            // floats per row of a 32 x 32 matrix in LDS
+
+struct DeltaBlocks {
+  float* o;                         // [T][heads * vdim]
+  DeltaRows<F32> in;
+  const float* a_log;
+  const float* dt_bias;
+  float* state;
+  float* scratch;
+  const int* query_start_loc;
+  const int* context_lens;
+  const int* state_slots;
+  int num_seqs, heads, kv_heads, dim, vdim;
+  bool vec_qk, vec_state;
+};
+
+// A block's operands lie in scratch as the walk's waves take them, lane for lane: [16 x 16 tile][lane][4].
+// (Lanes side by side in memory matter: with lanes 64 bytes apart the walk below took 192 us.)
+// Floats of a block's scratch: W | Q~ | K^ (each 32 x DP) | G_31 and a place for stores nobody wants
+// (padded to 4) | A (its three lower 16 x 16 tiles) | T V (32 x VP)
+__host__ __device__ __forceinline__ int64_t delta_block_floats(int dp, int vp) {
+  return (int64_t)3 * kRows * dp + 4 + 3 * 256 + kRows * vp;
+}
+
+// Which sequence and block a block slot is: sequence b's blocks are slots start_b / 32 + b + 0, 1, ...
+__device__ __forceinline__ bool find_delta_block(const DeltaBlocks& a, int slot, int& b, int& block) {
+  int lo = 0, hi = a.num_seqs - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (a.query_start_loc[mid] / kRows + mid <= slot)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  b = lo;
+  block = slot - (a.query_start_loc[b] / kRows + b);
+  return block >= 0 && block * kRows < a.query_start_loc[b + 1] - a.query_start_loc[b];
+}
+
+// LDS of the prepare kernel: unit keys and queries, then the waves' partial products, whose place the
+// 32 x 32 matrices take, then L (column 32: G), decays and betas
+__host__ __device__ constexpr size_t delta_prepare_lds_floats(int dp) {
+  return (size_t)2 * kRows * (dp + 4) + 4 * 6 * 256 + kRows * kMat + 2 * kRows;
+}
+
+template <int DX>
+__global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kernel(DeltaBlocks a) {
+  constexpr int DP = 64 * DX, RS = DP + 4;
+  extern __shared__ __align__(16) float lds[];
+  float* k_lds = lds;                                      // [32][RS]
+  float* q_lds = k_lds + kRows * RS;                       // [32][RS]
+  float* part = q_lds + kRows * RS;                        // [4 waves][6 tiles][64 lanes][4]
+  float* b_mat = part;                                     // B, strictly lower
+  float* t_mat = b_mat + kRows * kMat;                     // (I + B)^-1
+  float* p_mat = t_mat + kRows * kMat;                     // 16 x 16 between two products, rows of 20
+  float* l_mat = part + 4 * 6 * 256;                       // [32][kMat]
+  float* g_lds = l_mat + kRows * kMat;                     // [32]
+  float* beta_lds = g_lds + kRows;                         // [32]
+  const int slot = blockIdx.x, h = blockIdx.y;
+  int b, block;
+  if (!find_delta_block(a, slot, b, block)) return;
+  const int run = a.query_start_loc[b + 1] - a.query_start_loc[b];
+  if (run <= kStepRows) return;                            // the step kernel's
+  const int t0 = a.query_start_loc[b] + block * kRows, n = min(kRows, run - block * kRows);
+  const int D = a.dim, V = a.vdim, hg = h / (a.heads / a.kv_heads);
+  const int vb = (V + 15) / 16;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
+  float* out = a.scratch + ((int64_t)slot * a.heads + h) * delta_block_floats(DP, 16 * vb);
+  float* w_out = out;                                      // [DP / 16][2][lane][4]: row c, head row 4 g + e
+  float* q_out = w_out + kRows * DP;                       // the same
+  float* k_out = q_out + kRows * DP;                       // [DP / 16][2][lane][4]: head row c, row 4 g + e
+  float* g_out = k_out + kRows * DP;
+  float* a_out = g_out + 4;                                // [3 tiles][wave][lane]
+  float* u_out = a_out + 3 * 256;                          // [vb][2][lane][4]: column c, row 4 g + e
+  const int row = tid >> 3, eighth = tid & 7;              // 8 neighbouring lanes share a row
+
+  // a wave's columns of v, rows 4 g .. and 16 + 4 g ..: the first two tiles are asked for at the start
+  auto fetch_v = [&](float (&to)[2][4], int vt) {
+    const int col = 16 * vt + c;
+    const float* vr = a.in.v + (int64_t)h * V + min(col, V - 1);
+#pragma unroll
+    for (int it = 0; it < 2; ++it)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = 16 * it + 4 * g + e;
+        const float got = vr[(int64_t)(t0 + min(j, n - 1)) * a.in.v_stride];
+        to[it][e] = j < n && col < V ? got : 0.f;
+      }
+  };
+
+  // unit rows (zeros behind the run's end), decays and betas: every load ahead of everything else, and
+  // none behind a branch of its own
+  f32x4 qv[2 * DX], kv[2 * DX];
+  float v_a[2][4], v_b[2][4];
+  {
+    const bool live = row < n;
+    const int64_t t = t0 + (live ? row : 0);
+    const float* qr = a.in.q + t * a.in.q_stride + (int64_t)hg * D;
+    const float* kr = a.in.k + t * a.in.k_stride + (int64_t)hg * D;
+    const int64_t tr = t0 + min(tid & 31, n - 1);
+    const float z = a.in.dt[tr * a.in.dt_stride + h] + a.dt_bias[h], bt = a.in.beta[tr * a.in.beta_stride + h];
+    const float al = a.a_log[h];
+    if (a.vec_qk) {
+#pragma unroll
+      for (int x = 0; x < 2 * DX; ++x) {
+        const int d = min(4 * eighth + 32 * x, D - 4);
+        qv[x] = *reinterpret_cast<const f32x4*>(qr + d);
+        kv[x] = *reinterpret_cast<const f32x4*>(kr + d);
+      }
+    } else {
+#pragma unroll
+      for (int x = 0; x < 2 * DX; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int d = min(4 * eighth + 32 * x + e, D - 1);
+          qv[x][e] = qr[d];
+          kv[x][e] = kr[d];
+        }
+    }
+    fetch_v(v_a, min(w, vb - 1));
+    fetch_v(v_b, min(w + 4, vb - 1));
+    if (tid < kRows) {
+      g_lds[tid] = tid < n ? expf(-expf(al) * softplusf(z)) : 1.f;
+      beta_lds[tid] = tid < n ? 1.f / (1.f + expf(-bt)) : 0.f;
+    }
+    float qq = 0.f, kk = 0.f;
+#pragma unroll
+    for (int x = 0; x < 2 * DX; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (4 * eighth + 32 * x + e >= D) qv[x][e] = kv[x][e] = 0.f;
+        qq += qv[x][e] * qv[x][e];
+        kk += kv[x][e] * kv[x][e];
+      }
+    group_sums(qq, kk, 8);
+    const float qs = live ? 1.f / (sqrtf(qq + 1e-6f) * sqrtf((float)D)) : 0.f;
+    const float ks = live ? 1.f / sqrtf(kk + 1e-6f) : 0.f;
+#pragma unroll
+    for (int x = 0; x < 2 * DX; ++x) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        qv[x][e] *= qs;
+        kv[x][e] *= ks;
+      }
+      *reinterpret_cast<f32x4*>(q_lds + row * RS + 4 * eighth + 32 * x) = qv[x];
+      *reinterpret_cast<f32x4*>(k_lds + row * RS + 4 * eighth + 32 * x) = kv[x];
+    }
+  }
+  __syncthreads();
+
+  // k_i . k_j and q_i . k_j, lower 16 x 16 tiles; every wave takes a quarter of the head's rows (a lane
+  // holds four neighbouring ones: the contraction index may be relabelled as long as both operands are)
+  {
+    // L: lane j of wave 0 walks down column j (lane 32: from the block's start)
+    if (w == 0) {
+      f32x4 gv[kRows / 4];
+#pragma unroll
+      for (int i = 0; i < kRows / 4; ++i) gv[i] = *reinterpret_cast<const f32x4*>(g_lds + 4 * i);
+      const int j = lane < kRows ? lane : -1;
+      float r = 1.f;
+      if (lane <= kRows) {
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+          r *= i > j ? gv[i >> 2][i & 3] : 1.f;
+          l_mat[i * kMat + lane] = r;
+        }
+      }
+    }
+    f32x4 acc[6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < DX; ++x) {
+      const int d = 16 * (w * DX + x) + 4 * g;
+      const f32x4 k0 = *reinterpret_cast<const f32x4*>(k_lds + c * RS + d);
+      const f32x4 k1 = *reinterpret_cast<const f32x4*>(k_lds + (16 + c) * RS + d);
+      const f32x4 q0 = *reinterpret_cast<const f32x4*>(q_lds + c * RS + d);
+      const f32x4 q1 = *reinterpret_cast<const f32x4*>(q_lds + (16 + c) * RS + d);
+      qv[x] = q0;                                          // again: for Q~, which needs G
+      qv[DX + x] = q1;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        acc[0] = mfma4(k0[e], k0[e], acc[0]);
+        acc[1] = mfma4(k1[e], k0[e], acc[1]);
+        acc[2] = mfma4(k1[e], k1[e], acc[2]);
+        acc[3] = mfma4(q0[e], k0[e], acc[3]);
+        acc[4] = mfma4(q1[e], k0[e], acc[4]);
+        acc[5] = mfma4(q1[e], k1[e], acc[5]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 6; ++i) *reinterpret_cast<f32x4*>(part + ((w * 6 + i) * 64 + lane) * 4) = acc[i];
+  }
+  __syncthreads();
+  f32x4 sum[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int at = min(tid + 256 * u, 6 * 64 - 1);
+    sum[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ow = 0; ow < 4; ++ow) {
+      const f32x4 got = *reinterpret_cast<const f32x4*>(part + (ow * 6 * 64 + at) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[u][e] += got[e];
+    }
+  }
+  // Q~, from the operands of the products above
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const float gq = l_mat[(16 * it + c) * kMat + kRows];
+#pragma unroll
+    for (int x = 0; x < DX; ++x) {
+      const f32x4 q4 = qv[it * DX + x];
+      *reinterpret_cast<f32x4*>(q_out + (((w * DX + x) * 2 + it) * 64 + lane) * 4) =
+          f32x4{gq * q4[0], gq * q4[1], gq * q4[2], gq * q4[3]};
+    }
+  }
+  __syncthreads();                                         // the matrices take the partial products' place
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int at = tid + 256 * u, tile = at >> 6, kind = tile % 3;
+    if (at < 6 * 64) {
+      const int i0 = kind > 0 ? 16 : 0, j0 = kind > 1 ? 16 : 0, j = j0 + c;
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = sum[u][e] * l_mat[(i0 + 4 * g + e) * kMat + j];
+      if (tile < 3) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = i0 + 4 * g + e;
+          b_mat[i * kMat + j] = i > j ? beta_lds[i] * v[e] : 0.f;
+        }
+      } else {
+        // A as the walk's waves take it: wave c & 3 meets contraction index 4 (c >> 2) + (c & 3)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = i0 + 4 * g + e >= j ? v[e] : 0.f;
+        *reinterpret_cast<f32x4*>(a_out + (kind * 4 + (c & 3)) * 64 + ((c >> 2) << 4) + 4 * g) = f32x4{v[0], v[1], v[2], v[3]};
+      }
+    }
+  }
+  __syncthreads();
+
+  // waves 0 and 1 invert the diagonal blocks of I + B, waves 2 and 3 leave K^.  Lane (g, c) holds rows
+  // 4 g .. 4 g + 3 of column c: four rows become final at a time, within a lane, and go to the rows
+  // below through lane exchanges
+  if (w < 2) {
+    const int at = 16 * w;
+    f32x4 bv[4][4];                                        // [e][chunk]: B's row 4 g + e
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int ch = 0; ch < 4; ++ch)
+        bv[e][ch] = *reinterpret_cast<const f32x4*>(b_mat + (at + 4 * g + e) * kMat + at + 4 * ch);
+    float x[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = 4 * g + e == c ? 1.f : 0.f;
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) {
+      // rows 4 ch .. 4 ch + 3, right in the lanes g == ch (the others' results are not used)
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        y[e] = x[e];
+#pragma unroll
+        for (int f = 0; f < e; ++f) y[e] -= bv[e][ch][f] * y[f];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] = g == ch ? y[e] : x[e];
+        y[e] = __shfl(y[e], 16 * ch + c, 64);
+      }
+      // the chunk's own block is skipped, the ones above are zeros of B
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) x[e] -= (g > ch ? bv[e][ch][f] : 0.f) * y[f];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t_mat[(at + 4 * g + e) * kMat + at + c] = x[e];
+  } else {
+    if (tid == 128) g_out[0] = l_mat[(kRows - 1) * kMat + kRows];
+    for (int i = tid - 128; i < DP * (kRows / 4); i += 128) {
+      const int d = 16 * (i >> 7) + (i & 15), j = 4 * ((i >> 4) & 7);    // i: tile, half, lane
+      const f32x4 lv = *reinterpret_cast<const f32x4*>(l_mat + (kRows - 1) * kMat + j);
+      f32x4 kh;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) kh[e] = k_lds[(j + e) * RS + d] * lv[e];
+      *reinterpret_cast<f32x4*>(k_out + 4 * i) = kh;
+    }
+  }
+  __syncthreads();
+  // the block below them: -T22 (B21 T11), every wave for itself
+  f32x4 t21;
+  {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    const f32x4 b21 = *reinterpret_cast<const f32x4*>(b_mat + (16 + c) * kMat + 4 * g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = mfma4(b21[e], t_mat[(4 * g + e) * kMat + c], acc);
+    // acc is the next product's B operand where it lies: column c, contraction index 4 g + e
+    const f32x4 t22 = *reinterpret_cast<const f32x4*>(t_mat + (16 + c) * kMat + 16 + 4 * g);
+    f32x4 neg = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) neg = mfma4(t22[e], acc[e], neg);
+    // from column c, rows 4 g + e to row c, columns 4 g + e
+    float* mine = p_mat + w * 16 * 20;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mine[(4 * g + e) * 20 + c] = -neg[e];
+    wave_sync();
+    t21 = *reinterpret_cast<const f32x4*>(mine + c * 20 + 4 * g);
+  }
+
+  // rows of T diag(beta) as operands: 0: rows 0 .. 15; 1 and 2: rows 16 .. 31 with the first and the
+  // second half of the contraction
+  f32x4 tv[3], gj[2];
+  tv[0] = *reinterpret_cast<const f32x4*>(t_mat + c * kMat + 4 * g);
+  tv[1] = t21;
+  tv[2] = *reinterpret_cast<const f32x4*>(t_mat + (16 + c) * kMat + 16 + 4 * g);
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    const f32x4 be = *reinterpret_cast<const f32x4*>(beta_lds + (p > 1 ? 16 : 0) + 4 * g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tv[p][e] *= be[e];
+  }
+#pragma unroll
+  for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) gj[jt][e] = l_mat[(16 * jt + 4 * g + e) * kMat + kRows];
+#pragma unroll
+  for (int x = 0; x < DX; ++x) {
+    const int tile = w + 4 * x;
+    f32x4 xt[2];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) xt[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // transposed, so that a lane ends with four neighbouring rows of the head of one token
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float ka = k_lds[(4 * g + e) * RS + 16 * tile + c] * gj[0][e];
+      const float kb = k_lds[(16 + 4 * g + e) * RS + 16 * tile + c] * gj[1][e];
+      xt[0] = mfma4(ka, tv[0][e], xt[0]);
+      xt[1] = mfma4(ka, tv[1][e], xt[1]);
+      xt[1] = mfma4(kb, tv[2][e], xt[1]);
+    }
+#pragma unroll
+    for (int it = 0; it < 2; ++it)
+      *reinterpret_cast<f32x4*>(w_out + ((tile * 2 + it) * 64 + lane) * 4) = xt[it];
+  }
+  for (int vt = w; vt < vb; vt += 4) {
+    f32x4 xt[2];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) xt[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      xt[0] = mfma4(tv[0][e], v_a[0][e], xt[0]);
+      xt[1] = mfma4(tv[1][e], v_a[0][e], xt[1]);
+      xt[1] = mfma4(tv[2][e], v_a[1][e], xt[1]);
+    }
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      *reinterpret_cast<f32x4*>(u_out + ((vt * 2 + it) * 64 + lane) * 4) = xt[it];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v_a[it][e] = v_b[it][e];
+    }
+    if (vt + 8 < vb) fetch_v(v_b, vt + 8);
+  }
+}
+
+// What bounds it: a wave has 51 matrix-core instructions of 32 cycles per block (0.67 us) in a chain
+// product -> LDS -> barrier -> LDS -> product, one wave per SIMD and nobody to fill its waits: the
+// loads are a block ahead, the product for the outputs stands where the exchange of U is on its way.
+// Two prompts of 2999 and 1854 tokens, 16 heads of 128 x 128 (94 blocks in a row): 171 us, 1.8 us per
+// block, 118 of them without the loads; asking for blocks two ahead changes nothing.  With the prepare
+// kernel (100 us) and the norms (20 us) 275 us, where the token-by-token walk of the same prompts
+// takes 1051 us and its norms 36.
+template <int DX>
+__global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(DeltaBlocks a) {
+  constexpr int DP = 64 * DX;
+  __shared__ __align__(16) float u_part[2][4][2][64][4];   // a wave's part of W S
+  __shared__ __align__(16) float o_part[2][4][2][4][64];   // of the outputs, by component
+  // heads run fastest: the workgroups of a head's columns, which read the same scratch, share an XCD
+  // (and its L2) whenever the number of heads is a multiple of 8
+  const int h = blockIdx.x, v0 = 16 * blockIdx.y, b = blockIdx.z;
+  const int t_begin = a.query_start_loc[b], run = a.query_start_loc[b + 1] - t_begin;
+  if (run <= kStepRows) return;
+  const int D = a.dim, V = a.vdim, vp = (V + 15) / 16 * 16;
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = v0 + c;
+  const int64_t per = delta_block_floats(DP, vp);
+  const float* base = a.scratch + ((int64_t)(t_begin / kRows + b) * a.heads + h) * per;
+  const int64_t step = (int64_t)a.heads * per;
+  float* st = a.state + (((int64_t)a.state_slots[b] * a.heads + h) * V + (col < V ? col : 0)) * D;
+  const bool resume = a.context_lens[b] > 0;
+  f32x4 s[DX];
+#pragma unroll
+  for (int x = 0; x < DX; ++x) {
+    const int d = 16 * (w * DX + x) + 4 * g;
+    s[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (resume && col < V) s[x] = load4<F32>(st, d, D, a.vec_state);
+  }
+  const int blocks = (run + kRows - 1) / kRows;
+  struct Block {
+    f32x4 wv[DX][2], qv[DX][2], kv[DX][2], u[2];
+    float av[3], g_last;
+  };
+  const int at_x = w * DX * 2 * 256 + 4 * lane, at_a = w * 64 + lane, at_u = blockIdx.y * 2 * 256 + 4 * lane;
+  auto fetch = [&](Block& f, const float* p) {
+#pragma unroll
+    for (int x = 0; x < DX; ++x)
+#pragma unroll
+      for (int it = 0; it < 2; ++it) {
+        const float* px = p + at_x + (2 * x + it) * 256;
+        f.wv[x][it] = *reinterpret_cast<const f32x4*>(px);
+        f.qv[x][it] = *reinterpret_cast<const f32x4*>(px + kRows * DP);
+        f.kv[x][it] = *reinterpret_cast<const f32x4*>(px + 2 * kRows * DP);
+      }
+    const float* pa = p + 3 * kRows * DP;
+    f.g_last = pa[0];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) f.av[i] = pa[4 + at_a + 256 * i];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) f.u[it] = *reinterpret_cast<const f32x4*>(pa + 4 + 3 * 256 + at_u + 256 * it);
+  };
+  // wave w finishes rows 16 it + 4 g + w of a block's outputs; what has no place goes to the block's pad
+  const int64_t row_step = (int64_t)a.heads * V;
+  float* o_at = a.o + ((int64_t)(t_begin + 4 * g + w) * a.heads + h) * V + (col < V ? col : 0);
+  float* nowhere = a.scratch + ((int64_t)(t_begin / kRows + b) * a.heads + h) * per + 3 * kRows * DP + 1;
+  auto finish = [&](int i) {
+    const int buf = i & 1;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const float o = (o_part[buf][0][it][w][lane] + o_part[buf][1][it][w][lane]) +
+                      (o_part[buf][2][it][w][lane] + o_part[buf][3][it][w][lane]);
+      const bool live = i * kRows + 16 * it + 4 * g + w < run && col < V;
+      *(live ? o_at + 16 * it * row_step : nowhere) = o;
+    }
+    o_at += kRows * row_step;
+  };
+  auto advance = [&](const Block& f, int i) {
+    const int buf = i & 1;
+    f32x4 xu[2], xo[2];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) xu[it] = xo[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < DX; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int it = 0; it < 2; ++it) xu[it] = mfma4(f.wv[x][it][e], s[x][e], xu[it]);
+#pragma unroll
+    for (int it = 0; it < 2; ++it) *reinterpret_cast<f32x4*>(&u_part[buf][w][it][lane][0]) = xu[it];
+    __syncthreads();
+    f32x4 p[2][4];
+#pragma unroll
+    for (int it = 0; it < 2; ++it)
+#pragma unroll
+      for (int ow = 0; ow < 4; ++ow) p[it][ow] = *reinterpret_cast<const f32x4*>(&u_part[buf][ow][it][lane][0]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int x = 0; x < DX; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int it = 0; it < 2; ++it) xo[it] = mfma4(f.qv[x][it][e], s[x][e], xo[it]);
+    if (i > 0) finish(i - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 u[2];
+#pragma unroll
+    for (int it = 0; it < 2; ++it)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        u[it][e] = f.u[it][e] - ((p[it][0][e] + p[it][1][e]) + (p[it][2][e] + p[it][3][e]));
+#pragma unroll
+    for (int x = 0; x < DX; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[x][e] *= f.g_last;
+#pragma unroll
+    for (int it = 0; it < 2; ++it)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int x = 0; x < DX; ++x) s[x] = mfma4(f.kv[x][it][e], u[it][e], s[x]);
+    // A U: the wave takes contraction index 4 g + w, so that the sum over waves is the whole product
+    const float u0 = w == 0 ? u[0][0] : w == 1 ? u[0][1] : w == 2 ? u[0][2] : u[0][3];
+    const float u1 = w == 0 ? u[1][0] : w == 1 ? u[1][1] : w == 2 ? u[1][2] : u[1][3];
+    xo[0] = mfma4(f.av[0], u0, xo[0]);
+    xo[1] = mfma4(f.av[1], u0, xo[1]);
+    xo[1] = mfma4(f.av[2], u1, xo[1]);
+#pragma unroll
+    for (int it = 0; it < 2; ++it)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o_part[buf][w][it][e][lane] = xo[it][e];
+  };
+  // two blocks in turn, so that one is asked for while the other is worked on
+  Block f0, f1;
+  fetch(f0, base);
+  for (int i = 0; i < blocks; i += 2) {
+    fetch(f1, base + (int64_t)min(i + 1, blocks - 1) * step);
+    __builtin_amdgcn_sched_barrier(0);
+    advance(f0, i);
+    if (i + 1 >= blocks) break;
+    fetch(f0, base + (int64_t)min(i + 2, blocks - 1) * step);
+    __builtin_amdgcn_sched_barrier(0);
+    advance(f1, i + 1);
+  }
+  __syncthreads();
+  finish(blocks - 1);
+  if (col < V) {
+#pragma unroll
+    for (int x = 0; x < DX; ++x) {
+      const int d = 16 * (w * DX + x) + 4 * g;
+      if (a.vec_state) {
+        if (d < D) *reinterpret_cast<f32x4*>(st + d) = s[x];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (d + e < D) st[d + e] = s[x][e];
+      }
+    }
+  }
+}
+
+template <int DX>
+int launch_delta_blocks(const DeltaBlocks& a, int64_t slots, hipStream_t stream) {
+  constexpr size_t lds = delta_prepare_lds_floats(64 * DX) * sizeof(float);
+  static std::atomic<bool> raised{false};           // LDS limit: raised once per kernel, not per launch
+  if (lds > 64 * 1024 && !raised.load(std::memory_order_relaxed)) {
+    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_block_prepare_kernel<DX>),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    raised.store(true, std::memory_order_relaxed);
+  }
+  delta_block_prepare_kernel<DX><<<dim3((unsigned)slots, a.heads), 256, lds, stream>>>(a);
+  VLA_SEQ_HIP_CHECK(hipGetLastError());
+  delta_block_walk_kernel<DX><<<dim3(a.heads, (a.vdim + 15) / 16, a.num_seqs), 256, 0, stream>>>(a);
+  VLA_SEQ_HIP_CHECK(hipGetLastError());
+  return VLA_OK;
+}
+
+int64_t delta_block_slots(int num_tokens, int num_seqs) { return (int64_t)num_tokens / kRows + num_seqs; }
+
 // out = dtype(o / sqrt(mean_v(o^2) + eps) * weight * silu(gate)) per (token, head): one wave each
 template <class SI, class SO>
 __global__ __launch_bounds__(256) void delta_head_norm_kernel(
@@ -372,7 +930,57 @@ __global__ __launch_bounds__(256) void delta_head_norm_kernel(
   }
 }
 
+// The same for heads of up to 256 values, four per lane: `lanes` neighbours share a (token, head), 16, 32
+// or 64 of them.  Bound by HBM: 4853 tokens of 16 heads of 128 are 99 MB.
+template <class SO>
+__global__ __launch_bounds__(256) void delta_head_norm_vec_kernel(
+    typename SO::T* __restrict__ out, int64_t out_stride, const float* __restrict__ o,
+    const float* __restrict__ gate, int64_t gate_stride, const float* __restrict__ weight, float eps,
+    int rows, int heads, int vdim, int lanes) {
+  const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / lanes;      // token * heads + head
+  const int d = 4 * (threadIdx.x & (lanes - 1));
+  const bool live = row < rows && d < vdim;
+  const int64_t t = (row < rows ? row : 0) / heads;
+  const int h = (int)((row < rows ? row : 0) - t * heads);
+  f32x4 x = {0.f, 0.f, 0.f, 0.f}, gt = x, wt = x;
+  if (live) {
+    x = *reinterpret_cast<const f32x4*>(o + row * vdim + d);
+    gt = *reinterpret_cast<const f32x4*>(gate + t * gate_stride + (int64_t)h * vdim + d);
+    wt = *reinterpret_cast<const f32x4*>(weight + d);
+  }
+  float ss = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3], none = 0.f;
+  group_sums(ss, none, 16);
+  if (lanes > 16) ss += __shfl_xor(ss, 16, 64);
+  if (lanes > 32) ss += __shfl_xor(ss, 32, 64);
+  const float inv = 1.f / sqrtf(ss / (float)vdim + eps);
+  if (!live) return;
+  float y[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = x[e] * inv * wt[e] * (gt[e] / (1.f + expf(-gt[e])));
+  typename SO::T* dst = out + t * out_stride + (int64_t)h * vdim + d;
+  if constexpr (sizeof(typename SO::T) == 2)
+    *reinterpret_cast<u32x2*>(dst) = u32x2{pack16<SO>(y[0], y[1]), pack16<SO>(y[2], y[3])};
+  else
+    *reinterpret_cast<f32x4*>(dst) = f32x4{y[0], y[1], y[2], y[3]};
+}
+
 std::atomic<int> g_delta_kernel{0};
+
+// Blocks pay from about a block's rows on (us per call with its Python wrapper, 16 heads of 128, token by
+// token / in blocks: one run of 24 rows 33 / 35, 100 rows 44 / 36; six runs of 24 rows 33 / 39, 33 rows
+// 39 / 38, 48 rows 48 / 39, 100 rows 86 / 47).  Their scratch is 68 KB per block and head of 128 x 128;
+// a step that would want more than 4 GiB of it walks token by token.
+constexpr int kBlockMinRows = 33;
+
+int64_t delta_out_floats(int num_tokens, int heads, int vdim) {
+  return ((int64_t)num_tokens * heads * vdim + 3) / 4 * 4;
+}
+
+bool wants_blocks(int mode, int num_tokens, int num_seqs, int max_query_len, int heads, int dim, int vdim) {
+  if (mode != 0 || dim > kMaxBlockDim || max_query_len < kBlockMinRows || (vdim + 15) / 16 > 65535) return false;
+  return delta_block_slots(num_tokens, num_seqs) * heads *
+             delta_block_floats((dim + 63) / 64 * 64, (vdim + 15) / 16 * 16) <= ((int64_t)1 << 30);
+}
 
 int pow2_at_least(int n) {
   int p = 1;
@@ -387,18 +995,17 @@ int pow2_at_least(int n) {
 using namespace vla;
 using namespace vla::seq;
 
-extern "C" int64_t vla_seq_delta_rule_scratch_floats(int num_tokens, int heads, int vdim) {
-  return (int64_t)num_tokens * heads * vdim;
-}
+namespace {
 
-extern "C" int vla_seq_delta_rule_scan(
+// scratch_floats < 0: as many as vla_seq_delta_rule_scratch_floats says, which holds no blocks
+int delta_rule_scan(
     void* out, int64_t out_stride, int out_dtype, const void* q, int64_t q_stride, const void* k,
     int64_t k_stride, const void* v, int64_t v_stride, const void* gate, int64_t gate_stride,
     const void* beta, int64_t beta_stride, const void* dt, int64_t dt_stride, int in_dtype,
     const float* a_log, const float* dt_bias, const float* norm_weight, float* state,
     const int* query_start_loc, const int* context_lens, const int* state_slots, int num_tokens,
     int num_seqs, int max_query_len, int num_slots, int heads, int kv_heads, int dim, int vdim,
-    float eps, float* scratch, void* stream) {
+    float eps, float* scratch, int64_t scratch_floats, void* stream) {
   if (num_seqs == 0 || num_tokens == 0) return VLA_OK;
   if (!out || !q || !k || !v || !gate || !beta || !dt || !a_log || !dt_bias || !norm_weight ||
       !state || !scratch || !query_start_loc || !context_lens || !state_slots || num_seqs < 0 ||
@@ -444,12 +1051,47 @@ extern "C" int vla_seq_delta_rule_scan(
   const dim3 grid(col_groups, heads, num_seqs);
   // runs of at most four rows take the kernel without staging (modes 1 / 2: always / never, for tests)
   const int mode = g_delta_kernel.load(std::memory_order_relaxed);
-  const bool steps = mode == 1 || (mode == 0 && max_query_len > 0 && max_query_len <= 4);
+  const bool blocks = scratch_floats >= 0 && wants_blocks(mode, num_tokens, num_seqs, max_query_len, heads, dim, vdim);
+  const bool steps = blocks ? num_seqs > 1 : mode == 1 || (mode == 0 && max_query_len > 0 && max_query_len <= kStepRows);
+  const int64_t out_floats = delta_out_floats(num_tokens, heads, vdim);
+  if (blocks) {
+    DeltaBlocks a;
+    a.o = scratch;
+    a.in = in;
+    a.a_log = a_log;
+    a.dt_bias = dt_bias;
+    a.state = state;
+    a.scratch = scratch + out_floats;
+    a.query_start_loc = query_start_loc;
+    a.context_lens = context_lens;
+    a.state_slots = state_slots;
+    a.num_seqs = num_seqs;
+    a.heads = heads;
+    a.kv_heads = kv_heads;
+    a.dim = dim;
+    a.vdim = vdim;
+    auto fours = [&](const void* p, int64_t stride) {              // four values per access
+      return dim % 4 == 0 && stride % 4 == 0 && (uintptr_t)p % 16 == 0;
+    };
+    a.vec_qk = fours(q, q_stride) && fours(k, k_stride);
+    a.vec_state = fours(state, 0);
+    const int64_t slots = delta_block_slots(num_tokens, num_seqs);
+    if ((uintptr_t)scratch % 16 || scratch_floats < out_floats + slots * heads * delta_block_floats((dim + 63) / 64 * 64, (vdim + 15) / 16 * 16))
+      return VLA_ERR_ARG;
+    int rc = VLA_OK;
+    switch ((dim + 63) / 64) {
+      case 1: rc = launch_delta_blocks<1>(a, slots, (hipStream_t)stream); break;
+      case 2: rc = launch_delta_blocks<2>(a, slots, (hipStream_t)stream); break;
+      case 3: rc = launch_delta_blocks<3>(a, slots, (hipStream_t)stream); break;
+      default: rc = launch_delta_blocks<4>(a, slots, (hipStream_t)stream); break;
+    }
+    if (rc != VLA_OK) return rc;
+  }
   if (steps) {
     auto launch_step = [&](auto kernel) {
       kernel<<<grid, threads, 0, (hipStream_t)stream>>>(scratch, in, a_log, dt_bias, state, query_start_loc,
                                                         context_lens, state_slots, heads, kv_heads, dim, vdim,
-                                                        split, cols);
+                                                        split, cols, blocks ? kStepRows : 0);
     };
     switch (rows) {
       case 8: launch_step(delta_rule_step_kernel<SI, 8>); break;
@@ -463,7 +1105,7 @@ extern "C" int vla_seq_delta_rule_scan(
                                                         context_lens, state_slots, heads, kv_heads, dim,
                                                         vdim, split, cols, chunk);
   };
-  if (!steps) {
+  if (!steps && !blocks) {
     switch (rows) {
       case 8: launch(delta_rule_kernel<SI, 8>); break;
       case 16: launch(delta_rule_kernel<SI, 16>); break;
@@ -475,12 +1117,65 @@ extern "C" int vla_seq_delta_rule_scan(
   return with_dtype(out_dtype, [&](auto so) {
     using SO = decltype(so);
     const int64_t head_rows = (int64_t)num_tokens * heads;
+    const int quads = sizeof(typename SO::T) == 2 ? 8 : 16;         // bytes a lane writes
+    if (vdim % 4 == 0 && vdim <= 256 && gate_stride % 4 == 0 && (uintptr_t)gate % 16 == 0 && out_stride % 4 == 0 &&
+        (uintptr_t)out % quads == 0 && (uintptr_t)norm_weight % 16 == 0 && (uintptr_t)scratch % 16 == 0) {
+      const int lanes = vdim <= 64 ? 16 : vdim <= 128 ? 32 : 64;
+      delta_head_norm_vec_kernel<SO><<<(unsigned)((head_rows * lanes + 255) / 256), 256, 0, (hipStream_t)stream>>>(
+          (typename SO::T*)out, out_stride, scratch, (const float*)gate, gate_stride, norm_weight, eps, (int)head_rows,
+          heads, vdim, lanes);
+      VLA_SEQ_HIP_CHECK(hipGetLastError());
+      return VLA_OK;
+    }
     delta_head_norm_kernel<SI, SO><<<(unsigned)((head_rows + 3) / 4), 256, 0, (hipStream_t)stream>>>(
         (typename SO::T*)out, out_stride, scratch, (const float*)gate, gate_stride, norm_weight, eps,
         (int)head_rows, heads, vdim);
     VLA_SEQ_HIP_CHECK(hipGetLastError());
     return VLA_OK;
   });
+}
+
+}  // namespace
+
+extern "C" int64_t vla_seq_delta_rule_scratch_floats(int num_tokens, int heads, int vdim) {
+  return (int64_t)num_tokens * heads * vdim;
+}
+
+extern "C" int64_t vla_seq_delta_rule_block_scratch_floats(int num_tokens, int num_seqs, int max_query_len, int heads,
+                                                           int dim, int vdim) {
+  const int64_t o = delta_out_floats(num_tokens, heads, vdim);
+  if (!wants_blocks(g_delta_kernel.load(std::memory_order_relaxed), num_tokens, num_seqs, max_query_len, heads, dim, vdim))
+    return o;
+  return o + delta_block_slots(num_tokens, num_seqs) * heads * delta_block_floats((dim + 63) / 64 * 64, (vdim + 15) / 16 * 16);
+}
+
+extern "C" int vla_seq_delta_rule_scan(
+    void* out, int64_t out_stride, int out_dtype, const void* q, int64_t q_stride, const void* k,
+    int64_t k_stride, const void* v, int64_t v_stride, const void* gate, int64_t gate_stride,
+    const void* beta, int64_t beta_stride, const void* dt, int64_t dt_stride, int in_dtype,
+    const float* a_log, const float* dt_bias, const float* norm_weight, float* state,
+    const int* query_start_loc, const int* context_lens, const int* state_slots, int num_tokens,
+    int num_seqs, int max_query_len, int num_slots, int heads, int kv_heads, int dim, int vdim,
+    float eps, float* scratch, void* stream) {
+  return delta_rule_scan(out, out_stride, out_dtype, q, q_stride, k, k_stride, v, v_stride, gate, gate_stride, beta, beta_stride,
+                         dt, dt_stride, in_dtype, a_log, dt_bias, norm_weight, state, query_start_loc, context_lens,
+                         state_slots, num_tokens, num_seqs, max_query_len, num_slots, heads, kv_heads, dim, vdim, eps,
+                         scratch, -1, stream);
+}
+
+extern "C" int vla_seq_delta_rule_scan_blocks(
+    void* out, int64_t out_stride, int out_dtype, const void* q, int64_t q_stride, const void* k,
+    int64_t k_stride, const void* v, int64_t v_stride, const void* gate, int64_t gate_stride,
+    const void* beta, int64_t beta_stride, const void* dt, int64_t dt_stride, int in_dtype,
+    const float* a_log, const float* dt_bias, const float* norm_weight, float* state,
+    const int* query_start_loc, const int* context_lens, const int* state_slots, int num_tokens,
+    int num_seqs, int max_query_len, int num_slots, int heads, int kv_heads, int dim, int vdim,
+    float eps, float* scratch, int64_t scratch_floats, void* stream) {
+  if (scratch_floats < 0) return VLA_ERR_ARG;
+  return delta_rule_scan(out, out_stride, out_dtype, q, q_stride, k, k_stride, v, v_stride, gate, gate_stride, beta, beta_stride,
+                         dt, dt_stride, in_dtype, a_log, dt_bias, norm_weight, state, query_start_loc, context_lens,
+                         state_slots, num_tokens, num_seqs, max_query_len, num_slots, heads, kv_heads, dim, vdim, eps,
+                         scratch, scratch_floats, stream);
 }
 
 // 0: pick per step; 1: always the kernel without staging; 2: never (tests run both)
