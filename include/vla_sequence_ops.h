@@ -368,6 +368,25 @@ int vla_seq_embed_scaled(float* out, const void* table, const int64_t* ids, floa
 /* z <- cap * tanh(z / cap) over n fp32 values. */
 int vla_seq_softcap(float* z, int64_t n, float cap, void* stream);
 
+/* Latent attention over runs of rows with keys and values formed per head (16-bit types; dim, rot, vdim,
+ * rank multiples of 8, dim + rot <= 192, vdim <= 128; scale > 0).
+ * vla_seq_latent_gather: sequence b's visible cache rows (from max(0, context - window + 1) on, from 0
+ * without a window, to its last new row) behind those of the sequences before it: rows [num_rows, width].
+ * max_seq_rows: the most rows of one sequence.
+ * vla_seq_latent_prompt: out [T, heads * vdim] from q [T, heads * (dim + rot)] (a head's row: plain | rotated),
+ * keys [num_rows, heads * dim] and values [num_rows, heads * vdim] that the caller formed from the gathered
+ * latents, and the gathered rows themselves for the rotated parts behind them. */
+int vla_seq_latent_prompt_supported(int dim, int rot, int vdim, int rank, int dtype);
+int vla_seq_latent_gather(void* rows, int num_rows, const void* cache, const int* block_tables,
+                          int max_blocks, const int* query_start_loc, const int* context_lens, int num_seqs,
+                          int max_seq_rows, int width, int block_size, int num_blocks, int window, int dtype,
+                          void* stream);
+int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* keys,
+                          const void* values, const void* rows, int num_rows, const int* query_start_loc,
+                          const int* context_lens, int num_seqs, int max_query_len, int heads, int dim,
+                          int rot, int vdim, int rank, float scale, int window, const void* gate,
+                          int64_t gate_stride, const float* sinks, int dtype, void* stream);
+
 /* ---- gated delta rule ----------------------------------------------------------------------------- */
 
 /* Per head, with a state S fp32 [dim, vdim] per sequence (stored [num_slots, heads, vdim, dim]):

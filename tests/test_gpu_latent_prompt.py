@@ -1,0 +1,72 @@
+"""Latent attention with keys and values formed per head: runs around the tiles of 128 rows and 64 keys, head
+sizes around the padding of the two kernels (128 and 192 numbers a key, 64 and 128 a value), windows, gates,
+steps that mix long runs with single rows, and what must keep taking the latent kernel.  Oracle and bound
+(6 % of the largest value where operands and weights are rounded to bfloat16) are those of the other latent
+tests; against the latent kernel itself the bound is half of that, since both round alike."""
+import pytest
+import torch
+
+from tests.test_gpu_tekezen import DEV, latent_layer_of, latent_reference, rnd, run_latent
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(2, 128, 64, 128, 64), (3, 32, 16, 40, 32), (4, 64, 64, 72, 128), (2, 96, 0, 128, 512), (1, 136, 56, 8, 32),
+         (2, 8, 8, 64, 32)]
+
+
+@pytest.mark.parametrize("sizes", SIZES)
+@pytest.mark.parametrize("cuts,window", [([127, 1, 129], 0), ([257], 70), ([64, 65, 2, 130], 129), ([300], 1), ([128, 128], 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_runs_around_a_tile(sizes, cuts, window, dtype):
+    attn, uk, uv, nw = latent_layer_of(sizes, dtype, None, window)
+    H, D, Rr, V, C = sizes
+    n = sum(cuts)
+    q, kv, gate = (t.to(dtype).float() for t in (rnd((n, H * (D + Rr)), 5, 1.5), rnd((n, C + Rr), 6, 1.5), rnd((n, H), 7, 2.0)))
+    want, _ = latent_reference(sizes, q, kv, gate, uk, uv, nw, None, window)
+    assert attn.formed_min_rows() <= 127
+    attn.FORMED_MIN_WORK = 0
+    got = run_latent(attn, sizes, q, kv, gate, cuts, dtype)
+    assert float((got - want).abs().max()) <= 0.06 * float(want.abs().max())
+
+
+def step(lens, contexts, block_size=16):
+    from vllm_legacy_amd.attention.batch import SequenceBatch
+    need = [-(-(n + c) // block_size) for n, c in zip(lens, contexts)]
+    ids = torch.randperm(sum(need), generator=torch.Generator().manual_seed(1)).tolist()
+    tables = [ids[sum(need[:i]):sum(need[:i + 1])] for i in range(len(need))]
+    return SequenceBatch.build(lens, contexts, tables, list(range(len(lens))), block_size, DEV), sum(need)
+
+
+@pytest.mark.parametrize("lens,contexts", [([1, 1, 200, 130, 1], [50, 3, 0, 77, 400]), ([150], [333]),
+                                           ([140, 2, 150, 2, 160, 2], [0, 9, 10, 300, 5, 1]), ([31, 63, 300], [64, 0, 1])])
+@pytest.mark.parametrize("window,sinks", [(0, True), (100, False)])
+def test_stretches_of_a_step_agree_with_the_latent_kernel(lens, contexts, window, sinks):
+    from dataclasses import replace
+    from vllm_legacy_amd.attention.backends.latent_kv import LatentKVAttention
+    H, D, Rr, V, C = 4, 128, 64, 128, 128
+    batch, blocks = step(lens, contexts)
+    attn = LatentKVAttention(H, D, Rr, V, C, (D + Rr)**-0.5, Rr, 1e4, None, 1e-5, torch.bfloat16, DEV, window=window or None,
+                             sinks=sinks)
+    attn.set_weights(rnd((H * D, C), 1, C**-0.5), rnd((H * V, C), 2, C**-0.5), 1 + 0.1 * rnd((C, ), 3),
+                     rnd((H, ), 4) if sinks else None)
+    attn.FORMED_MIN_WORK = 0
+    T = sum(lens)
+    q, kv, gate = (rnd((T, w), s).to(torch.bfloat16).to(DEV) for w, s in ((H * (D + Rr), 5), (C + Rr, 6), (H + 3, 7)))
+    cache = rnd((blocks, 16, C + Rr), 8).to(torch.bfloat16).to(DEV)
+    stretches = attn._stretches(batch)
+    assert (stretches is None) == (len(lens) == 6)          # a step that alternates too often stays whole
+    got = attn(q.clone(), kv, cache.clone(), batch, gate[:, 1:H + 1])
+    want = attn(q.clone(), kv, cache.clone(), replace(batch, host_query_lens=None), gate[:, 1:H + 1])
+    assert float((got - want).abs().max()) <= 0.03 * float(want.abs().max())
+    assert torch.equal(got, want) == (stretches is None)
+
+
+def test_what_keeps_the_latent_kernel():
+    from vllm_legacy_amd.attention.backends.latent_kv import LatentKVAttention
+    batch, _ = step([200], [0])
+    for scale, rank, dtype, formed in ((0.1, 64, torch.bfloat16, True), (-0.1, 64, torch.bfloat16, False),
+                                       (0.0, 64, torch.bfloat16, False)):
+        attn = LatentKVAttention(2, 32, 0, 32, rank, scale, 0, 1e4, None, 1e-5, dtype, DEV)
+        assert attn._stretches(batch) is None           # too little work for the launches
+        attn.FORMED_MIN_WORK = 0
+        assert (attn._stretches(batch) is not None) == formed

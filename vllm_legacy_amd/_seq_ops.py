@@ -1042,3 +1042,54 @@ def latent_attention_tiles(out: torch.Tensor, q_lat: torch.Tensor, q_rot: torch.
             rot, BS, NB, float(scale), int(key_splits), _p(scratch), T, _dt(q_lat.dtype), int(window), _p(gate),
             0 if gate is None else _rows(gate, H), _p(sinks), _stream(q_lat.device)),
             "latent_attention_tiles")
+
+
+def latent_prompt_supported(q: torch.Tensor, dim: int, rot: int, vdim: int, rank: int, cache: torch.Tensor) -> bool:
+    """Whether latent_prompt takes these sizes, query rows [T, heads * (dim + rot)] and cache (never while
+    set_latent_attention_kernel keeps the matrix cores out, which the smallest sizes' answer tells)."""
+    if not _lib.seq_lib().vla_seq_latent_attention_tiles_supported(32, 0, _dt(q.dtype)):
+        return False
+    return (q.data_ptr() % 16 == 0 and (q.stride(0) % 8 == 0 or q.shape[0] == 1) and cache.data_ptr() % 16 == 0 and
+            bool(_lib.seq_lib().vla_seq_latent_prompt_supported(int(dim), int(rot), int(vdim), int(rank), _dt(q.dtype))))
+
+
+def latent_gather(rows: torch.Tensor, cache: torch.Tensor, block_tables: torch.Tensor, query_start_loc: torch.Tensor,
+                  context_lens: torch.Tensor, max_seq_rows: int, window: int = 0) -> None:
+    """rows [N, rank + rot] <- every sequence's cache rows that its new rows can see, one sequence behind the
+    other (N: their number, max_seq_rows: the most of one sequence)."""
+    _gpu(rows, cache, block_tables, query_start_loc, context_lens)
+    NB, BS, width = cache.shape
+    B = context_lens.numel()
+    assert rows.is_contiguous() and rows.dtype == cache.dtype and rows.shape[1] == width and cache.is_contiguous()
+    for t in (block_tables, query_start_loc, context_lens):
+        assert t.dtype == torch.int32 and t.is_contiguous()
+    assert block_tables.dim() == 2 and block_tables.shape[0] == B and query_start_loc.numel() == B + 1
+    with torch.cuda.device(cache.device):
+        seq_check(_lib.seq_lib().vla_seq_latent_gather(
+            rows.data_ptr(), rows.shape[0], cache.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
+            query_start_loc.data_ptr(), context_lens.data_ptr(), B, int(max_seq_rows), width, BS, NB, int(window),
+            _dt(cache.dtype), _stream(cache.device)), "latent_gather")
+
+
+def latent_prompt(out: torch.Tensor, q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, rows: torch.Tensor,
+                  query_start_loc: torch.Tensor, context_lens: torch.Tensor, max_query_len: int, heads: int, dim: int,
+                  rot: int, vdim: int, scale: float, window: int = 0, gate: Optional[torch.Tensor] = None,
+                  sinks: Optional[torch.Tensor] = None) -> None:
+    """out [T, H * vdim]; q [T, H * (dim + rot)] (views with free row strides); keys [N, H * dim] and values
+    [N, H * vdim] formed from the gathered rows [N, rank + rot] of latent_gather."""
+    _gpu(out, q, keys, values, rows, query_start_loc, context_lens, gate, sinks)
+    T, N, H, B = q.shape[0], rows.shape[0], int(heads), context_lens.numel()
+    assert out.dtype == q.dtype == keys.dtype == values.dtype == rows.dtype
+    assert keys.shape == (N, H * dim) and values.shape == (N, H * vdim) and out.shape == (T, H * vdim)
+    assert keys.is_contiguous() and values.is_contiguous() and rows.is_contiguous()
+    assert sinks is None or (sinks.dtype == torch.float32 and sinks.numel() == H and sinks.is_contiguous())
+    assert gate is None or gate.dtype == q.dtype
+    for t in (query_start_loc, context_lens):
+        assert t.dtype == torch.int32 and t.is_contiguous()
+    assert query_start_loc.numel() == B + 1
+    with torch.cuda.device(q.device):
+        seq_check(_lib.seq_lib().vla_seq_latent_prompt(
+            out.data_ptr(), _rows(out, H * vdim), q.data_ptr(), _rows(q, H * (dim + rot)), keys.data_ptr(),
+            values.data_ptr(), rows.data_ptr(), N, query_start_loc.data_ptr(), context_lens.data_ptr(), B,
+            int(max_query_len), H, int(dim), int(rot), int(vdim), rows.shape[1] - int(rot), float(scale), int(window),
+            _p(gate), 0 if gate is None else _rows(gate, H), _p(sinks), _dt(q.dtype), _stream(q.device)), "latent_prompt")

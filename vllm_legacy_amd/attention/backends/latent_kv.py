@@ -101,14 +101,104 @@ class LatentKVAttention(nn.Module):
         """Steps of few rows over long contexts (decode steps) share every row tile's keys out to
         several workgroups: enough of them to fill the part, none with fewer than KEYS_PER_SPLIT
         keys."""
+        return self._key_splits(batch.max_query_len, batch.num_seqs, batch.max_seq_len)
+
+    def _key_splits(self, max_query_len: int, num_seqs: int, keys: int) -> int:
         heads_per = min(self.num_heads, 32)
-        tiles = -(-batch.max_query_len // (32 // heads_per)) * -(-self.num_heads // heads_per) * batch.num_seqs
+        tiles = -(-max_query_len // (32 // heads_per)) * -(-self.num_heads // heads_per) * num_seqs
         if tiles >= self.SPLIT_BELOW_WORKGROUPS:
             return 1
-        keys = batch.max_seq_len
         if self.window:
-            keys = min(keys, self.window + batch.max_query_len)
+            keys = min(keys, self.window + max_query_len)
         return max(1, min(-(-self.SPLIT_BELOW_WORKGROUPS // tiles), keys // self.KEYS_PER_SPLIT, 32))
+
+    # the longest stretches of sequences a step is cut into; one that alternates more often stays whole
+    MAX_STRETCHES = 4
+
+    # multiply-adds of a step on the latent kernel (a fifth of a matrix product's rate) from which the other
+    # way's five launches more are paid back: rows x keys before them, 16 heads, latent / formed us per call:
+    # 256 x 0 113 / 127, 128 x 2000 121 / 128, four of 64 x 2000 181 / 166, 256 x 2000 188 / 125, sixteen of
+    # 48 x 1000 262 / 225, of 256 x 1000 1079 / 275
+    FORMED_MIN_WORK = 5e9
+
+    def formed_min_rows(self) -> int:
+        """Rows from which a run's keys and values are worth forming.  A (query, key) pair of a head costs the
+        latent kernel 2 rank + rot multiply-adds at a fifth of a matrix product's rate, the formed one
+        dim + rot + vdim at half of it; forming costs rank (dim + vdim) per key at the full rate.  (16 heads,
+        rank 512, 1000 and 2000 keys before the run: runs of 32 rows 189 / 220 us and 134 / 138 us latent /
+        formed, of 48 rows 262 / 225 and 181 / 160.)"""
+        C, D, R, V = self.rank, self.head_dim, self.rot_dim, self.value_dim
+        gain = 5 * (2 * C + R) - 2 * (D + R + V)
+        return max(48, -(-C * (D + V) // gain)) if gain > 0 else 1 << 30
+
+    def _stretches(self, batch: SequenceBatch):
+        """[[first sequence, one behind the last, first row, one behind the last, formed]]: neighbours that go
+        the same way; None when the whole step takes the latent kernel."""
+        least = self.formed_min_rows()
+        if batch.max_query_len < least or not self.scale > 0:
+            return None
+        q, ctx = batch.host_query_lens, batch.host_context_lens
+        if q is None or ctx is None:
+            return None
+        out, row, pairs = [], 0, 0
+        for b, (n, c) in enumerate(zip(q, ctx)):
+            if n >= least:
+                pairs += n * min(c, self.window or c) + (n * (n + 1) // 2 if not self.window else n * min(n, self.window))
+            if out and out[-1][4] == (n >= least):
+                out[-1][1], out[-1][3] = b + 1, row + n
+            else:
+                out.append([b, b + 1, row, row + n, n >= least])
+            row += n
+        if pairs * self.num_heads * (2 * self.rank + self.rot_dim) < self.FORMED_MIN_WORK:
+            return None
+        return out if len(out) <= self.MAX_STRETCHES else None
+
+    def _attend_formed(self, out, q, cache, batch: SequenceBatch, s0, s1, r0, r1, gate) -> None:
+        """Sequences s0 .. s1 - 1 (rows r0 .. r1 - 1) with keys and values formed per head."""
+        H, D, Rr, V, C = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.rank
+        ql, cl = batch.host_query_lens[s0:s1], batch.host_context_lens[s0:s1]
+        counts = [c + n - (max(0, c - self.window + 1) if self.window else 0) for n, c in zip(ql, cl)]
+        tables, ctx = batch.block_tables[s0:s1], batch.context_lens[s0:s1]
+        starts = batch.query_start_loc[s0:s1 + 1]
+        if r0:
+            starts = starts - r0
+        rows = torch.empty((sum(counts), C + Rr), dtype=q.dtype, device=q.device)
+        ops.latent_gather(rows, cache, tables, starts, ctx, max(counts), self.window)
+        latents = rows[:, :C]
+        keys = torch.mm(latents, self.w_uk.data.view(H * D, C).t())
+        values = torch.mm(latents, self.w_uv_t.data.transpose(0, 1).reshape(C, H * V))
+        ops.latent_prompt(out[r0:r1], q[r0:r1], keys, values, rows, starts, ctx, max(ql), H, D, Rr, V, self.scale,
+                          self.window, None if gate is None else gate[r0:r1],
+                          None if self.sinks is None else self.sinks.data)
+
+    def _attend_latent(self, q, cache, batch: SequenceBatch, s0, s1, r0, r1, gate) -> torch.Tensor:
+        """Sequences s0 .. s1 - 1 (rows r0 .. r1 - 1) on the cached latents -> [rows, heads * vdim]."""
+        H, D, Rr, V, C = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.rank
+        whole = s0 == 0 and s1 == batch.num_seqs
+        T = r1 - r0
+        sinks = None if self.sinks is None else self.sinks.data
+        q3 = q[r0:r1].view(T, H, D + Rr)
+        q_lat = torch.bmm(q3[:, :, :D].transpose(0, 1), self.w_uk.data)             # [H, T, C]
+        o_lat = torch.empty((H, T, C), dtype=q.dtype, device=q.device)
+        q_lat, q_rot, o_rows = q_lat.transpose(0, 1), q3[:, :, D:], o_lat.transpose(0, 1)
+        gate = None if gate is None else gate[r0:r1]
+        if ops.latent_attention_tiles_supported(q_lat, q_rot, cache):
+            # 16-bit models whose sizes fit: (token, head) rows in tiles of 32 on the matrix cores
+            if whole:
+                tables, starts, ctx, longest, splits = batch.block_tables, batch.query_start_loc, batch.context_lens, \
+                    batch.max_query_len, self.key_splits(batch)
+            else:
+                ql, cl = batch.host_query_lens[s0:s1], batch.host_context_lens[s0:s1]
+                tables, ctx, longest = batch.block_tables[s0:s1], batch.context_lens[s0:s1], max(ql)
+                starts = batch.query_start_loc[s0:s1 + 1] - r0
+                splits = self._key_splits(longest, s1 - s0, max(c + n for n, c in zip(ql, cl)))
+            ops.latent_attention_tiles(o_rows, q_lat, q_rot, cache, tables, starts, ctx, longest, self.scale, splits,
+                                       self.window, gate, sinks)
+        else:
+            ops.latent_attention(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.token_seq[r0:r1],
+                                 batch.positions[r0:r1], self.scale, self.window, gate, sinks)
+        o = torch.bmm(o_lat, self.w_uv_t.data)                                      # [H, T, V]
+        return o.transpose(0, 1).reshape(T, H * V)
 
     @staticmethod
     def get_cache_shape(num_blocks: int, block_size: int, rank: int, rot_dim: int) -> Tuple[int, ...]:
@@ -122,21 +212,16 @@ class LatentKVAttention(nn.Module):
         T = q.shape[0]
         H, D, Rr, V, C = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.rank
         assert (kv is not None) == self.own_latent
-        sinks = None if self.sinks is None else self.sinks.data
         if self.own_latent:
             ops.latent_rotary_write(q, D + Rr, D, H, kv, self.latent_norm.data, self.eps, cache, batch.positions,
                                     batch.slot_mapping, self.inv_freq, self.magnitude, self.rot_dims, self.interleaved)
-        q3 = q.view(T, H, D + Rr)
-        q_lat = torch.bmm(q3[:, :, :D].transpose(0, 1), self.w_uk.data)             # [H, T, C]
-        o_lat = torch.empty((H, T, C), dtype=q.dtype, device=q.device)
-        q_lat, q_rot, o_rows = q_lat.transpose(0, 1), q3[:, :, D:], o_lat.transpose(0, 1)
-        if ops.latent_attention_tiles_supported(q_lat, q_rot, cache):
-            # 16-bit models whose sizes fit: (token, head) rows in tiles of 32 on the matrix cores
-            ops.latent_attention_tiles(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.query_start_loc,
-                                       batch.context_lens, batch.max_query_len, self.scale,
-                                       self.key_splits(batch), self.window, gate, sinks)
-        else:
-            ops.latent_attention(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.token_seq, batch.positions,
-                                 self.scale, self.window, gate, sinks)
-        o = torch.bmm(o_lat, self.w_uv_t.data)                                      # [H, T, V]
-        return o.transpose(0, 1).reshape(T, H * V)
+        stretches = self._stretches(batch)
+        if stretches is None or not ops.latent_prompt_supported(q, D, Rr, V, C, cache):
+            return self._attend_latent(q, cache, batch, 0, batch.num_seqs, 0, T, gate)
+        out = torch.empty((T, H * V), dtype=q.dtype, device=q.device)
+        for s0, s1, r0, r1, formed in stretches:
+            if formed:
+                self._attend_formed(out, q, cache, batch, s0, s1, r0, r1, gate)
+            else:
+                out[r0:r1] = self._attend_latent(q, cache, batch, s0, s1, r0, r1, gate)
+        return out

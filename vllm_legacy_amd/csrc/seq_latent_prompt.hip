@@ -1,0 +1,423 @@
+// Latent attention over runs of rows with every head's keys and values formed from the cached latents.
+//
+// Scoring the cached latent itself costs a head 2 rank + rot numbers per (query, key) pair; a head's own
+// key and value cost dim + rot + vdim, and forming them rank (dim + vdim) per key and head, once for all
+// queries of the run.  A run of rows therefore gathers its visible cache rows into one place
+// (latent_gather_kernel), the caller multiplies them with the two up-projections, and
+// latent_prompt_kernel below is plain causal attention with keys [formed (dim) | shared rotated part
+// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 144 us (600 TFLOP/s) where
+// latent_attention_tile_kernel takes 1685, plus 8 us to gather and 35 for the two products (the products
+// on the query's side that they replace take 46).
+//
+// The rows of sequence b are its keys from first_b = max(0, context - window + 1) (0 without a window) to
+// its last new row; sequences follow each other, so a sequence's place is the sum of the counts before
+// it, which every workgroup forms for itself (nothing has to be planned on the host or copied there).
+//
+// latent_prompt_kernel<S, DB, VB>: a workgroup is 128 query rows of one head, 32 per wave, and walks key
+// tiles of 64.  Products on 32x32x16 MFMAs in transposed form (lane = (hf, c) = (lane >> 5, lane & 31)):
+//   S^T = K q^T   A = K: lane: key c, dims 16 ks + 8 hf .. + 7 (LDS);  B = q^T: query c (registers)
+//   O^T = V^T P^T B = P^T: the first product's result where it lies;   A = V^T: two transposing reads
+// Tiles come in by LDS-DMA, double-buffered, one barrier per tile and no staging registers.  A DMA
+// instruction writes 64 lanes x 16 bytes in a row, so rows cannot be padded; 16-byte pieces (values:
+// 64-byte ones) are exchanged within a row by the row's number instead, on the source's side, so that
+// the lanes of a read fall into different banks.  Two workgroups share a CU: one's softmax (about 30
+// vector cycles per score) runs under the other's products.  Workgroups of one head are 8 apart or a
+// multiple of it when heads are a multiple of 8, so they share an XCD's L2 for that head's keys.
+#include <algorithm>
+#include <atomic>
+
+#include "seq_common.h"
+
+namespace vla {
+namespace seq {
+namespace {
+
+constexpr int kKeys = 64;           // keys of a tile
+constexpr int kRowsPerWave = 32;
+constexpr int kWaves = 4;
+constexpr int kRowsPerGroup = kRowsPerWave * kWaves;
+constexpr int kGatherRows = 32;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef s16x4 __attribute__((address_space(3))) * lds_s16x4;
+
+template <class S>
+struct Mma;
+template <>
+struct Mma<BF16> {
+  static __device__ __forceinline__ f32x16 run(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float a, float b) {
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+  }
+};
+template <>
+struct Mma<F16> {
+  static __device__ __forceinline__ f32x16 run(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float a, float b) {
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
+  }
+};
+
+__device__ __forceinline__ int first_formed(int context, int window) { return window > 0 ? max(0, context - window + 1) : 0; }
+
+// where sequence b's rows begin among all gathered rows (one wave; every lane gets it)
+__device__ __forceinline__ int gathered_before(const int* __restrict__ query_start_loc,
+                                               const int* __restrict__ context_lens, int b, int window) {
+  int n = 0;
+  for (int i = threadIdx.x & 63; i < b; i += kWave)
+    n += context_lens[i] + query_start_loc[i + 1] - query_start_loc[i] - first_formed(context_lens[i], window);
+#pragma unroll
+  for (int m = 1; m < kWave; m <<= 1) n += __shfl_xor(n, m, 64);
+  return __builtin_amdgcn_readfirstlane(n);
+}
+
+// rows[k] = the cache row of the k-th visible key: kGatherRows rows per workgroup, 16 bytes per lane
+__global__ __launch_bounds__(256) void latent_gather_kernel(
+    u32x4* __restrict__ rows, const u32x4* __restrict__ cache, const int* __restrict__ block_tables,
+    int max_blocks, const int* __restrict__ query_start_loc, const int* __restrict__ context_lens,
+    int pieces, int block_size, int num_blocks, int window, int num_rows) {
+  const int b = blockIdx.y;
+  const int ctx = context_lens[b], first = first_formed(ctx, window);
+  const int n = ctx + query_start_loc[b + 1] - query_start_loc[b] - first;
+  const int r0 = blockIdx.x * kGatherRows;
+  if (r0 >= n) return;
+  const int base = gathered_before(query_start_loc, context_lens, b, window);
+  const int* table = block_tables + (int64_t)b * max_blocks;
+  const int count = min(kGatherRows, n - r0) * pieces;
+  for (int i = threadIdx.x; i < count; i += 256) {
+    const int r = i / pieces, v = i - r * pieces;
+    const int j = first + r0 + r;
+    int blk = table[j / block_size];
+    blk = (unsigned)blk < (unsigned)num_blocks ? blk : 0;  // a table the host filled wrongly reads block 0
+    if (base + r0 + r < num_rows)
+      rows[(int64_t)(base + r0 + r) * pieces + v] = cache[((int64_t)blk * block_size + j % block_size) * pieces + v];
+  }
+}
+
+struct LatentPrompt {
+  void* out;
+  int64_t out_stride;
+  const void* q;                // [T, heads * q_head]: a head's row is [plain (dim) | rotated (rot)]
+  int64_t q_stride;
+  const void* keys;             // [N, heads * dim]
+  const void* values;           // [N, heads * vdim]
+  const void* rows;             // [N, rank + rot]: the rotated part behind the latent
+  const int* query_start_loc;
+  const int* context_lens;
+  const void* gate;
+  int64_t gate_stride;
+  const float* sinks;
+  int heads, dim, rot, vdim, rank, window, num_rows, row_tiles;
+  float scale;
+};
+
+// 16 bytes per lane from each lane's own address into 1 KB of LDS (no register result)
+__device__ __forceinline__ void dma16(const void* src, uint32_t lds_at) {
+  unsigned keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(src), "s"(lds_at)
+      : "memory");
+}
+
+template <class S, int DB, int VB>
+__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
+  using T = typename S::T;
+  using M = Mma<S>;
+  constexpr int DQ = 32 * DB, VD = 32 * VB;
+  constexpr int KB = 2 * DQ, VBYTES = 2 * VD;              // bytes of a tile's rows
+  constexpr int KTILE = kKeys * KB, VTILE = kKeys * VBYTES, STAGE = KTILE + VTILE;
+  constexpr int KI = KTILE / 1024 / kWaves, VI = VTILE / 1024 / kWaves;      // DMA instructions per wave
+  // a key row is a whole number of 256 bytes (all 64 banks), or half of one more: which pieces change place
+  constexpr int KMASK = KB % 256 == 0 ? 15 : 7, KSHIFT = KB % 256 == 0 ? 0 : 1;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int h = blockIdx.x, b = blockIdx.z;
+  const int run = a.query_start_loc[b + 1] - a.query_start_loc[b];
+  const int tile = a.row_tiles - 1 - (int)blockIdx.y;       // the longest walks first
+  const int r0 = tile * kRowsPerGroup;
+  if (r0 >= run) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hf = lane >> 5, c = lane & 31;
+  const int ctx = a.context_lens[b], first = first_formed(ctx, a.window);
+  const int base = gathered_before(a.query_start_loc, a.context_lens, b, a.window);
+  if (base + ctx + run - first > a.num_rows) return;       // the host allocated for other lengths
+  const int n_rows = min(kRowsPerGroup, run - r0);         // rows of this workgroup
+  const int nq = min(kRowsPerWave, n_rows - kRowsPerWave * w);               // and of this wave (<= 0: none)
+  const int t0 = a.query_start_loc[b] + r0 + kRowsPerWave * w;
+  // positions, counted from the first gathered key
+  const int p0 = ctx + r0 + kRowsPerWave * w - first, pq = p0 + c;
+  const int p_end = ctx + r0 + n_rows - 1 - first, n_keys = ctx + run - first;
+  const int g_first = a.window > 0 ? max(0, ctx + r0 - first - a.window + 1) : 0;    // the group's first key
+  const int lo_q = a.window > 0 ? pq - a.window + 1 : 0;                       // this row's
+  const int lo_last = a.window > 0 ? p0 + kRowsPerWave - a.window : 0;         // the wave's last row's
+  const int lo_first = a.window > 0 ? p0 - a.window + 1 : 0;
+
+  u32x4 qf[DQ / 16];
+  const int width = a.dim + a.rot;
+#pragma unroll
+  for (int ks = 0; ks < DQ / 16; ++ks) {
+    u32x4 v = {0u, 0u, 0u, 0u};
+    const int d = 16 * ks + 8 * hf;
+    if (c < nq && d < width)
+      v = *reinterpret_cast<const u32x4*>((const T*)a.q + (int64_t)(t0 + c) * a.q_stride + (int64_t)h * width + d);
+    qf[ks] = v;
+  }
+  f32x16 o[VB];
+#pragma unroll
+  for (int n = 0; n < VB; ++n)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[n][i] = 0.f;
+  const float scale2 = a.scale * 1.4426950408889634f;      // scores in base 2; scale > 0
+  float m = -INFINITY, l = 0.f;
+  if (a.sinks != nullptr) {                                // the denominator's first term, counted in one lane half
+    m = a.sinks[h] * 1.4426950408889634f;
+    l = hf == 0 ? 1.f : 0.f;
+  }
+
+  // What this lane brings in: piece `at` of a tile in LDS is row at / pieces; which 16 bytes of the row
+  // stand there follows from the exchange.  Pieces past dim + rot (vdim) repeat the row's first ones; their
+  // products meet zeros of q (columns nobody writes).
+  const unsigned char* src_k[KI];
+  const unsigned char* src_v[VI];
+  int row_k[KI], row_v[VI];
+  int64_t step_k[KI];
+  const int64_t key_row = (int64_t)a.heads * a.dim * 2, value_row = (int64_t)a.heads * a.vdim * 2;
+  const int64_t lat_row = (int64_t)(a.rank + a.rot) * 2;
+#pragma unroll
+  for (int u = 0; u < KI; ++u) {
+    const int at = ((w * KI + u) * 1024 + 16 * lane) / 16, r = at / (KB / 16), s = at % (KB / 16);
+    const int piece = (s & ~KMASK) | ((s ^ (r >> KSHIFT)) & KMASK);
+    const int d = 8 * piece;
+    row_k[u] = r;
+    if (d < a.dim || d >= width) {
+      src_k[u] = (const unsigned char*)a.keys + (int64_t)base * key_row + ((int64_t)h * a.dim + (d < a.dim ? d : 0)) * 2;
+      step_k[u] = key_row;
+    } else {
+      src_k[u] = (const unsigned char*)a.rows + (int64_t)base * lat_row + (a.rank + d - a.dim) * 2;
+      step_k[u] = lat_row;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < VI; ++u) {
+    const int at = ((w * VI + u) * 1024 + 16 * lane) / 16, r = at / (VBYTES / 16), s = at % (VBYTES / 16);
+    const int f = VB == 4 ? r & 3 : (r >> 1) & (VB - 1);
+    const int d = 8 * ((((s >> 2) ^ f) << 2) | (s & 3));
+    row_v[u] = r;
+    src_v[u] = (const unsigned char*)a.values + (int64_t)base * value_row + ((int64_t)h * a.vdim + (d < a.vdim ? d : 0)) * 2;
+  }
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  auto bring = [&](int u0, int buf) {
+    const uint32_t to = lds0 + buf * STAGE;
+#pragma unroll
+    for (int u = 0; u < KI; ++u)
+      dma16(src_k[u] + (int64_t)min(u0 + row_k[u], n_keys - 1) * step_k[u], to + (w * KI + u) * 1024);
+#pragma unroll
+    for (int u = 0; u < VI; ++u)
+      dma16(src_v[u] + (int64_t)min(u0 + row_v[u], n_keys - 1) * value_row, to + KTILE + (w * VI + u) * 1024);
+  };
+  // where this lane reads: the exchanged piece of its key row, and the unit of its value rows
+  const int kx = (hf ^ ((c >> KSHIFT) & KMASK)) & KMASK;   // piece 2 ks + hf stands at 2 ks ^ kx within its group
+  const int i16 = c & 15;
+  const int vrow = 4 * hf + (i16 >> 2);
+  const int vf = VB == 4 ? vrow & 3 : (vrow >> 1) & (VB - 1);
+  const int vat = vrow * VBYTES + 32 * (c >> 4) + 8 * (i16 & 3);
+
+  int u0 = g_first & ~(kKeys - 1);
+  bring(u0, 0);
+  for (int it = 0; u0 <= p_end; u0 += kKeys, ++it) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (u0 + kKeys <= p_end) bring(u0 + kKeys, (it + 1) & 1);
+    const unsigned char* k_lds = smem + (it & 1) * STAGE;
+    const unsigned char* v_lds = k_lds + KTILE;
+    if (nq <= 0 || u0 > p0 + nq - 1 || u0 + kKeys <= lo_first) continue;     // no key of it concerns this wave
+    f32x16 st[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) st[kb][i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < DQ / 16; ++ks)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const int slot = ((2 * ks) & ~KMASK) | (((2 * ks) & KMASK) ^ kx);
+        const u32x4 ka = *reinterpret_cast<const u32x4*>(k_lds + (32 * kb + c) * KB + 16 * slot);
+        st[kb] = M::run(ka, qf[ks], st[kb]);
+      }
+    // every key of the tile visible to every row of the wave: no masks
+    if (!(u0 + kKeys - 1 <= p0 && u0 >= lo_last && nq == kRowsPerWave)) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int j = u0 + 32 * kb + (i & 3) + 8 * (i >> 2) + 4 * hf;
+          st[kb][i] = c < nq && j <= pq && j >= lo_q ? st[kb][i] : -INFINITY;
+        }
+    }
+    float mt = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mt = fmaxf(mt, st[kb][i]);
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64)) * scale2;
+    const float m_new = fmaxf(m, mt);
+    const float shift = m_new == -INFINITY ? 0.f : m_new;  // nothing seen yet: every weight is 2^-inf
+    const float corr = __builtin_amdgcn_exp2f(m - shift);
+    float psum = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kb][i], scale2, -shift));
+        st[kb][i] = pv;
+        psum += pv;
+      }
+    l = l * corr + psum;                                   // this lane's keys; the partner's half is added at the end
+    if (__any(m_new != m)) {                               // the running maximum of some row moved
+#pragma unroll
+      for (int n = 0; n < VB; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[n][i] *= corr;
+    }
+    m = m_new;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) {
+        u32x4 pb;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pb[e] = M::pack2(st[kb][8 * s2 + 2 * e], st[kb][8 * s2 + 2 * e + 1]);
+        const unsigned char* src = v_lds + vat + (32 * kb + 16 * s2) * VBYTES;
+#pragma unroll
+        for (int n = 0; n < VB; ++n) {
+          const unsigned char* at = src + 64 * (n ^ vf);
+          // 8 rows further on the exchange is the same for four units; for two it is too (8 / 2 even)
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)at);
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 8 * VBYTES));
+          const u32x2 lo2 = __builtin_bit_cast(u32x2, lo), hi2 = __builtin_bit_cast(u32x2, hi);
+          o[n] = M::run(u32x4{lo2[0], lo2[1], hi2[0], hi2[1]}, pb, o[n]);
+        }
+      }
+  }
+  l += __shfl_xor(l, 32, 64);
+  if (c >= nq) return;
+  float inv = 1.f / l;
+  if (a.gate != nullptr) inv /= 1.f + expf(-S::to_f32(((const T*)a.gate)[(int64_t)(t0 + c) * a.gate_stride + h]));
+  T* orow = (T*)a.out + (int64_t)(t0 + c) * a.out_stride + (int64_t)h * a.vdim + 4 * hf;
+#pragma unroll
+  for (int n = 0; n < VB; ++n)
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+      const int d = 32 * n + 8 * (i >> 2);
+      if (d + 4 * hf < a.vdim)
+        *reinterpret_cast<u32x2*>(orow + d) =
+            u32x2{M::pack2(o[n][i] * inv, o[n][i + 1] * inv), M::pack2(o[n][i + 2] * inv, o[n][i + 3] * inv)};
+    }
+}
+
+template <class S, int DB, int VB>
+int launch_latent_prompt(const LatentPrompt& a, dim3 grid, hipStream_t stream) {
+  constexpr size_t lds = 2 * kKeys * (64 * DB + 64 * VB);
+  static std::atomic<bool> raised{false};           // LDS limit: raised once per kernel, not per launch
+  if (lds > 64 * 1024 && !raised.load(std::memory_order_relaxed)) {
+    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_prompt_kernel<S, DB, VB>),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    raised.store(true, std::memory_order_relaxed);
+  }
+  latent_prompt_kernel<S, DB, VB><<<grid, 256, lds, stream>>>(a);
+  VLA_SEQ_HIP_CHECK(hipGetLastError());
+  return VLA_OK;
+}
+
+bool prompt_sizes(int dim, int rot, int vdim, int rank) {
+  return dim > 0 && dim % 8 == 0 && rot >= 0 && rot % 8 == 0 && vdim > 0 && vdim % 8 == 0 && rank > 0 && rank % 8 == 0 &&
+         dim + rot <= 192 && vdim <= 128;
+}
+
+}  // namespace
+}  // namespace seq
+}  // namespace vla
+
+using namespace vla;
+using namespace vla::seq;
+
+extern "C" int vla_seq_latent_prompt_supported(int dim, int rot, int vdim, int rank, int dtype) {
+  return (dtype == VLA_F16 || dtype == VLA_BF16) && prompt_sizes(dim, rot, vdim, rank);
+}
+
+extern "C" int vla_seq_latent_gather(void* rows, int num_rows, const void* cache, const int* block_tables,
+                                     int max_blocks, const int* query_start_loc, const int* context_lens,
+                                     int num_seqs, int max_seq_rows, int width, int block_size,
+                                     int num_blocks, int window, int dtype, void* stream) {
+  if (num_seqs == 0 || num_rows == 0) return VLA_OK;
+  if (!rows || !cache || !block_tables || !query_start_loc || !context_lens || num_seqs < 0 || num_seqs > 65535 ||
+      num_rows < 0 || max_seq_rows <= 0 || max_blocks <= 0 || width <= 0 || block_size <= 0 || num_blocks <= 0 ||
+      window < 0)
+    return VLA_ERR_ARG;
+  if (dtype != VLA_F16 && dtype != VLA_BF16) return VLA_ERR_DTYPE;
+  if (width % 8 || (uintptr_t)rows % 16 || (uintptr_t)cache % 16) return VLA_ERR_ARG;
+  latent_gather_kernel<<<dim3((max_seq_rows + kGatherRows - 1) / kGatherRows, num_seqs), 256, 0, (hipStream_t)stream>>>(
+      (u32x4*)rows, (const u32x4*)cache, block_tables, max_blocks, query_start_loc, context_lens, width / 8, block_size,
+      num_blocks, window, num_rows);
+  VLA_SEQ_HIP_CHECK(hipGetLastError());
+  return VLA_OK;
+}
+
+extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* q, int64_t q_stride,
+                                     const void* keys, const void* values, const void* rows, int num_rows,
+                                     const int* query_start_loc, const int* context_lens, int num_seqs,
+                                     int max_query_len, int heads, int dim, int rot, int vdim, int rank,
+                                     float scale, int window, const void* gate, int64_t gate_stride,
+                                     const float* sinks, int dtype, void* stream) {
+  if (num_seqs == 0 || max_query_len == 0) return VLA_OK;
+  if (!out || !q || !keys || !values || !rows || !query_start_loc || !context_lens || num_seqs < 0 ||
+      num_seqs > 65535 || max_query_len < 0 || num_rows <= 0 || heads <= 0 || heads > 65535 || !(scale > 0.f) ||
+      window < 0 || (gate && gate_stride < heads) || out_stride < (int64_t)heads * vdim ||
+      q_stride < (int64_t)heads * (dim + rot))
+    return VLA_ERR_ARG;
+  if (dtype != VLA_F16 && dtype != VLA_BF16) return VLA_ERR_DTYPE;
+  if (!prompt_sizes(dim, rot, vdim, rank)) return VLA_ERR_HEAD_SIZE;
+  if ((uintptr_t)q % 16 || q_stride % 8 || (uintptr_t)keys % 16 || (uintptr_t)values % 16 || (uintptr_t)rows % 16 ||
+      (uintptr_t)out % 8 || out_stride % 4)
+    return VLA_ERR_ARG;
+  LatentPrompt a;
+  a.out = out;
+  a.out_stride = out_stride;
+  a.q = q;
+  a.q_stride = q_stride;
+  a.keys = keys;
+  a.values = values;
+  a.rows = rows;
+  a.query_start_loc = query_start_loc;
+  a.context_lens = context_lens;
+  a.gate = gate;
+  a.gate_stride = gate_stride;
+  a.sinks = sinks;
+  a.heads = heads;
+  a.dim = dim;
+  a.rot = rot;
+  a.vdim = vdim;
+  a.rank = rank;
+  a.window = window;
+  a.num_rows = num_rows;
+  a.row_tiles = (max_query_len + kRowsPerGroup - 1) / kRowsPerGroup;
+  a.scale = scale;
+  if (a.row_tiles > 65535) return VLA_ERR_ARG;
+  const dim3 grid(heads, a.row_tiles, num_seqs);
+  auto go = [&](auto s) -> int {
+    using S = decltype(s);
+    const bool wide = dim + rot > 128;
+    if (vdim <= 64)
+      return wide ? launch_latent_prompt<S, 6, 2>(a, grid, (hipStream_t)stream)
+                  : launch_latent_prompt<S, 4, 2>(a, grid, (hipStream_t)stream);
+    return wide ? launch_latent_prompt<S, 6, 4>(a, grid, (hipStream_t)stream)
+                : launch_latent_prompt<S, 4, 4>(a, grid, (hipStream_t)stream);
+  };
+  return dtype == VLA_BF16 ? go(BF16{}) : go(F16{});
+}
