@@ -241,6 +241,19 @@ int vla_seq_kv_attention(void* out, int64_t out_stride, const void* q, int64_t q
                          int block_size, int num_blocks, int window, float scale, int dtype,
                          int keep_first, float softcap, int chunk, const float* sinks,
                          void* stream);
+/* The same with scratch (vla_seq_kv_attention_scratch_floats values; null and 0 if it says 0) in which the
+ * keys of a row may be shared out to several workgroups: few rows over long contexts.  max_keys: the most
+ * keys a row of the step sees. */
+int64_t vla_seq_kv_attention_scratch_floats(int num_tokens, int heads, int kv_heads, int dim, int vdim,
+                                            int max_keys, int dtype);
+int vla_seq_kv_attention_shared(void* out, int64_t out_stride, const void* q, int64_t q_stride,
+                         const void* gate, int64_t gate_stride, const void* key_cache,
+                         const void* value_cache, const int* block_tables, int max_blocks,
+                         const int* token_seq, const int64_t* positions, const float* out_inv_freq,
+                         int interleaved, int num_tokens, int heads, int kv_heads, int dim, int vdim,
+                         int block_size, int num_blocks, int window, float scale, int dtype,
+                         int keep_first, float softcap, int chunk, const float* sinks,
+                         int max_keys, float* scratch, int64_t scratch_floats, void* stream);
 
 /* The same attention for 16-bit activations, tiled over runs of 32 query rows of a sequence on
  * the matrix cores: rows query_start_loc[b] .. query_start_loc[b + 1] - 1 of sequence b sit at

@@ -449,12 +449,13 @@ def kv_attention(out: torch.Tensor, q: torch.Tensor, gate: Optional[torch.Tensor
                  value_cache: torch.Tensor, block_tables: torch.Tensor, token_seq: torch.Tensor,
                  positions: torch.Tensor, out_inv_freq: Optional[torch.Tensor], interleaved: bool, heads: int,
                  window: int, scale: float, keep_first: int = 0, softcap: float = 0.0, chunk: int = 0,
-                 sinks: Optional[torch.Tensor] = None) -> None:
+                 sinks: Optional[torch.Tensor] = None, max_keys: int = 0) -> None:
     """out [T, H*V] = softmax attention of q [T, H*D] over the caches, output pairs turned back by
     the position, times sigmoid(gate [T, H]).  With a window or a chunk the first keep_first tokens of a
     sequence stay visible; softcap > 0 caps the scores with softcap * tanh(score / softcap); chunk > 0:
     a row sees the keys of its own chunk of `chunk` positions only; sinks fp32 [H]: e^sinks joins a head's
-    softmax denominator."""
+    softmax denominator.  max_keys: the most keys a row of the step sees (0: unknown), by which the keys of
+    few rows are shared out to several workgroups."""
     _gpu(out, q, gate, key_cache, value_cache, block_tables, token_seq, positions, out_inv_freq, sinks)
     assert sinks is None or (sinks.dtype == torch.float32 and sinks.numel() == heads and sinks.is_contiguous())
     NB, BS, G, D = key_cache.shape
@@ -469,13 +470,17 @@ def kv_attention(out: torch.Tensor, q: torch.Tensor, gate: Optional[torch.Tensor
         assert out_inv_freq.dtype == torch.float32 and out_inv_freq.numel() == V // 2
     if gate is not None:
         assert gate.dtype == q.dtype
+    L = _lib.seq_lib()
+    need = L.vla_seq_kv_attention_scratch_floats(T, heads, G, D, V, int(max_keys), _dt(q.dtype))
+    scratch = torch.empty(need, dtype=torch.float32, device=q.device) if need else None
     with torch.cuda.device(q.device):
-        seq_check(_lib.seq_lib().vla_seq_kv_attention(
+        seq_check(L.vla_seq_kv_attention_shared(
             out.data_ptr(), _rows(out, heads * V), q.data_ptr(), _rows(q, heads * D), _p(gate),
             0 if gate is None else _rows(gate, heads), key_cache.data_ptr(), value_cache.data_ptr(),
             block_tables.data_ptr(), block_tables.shape[1], token_seq.data_ptr(), positions.data_ptr(),
             _p(out_inv_freq), int(bool(interleaved)), T, heads, G, D, V, BS, NB, int(window), float(scale),
-            _dt(q.dtype), int(keep_first), float(softcap), int(chunk), _p(sinks), _stream(q.device)), "kv_attention")
+            _dt(q.dtype), int(keep_first), float(softcap), int(chunk), _p(sinks), int(max_keys), _p(scratch), need,
+            _stream(q.device)), "kv_attention")
 
 
 def set_kv_attention_kernel(mode: int) -> None:

@@ -77,6 +77,11 @@ class RotaryKVAttention(nn.Module):
         return ((num_blocks, block_size, num_kv_heads, head_dim),
                 (num_blocks, block_size, num_kv_heads, value_dim))
 
+    def max_visible(self, keys: int) -> int:
+        """The most keys that a row at the end of `keys` tokens sees."""
+        limits = [x for x in (self.window, self.chunk) if x]
+        return min([keys] + [x + self.keep_first for x in limits])
+
     def forward(self, out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                 gate: Optional[torch.Tensor], key_cache: torch.Tensor, value_cache: torch.Tensor,
                 batch: SequenceBatch, v_other: Optional[torch.Tensor] = None,
@@ -100,5 +105,6 @@ class RotaryKVAttention(nn.Module):
         else:
             ops.kv_attention(out, q, gate, key_cache, value_cache, batch.block_tables, batch.token_seq,
                              batch.positions, self.value_inv_freq, self.interleaved, self.num_heads, self.window,
-                             self.scale, self.keep_first, self.softcap, self.chunk, self.sinks)
+                             self.scale, self.keep_first, self.softcap, self.chunk, self.sinks,
+                             self.max_visible(batch.max_seq_len))
         return out

@@ -907,6 +907,405 @@ __global__ __launch_bounds__(64 * kRowWaves) void kv_attention_heads_kernel(
   }
 }
 
+// kv_decode_kernel<S, DB, VB>: single rows again, for heads of 64 or 128 and values of 64 or 128 with at
+// most 16 query heads to a KV head, on 16x16x32 MFMAs (16 columns: the group's query heads; the 32x32
+// ones above leave 28 of 32 columns idle at a group of 4).  Bound by HBM: every key and value is read once.
+//   S^T = K q^T    A = K    lane (g, c) = (lane >> 4, lane & 15): key c, dims 32 ks + 8 g .. + 7
+//                  B = q^T  lane: head c, the same dims (registers)
+//                  C        lane: head c, keys 4 g .. 4 g + 3
+//   O^T = V^T P^T  B = P^T  lane: head c, keys 4 g .. + 3 of both halves of the tile, where they lie
+//                  A = V^T  lane: value dim 16 n + c of the same keys (two transposing reads)
+// A weight enters as the sum of two 16-bit numbers, as in the kernel above.  The four waves take tiles of 32
+// keys in turn, each through its own two LDS buffers that LDS-DMA fills a tile ahead: 64 KB on their way
+// per CU without a staging register, and no barrier in the loop.  A DMA instruction writes 64 lanes x 16
+// bytes in a row, so rows are not padded: 16-byte pieces of a key row and 32-byte units of a value row
+// are exchanged by the row's number, on the source's side, for reads without bank conflicts.  The block
+// table's part waits in LDS, because a table load inside the loop would have to wait for the DMA ahead of
+// it.  Few rows over long contexts: the keys of a row are shared out to `splits` workgroups, whose sums
+// kv_decode_merge_kernel joins.
+// 64 rows of 4096 keys, 16 / 4 heads of 128 (537 MB): 95 us = 5.6 TB/s (the kernel above 122; without the
+// nontemporal hint 108; one tile ahead instead of two, also without the hint, 106).
+constexpr int kDecodeWaves = 4;
+constexpr int kDecodeHeads = 16;
+constexpr int kDecodeKeys = 32;
+constexpr int kDecodeMinSplitKeys = 256;      // keys of a split, at least
+
+template <class S>
+struct Mma16x16;
+template <>
+struct Mma16x16<BF16> {
+  static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+};
+template <>
+struct Mma16x16<F16> {
+  static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+};
+
+struct KvDecode {
+  void* out;
+  int64_t out_stride;
+  const void* q;
+  int64_t q_stride;
+  const void* gate;
+  int64_t gate_stride;
+  const void* key_cache;
+  const void* value_cache;
+  const int* block_tables;
+  int max_blocks;
+  const int* token_seq;
+  const int64_t* positions;
+  const float* out_inv_freq;
+  const float* sinks;
+  float* parts;                 // [splits][T][heads][2 + VD]
+  int interleaved, num_tokens, heads, kv_heads, block_size, num_blocks, window, keep_first, chunk, v_row, v_first;
+  int splits, table_slots;
+  float scale, softcap;
+};
+
+// a head's output dim d (ov: its pair's other dim) turned back, gated and stored
+template <class S>
+__device__ __forceinline__ void finish_decode(const KvDecode& a, int64_t t, int h, int d, int vd, float val, float ov) {
+  if (a.out_inv_freq != nullptr) {
+    const bool is_a = a.interleaved ? (d & 1) == 0 : d < vd / 2;
+    const int f = a.interleaved ? d >> 1 : (is_a ? d : d - vd / 2);
+    float s, c;
+    sincosf((float)a.positions[t] * a.out_inv_freq[f], &s, &c);
+    val = is_a ? val * c + ov * s : val * c - ov * s;
+  }
+  using T = typename S::T;
+  if (a.gate != nullptr) val *= 1.f / (1.f + expf(-S::to_f32(((const T*)a.gate)[t * a.gate_stride + h])));
+  ((T*)a.out)[t * a.out_stride + (int64_t)h * a.v_row + a.v_first + d] = S::from_f32(val);
+}
+__device__ __forceinline__ int pair_of(const KvDecode& a, int d, int vd) {
+  return a.interleaved ? (d ^ 1) : (d < vd / 2 ? d + vd / 2 : d - vd / 2);
+}
+
+// 16 bytes per lane from each lane's own address into 1 KB of LDS (no register result); NT: read once, not kept
+template <bool NT>
+__device__ __forceinline__ void kv_dma16(const void* src, uint32_t lds_at) {
+  unsigned keep;
+  if constexpr (NT)
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt\n\ts_mov_b32 m0, %0"
+        : "=&s"(keep)
+        : "v"(src), "s"(lds_at)
+        : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+        : "=&s"(keep)
+        : "v"(src), "s"(lds_at)
+        : "memory");
+}
+// all DMA but the N youngest instructions has landed
+template <int N>
+__device__ __forceinline__ void kv_dma_landed() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <class S, int DB, int VB, bool NT>
+__global__ __launch_bounds__(64 * kDecodeWaves) void kv_decode_kernel(KvDecode a) {
+  using T = typename S::T;
+  using M = Mma16x16<S>;
+  constexpr int D = 32 * DB, VD = 32 * VB;
+  constexpr int KB = 2 * D, VBYTES = 2 * VD;               // bytes of a row of one KV head
+  constexpr int KTILE = kDecodeKeys * KB, STAGE = KTILE + kDecodeKeys * VBYTES;
+  constexpr int KI = KTILE / 1024, VI = STAGE / 1024 - KI; // DMA instructions of a tile
+  constexpr int KP = KB / 16, VP = VBYTES / 16;            // pieces of a row
+  static_assert((DB == 2 || DB == 4) && (VB == 2 || VB == 4), "rows of 128 or 256 bytes");
+  extern __shared__ __align__(16) unsigned char smem[];
+  int* table_lds = reinterpret_cast<int*>(smem + kDecodeWaves * 2 * STAGE);
+  const int t = blockIdx.x, g_kv = blockIdx.y, split = blockIdx.z;
+  const int group = a.heads / a.kv_heads, h0 = g_kv * group;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  const int p = (int)a.positions[t];
+  const int* table = a.block_tables + (int64_t)a.token_seq[t] * a.max_blocks;
+  const int lo = first_key(p, a.window, a.chunk);
+  const int nk = min(a.keep_first, lo);                    // kept keys ahead of the window
+  const int total = nk + p - lo + 1;
+  const int share = ((total + a.splits - 1) / a.splits + kDecodeKeys - 1) / kDecodeKeys * kDecodeKeys;
+  const int u_begin = split * share, u_end = min(total, u_begin + share);
+  auto key_of = [&](int u) { return u < nk ? u : u - nk + lo; };
+  const bool live = c < group;
+
+  u32x4 qf[DB];
+#pragma unroll
+  for (int ks = 0; ks < DB; ++ks) {
+    qf[ks] = u32x4{0u, 0u, 0u, 0u};
+    if (live) qf[ks] = *reinterpret_cast<const u32x4*>((const T*)a.q + (int64_t)t * a.q_stride + (int64_t)(h0 + c) * D + 32 * ks + 8 * g);
+  }
+  // the blocks of the kept keys, then those of the rest of this share; an id outside the pool (a table the
+  // host filled wrongly) reads block 0
+  const int kept_blocks = u_begin < nk ? (nk + a.block_size - 1) / a.block_size : 0;
+  const int first_block = key_of(max(u_begin, nk)) / a.block_size;
+  if (u_begin < u_end) {
+    const int last_block = key_of(u_end - 1) / a.block_size;
+    const int n = min(a.table_slots, kept_blocks + max(0, last_block - first_block + 1));
+    for (int i = tid; i < n; i += 64 * kDecodeWaves) {
+      const int blk = table[i < kept_blocks ? i : i - kept_blocks + first_block];
+      table_lds[i] = (unsigned)blk < (unsigned)a.num_blocks ? blk : 0;
+    }
+  }
+  __syncthreads();
+
+  f32x4 o[2 * VB];
+#pragma unroll
+  for (int n = 0; n < 2 * VB; ++n) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr float kLog2e = 1.4426950408889634f;
+  const float scale2 = a.scale * kLog2e;                   // scores in base 2
+  const float cap2 = a.softcap * kLog2e, cap_arg = a.softcap > 0.f ? 2.f * kLog2e / a.softcap : 0.f;
+  float m = -INFINITY, l = 0.f;
+  if (a.sinks != nullptr && live && w == 0 && split == 0) {     // the denominator's first term, counted once
+    m = a.sinks[h0 + c] * kLog2e;
+    l = g == 0 ? 1.f : 0.f;
+  }
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)smem + w * 2 * STAGE;
+  const unsigned char* mine = smem + w * 2 * STAGE;
+  const uint32_t key_step = (uint32_t)a.kv_heads * KB, value_step = (uint32_t)a.kv_heads * a.v_row * 2;
+  const unsigned char* keys = (const unsigned char*)a.key_cache + (size_t)g_kv * KB;
+  const unsigned char* values = (const unsigned char*)a.value_cache + ((size_t)g_kv * a.v_row + a.v_first) * 2;
+  // where a tile's keys lie (lane & 31: the key); behind the end: the last key again
+  auto places = [&](int u0) {
+    const int j = key_of(min(u0 + (lane & 31), u_end - 1));
+    const int blk = j / a.block_size;
+    const int at = j < lo ? blk : blk - first_block + kept_blocks;
+    return table_lds[min(at, a.table_slots - 1)] * a.block_size + (j - blk * a.block_size);
+  };
+  // a tile's DMA: a lane's rows and pieces (a piece's place within the row is exchanged by the row's number)
+  auto bring_keys = [&](int slot, int buf) {
+#pragma unroll
+    for (int u = 0; u < KI; ++u) {
+      const int r = u * (64 / KP) + lane / KP, s = lane % KP;
+      const int piece = s ^ (KP == 16 ? r & 15 : (r >> 1) & 7);
+      const uint32_t row = (uint32_t)__shfl(slot, r, 64);
+      kv_dma16<NT>(keys + (uint64_t)row * key_step + 16 * piece, lds0 + buf * STAGE + 1024 * u);
+    }
+  };
+  auto bring_values = [&](int slot, int buf) {
+#pragma unroll
+    for (int u = 0; u < VI; ++u) {
+      const int r = u * (64 / VP) + lane / VP, s = lane % VP;
+      const int piece = (((s >> 1) ^ (VP == 16 ? r & 7 : (r >> 1) & 3)) << 1) | (s & 1);
+      const uint32_t row = (uint32_t)__shfl(slot, r, 64);
+      kv_dma16<NT>(values + (uint64_t)row * value_step + 16 * piece, lds0 + buf * STAGE + KTILE + 1024 * u);
+    }
+  };
+  const int kx = KP == 16 ? c & 15 : (c >> 1) & 7;         // key rows c and 16 + c
+  const int vrow = 4 * g + (c >> 2);                       // value rows vrow and 16 + vrow
+  const int vx = VP == 16 ? vrow & 7 : (vrow >> 1) & 3;
+  // Two tiles are under way: the keys of tile it + 2 are asked for as soon as those of tile `it` are used,
+  // its values behind tile it's values.
+  constexpr int STEP = kDecodeWaves * kDecodeKeys;
+  int u0 = u_begin + w * kDecodeKeys;
+  if (u0 < u_end) {
+    const int slot = places(u0);
+    bring_keys(slot, 0);
+    bring_values(slot, 0);
+  }
+  if (u0 + STEP < u_end) {
+    const int slot = places(u0 + STEP);
+    bring_keys(slot, 1);
+    bring_values(slot, 1);
+  }
+  for (int buf = 0; u0 < u_end; u0 += STEP, buf ^= 1) {
+    const bool ahead = u0 + 2 * STEP < u_end;
+    const int slot = ahead ? places(u0 + 2 * STEP) : 0;
+    if (u0 + STEP < u_end)
+      kv_dma_landed<KI + 2 * VI>();
+    else
+      kv_dma_landed<0>();
+    const unsigned char* k_lds = mine + buf * STAGE;
+    const unsigned char* v_lds = k_lds + KTILE;
+    f32x4 st[2];
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+      st[kh] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < DB; ++ks) {
+        const u32x4 ka = *reinterpret_cast<const u32x4*>(k_lds + (16 * kh + c) * KB + 16 * ((4 * ks + g) ^ kx));
+        st[kh] = M::run(ka, qf[ks], st[kh]);
+      }
+    }
+    if (ahead) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the keys are read
+      bring_keys(slot, buf);
+    }
+    float mt = -INFINITY;
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v = st[kh][e] * scale2;
+        if (a.softcap > 0.f) v = cap_score_fast(st[kh][e] * a.scale, cap2, cap_arg);
+        st[kh][e] = u0 + 16 * kh + 4 * g + e < u_end ? v : -INFINITY;
+        mt = fmaxf(mt, st[kh][e]);
+      }
+    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    const float m_new = fmaxf(m, mt);
+    const float shift = m_new == -INFINITY ? 0.f : m_new;
+    const float corr = __builtin_amdgcn_exp2f(m - shift);
+    u32x4 hi, low;
+    float psum = 0.f;
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int e2 = 0; e2 < 2; ++e2) {
+        uint32_t hb[2], lb[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float pv = __builtin_amdgcn_exp2f(st[kh][2 * e2 + e] - shift);
+          psum += pv;
+          hb[e] = bits16<S>(pv);
+          lb[e] = bits16<S>(pv - from_bits16<S>(hb[e]));
+        }
+        hi[2 * kh + e2] = hb[0] | (hb[1] << 16);
+        low[2 * kh + e2] = lb[0] | (lb[1] << 16);
+      }
+    l = l * corr + psum;
+    if (__any(m_new != m)) {
+#pragma unroll
+      for (int n = 0; n < 2 * VB; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[n][e] *= corr;
+    }
+    m = m_new;
+    if (ahead)
+      kv_dma_landed<2 * KI + VI>();
+    else
+      kv_dma_landed<0>();
+#pragma unroll
+    for (int n = 0; n < 2 * VB; ++n) {
+      const unsigned char* at = v_lds + vrow * VBYTES + 32 * (n ^ vx) + 8 * (c & 3);
+      // 16 rows further on the exchange is the same
+      const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)at);
+      const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 16 * VBYTES));
+      const u32x2 x0 = __builtin_bit_cast(u32x2, v0), x1 = __builtin_bit_cast(u32x2, v1);
+      const u32x4 va = {x0[0], x0[1], x1[0], x1[1]};
+      o[n] = M::run(va, hi, o[n]);
+      o[n] = M::run(va, low, o[n]);
+    }
+    if (ahead) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // and the values
+      bring_values(slot, buf);
+    }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  // merge the waves through LDS (the tiles are done with): [wave][head][2 + VD]
+  __syncthreads();
+  float* merge = reinterpret_cast<float*>(smem);
+  if (live) {
+    float* to = merge + (w * kDecodeHeads + c) * (2 + VD);
+    if (g == 0) {
+      to[0] = m;
+      to[1] = l;
+    }
+#pragma unroll
+    for (int n = 0; n < 2 * VB; ++n)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) to[2 + 16 * n + 4 * g + e] = o[n][e];
+  }
+  __syncthreads();
+  auto merged = [&](int hh, int d, float& mm, float& ll) {
+    mm = -INFINITY;
+#pragma unroll
+    for (int ww = 0; ww < kDecodeWaves; ++ww) mm = fmaxf(mm, merge[(ww * kDecodeHeads + hh) * (2 + VD)]);
+    float ov = 0.f;
+    ll = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < kDecodeWaves; ++ww) {
+      const float* src = merge + (ww * kDecodeHeads + hh) * (2 + VD);
+      const float f = src[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(src[0] - mm);
+      ll += src[1] * f;
+      ov += src[2 + d] * f;
+    }
+    return ov;
+  };
+  for (int i = tid; i < group * VD; i += 64 * kDecodeWaves) {
+    const int hh = i / VD, d = i - hh * VD;
+    float mm, ll;
+    const float ov = merged(hh, d, mm, ll);
+    if (a.splits > 1) {
+      float* to = a.parts + (((int64_t)split * a.num_tokens + t) * a.heads + h0 + hh) * (2 + VD);
+      to[2 + d] = ov;
+      if (d == 0) {
+        to[0] = mm;
+        to[1] = ll;
+      }
+    } else {
+      const float other = a.out_inv_freq != nullptr ? merged(hh, pair_of(a, d, VD), mm, ll) / ll : 0.f;
+      finish_decode<S>(a, t, h0 + hh, d, VD, ov / ll, other);
+    }
+  }
+}
+
+template <class S, int VB>
+__global__ __launch_bounds__(32 * VB) void kv_decode_merge_kernel(KvDecode a) {
+  constexpr int VD = 32 * VB;
+  const int64_t t = blockIdx.x;
+  const int h = blockIdx.y, d = threadIdx.x;
+  const int64_t step = (int64_t)a.num_tokens * a.heads * (2 + VD);
+  const float* src = a.parts + (t * a.heads + h) * (2 + VD);
+  float mm = -INFINITY;
+  for (int s = 0; s < a.splits; ++s) mm = fmaxf(mm, src[s * step]);
+  float ll = 0.f, val = 0.f, ov = 0.f;
+  const int other = pair_of(a, d, VD);
+#pragma unroll 4
+  for (int s = 0; s < a.splits; ++s) {
+    const float f = src[s * step] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(src[s * step] - mm);
+    ll += src[s * step + 1] * f;
+    val += src[s * step + 2 + d] * f;
+    if (a.out_inv_freq != nullptr) ov += src[s * step + 2 + other] * f;
+  }
+  finish_decode<S>(a, t, h, d, VD, val / ll, ov / ll);
+}
+
+// Workgroups that a row's keys are shared out to: as many as bring the launch to one per CU, none with fewer
+// than kDecodeMinSplitKeys keys.  max_keys 0 (unknown): one.
+int decode_splits(int num_tokens, int kv_heads, int max_keys) {
+  const int64_t groups = (int64_t)num_tokens * kv_heads;
+  if (groups >= 256 || max_keys <= 0) return 1;
+  return (int)std::max<int64_t>(1, std::min<int64_t>((256 + groups - 1) / groups, max_keys / kDecodeMinSplitKeys));
+}
+
+bool decode_sizes(int dim, int vdim, int heads, int kv_heads) {
+  return (dim == 64 || dim == 128) && (vdim == 64 || vdim == 128) && heads / kv_heads <= kDecodeHeads;
+}
+
+template <class S, int DB, int VB, bool NT>
+int launch_decode_one(const KvDecode& a, hipStream_t stream) {
+  const size_t tiles = (size_t)kDecodeWaves * 2 * kDecodeKeys * 64 * (DB + VB);
+  const size_t merge = (size_t)kDecodeWaves * kDecodeHeads * (2 + 32 * VB) * sizeof(float);
+  const size_t lds = std::max(tiles + a.table_slots * sizeof(int), merge);
+  static std::atomic<size_t> allowed{64 * 1024};   // raised once per kernel, not per launch
+  if (lds > allowed.load(std::memory_order_relaxed)) {
+    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&kv_decode_kernel<S, DB, VB, NT>),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    allowed.store(160 * 1024, std::memory_order_relaxed);
+  }
+  kv_decode_kernel<S, DB, VB, NT><<<dim3(a.num_tokens, a.kv_heads, a.splits), 64 * kDecodeWaves, lds, stream>>>(a);
+  VLA_SEQ_HIP_CHECK(hipGetLastError());
+  if (a.splits > 1) {
+    kv_decode_merge_kernel<S, VB><<<dim3(a.num_tokens, a.heads), 32 * VB, 0, stream>>>(a);
+    VLA_SEQ_HIP_CHECK(hipGetLastError());
+  }
+  return VLA_OK;
+}
+
+// keys and values of a launch that Infinity Cache (256 MiB) cannot hold are read past it
+template <class S, int DB, int VB>
+int launch_decode(const KvDecode& a, int max_keys, hipStream_t stream) {
+  const int64_t bytes = (int64_t)a.num_tokens * max_keys * a.kv_heads * 64 * (DB + VB);
+  return bytes > ((int64_t)256 << 20) ? launch_decode_one<S, DB, VB, true>(a, stream)
+                                      : launch_decode_one<S, DB, VB, false>(a, stream);
+}
+
 template <class S, int DB, int VB>
 int launch_heads_one(dim3 grid, hipStream_t stream, typename S::T* out, int64_t out_stride,
                      const typename S::T* q, int64_t q_stride, const typename S::T* gate,
@@ -1044,7 +1443,10 @@ extern "C" int vla_seq_rotary_kv_write(void* q, int64_t q_stride, const void* k,
   });
 }
 
-extern "C" int vla_seq_kv_attention(void* out, int64_t out_stride, const void* q, int64_t q_stride,
+namespace {
+
+// scratch null: one workgroup per row and KV head, whatever max_keys says
+int kv_attention(void* out, int64_t out_stride, const void* q, int64_t q_stride,
                                     const void* gate, int64_t gate_stride, const void* key_cache,
                                     const void* value_cache, const int* block_tables,
                                     int max_blocks, const int* token_seq, const int64_t* positions,
@@ -1052,7 +1454,7 @@ extern "C" int vla_seq_kv_attention(void* out, int64_t out_stride, const void* q
                                     int heads, int kv_heads, int dim, int vdim, int block_size,
                                     int num_blocks, int window, float scale, int dtype,
                                     int keep_first, float softcap, int chunk, const float* sinks,
-                                    void* stream) {
+                                    int max_keys, float* scratch, int64_t scratch_floats, void* stream) {
   if (num_tokens == 0) return VLA_OK;
   if (!out || !q || !key_cache || !value_cache || !block_tables || !token_seq || !positions ||
       num_tokens < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || block_size <= 0 ||
@@ -1070,6 +1472,50 @@ extern "C" int vla_seq_kv_attention(void* out, int64_t out_stride, const void* q
       if (g_kv_kernel.load(std::memory_order_relaxed) == 0 && mfma_sizes(dim, vdim, out_inv_freq != nullptr) &&
           ((uintptr_t)q % 8) == 0 && ((q_stride * 2) % 8) == 0 && ((uintptr_t)key_cache % 8) == 0 &&
           ((uintptr_t)value_cache % 8) == 0) {
+        const int splits = scratch ? decode_splits(num_tokens, kv_heads, max_keys) : 1;
+        // blocks of a share, and of the kept keys, that the kernel has to keep in LDS: 160 KB less its tiles
+        const int64_t slots = (max_blocks + splits - 1) / splits + kDecodeKeys / block_size + 3 + keep_first / block_size + 1;
+        const size_t tiles = (size_t)kDecodeWaves * 2 * kDecodeKeys * 2 * (dim + vdim);
+        if (decode_sizes(dim, vdim, heads, kv_heads) && tiles + slots * 4 <= 160 * 1024 &&
+            (uint64_t)num_blocks * block_size < ((uint64_t)1 << 31) && (uint64_t)kv_heads * std::max(dim, vdim) * 2 < ((uint64_t)1 << 32) &&
+            num_tokens <= 0x7fffffff && kv_heads <= 65535 && heads <= 65535 && (uintptr_t)q % 16 == 0 && q_stride % 8 == 0 &&
+            (uintptr_t)key_cache % 16 == 0 && (uintptr_t)value_cache % 16 == 0) {
+          if (splits > 1 && scratch_floats < (int64_t)splits * num_tokens * heads * (2 + vdim)) return (int)VLA_ERR_ARG;
+          KvDecode a;
+          a.out = out;
+          a.out_stride = out_stride;
+          a.q = q;
+          a.q_stride = q_stride;
+          a.gate = gate;
+          a.gate_stride = gate_stride;
+          a.key_cache = key_cache;
+          a.value_cache = value_cache;
+          a.block_tables = block_tables;
+          a.max_blocks = max_blocks;
+          a.token_seq = token_seq;
+          a.positions = positions;
+          a.out_inv_freq = out_inv_freq;
+          a.sinks = sinks;
+          a.parts = scratch;
+          a.interleaved = interleaved;
+          a.num_tokens = num_tokens;
+          a.heads = heads;
+          a.kv_heads = kv_heads;
+          a.block_size = block_size;
+          a.num_blocks = num_blocks;
+          a.window = window;
+          a.keep_first = keep_first;
+          a.chunk = chunk;
+          a.v_row = vdim;
+          a.v_first = 0;
+          a.splits = splits;
+          a.table_slots = (int)slots;
+          a.scale = scale;
+          a.softcap = softcap;
+          if (dim == 128)
+            return vdim == 128 ? launch_decode<S, 4, 4>(a, max_keys, (hipStream_t)stream) : launch_decode<S, 4, 2>(a, max_keys, (hipStream_t)stream);
+          return vdim == 128 ? launch_decode<S, 2, 4>(a, max_keys, (hipStream_t)stream) : launch_decode<S, 2, 2>(a, max_keys, (hipStream_t)stream);
+        }
         const int group = heads / kv_heads;
         const dim3 grid(num_tokens, kv_heads * ((group + 31) / 32));
         const int rc = by_value_slices(vdim, [&](int vb, int v_first) {
@@ -1097,6 +1543,45 @@ extern "C" int vla_seq_kv_attention(void* out, int64_t out_stride, const void* q
     VLA_SEQ_HIP_CHECK(hipGetLastError());
     return VLA_OK;
   });
+}
+
+}  // namespace
+
+extern "C" int vla_seq_kv_attention(void* out, int64_t out_stride, const void* q, int64_t q_stride,
+                                    const void* gate, int64_t gate_stride, const void* key_cache,
+                                    const void* value_cache, const int* block_tables,
+                                    int max_blocks, const int* token_seq, const int64_t* positions,
+                                    const float* out_inv_freq, int interleaved, int num_tokens,
+                                    int heads, int kv_heads, int dim, int vdim, int block_size,
+                                    int num_blocks, int window, float scale, int dtype,
+                                    int keep_first, float softcap, int chunk, const float* sinks,
+                                    void* stream) {
+  return kv_attention(out, out_stride, q, q_stride, gate, gate_stride, key_cache, value_cache, block_tables, max_blocks, token_seq,
+                      positions, out_inv_freq, interleaved, num_tokens, heads, kv_heads, dim, vdim, block_size, num_blocks, window,
+                      scale, dtype, keep_first, softcap, chunk, sinks, 0, nullptr, 0, stream);
+}
+
+extern "C" int64_t vla_seq_kv_attention_scratch_floats(int num_tokens, int heads, int kv_heads, int dim, int vdim,
+                                                       int max_keys, int dtype) {
+  if ((dtype != VLA_F16 && dtype != VLA_BF16) || heads <= 0 || kv_heads <= 0 || heads % kv_heads ||
+      !decode_sizes(dim, vdim, heads, kv_heads))
+    return 0;
+  const int splits = decode_splits(num_tokens, kv_heads, max_keys);
+  return splits > 1 ? (int64_t)splits * num_tokens * heads * (2 + vdim) : 0;
+}
+
+extern "C" int vla_seq_kv_attention_shared(void* out, int64_t out_stride, const void* q, int64_t q_stride,
+                                    const void* gate, int64_t gate_stride, const void* key_cache,
+                                    const void* value_cache, const int* block_tables,
+                                    int max_blocks, const int* token_seq, const int64_t* positions,
+                                    const float* out_inv_freq, int interleaved, int num_tokens,
+                                    int heads, int kv_heads, int dim, int vdim, int block_size,
+                                    int num_blocks, int window, float scale, int dtype,
+                                    int keep_first, float softcap, int chunk, const float* sinks,
+                                    int max_keys, float* scratch, int64_t scratch_floats, void* stream) {
+  return kv_attention(out, out_stride, q, q_stride, gate, gate_stride, key_cache, value_cache, block_tables, max_blocks, token_seq,
+                      positions, out_inv_freq, interleaved, num_tokens, heads, kv_heads, dim, vdim, block_size, num_blocks, window,
+                      scale, dtype, keep_first, softcap, chunk, sinks, max_keys, scratch, scratch_floats, stream);
 }
 
 // 0: pick per shape; 1: always the one-wave-per-(row, head) kernel (tests run both)
