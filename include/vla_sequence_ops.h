@@ -328,9 +328,22 @@ int vla_seq_grouped_linear(void* out, int64_t out_stride, int out_dtype, const v
                            int64_t a_stride, const int* row_token, const void* weight,
                            const int* tile_expert, int max_tiles, int n_out, int k_in, int act,
                            const float* row_scale, int dtype, void* stream);
+/* The same, told how many experts there are (vla_seq_grouped_linear launches for as many as tiles). */
+int vla_seq_grouped_linear_of(void* out, int64_t out_stride, int out_dtype, const void* a,
+                           int64_t a_stride, const int* row_token, const void* weight,
+                           const int* tile_expert, int max_tiles, int n_out, int k_in, int act,
+                           const float* row_scale, int dtype, int num_experts, void* stream);
+/* The gated first product in one launch (16-bit types, k_in a multiple of 64): weight [experts, 2 n_out, k_in],
+ * W_gate's rows ahead of W_up's; out[row] = act(g) * u, or (clamped) g sigmoid(alpha g) (u + shift) with
+ * g = min(g, limit), u = clamp(u, -limit, limit), of the fp32 sums g, u times row_scale[row]. */
+int vla_seq_grouped_glu_supported(int k_in, int dtype);
+int vla_seq_grouped_glu(void* out, int64_t out_stride, const void* a, int64_t a_stride, const int* row_token,
+                        const void* weight, const int* tile_expert, int max_tiles, int n_out, int k_in,
+                        int act, int clamped, float limit, float alpha, float shift, const float* row_scale,
+                        int dtype, int num_experts, void* stream);
 
 /* Form of the 16-bit product for tests: 0 = per shape, 1 = one-wave workgroups (decode steps),
- * 2 = runs of tiles per workgroup (prompts). */
+ * 2 = runs of tiles per workgroup (prompts), 3 and 4 = the LDS-DMA forms for few and for many rows. */
 int vla_seq_set_grouped_linear_form(int mode);
 
 /* out[t] (fp32 [T, width]) = sum_k weights[t, k] * (y[pair_row[t, k]] or, where pair_row is -1,

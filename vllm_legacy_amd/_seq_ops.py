@@ -618,14 +618,45 @@ def grouped_linear(out: torch.Tensor, a: torch.Tensor, row_token: Optional[torch
         assert a.shape[0] == out.shape[0]
     assert row_scale is None or (row_scale.dtype == torch.float32 and row_scale.numel() == out.shape[0])
     with torch.cuda.device(a.device):
-        seq_check(L.vla_seq_grouped_linear(
+        seq_check(L.vla_seq_grouped_linear_of(
             out.data_ptr(), N, _dt(out.dtype), a.data_ptr(), _rows(a, K), _p(row_token), weight.data_ptr(),
-            tile_expert.data_ptr(), tiles, N, K, ACT[act], _p(row_scale), _dt(a.dtype), _stream(a.device)),
+            tile_expert.data_ptr(), tiles, N, K, ACT[act], _p(row_scale), _dt(a.dtype), E, _stream(a.device)),
             "grouped_linear")
 
 
+def grouped_glu_supported(a: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether grouped_glu takes these rows and weights."""
+    return bool(_lib.seq_lib().vla_seq_grouped_glu_supported(weight.shape[2], _dt(a.dtype))) and a.data_ptr() % 16 == 0 and \
+        (a.stride(0) % 8 == 0 or a.shape[0] == 1) and weight.data_ptr() % 16 == 0
+
+
+def grouped_glu(out: torch.Tensor, a: torch.Tensor, row_token: Optional[torch.Tensor], weight: torch.Tensor,
+                tile_expert: torch.Tensor, act: str, row_scale: Optional[torch.Tensor] = None, limit: float = 0.0,
+                alpha: float = 0.0, shift: float = 0.0) -> None:
+    """out [tiles * tile rows, F] = act(g) * u, g and u the first and second F sums of weight[e] a[src(row)] times
+    row_scale[row] in fp32; weight [E, 2 F, K]; act "clamped_glu": the clamped form with limit, alpha, shift."""
+    _gpu(out, a, row_token, weight, tile_expert, row_scale)
+    E, N, K = weight.shape
+    F = N // 2
+    assert N % 2 == 0 and weight.is_contiguous() and weight.dtype == a.dtype == out.dtype and a.shape[1] == K
+    L = _lib.seq_lib()
+    tiles = tile_expert.numel()
+    assert out.shape == (tiles * L.vla_seq_moe_tile_rows(), F) and out.is_contiguous()
+    assert row_token is None or (row_token.dtype == torch.int32 and row_token.numel() == out.shape[0])
+    if row_token is None:
+        assert a.shape[0] == out.shape[0]
+    assert row_scale is None or (row_scale.dtype == torch.float32 and row_scale.numel() == out.shape[0])
+    clamped = act == "clamped_glu"
+    with torch.cuda.device(a.device):
+        seq_check(L.vla_seq_grouped_glu(
+            out.data_ptr(), F, a.data_ptr(), a.stride(0) if a.shape[0] > 1 else K, _p(row_token), weight.data_ptr(),
+            tile_expert.data_ptr(), tiles, F, K, 0 if clamped else ACT[act], int(clamped), float(limit), float(alpha),
+            float(shift), _p(row_scale), _dt(a.dtype), E, _stream(a.device)), "grouped_glu")
+
+
 def set_grouped_linear_form(mode: int) -> None:
-    """0: grouped_linear picks its 16-bit form per shape; 1: one-wave workgroups; 2: runs of tiles."""
+    """0: grouped_linear picks its 16-bit form per shape; 1: one-wave workgroups; 2: runs of tiles; 3, 4: the
+    LDS-DMA forms for few and for many rows."""
     seq_check(_lib.seq_lib().vla_seq_set_grouped_linear_form(mode), "set_grouped_linear_form")
 
 

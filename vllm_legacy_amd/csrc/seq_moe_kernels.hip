@@ -11,6 +11,7 @@
 //   moe_combine    per token: weighted sum of its experts' rows (a choice without a row is an
 //                  identity expert: the token's own input), plus the gated shared expert
 // A row's result does not depend on which other rows share its tile or on where the plan put it.
+#include <algorithm>
 #include <atomic>
 
 #include "seq_common.h"
@@ -391,116 +392,383 @@ __global__ __launch_bounds__(256) void grouped_linear_mfma16_kernel(
   }
 }
 
-// The form for many tiles and k_in a multiple of 64: the activation rows of a run of tiles (up to
-// 128 rows) walk through LDS in chunks of 64 values, staged once for the four waves of the
-// workgroup (double-buffered, one barrier per chunk, loaded one chunk ahead); a wave's weight
-// fragments still come straight from memory (no other wave wants them), one 16-byte load per 16
-// values and 32 columns, used for every tile of the run.
-constexpr int kChunk = 64;
-constexpr int kARow = kChunk + 8;     // elements: 144-byte rows, 16 lanes' 16-byte reads fall into different banks
+// ---------------------------------------------------------------------------------------------
+// The forms for k_in a multiple of 64 with both operands brought in by LDS-DMA.  GLU: the weight's rows are
+// [gate (n_out) | up (n_out)] and the output is act(gate) * up (or the clamped form): a lane ends with both
+// sums of an element, so the pair never leaves the registers as 16-bit numbers.
+struct GroupedDma {
+  void* out;
+  int64_t out_stride;
+  const void* a;
+  int64_t a_stride;
+  const int* row_token;
+  const void* weight;
+  const int* tile_expert;
+  const float* row_scale;
+  int max_tiles, n_out, k_in, act;
+  float limit, alpha, shift;        // the clamped form's, act == kActClamped
+  int col_tiles;
+  int64_t groups;                   // workgroups along the rows
+};
+constexpr int kActClamped = 100;
+constexpr int kStep = 64;           // contraction values of a stage: rows of 128 bytes
+constexpr int kRunRows = 4;         // row tiles of a run, at most (a power of two)
 
-template <class S, class SO, int C>
-__device__ __forceinline__ void grouped_run_lds(typename S::T* __restrict__ a_lds,
-                                                typename SO::T* __restrict__ out, int64_t out_stride,
-                                                const typename S::T* __restrict__ a, int64_t a_stride,
-                                                const int* __restrict__ row_token,
-                                                const typename S::T* __restrict__ wr, int first_tile, int n0,
-                                                int n_out, int k_in, int act,
-                                            const float* __restrict__ row_scale, int hf, int c) {
-  using T = typename S::T;
-  const int tid = threadIdx.x;
-  // staging: C pieces of 16 bytes per thread and chunk; piece p = tid + 256 u is row p / 8, values 8 (p % 8) ..
-  const T* src[C];
-#pragma unroll
-  for (int u = 0; u < C; ++u) {
-    const int p = tid + 256 * u;
-    const int row = first_tile * kTile + p / 8;
-    const int tok = row_token != nullptr ? row_token[row] : row;
-    src[u] = tok < 0 ? nullptr : a + (int64_t)tok * a_stride + 8 * (p % 8);
+__device__ __forceinline__ float glu_apply(float g, float u, const GroupedDma& a) {
+  if (a.act == kActClamped) {
+    const float gc = fminf(g, a.limit), uc = fminf(fmaxf(u, -a.limit), a.limit);
+    return gc / (1.f + expf(-a.alpha * gc)) * (uc + a.shift);
   }
-  u32x4 xa[C];
-  auto fetch = [&](int ch) {
+  return act_apply(g, a.act) * u;
+}
+
+// 16 bytes per lane from each lane's own address into 1 KB of LDS (no register result)
+__device__ __forceinline__ void moe_dma16(const void* src, uint32_t lds_at) {
+  unsigned keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(src), "s"(lds_at)
+      : "memory");
+}
+
+// Where a column tile of the few-rows form starts in the contraction.  Rows are a power of two apart in most
+// models (2048 values: 4096 bytes), so workgroups in step would ask the same few memory channels; neighbouring
+// column tiles start three stages apart (64 tokens, two of 16 experts of 2 x 1408 x 2048: 45.6 -> 41.7 us).  A
+// row's result still depends on nothing but its column.
+__device__ __forceinline__ int first_step(int col, int steps) { return (int)((unsigned)col * 3u % (unsigned)steps); }
+
+// four neighbouring values of a row of the result
+template <class SO>
+__device__ __forceinline__ void store4(typename SO::T* to, const float (&v)[4], int n, int n_out, bool vec) {
+  if (vec && n + 3 < n_out) {
+    if constexpr (sizeof(typename SO::T) == 2)
+      *reinterpret_cast<u32x2*>(to) = u32x2{pack16<SO>(v[0], v[1]), pack16<SO>(v[2], v[3])};
+    else
+      *reinterpret_cast<f32x4*>(to) = f32x4{v[0], v[1], v[2], v[3]};
+  } else {
 #pragma unroll
-    for (int u = 0; u < C; ++u)
-      xa[u] = src[u] != nullptr ? *reinterpret_cast<const u32x4*>(src[u] + ch * kChunk) : u32x4{0u, 0u, 0u, 0u};
-  };
-  auto land = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < C; ++u) {
-      const int p = tid + 256 * u;
-      *reinterpret_cast<u32x4*>(a_lds + (size_t)buf * 4 * kTile * kARow + (p / 8) * kARow + 8 * (p % 8)) = xa[u];
-    }
-  };
-  f32x16 acc[C];
-#pragma unroll
-  for (int r = 0; r < C; ++r)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[r][i] = 0.f;
-  const int chunks = k_in / kChunk;
-  fetch(0);
-  land(0);
-  if (chunks > 1) fetch(1);
-  __syncthreads();
-  for (int ch = 0; ch < chunks; ++ch) {
-    const T* tile = a_lds + (size_t)(ch & 1) * 4 * kTile * kARow + c * kARow + 8 * hf;
-    u32x4 wv[kChunk / 16];
-#pragma unroll
-    for (int ks = 0; ks < kChunk / 16; ++ks) wv[ks] = *reinterpret_cast<const u32x4*>(wr + ch * kChunk + 16 * ks);
-#pragma unroll
-    for (int ks = 0; ks < kChunk / 16; ++ks)
-#pragma unroll
-      for (int r = 0; r < C; ++r) {
-        const u32x4 av = *reinterpret_cast<const u32x4*>(tile + r * kTile * kARow + 16 * ks);
-        acc[r] = Mma16<S>::run(wv[ks], av, acc[r]);
-      }
-    if (ch + 1 < chunks) land((ch + 1) & 1);
-    if (ch + 2 < chunks) fetch(ch + 2);
-    __syncthreads();
-  }
-  if (n0 >= n_out) return;
-#pragma unroll
-  for (int r = 0; r < C; ++r) {
-    const int row = (first_tile + r) * kTile + c;
-    // a padding row's sums are zeros and its scale was never written
-    const float sc = row_scale != nullptr && (row_token == nullptr || row_token[row] >= 0) ? row_scale[row] : 1.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int n = n0 + (i & 3) + 8 * (i >> 2) + 4 * hf;
-      if (n < n_out) out[(int64_t)row * out_stride + n] = SO::from_f32(act_apply(acc[r][i] * sc, act));
-    }
+    for (int e = 0; e < 4; ++e)
+      if (n + e < n_out) to[e] = SO::from_f32(v[e]);
   }
 }
 
-template <class S, class SO>
-__global__ __launch_bounds__(256) void grouped_linear_lds_kernel(
-    typename SO::T* __restrict__ out, int64_t out_stride, const typename S::T* __restrict__ a,
-    int64_t a_stride, const int* __restrict__ row_token, const typename S::T* __restrict__ weight,
-    const int* __restrict__ tile_expert, int max_tiles, int n_out, int k_in, int act,
-    const float* __restrict__ row_scale) {
-  __shared__ __align__(16) typename S::T a_lds[2 * 4 * kTile * kARow];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int hf = lane >> 5, c = lane & 31;
-  const int n0 = blockIdx.y * 128 + w * 32;        // waves past the last column still stage and wait
-  const int first = blockIdx.x * kRunTiles;
-  const int last = min(first + kRunTiles, max_tiles);
-  int i = first;
-  while (i < last) {
-    const int e = tile_expert[i];
-    if (e < 0) {
-      ++i;
-      continue;
+// The run of at most kRunRows row tiles of one expert that is number `want` among all such runs: (first tile,
+// count), count 0 behind the last.  An expert's tiles are neighbours, so runs start at every kRunRows-th
+// tile from an expert's first one; every wave scans the tiles' experts for itself.
+__device__ __forceinline__ int2 find_run(const int* __restrict__ tile_expert, int max_tiles, int want) {
+  const int lane = threadIdx.x & 63;
+  int seen = 0, first = 0;                                 // runs before this stretch of 64; its expert's first tile
+  for (int i0 = 0; i0 < max_tiles; i0 += kWave) {
+    const int i = i0 + lane;
+    const int e = i < max_tiles ? tile_expert[i] : -1, before = i > 0 && i < max_tiles ? tile_expert[i - 1] : -1;
+    const uint64_t edges = __ballot(e != before || i == 0);
+    const uint64_t upto = edges & (~0ull >> (63 - lane));
+    const int f = upto ? i0 + 63 - __builtin_clzll(upto) : first;
+    const uint64_t starts = __ballot(e >= 0 && ((i - f) & (kRunRows - 1)) == 0);
+    const int n = __builtin_popcountll(starts);
+    if (want < seen + n) {
+      uint64_t left = starts;
+      for (int k = want - seen; k > 0; --k) left &= left - 1;
+      const int at = __builtin_ctzll(left);
+      const int tile = i0 + at, mine = tile_expert[tile];
+      int count = 1;
+      while (count < kRunRows && tile + count < max_tiles && tile_expert[tile + count] == mine) ++count;
+      return make_int2(tile, count);
     }
-    int j = i + 1;
-    while (j < last && tile_expert[j] == e) ++j;
-    const typename S::T* wr = weight + ((int64_t)e * n_out + min(n0 + c, n_out - 1)) * k_in + 8 * hf;
-    switch (j - i) {
-      case 1: grouped_run_lds<S, SO, 1>(a_lds, out, out_stride, a, a_stride, row_token, wr, i, n0, n_out, k_in, act, row_scale, hf, c); break;
-      case 2: grouped_run_lds<S, SO, 2>(a_lds, out, out_stride, a, a_stride, row_token, wr, i, n0, n_out, k_in, act, row_scale, hf, c); break;
-      case 3: grouped_run_lds<S, SO, 3>(a_lds, out, out_stride, a, a_stride, row_token, wr, i, n0, n_out, k_in, act, row_scale, hf, c); break;
-      default: grouped_run_lds<S, SO, 4>(a_lds, out, out_stride, a, a_stride, row_token, wr, i, n0, n_out, k_in, act, row_scale, hf, c); break;
-    }
-    i = j;
+    seen += n;
+    first = edges ? i0 + 63 - __builtin_clzll(edges) : first;
   }
+  return make_int2(0, 0);
+}
+
+// Many rows.  A workgroup is a run of up to 128 rows of one expert by 256 weight rows (GLU: 128 gates and
+// their 128 ups), eight waves of 64 x 64 each; three stages of 48 KB that LDS-DMA fills two steps ahead, one
+// barrier per 64 contraction values, one workgroup per CU.  A stage's row is 128 bytes: its 16-byte pieces
+// are exchanged by the row's number (on the source's side, LDS-DMA writes a row in a row), so the 32 lanes
+// of a fragment read meet all banks.  The launch is cut among the 8 XCDs in contiguous stretches
+// (workgroups go to them round robin), and a stretch goes over up to eight column tiles for each run of rows,
+// so that what runs together shares rows and weights in one L2.  4096 rows of 2048, two of 16 experts of
+// 1408: gate | up and activation 184 us (the LDS form with registers on the way 311 and 17), down 113
+// (189).  A step takes 1.3 us where its products need 0.43; a third of the CUs' time is the last round of
+// workgroups.  128 x 128 tiles with two workgroups per CU and two stages take 190 and 110, four waves
+// of 256 x 64 (less LDS traffic, nothing beside a wave on its SIMD) 304 and 206, column tiles that start
+// at different places of the contraction 190 and 117.
+template <class S, class SO, bool GLU>
+__global__ __launch_bounds__(512, 2) void grouped_dma_kernel(GroupedDma a) {
+  constexpr int ROWS = 32 * kRunRows, WROWS = 256, STAGE = (ROWS + WROWS) * 128, RING = 3;
+  extern __shared__ __align__(16) unsigned char smem[];
+  // stretches of XCDs, then (eight column tiles)(rows)(column tile)
+  const int64_t total = a.groups * a.col_tiles, per = (total + 7) / 8;
+  const int64_t id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int64_t)(blockIdx.x >> 3) >= per || id >= total) return;
+  const int64_t wide = a.groups * 8;
+  const int cb = (int)(id / wide);
+  const int width = min(8, a.col_tiles - 8 * cb);
+  const int64_t rest = id - cb * wide;
+  const int col = 8 * cb + (int)(rest % width);
+  const int2 run = find_run(a.tile_expert, a.max_tiles, (int)(rest / width));
+  if (run.y == 0) return;
+  const int e = a.tile_expert[run.x];
+  const int n0 = col * (GLU ? 128 : 256);
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hf = lane >> 5, c = lane & 31, wm = w & 1, wn = w >> 1;
+  const int rows = run.y * kTile;
+
+  // wave w brings 16 rows and 32 weight rows, eight per instruction
+  const unsigned char* src_a[2];
+  const unsigned char* src_w[4];
+  const int64_t weight_rows = (int64_t)(GLU ? 2 : 1) * a.n_out;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int r = 16 * w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
+    const int row = run.x * kTile + min(r, rows - 1);
+    const int src = a.row_token != nullptr ? max(0, a.row_token[row]) : row;     // padding reads token 0
+    src_a[u] = (const unsigned char*)a.a + (int64_t)src * a.a_stride * 2 + 16 * piece;
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int r = 32 * w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
+    const int n = GLU ? (r < 128 ? min(n0 + r, a.n_out - 1) : a.n_out + min(n0 + r - 128, a.n_out - 1)) : min(n0 + r, a.n_out - 1);
+    src_w[u] = (const unsigned char*)a.weight + ((int64_t)e * weight_rows + n) * a.k_in * 2 + 16 * piece;
+  }
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  auto bring = [&](int step, int buf) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) moe_dma16(src_a[u] + step * (2 * kStep), lds0 + buf * STAGE + w * 2048 + 1024 * u);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      moe_dma16(src_w[u] + step * (2 * kStep), lds0 + buf * STAGE + ROWS * 128 + w * 4096 + 1024 * u);
+  };
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
+  const int x = hf ^ ((c >> 1) & 7);                       // piece 2 ks + hf stands at (2 ks) ^ x
+  const bool active = 64 * wm < rows;
+  const int steps = a.k_in / kStep;
+  bring(0, 0);
+  if (steps > 1) bring(1, 1);
+  int buf = 0;
+  for (int it = 0; it < steps; ++it) {
+    if (it + 1 < steps)
+      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");      // all but the next stage
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (it + 2 < steps) bring(it + 2, buf >= 1 ? buf - 1 : RING - 1);
+    const unsigned char* stage = smem + buf * STAGE;
+    buf = buf + 1 < RING ? buf + 1 : 0;
+    if (!active) continue;
+    const unsigned char* a_lds = stage + (64 * wm + c) * 128;
+    const unsigned char* w_lds = stage + ROWS * 128 + ((GLU ? 32 : 64) * wn + c) * 128;
+#pragma unroll
+    for (int ks = 0; ks < kStep / 16; ++ks) {
+      u32x4 av[2], wv[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        av[b] = *reinterpret_cast<const u32x4*>(a_lds + b * 32 * 128 + 16 * ((2 * ks) ^ x));
+        wv[b] = *reinterpret_cast<const u32x4*>(w_lds + b * (GLU ? 128 : 32) * 128 + 16 * ((2 * ks) ^ x));
+      }
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = Mma16<S>::run(wv[nb], av[mb], acc[mb][nb]);
+    }
+  }
+  const bool vec = a.out_stride % 4 == 0 && (uintptr_t)a.out % 16 == 0;
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb) {
+    const int r = 64 * wm + 32 * mb + c;
+    if (r >= rows) continue;
+    const int row = run.x * kTile + r;
+    const bool live = a.row_token == nullptr || a.row_token[row] >= 0;
+    // a padding row leaves what zeros would; its scale was never written
+    const float sc = live ? (a.row_scale != nullptr ? a.row_scale[row] : 1.f) : 0.f;
+    typename SO::T* to = (typename SO::T*)a.out + (int64_t)row * a.out_stride;
+#pragma unroll
+    for (int nb = 0; nb < (GLU ? 1 : 2); ++nb)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const int n = n0 + (GLU ? 32 * wn : 64 * wn + 32 * nb) + 8 * i4 + 4 * hf;
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float z = live ? acc[mb][nb][4 * i4 + k] * sc : 0.f;
+          if constexpr (GLU)
+            v[k] = glu_apply(z, live ? acc[mb][1][4 * i4 + k] * sc : 0.f, a);
+          else
+            v[k] = act_apply(z, a.act);
+        }
+        store4<SO>(to + n, v, n, a.n_out, vec);
+      }
+  }
+}
+
+// Few rows (decode steps): bound by reading every chosen expert's weights once.  A workgroup is one row tile
+// by 64 weight rows (GLU: 32 gates and their 32 ups); its four waves take every fourth step of 64
+// contraction values, each through its own ring of three stages of 12 KB that LDS-DMA fills two steps
+// ahead (96 KB on their way per CU, no barrier), and add their sums at the end.  A stage row is 128
+// neighbouring bytes of one weight row; the one-wave form's fragment reads meet 32 rows with 32 bytes
+// each.  64 tokens, two of 16 experts of 1408, width 2048: gate | up and activation 42 us = 4.4 TB/s of
+// weights (one-wave form 61 and 5), down 23 = 4.0 TB/s (39).
+template <class S, class SO, bool GLU>
+__global__ __launch_bounds__(256) void grouped_stream_kernel(GroupedDma a) {
+  constexpr int STAGE = (kTile + 64) * 128, RING = 3;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tile = blockIdx.y;
+  const int e = a.tile_expert[tile];
+  if (e < 0) return;
+  const int n0 = blockIdx.x * (GLU ? 32 : 64);
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hf = lane >> 5, c = lane & 31;
+  const unsigned char* src_a[4];
+  const unsigned char* src_w[8];
+  const int64_t weight_rows = (int64_t)(GLU ? 2 : 1) * a.n_out;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int r = 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
+    const int n = GLU ? (r < 32 ? min(n0 + r, a.n_out - 1) : a.n_out + min(n0 + r - 32, a.n_out - 1)) : min(n0 + r, a.n_out - 1);
+    src_w[u] = (const unsigned char*)a.weight + ((int64_t)e * weight_rows + n) * a.k_in * 2 + 16 * piece;
+    if (u < 4) {
+      const int row = tile * kTile + r;
+      const int src = a.row_token != nullptr ? max(0, a.row_token[row]) : row;   // padding reads token 0
+      src_a[u] = (const unsigned char*)a.a + (int64_t)src * a.a_stride * 2 + 16 * piece;
+    }
+  }
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)smem + w * RING * STAGE;
+  const unsigned char* mine = smem + w * RING * STAGE;
+  const int steps = a.k_in / kStep, turn = first_step(blockIdx.x, steps);
+  auto bring = [&](int it, int buf) {
+    const int step = it + turn < steps ? it + turn : it + turn - steps;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) moe_dma16(src_a[u] + step * (2 * kStep), lds0 + buf * STAGE + 1024 * u);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) moe_dma16(src_w[u] + step * (2 * kStep), lds0 + buf * STAGE + kTile * 128 + 1024 * u);
+  };
+  f32x16 acc[2];
+#pragma unroll
+  for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[nb][i] = 0.f;
+  const int x = hf ^ ((c >> 1) & 7);
+  if (w < steps) bring(w, 0);
+  if (w + 4 < steps) bring(w + 4, 1);
+  int buf = 0;
+  for (int it = w; it < steps; it += 4) {
+    if (it + 8 < steps) {
+      bring(it + 8, buf >= 1 ? buf - 1 : RING - 1);
+      asm volatile("s_waitcnt vmcnt(24)" ::: "memory");     // all but the two youngest stages
+    } else if (it + 4 < steps) {
+      asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const unsigned char* a_lds = mine + buf * STAGE + c * 128;
+    const unsigned char* w_lds = mine + buf * STAGE + (kTile + c) * 128;
+#pragma unroll
+    for (int ks = 0; ks < kStep / 16; ++ks) {
+      const u32x4 av = *reinterpret_cast<const u32x4*>(a_lds + 16 * ((2 * ks) ^ x));
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+        acc[nb] = Mma16<S>::run(*reinterpret_cast<const u32x4*>(w_lds + nb * 32 * 128 + 16 * ((2 * ks) ^ x)), av, acc[nb]);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the stage is read before it is filled again
+    buf = buf + 1 < RING ? buf + 1 : 0;
+  }
+  // the waves' sums through LDS, [wave][2][4 quads][64 lanes][4]; thread (nb, quad, lane) adds up
+  __syncthreads();
+  float* part = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4)
+      *reinterpret_cast<f32x4*>(part + (((w * 2 + nb) * 4 + i4) * 64 + lane) * 4) =
+          f32x4{acc[nb][4 * i4], acc[nb][4 * i4 + 1], acc[nb][4 * i4 + 2], acc[nb][4 * i4 + 3]};
+  __syncthreads();
+  const int row = tile * kTile + c;
+  const bool live = a.row_token == nullptr || a.row_token[row] >= 0;
+  const float sc = live ? (a.row_scale != nullptr ? a.row_scale[row] : 1.f) : 0.f;
+  const bool vec = a.out_stride % 4 == 0 && (uintptr_t)a.out % 16 == 0;
+  typename SO::T* to = (typename SO::T*)a.out + (int64_t)row * a.out_stride;
+  auto sum = [&](int nb, int i4, float (&v)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = 0.f;
+#pragma unroll
+    for (int ow = 0; ow < 4; ++ow) {
+      const f32x4 p = *reinterpret_cast<const f32x4*>(part + (((ow * 2 + nb) * 4 + i4) * 64 + lane) * 4);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] += p[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = live ? v[k] * sc : 0.f;
+  };
+#pragma unroll
+  for (int nb = 0; nb < (GLU ? 1 : 2); ++nb) {
+    const int n = n0 + 32 * nb + 8 * w + 4 * hf;            // wave w finishes quad w
+    float v[4];
+    sum(nb, w, v);
+    if constexpr (GLU) {
+      float up[4];
+      sum(1, w, up);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = glu_apply(v[k], up[k], a);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = act_apply(v[k], a.act);
+    }
+    store4<SO>(to + n, v, n, a.n_out, vec);
+  }
+}
+
+template <class S, class SO, bool GLU>
+int launch_grouped_dma(GroupedDma a, int num_experts, bool few, hipStream_t stream) {
+  if (few && a.max_tiles <= 65535) {
+    constexpr int lds = 4 * 3 * (kTile + 64) * 128;
+    static std::atomic<bool> raised{false};           // LDS limit: raised once per kernel, not per launch
+    if (!raised.load(std::memory_order_relaxed)) {
+      VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&grouped_stream_kernel<S, SO, GLU>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+      raised.store(true, std::memory_order_relaxed);
+    }
+    const int cols = GLU ? 32 : 64;
+    grouped_stream_kernel<S, SO, GLU><<<dim3((a.n_out + cols - 1) / cols, a.max_tiles), 256, lds, stream>>>(a);
+  } else {
+    constexpr int lds = 3 * (32 * kRunRows + 256) * 128;
+    static std::atomic<bool> raised{false};
+    if (!raised.load(std::memory_order_relaxed)) {
+      VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&grouped_dma_kernel<S, SO, GLU>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+      raised.store(true, std::memory_order_relaxed);
+    }
+    const int cols = GLU ? 128 : 256;
+    a.col_tiles = (a.n_out + cols - 1) / cols;
+    // every expert adds at most one run that is not full
+    a.groups = a.max_tiles / kRunRows + std::min(num_experts, a.max_tiles) + 1;
+    const int64_t total = a.groups * a.col_tiles;
+    grouped_dma_kernel<S, SO, GLU><<<(unsigned)((total + 7) / 8 * 8), 512, lds, stream>>>(a);
+  }
+  VLA_SEQ_HIP_CHECK(hipGetLastError());
+  return VLA_OK;
+}
+
+// Whether a launch is bound by the weights, which in the forms for few rows every tile of 32 rows reads for
+// itself.  The plan leaves room for a tile per expert beside the full ones, so 2.5 tiles per expert are 48
+// rows each (us of the whole block, few / many rows form: 16 experts of 1408 x 2048, top 2: 128 tokens 102 /
+// 107, 256 127 / 149, 384 147 / 151, 512 155 / 154, 1024 215 / 184; 32 experts of 1408 x 4096, top 4: 128
+// 288 / 318, 256 339 / 371, 384 422 / 419, 512 461 / 413).  Without the number of experts: the workgroups
+// of the form for many rows would fill the part.
+bool few_tiles(int max_tiles, int weight_rows, int num_experts) {
+  return num_experts > 0 ? 2 * (int64_t)max_tiles <= 5 * (int64_t)num_experts
+                         : (int64_t)max_tiles * ((weight_rows + 127) / 128) <= 1024;
+}
+
+// 16-byte pieces of both operands, whole steps of the contraction
+bool dma_fits(const void* a, int64_t a_stride, const void* weight, int k_in) {
+  return k_in % kStep == 0 && (uintptr_t)a % 16 == 0 && a_stride % 8 == 0 && (uintptr_t)weight % 16 == 0;
 }
 
 // Any dtype and size, fp32 arithmetic: wave w of a workgroup takes eight rows of the tile, lane =
@@ -620,10 +888,12 @@ extern "C" int vla_seq_moe_plan(const int* experts, int num_tokens, int top, int
   return VLA_OK;
 }
 
-extern "C" int vla_seq_grouped_linear(void* out, int64_t out_stride, int out_dtype, const void* a,
+namespace {
+
+int grouped_linear(void* out, int64_t out_stride, int out_dtype, const void* a,
                                       int64_t a_stride, const int* row_token, const void* weight,
                                       const int* tile_expert, int max_tiles, int n_out, int k_in,
-                                      int act, const float* row_scale, int dtype, void* stream) {
+                                      int act, const float* row_scale, int dtype, int num_experts, void* stream) {
   if (max_tiles == 0) return VLA_OK;
   if (!out || !a || !weight || !tile_expert || max_tiles < 0 || n_out <= 0 || k_in <= 0 ||
       out_stride < n_out || a_stride < k_in || act < VLA_ACT_NONE || act > VLA_ACT_GELU_TANH)
@@ -639,14 +909,12 @@ extern "C" int vla_seq_grouped_linear(void* out, int64_t out_stride, int out_dty
         // every (tile, 32 columns) is a one-wave workgroup of its own; many tiles: four waves
         // and runs of tiles that share the weight fragments
         const int form = g_grouped_form.load(std::memory_order_relaxed);
-        const bool few = form == 0 ? (int64_t)max_tiles * ((n_out + 127) / 128) <= 1024 : form == 1;
-        if (!few && k_in % kChunk == 0) {
-          grouped_linear_lds_kernel<S, SO>
-              <<<dim3((max_tiles + kRunTiles - 1) / kRunTiles, (n_out + 127) / 128), 256, 0, st>>>(
-                  (typename SO::T*)out, out_stride, (const T*)a, a_stride, row_token, (const T*)weight,
-                  tile_expert, max_tiles, n_out, k_in, act, row_scale);
-          VLA_SEQ_HIP_CHECK(hipGetLastError());
-          return VLA_OK;
+        const bool few = form == 0 ? few_tiles(max_tiles, n_out, 0) : form == 1;
+        if (dma_fits(a, a_stride, weight, k_in) && (form == 0 || form == 3 || form == 4)) {
+          GroupedDma d{out, out_stride, a, a_stride, row_token, weight, tile_expert, row_scale, max_tiles, n_out, k_in, act,
+                       0.f, 0.f, 0.f, 0, 0};
+          return launch_grouped_dma<S, SO, false>(d, num_experts > 0 ? num_experts : max_tiles,
+                                                  form == 0 ? few_tiles(max_tiles, n_out, num_experts) : form == 3, st);
         }
         const int waves = few ? 1 : 4, per = few ? 1 : kRunTiles;
         grouped_linear_mfma16_kernel<S, SO>
@@ -672,6 +940,52 @@ extern "C" int vla_seq_grouped_linear(void* out, int64_t out_stride, int out_dty
   });
 }
 
+}  // namespace
+
+extern "C" int vla_seq_grouped_linear(void* out, int64_t out_stride, int out_dtype, const void* a,
+                                      int64_t a_stride, const int* row_token, const void* weight,
+                                      const int* tile_expert, int max_tiles, int n_out, int k_in,
+                                      int act, const float* row_scale, int dtype, void* stream) {
+  return grouped_linear(out, out_stride, out_dtype, a, a_stride, row_token, weight, tile_expert, max_tiles, n_out, k_in,
+                        act, row_scale, dtype, 0, stream);
+}
+
+extern "C" int vla_seq_grouped_linear_of(void* out, int64_t out_stride, int out_dtype, const void* a,
+                                         int64_t a_stride, const int* row_token, const void* weight,
+                                         const int* tile_expert, int max_tiles, int n_out, int k_in,
+                                         int act, const float* row_scale, int dtype, int num_experts, void* stream) {
+  if (num_experts <= 0) return VLA_ERR_ARG;
+  return grouped_linear(out, out_stride, out_dtype, a, a_stride, row_token, weight, tile_expert, max_tiles, n_out, k_in,
+                        act, row_scale, dtype, num_experts, stream);
+}
+
+extern "C" int vla_seq_grouped_glu_supported(int k_in, int dtype) {
+  const int form = g_grouped_form.load(std::memory_order_relaxed);
+  return (dtype == VLA_F16 || dtype == VLA_BF16) && k_in > 0 && k_in % kStep == 0 && (form == 0 || form == 3 || form == 4);
+}
+
+extern "C" int vla_seq_grouped_glu(void* out, int64_t out_stride, const void* a, int64_t a_stride, const int* row_token,
+                                   const void* weight, const int* tile_expert, int max_tiles, int n_out, int k_in, int act,
+                                   int clamped, float limit, float alpha, float shift, const float* row_scale, int dtype,
+                                   int num_experts, void* stream) {
+  if (max_tiles == 0) return VLA_OK;
+  if (!out || !a || !weight || !tile_expert || max_tiles < 0 || n_out <= 0 || k_in <= 0 || out_stride < n_out ||
+      a_stride < k_in || act < VLA_ACT_NONE || act > VLA_ACT_GELU_TANH || num_experts <= 0 ||
+      !dma_fits(a, a_stride, weight, k_in))
+    return VLA_ERR_ARG;
+  const int form = g_grouped_form.load(std::memory_order_relaxed);
+  const bool few = form == 0 ? few_tiles(max_tiles, 2 * n_out, num_experts) : form == 3;
+  auto go = [&](auto s) -> int {
+    using S = decltype(s);
+    const GroupedDma d{out, out_stride, a, a_stride, row_token, weight, tile_expert, row_scale, max_tiles, n_out, k_in,
+                       clamped ? kActClamped : act, limit, alpha, shift, 0, 0};
+    return launch_grouped_dma<S, S, true>(d, num_experts, few, (hipStream_t)stream);
+  };
+  if (dtype == VLA_BF16) return go(BF16{});
+  if (dtype == VLA_F16) return go(F16{});
+  return VLA_ERR_DTYPE;
+}
+
 extern "C" int vla_seq_moe_combine(float* out, const float* y, const int* pair_row,
                                    const float* weights, const void* h, int64_t h_stride,
                                    const float* shared_y, const float* shared_gate, int num_tokens,
@@ -691,9 +1005,10 @@ extern "C" int vla_seq_moe_combine(float* out, const float* y, const int* pair_r
 }
 
 // 0: grouped_linear picks its 16-bit form per shape; 1: always one-wave workgroups; 2: always runs of
-// tiles (through LDS when k_in allows).  Tests run all.
+// tiles; 3, 4: the LDS-DMA forms for few and for many rows where k_in allows.
+// Tests run all.
 extern "C" int vla_seq_set_grouped_linear_form(int mode) {
-  if (mode < 0 || mode > 2) return VLA_ERR_ARG;
+  if (mode < 0 || mode > 4) return VLA_ERR_ARG;
   g_grouped_form.store(mode, std::memory_order_relaxed);
   return VLA_OK;
 }

@@ -157,7 +157,10 @@ class RoutedExperts(nn.Module):
                 pair_row, row_token, tile_expert = ops.moe_plan(experts, self.num_experts)
             rows = row_token.numel()
             u = torch.empty((rows, self.expert_ff), dtype=h.dtype, device=h.device)
-            if self.gated:
+            if self.gated and ops.grouped_glu_supported(h, self.w_up.data):
+                ops.grouped_glu(u, h, row_token, self.w_up.data, tile_expert, self.act, row_scale, self.act_limit,
+                                self.act_alpha, self.act_shift)
+            elif self.gated:
                 both = torch.empty((rows, 2 * self.expert_ff), dtype=h.dtype, device=h.device)
                 ops.grouped_linear(both, h, row_token, self.w_up.data, tile_expert, row_scale=row_scale)
                 self._glu(u, both, self.expert_ff, self.act, self.act_limit)
