@@ -394,6 +394,23 @@ int vla_seq_embed_scaled(float* out, const void* table, const int64_t* ids, floa
 /* z <- cap * tanh(z / cap) over n fp32 values. */
 int vla_seq_softcap(float* z, int64_t n, float cap, void* stream);
 
+/* The whole gated linear recurrence of a step with runs of rows, in chunks of 64 rows worked on at once: decays
+ * ln a = ln(sigmoid(y w2^T + bias)) * inv_tau, S <- diag(a) S + k v^T, o = S^T (q * q_scale),
+ * out = dtype(o / sqrt(mean_v(o^2) + eps) * norm_weight * silu(gate) * out_scale).  q, k [T, heads * dim], v, gate,
+ * out [T, heads * vdim], y [T, rank], w2 [heads * dim, rank]: `dtype` rows, those of q, k, v four values aligned;
+ * bias fp32 [heads * dim] or null, norm_weight fp32 [vdim], state fp32 [num_slots, heads, dim, vdim] (a sequence
+ * with context 0 starts from zero).  dim 16, 32, 64 or 128, vdim a multiple of 16 up to 128, rank up to 32.
+ * scratch: vla_seq_gla_chunks_scratch_floats values, 16-byte aligned (0: these sizes do not go in chunks). */
+int64_t vla_seq_gla_chunks_scratch_floats(int num_tokens, int num_seqs, int heads, int dim, int vdim, int rank);
+int vla_seq_gla_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k,
+                       int64_t k_stride, const void* v, int64_t v_stride, const void* gate, int64_t gate_stride,
+                       const void* y, int64_t y_stride, const void* w2, const float* bias,
+                       const float* norm_weight, float* state, const int* query_start_loc,
+                       const int* context_lens, const int* state_slots, int num_tokens, int num_seqs,
+                       int num_slots, int heads, int dim, int vdim, int rank, float q_scale, float inv_tau,
+                       float eps, float out_scale, float* scratch, int64_t scratch_floats, int dtype,
+                       void* stream);
+
 /* Latent attention over runs of rows with keys and values formed per head (16-bit types; dim, rot, vdim,
  * rank multiples of 8, dim + rot <= 192, vdim <= 128; scale > 0).
  * vla_seq_latent_gather: sequence b's visible cache rows (from max(0, context - window + 1) on, from 0

@@ -1,0 +1,79 @@
+"""The gated linear recurrence in chunks of 64 rows: runs around one and two chunks and blocks of 16 beside
+single rows and continued sequences, every head size it takes, ranks 1 to 32, decays that underflow beside
+decays of one, 16-bit rows -- against the float64 oracle of the recurrence's other tests and their bound for
+fp32 rows (sums of a few hundred terms: 3e-5 of the largest value; 16-bit results: one rounding, 2^-8)."""
+import pytest
+import torch
+
+from tests import lusadra_oracle as R
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def close(got, want, tol):
+    assert float((got.double().cpu() - want).abs().max()) <= tol * float(want.abs().max())
+
+
+def run(H, D, V, rank, lens, ctx, dtype, bias_of=None, offset=0):
+    from vllm_legacy_amd.attention.batch import SequenceBatch
+    from vllm_legacy_amd.attention.recurrent import GatedLinearRecurrence
+    tau, eps, T = 5.0, 1e-5, sum(lens)
+    layer = GatedLinearRecurrence(H, D, V, tau, eps)
+    g = torch.Generator().manual_seed(D + V + T)
+    slots = list(range(len(lens)))[::-1]
+    state = torch.randn(GatedLinearRecurrence.get_state_shape(len(lens), H, D, V), generator=g).to(DEV)
+    before = state.cpu().double()
+    w2 = (torch.randn(H * D, rank, generator=g) * 0.5).to(dtype)
+    bias = torch.randn(H * D, generator=g) + 2 if bias_of is None else bias_of(H * D)
+    norm_w = torch.randn(V, generator=g)
+    widths = [H * D, H * D, H * V, H * V, rank]
+    wide = torch.randn(T, sum(widths) + 8, generator=g).to(dtype)
+    q, k, v, gate, y = wide[:, offset:offset + sum(widths)].split(widths, 1)
+    q, k, v, gate, y = wide.to(DEV)[:, offset:offset + sum(widths)].split(widths, 1)
+    b = SequenceBatch.build(lens, ctx, [[0] * 64] * len(lens), slots, 16, DEV)
+    out = torch.empty(T, H * V, device=DEV, dtype=dtype)
+    layer(out, q, k, v, gate, y, w2.to(DEV), bias.to(DEV), norm_w.to(DEV), state, b, 0.8)
+    F, at, bar = R.F, 0, 3e-5 if dtype == torch.float32 else 2.0**-8
+    q, k, v, gate, y = (t.cpu().to(F) for t in (q, k, v, gate, y))
+    for i, (n, c) in enumerate(zip(lens, ctx)):
+        rows = slice(at, at + n)
+        ln_a = R.log_decay(y[rows], w2.to(F), bias.to(F), tau)
+        S = before[slots[i]] if c else torch.zeros(H, D, V, dtype=F)
+        a, o = torch.exp(ln_a).view(n, H, D), torch.empty(n, H, V, dtype=F)
+        for t in range(n):
+            S = a[t][:, :, None] * S + k[rows][t].view(H, D, 1) * v[rows][t].view(H, 1, V)
+            o[t] = (S * (q[rows][t] * D**-0.5).view(H, D, 1)).sum(1)
+        want = R.gated_head_norm(o, norm_w.to(F), gate[rows], eps, 0.8).reshape(n, H * V)
+        close(out[rows], want, bar)
+        close(state[slots[i]], S, 3e-5)
+        at += n
+    return layer
+
+
+@pytest.mark.parametrize("shape", [(2, 16, 16, 1), (3, 32, 48, 5), (2, 64, 128, 16), (1, 128, 128, 32), (2, 128, 112, 7)])
+@pytest.mark.parametrize("lens,ctx", [([64], [0]), ([63, 1, 65], [0, 7, 3]), ([130, 17, 2, 128], [5, 0, 1, 0]), ([1, 200], [0, 0])])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_runs_around_a_chunk(shape, lens, ctx, dtype):
+    run(*shape, lens, ctx, dtype)
+
+
+def test_decays_of_nothing_and_of_one():
+    def bias_of(n):
+        b = torch.full((n, ), 60.0)         # 1
+        b[::3] = -500.0                     # 0
+        b[1::3] = -8.0
+        return b
+
+    run(2, 64, 128, 4, [150, 70], [3, 0], torch.float32, bias_of)
+
+
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_rows_at_odd_addresses_go_the_other_way(offset):
+    from vllm_legacy_amd import _seq_ops as ops
+    run(2, 32, 32, 3, [100], [0], torch.bfloat16, offset=offset)
+    rows = torch.empty((100, 200), dtype=torch.bfloat16, device=DEV)[:, offset:offset + 64]
+    assert (ops.gla_chunks_scratch(rows, rows, rows, 2, 32, 32, 3, 1) > 0) == (offset % 4 == 0)
+    rows = torch.empty((100, 200), dtype=torch.bfloat16, device=DEV)[:, :64]
+    assert ops.gla_chunks_scratch(rows, rows, rows, 2, 24, 32, 3, 1) == 0
+    assert ops.gla_chunks_scratch(rows, rows, rows, 2, 32, 32, 33, 1) == 0

@@ -263,6 +263,44 @@ MOE_SCORE = {"softmax": 0, "sigmoid": 1}
 GATE = {"silu": 0, "sigmoid": 1}
 
 
+def gla_chunks_scratch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, dim: int, vdim: int, rank: int,
+                       num_seqs: int) -> int:
+    """fp32 values gla_chunks wants for these rows; 0 where they do not go in chunks."""
+    size = 16 if q.dtype == torch.float32 else 8
+    if any(t.data_ptr() % size or (t.shape[0] > 1 and t.stride(0) % 4) for t in (q, k, v)) or (heads * dim) % 4 or \
+            (heads * vdim) % 4:
+        return 0
+    return int(_lib.seq_lib().vla_seq_gla_chunks_scratch_floats(q.shape[0], num_seqs, heads, dim, vdim, rank))
+
+
+def gla_chunks(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor, y: torch.Tensor,
+               w2: torch.Tensor, bias: Optional[torch.Tensor], norm_weight: torch.Tensor, state: torch.Tensor,
+               query_start_loc: torch.Tensor, context_lens: torch.Tensor, state_slots: torch.Tensor, q_scale: float,
+               inv_tau: float, eps: float, out_scale: float, need: int) -> None:
+    """The gated linear recurrence of a step in chunks of 64 rows, head norm and gate included: q, k [T, H*D];
+    v, gate, out [T, H*V]; y [T, R] (views with free row strides); w2 [H*D, R]; bias fp32 [H*D]; norm_weight
+    fp32 [V]; state fp32 [slots, H, D, V]; need: gla_chunks_scratch's answer."""
+    _gpu(out, q, k, v, gate, y, w2, bias, norm_weight, state, query_start_loc, context_lens, state_slots)
+    slots, H, D, V = state.shape
+    T, B, R = q.shape[0], context_lens.numel(), w2.shape[1]
+    assert state.dtype == torch.float32 and state.is_contiguous() and need > 0
+    assert q.dtype == k.dtype == v.dtype == gate.dtype == y.dtype == w2.dtype == out.dtype
+    assert w2.is_contiguous() and w2.shape[0] == H * D
+    assert bias is None or (bias.dtype == torch.float32 and bias.numel() == H * D and bias.is_contiguous())
+    assert norm_weight.dtype == torch.float32 and norm_weight.numel() == V and norm_weight.is_contiguous()
+    for t in (query_start_loc, context_lens, state_slots):
+        assert t.dtype == torch.int32 and t.is_contiguous()
+    assert query_start_loc.numel() == B + 1 and state_slots.numel() == B
+    scratch = torch.empty(need, dtype=torch.float32, device=q.device)
+    with torch.cuda.device(q.device):
+        seq_check(_lib.seq_lib().vla_seq_gla_chunks(
+            out.data_ptr(), _rows(out, H * V), q.data_ptr(), _rows(q, H * D), k.data_ptr(), _rows(k, H * D), v.data_ptr(),
+            _rows(v, H * V), gate.data_ptr(), _rows(gate, H * V), y.data_ptr(), _rows(y, R), w2.data_ptr(), _p(bias),
+            norm_weight.data_ptr(), state.data_ptr(), query_start_loc.data_ptr(), context_lens.data_ptr(),
+            state_slots.data_ptr(), T, B, slots, H, D, V, R, float(q_scale), float(inv_tau), float(eps), float(out_scale),
+            scratch.data_ptr(), need, _dt(q.dtype), _stream(q.device)), "gla_chunks")
+
+
 def residual_norms(x: torch.Tensor, y: Optional[torch.Tensor] = None, y_bias: Optional[torch.Tensor] = None,
                    post_weight: Optional[torch.Tensor] = None,
                    layer_scale: Optional[torch.Tensor] = None, add_row: Optional[torch.Tensor] = None,

@@ -6,7 +6,9 @@ fp32 tensor [num_slots, heads, dim, vdim] that the engine's cache manager hands 
 sequence whose context length is 0 starts from zero whatever its slot held before.  The output of
 each head is RMS-normed over vdim, gated with silu and scaled before the output projection.
 
-A long run of rows (a prompt, a large portion) is cut into pieces of PIECE_ROWS rows that are
+Steps with runs of rows go in chunks of 64 rows that are worked on at the same time
+(csrc/seq_linear_chunks.hip: decays, chunk states, outputs, head norm and gate in three launches).  Sizes that
+kernel does not take: a long run of rows (a prompt, a large portion) is cut into pieces of PIECE_ROWS rows that are
 walked at the same time, each from a zero state in a scratch slot behind the sequences' slots;
 the state a piece should have started from then reaches its outputs through one batched matrix
 product (o_t += (q_t exp(c_t))^T S_start, c_t the log decays summed from the piece's first row)
@@ -29,6 +31,13 @@ class GatedLinearRecurrence(nn.Module):
     # rows of a piece; runs of at least two pieces are cut (VLA_GLA_PIECE_ROWS: another size, for studies)
     PIECE_ROWS = int(os.environ.get("VLA_GLA_PIECE_ROWS", "256"))
     SCRATCH_SLOTS = 64      # state slots behind the sequences' own, for the pieces of a step
+    # A step goes in chunks of 64 rows (where the sizes allow it) if its longest run has that many.  16 heads of
+    # 64 x 128, bf16, walked token by token / in chunks, us: 1 run of 64 rows 48/46, of 300 128/49; 6 of 48 48/49,
+    # of 64 54/53, of 128 99/67; 32 of 32 125/107, of 64 195/133, of 300 758/348.  A single row costs a whole
+    # chunk, so many beside one run need a long run (the walk's time is its longest run's).
+    CHUNK_MIN_ROWS = 64
+    CHUNK_MEAN_ROWS = 16    # rows per run on average ...
+    CHUNK_LONG_ROWS = 512   # ... unless a run is this long
 
     def __init__(self, num_heads: int, head_dim: int, value_dim: int, tau: float, eps: float,
                  q_scale: Optional[float] = None) -> None:
@@ -91,6 +100,15 @@ class GatedLinearRecurrence(nn.Module):
         """q, k [T, H*D]; v, gate, out [T, H*V]; y [T, R] (views with free row strides);
         w2 [H*D, R]; bias fp32 [H*D]; norm_weight fp32 [V]."""
         T, H, D, V = q.shape[0], self.num_heads, self.head_dim, self.value_dim
+        longest = batch.max_query_len
+        if (longest >= self.CHUNK_MIN_ROWS
+                and (T >= self.CHUNK_MEAN_ROWS * batch.num_seqs or longest >= self.CHUNK_LONG_ROWS)
+                and q.dtype == gate.dtype == out.dtype == w2.dtype == y.dtype):
+            need = ops.gla_chunks_scratch(q, k, v, H, D, V, w2.shape[1], batch.num_seqs)
+            if need:
+                ops.gla_chunks(out, q, k, v, gate, y, w2, bias, norm_weight, state, batch.query_start_loc,
+                               batch.context_lens, batch.state_slots, self.q_scale, self.inv_tau, self.eps, out_scale, need)
+                return out
         log_decay = torch.empty((T, H * D), dtype=torch.float32, device=q.device)
         ops.gla_log_decay(log_decay, y, w2, bias, self.inv_tau)
         o = torch.empty((T, H, V), dtype=torch.float32, device=q.device)
