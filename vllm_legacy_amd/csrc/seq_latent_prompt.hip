@@ -231,7 +231,10 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
   int u0 = g_first & ~(kKeys - 1);
   bring(u0, 0);
   for (int it = 0; u0 <= p_end; u0 += kKeys, ++it) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // the builtin and not asm: the compiler then knows that the query rows have arrived, and does not wait for
+    // vmcnt(0), and so for the DMA just started, at their first use in every step
+    __builtin_amdgcn_s_waitcnt(0x0f70);                // vmcnt(0)
+    asm volatile("" ::: "memory");
     __syncthreads();
     if (u0 + kKeys <= p_end) bring(u0 + kKeys, (it + 1) & 1);
     const unsigned char* k_lds = smem + (it & 1) * STAGE;
