@@ -407,9 +407,8 @@ __device__ __forceinline__ void turn_back(f32x16 (&o)[VB], int hf, float p,
 // workgroup per (sequence, tile of query rows, KV head, chunk of its query heads).  Its four waves
 // are (query head of the chunk) x (block of 32 consecutive rows): 4 x 1 for groups of three heads
 // and more, 2 x 2 for two, 1 x 4 for one, so a tile is 32, 64 or 128 rows.  Keys and values from
-// the first row's window start to the last row walk through LDS in tiles of 64, row-major, staged
-// once for all waves and loaded one tile ahead; the rows' places in the paged caches are looked up
-// once per tile by 64 threads, two tiles ahead.
+// the first row's window start to the last row walk through LDS in tiles of 64; the rows' places in
+// the paged caches are looked up once per tile by 64 threads, two tiles ahead.
 //   S^T = K q^T   A = K    lane: key c of a 32-key block, dims 16 ks + 8 hf .. + 7   (LDS, 16 bytes)
 //                 B = q^T  lane: query c, the same dims (registers, loaded once)
 //                 C        lane: query c, keys (i & 3) + 8 (i >> 2) + 4 hf, i = 0 .. 15
@@ -420,6 +419,19 @@ __device__ __forceinline__ void turn_back(f32x16 (&o)[VB], int hf, float p,
 // first product's result to the second's operand without leaving the lane.  Scores, running
 // max / sum (base 2) and the accumulators are fp32; a weight enters the second product rounded to
 // the model dtype.
+//
+// Bound by the products and the softmax between them (about 30 vector cycles per score), so the tiles
+// come in by LDS-DMA: no staging registers, no waits before the stores to LDS, one barrier per tile, two
+// tiles in LDS (at most 64 KB: two workgroups share a CU and one's softmax runs under the other's
+// products).  A DMA instruction writes 64 lanes x 16 bytes in a row, so rows cannot be padded: 16-byte
+// pieces of a key row and 64-byte units of a value row are exchanged by the row's number on the source's
+// side, so that the lanes of a read fall into different banks.  What only some calls need (a cap, masks)
+// is a loop of its own behind one branch.  Workgroups go out longest walk first over all sequences, and those
+// of a (sequence, head) share an XCD's L2 when their number is a multiple of 8.  Where the workgroups are few,
+// each has two groups of four waves (KG = 2) that take every other tile and join their sums at the end.  Four
+// prompts of up to 2047 rows, 16 heads on 4 of 128: 102 us, against 172 with tiles staged through registers
+// into padded rows.  A wave alone takes 2.6 us per tile, 0.45 of them products: what is left is the chain
+// from the scores over their maximum and the exponentials to the second product.
 template <class S>
 struct Mfma16;
 template <>
@@ -455,38 +467,61 @@ __device__ __forceinline__ uint32_t pack2<BF16>(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
-template <class S, int DB, int VB>
-__global__ __launch_bounds__(256, 2) void kv_attention_tile_kernel(
+// which units of 64 bytes of a value row change place: rows whose units would meet in the banks
+template <int VB>
+__device__ __forceinline__ int value_exchange(int r) {
+  return VB == 4 ? r & 3 : VB == 2 ? (r >> 1) & 1 : 0;
+}
+
+// 16 bytes per lane from each lane's own address into 1 KB of LDS (no register result)
+__device__ __forceinline__ void tile_dma16(const void* src, uint32_t lds_at) {
+  unsigned keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(src), "s"(lds_at)
+      : "memory");
+}
+
+template <class S, int DB, int VB, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
     typename S::T* __restrict__ out, int64_t out_stride, const typename S::T* __restrict__ q,
     int64_t q_stride, const typename S::T* __restrict__ gate, int64_t gate_stride,
     const typename S::T* __restrict__ key_cache, const typename S::T* __restrict__ value_cache,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ query_start_loc,
     const int* __restrict__ context_lens, const float* __restrict__ out_inv_freq, int interleaved,
-    int heads, int kv_heads, int block_size, int num_blocks, int window, float scale, int head_waves,
-    int keep_first, float softcap, int chunk, const float* __restrict__ sinks, int v_row, int v_first) {
+    int heads, int kv_heads, int head_groups, int block_size, int num_blocks, int window, float scale, int head_waves,
+    int keep_first, float softcap, int chunk, const float* __restrict__ sinks, int v_row, int v_first,
+    int last_tile) {
   using T = typename S::T;
   using M = Mfma16<S>;
   constexpr int D = 32 * DB, VD = 32 * VB;
-  // elements; rows stay 16-byte aligned, and four value rows a transposing read takes fall into
-  // different banks
-  constexpr int KROW = D + 8, VROW = VD + 16;
-  __shared__ __align__(16) T k_lds2[2][kKeys * KROW];  // two tiles: one is read while the next lands
-  __shared__ __align__(16) T v_lds2[2][kKeys * VROW];
-  __shared__ long long rows_lds[2][kKeys];            // token row of each key of a tile, -1: none
-  const int b = blockIdx.z;
+  constexpr int KB = 2 * D, VBYTES = 2 * VD;           // bytes of a tile's rows
+  constexpr int kStep = kKeys * KG;                    // keys of a step: a tile for every group of four waves
+  constexpr int KTILE = kKeys * KB, VTILE = kKeys * VBYTES, STAGE = KTILE + VTILE;
+  // which 16-byte pieces of a key row change place: the rows of 16 lanes begin at one, two or four places
+  // among the banks, and the exchange spreads those that begin at the same one
+  constexpr int KMASK = DB == 4 ? 15 : DB == 2 ? 7 : 3, KSHIFT = DB == 4 ? 0 : DB == 2 ? 1 : 2;
+  // two tiles for every group of waves: one is read while the next lands
+  __shared__ __align__(16) unsigned char all_tiles[KG * 2 * STAGE];
+  __shared__ long long all_rows[KG][2][2][kKeys];      // first byte of each key and value row of a tile
+  const int b = blockIdx.x / head_groups, yb = blockIdx.x - b * head_groups;
   const int row_blocks = 4 / head_waves;              // blocks of 32 query rows per workgroup
   const int tile_rows = kTile * row_blocks;
   // the last tiles of a run have the most keys to walk: they are dispatched first
-  const int tile_x = gridDim.x - 1 - blockIdx.x;
+  const int tile_x = last_tile - (int)blockIdx.y;
   const int t_first = query_start_loc[b] + tile_rows * tile_x;
   const int n_tile = min(tile_rows, query_start_loc[b + 1] - t_first);
   if (n_tile <= 0) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);      // group of waves
+  const int tid = threadIdx.x & 255, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned char* tiles = all_tiles + kg * 2 * STAGE;
+  auto& rows_lds = all_rows[kg];
   const int hf = lane >> 5, c = lane & 31;
   const int group = heads / kv_heads;
   const int chunks = (group + head_waves - 1) / head_waves;
-  const int g = blockIdx.y / chunks;
-  const int h = g * group + (blockIdx.y % chunks) * head_waves + w % head_waves;
+  const int g = yb / chunks;
+  const int h = g * group + (yb % chunks) * head_waves + w % head_waves;
   const int rb = w / head_waves;                      // this wave's block of rows
   const int t0 = t_first + kTile * rb;
   const int nq = min(kTile, n_tile - kTile * rb);     // <= 0: no rows for this wave
@@ -506,6 +541,9 @@ __global__ __launch_bounds__(256, 2) void kv_attention_tile_kernel(
   const int* table = block_tables + (int64_t)b * max_blocks;
   const float scale2 = scale * 1.4426950408889634f;   // scores in base 2
   const float cap2 = softcap * 1.4426950408889634f, cap_arg = softcap > 0.f ? 2.f * 1.4426950408889634f / softcap : 0.f;
+  // a positive scale is left to the exponent's fused product; otherwise scores are scaled before the maximum
+  const bool late = softcap <= 0.f && scale2 > 0.f;
+  const float factor = late ? scale2 : 1.f;
 
   u32x4 qf[D / 16];
 #pragma unroll
@@ -521,167 +559,210 @@ __global__ __launch_bounds__(256, 2) void kv_attention_tile_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[n][i] = 0.f;
   float m = -INFINITY, l = 0.f;
-  if (sinks != nullptr && active) {       // the denominator's first term, counted in one lane half
+  if (sinks != nullptr && active && kg == 0) {     // the denominator's first term, counted in one lane half
     m = sinks[h] * 1.4426950408889634f;
     l = hf == 0 ? 1.f : 0.f;
   }
 
   // threads 0 .. 63 look the rows of a tile up: the block id is read one step before it is used
-  auto load_block = [&](int u0) {
-    const int u = u0 + tid;
-    int blk = -1;
-    if (u < total) {
-      blk = table[key_of(u) / block_size];
-      blk = (unsigned)blk < (unsigned)num_blocks ? blk : 0;
-    }
-    return blk;
+  const bool shifts = (block_size & (block_size - 1)) == 0;
+  const int shift = __builtin_ctz(block_size);
+  struct Place {
+    int blk, at;
   };
-  auto store_row = [&](int u0, int blk, int buf) {
-    const int j = key_of(u0 + tid);
-    rows_lds[buf][tid] = blk < 0 ? -1 : ((long long)blk * block_size + j % block_size) * kv_heads + g;
+  auto look_up = [&](int u0) {
+    const int j = key_of(min(u0 + tid, total - 1));    // behind the end: the last key again, masked
+    const int nb = shifts ? j >> shift : j / block_size;
+    const int blk = table[nb];
+    return Place{(unsigned)blk < (unsigned)num_blocks ? blk : 0, j - nb * block_size};
   };
-  // staging: DB + VB pieces of 16 bytes per thread and tile
-  u32x4 xk[DB], xv[VB];
-  auto fetch = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < DB; ++u) {
-      const int i = tid + 256 * u;
-      const int r = i / (D / 8), v = i % (D / 8);
-      const long long row = rows_lds[buf][r];
-      const u32x4 got = *reinterpret_cast<const u32x4*>(key_cache + (row >= 0 ? row * D + 8 * v : 0));
-      xk[u] = row >= 0 ? got : u32x4{0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int u = 0; u < VB; ++u) {
-      const int i = tid + 256 * u;
-      const int r = i / (VD / 8), v = i % (VD / 8);
-      const long long row = rows_lds[buf][r];
-      const u32x4 got = *reinterpret_cast<const u32x4*>(value_cache + (row >= 0 ? row * v_row + v_first + 8 * v : 0));
-      xv[u] = row >= 0 ? got : u32x4{0u, 0u, 0u, 0u};
-    }
+  auto store_row = [&](Place p, int buf) {
+    const long long row = ((long long)p.blk * block_size + p.at) * kv_heads + g;
+    rows_lds[buf][0][tid] = row * (2 * D);
+    rows_lds[buf][1][tid] = row * (2 * v_row);
   };
-  auto land = [&](int buf) {                           // the fetched tile into LDS
+  // what this lane brings in: the row of a tile, and the piece of it that stands at the lane's place
+  int row_k[DB], at_k[DB], row_v[VB], at_v[VB];
 #pragma unroll
-    for (int u = 0; u < DB; ++u) {
-      const int i = tid + 256 * u;
-      const int r = i / (D / 8), v = i % (D / 8);
-      *reinterpret_cast<u32x4*>(k_lds2[buf] + r * KROW + 8 * v) = xk[u];
-    }
+  for (int u = 0; u < DB; ++u) {
+    const int at = (w * DB + u) * 64 + lane, r = at / (KB / 16), p = at % (KB / 16);
+    row_k[u] = r;
+    at_k[u] = 16 * ((p & ~KMASK) | ((p ^ (r >> KSHIFT)) & KMASK));
+  }
 #pragma unroll
-    for (int u = 0; u < VB; ++u) {
-      const int i = tid + 256 * u;
-      const int r = i / (VD / 8), v = i % (VD / 8);
-      *reinterpret_cast<u32x4*>(v_lds2[buf] + r * VROW + 8 * v) = xv[u];
-    }
+  for (int u = 0; u < VB; ++u) {
+    const int at = (w * VB + u) * 64 + lane, r = at / (VBYTES / 16), p = at % (VBYTES / 16);
+    row_v[u] = r;
+    at_v[u] = 2 * v_first + 16 * ((((p >> 2) ^ value_exchange<VB>(r)) << 2) | (p & 3));
+  }
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)tiles;
+  auto bring = [&](int buf) {                          // the tile whose rows are in rows_lds[buf] into buffer buf
+    const uint32_t to = lds0 + buf * STAGE;
+    const unsigned char *sk[DB], *sv[VB];              // all of them first: one wait for LDS
+#pragma unroll
+    for (int u = 0; u < DB; ++u) sk[u] = (const unsigned char*)key_cache + (rows_lds[buf][0][row_k[u]] + at_k[u]);
+#pragma unroll
+    for (int u = 0; u < VB; ++u) sv[u] = (const unsigned char*)value_cache + (rows_lds[buf][1][row_v[u]] + at_v[u]);
+#pragma unroll
+    for (int u = 0; u < DB; ++u) tile_dma16(sk[u], to + (w * DB + u) * 1024);
+#pragma unroll
+    for (int u = 0; u < VB; ++u) tile_dma16(sv[u], to + KTILE + (w * VB + u) * 1024);
   };
-  // One barrier per tile.  At the top of step `it`: tile `it` is in LDS buffer it & 1, tile it + 1
-  // in the staging registers, the rows of tile it + 2 in rows_lds[it & 1], and threads 0 .. 63 hold
-  // the block ids of tile it + 3 (whose rows go to rows_lds[(it + 1) & 1] during the step).
-  int blk_next = -1;
+  // where this lane reads: the exchanged piece of its key row, and the unit of its value rows
+  const int kx = (hf ^ (c >> KSHIFT)) & KMASK;         // piece 2 ks + hf stands at 2 ks ^ kx within its group
+  const int i16 = c & 15;
+  const int vr = 4 * hf + (i16 >> 2);
+  const int vf = value_exchange<VB>(vr);               // 8 and 16 rows further on it is the same
+  const int vat = vr * VBYTES + 32 * (c >> 4) + 8 * (i16 & 3);
+
+  // One barrier per tile.  Behind it in step `it`: tile `it` is in its buffer, the rows of tile it + 1 are in
+  // rows_lds[(it + 1) & 1], and threads 0 .. 63 hold the block ids of tile it + 2.
+  Place next = {0, 0};
   if (tid < kKeys) {
-    store_row(0, load_block(0), 0);
-    store_row(kKeys, load_block(kKeys), 1);
+    const int u = kg * kKeys;
+    store_row(look_up(u), 0);
+    store_row(look_up(u + kStep), 1);
+    next = look_up(u + 2 * kStep);
   }
   __syncthreads();
-  fetch(0);
-  land(0);
-  fetch(1);
-  __syncthreads();                                     // rows_lds[0] is read: tile 2's rows may go there
-  if (tid < kKeys) {
-    store_row(2 * kKeys, load_block(2 * kKeys), 0);
-    blk_next = load_block(3 * kKeys);
-  }
-  __syncthreads();
-  int it = 0;
-  for (int u0 = 0; u0 < total; u0 += kKeys, ++it) {
-    const T* k_lds = k_lds2[it & 1];
-    const T* v_lds = v_lds2[it & 1];
+  if (kg * kKeys < total) bring(0);
+  const int steps = (total + kStep - 1) / kStep;
+  for (int it = 0; it < steps; ++it) {
+    const int u0 = it * kStep + kg * kKeys;
+    // the builtin and not asm: the compiler then knows that the query rows have arrived, and does not wait for
+    // vmcnt(0), and so for the DMA just started, at their first use in every step
+    __builtin_amdgcn_s_waitcnt(0x0f70);                // vmcnt(0)
+    asm volatile("" ::: "memory");
+    __syncthreads();
+    // ahead of the next DMA, whose end the use of a loaded block id would otherwise wait for
+    // (rows of tile `it` were read ahead of the barrier)
+    if (tid < kKeys) store_row(next, it & 1);
+    if (u0 + kStep < total) bring((it + 1) & 1);
+    if (tid < kKeys) next = look_up(u0 + 3 * kStep);
+    const unsigned char* k_lds = tiles + (it & 1) * STAGE;
+    const unsigned char* v_lds = k_lds + KTILE;
     // a tile with kept tokens ahead of the window concerns every row; of the others, a tile whose
     // keys lie past this wave's last row, or before its first row's window (and are not kept ones),
     // is none of its business
     const bool kept_tile = u0 < nk;
     const int j0 = u0 - nk + j_lo;            // the tile's first key when it holds window keys only
-    if (active && (kept_tile || (j0 <= p0 + nq - 1 &&
-                                 !(j0 + kKeys - 1 < lo_first && j0 >= keep_first)))) {
-      f32x16 st[2];
+    if (!active || u0 >= total || !(kept_tile || (j0 <= p0 + nq - 1 && !(j0 + kKeys - 1 < lo_first && j0 >= keep_first)))) continue;
+    f32x16 st[2];
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) st[kb][i] = 0.f;
+      for (int i = 0; i < 16; ++i) st[kb][i] = 0.f;
+    // keys are read two steps ahead of their products, which the compiler would not do by itself
+    auto key_at = [&](int ks, int kb) {
+      const int slot = ((2 * ks) & ~KMASK) | (((2 * ks) & KMASK) ^ kx);
+      return *reinterpret_cast<const u32x4*>(k_lds + (32 * kb + c) * KB + 16 * slot);
+    };
+    u32x4 ka[3][2];
 #pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks) {
-          const u32x4 a = *reinterpret_cast<const u32x4*>(k_lds + (32 * kb + c) * KROW + 16 * ks + 8 * hf);
-          st[kb] = M::run(a, qf[ks], st[kb]);
-        }
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) ka[ks][kb] = key_at(ks, kb);
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      if (ks + 2 < D / 16) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) ka[(ks + 2) % 3][kb] = key_at(ks + 2, kb);
       }
-      // every key of the tile visible to every row of the wave: no masks
-      const bool full = !kept_tile && j0 + kKeys - 1 <= p0 && nq == kTile && j0 >= lo_last;
-      float mt = -INFINITY;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) st[kb] = M::run(ka[ks % 3][kb], qf[ks], st[kb]);
+    }
+    if (softcap > 0.f) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st[kb][i] = cap_score_fast(st[kb][i] * scale, cap2, cap_arg);
+    } else if (!late) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st[kb][i] *= scale2;
+    }
+    // every key of the tile visible to every row of the wave: no masks
+    if (kept_tile || j0 + kKeys - 1 > p0 || nq != kTile || j0 < lo_last) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          float v = st[kb][i] * scale2;
-          if (softcap > 0.f) v = cap_score_fast(st[kb][i] * scale, cap2, cap_arg);
-          if (!full) {
-            const int j = key_of(u0 + 32 * kb + (i & 3) + 8 * (i >> 2) + 4 * hf);
-            const bool ok = c < nq && j <= pq && (j >= lo_q || j < keep_first);
-            v = ok ? v : -INFINITY;
-          }
-          st[kb][i] = v;
-          mt = fmaxf(mt, v);
-        }
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-      const float m_new = fmaxf(m, mt);
-      const bool none = m_new == -INFINITY;
-      const float corr = none ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
-      float psum = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float pv = none ? 0.f : __builtin_amdgcn_exp2f(st[kb][i] - m_new);
-          st[kb][i] = pv;
-          psum += pv;
-        }
-      l = l * corr + psum;          // this lane's keys; the partner's half is added at the end
-      m = m_new;
-      if (__any(corr != 1.f)) {     // the running max of some row moved
-#pragma unroll
-        for (int n = 0; n < VB; ++n)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[n][i] *= corr;
-      }
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          u32x4 pb;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) pb[e] = pack2<S>(st[kb][8 * s2 + 2 * e], st[kb][8 * s2 + 2 * e + 1]);
-          // transposing read of the row-major tile: a group of 16 lanes reads 4 keys x 16 dims, 8
-          // bytes per lane (key i16 >> 2, dims 4 (i16 & 3) .. + 3), and every lane receives the four
-          // keys of dim i16 of the group
-          const int i16 = c & 15;
-          const T* src = v_lds + (32 * kb + 16 * s2 + 4 * hf + (i16 >> 2)) * VROW + 16 * (c >> 4) + 4 * (i16 & 3);
-#pragma unroll
-          for (int n = 0; n < VB; ++n) {
-            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(src + 32 * n));
-            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(src + 32 * n + 8 * VROW));
-            const u32x2 lo2 = __builtin_bit_cast(u32x2, lo), hi2 = __builtin_bit_cast(u32x2, hi);
-            const u32x4 a = {lo2[0], lo2[1], hi2[0], hi2[1]};
-            o[n] = M::run(a, pb, o[n]);
-          }
+          const int j = key_of(u0 + 32 * kb + (i & 3) + 8 * (i >> 2) + 4 * hf);
+          st[kb][i] = c < nq && j <= pq && (j >= lo_q || j < keep_first) ? st[kb][i] : -INFINITY;
         }
     }
-    if (u0 + kKeys < total) land((it + 1) & 1);                // tile it + 1, fetched a step ago
-    if (u0 + 2 * kKeys < total) fetch(it & 1);                 // tile it + 2 on its way
-    if (tid < kKeys && u0 + 3 * kKeys < total) {
-      // rows of tile it + 3 into the buffer the step before read tile it + 1's from
-      store_row(u0 + 3 * kKeys, blk_next, (it + 1) & 1);
-      blk_next = load_block(u0 + 4 * kKeys);
+    float mt = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mt = fmaxf(mt, st[kb][i]);
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64)) * factor;
+    const float m_new = fmaxf(m, mt);
+    const float shift = m_new == -INFINITY ? 0.f : m_new;  // nothing seen yet: every weight is 2^-inf
+    const float corr = __builtin_amdgcn_exp2f(m - shift);
+    float psum = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kb][i], factor, -shift));
+        st[kb][i] = pv;
+        psum += pv;
+      }
+    l = l * corr + psum;            // this lane's keys; the partner's half is added at the end
+    if (__any(m_new != m)) {        // the running max of some row moved
+#pragma unroll
+      for (int n = 0; n < VB; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[n][i] *= corr;
+    }
+    m = m_new;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) {
+        u32x4 pb;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pb[e] = pack2<S>(st[kb][8 * s2 + 2 * e], st[kb][8 * s2 + 2 * e + 1]);
+        // transposing read of the row-major tile: a group of 16 lanes reads 4 keys x 16 dims, 8
+        // bytes per lane (key i16 >> 2, dims 4 (i16 & 3) .. + 3), and every lane receives the four
+        // keys of dim i16 of the group
+        const unsigned char* src = v_lds + vat + (32 * kb + 16 * s2) * VBYTES;
+#pragma unroll
+        for (int n = 0; n < VB; ++n) {
+          const unsigned char* at = src + 64 * (n ^ vf);
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)at);
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 8 * VBYTES));
+          const u32x2 lo2 = __builtin_bit_cast(u32x2, lo), hi2 = __builtin_bit_cast(u32x2, hi);
+          const u32x4 a = {lo2[0], lo2[1], hi2[0], hi2[1]};
+          o[n] = M::run(a, pb, o[n]);
+        }
+      }
+  }
+  if constexpr (KG == 2) {
+    // the second group hands its sums over: registers lie lane for lane in the tiles' place
+    __syncthreads();
+    float* part = reinterpret_cast<float*>(all_tiles) + w * (VB * 16 + 2) * kWave + lane;
+    if (kg == 1) {
+      part[0] = m;
+      part[kWave] = l;
+#pragma unroll
+      for (int n = 0; n < VB; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[(2 + 16 * n + i) * kWave] = o[n][i];
     }
     __syncthreads();
+    if (kg == 1) return;
+    const float m2 = part[0], m_new = fmaxf(m, m2);
+    const float shift = m_new == -INFINITY ? 0.f : m_new;
+    const float f = __builtin_amdgcn_exp2f(m - shift), f2 = __builtin_amdgcn_exp2f(m2 - shift);
+    l = l * f + part[kWave] * f2;
+#pragma unroll
+    for (int n = 0; n < VB; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[n][i] = o[n][i] * f + part[(2 + 16 * n + i) * kWave] * f2;
   }
   if (!active) return;
   l += __shfl_xor(l, 32, 64);
@@ -694,11 +775,20 @@ __global__ __launch_bounds__(256, 2) void kv_attention_tile_kernel(
   if (out_inv_freq != nullptr) turn_back<VB>(o, hf, (float)pq, out_inv_freq, interleaved);
   float gv = 1.f;
   if (gate != nullptr) gv = 1.f / (1.f + expf(-S::to_f32(gate[(int64_t)(t0 + c) * gate_stride + h])));
+  T* orow = out + (int64_t)(t0 + c) * out_stride + (int64_t)h * v_row + v_first;
+  if (((uintptr_t)out | (uintptr_t)(out_stride * 2)) % 8 == 0) {
 #pragma unroll
-  for (int n = 0; n < VB; ++n)
+    for (int n = 0; n < VB; ++n)
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      out[(int64_t)(t0 + c) * out_stride + (int64_t)h * v_row + v_first + out_dim(n, i, hf)] = S::from_f32(o[n][i] * gv);
+      for (int i = 0; i < 16; i += 4)
+        *reinterpret_cast<u32x2*>(orow + out_dim(n, i, hf)) =
+            u32x2{pack2<S>(o[n][i] * gv, o[n][i + 1] * gv), pack2<S>(o[n][i + 2] * gv, o[n][i + 3] * gv)};
+  } else {
+#pragma unroll
+    for (int n = 0; n < VB; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) orow[out_dim(n, i, hf)] = S::from_f32(o[n][i] * gv);
+  }
 }
 
 // kv_attention_heads_kernel<S, DB, VB>: single rows (decode steps).  One workgroup per (row, KV
@@ -1345,12 +1435,19 @@ int launch_tiles_one(dim3 grid, hipStream_t stream, typename S::T* out, int64_t 
                      const int* qsl, const int* ctx, const float* out_inv_freq, int interleaved,
                      int heads, int kv_heads, int block_size, int num_blocks, int window,
                      float scale, int head_waves, int keep_first, float softcap, int chunk,
-                     const float* sinks, int v_row, int v_first) {
-  kv_attention_tile_kernel<S, DB, VB><<<grid, 256, 0, stream>>>(
-      out, out_stride, q, q_stride, gate, gate_stride, key_cache, value_cache, block_tables,
-      max_blocks, qsl, ctx, out_inv_freq, interleaved, heads, kv_heads, block_size, num_blocks,
-      window, scale, head_waves, keep_first, softcap, chunk, sinks, v_row, v_first);
-  VLA_SEQ_HIP_CHECK(hipGetLastError());
+                     const float* sinks, int key_groups, int v_row, int v_first) {
+  // grid: (sequences x groups of heads, row tiles); more tiles than a grid's second side takes go in several
+  // launches, the last rows first
+  constexpr int kSide = 65535;
+  for (int left = grid.y; left > 0; left -= kSide) {
+    const dim3 part(grid.x, left < kSide ? left : kSide);
+    auto* kernel = key_groups == 2 ? &kv_attention_tile_kernel<S, DB, VB, 2> : &kv_attention_tile_kernel<S, DB, VB, 1>;
+    kernel<<<part, 256 * key_groups, 0, stream>>>(
+        out, out_stride, q, q_stride, gate, gate_stride, key_cache, value_cache, block_tables,
+        max_blocks, qsl, ctx, out_inv_freq, interleaved, heads, kv_heads, (int)grid.z, block_size, num_blocks,
+        window, scale, head_waves, keep_first, softcap, chunk, sinks, v_row, v_first, left - 1);
+    VLA_SEQ_HIP_CHECK(hipGetLastError());
+  }
   return VLA_OK;
 }
 
@@ -1625,8 +1722,15 @@ extern "C" int vla_seq_kv_attention_tiles(
   const int group = heads / kv_heads;
   const int head_waves = group >= 3 ? 4 : group;      // waves of a workgroup that are heads
   const int tile_rows = kTile * (4 / head_waves);
-  const dim3 grid((max_query_len + tile_rows - 1) / tile_rows,
-                  kv_heads * ((group + head_waves - 1) / head_waves), num_seqs);
+  const int head_groups = kv_heads * ((group + head_waves - 1) / head_waves);
+  // more workgroups in a row than the hardware counts: no such batch fits into memory
+  if ((int64_t)head_groups * num_seqs > 0x7fffffff / 256) return VLA_ERR_ARG;
+  // few workgroups share their keys out to two groups of four waves: of 2047 rows, 16 heads on 4 of 128, one run
+  // (256 workgroups) takes 68 us instead of 88, two take 76 instead of 100; four fill the chip with independent
+  // ones (116 instead of 138: two workgroups of a CU do not wait for each other)
+  const int64_t workgroups = (int64_t)head_groups * num_seqs * ((max_query_len + tile_rows - 1) / tile_rows);
+  const int key_groups = workgroups <= 512 ? 2 : 1;
+  const dim3 grid(head_groups * num_seqs, (max_query_len + tile_rows - 1) / tile_rows, head_groups);
   auto go = [&](auto tag) {
     using S = decltype(tag);
     using T = typename S::T;
@@ -1635,7 +1739,7 @@ extern "C" int vla_seq_kv_attention_tiles(
                              (const T*)gate, gate_stride, (const T*)key_cache, (const T*)value_cache,
                              block_tables, max_blocks, query_start_loc, context_lens, out_inv_freq,
                              interleaved, heads, kv_heads, block_size, num_blocks, window, scale,
-                             head_waves, keep_first, softcap, chunk, sinks, vdim, v_first);
+                             head_waves, keep_first, softcap, chunk, sinks, key_groups, vdim, v_first);
     });
   };
   return dtype == VLA_BF16 ? go(BF16{}) : go(F16{});
