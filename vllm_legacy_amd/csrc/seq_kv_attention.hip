@@ -1746,8 +1746,8 @@ extern "C" int vla_seq_kv_attention_tiles(
   const int head_waves = group >= 3 ? 4 : group;      // waves of a workgroup that are heads
   const int tile_rows = kTile * (4 / head_waves);
   const int head_groups = kv_heads * ((group + head_waves - 1) / head_waves);
-  // more workgroups in a row than the hardware counts: no such batch fits into memory
-  if ((int64_t)head_groups * num_seqs > 0x7fffffff / 256) return VLA_ERR_ARG;
+  // a launch counts its threads in 32 bits; 65535 sequences reach that with more than 256 groups of heads
+  if ((int64_t)head_groups * num_seqs > 0xffffffffll / 256) return VLA_ERR_ARG;
   // few workgroups share their keys out to two groups of four waves: of 2047 rows, 16 heads on 4 of 128, one run
   // (256 workgroups) takes 68 us instead of 88, two take 76 instead of 100; four fill the chip with independent
   // ones (116 instead of 138: two workgroups of a CU do not wait for each other)
