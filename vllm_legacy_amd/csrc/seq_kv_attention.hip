@@ -1042,6 +1042,7 @@ constexpr int kDecodeWaves = 4;
 constexpr int kDecodeHeads = 16;
 constexpr int kDecodeKeys = 32;
 constexpr int kDecodeMinSplitKeys = 256;      // keys of a split, at least
+constexpr int kDecodeWholeKeys = 2048;        // rows that see no more than these are not split
 
 template <class S>
 struct Mma16x16;
@@ -1380,10 +1381,13 @@ __global__ __launch_bounds__(32 * VB) void kv_decode_merge_kernel(KvDecode a) {
 }
 
 // Workgroups that a row's keys are shared out to: as many as bring the launch to one per CU, none with fewer
-// than kDecodeMinSplitKeys keys.  max_keys 0 (unknown): one.
+// than kDecodeMinSplitKeys keys.  max_keys 0 (unknown): one.  The merge is a launch and a scratch allocation more,
+// about 4 us per call, which up to 2048 keys are not worth (16 / 4 heads of 128, us per call, shared / one
+// workgroup: 2 rows of 512 keys 45 / 40, of 2048 44 / 40, of 4096 45 / 65; 8 rows of 2048 42 / 42, of 4096
+// 43 / 68; 32 rows of 1024 43 / 38, of 4096 59 / 70).
 int decode_splits(int num_tokens, int kv_heads, int max_keys) {
   const int64_t groups = (int64_t)num_tokens * kv_heads;
-  if (groups >= 256 || max_keys <= 0) return 1;
+  if (groups >= 256 || max_keys <= kDecodeWholeKeys) return 1;
   return (int)std::max<int64_t>(1, std::min<int64_t>((256 + groups - 1) / groups, max_keys / kDecodeMinSplitKeys));
 }
 
