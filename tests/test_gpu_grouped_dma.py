@@ -91,3 +91,29 @@ def test_gated_products(counts, ff, k, form, act):
     finally:
         ops.set_grouped_linear_form(0)
     assert float((out.cpu()[rows] - want).abs().max()) <= 2.0**-8 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("experts", [[0, 1] * 20, [2, -1, 0, 0, -1, 1, 2, 2, 2, 2, 2, 0], [1] * 9 + [0] + [1] * 4])
+@pytest.mark.parametrize("form", [0, 3, 4])
+def test_tiles_in_any_order(experts, form):
+    """Tiles that no plan put in order: an expert's tiles apart from each other, unused ones between them."""
+    from vllm_legacy_amd import _seq_ops as ops
+    n, k, E, dtype = 72, 128, 3, torch.bfloat16
+    rows = 32 * len(experts)
+    a, w = rnd((rows, k), 2).to(dtype), rnd((E, 2 * n, k), 3, k**-0.5).to(dtype)
+    want = torch.stack([w[max(e, 0)].to(F) @ a[32 * i:32 * i + 32].to(F).t() for i, e in enumerate(experts)]).transpose(1, 2)
+    used = torch.tensor(experts) >= 0
+    tile_expert = torch.tensor(experts, dtype=torch.int32, device=DEV)
+    ops.set_grouped_linear_form(form)
+    try:
+        y = torch.full((rows, 2 * n), float("nan"), device=DEV)
+        ops.grouped_linear(y, a.to(DEV), None, w.to(DEV), tile_expert)
+        z = torch.full((rows, n), float("nan"), dtype=dtype, device=DEV)
+        ops.grouped_glu(z, a.to(DEV), None, w.to(DEV), tile_expert, "silu")
+    finally:
+        ops.set_grouped_linear_form(0)
+    y, z = y.cpu().view(-1, 32, 2 * n), z.cpu().view(-1, 32, n)
+    assert float((y - want)[used].abs().max()) <= 1e-5 * float(want.abs().max())
+    glu = act_of(want[..., :n], "silu") * want[..., n:]
+    assert float((z - glu)[used].abs().max()) <= 2.0**-8 * float(glu.abs().max())
+    assert bool(y[~used].isnan().all() and z[~used].isnan().all())          # unused tiles are left alone

@@ -454,8 +454,8 @@ __device__ __forceinline__ void store4(typename SO::T* to, const float (&v)[4], 
 }
 
 // The run of at most kRunRows row tiles of one expert that is number `want` among all such runs: (first tile,
-// count), count 0 behind the last.  An expert's tiles are neighbours, so runs start at every kRunRows-th
-// tile from an expert's first one; every wave scans the tiles' experts for itself.
+// count), count 0 behind the last.  Runs start at every kRunRows-th tile from the first of neighbours that have
+// the same expert; every wave scans the tiles' experts for itself.
 __device__ __forceinline__ int2 find_run(const int* __restrict__ tile_expert, int max_tiles, int want) {
   const int lane = threadIdx.x & 63;
   int seen = 0, first = 0;                                 // runs before this stretch of 64; its expert's first tile
@@ -507,104 +507,110 @@ __global__ __launch_bounds__(512, 2) void grouped_dma_kernel(GroupedDma a) {
   const int width = min(8, a.col_tiles - 8 * cb);
   const int64_t rest = id - cb * wide;
   const int col = 8 * cb + (int)(rest % width);
-  const int2 run = find_run(a.tile_expert, a.max_tiles, (int)(rest / width));
-  if (run.y == 0) return;
-  const int e = a.tile_expert[run.x];
   const int n0 = col * (GLU ? 128 : 256);
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hf = lane >> 5, c = lane & 31, wm = w & 1, wn = w >> 1;
-  const int rows = run.y * kTile;
-
-  // wave w brings 16 rows and 32 weight rows, eight per instruction
-  const unsigned char* src_a[2];
-  const unsigned char* src_w[4];
-  const int64_t weight_rows = (int64_t)(GLU ? 2 : 1) * a.n_out;
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int r = 16 * w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
-    const int row = run.x * kTile + min(r, rows - 1);
-    const int src = a.row_token != nullptr ? max(0, a.row_token[row]) : row;     // padding reads token 0
-    src_a[u] = (const unsigned char*)a.a + (int64_t)src * a.a_stride * 2 + 16 * piece;
-  }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int r = 32 * w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
-    const int n = GLU ? (r < 128 ? min(n0 + r, a.n_out - 1) : a.n_out + min(n0 + r - 128, a.n_out - 1)) : min(n0 + r, a.n_out - 1);
-    src_w[u] = (const unsigned char*)a.weight + ((int64_t)e * weight_rows + n) * a.k_in * 2 + 16 * piece;
-  }
   const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
-  auto bring = [&](int step, int buf) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) moe_dma16(src_a[u] + step * (2 * kStep), lds0 + buf * STAGE + w * 2048 + 1024 * u);
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      moe_dma16(src_w[u] + step * (2 * kStep), lds0 + buf * STAGE + ROWS * 128 + w * 4096 + 1024 * u);
-  };
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
   const int x = hf ^ ((c >> 1) & 7);                       // piece 2 ks + hf stands at (2 ks) ^ x
-  const bool active = 64 * wm < rows;
   const int steps = a.k_in / kStep;
-  bring(0, 0);
-  if (steps > 1) bring(1, 1);
-  int buf = 0;
-  for (int it = 0; it < steps; ++it) {
-    if (it + 1 < steps)
-      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");      // all but the next stage
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (it + 2 < steps) bring(it + 2, buf >= 1 ? buf - 1 : RING - 1);
-    const unsigned char* stage = smem + buf * STAGE;
-    buf = buf + 1 < RING ? buf + 1 : 0;
-    if (!active) continue;
-    const unsigned char* a_lds = stage + (64 * wm + c) * 128;
-    const unsigned char* w_lds = stage + ROWS * 128 + ((GLU ? 32 : 64) * wn + c) * 128;
-#pragma unroll
-    for (int ks = 0; ks < kStep / 16; ++ks) {
-      u32x4 av[2], wv[2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        av[b] = *reinterpret_cast<const u32x4*>(a_lds + b * 32 * 128 + 16 * ((2 * ks) ^ x));
-        wv[b] = *reinterpret_cast<const u32x4*>(w_lds + b * (GLU ? 128 : 32) * 128 + 16 * ((2 * ks) ^ x));
-      }
-#pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = Mma16<S>::run(wv[nb], av[mb], acc[mb][nb]);
-    }
-  }
   const bool vec = a.out_stride % 4 == 0 && (uintptr_t)a.out % 16 == 0;
+  // one run per workgroup; those of the last number, which has no run while an expert's tiles are neighbours, take
+  // all that are left
+  for (int64_t want = rest / width;; ++want) {
+    const int2 run = find_run(a.tile_expert, a.max_tiles, (int)want);
+    if (run.y == 0) return;
+    const int e = a.tile_expert[run.x];
+    const int rows = run.y * kTile;
+
+    // wave w brings 16 rows and 32 weight rows, eight per instruction
+    const unsigned char* src_a[2];
+    const unsigned char* src_w[4];
+    const int64_t weight_rows = (int64_t)(GLU ? 2 : 1) * a.n_out;
 #pragma unroll
-  for (int mb = 0; mb < 2; ++mb) {
-    const int r = 64 * wm + 32 * mb + c;
-    if (r >= rows) continue;
-    const int row = run.x * kTile + r;
-    const bool live = a.row_token == nullptr || a.row_token[row] >= 0;
-    // a padding row leaves what zeros would; its scale was never written
-    const float sc = live ? (a.row_scale != nullptr ? a.row_scale[row] : 1.f) : 0.f;
-    typename SO::T* to = (typename SO::T*)a.out + (int64_t)row * a.out_stride;
+    for (int u = 0; u < 2; ++u) {
+      const int r = 16 * w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
+      const int row = run.x * kTile + min(r, rows - 1);
+      const int src = a.row_token != nullptr ? max(0, a.row_token[row]) : row;     // padding reads token 0
+      src_a[u] = (const unsigned char*)a.a + (int64_t)src * a.a_stride * 2 + 16 * piece;
+    }
 #pragma unroll
-    for (int nb = 0; nb < (GLU ? 1 : 2); ++nb)
+    for (int u = 0; u < 4; ++u) {
+      const int r = 32 * w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
+      const int n = GLU ? (r < 128 ? min(n0 + r, a.n_out - 1) : a.n_out + min(n0 + r - 128, a.n_out - 1)) : min(n0 + r, a.n_out - 1);
+      src_w[u] = (const unsigned char*)a.weight + ((int64_t)e * weight_rows + n) * a.k_in * 2 + 16 * piece;
+    }
+    auto bring = [&](int step, int buf) {
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int n = n0 + (GLU ? 32 * wn : 64 * wn + 32 * nb) + 8 * i4 + 4 * hf;
-        float v[4];
+      for (int u = 0; u < 2; ++u) moe_dma16(src_a[u] + step * (2 * kStep), lds0 + buf * STAGE + w * 2048 + 1024 * u);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float z = live ? acc[mb][nb][4 * i4 + k] * sc : 0.f;
-          if constexpr (GLU)
-            v[k] = glu_apply(z, live ? acc[mb][1][4 * i4 + k] * sc : 0.f, a);
-          else
-            v[k] = act_apply(z, a.act);
+      for (int u = 0; u < 4; ++u)
+        moe_dma16(src_w[u] + step * (2 * kStep), lds0 + buf * STAGE + ROWS * 128 + w * 4096 + 1024 * u);
+    };
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
+    const bool active = 64 * wm < rows;
+    bring(0, 0);
+    if (steps > 1) bring(1, 1);
+    int buf = 0;
+    for (int it = 0; it < steps; ++it) {
+      if (it + 1 < steps)
+        asm volatile("s_waitcnt vmcnt(6)" ::: "memory");      // all but the next stage
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (it + 2 < steps) bring(it + 2, buf >= 1 ? buf - 1 : RING - 1);
+      const unsigned char* stage = smem + buf * STAGE;
+      buf = buf + 1 < RING ? buf + 1 : 0;
+      if (!active) continue;
+      const unsigned char* a_lds = stage + (64 * wm + c) * 128;
+      const unsigned char* w_lds = stage + ROWS * 128 + ((GLU ? 32 : 64) * wn + c) * 128;
+#pragma unroll
+      for (int ks = 0; ks < kStep / 16; ++ks) {
+        u32x4 av[2], wv[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          av[b] = *reinterpret_cast<const u32x4*>(a_lds + b * 32 * 128 + 16 * ((2 * ks) ^ x));
+          wv[b] = *reinterpret_cast<const u32x4*>(w_lds + b * (GLU ? 128 : 32) * 128 + 16 * ((2 * ks) ^ x));
         }
-        store4<SO>(to + n, v, n, a.n_out, vec);
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+          for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = Mma16<S>::run(wv[nb], av[mb], acc[mb][nb]);
       }
+    }
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+      const int r = 64 * wm + 32 * mb + c;
+      if (r >= rows) continue;
+      const int row = run.x * kTile + r;
+      const bool live = a.row_token == nullptr || a.row_token[row] >= 0;
+      // a padding row leaves what zeros would; its scale was never written
+      const float sc = live ? (a.row_scale != nullptr ? a.row_scale[row] : 1.f) : 0.f;
+      typename SO::T* to = (typename SO::T*)a.out + (int64_t)row * a.out_stride;
+#pragma unroll
+      for (int nb = 0; nb < (GLU ? 1 : 2); ++nb)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const int n = n0 + (GLU ? 32 * wn : 64 * wn + 32 * nb) + 8 * i4 + 4 * hf;
+          float v[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float z = live ? acc[mb][nb][4 * i4 + k] * sc : 0.f;
+            if constexpr (GLU)
+              v[k] = glu_apply(z, live ? acc[mb][1][4 * i4 + k] * sc : 0.f, a);
+            else
+              v[k] = act_apply(z, a.act);
+          }
+          store4<SO>(to + n, v, n, a.n_out, vec);
+        }
+    }
+    if (want + 1 < a.groups) return;
+    __syncthreads();                                       // the stages are read
   }
 }
 
@@ -746,7 +752,8 @@ int launch_grouped_dma(GroupedDma a, int num_experts, bool few, hipStream_t stre
     }
     const int cols = GLU ? 128 : 256;
     a.col_tiles = (a.n_out + cols - 1) / cols;
-    // every expert adds at most one run that is not full
+    // where an expert's tiles are neighbours (as moe_plan leaves them) it adds at most one run that is not full, and
+    // the last number has none; tiles in another order are more runs, which the workgroups of that number walk
     a.groups = a.max_tiles / kRunRows + std::min(num_experts, a.max_tiles) + 1;
     const int64_t total = a.groups * a.col_tiles;
     grouped_dma_kernel<S, SO, GLU><<<(unsigned)((total + 7) / 8 * 8), 512, lds, stream>>>(a);
