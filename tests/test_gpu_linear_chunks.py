@@ -77,3 +77,46 @@ def test_rows_at_odd_addresses_go_the_other_way(offset):
     rows = torch.empty((100, 200), dtype=torch.bfloat16, device=DEV)[:, :64]
     assert ops.gla_chunks_scratch(rows, rows, rows, 2, 24, 32, 3, 1) == 0
     assert ops.gla_chunks_scratch(rows, rows, rows, 2, 32, 32, 33, 1) == 0
+
+
+@pytest.mark.parametrize("what,value", [("v", float("inf")), ("v", float("nan")), ("k", float("-inf")), ("y", float("nan")),
+                                        ("q", float("inf"))])
+@pytest.mark.parametrize("row", [0, 5, 15, 16, 63, 64, 100, 129])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_ahead_of_one_that_is_not_finite(what, value, row, dtype):
+    """Bit for bit what they are without it, as token by token; it and the rows behind it are not finite exactly
+    where a walk in float64 says so; other heads and sequences know nothing of it."""
+    from vllm_legacy_amd.attention.batch import SequenceBatch
+    from vllm_legacy_amd.attention.recurrent import GatedLinearRecurrence
+    H, D, V, rank, lens = 2, 32, 48, 3, [130, 70]
+    T, g = sum(lens), torch.Generator().manual_seed(row)
+    layer = GatedLinearRecurrence(H, D, V, 5.0, 1e-5)
+    rows = {"q": H * D, "k": H * D, "v": H * V, "gate": H * V, "y": rank}
+    rows = {name: torch.randn(T, n, generator=g).to(dtype) for name, n in rows.items()}
+    w2, bias, norm_w = torch.randn(H * D, rank, generator=g).to(dtype), torch.randn(H * D, generator=g) + 2, torch.ones(V)
+    b = SequenceBatch.build(lens, [0, 0], [[0] * 64] * 2, [0, 1], 16, DEV)
+
+    def go(r):
+        state = torch.zeros(GatedLinearRecurrence.get_state_shape(2, H, D, V), device=DEV)
+        out = torch.empty(T, H * V, device=DEV, dtype=dtype)
+        layer(out, *(r[name].to(DEV) for name in ("q", "k", "v", "gate", "y")), w2.to(DEV), bias.to(DEV), norm_w.to(DEV), state, b,
+              1.0)
+        return out.float().cpu().view(T, H, V), state.cpu()
+
+    clean, clean_state = go(rows)
+    rows[what] = rows[what].clone()
+    rows[what][row, 1] = value                  # head 0 (a decay's row: both heads)
+    got, state = go(rows)
+    assert torch.equal(got[:row], clean[:row]) and torch.equal(got[lens[0]:], clean[lens[0]:])
+    assert torch.equal(state[1], clean_state[1])
+    if what != "y":
+        assert torch.equal(got[:, 1], clean[:, 1]) and torch.equal(state[0, 1], clean_state[0, 1])
+    q, k, v, y = (rows[name].to(R.F)[:lens[0]] for name in ("q", "k", "v", "y"))
+    a = torch.exp(R.log_decay(y, w2.to(R.F), bias.to(R.F), 5.0)).view(-1, H, D)
+    S, o = torch.zeros(H, D, V, dtype=R.F), torch.empty(lens[0], H, V, dtype=R.F)
+    for t in range(lens[0]):
+        S = a[t][:, :, None] * S + k[t].view(H, D, 1) * v[t].view(H, 1, V)
+        o[t] = (S * q[t].view(H, D, 1)).sum(1)
+    want = R.gated_head_norm(o, norm_w.to(R.F), rows["gate"].to(R.F)[:lens[0]], 1e-5, 1.0).reshape(-1, H, V)
+    assert torch.equal(got[:lens[0]].isfinite(), want.isfinite())
+    assert torch.equal(state[0].isfinite(), S.isfinite())

@@ -120,6 +120,8 @@ __device__ __forceinline__ f32x4 load4(const typename S::T* row, int d, int dim,
   return r;
 }
 
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) <= 3.402823466e38f; }
+
 __device__ __forceinline__ float softplusf(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 
 }  // namespace seq

@@ -365,13 +365,16 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
   for (int x = 0; x < 8; ++x)
     if (4 * quarter + 16 * x < V) held[x] = row4<S>(vr + 4 * quarter + 16 * x);
   __syncthreads();
+  bool odd = false;
 #pragma unroll
   for (int x = 0; x < 8; ++x)
     if (4 * quarter + 16 * x < V) {
       if (!live) held[x] = f32x4{0.f, 0.f, 0.f, 0.f};
       *reinterpret_cast<f32x4*>(v_lds + row * VR + 4 * quarter + 16 * x) = held[x];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) odd |= !finite(held[x][e]);
     }
-  __syncthreads();
+  const bool some_bad = __syncthreads_or(odd);
 
   f32x4 acc[8];
   f32x4 qs[DT];
@@ -389,15 +392,30 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
       f32x4 sv[DT];
 #pragma unroll
       for (int x = 0; x < DT; ++x) sv[x] = *reinterpret_cast<const f32x4*>(s_in + ((int64_t)(x * vt_n + vt) * 64 + lane) * 4);
-      for (int o = 0; o <= w; ++o) {
+      for (int o = 0; o < w; ++o) {
         const f32x4 am = *reinterpret_cast<const f32x4*>(a_mat + (kBlock * w + c) * kAMat + kBlock * o + 4 * g);
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[vt] = mfma4(am[e], v_lds[(kBlock * o + 4 * g + e) * VR + 16 * vt + c], acc[vt]);
       }
+      // A row's product with the rows behind it is 0 times their values, which must be finite for that; and a column
+      // in which one was not stays so, as it does in the state of a walk.
+      int bad = kBlock;                                    // the block's first such row in column c
+      if (some_bad) {
+        for (int j = kBlock * (w + 1) - 1; j >= 0; --j)
+          if (!finite(v_lds[j * VR + 16 * vt + c])) bad = max(j - kBlock * w, 0);
+      }
+      const f32x4 am = *reinterpret_cast<const f32x4*>(a_mat + (kBlock * w + c) * kAMat + kBlock * w + 4 * g);
+      f32x4 vv;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vv[e] = v_lds[(kBlock * w + 4 * g + e) * VR + 16 * vt + c];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[vt] = mfma4(am[e], 4 * g + e < bad ? vv[e] : 0.f, acc[vt]);
 #pragma unroll
       for (int x = 0; x < DT; ++x)
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[vt] = mfma4(qs[x][e], sv[x][e], acc[vt]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[vt][e] = 4 * g + e < bad ? acc[vt][e] : NAN;
 #pragma unroll
       for (int e = 0; e < 4; ++e) ss[e] += acc[vt][e] * acc[vt][e];
     }
