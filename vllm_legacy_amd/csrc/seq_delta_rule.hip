@@ -408,10 +408,16 @@ __device__ __forceinline__ bool find_delta_block(const DeltaBlocks& a, int slot,
   return block >= 0 && block * kRows < a.query_start_loc[b + 1] - a.query_start_loc[b];
 }
 
-// LDS of the prepare kernel: unit keys and queries, then the waves' partial products, whose place the
-// 32 x 32 matrices take, then L (column 32: G), decays and betas
+// LDS of the prepare kernel: keys and queries, then the waves' partial products, whose place the
+// 32 x 32 matrices take, then L (column 32: G), decays, betas and what makes keys and queries unit rows
 __host__ __device__ constexpr size_t delta_prepare_lds_floats(int dp) {
-  return (size_t)2 * kRows * (dp + 4) + 4 * 6 * 256 + kRows * kMat + 2 * kRows;
+  return (size_t)2 * kRows * (dp + 4) + 4 * 6 * 256 + kRows * kMat + 4 * kRows;
+}
+
+// one 16x16x4 matrix-core step in 64 bits: operands as mfma4's, lane (g, c) ends with column c, rows g + 4 i
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f64x4 mfma4_f64(double a, double b, f64x4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
 template <int DX>
@@ -427,6 +433,8 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
   float* l_mat = part + 4 * 6 * 256;                       // [32][kMat]
   float* g_lds = l_mat + kRows * kMat;                     // [32]
   float* beta_lds = g_lds + kRows;                         // [32]
+  float* ks_lds = beta_lds + kRows;                        // [32]
+  float* qs_lds = ks_lds + kRows;                          // [32]
   const int slot = blockIdx.x, h = blockIdx.y;
   int b, block;
   if (!find_delta_block(a, slot, b, block)) return;
@@ -459,7 +467,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
       }
   };
 
-  // unit rows (zeros behind the run's end), decays and betas: every load ahead of everything else, and
+  // rows (zeros behind the run's end) and their factors, decays and betas: every load ahead of everything else, and
   // none behind a branch of its own
   f32x4 qv[2 * DX], kv[2 * DX];
   float v_a[2][4], v_b[2][4];
@@ -510,17 +518,26 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
     for (int x = 0; x < 2 * DX; ++x) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        qv[x][e] *= qs;
-        kv[x][e] *= ks;
+        qv[x][e] = live ? qv[x][e] : 0.f;
+        kv[x][e] = live ? kv[x][e] : 0.f;
       }
       *reinterpret_cast<f32x4*>(q_lds + row * RS + 4 * eighth + 32 * x) = qv[x];
       *reinterpret_cast<f32x4*>(k_lds + row * RS + 4 * eighth + 32 * x) = kv[x];
+    }
+    if (eighth == 0) {
+      ks_lds[row] = ks;
+      qs_lds[row] = qs;
     }
   }
   __syncthreads();
 
   // k_i . k_j and q_i . k_j, lower 16 x 16 tiles; every wave takes a quarter of the head's rows (a lane
-  // holds four neighbouring ones: the contraction index may be relabelled as long as both operands are)
+  // holds four neighbouring ones: the contraction index may be relabelled as long as both operands are).  In 64
+  // bits and of the rows as they are, and L in 64 bits too: an error in one of them is in all columns of u alike
+  // and, where keys are alike, in every u behind it.  Relative errors against 64 bits of outputs / states after
+  // 1024 rows of 128 x 128 with slow decays, in 1e-7: token by token, this, and unit rows in 32 bits:
+  // independent keys 1.9 / 1.7, 1.9 / 1.8, 2.4 / 2.2; keys with a common part as large as the rest 2.0 / 1.9,
+  // 2.2 / 2.2, 2.9 / 2.7; with one three times as large 2.5 / 2.1, 3.0 / 3.3, 4.4 / 4.1.
   {
     // L: lane j of wave 0 walks down column j (lane 32: from the block's start)
     if (w == 0) {
@@ -528,18 +545,18 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
 #pragma unroll
       for (int i = 0; i < kRows / 4; ++i) gv[i] = *reinterpret_cast<const f32x4*>(g_lds + 4 * i);
       const int j = lane < kRows ? lane : -1;
-      float r = 1.f;
+      double r = 1.;
       if (lane <= kRows) {
 #pragma unroll
         for (int i = 0; i < kRows; ++i) {
-          r *= i > j ? gv[i >> 2][i & 3] : 1.f;
-          l_mat[i * kMat + lane] = r;
+          r *= i > j ? (double)gv[i >> 2][i & 3] : 1.;
+          l_mat[i * kMat + lane] = (float)r;
         }
       }
     }
-    f32x4 acc[6];
+    f64x4 acc[6];
 #pragma unroll
-    for (int i = 0; i < 6; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 6; ++i) acc[i] = f64x4{0., 0., 0., 0.};
 #pragma unroll
     for (int x = 0; x < DX; ++x) {
       const int d = 16 * (w * DX + x) + 4 * g;
@@ -551,34 +568,38 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
       qv[DX + x] = q1;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        acc[0] = mfma4(k0[e], k0[e], acc[0]);
-        acc[1] = mfma4(k1[e], k0[e], acc[1]);
-        acc[2] = mfma4(k1[e], k1[e], acc[2]);
-        acc[3] = mfma4(q0[e], k0[e], acc[3]);
-        acc[4] = mfma4(q1[e], k0[e], acc[4]);
-        acc[5] = mfma4(q1[e], k1[e], acc[5]);
+        const double k0d = k0[e], k1d = k1[e], q0d = q0[e], q1d = q1[e];
+        acc[0] = mfma4_f64(k0d, k0d, acc[0]);
+        acc[1] = mfma4_f64(k1d, k0d, acc[1]);
+        acc[2] = mfma4_f64(k1d, k1d, acc[2]);
+        acc[3] = mfma4_f64(q0d, k0d, acc[3]);
+        acc[4] = mfma4_f64(q1d, k0d, acc[4]);
+        acc[5] = mfma4_f64(q1d, k1d, acc[5]);
       }
     }
+    // [tile][lane of mfma4's result][4]
 #pragma unroll
-    for (int i = 0; i < 6; ++i) *reinterpret_cast<f32x4*>(part + ((w * 6 + i) * 64 + lane) * 4) = acc[i];
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part[((w * 6 + i) * 64 + 16 * e + c) * 4 + g] = (float)acc[i][e];
   }
   __syncthreads();
-  f32x4 sum[2];
+  f64x4 sum[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int at = min(tid + 256 * u, 6 * 64 - 1);
-    sum[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    sum[u] = f64x4{0., 0., 0., 0.};
 #pragma unroll
     for (int ow = 0; ow < 4; ++ow) {
       const f32x4 got = *reinterpret_cast<const f32x4*>(part + (ow * 6 * 64 + at) * 4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sum[u][e] += got[e];
+      for (int e = 0; e < 4; ++e) sum[u][e] += (double)got[e];
     }
   }
   // Q~, from the operands of the products above
 #pragma unroll
   for (int it = 0; it < 2; ++it) {
-    const float gq = l_mat[(16 * it + c) * kMat + kRows];
+    const float gq = l_mat[(16 * it + c) * kMat + kRows] * qs_lds[16 * it + c];
 #pragma unroll
     for (int x = 0; x < DX; ++x) {
       const f32x4 q4 = qv[it * DX + x];
@@ -594,7 +615,10 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
       const int i0 = kind > 0 ? 16 : 0, j0 = kind > 1 ? 16 : 0, j = j0 + c;
       float v[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = sum[u][e] * l_mat[(i0 + 4 * g + e) * kMat + j];
+      for (int e = 0; e < 4; ++e) {
+        const double unit = sum[u][e] * (double)(tile < 3 ? ks_lds : qs_lds)[i0 + 4 * g + e] * (double)ks_lds[j];
+        v[e] = (float)(unit * (double)l_mat[(i0 + 4 * g + e) * kMat + j]);
+      }
       if (tile < 3) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -653,9 +677,10 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
     for (int i = tid - 128; i < DP * (kRows / 4); i += 128) {
       const int d = 16 * (i >> 7) + (i & 15), j = 4 * ((i >> 4) & 7);    // i: tile, half, lane
       const f32x4 lv = *reinterpret_cast<const f32x4*>(l_mat + (kRows - 1) * kMat + j);
+      const f32x4 ks = *reinterpret_cast<const f32x4*>(ks_lds + j);
       f32x4 kh;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) kh[e] = k_lds[(j + e) * RS + d] * lv[e];
+      for (int e = 0; e < 4; ++e) kh[e] = (float)((double)lv[e] * (double)ks[e] * (double)k_lds[(j + e) * RS + d]);
       *reinterpret_cast<f32x4*>(k_out + 4 * i) = kh;
     }
   }
@@ -695,7 +720,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
 #pragma unroll
   for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) gj[jt][e] = l_mat[(16 * jt + 4 * g + e) * kMat + kRows];
+    for (int e = 0; e < 4; ++e) gj[jt][e] = l_mat[(16 * jt + 4 * g + e) * kMat + kRows] * ks_lds[16 * jt + 4 * g + e];
 #pragma unroll
   for (int x = 0; x < DX; ++x) {
     const int tile = w + 4 * x;
@@ -840,16 +865,16 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         u[it][e] = f.u[it][e] - ((p[it][0][e] + p[it][1][e]) + (p[it][2][e] + p[it][3][e]));
+    // what the block adds is summed by itself: one rounding of the state per block
+    f32x4 ds[DX];
 #pragma unroll
-    for (int x = 0; x < DX; ++x)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[x][e] *= f.g_last;
+    for (int x = 0; x < DX; ++x) ds[x] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int it = 0; it < 2; ++it)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int x = 0; x < DX; ++x) s[x] = mfma4(f.kv[x][it][e], u[it][e], s[x]);
+        for (int x = 0; x < DX; ++x) ds[x] = mfma4(f.kv[x][it][e], u[it][e], ds[x]);
     // A U: the wave takes contraction index 4 g + w, so that the sum over waves is the whole product
     const float u0 = w == 0 ? u[0][0] : w == 1 ? u[0][1] : w == 2 ? u[0][2] : u[0][3];
     const float u1 = w == 0 ? u[1][0] : w == 1 ? u[1][1] : w == 2 ? u[1][2] : u[1][3];
@@ -860,6 +885,10 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
     for (int it = 0; it < 2; ++it)
 #pragma unroll
       for (int e = 0; e < 4; ++e) o_part[buf][w][it][e][lane] = xo[it][e];
+#pragma unroll
+    for (int x = 0; x < DX; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[x][e] = f.g_last * s[x][e] + ds[x][e];
   };
   // two blocks in turn, so that one is asked for while the other is worked on
   Block f0, f1;
