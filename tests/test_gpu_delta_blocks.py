@@ -88,3 +88,43 @@ def test_as_close_to_64_bits_as_token_by_token(common, outputs, states):
         errors.append([float((x.to(F) - want).norm() / want.norm())
                        for x, want in ((out.view(n, H, V), o), (state[0].transpose(1, 2), S))])
     assert errors[1][0] <= outputs * errors[0][0] and errors[1][1] <= states * errors[0][1], errors
+
+
+@pytest.mark.parametrize("what,value", [("v", float("inf")), ("v", float("nan")), ("k", float("-inf")), ("k", float("nan")),
+                                        ("beta", float("nan")), ("dt", float("nan")), ("q", float("inf"))])
+@pytest.mark.parametrize("row", [0, 3, 15, 16, 22, 31, 32, 60, 65])
+@pytest.mark.parametrize("V", [128, 40])
+def test_rows_ahead_of_one_that_is_not_finite(what, value, row, V):
+    """Bit for bit what they are without it, as token by token; the rows behind it are not finite exactly where
+    the walk says so, and it itself nowhere (an infinity among a row's outputs leaves zeros beside it in the walk);
+    other heads, columns and sequences know nothing of it."""
+    from vllm_legacy_amd import _seq_ops as ops
+    H, D, lens = 2, 64, [66, 40]
+    n = sum(lens)
+    rows = {"q": H * D, "k": H * D, "v": H * V, "gate": H * V, "beta": H, "dt": H}
+    rows = {name: rnd((n, w), i) for i, (name, w) in enumerate(rows.items())}
+    batch = make_batch(lens, [0, 0], slots=[0, 1])
+    zero, one = torch.zeros(H, device=DEV), torch.ones(V, device=DEV)
+
+    def go(kernel=0):
+        out, state = torch.empty((n, H * V), device=DEV), torch.zeros((2, H, V, D), device=DEV)
+        ops.set_delta_kernel(kernel)
+        try:
+            ops.delta_rule_scan(out, *(rows[x].to(DEV) for x in ("q", "k", "v", "gate", "beta", "dt")), zero, zero, one, state,
+                                batch.query_start_loc, batch.context_lens, batch.state_slots, H, 1e-5, max(lens))
+        finally:
+            ops.set_delta_kernel(0)
+        return out.cpu().view(n, H, V), state.cpu()
+
+    clean, clean_state = go()
+    rows[what] = rows[what].clone()
+    rows[what][row, 0 if what in ("beta", "dt") else 1] = value                 # head 0
+    got, state = go()
+    want, want_state = go(2)
+    assert torch.equal(got[:row], clean[:row]) and torch.equal(got[lens[0]:], clean[lens[0]:])
+    assert torch.equal(got[:, 1], clean[:, 1]) and torch.equal(state[0, 1], clean_state[0, 1])
+    assert torch.equal(state[1], clean_state[1])
+    got, want = got.isfinite(), want.isfinite()
+    assert not got[row, 0].any() and not want[row, 0].all()
+    got[row, 0] = want[row, 0]
+    assert torch.equal(got, want) and torch.equal(state.isfinite(), want_state.isfinite())

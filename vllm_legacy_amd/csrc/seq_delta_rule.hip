@@ -388,9 +388,9 @@ struct DeltaBlocks {
 // A block's operands lie in scratch as the walk's waves take them, lane for lane: [16 x 16 tile][lane][4].
 // (Lanes side by side in memory matter: with lanes 64 bytes apart the walk below took 192 us.)
 // Floats of a block's scratch: W | Q~ | K^ (each 32 x DP) | G_31 and a place for stores nobody wants
-// (padded to 4) | A (its three lower 16 x 16 tiles) | T V (32 x VP)
+// (padded to 4) | A (its three lower 16 x 16 tiles) | T V (32 x VP) | from which row on a column is not finite (VP)
 __host__ __device__ __forceinline__ int64_t delta_block_floats(int dp, int vp) {
-  return (int64_t)3 * kRows * dp + 4 + 3 * 256 + kRows * vp;
+  return (int64_t)3 * kRows * dp + 4 + 3 * 256 + kRows * vp + vp;
 }
 
 // Which sequence and block a block slot is: sequence b's blocks are slots start_b / 32 + b + 0, 1, ...
@@ -409,9 +409,10 @@ __device__ __forceinline__ bool find_delta_block(const DeltaBlocks& a, int slot,
 }
 
 // LDS of the prepare kernel: keys and queries, then the waves' partial products, whose place the
-// 32 x 32 matrices take, then L (column 32: G), decays, betas and what makes keys and queries unit rows
+// 32 x 32 matrices take, then L (column 32: G), decays, betas, what makes keys and queries unit rows, and
+// which rows are not finite
 __host__ __device__ constexpr size_t delta_prepare_lds_floats(int dp) {
-  return (size_t)2 * kRows * (dp + 4) + 4 * 6 * 256 + kRows * kMat + 4 * kRows;
+  return (size_t)2 * kRows * (dp + 4) + 4 * 6 * 256 + kRows * kMat + 6 * kRows;
 }
 
 // one 16x16x4 matrix-core step in 64 bits: operands as mfma4's, lane (g, c) ends with column c, rows g + 4 i
@@ -435,6 +436,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
   float* beta_lds = g_lds + kRows;                         // [32]
   float* ks_lds = beta_lds + kRows;                        // [32]
   float* qs_lds = ks_lds + kRows;                          // [32]
+  float* odd_lds = qs_lds + kRows;                         // [2][32]: decay or beta, key
   const int slot = blockIdx.x, h = blockIdx.y;
   int b, block;
   if (!find_delta_block(a, slot, b, block)) return;
@@ -498,28 +500,36 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
     }
     fetch_v(v_a, min(w, vb - 1));
     fetch_v(v_b, min(w + 4, vb - 1));
+    // Rows with a key, decay or beta that is not finite take no part in the products, where 0 times them would
+    // reach the rows ahead of them; U of the first of them and of all rows behind it is NaN.
     if (tid < kRows) {
-      g_lds[tid] = tid < n ? expf(-expf(al) * softplusf(z)) : 1.f;
-      beta_lds[tid] = tid < n ? 1.f / (1.f + expf(-bt)) : 0.f;
+      const float gd = expf(-expf(al) * softplusf(z)), be = 1.f / (1.f + expf(-bt));
+      const bool odd = tid < n && !(finite(gd) && finite(be));
+      g_lds[tid] = tid < n && !odd ? gd : 1.f;
+      beta_lds[tid] = tid < n && !odd ? be : 0.f;
+      odd_lds[tid] = odd ? 1.f : 0.f;
     }
-    float qq = 0.f, kk = 0.f;
+    float qq = 0.f, kk = 0.f, odd = 0.f, none = 0.f;
 #pragma unroll
     for (int x = 0; x < 2 * DX; ++x)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         if (4 * eighth + 32 * x + e >= D) qv[x][e] = kv[x][e] = 0.f;
+        odd = finite(kv[x][e]) ? odd : 1.f;
         qq += qv[x][e] * qv[x][e];
         kk += kv[x][e] * kv[x][e];
       }
     group_sums(qq, kk, 8);
+    group_sums(odd, none, 8);
     const float qs = live ? 1.f / (sqrtf(qq + 1e-6f) * sqrtf((float)D)) : 0.f;
-    const float ks = live ? 1.f / sqrtf(kk + 1e-6f) : 0.f;
+    const bool whole = live && finite(kk);               // (a sum that overflows makes a unit row of zeros)
+    const float ks = whole ? 1.f / sqrtf(kk + 1e-6f) : 0.f;
 #pragma unroll
     for (int x = 0; x < 2 * DX; ++x) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         qv[x][e] = live ? qv[x][e] : 0.f;
-        kv[x][e] = live ? kv[x][e] : 0.f;
+        kv[x][e] = whole ? kv[x][e] : 0.f;
       }
       *reinterpret_cast<f32x4*>(q_lds + row * RS + 4 * eighth + 32 * x) = qv[x];
       *reinterpret_cast<f32x4*>(k_lds + row * RS + 4 * eighth + 32 * x) = kv[x];
@@ -527,9 +537,12 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
     if (eighth == 0) {
       ks_lds[row] = ks;
       qs_lds[row] = qs;
+      odd_lds[kRows + row] = live ? odd : 0.f;
     }
   }
   __syncthreads();
+  const uint64_t odd_rows = __ballot(lane < kRows && odd_lds[lane & 31] + odd_lds[kRows + (lane & 31)] > 0.f);
+  const int odd_from = odd_rows ? __builtin_ctzll(odd_rows) : kRows;
 
   // k_i . k_j and q_i . k_j, lower 16 x 16 tiles; every wave takes a quarter of the head's rows (a lane
   // holds four neighbouring ones: the contraction index may be relabelled as long as both operands are).  In 64
@@ -741,6 +754,20 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
       *reinterpret_cast<f32x4*>(w_out + ((tile * 2 + it) * 64 + lane) * 4) = xt[it];
   }
   for (int vt = w; vt < vb; vt += 4) {
+    int from = odd_from;                                   // column c's first row that is not finite
+#pragma unroll
+    for (int it = 0; it < 2; ++it)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!finite(v_a[it][e])) {
+          from = min(from, 16 * it + 4 * g + e);
+          v_a[it][e] = 0.f;
+        }
+    if (__any(from < kRows)) {
+      from = min(from, __shfl_xor(from, 16, 64));
+      from = min(from, __shfl_xor(from, 32, 64));
+    }
+    if (g == 0) u_out[kRows * 16 * vb + 16 * vt + c] = (float)from;
     f32x4 xt[2];
 #pragma unroll
     for (int it = 0; it < 2; ++it) xt[it] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -752,6 +779,8 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
     }
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xt[it][e] = 16 * it + 4 * g + e < from ? xt[it][e] : NAN;
       *reinterpret_cast<f32x4*>(u_out + ((vt * 2 + it) * 64 + lane) * 4) = xt[it];
 #pragma unroll
       for (int e = 0; e < 4; ++e) v_a[it][e] = v_b[it][e];
@@ -796,7 +825,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
   const int blocks = (run + kRows - 1) / kRows;
   struct Block {
     f32x4 wv[DX][2], qv[DX][2], kv[DX][2], u[2];
-    float av[3], g_last;
+    float av[3], g_last, from;
   };
   const int at_x = w * DX * 2 * 256 + 4 * lane, at_a = w * 64 + lane, at_u = blockIdx.y * 2 * 256 + 4 * lane;
   auto fetch = [&](Block& f, const float* p) {
@@ -815,11 +844,15 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
     for (int i = 0; i < 3; ++i) f.av[i] = pa[4 + at_a + 256 * i];
 #pragma unroll
     for (int it = 0; it < 2; ++it) f.u[it] = *reinterpret_cast<const f32x4*>(pa + 4 + 3 * 256 + at_u + 256 * it);
+    f.from = pa[4 + 3 * 256 + kRows * vp + col];
   };
   // wave w finishes rows 16 it + 4 g + w of a block's outputs; what has no place goes to the block's pad
   const int64_t row_step = (int64_t)a.heads * V;
   float* o_at = a.o + ((int64_t)(t_begin + 4 * g + w) * a.heads + h) * V + (col < V ? col : 0);
   float* nowhere = a.scratch + ((int64_t)(t_begin / kRows + b) * a.heads + h) * per + 3 * kRows * DP + 1;
+  // column c is NaN from its first row on that is not finite, as the state that a walk reads it with
+  const float row_w = (float)(4 * g + w);
+  float from = (float)kRows;                               // of the block to finish
   auto finish = [&](int i) {
     const int buf = i & 1;
 #pragma unroll
@@ -827,7 +860,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
       const float o = (o_part[buf][0][it][w][lane] + o_part[buf][1][it][w][lane]) +
                       (o_part[buf][2][it][w][lane] + o_part[buf][3][it][w][lane]);
       const bool live = i * kRows + 16 * it + 4 * g + w < run && col < V;
-      *(live ? o_at + 16 * it * row_step : nowhere) = o;
+      *(live ? o_at + 16 * it * row_step : nowhere) = row_w + 16.f * it < from ? o : NAN;
     }
     o_at += kRows * row_step;
   };
@@ -875,9 +908,13 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int x = 0; x < DX; ++x) ds[x] = mfma4(f.kv[x][it][e], u[it][e], ds[x]);
-    // A U: the wave takes contraction index 4 g + w, so that the sum over waves is the whole product
-    const float u0 = w == 0 ? u[0][0] : w == 1 ? u[0][1] : w == 2 ? u[0][2] : u[0][3];
-    const float u1 = w == 0 ? u[1][0] : w == 1 ? u[1][1] : w == 2 ? u[1][2] : u[1][3];
+    // A U: the wave takes contraction index 4 g + w, so that the sum over waves is the whole product.  A row's product
+    // with the rows behind it is 0 times their U: those that are not finite stay out.
+    float u0 = w == 0 ? u[0][0] : w == 1 ? u[0][1] : w == 2 ? u[0][2] : u[0][3];
+    float u1 = w == 0 ? u[1][0] : w == 1 ? u[1][1] : w == 2 ? u[1][2] : u[1][3];
+    u0 = row_w < f.from ? u0 : 0.f;
+    u1 = row_w + 16.f < f.from ? u1 : 0.f;
+    from = f.from;
     xo[0] = mfma4(f.av[0], u0, xo[0]);
     xo[1] = mfma4(f.av[1], u0, xo[1]);
     xo[1] = mfma4(f.av[2], u1, xo[1]);
