@@ -128,3 +128,23 @@ def test_rows_ahead_of_one_that_is_not_finite(what, value, row, V):
     assert not got[row, 0].any() and not want[row, 0].all()
     got[row, 0] = want[row, 0]
     assert torch.equal(got, want) and torch.equal(state.isfinite(), want_state.isfinite())
+
+
+@pytest.mark.parametrize("rows", [1, 4, 5, 33])
+@pytest.mark.parametrize("hint", [0, 33, 500])
+def test_a_lone_run_shorter_than_the_hint(rows, hint):
+    """max_query_len bounds the rows of a run; how many there are is read on the device."""
+    from vllm_legacy_amd import _seq_ops as ops
+    H, D, V = 2, 64, 48
+    x = {name: rnd((rows, w), i).to(DEV) for i, (name, w) in enumerate(
+        {"q": H * D, "k": H * D, "v": H * V, "gate": H * V, "beta": H, "dt": H}.items())}
+    batch, zero, one = make_batch([rows], [0], slots=[0]), torch.zeros(H, device=DEV), torch.ones(V, device=DEV)
+
+    def go(most):
+        out, state = torch.full((rows, H * V), 7.0, device=DEV), torch.full((1, H, V, D), 7.0, device=DEV)
+        ops.delta_rule_scan(out, *x.values(), zero, zero, one, state, batch.query_start_loc, batch.context_lens,
+                            batch.state_slots, H, 1e-5, most)
+        return out, state
+
+    for got, want in zip(go(hint), go(min(rows, 32))):
+        assert float((got - want).abs().max()) <= 3e-5 * float(want.abs().max())

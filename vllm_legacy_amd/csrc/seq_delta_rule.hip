@@ -382,6 +382,7 @@ struct DeltaBlocks {
   const int* context_lens;
   const int* state_slots;
   int num_seqs, heads, kv_heads, dim, vdim;
+  int step_rows;                    // runs of at most this many rows are the step kernel's
   bool vec_qk, vec_state;
 };
 
@@ -441,7 +442,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
   int b, block;
   if (!find_delta_block(a, slot, b, block)) return;
   const int run = a.query_start_loc[b + 1] - a.query_start_loc[b];
-  if (run <= kStepRows) return;                            // the step kernel's
+  if (run <= a.step_rows) return;
   const int t0 = a.query_start_loc[b] + block * kRows, n = min(kRows, run - block * kRows);
   const int D = a.dim, V = a.vdim, hg = h / (a.heads / a.kv_heads);
   const int vb = (V + 15) / 16;
@@ -805,7 +806,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
   // (and its L2) whenever the number of heads is a multiple of 8
   const int h = blockIdx.x, v0 = 16 * blockIdx.y, b = blockIdx.z;
   const int t_begin = a.query_start_loc[b], run = a.query_start_loc[b + 1] - t_begin;
-  if (run <= kStepRows) return;
+  if (run <= a.step_rows) return;
   const int D = a.dim, V = a.vdim, vp = (V + 15) / 16 * 16;
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1118,6 +1119,7 @@ int delta_rule_scan(
   // runs of at most four rows take the kernel without staging (modes 1 / 2: always / never, for tests)
   const int mode = g_delta_kernel.load(std::memory_order_relaxed);
   const bool blocks = scratch_floats >= 0 && wants_blocks(mode, num_tokens, num_seqs, max_query_len, heads, dim, vdim);
+  // (a lone run goes in blocks however short it is: max_query_len may be more than its rows)
   const bool steps = blocks ? num_seqs > 1 : mode == 1 || (mode == 0 && max_query_len > 0 && max_query_len <= kStepRows);
   const int64_t out_floats = delta_out_floats(num_tokens, heads, vdim);
   if (blocks) {
@@ -1136,6 +1138,7 @@ int delta_rule_scan(
     a.kv_heads = kv_heads;
     a.dim = dim;
     a.vdim = vdim;
+    a.step_rows = steps ? kStepRows : 0;
     auto fours = [&](const void* p, int64_t stride) {              // four values per access
       return dim % 4 == 0 && stride % 4 == 0 && (uintptr_t)p % 16 == 0;
     };
