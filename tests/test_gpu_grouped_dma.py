@@ -117,3 +117,12 @@ def test_tiles_in_any_order(experts, form):
     glu = act_of(want[..., :n], "silu") * want[..., n:]
     assert float((z - glu)[used].abs().max()) <= 2.0**-8 * float(glu.abs().max())
     assert bool(y[~used].isnan().all() and z[~used].isnan().all())          # unused tiles are left alone
+
+
+def test_gated_products_refuse_rows_whose_values_lie_apart():
+    from vllm_legacy_amd import _seq_ops as ops
+    k, ff = 64, 32
+    w, tile_expert = torch.zeros((1, 2 * ff, k), dtype=torch.bfloat16, device=DEV), torch.zeros(1, dtype=torch.int32, device=DEV)
+    a, out = torch.zeros((k, 32), dtype=torch.bfloat16, device=DEV).t(), torch.empty((32, ff), dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(AssertionError):
+        ops.grouped_glu(out, a, None, w, tile_expert, "silu")

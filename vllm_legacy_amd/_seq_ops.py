@@ -677,6 +677,7 @@ def grouped_glu(out: torch.Tensor, a: torch.Tensor, row_token: Optional[torch.Te
     E, N, K = weight.shape
     F = N // 2
     assert N % 2 == 0 and weight.is_contiguous() and weight.dtype == a.dtype == out.dtype and a.shape[1] == K
+    assert a.stride(1) == 1 or K == 1
     L = _lib.seq_lib()
     tiles = tile_expert.numel()
     assert out.shape == (tiles * L.vla_seq_moe_tile_rows(), F) and out.is_contiguous()
