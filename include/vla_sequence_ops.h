@@ -243,7 +243,8 @@ int vla_seq_kv_attention(void* out, int64_t out_stride, const void* q, int64_t q
                          void* stream);
 /* The same with scratch (vla_seq_kv_attention_scratch_floats values; null and 0 if it says 0) in which the
  * keys of a row may be shared out to several workgroups: few rows over long contexts.  max_keys: the most
- * keys a row of the step sees. */
+ * keys a row of the step sees (up to VLA_KV_WHOLE_KEYS nothing is shared out and no scratch wanted). */
+#define VLA_KV_WHOLE_KEYS 2048
 int64_t vla_seq_kv_attention_scratch_floats(int num_tokens, int heads, int kv_heads, int dim, int vdim,
                                             int max_keys, int dtype);
 int vla_seq_kv_attention_shared(void* out, int64_t out_stride, const void* q, int64_t q_stride,

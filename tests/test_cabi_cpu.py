@@ -75,3 +75,15 @@ def test_v1_v2_selection_rules():
     assert not P.use_v1(4096, 8, 32, 8) and P.use_v1(4096, 16, 32, 8)
     assert P.use_v1(16384, 32, 32, 8) and not P.use_v1(16384, 8, 32, 8)
     assert not P.use_v1(4096, 64, 8, 1) and P.use_v1(4096, 128, 8, 1)   # one KV head per rank
+
+
+def test_keys_up_to_which_nothing_is_shared_out():
+    """The scratch question need not be asked for as many keys as _seq_ops.KV_WHOLE_KEYS."""
+    from vllm_legacy_amd import _lib, _seq_ops
+    L = _lib.seq_lib()
+    for tokens in (1, 3, 64):
+        for heads, groups in ((1, 1), (16, 1), (32, 8)):
+            most = _seq_ops.KV_WHOLE_KEYS
+            assert L.vla_seq_kv_attention_scratch_floats(tokens, heads, groups, 128, 128, most, _lib.BF16) == 0
+            assert (L.vla_seq_kv_attention_scratch_floats(tokens, heads, groups, 128, 128, most + 1, _lib.BF16) > 0) == \
+                (tokens * groups < 256)

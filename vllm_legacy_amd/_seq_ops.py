@@ -483,6 +483,10 @@ def rotary_kv_write(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, key_cache
             "rotary_kv_write")
 
 
+# keys up to which a row's stay with one workgroup and no scratch is asked for (VLA_KV_WHOLE_KEYS)
+KV_WHOLE_KEYS = 2048
+
+
 def kv_attention(out: torch.Tensor, q: torch.Tensor, gate: Optional[torch.Tensor], key_cache: torch.Tensor,
                  value_cache: torch.Tensor, block_tables: torch.Tensor, token_seq: torch.Tensor,
                  positions: torch.Tensor, out_inv_freq: Optional[torch.Tensor], interleaved: bool, heads: int,
@@ -509,7 +513,8 @@ def kv_attention(out: torch.Tensor, q: torch.Tensor, gate: Optional[torch.Tensor
     if gate is not None:
         assert gate.dtype == q.dtype
     L = _lib.seq_lib()
-    need = L.vla_seq_kv_attention_scratch_floats(T, heads, G, D, V, int(max_keys), _dt(q.dtype))
+    need = 0 if max_keys <= KV_WHOLE_KEYS else \
+        L.vla_seq_kv_attention_scratch_floats(T, heads, G, D, V, int(max_keys), _dt(q.dtype))
     scratch = torch.empty(need, dtype=torch.float32, device=q.device) if need else None
     with torch.cuda.device(q.device):
         seq_check(L.vla_seq_kv_attention_shared(

@@ -103,8 +103,9 @@ class RotaryKVAttention(nn.Module):
                                    self.value_inv_freq, self.interleaved, self.num_heads, self.window, self.scale,
                                    self.keep_first, self.softcap, self.chunk, self.sinks)
         else:
+            keys = batch.max_seq_len
             ops.kv_attention(out, q, gate, key_cache, value_cache, batch.block_tables, batch.token_seq,
                              batch.positions, self.value_inv_freq, self.interleaved, self.num_heads, self.window,
                              self.scale, self.keep_first, self.softcap, self.chunk, self.sinks,
-                             self.max_visible(batch.max_seq_len))
+                             keys if keys <= ops.KV_WHOLE_KEYS else self.max_visible(keys))
         return out

@@ -1042,7 +1042,6 @@ constexpr int kDecodeWaves = 4;
 constexpr int kDecodeHeads = 16;
 constexpr int kDecodeKeys = 32;
 constexpr int kDecodeMinSplitKeys = 256;      // keys of a split, at least
-constexpr int kDecodeWholeKeys = 2048;        // rows that see no more than these are not split
 
 template <class S>
 struct Mma16x16;
@@ -1387,7 +1386,7 @@ __global__ __launch_bounds__(32 * VB) void kv_decode_merge_kernel(KvDecode a) {
 // 43 / 68; 32 rows of 1024 43 / 38, of 4096 59 / 70).
 int decode_splits(int num_tokens, int kv_heads, int max_keys) {
   const int64_t groups = (int64_t)num_tokens * kv_heads;
-  if (groups >= 256 || max_keys <= kDecodeWholeKeys) return 1;
+  if (groups >= 256 || max_keys <= VLA_KV_WHOLE_KEYS) return 1;
   return (int)std::max<int64_t>(1, std::min<int64_t>((256 + groups - 1) / groups, max_keys / kDecodeMinSplitKeys));
 }
 
