@@ -87,3 +87,11 @@ def test_keys_up_to_which_nothing_is_shared_out():
             assert L.vla_seq_kv_attention_scratch_floats(tokens, heads, groups, 128, 128, most, _lib.BF16) == 0
             assert (L.vla_seq_kv_attention_scratch_floats(tokens, heads, groups, 128, 128, most + 1, _lib.BF16) > 0) == \
                 (tokens * groups < 256)
+
+
+def test_launches_without_room_for_a_chunked_recurrence():
+    from vllm_legacy_amd import _lib
+    L = _lib.seq_lib()
+    assert L.vla_seq_gla_chunks_scratch_floats(1 << 20, 65535, 1, 16, 16, 1) > 0
+    assert L.vla_seq_gla_chunks_scratch_floats(1 << 20, 65536, 1, 16, 16, 1) == 0
+    assert L.vla_seq_gla_chunks_scratch_floats(64, 1, 65536, 16, 16, 1) == 0

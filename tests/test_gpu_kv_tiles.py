@@ -68,3 +68,16 @@ def test_runs_of_rows(case, dtype, copies):
     tol = (0.01 if dtype == torch.bfloat16 else 0.01 / 8) * float(want.abs().max())
     assert float((got - want).abs().max()) <= tol
     assert bool((out[:, :odd] == 7).all()) and bool((out[:, odd + H * V:] == 7).all())
+
+
+def test_more_groups_of_heads_than_a_launch_takes():
+    """65535 sequences of one row with 257 KV heads: a row that sees one key is that key's value."""
+    from vllm_legacy_amd import _seq_ops as ops
+    B, H, D = 65535, 257, 32
+    q = torch.zeros((B, H * D), dtype=torch.bfloat16, device=DEV)
+    kc, vc = (rnd((4, 1, H, D), s).to(torch.bfloat16).to(DEV) for s in (1, 2))
+    table = (torch.arange(B, dtype=torch.int32, device=DEV) % 4).view(B, 1)
+    out = torch.empty_like(q)
+    ops.kv_attention_tiles(out, q, None, kc, vc, table, torch.arange(B + 1, dtype=torch.int32, device=DEV),
+                           torch.zeros(B, dtype=torch.int32, device=DEV), 1, None, True, H, 0, 0.1)
+    assert torch.equal(out.view(B, H, D), vc[table[:, 0].long(), 0])

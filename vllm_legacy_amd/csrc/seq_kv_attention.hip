@@ -1749,23 +1749,28 @@ extern "C" int vla_seq_kv_attention_tiles(
   const int head_waves = group >= 3 ? 4 : group;      // waves of a workgroup that are heads
   const int tile_rows = kTile * (4 / head_waves);
   const int head_groups = kv_heads * ((group + head_waves - 1) / head_waves);
-  // a launch counts its threads in 32 bits; 65535 sequences reach that with more than 256 groups of heads
-  if ((int64_t)head_groups * num_seqs > 0xffffffffll / 256) return VLA_ERR_ARG;
   // few workgroups share their keys out to two groups of four waves: of 2047 rows, 16 heads on 4 of 128, one run
   // (256 workgroups) takes 68 us instead of 88, two take 76 instead of 100; four fill the chip with independent
   // ones (116 instead of 138: two workgroups of a CU do not wait for each other)
   const int64_t workgroups = (int64_t)head_groups * num_seqs * ((max_query_len + tile_rows - 1) / tile_rows);
   const int key_groups = workgroups <= 512 ? 2 : 1;
-  const dim3 grid(head_groups * num_seqs, (max_query_len + tile_rows - 1) / tile_rows, head_groups);
+  // a launch counts its threads in 32 bits: more than 16.7 million groups of heads go in several launches
+  const int most = std::max(1, 0xffffff / head_groups);
   auto go = [&](auto tag) {
     using S = decltype(tag);
     using T = typename S::T;
-    return by_value_slices(vdim, [&](int vb, int v_first) {
-      return launch_tiles<S>(dim / 32, vb, grid, (hipStream_t)stream, (T*)out, out_stride, (const T*)q, q_stride,
+    return by_value_slices(vdim, [&](int vb, int v_first) -> int {
+      for (int b0 = 0; b0 < num_seqs; b0 += most) {
+        const dim3 grid(head_groups * std::min(most, num_seqs - b0), (max_query_len + tile_rows - 1) / tile_rows, head_groups);
+        const int rc = launch_tiles<S>(
+                             dim / 32, vb, grid, (hipStream_t)stream, (T*)out, out_stride, (const T*)q, q_stride,
                              (const T*)gate, gate_stride, (const T*)key_cache, (const T*)value_cache,
-                             block_tables, max_blocks, query_start_loc, context_lens, out_inv_freq,
+                             block_tables + (int64_t)b0 * max_blocks, max_blocks, query_start_loc + b0, context_lens + b0, out_inv_freq,
                              interleaved, heads, kv_heads, block_size, num_blocks, window, scale,
                              head_waves, keep_first, softcap, chunk, sinks, key_groups, vdim, v_first);
+        if (rc != VLA_OK) return rc;
+      }
+      return VLA_OK;
     });
   };
   return dtype == VLA_BF16 ? go(BF16{}) : go(F16{});

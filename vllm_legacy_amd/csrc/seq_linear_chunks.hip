@@ -473,9 +473,11 @@ int launch_out(const GlaChunks& a, dim3 grid, hipStream_t stream) {
 using namespace vla;
 using namespace vla::seq;
 
-// 0 where the sizes do not fit or the chunks would want more than 4 GiB
+// 0 where the sizes do not fit, a launch has no room for the sequences or heads, or the chunks would want more than 4 GiB
 extern "C" int64_t vla_seq_gla_chunks_scratch_floats(int num_tokens, int num_seqs, int heads, int dim, int vdim, int rank) {
-  if (num_tokens <= 0 || num_seqs <= 0 || heads <= 0 || !chunk_sizes(dim, vdim, rank)) return 0;
+  if (num_tokens <= 0 || num_seqs <= 0 || num_seqs > 65535 || heads <= 0 || heads > 65535 ||
+      !chunk_sizes(dim, vdim, rank))
+    return 0;
   const int64_t need = chunk_slots(num_tokens, num_seqs) * heads * chunk_floats(dim, vdim);
   return need <= ((int64_t)1 << 30) ? need : 0;
 }
