@@ -70,3 +70,35 @@ def test_what_keeps_the_latent_kernel():
         assert attn._stretches(batch) is None           # too little work for the launches
         attn.FORMED_MIN_WORK = 0
         assert (attn._stretches(batch) is not None) == formed
+
+
+@pytest.mark.parametrize("common", [0.0, 3.0])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_no_further_from_64_bits_than_the_latent_kernel(common, dtype):
+    """Latents with and without a part that all tokens share, values that do not see it, scores four times as large
+    as usual: where a key's own rounding would show, since a query's is the same for all keys of a row.  (With keys
+    rounded to 16 bits the errors' ratio is 1.03 without a common part.)"""
+    from dataclasses import replace
+    from vllm_legacy_amd.attention.backends.latent_kv import LatentKVAttention
+    n, H, D, Rr, V, C, F = 512, 4, 128, 64, 128, 512, torch.float64
+    batch, blocks = step([n], [0])
+    attn = LatentKVAttention(H, D, Rr, V, C, 4 * (D + Rr)**-0.5, 0, 1e4, None, 1e-5, dtype, DEV)
+    shared, uv = rnd((1, C), 9), rnd((H * V, C), 2, C**-0.5)
+    uv = uv - (uv @ shared.t()) @ shared / (shared @ shared.t())
+    attn.set_weights(rnd((H * D, C), 1, C**-0.5), uv, torch.ones(C))
+    attn.FORMED_MIN_WORK = 0
+    q = rnd((n, H * (D + Rr)), 5).to(dtype).to(DEV)
+    kv = torch.cat([rnd((n, C), 6) + common * shared, rnd((n, Rr), 7)], 1).to(dtype).to(DEV)
+    cache = torch.zeros((blocks, 16, C + Rr), dtype=dtype, device=DEV)
+    formed = attn(q.clone(), kv, cache, batch)
+    latent = attn(q.clone(), kv, cache, replace(batch, host_query_lens=None))
+    rows = cache[batch.block_tables[0].long()].view(-1, C + Rr)[:n].to(F)
+    unseen = torch.ones((n, n), dtype=torch.bool, device=DEV).triu(1)
+    want = []
+    for h in range(H):
+        qh = q.view(n, H, D + Rr)[:, h].to(F)
+        s = (qh[:, :D] @ (rows[:, :C] @ attn.w_uk.data[h].to(F).t()).t() + qh[:, D:] @ rows[:, C:].t()) * attn.scale
+        want.append(torch.softmax(s.masked_fill(unseen, float("-inf")), 1) @ (rows[:, :C] @ attn.w_uv_t.data[h].to(F)))
+    want = torch.stack(want, 1)
+    errors = [float((x.view(n, H, V).to(F) - want).norm() / want.norm()) for x in (formed, latent)]
+    assert errors[0] <= errors[1], errors

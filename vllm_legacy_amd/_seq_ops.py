@@ -1151,16 +1151,17 @@ def latent_gather(rows: torch.Tensor, cache: torch.Tensor, block_tables: torch.T
             _dt(cache.dtype), _stream(cache.device)), "latent_gather")
 
 
-def latent_prompt(out: torch.Tensor, q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, rows: torch.Tensor,
-                  query_start_loc: torch.Tensor, context_lens: torch.Tensor, max_query_len: int, heads: int, dim: int,
+def latent_prompt(out: torch.Tensor, q: torch.Tensor, keys: torch.Tensor, keys_rest: torch.Tensor,
+                  values: torch.Tensor, rows: torch.Tensor, query_start_loc: torch.Tensor, context_lens: torch.Tensor, max_query_len: int, heads: int, dim: int,
                   rot: int, vdim: int, scale: float, window: int = 0, gate: Optional[torch.Tensor] = None,
                   sinks: Optional[torch.Tensor] = None) -> None:
     """out [T, H * vdim]; q [T, H * (dim + rot)] (views with free row strides); keys [N, H * dim] and values
-    [N, H * vdim] formed from the gathered rows [N, rank + rot] of latent_gather."""
-    _gpu(out, q, keys, values, rows, query_start_loc, context_lens, gate, sinks)
+    [N, H * vdim] formed from the gathered rows [N, rank + rot] of latent_gather; keys_rest [N, H * dim]: what the
+    keys lost to rounding."""
+    _gpu(out, q, keys, keys_rest, values, rows, query_start_loc, context_lens, gate, sinks)
     T, N, H, B = q.shape[0], rows.shape[0], int(heads), context_lens.numel()
-    assert out.dtype == q.dtype == keys.dtype == values.dtype == rows.dtype
-    assert keys.shape == (N, H * dim) and values.shape == (N, H * vdim) and out.shape == (T, H * vdim)
+    assert out.dtype == q.dtype == keys.dtype == keys_rest.dtype == values.dtype == rows.dtype
+    assert keys.shape == keys_rest.shape == (N, H * dim) and keys_rest.is_contiguous() and values.shape == (N, H * vdim) and out.shape == (T, H * vdim)
     assert keys.is_contiguous() and values.is_contiguous() and rows.is_contiguous()
     assert sinks is None or (sinks.dtype == torch.float32 and sinks.numel() == H and sinks.is_contiguous())
     assert gate is None or gate.dtype == q.dtype
@@ -1170,6 +1171,6 @@ def latent_prompt(out: torch.Tensor, q: torch.Tensor, keys: torch.Tensor, values
     with torch.cuda.device(q.device):
         seq_check(_lib.seq_lib().vla_seq_latent_prompt(
             out.data_ptr(), _rows(out, H * vdim), q.data_ptr(), _rows(q, H * (dim + rot)), keys.data_ptr(),
-            values.data_ptr(), rows.data_ptr(), N, query_start_loc.data_ptr(), context_lens.data_ptr(), B,
+            keys_rest.data_ptr(), values.data_ptr(), rows.data_ptr(), N, query_start_loc.data_ptr(), context_lens.data_ptr(), B,
             int(max_query_len), H, int(dim), int(rot), int(vdim), rows.shape[1] - int(rot), float(scale), int(window),
             _p(gate), 0 if gate is None else _rows(gate, H), _p(sinks), _dt(q.dtype), _stream(q.device)), "latent_prompt")

@@ -165,9 +165,13 @@ class LatentKVAttention(nn.Module):
         rows = torch.empty((sum(counts), C + Rr), dtype=q.dtype, device=q.device)
         ops.latent_gather(rows, cache, tables, starts, ctx, max(counts), self.window)
         latents = rows[:, :C]
-        keys = torch.mm(latents, self.w_uk.data.view(H * D, C).t())
+        # A key's rounding is its own, where that of a query on the latents' side is the same for all keys and mostly
+        # cancels in the softmax: the keys keep what they lose.
+        w_uk = self.w_uk.data.view(H * D, C).t()
+        keys = torch.mm(latents, w_uk)
+        keys_rest = torch.addmm(keys, latents, w_uk, beta=-1)
         values = torch.mm(latents, self.w_uv_t.data.transpose(0, 1).reshape(C, H * V))
-        ops.latent_prompt(out[r0:r1], q[r0:r1], keys, values, rows, starts, ctx, max(ql), H, D, Rr, V, self.scale,
+        ops.latent_prompt(out[r0:r1], q[r0:r1], keys, keys_rest, values, rows, starts, ctx, max(ql), H, D, Rr, V, self.scale,
                           self.window, None if gate is None else gate[r0:r1],
                           None if self.sinks is None else self.sinks.data)
 

@@ -5,19 +5,25 @@
 // queries of the run.  A run of rows therefore gathers its visible cache rows into one place
 // (latent_gather_kernel), the caller multiplies them with the two up-projections, and
 // latent_prompt_kernel below is plain causal attention with keys [formed (dim) | shared rotated part
-// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 144 us (600 TFLOP/s) where
-// latent_attention_tile_kernel takes 1685, plus 8 us to gather and 35 for the two products (the products
-// on the query's side that they replace take 46).
+// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 182 us (480 TFLOP/s; 620
+// with the remainders' product) where latent_attention_tile_kernel takes 1685, plus 9 us to gather and 60 for the
+// three products (the products on the query's side that they replace take 46).
+//
+// Keys come as two 16-bit numbers, the rounded one and what rounding took.  The latent kernel rounds the query's
+// side, which is the same for all keys of a row and mostly cancels in the softmax; a key's rounding is its own.
+// Outputs' error against 64 bits, this / one 16-bit number / the latent kernel, bf16, 1e-3: independent latents
+// 2.5 / 2.8 / 2.8, with scores four times as large 2.4 / 3.8 / 3.6 (float16: an eighth of each).  One number
+// per key takes 136 us, and 189 instead of 258 for the whole layer.
 //
 // The rows of sequence b are its keys from first_b = max(0, context - window + 1) (0 without a window) to
 // its last new row; sequences follow each other, so a sequence's place is the sum of the counts before
 // it, which every workgroup forms for itself (nothing has to be planned on the host or copied there).
 //
-// latent_prompt_kernel<S, DB, VB>: a workgroup is 128 query rows of one head, 32 per wave, and walks key
+// latent_prompt_kernel<S, DB, VB, LB>: a workgroup is 128 query rows of one head, 32 per wave, and walks key
 // tiles of 64.  Products on 32x32x16 MFMAs in transposed form (lane = (hf, c) = (lane >> 5, lane & 31)):
 //   S^T = K q^T   A = K: lane: key c, dims 16 ks + 8 hf .. + 7 (LDS);  B = q^T: query c (registers)
 //   O^T = V^T P^T B = P^T: the first product's result where it lies;   A = V^T: two transposing reads
-// Tiles come in by LDS-DMA, double-buffered, one barrier per tile and no staging registers.  A DMA
+// Tiles come in by LDS-DMA, keys and values in turn (one tile of each in LDS: 56 KB), without staging registers.  A DMA
 // instruction writes 64 lanes x 16 bytes in a row, so rows cannot be padded; 16-byte pieces (values:
 // 64-byte ones) are exchanged within a row by the row's number instead, on the source's side, so that
 // the lanes of a read fall into different banks.  Two workgroups share a CU: one's softmax (about 30
@@ -25,6 +31,7 @@
 // multiple of it when heads are a multiple of 8, so they share an XCD's L2 for that head's keys.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "seq_common.h"
 
@@ -105,6 +112,7 @@ struct LatentPrompt {
   const void* q;                // [T, heads * q_head]: a head's row is [plain (dim) | rotated (rot)]
   int64_t q_stride;
   const void* keys;             // [N, heads * dim]
+  const void* keys_rest;        // the same: what the keys lost when they were rounded
   const void* values;           // [N, heads * vdim]
   const void* rows;             // [N, rank + rot]: the rotated part behind the latent
   const int* query_start_loc;
@@ -126,16 +134,20 @@ __device__ __forceinline__ void dma16(const void* src, uint32_t lds_at) {
       : "memory");
 }
 
-template <class S, int DB, int VB>
+// for pieces of LDS rows behind a row's end
+__device__ const u32x4 kNothing = {0u, 0u, 0u, 0u};
+
+template <class S, int DB, int VB, int LB>
 __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
   using T = typename S::T;
   using M = Mma<S>;
-  constexpr int DQ = 32 * DB, VD = 32 * VB;
-  constexpr int KB = 2 * DQ, VBYTES = 2 * VD;              // bytes of a tile's rows
-  constexpr int KTILE = kKeys * KB, VTILE = kKeys * VBYTES, STAGE = KTILE + VTILE;
-  constexpr int KI = KTILE / 1024 / kWaves, VI = VTILE / 1024 / kWaves;      // DMA instructions per wave
+  constexpr int DQ = 32 * DB, VD = 32 * VB, LD = 32 * LB;
+  constexpr int KB = 2 * DQ, VBYTES = 2 * VD, RB = 2 * LD;                   // bytes of a tile's rows
+  constexpr int KTILE = kKeys * KB, RTILE = kKeys * RB, VTILE = kKeys * VBYTES;
+  constexpr int KI = KTILE / 1024 / kWaves, RI = RTILE / 1024 / kWaves, VI = VTILE / 1024 / kWaves;    // DMA instructions per wave
   // a key row is a whole number of 256 bytes (all 64 banks), or half of one more: which pieces change place
   constexpr int KMASK = KB % 256 == 0 ? 15 : 7, KSHIFT = KB % 256 == 0 ? 0 : 1;
+  constexpr int RMASK = RB % 256 == 0 ? 15 : 7, RSHIFT = RB % 256 == 0 ? 0 : 1;
   extern __shared__ __align__(16) unsigned char smem[];
   const int h = blockIdx.x, b = blockIdx.z;
   const int run = a.query_start_loc[b + 1] - a.query_start_loc[b];
@@ -181,27 +193,36 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
   }
 
   // What this lane brings in: piece `at` of a tile in LDS is row at / pieces; which 16 bytes of the row
-  // stand there follows from the exchange.  Pieces past dim + rot (vdim) repeat the row's first ones; their
-  // products meet zeros of q (columns nobody writes).
-  const unsigned char* src_k[KI];
-  const unsigned char* src_v[VI];
-  int row_k[KI], row_v[VI];
-  int64_t step_k[KI];
-  const int64_t key_row = (int64_t)a.heads * a.dim * 2, value_row = (int64_t)a.heads * a.vdim * 2;
-  const int64_t lat_row = (int64_t)(a.rank + a.rot) * 2;
+  // stand there follows from the exchange.  Pieces past the end of a key are zeros; those past a value's repeat its
+  // first ones, for columns nobody writes.
+  const unsigned char *src_k[KI], *src_r[RI], *src_v[VI];
+  int row_k[KI], row_r[RI], row_v[VI];
+  unsigned step_k[KI], step_r[RI];
+  const unsigned key_row = (unsigned)a.heads * a.dim * 2, value_row = (unsigned)a.heads * a.vdim * 2;
+  const unsigned lat_row = (unsigned)(a.rank + a.rot) * 2;
+  const int64_t first_key = (int64_t)base * key_row + (int64_t)h * a.dim * 2;
 #pragma unroll
   for (int u = 0; u < KI; ++u) {
     const int at = ((w * KI + u) * 1024 + 16 * lane) / 16, r = at / (KB / 16), s = at % (KB / 16);
     const int piece = (s & ~KMASK) | ((s ^ (r >> KSHIFT)) & KMASK);
     const int d = 8 * piece;
     row_k[u] = r;
-    if (d < a.dim || d >= width) {
-      src_k[u] = (const unsigned char*)a.keys + (int64_t)base * key_row + ((int64_t)h * a.dim + (d < a.dim ? d : 0)) * 2;
-      step_k[u] = key_row;
-    } else {
-      src_k[u] = (const unsigned char*)a.rows + (int64_t)base * lat_row + (a.rank + d - a.dim) * 2;
-      step_k[u] = lat_row;
+    src_k[u] = d < a.dim ? (const unsigned char*)a.keys + first_key + 2 * d
+                         : (const unsigned char*)a.rows + (int64_t)base * lat_row + (a.rank + d - a.dim) * 2;
+    step_k[u] = d < a.dim ? key_row : lat_row;
+    if (d >= width) {
+      src_k[u] = (const unsigned char*)&kNothing;
+      step_k[u] = 0;
     }
+  }
+#pragma unroll
+  for (int u = 0; u < RI; ++u) {
+    const int at = ((w * RI + u) * 1024 + 16 * lane) / 16, r = at / (RB / 16), s = at % (RB / 16);
+    const int piece = (s & ~RMASK) | ((s ^ (r >> RSHIFT)) & RMASK);
+    const int d = 8 * piece;
+    row_r[u] = r;
+    src_r[u] = d < a.dim ? (const unsigned char*)a.keys_rest + first_key + 2 * d : (const unsigned char*)&kNothing;
+    step_r[u] = d < a.dim ? key_row : 0;
   }
 #pragma unroll
   for (int u = 0; u < VI; ++u) {
@@ -212,47 +233,71 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
     src_v[u] = (const unsigned char*)a.values + (int64_t)base * value_row + ((int64_t)h * a.vdim + (d < a.vdim ? d : 0)) * 2;
   }
   const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
-  auto bring = [&](int u0, int buf) {
-    const uint32_t to = lds0 + buf * STAGE;
+  auto bring_keys = [&](int u0) {
 #pragma unroll
     for (int u = 0; u < KI; ++u)
-      dma16(src_k[u] + (int64_t)min(u0 + row_k[u], n_keys - 1) * step_k[u], to + (w * KI + u) * 1024);
+      dma16(src_k[u] + (uint64_t)(unsigned)min(u0 + row_k[u], n_keys - 1) * step_k[u], lds0 + (w * KI + u) * 1024);
+#pragma unroll
+    for (int u = 0; u < RI; ++u)
+      dma16(src_r[u] + (uint64_t)(unsigned)min(u0 + row_r[u], n_keys - 1) * step_r[u], lds0 + KTILE + (w * RI + u) * 1024);
+  };
+  auto bring_values = [&](int u0) {
 #pragma unroll
     for (int u = 0; u < VI; ++u)
-      dma16(src_v[u] + (int64_t)min(u0 + row_v[u], n_keys - 1) * value_row, to + KTILE + (w * VI + u) * 1024);
+      dma16(src_v[u] + (uint64_t)(unsigned)min(u0 + row_v[u], n_keys - 1) * value_row, lds0 + KTILE + RTILE + (w * VI + u) * 1024);
   };
   // where this lane reads: the exchanged piece of its key row, and the unit of its value rows
   const int kx = (hf ^ ((c >> KSHIFT) & KMASK)) & KMASK;   // piece 2 ks + hf stands at 2 ks ^ kx within its group
+  const int rx = (hf ^ ((c >> RSHIFT) & RMASK)) & RMASK;
   const int i16 = c & 15;
   const int vrow = 4 * hf + (i16 >> 2);
   const int vf = VB == 4 ? vrow & 3 : (vrow >> 1) & (VB - 1);
   const int vat = vrow * VBYTES + 32 * (c >> 4) + 8 * (i16 & 3);
 
-  int u0 = g_first & ~(kKeys - 1);
-  bring(u0, 0);
-  for (int it = 0; u0 <= p_end; u0 += kKeys, ++it) {
+  // Keys and values take turns: a tile's values come in under the first product, the next tile's keys under the
+  // softmax and the second one.
+  const unsigned char* k_lds = smem;
+  const unsigned char* r_lds = smem + KTILE;
+  const unsigned char* v_lds = smem + KTILE + RTILE;
+  auto landed = [&]() {
     // the builtin and not asm: the compiler then knows that the query rows have arrived, and does not wait for
     // vmcnt(0), and so for the DMA just started, at their first use in every step
     __builtin_amdgcn_s_waitcnt(0x0f70);                // vmcnt(0)
     asm volatile("" ::: "memory");
     __syncthreads();
-    if (u0 + kKeys <= p_end) bring(u0 + kKeys, (it + 1) & 1);
-    const unsigned char* k_lds = smem + (it & 1) * STAGE;
-    const unsigned char* v_lds = k_lds + KTILE;
-    if (nq <= 0 || u0 > p0 + nq - 1 || u0 + kKeys <= lo_first) continue;     // no key of it concerns this wave
+  };
+  int u0 = g_first & ~(kKeys - 1);
+  bring_keys(u0);
+  for (; u0 <= p_end; u0 += kKeys) {
+    landed();
+    bring_values(u0);
+    const bool concerned = nq > 0 && u0 <= p0 + nq - 1 && u0 + kKeys > lo_first;     // some key of it concerns this wave
     f32x16 st[2];
+    if (concerned) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) st[kb][i] = 0.f;
+        for (int i = 0; i < 16; ++i) st[kb][i] = 0.f;
 #pragma unroll
-    for (int ks = 0; ks < DQ / 16; ++ks)
+      for (int ks = 0; ks < DQ / 16; ++ks)
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const int slot = ((2 * ks) & ~KMASK) | (((2 * ks) & KMASK) ^ kx);
-        const u32x4 ka = *reinterpret_cast<const u32x4*>(k_lds + (32 * kb + c) * KB + 16 * slot);
-        st[kb] = M::run(ka, qf[ks], st[kb]);
-      }
+        for (int kb = 0; kb < 2; ++kb) {
+          const int slot = ((2 * ks) & ~KMASK) | (((2 * ks) & KMASK) ^ kx);
+          const u32x4 ka = *reinterpret_cast<const u32x4*>(k_lds + (32 * kb + c) * KB + 16 * slot);
+          st[kb] = M::run(ka, qf[ks], st[kb]);
+        }
+#pragma unroll
+      for (int ks = 0; ks < LD / 16; ++ks)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          const int slot = ((2 * ks) & ~RMASK) | (((2 * ks) & RMASK) ^ rx);
+          const u32x4 ra = *reinterpret_cast<const u32x4*>(r_lds + (32 * kb + c) * RB + 16 * slot);
+          st[kb] = M::run(ra, qf[ks], st[kb]);
+        }
+    }
+    landed();
+    if (u0 + kKeys <= p_end) bring_keys(u0 + kKeys);
+    if (!concerned) continue;
     // every key of the tile visible to every row of the wave: no masks
     if (!(u0 + kKeys - 1 <= p0 && u0 >= lo_last && nq == kRowsPerWave)) {
 #pragma unroll
@@ -324,16 +369,16 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
     }
 }
 
-template <class S, int DB, int VB>
+template <class S, int DB, int VB, int LB>
 int launch_latent_prompt(const LatentPrompt& a, dim3 grid, hipStream_t stream) {
-  constexpr size_t lds = 2 * kKeys * (64 * DB + 64 * VB);
+  constexpr size_t lds = kKeys * 64 * (DB + VB + LB);
   static std::atomic<bool> raised{false};           // LDS limit: raised once per kernel, not per launch
   if (lds > 64 * 1024 && !raised.load(std::memory_order_relaxed)) {
-    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_prompt_kernel<S, DB, VB>),
+    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_prompt_kernel<S, DB, VB, LB>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     raised.store(true, std::memory_order_relaxed);
   }
-  latent_prompt_kernel<S, DB, VB><<<grid, 256, lds, stream>>>(a);
+  latent_prompt_kernel<S, DB, VB, LB><<<grid, 256, lds, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   return VLA_OK;
 }
@@ -373,20 +418,21 @@ extern "C" int vla_seq_latent_gather(void* rows, int num_rows, const void* cache
 }
 
 extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* q, int64_t q_stride,
-                                     const void* keys, const void* values, const void* rows, int num_rows,
+                                     const void* keys, const void* keys_rest, const void* values,
+                                     const void* rows, int num_rows,
                                      const int* query_start_loc, const int* context_lens, int num_seqs,
                                      int max_query_len, int heads, int dim, int rot, int vdim, int rank,
                                      float scale, int window, const void* gate, int64_t gate_stride,
                                      const float* sinks, int dtype, void* stream) {
   if (num_seqs == 0 || max_query_len == 0) return VLA_OK;
-  if (!out || !q || !keys || !values || !rows || !query_start_loc || !context_lens || num_seqs < 0 ||
+  if (!out || !q || !keys || !keys_rest || !values || !rows || !query_start_loc || !context_lens || num_seqs < 0 ||
       num_seqs > 65535 || max_query_len < 0 || num_rows <= 0 || heads <= 0 || heads > 65535 || !(scale > 0.f) ||
       window < 0 || (gate && gate_stride < heads) || out_stride < (int64_t)heads * vdim ||
       q_stride < (int64_t)heads * (dim + rot))
     return VLA_ERR_ARG;
   if (dtype != VLA_F16 && dtype != VLA_BF16) return VLA_ERR_DTYPE;
   if (!prompt_sizes(dim, rot, vdim, rank)) return VLA_ERR_HEAD_SIZE;
-  if ((uintptr_t)q % 16 || q_stride % 8 || (uintptr_t)keys % 16 || (uintptr_t)values % 16 || (uintptr_t)rows % 16 ||
+  if ((uintptr_t)q % 16 || q_stride % 8 || (uintptr_t)keys % 16 || (uintptr_t)keys_rest % 16 || (uintptr_t)values % 16 || (uintptr_t)rows % 16 ||
       (uintptr_t)out % 8 || out_stride % 4)
     return VLA_ERR_ARG;
   LatentPrompt a;
@@ -395,6 +441,7 @@ extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* 
   a.q = q;
   a.q_stride = q_stride;
   a.keys = keys;
+  a.keys_rest = keys_rest;
   a.values = values;
   a.rows = rows;
   a.query_start_loc = query_start_loc;
@@ -415,12 +462,13 @@ extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* 
   const dim3 grid(heads, a.row_tiles, num_seqs);
   auto go = [&](auto s) -> int {
     using S = decltype(s);
-    const bool wide = dim + rot > 128;
-    if (vdim <= 64)
-      return wide ? launch_latent_prompt<S, 6, 2>(a, grid, (hipStream_t)stream)
-                  : launch_latent_prompt<S, 4, 2>(a, grid, (hipStream_t)stream);
-    return wide ? launch_latent_prompt<S, 6, 4>(a, grid, (hipStream_t)stream)
-                : launch_latent_prompt<S, 4, 4>(a, grid, (hipStream_t)stream);
+    auto with_values = [&](auto vb) -> int {
+      constexpr int VB = decltype(vb)::value;
+      if (dim > 128) return launch_latent_prompt<S, 6, VB, 6>(a, grid, (hipStream_t)stream);
+      return dim + rot > 128 ? launch_latent_prompt<S, 6, VB, 4>(a, grid, (hipStream_t)stream)
+                             : launch_latent_prompt<S, 4, VB, 4>(a, grid, (hipStream_t)stream);
+    };
+    return vdim <= 64 ? with_values(std::integral_constant<int, 2>{}) : with_values(std::integral_constant<int, 4>{});
   };
   return dtype == VLA_BF16 ? go(BF16{}) : go(F16{});
 }
