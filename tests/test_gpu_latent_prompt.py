@@ -102,3 +102,31 @@ def test_no_further_from_64_bits_than_the_latent_kernel(common, dtype):
     want = torch.stack(want, 1)
     errors = [float((x.view(n, H, V).to(F) - want).norm() / want.norm()) for x in (formed, latent)]
     assert errors[0] <= errors[1], errors
+
+
+def layer_and_step(lens, contexts, sizes, window=0, sinks=False, dtype=torch.bfloat16):
+    from vllm_legacy_amd.attention.backends.latent_kv import LatentKVAttention
+    H, D, Rr, V, C = sizes
+    batch, blocks = step(lens, contexts)
+    attn = LatentKVAttention(H, D, Rr, V, C, (D + Rr)**-0.5, Rr, 1e4, None, 1e-5, dtype, DEV, window=window or None, sinks=sinks)
+    attn.set_weights(rnd((H * D, C), 1, C**-0.5), rnd((H * V, C), 2, C**-0.5), 1 + 0.1 * rnd((C, ), 3),
+                     rnd((H, ), 4) if sinks else None)
+    attn.FORMED_MIN_WORK = 0
+    T = sum(lens)
+    q, kv, gate = (rnd((T, w), s).to(dtype).to(DEV) for w, s in ((H * (D + Rr), 5), (C + Rr, 6), (H, 7)))
+    return attn, batch, q, kv, gate, rnd((blocks, 16, C + Rr), 8).to(dtype).to(DEV)
+
+
+@pytest.mark.parametrize("row", [0, 1, 31, 40, 63, 64, 127, 200])
+@pytest.mark.parametrize("window", [0, 70])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_rows_that_do_not_see_one_that_is_not_finite(row, window, value):
+    """Bit for bit what they are without it."""
+    attn, batch, q, kv, gate, cache = layer_and_step([230, 66], [30, 0], (4, 128, 64, 128, 128), window)
+    clean = attn(q.clone(), kv, cache.clone(), batch, gate)
+    assert bool(clean.isfinite().all())
+    kv[row, 5] = value
+    got = attn(q.clone(), kv, cache.clone(), batch, gate)
+    sees = torch.zeros(len(got), dtype=torch.bool, device=DEV)
+    sees[row:min(230, row + window) if window else 230] = True
+    assert torch.equal(got[~sees], clean[~sees]) and not got[sees].isfinite().any()

@@ -70,6 +70,13 @@ struct Mma<F16> {
   }
 };
 
+// 0xffff for each of two 16-bit numbers that is not finite
+template <class S>
+__device__ __forceinline__ uint32_t odd_halves(uint32_t x) {
+  constexpr uint32_t kLow = std::is_same<S, BF16>::value ? 0x7f80u : 0x7c00u, kHigh = kLow << 16;      // exponents of ones
+  return ((x & kLow) == kLow ? 0xffffu : 0u) | ((x & kHigh) == kHigh ? 0xffff0000u : 0u);
+}
+
 __device__ __forceinline__ int first_formed(int context, int window) { return window > 0 ? max(0, context - window + 1) : 0; }
 
 // where sequence b's rows begin among all gathered rows (one wave; every lane gets it)
@@ -166,6 +173,7 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
   const int p0 = ctx + r0 + kRowsPerWave * w - first, pq = p0 + c;
   const int p_end = ctx + r0 + n_rows - 1 - first, n_keys = ctx + run - first;
   const int g_first = a.window > 0 ? max(0, ctx + r0 - first - a.window + 1) : 0;    // the group's first key
+  const int g_p0 = ctx + r0 - first, g_lo_last = a.window > 0 ? g_p0 + kRowsPerGroup - a.window : 0;    // the group's
   const int lo_q = a.window > 0 ? pq - a.window + 1 : 0;                       // this row's
   const int lo_last = a.window > 0 ? p0 + kRowsPerWave - a.window : 0;         // the wave's last row's
   const int lo_first = a.window > 0 ? p0 - a.window + 1 : 0;
@@ -297,6 +305,25 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
     }
     landed();
     if (u0 + kKeys <= p_end) bring_keys(u0 + kKeys);
+    // A hidden key's weight is 0, which times an infinity or a NaN would not be: a tile that hides keys from some row
+    // goes without values that are not finite.  Rows that see such a key are NaN by their scores: a key of the same
+    // latent is not finite either, and it and what it lost to rounding never sum to a number.
+    if (u0 + kKeys - 1 > g_p0 || u0 < g_lo_last) {
+#pragma unroll
+      for (int u = 0; u < VI; ++u) {
+        u32x4* at = reinterpret_cast<u32x4*>(smem + KTILE + RTILE + (w * VI + u) * 1024 + 16 * lane);
+        u32x4 x = *at;
+        uint32_t some = 0u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t odd = odd_halves<S>(x[e]);
+          x[e] &= ~odd;
+          some |= odd;
+        }
+        if (some != 0u) *at = x;
+      }
+      __syncthreads();
+    }
     if (!concerned) continue;
     // every key of the tile visible to every row of the wave: no masks
     if (!(u0 + kKeys - 1 <= p0 && u0 >= lo_last && nq == kRowsPerWave)) {
