@@ -419,7 +419,8 @@ int vla_seq_gla_chunks(void* out, int64_t out_stride, const void* q, int64_t q_s
  * max_seq_rows: the most rows of one sequence.
  * vla_seq_latent_prompt: out [T, heads * vdim] from q [T, heads * (dim + rot)] (a head's row: plain | rotated),
  * keys [num_rows, heads * dim] and values [num_rows, heads * vdim] that the caller formed from the gathered
- * latents, keys_rest (as keys) what rounding to 16 bits took from the keys (scores are of their sum), and the gathered rows themselves for the rotated parts behind them. */
+ * latents, keys_rest (as keys) what rounding to 16 bits took from the keys (scores are of their sum), and the gathered rows themselves for the rotated parts behind them.
+ * Rows of a sequence whose lengths on the device are beyond those that rows were gathered for are NaN. */
 int vla_seq_latent_prompt_supported(int dim, int rot, int vdim, int rank, int dtype);
 int vla_seq_latent_gather(void* rows, int num_rows, const void* cache, const int* block_tables,
                           int max_blocks, const int* query_start_loc, const int* context_lens, int num_seqs,

@@ -130,3 +130,20 @@ def test_rows_that_do_not_see_one_that_is_not_finite(row, window, value):
     sees = torch.zeros(len(got), dtype=torch.bool, device=DEV)
     sees[row:min(230, row + window) if window else 230] = True
     assert torch.equal(got[~sees], clean[~sees]) and not got[sees].isfinite().any()
+
+
+def test_lengths_that_are_not_the_hosts():
+    """Rows of a sequence that grew on the device are NaN, not what memory held; a captured step takes the latent
+    kernel, which follows the device."""
+    from dataclasses import replace
+    attn, batch, q, kv, gate, cache = layer_and_step([100, 80], [200, 40], (2, 64, 0, 64, 64))
+    good = attn(q.clone(), kv, cache.clone(), batch, gate)
+    got = attn(q.clone(), kv, cache.clone(), replace(batch, host_context_lens=[136, 40]), gate)
+    assert bool(got[100:].isnan().all()) and torch.equal(got[:100], good[:100])
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    assert attn._stretches(batch) is not None
+    with torch.cuda.stream(stream):
+        graph.capture_begin()
+        inside = attn._stretches(batch)
+        graph.capture_end()
+    assert inside is None

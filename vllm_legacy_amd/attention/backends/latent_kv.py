@@ -138,8 +138,8 @@ class LatentKVAttention(nn.Module):
         if batch.max_query_len < least or not self.scale > 0:
             return None
         q, ctx = batch.host_query_lens, batch.host_context_lens
-        if q is None or ctx is None:
-            return None
+        if q is None or ctx is None or torch.cuda.is_current_stream_capturing():
+            return None                 # a captured step is replayed with other lengths than the host's
         out, row, pairs = [], 0, 0
         for b, (n, c) in enumerate(zip(q, ctx)):
             if n >= least:

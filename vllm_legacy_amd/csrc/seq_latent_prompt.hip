@@ -98,18 +98,20 @@ __global__ __launch_bounds__(256) void latent_gather_kernel(
   const int b = blockIdx.y;
   const int ctx = context_lens[b], first = first_formed(ctx, window);
   const int n = ctx + query_start_loc[b + 1] - query_start_loc[b] - first;
-  const int r0 = blockIdx.x * kGatherRows;
-  if (r0 >= n) return;
+  if ((int)blockIdx.x * kGatherRows >= n) return;
   const int base = gathered_before(query_start_loc, context_lens, b, window);
   const int* table = block_tables + (int64_t)b * max_blocks;
-  const int count = min(kGatherRows, n - r0) * pieces;
-  for (int i = threadIdx.x; i < count; i += 256) {
-    const int r = i / pieces, v = i - r * pieces;
-    const int j = first + r0 + r;
-    int blk = table[j / block_size];
-    blk = (unsigned)blk < (unsigned)num_blocks ? blk : 0;  // a table the host filled wrongly reads block 0
-    if (base + r0 + r < num_rows)
+  const int end = min(n, num_rows - base);
+  // (a second time round only where the sequence is longer than the host's lengths say)
+  for (int r0 = blockIdx.x * kGatherRows; r0 < end; r0 += gridDim.x * kGatherRows) {
+    const int count = min(kGatherRows, end - r0) * pieces;
+    for (int i = threadIdx.x; i < count; i += 256) {
+      const int r = i / pieces, v = i - r * pieces;
+      const int j = first + r0 + r;
+      int blk = table[j / block_size];
+      blk = (unsigned)blk < (unsigned)num_blocks ? blk : 0;  // a table the host filled wrongly reads block 0
       rows[(int64_t)(base + r0 + r) * pieces + v] = cache[((int64_t)blk * block_size + j % block_size) * pieces + v];
+    }
   }
 }
 
@@ -165,10 +167,16 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
   const int hf = lane >> 5, c = lane & 31;
   const int ctx = a.context_lens[b], first = first_formed(ctx, a.window);
   const int base = gathered_before(a.query_start_loc, a.context_lens, b, a.window);
-  if (base + ctx + run - first > a.num_rows) return;       // the host allocated for other lengths
   const int n_rows = min(kRowsPerGroup, run - r0);         // rows of this workgroup
   const int nq = min(kRowsPerWave, n_rows - kRowsPerWave * w);               // and of this wave (<= 0: none)
   const int t0 = a.query_start_loc[b] + r0 + kRowsPerWave * w;
+  T* orow = (T*)a.out + (int64_t)(t0 + c) * a.out_stride + (int64_t)h * a.vdim + 4 * hf;
+  if (base + ctx + run - first > a.num_rows) {
+    // the host gathered for other lengths than the device has: no answer, and none that looks like one
+    const uint32_t nan2 = M::pack2(NAN, NAN);
+    for (int d = 0; c < nq && d + 4 * hf < a.vdim; d += 8) *reinterpret_cast<u32x2*>(orow + d) = u32x2{nan2, nan2};
+    return;
+  }
   // positions, counted from the first gathered key
   const int p0 = ctx + r0 + kRowsPerWave * w - first, pq = p0 + c;
   const int p_end = ctx + r0 + n_rows - 1 - first, n_keys = ctx + run - first;
@@ -384,7 +392,6 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
   if (c >= nq) return;
   float inv = 1.f / l;
   if (a.gate != nullptr) inv /= 1.f + expf(-S::to_f32(((const T*)a.gate)[(int64_t)(t0 + c) * a.gate_stride + h]));
-  T* orow = (T*)a.out + (int64_t)(t0 + c) * a.out_stride + (int64_t)h * a.vdim + 4 * hf;
 #pragma unroll
   for (int n = 0; n < VB; ++n)
 #pragma unroll
