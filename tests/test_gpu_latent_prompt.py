@@ -111,7 +111,7 @@ def layer_and_step(lens, contexts, sizes, window=0, sinks=False, dtype=torch.bfl
     attn = LatentKVAttention(H, D, Rr, V, C, (D + Rr)**-0.5, Rr, 1e4, None, 1e-5, dtype, DEV, window=window or None, sinks=sinks)
     attn.set_weights(rnd((H * D, C), 1, C**-0.5), rnd((H * V, C), 2, C**-0.5), 1 + 0.1 * rnd((C, ), 3),
                      rnd((H, ), 4) if sinks else None)
-    attn.FORMED_MIN_WORK = 0
+    attn.FORMED_MIN_WORK, attn.FORMED_MIN_ROWS = 0, 32
     T = sum(lens)
     q, kv, gate = (rnd((T, w), s).to(dtype).to(DEV) for w, s in ((H * (D + Rr), 5), (C + Rr, 6), (H, 7)))
     return attn, batch, q, kv, gate, rnd((blocks, 16, C + Rr), 8).to(dtype).to(DEV)

@@ -115,27 +115,30 @@ class LatentKVAttention(nn.Module):
     # the longest stretches of sequences a step is cut into; one that alternates more often stays whole
     MAX_STRETCHES = 4
 
-    # multiply-adds of a step on the latent kernel (a fifth of a matrix product's rate) from which the other
-    # way's five launches more are paid back: rows x keys before them, 16 heads, latent / formed us per call:
-    # 256 x 0 113 / 127, 128 x 2000 121 / 128, four of 64 x 2000 181 / 166, 256 x 2000 188 / 125, sixteen of
-    # 48 x 1000 262 / 225, of 256 x 1000 1079 / 275
-    FORMED_MIN_WORK = 5e9
+    # Multiply-adds of a step on the latent kernel (a fifth of a matrix product's rate) from which the other way's
+    # seven launches more are paid back.  Rows x keys before them, 16 heads of 128 + 64, rank 512, latent / formed us
+    # per call: 128 x 2000 (4.6e9) 118 / 160, 192 x 2000 (7.0e9) 183 / 154, four of 384 x 0 (5.1e9) 137 / 140.
+    FORMED_MIN_WORK = 6e9
+    # Rows of a run at least: forming a key's numbers costs as much for few rows as for many.  Sixteen of 64 rows x
+    # 1000 268 / 349, of 96 389 / 346; four of 64 x 2000 176 / 243, of 96 282 / 238.
+    FORMED_MIN_ROWS = 96
 
     def formed_min_rows(self) -> int:
         """Rows from which a run's keys and values are worth forming.  A (query, key) pair of a head costs the
-        latent kernel 2 rank + rot multiply-adds at a fifth of a matrix product's rate, the formed one
-        dim + rot + vdim at half of it; forming costs rank (dim + vdim) per key at the full rate.  (16 heads,
-        rank 512, 1000 and 2000 keys before the run: runs of 32 rows 189 / 220 us and 134 / 138 us latent /
-        formed, of 48 rows 262 / 225 and 181 / 160.)"""
+        latent kernel 2 rank + rot multiply-adds at a fifth of a matrix product's rate (less where the rank is small),
+        the formed one dim + rot + vdim at about half of it; forming costs rank (dim + vdim) per key at the full rate.
+        (A rank of 64 beside heads of 128 + 64: 2048 rows 190 / 160 us, 4096 585 / 249.)"""
         C, D, R, V = self.rank, self.head_dim, self.rot_dim, self.value_dim
         gain = 5 * (2 * C + R) - 2 * (D + R + V)
-        return max(48, -(-C * (D + V) // gain)) if gain > 0 else 1 << 30
+        return max(self.FORMED_MIN_ROWS, -(-C * (D + V) // gain)) if gain > 0 else 1 << 30
 
     def _stretches(self, batch: SequenceBatch):
         """[[first sequence, one behind the last, first row, one behind the last, formed]]: neighbours that go
         the same way; None when the whole step takes the latent kernel."""
+        if batch.max_query_len < self.FORMED_MIN_ROWS or not self.scale > 0:
+            return None
         least = self.formed_min_rows()
-        if batch.max_query_len < least or not self.scale > 0:
+        if batch.max_query_len < least:
             return None
         q, ctx = batch.host_query_lens, batch.host_context_lens
         if q is None or ctx is None or torch.cuda.is_current_stream_capturing():
