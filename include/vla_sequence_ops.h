@@ -417,20 +417,27 @@ int vla_seq_gla_chunks(void* out, int64_t out_stride, const void* q, int64_t q_s
  * vla_seq_latent_gather: sequence b's visible cache rows (from max(0, context - window + 1) on, from 0
  * without a window, to its last new row) behind those of the sequences before it: rows [num_rows, width].
  * max_seq_rows: the most rows of one sequence.
+ * key_first > 0 (one sequence): from its visible row key_first on.
  * vla_seq_latent_prompt: out [T, heads * vdim] from q [T, heads * (dim + rot)] (a head's row: plain | rotated),
  * keys [num_rows, heads * dim] and values [num_rows, heads * vdim] that the caller formed from the gathered
- * latents, keys_rest (as keys) what rounding to 16 bits took from the keys (scores are of their sum), and the gathered rows themselves for the rotated parts behind them.
- * Rows of a sequence whose lengths on the device are beyond those that rows were gathered for are NaN. */
+ * latents, keys_rest (as keys) what rounding to 16 bits took from the keys (scores are of their sum), and the
+ * gathered rows themselves for the rotated parts behind them.
+ * One sequence's keys may come in ranges, one call after the other: num_rows rows from row key_first (a multiple of
+ * 64) of its key_total visible ones on, whole tiles of 64 except at the end, and carry, fp32 [T, heads, 68 or
+ * (vdim above 64) 132], 16-byte aligned, in which a call leaves what the next goes on from.  The call with
+ * key_first 0 starts, the one that ends at key_total writes out.  All keys at once: 0, 0 and null.
+ * Rows of a sequence whose lengths on the device are not those that rows were gathered for are NaN. */
 int vla_seq_latent_prompt_supported(int dim, int rot, int vdim, int rank, int dtype);
 int vla_seq_latent_gather(void* rows, int num_rows, const void* cache, const int* block_tables,
                           int max_blocks, const int* query_start_loc, const int* context_lens, int num_seqs,
-                          int max_seq_rows, int width, int block_size, int num_blocks, int window, int dtype,
-                          void* stream);
+                          int max_seq_rows, int width, int block_size, int num_blocks, int window, int key_first,
+                          int dtype, void* stream);
 int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* keys,
                           const void* keys_rest, const void* values, const void* rows, int num_rows, const int* query_start_loc,
                           const int* context_lens, int num_seqs, int max_query_len, int heads, int dim,
                           int rot, int vdim, int rank, float scale, int window, const void* gate,
-                          int64_t gate_stride, const float* sinks, int dtype, void* stream);
+                          int64_t gate_stride, const float* sinks, int key_first, int key_total, float* carry,
+                          int dtype, void* stream);
 
 /* ---- gated delta rule ----------------------------------------------------------------------------- */
 

@@ -117,6 +117,50 @@ def layer_and_step(lens, contexts, sizes, window=0, sinks=False, dtype=torch.bfl
     return attn, batch, q, kv, gate, rnd((blocks, 16, C + Rr), 8).to(dtype).to(DEV)
 
 
+@pytest.mark.parametrize("sizes", [(4, 128, 64, 128, 128), (3, 40, 16, 56, 64), (2, 136, 56, 72, 32)])
+@pytest.mark.parametrize("lens,contexts", [([70, 64, 200], [500, 64, 0]), ([300], [1000]), ([50, 60], [1500, 3])])
+@pytest.mark.parametrize("window,sinks", [(0, True), (150, False), (700, True)])
+def test_a_workspace_of_few_keys(sizes, lens, contexts, window, sinks):
+    """Sequences and ranges of a sequence's keys one after the other: as with all keys at once (the products over
+    fewer rows may sum in another order: one rounding of a key), in no more memory than the workspace."""
+    attn, batch, q, kv, gate, cache = layer_and_step(lens, contexts, sizes, window, sinks)
+    want = attn(q.clone(), kv, cache.clone(), batch, gate)
+    H, D, Rr, V, C = sizes
+    each = 2 * (C + Rr + H * (2 * D + V))
+    for keys in (64, 192, 640):
+        attn.FORMED_WORKSPACE = keys * each
+        assert attn.formed_keys(2) == keys
+        q2, cache2 = q.clone(), cache.clone()
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        held = torch.cuda.memory_allocated()
+        got = attn(q2, kv, cache2, batch, gate)
+        assert float((got - want).abs().max()) <= 0.008 * float(want.abs().max())
+        rows_own = sum(lens) * H * (4 * 132 + 2 * V) + 2 * H * C * V
+        assert torch.cuda.max_memory_allocated() - held <= keys * each + rows_own + (1 << 20)
+
+
+@pytest.mark.parametrize("lens,contexts,most", [([48], [1 << 17], 19968), ([100, 3000, 64, 64], [0, 50000, 9, 900], 4096),
+                                                ([64] * 40, [1000] * 40, 2048), ([64, 64], [0, 0], 64)])
+@pytest.mark.parametrize("window", [0, 1024])
+def test_parts_of_a_step(lens, contexts, most, window):
+    """Every visible key of every sequence once, in order, at most so many at a time."""
+    from vllm_legacy_amd.attention.backends.latent_kv import LatentKVAttention
+    attn = LatentKVAttention(2, 32, 0, 32, 64, 0.1, 0, 1e4, None, 1e-5, torch.bfloat16, DEV, window=window or None)
+    parts = attn._formed_parts(lens, contexts, most)
+    counts = [c + n - (max(0, c - window + 1) if window else 0) for n, c in zip(lens, contexts)]
+    at = key = 0
+    for b0, b1, k0, count, total in parts:
+        assert 0 < count <= most and (b0, k0) == (at, key)
+        if b1 > b0 + 1 or count == total:
+            assert k0 == 0 and count == total == sum(counts[b0:b1])
+            at = b1
+        else:
+            assert total == counts[b0] and (count % 64 == 0 or k0 + count == total)
+            at, key = (b1, 0) if k0 + count == total else (b0, k0 + count)
+    assert (at, key) == (len(lens), 0)
+
+
 @pytest.mark.parametrize("row", [0, 1, 31, 40, 63, 64, 127, 200])
 @pytest.mark.parametrize("window", [0, 70])
 @pytest.mark.parametrize("value", [float("nan"), float("inf")])
@@ -140,6 +184,9 @@ def test_lengths_that_are_not_the_hosts():
     good = attn(q.clone(), kv, cache.clone(), batch, gate)
     got = attn(q.clone(), kv, cache.clone(), replace(batch, host_context_lens=[136, 40]), gate)
     assert bool(got[100:].isnan().all()) and torch.equal(got[:100], good[:100])
+    attn.FORMED_WORKSPACE = 0
+    got = attn(q.clone(), kv, cache.clone(), replace(batch, host_context_lens=[136, 40]), gate)
+    assert bool(got[:100].isnan().all())
     stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
     assert attn._stretches(batch) is not None
     with torch.cuda.stream(stream):
@@ -147,3 +194,16 @@ def test_lengths_that_are_not_the_hosts():
         inside = attn._stretches(batch)
         graph.capture_end()
     assert inside is None
+
+
+@pytest.mark.parametrize("workspace", [1 << 28, 1 << 22])
+def test_a_portion_of_a_long_context(workspace):
+    """A hundred thousand cached tokens, all at once and in ranges, beside the latent kernel."""
+    from dataclasses import replace
+    attn, batch, q, kv, gate, cache = layer_and_step([70, 50], [100000, 33], (2, 64, 32, 64, 64))
+    attn.FORMED_WORKSPACE = workspace
+    assert (attn.formed_keys(2) > 100200) == (workspace == 1 << 28)
+    got = attn(q.clone(), kv, cache.clone(), batch, gate)
+    want = attn(q.clone(), kv, cache.clone(), replace(batch, host_query_lens=None), gate)
+    for rows in (slice(0, 70), slice(70, 120)):
+        assert float((got[rows] - want[rows]).abs().max()) <= 0.03 * float(want[rows].abs().max())

@@ -151,8 +151,8 @@ def seq_lib():
         L.vla_seq_gla_chunks.argtypes = [p, i64, p, i64, p, i64, p, i64, p, i64, p, i64, p, p, p, p, p, p, p, i, i, i, i,
                                          i, i, i, f, f, f, f, p, i64, i, p]
         L.vla_seq_latent_prompt_supported.argtypes = [i, i, i, i, i]
-        L.vla_seq_latent_gather.argtypes = [p, i, p, p, i, p, p, i, i, i, i, i, i, i, p]
-        L.vla_seq_latent_prompt.argtypes = [p, i64, p, i64, p, p, p, p, i, p, p, i, i, i, i, i, i, i, f, i, p, i64, p, i, p]
+        L.vla_seq_latent_gather.argtypes = [p, i, p, p, i, p, p, i, i, i, i, i, i, i, i, p]
+        L.vla_seq_latent_prompt.argtypes = [p, i64, p, i64, p, p, p, p, i, p, p, i, i, i, i, i, i, i, f, i, p, i64, p, i, i, p, i, p]
         L.vla_seq_delta_rule_scan_blocks.argtypes = L.vla_seq_delta_rule_scan.argtypes[:-1] + [i64, p]
         L.vla_seq_delta_rule_block_scratch_floats.argtypes = [i, i, i, i, i, i]
         L.vla_seq_delta_rule_block_scratch_floats.restype = i64

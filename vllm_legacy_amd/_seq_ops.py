@@ -1134,9 +1134,10 @@ def latent_prompt_supported(q: torch.Tensor, dim: int, rot: int, vdim: int, rank
 
 
 def latent_gather(rows: torch.Tensor, cache: torch.Tensor, block_tables: torch.Tensor, query_start_loc: torch.Tensor,
-                  context_lens: torch.Tensor, max_seq_rows: int, window: int = 0) -> None:
+                  context_lens: torch.Tensor, max_seq_rows: int, window: int = 0, key_first: int = 0) -> None:
     """rows [N, rank + rot] <- every sequence's cache rows that its new rows can see, one sequence behind the
-    other (N: their number, max_seq_rows: the most of one sequence)."""
+    other (N: their number, max_seq_rows: the most of one sequence); key_first > 0: the one sequence's from that
+    row on."""
     _gpu(rows, cache, block_tables, query_start_loc, context_lens)
     NB, BS, width = cache.shape
     B = context_lens.numel()
@@ -1148,17 +1149,24 @@ def latent_gather(rows: torch.Tensor, cache: torch.Tensor, block_tables: torch.T
         seq_check(_lib.seq_lib().vla_seq_latent_gather(
             rows.data_ptr(), rows.shape[0], cache.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
             query_start_loc.data_ptr(), context_lens.data_ptr(), B, int(max_seq_rows), width, BS, NB, int(window),
-            _dt(cache.dtype), _stream(cache.device)), "latent_gather")
+            int(key_first), _dt(cache.dtype), _stream(cache.device)), "latent_gather")
+
+
+def latent_prompt_carry(q: torch.Tensor, heads: int, vdim: int) -> torch.Tensor:
+    """What latent_prompt keeps of the rows q between ranges of keys."""
+    return torch.empty((q.shape[0], heads, 68 if vdim <= 64 else 132), dtype=torch.float32, device=q.device)
 
 
 def latent_prompt(out: torch.Tensor, q: torch.Tensor, keys: torch.Tensor, keys_rest: torch.Tensor,
                   values: torch.Tensor, rows: torch.Tensor, query_start_loc: torch.Tensor, context_lens: torch.Tensor, max_query_len: int, heads: int, dim: int,
                   rot: int, vdim: int, scale: float, window: int = 0, gate: Optional[torch.Tensor] = None,
-                  sinks: Optional[torch.Tensor] = None) -> None:
+                  sinks: Optional[torch.Tensor] = None, key_first: int = 0, key_total: int = 0,
+                  carry: Optional[torch.Tensor] = None) -> None:
     """out [T, H * vdim]; q [T, H * (dim + rot)] (views with free row strides); keys [N, H * dim] and values
     [N, H * vdim] formed from the gathered rows [N, rank + rot] of latent_gather; keys_rest [N, H * dim]: what the
-    keys lost to rounding."""
-    _gpu(out, q, keys, keys_rest, values, rows, query_start_loc, context_lens, gate, sinks)
+    keys lost to rounding.  carry (latent_prompt_carry): one sequence's key_total keys come in ranges, this one
+    from key_first on, a call for each."""
+    _gpu(out, q, keys, keys_rest, values, rows, query_start_loc, context_lens, gate, sinks, carry)
     T, N, H, B = q.shape[0], rows.shape[0], int(heads), context_lens.numel()
     assert out.dtype == q.dtype == keys.dtype == keys_rest.dtype == values.dtype == rows.dtype
     assert keys.shape == keys_rest.shape == (N, H * dim) and keys_rest.is_contiguous() and values.shape == (N, H * vdim) and out.shape == (T, H * vdim)
@@ -1168,9 +1176,12 @@ def latent_prompt(out: torch.Tensor, q: torch.Tensor, keys: torch.Tensor, keys_r
     for t in (query_start_loc, context_lens):
         assert t.dtype == torch.int32 and t.is_contiguous()
     assert query_start_loc.numel() == B + 1
+    assert carry is None or (carry.shape == (T, H, 68 if vdim <= 64 else 132) and carry.dtype == torch.float32 and
+                             carry.is_contiguous())
     with torch.cuda.device(q.device):
         seq_check(_lib.seq_lib().vla_seq_latent_prompt(
             out.data_ptr(), _rows(out, H * vdim), q.data_ptr(), _rows(q, H * (dim + rot)), keys.data_ptr(),
             keys_rest.data_ptr(), values.data_ptr(), rows.data_ptr(), N, query_start_loc.data_ptr(), context_lens.data_ptr(), B,
             int(max_query_len), H, int(dim), int(rot), int(vdim), rows.shape[1] - int(rot), float(scale), int(window),
-            _p(gate), 0 if gate is None else _rows(gate, H), _p(sinks), _dt(q.dtype), _stream(q.device)), "latent_prompt")
+            _p(gate), 0 if gate is None else _rows(gate, H), _p(sinks), int(key_first), int(key_total), _p(carry),
+            _dt(q.dtype), _stream(q.device)), "latent_prompt")

@@ -3,8 +3,8 @@
 Per token the layer caches one row [c | k_rot]: the RMS-normed latent c (`rank` numbers) and a
 rotated key part (`rot` numbers) that all heads share -- cache [num_blocks, block_size, rank + rot].
 Head h scores a query (q_plain [dim], q_rot [rot]) against key j as
-(q_plain . W_uk,h c_j + q_rot . k_rot_j) * scale and sums values W_uv,h c_j.  Both up-projections
-are moved to the query's side, where they cost one batched matrix product per step each:
+(q_plain . W_uk,h c_j + q_rot . k_rot_j) * scale and sums values W_uv,h c_j.  For single rows and
+short runs both up-projections are moved to the query's side, where they cost one batched matrix product per step each:
 q_lat,h = W_uk,h^T q_plain,h scores the cached latent directly, and the head's output is
 W_uv,h (sum_j p_j c_j).  Rotation: pairs (2i, 2i + 1) when `interleaved`, (i, i + rot_dims / 2)
 otherwise, of the first `rot_dims` elements of the rotated parts turn by position * f_i, sine and
@@ -14,10 +14,11 @@ an optional gate [T, heads] multiplies each head's output by its sigmoid (applie
 sums, ahead of the linear up-projection).  `sinks` gives every head a learned number whose
 exponential joins its softmax denominator (a key without a value, not scaled).  With
 `own_latent=False` the layer forms no latents: it reads the cache another layer fills (same rank, no
-rotated part), with queries and up-projections of its own.  Prompts, portions of prompts and decode
-steps are one case: the step's rows are written to the cache, then every query row reads from there
+rotated part), with queries and up-projections of its own.  In prompts, portions of prompts
+and decode steps alike the step's rows are written to the cache, then every query row reads from there
 (csrc/seq_latent_attention.hip: a matrix-core kernel for 16-bit models whose rank is a multiple of 32 and whose rotated part is a multiple of 16,
-and an fp32 kernel for any dtype and size).
+and an fp32 kernel for any dtype and size).  Runs of many rows with enough work form every head's keys and values from
+the cached latents instead, in a workspace of fixed size, and score those (csrc/seq_latent_prompt.hip).
 """
 import math
 from typing import Dict, Optional, Tuple
@@ -156,27 +157,64 @@ class LatentKVAttention(nn.Module):
             return None
         return out if len(out) <= self.MAX_STRETCHES else None
 
+    # bytes of gathered rows and formed keys and values at a time: 20 thousand keys of 16 heads of 128 + 128
+    FORMED_WORKSPACE = 1 << 28
+
+    def formed_keys(self, size: int) -> int:
+        """Keys that FORMED_WORKSPACE holds (whole tiles of 64, at least one): their cache rows, keys in two parts
+        and values, `size` bytes a number."""
+        each = size * (self.rank + self.rot_dim + self.num_heads * (2 * self.head_dim + self.value_dim))
+        return max(64, self.FORMED_WORKSPACE // each // 64 * 64)
+
+    def _formed_parts(self, lens, contexts, most: int):
+        """[(first sequence, one behind the last, first key, keys, all keys)]: neighbours whose visible keys are at
+        most `most` together, and ranges of the keys of one that has more by itself."""
+        parts, first, held = [], 0, 0
+        for b, (n, c) in enumerate(zip(lens, contexts)):
+            count = c + n - (max(0, c - self.window + 1) if self.window else 0)
+            if held and held + count > most:
+                parts.append((first, b, 0, held, held))
+                held = 0
+            if count > most:
+                parts += [(b, b + 1, k, min(most, count - k), count) for k in range(0, count, most)]
+                first = b + 1
+            else:
+                first = first if held else b
+                held += count
+        if held:
+            parts.append((first, len(lens), 0, held, held))
+        return parts
+
     def _attend_formed(self, out, q, cache, batch: SequenceBatch, s0, s1, r0, r1, gate) -> None:
         """Sequences s0 .. s1 - 1 (rows r0 .. r1 - 1) with keys and values formed per head."""
         H, D, Rr, V, C = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.rank
         ql, cl = batch.host_query_lens[s0:s1], batch.host_context_lens[s0:s1]
-        counts = [c + n - (max(0, c - self.window + 1) if self.window else 0) for n, c in zip(ql, cl)]
-        tables, ctx = batch.block_tables[s0:s1], batch.context_lens[s0:s1]
-        starts = batch.query_start_loc[s0:s1 + 1]
-        if r0:
-            starts = starts - r0
-        rows = torch.empty((sum(counts), C + Rr), dtype=q.dtype, device=q.device)
-        ops.latent_gather(rows, cache, tables, starts, ctx, max(counts), self.window)
-        latents = rows[:, :C]
-        # A key's rounding is its own, where that of a query on the latents' side is the same for all keys and mostly
-        # cancels in the softmax: the keys keep what they lose.
-        w_uk = self.w_uk.data.view(H * D, C).t()
-        keys = torch.mm(latents, w_uk)
-        keys_rest = torch.addmm(keys, latents, w_uk, beta=-1)
-        values = torch.mm(latents, self.w_uv_t.data.transpose(0, 1).reshape(C, H * V))
-        ops.latent_prompt(out[r0:r1], q[r0:r1], keys, keys_rest, values, rows, starts, ctx, max(ql), H, D, Rr, V, self.scale,
-                          self.window, None if gate is None else gate[r0:r1],
-                          None if self.sinks is None else self.sinks.data)
+        sinks = None if self.sinks is None else self.sinks.data
+        w_uk = self.w_uk.data.reshape(H * D, C).t()
+        w_uv = self.w_uv_t.data.transpose(0, 1).reshape(C, H * V)
+        carry = None
+        for b0, b1, k0, count, total in self._formed_parts(ql, cl, self.formed_keys(q.element_size())):
+            if k0 == 0:
+                t0 = r0 + sum(ql[:b0])
+                t1 = t0 + sum(ql[b0:b1])
+                tables, ctx = batch.block_tables[s0 + b0:s0 + b1], batch.context_lens[s0 + b0:s0 + b1]
+                starts = batch.query_start_loc[s0 + b0:s0 + b1 + 1]
+                if t0:
+                    starts = starts - t0
+                carry = ops.latent_prompt_carry(q[t0:t1], H, V) if count < total else None
+            rows = torch.empty((count, C + Rr), dtype=q.dtype, device=q.device)
+            longest = count if b1 == b0 + 1 else max(c + n for n, c in zip(ql[b0:b1], cl[b0:b1]))
+            ops.latent_gather(rows, cache, tables, starts, ctx, longest, self.window, k0)
+            latents = rows[:, :C]
+            # A key's rounding is its own, where that of a query on the latents' side is the same for all keys and
+            # mostly cancels in the softmax: the keys keep what they lose.
+            keys = torch.mm(latents, w_uk)
+            keys_rest = torch.addmm(keys, latents, w_uk, beta=-1)
+            values = torch.mm(latents, w_uv)
+            ops.latent_prompt(out[t0:t1], q[t0:t1], keys, keys_rest, values, rows, starts, ctx, max(ql[b0:b1]), H, D, Rr, V,
+                              self.scale, self.window, None if gate is None else gate[t0:t1], sinks, k0,
+                              total if carry is not None else 0, carry)
+            del rows, latents, keys, keys_rest, values          # the next part's take their place
 
     def _attend_latent(self, q, cache, batch: SequenceBatch, s0, s1, r0, r1, gate) -> torch.Tensor:
         """Sequences s0 .. s1 - 1 (rows r0 .. r1 - 1) on the cached latents -> [rows, heads * vdim]."""

@@ -94,9 +94,9 @@ __device__ __forceinline__ int gathered_before(const int* __restrict__ query_sta
 __global__ __launch_bounds__(256) void latent_gather_kernel(
     u32x4* __restrict__ rows, const u32x4* __restrict__ cache, const int* __restrict__ block_tables,
     int max_blocks, const int* __restrict__ query_start_loc, const int* __restrict__ context_lens,
-    int pieces, int block_size, int num_blocks, int window, int num_rows) {
+    int pieces, int block_size, int num_blocks, int window, int num_rows, int key_first) {
   const int b = blockIdx.y;
-  const int ctx = context_lens[b], first = first_formed(ctx, window);
+  const int ctx = context_lens[b], first = first_formed(ctx, window) + key_first;
   const int n = ctx + query_start_loc[b + 1] - query_start_loc[b] - first;
   if ((int)blockIdx.x * kGatherRows >= n) return;
   const int base = gathered_before(query_start_loc, context_lens, b, window);
@@ -129,7 +129,9 @@ struct LatentPrompt {
   const void* gate;
   int64_t gate_stride;
   const float* sinks;
+  float* carry;                 // one sequence whose keys come in ranges: [T, heads, VD + 4], null otherwise
   int heads, dim, rot, vdim, rank, window, num_rows, row_tiles;
+  int key_first, key_total;     // the range's first key and all keys of the sequence
   float scale;
 };
 
@@ -165,21 +167,23 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
   if (r0 >= run) return;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hf = lane >> 5, c = lane & 31;
-  const int ctx = a.context_lens[b], first = first_formed(ctx, a.window);
-  const int base = gathered_before(a.query_start_loc, a.context_lens, b, a.window);
+  const bool ranged = a.carry != nullptr, last_range = !ranged || a.key_first + a.num_rows == a.key_total;
+  const int ctx = a.context_lens[b], first = first_formed(ctx, a.window) + (ranged ? a.key_first : 0);
+  const int base = ranged ? 0 : gathered_before(a.query_start_loc, a.context_lens, b, a.window);
   const int n_rows = min(kRowsPerGroup, run - r0);         // rows of this workgroup
   const int nq = min(kRowsPerWave, n_rows - kRowsPerWave * w);               // and of this wave (<= 0: none)
   const int t0 = a.query_start_loc[b] + r0 + kRowsPerWave * w;
+  // positions, counted from the first gathered key
+  const int p0 = ctx + r0 + kRowsPerWave * w - first, pq = p0 + c;
+  const int n_keys = min(ctx + run - first, a.num_rows);
+  const int p_end = min(ctx + r0 + n_rows - 1 - first, n_keys - 1);
   T* orow = (T*)a.out + (int64_t)(t0 + c) * a.out_stride + (int64_t)h * a.vdim + 4 * hf;
-  if (base + ctx + run - first > a.num_rows) {
+  if (ranged ? ctx + run - first != a.key_total - a.key_first : base + ctx + run - first > a.num_rows) {
     // the host gathered for other lengths than the device has: no answer, and none that looks like one
     const uint32_t nan2 = M::pack2(NAN, NAN);
     for (int d = 0; c < nq && d + 4 * hf < a.vdim; d += 8) *reinterpret_cast<u32x2*>(orow + d) = u32x2{nan2, nan2};
     return;
   }
-  // positions, counted from the first gathered key
-  const int p0 = ctx + r0 + kRowsPerWave * w - first, pq = p0 + c;
-  const int p_end = ctx + r0 + n_rows - 1 - first, n_keys = ctx + run - first;
   const int g_first = a.window > 0 ? max(0, ctx + r0 - first - a.window + 1) : 0;    // the group's first key
   const int g_p0 = ctx + r0 - first, g_lo_last = a.window > 0 ? g_p0 + kRowsPerGroup - a.window : 0;    // the group's
   const int lo_q = a.window > 0 ? pq - a.window + 1 : 0;                       // this row's
@@ -206,6 +210,19 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
   if (a.sinks != nullptr) {                                // the denominator's first term, counted in one lane half
     m = a.sinks[h] * 1.4426950408889634f;
     l = hf == 0 ? 1.f : 0.f;
+  }
+  float* carry = a.carry + ((int64_t)(t0 + c) * a.heads + h) * (VD + 4);
+  if (ranged && a.key_first > 0 && c < nq) {               // where the range before this one ended
+    m = carry[0];
+    l = carry[1 + hf];
+#pragma unroll
+    for (int n = 0; n < VB; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; i += 4) {
+        const f32x4 got = *reinterpret_cast<const f32x4*>(carry + 4 + 32 * n + 8 * (i >> 2) + 4 * hf);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[n][i + e] = got[e];
+      }
   }
 
   // What this lane brings in: piece `at` of a tile in LDS is row at / pieces; which 16 bytes of the row
@@ -283,7 +300,7 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
     __syncthreads();
   };
   int u0 = g_first & ~(kKeys - 1);
-  bring_keys(u0);
+  if (u0 <= p_end) bring_keys(u0);
   for (; u0 <= p_end; u0 += kKeys) {
     landed();
     bring_values(u0);
@@ -388,6 +405,17 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
         }
       }
   }
+  if (!last_range) {
+    if (c >= nq) return;
+    if (hf == 0) carry[0] = m;
+    carry[1 + hf] = l;
+#pragma unroll
+    for (int n = 0; n < VB; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; i += 4)
+        *reinterpret_cast<f32x4*>(carry + 4 + 32 * n + 8 * (i >> 2) + 4 * hf) = f32x4{o[n][i], o[n][i + 1], o[n][i + 2], o[n][i + 3]};
+    return;
+  }
   l += __shfl_xor(l, 32, 64);
   if (c >= nq) return;
   float inv = 1.f / l;
@@ -436,17 +464,17 @@ extern "C" int vla_seq_latent_prompt_supported(int dim, int rot, int vdim, int r
 extern "C" int vla_seq_latent_gather(void* rows, int num_rows, const void* cache, const int* block_tables,
                                      int max_blocks, const int* query_start_loc, const int* context_lens,
                                      int num_seqs, int max_seq_rows, int width, int block_size,
-                                     int num_blocks, int window, int dtype, void* stream) {
+                                     int num_blocks, int window, int key_first, int dtype, void* stream) {
   if (num_seqs == 0 || num_rows == 0) return VLA_OK;
   if (!rows || !cache || !block_tables || !query_start_loc || !context_lens || num_seqs < 0 || num_seqs > 65535 ||
       num_rows < 0 || max_seq_rows <= 0 || max_blocks <= 0 || width <= 0 || block_size <= 0 || num_blocks <= 0 ||
-      window < 0)
+      window < 0 || key_first < 0 || (key_first > 0 && num_seqs > 1))
     return VLA_ERR_ARG;
   if (dtype != VLA_F16 && dtype != VLA_BF16) return VLA_ERR_DTYPE;
   if (width % 8 || (uintptr_t)rows % 16 || (uintptr_t)cache % 16) return VLA_ERR_ARG;
   latent_gather_kernel<<<dim3((max_seq_rows + kGatherRows - 1) / kGatherRows, num_seqs), 256, 0, (hipStream_t)stream>>>(
       (u32x4*)rows, (const u32x4*)cache, block_tables, max_blocks, query_start_loc, context_lens, width / 8, block_size,
-      num_blocks, window, num_rows);
+      num_blocks, window, num_rows, key_first);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   return VLA_OK;
 }
@@ -457,7 +485,8 @@ extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* 
                                      const int* query_start_loc, const int* context_lens, int num_seqs,
                                      int max_query_len, int heads, int dim, int rot, int vdim, int rank,
                                      float scale, int window, const void* gate, int64_t gate_stride,
-                                     const float* sinks, int dtype, void* stream) {
+                                     const float* sinks, int key_first, int key_total, float* carry, int dtype,
+                                     void* stream) {
   if (num_seqs == 0 || max_query_len == 0) return VLA_OK;
   if (!out || !q || !keys || !keys_rest || !values || !rows || !query_start_loc || !context_lens || num_seqs < 0 ||
       num_seqs > 65535 || max_query_len < 0 || num_rows <= 0 || heads <= 0 || heads > 65535 || !(scale > 0.f) ||
@@ -468,6 +497,11 @@ extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* 
   if (!prompt_sizes(dim, rot, vdim, rank)) return VLA_ERR_HEAD_SIZE;
   if ((uintptr_t)q % 16 || q_stride % 8 || (uintptr_t)keys % 16 || (uintptr_t)keys_rest % 16 || (uintptr_t)values % 16 || (uintptr_t)rows % 16 ||
       (uintptr_t)out % 8 || out_stride % 4)
+    return VLA_ERR_ARG;
+  // a range begins with a tile, and a tile ends with it or with the sequence
+  if (carry ? num_seqs > 1 || key_first < 0 || key_first % kKeys || key_total - num_rows < key_first ||
+                  (key_total - num_rows > key_first && num_rows % kKeys) || (uintptr_t)carry % 16
+            : key_first != 0)
     return VLA_ERR_ARG;
   LatentPrompt a;
   a.out = out;
@@ -483,6 +517,9 @@ extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* 
   a.gate = gate;
   a.gate_stride = gate_stride;
   a.sinks = sinks;
+  a.carry = carry;
+  a.key_first = key_first;
+  a.key_total = key_total;
   a.heads = heads;
   a.dim = dim;
   a.rot = rot;
