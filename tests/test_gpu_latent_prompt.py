@@ -1,8 +1,8 @@
 """Latent attention with keys and values formed per head: runs around the tiles of 128 rows and 64 keys, head
 sizes around the padding of the two kernels (128 and 192 numbers a key, 64 and 128 a value), windows, gates,
 steps that mix long runs with single rows, and what must keep taking the latent kernel.  Oracle and bound
-(6 % of the largest value where operands and weights are rounded to bfloat16) are those of the other latent
-tests; against the latent kernel itself the bound is half of that, since both round alike."""
+(6 % of the largest value where operands and weights are rounded to bfloat16, an eighth of that in float16) are
+those of the other latent tests; against the latent kernel itself the bound is half of that, since both round alike."""
 import pytest
 import torch
 
@@ -26,7 +26,8 @@ def test_runs_around_a_tile(sizes, cuts, window, dtype):
     assert attn.formed_min_rows() <= 127
     attn.FORMED_MIN_WORK = 0
     got = run_latent(attn, sizes, q, kv, gate, cuts, dtype)
-    assert float((got - want).abs().max()) <= 0.06 * float(want.abs().max())
+    bar = 0.06 if dtype == torch.bfloat16 else 0.06 / 8     # three bits more
+    assert float((got - want).abs().max()) <= bar * float(want.abs().max())
 
 
 def step(lens, contexts, block_size=16):
