@@ -136,10 +136,8 @@ class LatentKVAttention(nn.Module):
     def _stretches(self, batch: SequenceBatch):
         """[[first sequence, one behind the last, first row, one behind the last, formed]]: neighbours that go
         the same way; None when the whole step takes the latent kernel."""
-        if batch.max_query_len < self.FORMED_MIN_ROWS or not self.scale > 0:
-            return None
         least = self.formed_min_rows()
-        if batch.max_query_len < least:
+        if batch.max_query_len < least or not self.scale > 0:
             return None
         q, ctx = batch.host_query_lens, batch.host_context_lens
         if q is None or ctx is None or torch.cuda.is_current_stream_capturing():
@@ -222,11 +220,12 @@ class LatentKVAttention(nn.Module):
         whole = s0 == 0 and s1 == batch.num_seqs
         T = r1 - r0
         sinks = None if self.sinks is None else self.sinks.data
-        q3 = q[r0:r1].view(T, H, D + Rr)
+        if not whole:
+            q, gate = q[r0:r1], None if gate is None else gate[r0:r1]
+        q3 = q.view(T, H, D + Rr)
         q_lat = torch.bmm(q3[:, :, :D].transpose(0, 1), self.w_uk.data)             # [H, T, C]
         o_lat = torch.empty((H, T, C), dtype=q.dtype, device=q.device)
         q_lat, q_rot, o_rows = q_lat.transpose(0, 1), q3[:, :, D:], o_lat.transpose(0, 1)
-        gate = None if gate is None else gate[r0:r1]
         if ops.latent_attention_tiles_supported(q_lat, q_rot, cache):
             # 16-bit models whose sizes fit: (token, head) rows in tiles of 32 on the matrix cores
             if whole:
@@ -260,7 +259,7 @@ class LatentKVAttention(nn.Module):
         if self.own_latent:
             ops.latent_rotary_write(q, D + Rr, D, H, kv, self.latent_norm.data, self.eps, cache, batch.positions,
                                     batch.slot_mapping, self.inv_freq, self.magnitude, self.rot_dims, self.interleaved)
-        stretches = self._stretches(batch)
+        stretches = None if batch.max_query_len < self.FORMED_MIN_ROWS else self._stretches(batch)
         if stretches is None or not ops.latent_prompt_supported(q, D, Rr, V, C, cache):
             return self._attend_latent(q, cache, batch, 0, batch.num_seqs, 0, T, gate)
         out = torch.empty((T, H * V), dtype=q.dtype, device=q.device)
