@@ -445,8 +445,8 @@ __device__ __forceinline__ void turn_back(f32x16 (&o)[VB], int hf, float p,
 //
 // Bound by the products and the softmax between them (about 30 vector cycles per score), so the tiles
 // come in by LDS-DMA: no staging registers, no waits before the stores to LDS, one barrier per tile, two
-// tiles in LDS (at most 64 KB: two workgroups share a CU and one's softmax runs under the other's
-// products).  A DMA instruction writes 64 lanes x 16 bytes in a row, so rows cannot be padded: 16-byte
+// tiles in LDS (64 KB at most and 2 KB of the rows' places: two workgroups share a CU and one's softmax runs under
+// the other's products).  A DMA instruction writes 64 lanes x 16 bytes in a row, so rows cannot be padded: 16-byte
 // pieces of a key row and 64-byte units of a value row are exchanged by the row's number on the source's
 // side, so that the lanes of a read fall into different banks.  What only some calls need (a cap, masks)
 // is a loop of its own behind one branch.  Workgroups go out longest walk first over all sequences, and those
@@ -1029,15 +1029,16 @@ __global__ __launch_bounds__(64 * kRowWaves) void kv_attention_heads_kernel(
 //   O^T = V^T P^T  B = P^T  lane: head c, keys 4 g .. + 3 of both halves of the tile, where they lie
 //                  A = V^T  lane: value dim 16 n + c of the same keys (two transposing reads)
 // A weight enters as the sum of two 16-bit numbers, as in the kernel above.  The four waves take tiles of 32
-// keys in turn, each through its own two LDS buffers that LDS-DMA fills a tile ahead: 64 KB on their way
-// per CU without a staging register, and no barrier in the loop.  A DMA instruction writes 64 lanes x 16
+// keys in turn, each through its own two LDS buffers: while one tile is worked on the next is on its way, and the one
+// behind that is asked for, keys and values each, as soon as their place is free.  64 KB on their way per CU
+// without a staging register, and no barrier in the loop.  A DMA instruction writes 64 lanes x 16
 // bytes in a row, so rows are not padded: 16-byte pieces of a key row and 32-byte units of a value row
 // are exchanged by the row's number, on the source's side, for reads without bank conflicts.  The block
 // table's part waits in LDS, because a table load inside the loop would have to wait for the DMA ahead of
 // it.  Few rows over long contexts: the keys of a row are shared out to `splits` workgroups, whose sums
 // kv_decode_merge_kernel joins.
 // 64 rows of 4096 keys, 16 / 4 heads of 128 (537 MB): 95 us = 5.6 TB/s (the kernel above 122; without the
-// nontemporal hint 108; one tile ahead instead of two, also without the hint, 106).
+// nontemporal hint 108; a tile asked for only when the one before it is done with, also without the hint, 106).
 constexpr int kDecodeWaves = 4;
 constexpr int kDecodeHeads = 16;
 constexpr int kDecodeKeys = 32;
@@ -1749,6 +1750,7 @@ extern "C" int vla_seq_kv_attention_tiles(
   const int head_waves = group >= 3 ? 4 : group;      // waves of a workgroup that are heads
   const int tile_rows = kTile * (4 / head_waves);
   const int head_groups = kv_heads * ((group + head_waves - 1) / head_waves);
+  // (the launch counts every sequence as long as the longest: a prompt beside many single rows keeps one group)
   // few workgroups share their keys out to two groups of four waves: of 2047 rows, 16 heads on 4 of 128, one run
   // (256 workgroups) takes 68 us instead of 88, two take 76 instead of 100; four fill the chip with independent
   // ones (116 instead of 138: two workgroups of a CU do not wait for each other)

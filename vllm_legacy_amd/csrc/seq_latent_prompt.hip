@@ -5,7 +5,7 @@
 // queries of the run.  A run of rows therefore gathers its visible cache rows into one place
 // (latent_gather_kernel), the caller multiplies them with the two up-projections, and
 // latent_prompt_kernel below is plain causal attention with keys [formed (dim) | shared rotated part
-// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 182 us (480 TFLOP/s; 620
+// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 184 us (470 TFLOP/s; 650
 // with the remainders' product) where latent_attention_tile_kernel takes 1685, plus 9 us to gather and 60 for the
 // three products (the products on the query's side that they replace take 46).
 //
@@ -13,7 +13,7 @@
 // side, which is the same for all keys of a row and mostly cancels in the softmax; a key's rounding is its own.
 // Outputs' error against 64 bits, this / one 16-bit number / the latent kernel, bf16, 1e-3: independent latents
 // 2.5 / 2.8 / 2.8, with scores four times as large 2.4 / 3.8 / 3.6 (float16: an eighth of each).  One number
-// per key takes 136 us, and 189 instead of 258 for the whole layer.
+// per key takes 136 us, and 189 instead of 257 for the whole layer.
 //
 // The rows of sequence b are its keys from first_b = max(0, context - window + 1) (0 without a window) to
 // its last new row; sequences follow each other, so a sequence's place is the sum of the counts before

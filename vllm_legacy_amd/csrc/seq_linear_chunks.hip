@@ -16,7 +16,7 @@
 // states after 4096 rows several times as far from 64 bits).
 // All products run on 16x16x4 fp32 matrix cores.  Operands that later kernels read lie in scratch lane for
 // lane.  Bound by memory and the launches: 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB
-// of chunk states and decays; 158 us (56 + 23 + 79) where the pieces of 256 rows walked
+// of chunk states and decays; 152 us per call (57 + 23 + 82 under the tracer) where the pieces of 256 rows walked
 // token by token and joined by matrix products took 408.
 #include <atomic>
 
