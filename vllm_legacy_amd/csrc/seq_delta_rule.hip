@@ -31,7 +31,7 @@
 // delta_block_prepare_kernel forms it for all blocks at once, one workgroup per block and head, and
 // leaves W, Q~, K^, G_31, A and T V in scratch; delta_block_walk_kernel goes over a run's blocks in
 // order, a workgroup per 16 columns of S, whose rows its four waves share and keep in registers.  All
-// products run on 16x16x4 fp32 matrix cores.
+// products run on 16x16x4 matrix cores: what the preparation forms and K^^T U in 64 bits, those with S in 32.
 #include <algorithm>
 #include <atomic>
 
@@ -370,6 +370,8 @@ constexpr int kRows = 32;
 constexpr int kStepRows = 4;        // runs of at most this many rows go token by token beside blocks
 constexpr int kMaxBlockDim = 256;
 constexpr int kMat = 36;            // floats per row of a 32 x 32 matrix in LDS
+constexpr int kMatB = 34;           // and of one in 64 bits
+constexpr int kMatT = 18;           // and of a 16 x 16 one
 
 struct DeltaBlocks {
   float* o;                         // [T][heads * vdim]
@@ -429,9 +431,9 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
   float* k_lds = lds;                                      // [32][RS]
   float* q_lds = k_lds + kRows * RS;                       // [32][RS]
   float* part = q_lds + kRows * RS;                        // [4 waves][6 tiles][64 lanes][4]
-  float* b_mat = part;                                     // B, strictly lower
-  float* t_mat = b_mat + kRows * kMat;                     // (I + B)^-1
-  float* p_mat = t_mat + kRows * kMat;                     // 16 x 16 between two products, rows of 20
+  double* b_mat = reinterpret_cast<double*>(part);         // B, strictly lower
+  double* t_mat = b_mat + kRows * kMatB;                   // the 16 x 16 blocks on the diagonal of (I + B)^-1
+  double* p_mat = t_mat + 2 * 16 * kMatT;                  // [4 waves]: one between two products
   float* l_mat = part + 4 * 6 * 256;                       // [32][kMat]
   float* g_lds = l_mat + kRows * kMat;                     // [32]
   float* beta_lds = g_lds + kRows;                         // [32]
@@ -450,7 +452,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
   float* out = a.scratch + ((int64_t)slot * a.heads + h) * delta_block_floats(DP, 16 * vb);
   float* w_out = out;                                      // [DP / 16][2][lane][4]: row c, head row 4 g + e
   float* q_out = w_out + kRows * DP;                       // the same
-  float* k_out = q_out + kRows * DP;                       // [DP / 16][2][lane][4]: head row c, row 4 g + e
+  float* k_out = q_out + kRows * DP;                       // [DP / 16][2][lane][4]: head row pc (below), row 4 g + e
   float* g_out = k_out + kRows * DP;
   float* a_out = g_out + 4;                                // [3 tiles][wave][lane]
   float* u_out = a_out + 3 * 256;                          // [vb][2][lane][4]: column c, row 4 g + e
@@ -547,11 +549,12 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
 
   // k_i . k_j and q_i . k_j, lower 16 x 16 tiles; every wave takes a quarter of the head's rows (a lane
   // holds four neighbouring ones: the contraction index may be relabelled as long as both operands are).  In 64
-  // bits and of the rows as they are, and L in 64 bits too: an error in one of them is in all columns of u alike
-  // and, where keys are alike, in every u behind it.  Relative errors against 64 bits of outputs / states after
-  // 1024 rows of 128 x 128 with slow decays, in 1e-7: token by token, this, and unit rows in 32 bits:
-  // independent keys 1.9 / 1.7, 1.9 / 1.8, 2.4 / 2.2; keys with a common part as large as the rest 2.0 / 1.9,
-  // 2.2 / 2.2, 2.9 / 2.7; with one three times as large 2.5 / 2.1, 3.0 / 3.3, 4.4 / 4.1.
+  // bits and of the rows as they are, as are L, T, W and T V, each rounded once: an error in one of them is in all
+  // columns of u alike and, where keys are alike, in every u behind it.  Relative errors against 64 bits of outputs /
+  // states after 1024 rows of 128 x 128 with slow decays, in 1e-7: token by token, this, and all of it in 32 bits:
+  // independent keys 1.9 / 1.7, 1.5 / 1.4, 2.4 / 2.2; keys with a common part as large as the rest 2.0 / 1.8,
+  // 1.7 / 1.6, 2.9 / 2.7; with one three times as large 2.4 / 2.0, 2.1 / 2.1, 4.4 / 4.1; eight times 3.3 / 2.2, 2.9 / 2.6.
+  // T, W and T V in 32 bits are 8 us less per call of the size below, and 2.7 / 3.2 for keys of three times.
   {
     // L: lane j of wave 0 walks down column j (lane 32: from the block's start)
     if (w == 0) {
@@ -627,22 +630,23 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
     const int at = tid + 256 * u, tile = at >> 6, kind = tile % 3;
     if (at < 6 * 64) {
       const int i0 = kind > 0 ? 16 : 0, j0 = kind > 1 ? 16 : 0, j = j0 + c;
-      float v[4];
+      double got[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const double unit = sum[u][e] * (double)(tile < 3 ? ks_lds : qs_lds)[i0 + 4 * g + e] * (double)ks_lds[j];
-        v[e] = (float)(unit * (double)l_mat[(i0 + 4 * g + e) * kMat + j]);
+        got[e] = unit * (double)l_mat[(i0 + 4 * g + e) * kMat + j];
       }
       if (tile < 3) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int i = i0 + 4 * g + e;
-          b_mat[i * kMat + j] = i > j ? beta_lds[i] * v[e] : 0.f;
+          b_mat[i * kMatB + j] = i > j ? (double)beta_lds[i] * got[e] : 0.;
         }
       } else {
         // A as the walk's waves take it: wave c & 3 meets contraction index 4 (c >> 2) + (c & 3)
+        float v[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = i0 + 4 * g + e >= j ? v[e] : 0.f;
+        for (int e = 0; e < 4; ++e) v[e] = i0 + 4 * g + e >= j ? (float)got[e] : 0.f;
         *reinterpret_cast<f32x4*>(a_out + (kind * 4 + (c & 3)) * 64 + ((c >> 2) << 4) + 4 * g) = f32x4{v[0], v[1], v[2], v[3]};
       }
     }
@@ -654,19 +658,20 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
   // below through lane exchanges
   if (w < 2) {
     const int at = 16 * w;
-    f32x4 bv[4][4];                                        // [e][chunk]: B's row 4 g + e
+    f64x4 bv[4][4];                                        // [e][chunk]: B's row 4 g + e
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int ch = 0; ch < 4; ++ch)
-        bv[e][ch] = *reinterpret_cast<const f32x4*>(b_mat + (at + 4 * g + e) * kMat + at + 4 * ch);
-    float x[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = 4 * g + e == c ? 1.f : 0.f;
+        for (int f = 0; f < 4; ++f) bv[e][ch][f] = b_mat[(at + 4 * g + e) * kMatB + at + 4 * ch + f];
+    double x[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = 4 * g + e == c ? 1. : 0.;
 #pragma unroll
     for (int ch = 0; ch < 4; ++ch) {
       // rows 4 ch .. 4 ch + 3, right in the lanes g == ch (the others' results are not used)
-      float y[4];
+      double y[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         y[e] = x[e];
@@ -682,14 +687,14 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int f = 0; f < 4; ++f) x[e] -= (g > ch ? bv[e][ch][f] : 0.f) * y[f];
+        for (int f = 0; f < 4; ++f) x[e] -= (g > ch ? bv[e][ch][f] : 0.) * y[f];
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) t_mat[(at + 4 * g + e) * kMat + at + c] = x[e];
+    for (int e = 0; e < 4; ++e) t_mat[(at + 4 * g + e) * kMatT + c] = x[e];
   } else {
     if (tid == 128) g_out[0] = l_mat[(kRows - 1) * kMat + kRows];
     for (int i = tid - 128; i < DP * (kRows / 4); i += 128) {
-      const int d = 16 * (i >> 7) + (i & 15), j = 4 * ((i >> 4) & 7);    // i: tile, half, lane
+      const int d = 16 * (i >> 7) + 4 * (i & 3) + ((i >> 2) & 3), j = 4 * ((i >> 4) & 7);    // i: tile, half, lane (row pc)
       const f32x4 lv = *reinterpret_cast<const f32x4*>(l_mat + (kRows - 1) * kMat + j);
       const f32x4 ks = *reinterpret_cast<const f32x4*>(ks_lds + j);
       f32x4 kh;
@@ -699,60 +704,64 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
     }
   }
   __syncthreads();
+  // Row `pc` of an operand is row c of a 64-bit product, so that a lane's four results are neighbours: rows g + 4 i of
+  // the product are rows 4 g + i.
+  const int pc = 4 * (c & 3) + (c >> 2);
   // the block below them: -T22 (B21 T11), every wave for itself
-  f32x4 t21;
+  double t21[4];
   {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    const f32x4 b21 = *reinterpret_cast<const f32x4*>(b_mat + (16 + c) * kMat + 4 * g);
+    f64x4 acc = {0., 0., 0., 0.}, neg = {0., 0., 0., 0.};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc = mfma4(b21[e], t_mat[(4 * g + e) * kMat + c], acc);
+    for (int e = 0; e < 4; ++e) acc = mfma4_f64(b_mat[(16 + pc) * kMatB + 4 * g + e], t_mat[(4 * g + e) * kMatT + c], acc);
     // acc is the next product's B operand where it lies: column c, contraction index 4 g + e
-    const f32x4 t22 = *reinterpret_cast<const f32x4*>(t_mat + (16 + c) * kMat + 16 + 4 * g);
-    f32x4 neg = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) neg = mfma4(t22[e], acc[e], neg);
-    // from column c, rows 4 g + e to row c, columns 4 g + e
-    float* mine = p_mat + w * 16 * 20;
+    for (int e = 0; e < 4; ++e) neg = mfma4_f64(t_mat[(16 + pc) * kMatT + 4 * g + e], acc[e], neg);
+    // from column c, rows 4 g + e to row pc, columns 4 g + e
+    double* mine = p_mat + w * 16 * kMatT;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) mine[(4 * g + e) * 20 + c] = -neg[e];
+    for (int e = 0; e < 4; ++e) mine[(4 * g + e) * kMatT + c] = -neg[e];
     wave_sync();
-    t21 = *reinterpret_cast<const f32x4*>(mine + c * 20 + 4 * g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t21[e] = mine[pc * kMatT + 4 * g + e];
   }
 
   // rows of T diag(beta) as operands: 0: rows 0 .. 15; 1 and 2: rows 16 .. 31 with the first and the
   // second half of the contraction
-  f32x4 tv[3], gj[2];
-  tv[0] = *reinterpret_cast<const f32x4*>(t_mat + c * kMat + 4 * g);
-  tv[1] = t21;
-  tv[2] = *reinterpret_cast<const f32x4*>(t_mat + (16 + c) * kMat + 16 + 4 * g);
+  double tv[3][4], gj[2][4];
 #pragma unroll
-  for (int p = 0; p < 3; ++p) {
-    const f32x4 be = *reinterpret_cast<const f32x4*>(beta_lds + (p > 1 ? 16 : 0) + 4 * g);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) tv[p][e] *= be[e];
+  for (int e = 0; e < 4; ++e) {
+    const double be0 = beta_lds[4 * g + e], be1 = beta_lds[16 + 4 * g + e];
+    tv[0][e] = t_mat[pc * kMatT + 4 * g + e] * be0;
+    tv[1][e] = t21[e] * be0;
+    tv[2][e] = t_mat[(16 + pc) * kMatT + 4 * g + e] * be1;
   }
 #pragma unroll
   for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) gj[jt][e] = l_mat[(16 * jt + 4 * g + e) * kMat + kRows] * ks_lds[16 * jt + 4 * g + e];
+    for (int e = 0; e < 4; ++e)
+      gj[jt][e] = (double)l_mat[(16 * jt + 4 * g + e) * kMat + kRows] * (double)ks_lds[16 * jt + 4 * g + e];
 #pragma unroll
   for (int x = 0; x < DX; ++x) {
     const int tile = w + 4 * x;
-    f32x4 xt[2];
+    f64x4 xt[2];
 #pragma unroll
-    for (int it = 0; it < 2; ++it) xt[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // transposed, so that a lane ends with four neighbouring rows of the head of one token
+    for (int it = 0; it < 2; ++it) xt[it] = f64x4{0., 0., 0., 0.};
+    // transposed, so that a lane ends with four neighbouring rows of the head of one token (row pc)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float ka = k_lds[(4 * g + e) * RS + 16 * tile + c] * gj[0][e];
-      const float kb = k_lds[(16 + 4 * g + e) * RS + 16 * tile + c] * gj[1][e];
-      xt[0] = mfma4(ka, tv[0][e], xt[0]);
-      xt[1] = mfma4(ka, tv[1][e], xt[1]);
-      xt[1] = mfma4(kb, tv[2][e], xt[1]);
+      const double ka = (double)k_lds[(4 * g + e) * RS + 16 * tile + pc] * gj[0][e];
+      const double kb = (double)k_lds[(16 + 4 * g + e) * RS + 16 * tile + pc] * gj[1][e];
+      xt[0] = mfma4_f64(ka, tv[0][e], xt[0]);
+      xt[1] = mfma4_f64(ka, tv[1][e], xt[1]);
+      xt[1] = mfma4_f64(kb, tv[2][e], xt[1]);
     }
 #pragma unroll
-    for (int it = 0; it < 2; ++it)
-      *reinterpret_cast<f32x4*>(w_out + ((tile * 2 + it) * 64 + lane) * 4) = xt[it];
+    for (int it = 0; it < 2; ++it) {
+      f32x4 put;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) put[e] = (float)xt[it][e];
+      *reinterpret_cast<f32x4*>(w_out + ((tile * 2 + it) * 64 + 16 * g + pc) * 4) = put;
+    }
   }
   for (int vt = w; vt < vb; vt += 4) {
     int from = odd_from;                                   // column c's first row that is not finite
@@ -769,20 +778,22 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
       from = min(from, __shfl_xor(from, 32, 64));
     }
     if (g == 0) u_out[kRows * 16 * vb + 16 * vt + c] = (float)from;
-    f32x4 xt[2];
+    f64x4 xt[2];
 #pragma unroll
-    for (int it = 0; it < 2; ++it) xt[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int it = 0; it < 2; ++it) xt[it] = f64x4{0., 0., 0., 0.};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      xt[0] = mfma4(tv[0][e], v_a[0][e], xt[0]);
-      xt[1] = mfma4(tv[1][e], v_a[0][e], xt[1]);
-      xt[1] = mfma4(tv[2][e], v_a[1][e], xt[1]);
+      const double va = v_a[0][e], vb2 = v_a[1][e];
+      xt[0] = mfma4_f64(tv[0][e], va, xt[0]);
+      xt[1] = mfma4_f64(tv[1][e], va, xt[1]);
+      xt[1] = mfma4_f64(tv[2][e], vb2, xt[1]);
     }
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
+      f32x4 put;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) xt[it][e] = 16 * it + 4 * g + e < from ? xt[it][e] : NAN;
-      *reinterpret_cast<f32x4*>(u_out + ((vt * 2 + it) * 64 + lane) * 4) = xt[it];
+      for (int e = 0; e < 4; ++e) put[e] = 16 * it + 4 * g + e < from ? (float)xt[it][e] : NAN;
+      *reinterpret_cast<f32x4*>(u_out + ((vt * 2 + it) * 64 + lane) * 4) = put;
 #pragma unroll
       for (int e = 0; e < 4; ++e) v_a[it][e] = v_b[it][e];
     }
@@ -790,13 +801,14 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
   }
 }
 
-// What bounds it: a wave has 51 matrix-core instructions of 32 cycles per block (0.67 us) in a chain
-// product -> LDS -> barrier -> LDS -> product, one wave per SIMD and nobody to fill its waits: the
+// What bounds it: a wave has 35 matrix-core instructions of 32 cycles per block and 16 of 64 (1.1 us of 128 x 128) in a
+// chain product -> LDS -> barrier -> LDS -> product, one wave per SIMD and nobody to fill its waits: the
 // loads are a block ahead, the product for the outputs stands where the exchange of U is on its way.
-// Two prompts of 2999 and 1854 tokens, 16 heads of 128 x 128 (94 blocks in a row): 171 us, 1.8 us per
-// block, 118 of them without the loads; asking for blocks two ahead changes nothing.  Under the tracer the walk takes
-// 174 us, the prepare kernel 115 (101 with products in 32 bits and no look at what is not finite), the norms 20 and
-// the step kernel's empty launch 5; a call 290, where the token-by-token walk of the same prompts takes 1079.
+// Two prompts of 2999 and 1854 tokens, 16 heads of 128 x 128 (94 blocks in a row), under the tracer: the walk 212 us,
+// 2.3 us per block; the prepare kernel 124 (101 with every product in 32 bits and no look at what is not finite), the
+// norms 20 and the step kernel's empty launch 5; a call 333, where the token-by-token walk of the same prompts takes 1079.
+// What a block adds to the state is summed in 64 bits: in 32 a call is 32 us less and states are 1.2 times as far
+// from 64 bits as token by token where keys share a part three times as large as the rest (1.0).
 template <int DX>
 __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(DeltaBlocks a) {
   constexpr int DP = 64 * DX;
@@ -867,17 +879,26 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
   };
   auto advance = [&](const Block& f, int i) {
     const int buf = i & 1;
-    f32x4 xu[2], xo[2];
+    // sums in several parts: half the roundings in a row
+    constexpr int kParts = DX > 1 ? 2 : 1;
+    f32x4 xu[2][kParts], xo[2][kParts];
 #pragma unroll
-    for (int it = 0; it < 2; ++it) xu[it] = xo[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int it = 0; it < 2; ++it)
+#pragma unroll
+      for (int p = 0; p < kParts; ++p) xu[it][p] = xo[it][p] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int x = 0; x < DX; ++x)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int it = 0; it < 2; ++it) xu[it] = mfma4(f.wv[x][it][e], s[x][e], xu[it]);
+        for (int it = 0; it < 2; ++it) xu[it][x % kParts] = mfma4(f.wv[x][it][e], s[x][e], xu[it][x % kParts]);
 #pragma unroll
-    for (int it = 0; it < 2; ++it) *reinterpret_cast<f32x4*>(&u_part[buf][w][it][lane][0]) = xu[it];
+    for (int it = 0; it < 2; ++it) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if constexpr (kParts > 1) xu[it][0][e] += xu[it][1][e];
+      *reinterpret_cast<f32x4*>(&u_part[buf][w][it][lane][0]) = xu[it][0];
+    }
     __syncthreads();
     f32x4 p[2][4];
 #pragma unroll
@@ -890,7 +911,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int it = 0; it < 2; ++it) xo[it] = mfma4(f.qv[x][it][e], s[x][e], xo[it]);
+        for (int it = 0; it < 2; ++it) xo[it][x % kParts] = mfma4(f.qv[x][it][e], s[x][e], xo[it][x % kParts]);
     if (i > 0) finish(i - 1);
     __builtin_amdgcn_sched_barrier(0);
     f32x4 u[2];
@@ -899,16 +920,16 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         u[it][e] = f.u[it][e] - ((p[it][0][e] + p[it][1][e]) + (p[it][2][e] + p[it][3][e]));
-    // what the block adds is summed by itself: one rounding of the state per block
-    f32x4 ds[DX];
+    // what the block adds is summed by itself, in 64 bits: one rounding of the state per block
+    f64x4 ds[DX];
 #pragma unroll
-    for (int x = 0; x < DX; ++x) ds[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int x = 0; x < DX; ++x) ds[x] = f64x4{0., 0., 0., 0.};
 #pragma unroll
     for (int it = 0; it < 2; ++it)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int x = 0; x < DX; ++x) ds[x] = mfma4(f.kv[x][it][e], u[it][e], ds[x]);
+        for (int x = 0; x < DX; ++x) ds[x] = mfma4_f64((double)f.kv[x][it][e], (double)u[it][e], ds[x]);
     // A U: the wave takes contraction index 4 g + w, so that the sum over waves is the whole product.  A row's product
     // with the rows behind it is 0 times their U: those that are not finite stay out.
     float u0 = w == 0 ? u[0][0] : w == 1 ? u[0][1] : w == 2 ? u[0][2] : u[0][3];
@@ -916,17 +937,20 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
     u0 = row_w < f.from ? u0 : 0.f;
     u1 = row_w + 16.f < f.from ? u1 : 0.f;
     from = f.from;
-    xo[0] = mfma4(f.av[0], u0, xo[0]);
-    xo[1] = mfma4(f.av[1], u0, xo[1]);
-    xo[1] = mfma4(f.av[2], u1, xo[1]);
+    xo[0][0] = mfma4(f.av[0], u0, xo[0][0]);
+    xo[1][0] = mfma4(f.av[1], u0, xo[1][0]);
+    xo[1][0] = mfma4(f.av[2], u1, xo[1][0]);
 #pragma unroll
     for (int it = 0; it < 2; ++it)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o_part[buf][w][it][e][lane] = xo[it][e];
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (kParts > 1) xo[it][0][e] += xo[it][1][e];
+        o_part[buf][w][it][e][lane] = xo[it][0][e];
+      }
 #pragma unroll
     for (int x = 0; x < DX; ++x)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[x][e] = f.g_last * s[x][e] + ds[x][e];
+      for (int e = 0; e < 4; ++e) s[x][e] = (float)((double)f.g_last * (double)s[x][e] + ds[x][e]);
   };
   // two blocks in turn, so that one is asked for while the other is worked on
   Block f0, f1;
@@ -1033,9 +1057,9 @@ __global__ __launch_bounds__(256) void delta_head_norm_vec_kernel(
 
 std::atomic<int> g_delta_kernel{0};
 
-// Blocks pay from about a block's rows on (us per call with its Python wrapper, 16 heads of 128, token by
-// token / in blocks: one run of 24 rows 33 / 35, 100 rows 44 / 36; six runs of 24 rows 33 / 39, 33 rows
-// 39 / 38, 48 rows 48 / 39, 100 rows 86 / 47).  Their scratch is 68 KB per block and head of 128 x 128;
+// Blocks pay from about a block's rows on (us on the GPU, calls back to back, 16 heads of 128, token by token / in
+// blocks: one run of 33 rows 21 / 23, 48 rows 24 / 23, 100 rows 43 / 28; six runs of 64 rows 55 / 44; 32 runs of 33
+// rows 140 / 114, of 64 217 / 129; one of 33 beside 31 single rows 50 / 41).  Their scratch is 68 KB per block and head of 128 x 128;
 // a step that would want more than 4 GiB of it walks token by token.
 constexpr int kBlockMinRows = 33;
 
