@@ -11,7 +11,7 @@ from tests.test_gpu_tekezen import DEV, latent_layer_of, latent_reference, rnd, 
 pytestmark = pytest.mark.gpu
 
 SIZES = [(2, 128, 64, 128, 64), (3, 32, 16, 40, 32), (4, 64, 64, 72, 128), (2, 96, 0, 128, 512), (1, 136, 56, 8, 32),
-         (2, 8, 8, 64, 32)]
+         (2, 8, 8, 64, 32), (1, 136, 48, 8, 32), (2, 8, 16, 64, 64)]
 
 
 @pytest.mark.parametrize("sizes", SIZES)
@@ -118,7 +118,7 @@ def layer_and_step(lens, contexts, sizes, window=0, sinks=False, dtype=torch.bfl
     return attn, batch, q, kv, gate, rnd((blocks, 16, C + Rr), 8).to(dtype).to(DEV)
 
 
-@pytest.mark.parametrize("sizes", [(4, 128, 64, 128, 128), (3, 40, 16, 56, 64), (2, 136, 56, 72, 32)])
+@pytest.mark.parametrize("sizes", [(4, 128, 64, 128, 128), (3, 40, 16, 56, 64), (2, 136, 56, 72, 32), (2, 136, 48, 72, 32)])
 @pytest.mark.parametrize("lens,contexts", [([70, 64, 200], [500, 64, 0]), ([300], [1000]), ([50, 60], [1500, 3])])
 @pytest.mark.parametrize("window,sinks", [(0, True), (150, False), (700, True)])
 def test_a_workspace_of_few_keys(sizes, lens, contexts, window, sinks):
@@ -139,6 +139,19 @@ def test_a_workspace_of_few_keys(sizes, lens, contexts, window, sinks):
         assert float((got - want).abs().max()) <= 0.008 * float(want.abs().max())
         rows_own = sum(lens) * H * (4 * 132 + 2 * V) + 2 * H * C * V
         assert torch.cuda.max_memory_allocated() - held <= keys * each + rows_own + (1 << 20)
+
+
+@pytest.mark.parametrize("sizes,formed", [((2, 64, 8, 64, 64), False), ((2, 64, 0, 64, 40), False), ((2, 128, 64, 128, 48), False),
+                                          ((2, 64, 16, 64, 64), True)])
+def test_sizes_whose_weights_have_32_bits(sizes, formed):
+    """Ranks and rotated parts that the matrix-core latent kernel does not take go to the kernel that keeps a weight in
+    32 bits, whatever the run's length."""
+    from dataclasses import replace
+    attn, batch, q, kv, gate, cache = layer_and_step([200, 3], [40, 9], sizes)
+    assert attn._stretches(batch) is not None
+    got = attn(q.clone(), kv, cache.clone(), batch, gate)
+    want = attn(q.clone(), kv, cache.clone(), replace(batch, host_query_lens=None), gate)
+    assert torch.equal(got, want) != formed
 
 
 @pytest.mark.parametrize("lens,contexts,most", [([48], [1 << 17], 19968), ([100, 3000, 64, 64], [0, 50000, 9, 900], 4096),

@@ -1125,12 +1125,13 @@ def latent_attention_tiles(out: torch.Tensor, q_lat: torch.Tensor, q_rot: torch.
 
 
 def latent_prompt_supported(q: torch.Tensor, dim: int, rot: int, vdim: int, rank: int, cache: torch.Tensor) -> bool:
-    """Whether latent_prompt takes these sizes, query rows [T, heads * (dim + rot)] and cache (never while
-    set_latent_attention_kernel keeps the matrix cores out, which the smallest sizes' answer tells)."""
-    if not _lib.seq_lib().vla_seq_latent_attention_tiles_supported(32, 0, _dt(q.dtype)):
-        return False
+    """Whether latent_prompt takes these sizes, query rows [T, heads * (dim + rot)] and cache: only where the
+    matrix-core latent kernel takes them too, whose weights have 16 bits as latent_prompt's (those of the kernel for all
+    other sizes have 32)."""
+    L = _lib.seq_lib()
     return (q.data_ptr() % 16 == 0 and (q.stride(0) % 8 == 0 or q.shape[0] == 1) and cache.data_ptr() % 16 == 0 and
-            bool(_lib.seq_lib().vla_seq_latent_prompt_supported(int(dim), int(rot), int(vdim), int(rank), _dt(q.dtype))))
+            bool(L.vla_seq_latent_attention_tiles_supported(int(rank), int(rot), _dt(q.dtype))) and
+            bool(L.vla_seq_latent_prompt_supported(int(dim), int(rot), int(vdim), int(rank), _dt(q.dtype))))
 
 
 def latent_gather(rows: torch.Tensor, cache: torch.Tensor, block_tables: torch.Tensor, query_start_loc: torch.Tensor,

@@ -17,8 +17,9 @@ exponential joins its softmax denominator (a key without a value, not scaled).  
 rotated part), with queries and up-projections of its own.  In prompts, portions of prompts
 and decode steps alike the step's rows are written to the cache, then every query row reads from there
 (csrc/seq_latent_attention.hip: a matrix-core kernel for 16-bit models whose rank is a multiple of 32 and whose rotated part is a multiple of 16,
-and an fp32 kernel for any dtype and size).  Runs of many rows with enough work form every head's keys and values from
-the cached latents instead, in a workspace of fixed size, and score those (csrc/seq_latent_prompt.hip).
+and an fp32 kernel for any dtype and size).  Runs of many rows with enough work, of sizes that the matrix-core
+kernel takes, form every head's keys and values from the cached latents instead, in a workspace of fixed size, and
+score those (csrc/seq_latent_prompt.hip).
 """
 import math
 from typing import Dict, Optional, Tuple
