@@ -149,3 +149,31 @@ def test_a_lone_run_shorter_than_the_hint(rows, hint):
 
     for got, want in zip(go(hint), go(min(rows, 32))):
         assert float((got - want).abs().max()) <= 3e-5 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("H,lens,blocks", [(2, [87], False), (2, [88], True), (2, [32] * 3, False), (128, [33, 30], False),
+                                           (128, [33, 31], True), (128, [32, 32], False)])
+def test_steps_that_go_in_blocks(H, lens, blocks):
+    """The layer's choice, and both kernels' results."""
+    from vllm_legacy_amd import _seq_ops as ops
+    from vllm_legacy_amd.attention.recurrent import GatedDeltaRule
+    D, V, n = 16, 64, sum(lens)
+    layer = GatedDeltaRule(H, H, D, V, 1e-5, DEV)
+    x = {name: rnd((n, w), i).to(DEV) for i, (name, w) in enumerate(
+        {"q": H * D, "k": H * D, "v": H * V, "gate": H * V, "beta": H, "dt": H}.items())}
+    batch = make_batch(lens, [0] * len(lens), slots=list(range(len(lens))))
+
+    def go(which):
+        out, state = torch.empty((n, H * V), device=DEV), torch.zeros((len(lens), H, V, D), device=DEV)
+        if which is None:
+            layer(out, *x.values(), state, batch)
+        else:
+            ops.delta_rule_scan(out, *x.values(), layer.a_log.data, layer.dt_bias.data, layer.norm_weight.data, state,
+                                batch.query_start_loc, batch.context_lens, batch.state_slots, H, 1e-5, max(lens), which)
+        return out, state
+
+    got, walk, block = go(None), go(False), go(True)
+    assert torch.equal(got[1], (block if blocks else walk)[1])
+    assert not torch.equal(walk[1], block[1]) or max(lens) < 33
+    for a, b in zip(walk, block):
+        assert float((a - b).abs().max()) <= 3e-5 * float(b.abs().max())

@@ -183,6 +183,13 @@ class GatedDeltaRule(nn.Module):
     them so); the state is fp32 [num_slots, heads, vdim, dim] and a sequence whose context length
     is 0 starts from zero whatever its slot held (csrc/seq_delta_rule.hip)."""
 
+    # Blocks are two launches more than a walk, so short runs want some rows beside them to pay.  Heads of 128 x 128,
+    # walked token by token / in blocks, us: 16 heads, 1 run of 48 rows 37/39, of 80 36/38, of 100 44/37; 3 of 55 36/42,
+    # of 64 35/41, of 80 40/39; 6 of 33 38/40, of 48 47/42; 12 of 33 59/57; 32 heads, 1 of 80 37/36, of 100 44/36; 3 of 33
+    # 38/39, of 55 51/42; 65, 40 and 16 34/40.
+    BLOCK_ALONE_ROWS = 88       # the longest run's from which they pay by themselves ...
+    BLOCK_WORK = 1 << 19        # ... or outputs of the step (33 rows and more in a run, by the kernel's own rule)
+
     def __init__(self, heads: int, kv_heads: int, dim: int, vdim: int, eps: float, device=None) -> None:
         super().__init__()
         assert heads % kv_heads == 0
@@ -202,7 +209,9 @@ class GatedDeltaRule(nn.Module):
         """q, k [T, G*D]; v, gate, out [T, H*V]; beta, dt [T, H]: views with free row strides."""
         ops.delta_rule_scan(out, q, k, v, gate, beta, dt, self.a_log.data, self.dt_bias.data, self.norm_weight.data,
                             state, batch.query_start_loc, batch.context_lens, batch.state_slots, self.kv_heads,
-                            self.eps, batch.max_query_len)
+                            self.eps, batch.max_query_len,
+                            batch.max_query_len >= self.BLOCK_ALONE_ROWS or
+                            q.shape[0] * self.heads * self.vdim >= self.BLOCK_WORK)
         return out
 
 
