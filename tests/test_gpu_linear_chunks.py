@@ -20,6 +20,7 @@ def run(H, D, V, rank, lens, ctx, dtype, bias_of=None, offset=0):
     from vllm_legacy_amd.attention.recurrent import GatedLinearRecurrence
     tau, eps, T = 5.0, 1e-5, sum(lens)
     layer = GatedLinearRecurrence(H, D, V, tau, eps)
+    layer.CHUNK_ALONE_ROWS = 0              # however little there is to do
     g = torch.Generator().manual_seed(D + V + T)
     slots = list(range(len(lens)))[::-1]
     state = torch.randn(GatedLinearRecurrence.get_state_shape(len(lens), H, D, V), generator=g).to(DEV)
@@ -120,3 +121,27 @@ def test_rows_ahead_of_one_that_is_not_finite(what, value, row, dtype):
     want = R.gated_head_norm(o, norm_w.to(R.F), rows["gate"].to(R.F)[:lens[0]], 1e-5, 1.0).reshape(-1, H, V)
     assert torch.equal(got[:lens[0]].isfinite(), want.isfinite())
     assert torch.equal(state[0].isfinite(), S.isfinite())
+
+
+@pytest.mark.parametrize("H,lens,chunks", [(2, [99], False), (2, [100], True), (2, [100] + [1] * 6, False), (70, [64, 35], False),
+                                           (70, [64, 36], True), (70, [63, 63], False)])
+def test_steps_that_go_in_chunks(H, lens, chunks, monkeypatch):
+    from vllm_legacy_amd import _seq_ops as ops
+    from vllm_legacy_amd.attention.batch import SequenceBatch
+    from vllm_legacy_amd.attention.recurrent import GatedLinearRecurrence
+    D, V, rank, T, went = 16, 16, 1, sum(lens), []
+    layer, taken = GatedLinearRecurrence(H, D, V, 5.0, 1e-5), ops.gla_chunks
+    monkeypatch.setattr(ops, "gla_chunks", lambda *a: (went.append(1), taken(*a)))
+    b = SequenceBatch.build(lens, [0] * len(lens), [[0] * 64] * len(lens), list(range(len(lens))), 16, DEV)
+    q, k, v, gate, y, w2 = (torch.randn(*shape, generator=torch.Generator().manual_seed(i)).to(DEV) for i, shape in enumerate(
+        [(T, H * D), (T, H * D), (T, H * V), (T, H * V), (T, rank), (H * D, rank)]))
+    outs = []
+    for alone in (None, 1 << 30):
+        if alone:
+            layer.CHUNK_ALONE_ROWS = layer.CHUNK_HEAD_ROWS = alone
+        state = torch.zeros(GatedLinearRecurrence.get_state_shape(len(lens), H, D, V), device=DEV)
+        out = torch.empty(T, H * V, device=DEV)
+        layer(out, q, k, v, gate, y, w2, torch.ones(H * D, device=DEV), torch.ones(V, device=DEV), state, b, 1.0)
+        outs.append(out)
+    assert len(went) == int(chunks)
+    assert float((outs[0] - outs[1]).abs().max()) <= 6e-5 * float(outs[1].abs().max())

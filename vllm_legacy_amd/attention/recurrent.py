@@ -31,11 +31,15 @@ class GatedLinearRecurrence(nn.Module):
     # rows of a piece; runs of at least two pieces are cut (VLA_GLA_PIECE_ROWS: another size, for studies)
     PIECE_ROWS = int(os.environ.get("VLA_GLA_PIECE_ROWS", "256"))
     SCRATCH_SLOTS = 64      # state slots behind the sequences' own, for the pieces of a step
-    # A step goes in chunks of 64 rows (where the sizes allow it) if its longest run has that many.  16 heads of
-    # 64 x 128, bf16, walked token by token / in chunks, us: 1 run of 64 rows 48/46, of 300 128/49; 6 of 48 48/49,
-    # of 64 54/53, of 128 99/67; 32 of 32 125/107, of 64 195/133, of 300 758/348.  A single row costs a whole
-    # chunk, so many beside one run need a long run (the walk's time is its longest run's).
+    # A step goes in chunks of 64 rows (where the sizes allow it) if its longest run has that many and there is enough
+    # for them to do: three short chunks' kernels take 50 us however few the rows.  Heads of 64 x 128, bf16, walked token
+    # by token / in chunks, us: 16 heads, 1 run of 64 rows 46/50, of 100 52/50, of 128 59/50, of 200 89/51; runs of 65,
+    # 40 and 16 46/51; 3 of 80 50/53; 6 of 64 52/56; 16 of 64 113/77; 32 heads, 3 of 64 52/56, of 80 63/59, 6 of 64
+    # 109/74.  A single row costs a whole chunk, so many beside one run need a long run (the walk's time is its longest
+    # run's): one of 200 beside 32 single rows 157/166.
     CHUNK_MIN_ROWS = 64
+    CHUNK_ALONE_ROWS = 100  # the longest run's from which it pays by itself ...
+    CHUNK_HEAD_ROWS = 7000  # ... or rows times heads of the step
     CHUNK_MEAN_ROWS = 16    # rows per run on average ...
     CHUNK_LONG_ROWS = 512   # ... unless a run is this long
 
@@ -102,6 +106,7 @@ class GatedLinearRecurrence(nn.Module):
         T, H, D, V = q.shape[0], self.num_heads, self.head_dim, self.value_dim
         longest = batch.max_query_len
         if (longest >= self.CHUNK_MIN_ROWS
+                and (longest >= self.CHUNK_ALONE_ROWS or T * H >= self.CHUNK_HEAD_ROWS)
                 and (T >= self.CHUNK_MEAN_ROWS * batch.num_seqs or longest >= self.CHUNK_LONG_ROWS)
                 and q.dtype == gate.dtype == out.dtype == w2.dtype == y.dtype):
             need = ops.gla_chunks_scratch(q, k, v, H, D, V, w2.shape[1], batch.num_seqs)
