@@ -137,6 +137,9 @@ class LatentKVAttention(nn.Module):
     def _stretches(self, batch: SequenceBatch):
         """[[first sequence, one behind the last, first row, one behind the last, formed]]: neighbours that go
         the same way; None when the whole step takes the latent kernel."""
+        each = self.num_heads * (2 * self.rank + self.rot_dim)          # multiply-adds of a (query, key) pair
+        if batch.num_tokens * batch.max_seq_len * each < self.FORMED_MIN_WORK:
+            return None                 # most steps: no more than this is asked of them
         least = self.formed_min_rows()
         if batch.max_query_len < least or not self.scale > 0:
             return None
@@ -152,7 +155,7 @@ class LatentKVAttention(nn.Module):
             else:
                 out.append([b, b + 1, row, row + n, n >= least])
             row += n
-        if pairs * self.num_heads * (2 * self.rank + self.rot_dim) < self.FORMED_MIN_WORK:
+        if pairs * each < self.FORMED_MIN_WORK:
             return None
         return out if len(out) <= self.MAX_STRETCHES else None
 
@@ -215,35 +218,38 @@ class LatentKVAttention(nn.Module):
                               total if carry is not None else 0, carry)
             del rows, latents, keys, keys_rest, values          # the next part's take their place
 
-    def _attend_latent(self, q, cache, batch: SequenceBatch, s0, s1, r0, r1, gate) -> torch.Tensor:
-        """Sequences s0 .. s1 - 1 (rows r0 .. r1 - 1) on the cached latents -> [rows, heads * vdim]."""
-        H, D, Rr, V, C = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.rank
-        whole = s0 == 0 and s1 == batch.num_seqs
-        T = r1 - r0
+    def _attend_latent(self, q, cache, batch: SequenceBatch, gate, part=None) -> torch.Tensor:
+        """The step, or of part (s0, s1, r0, r1) sequences s0 .. s1 - 1 (rows r0 .. r1 - 1), on the cached latents ->
+        [rows, heads * vdim]."""
+        H, D, Rr, C = self.num_heads, self.head_dim, self.rot_dim, self.rank
         sinks = None if self.sinks is None else self.sinks.data
-        if not whole:
+        if part is not None:
+            s0, s1, r0, r1 = part
             q, gate = q[r0:r1], None if gate is None else gate[r0:r1]
+        T = q.shape[0]
         q3 = q.view(T, H, D + Rr)
-        q_lat = torch.bmm(q3[:, :, :D].transpose(0, 1), self.w_uk.data)             # [H, T, C]
+        q_lat = torch.bmm(q3.narrow(2, 0, D).transpose(0, 1), self.w_uk.data)       # [H, T, C]
         o_lat = torch.empty((H, T, C), dtype=q.dtype, device=q.device)
-        q_lat, q_rot, o_rows = q_lat.transpose(0, 1), q3[:, :, D:], o_lat.transpose(0, 1)
+        q_lat, q_rot, o_rows = q_lat.transpose(0, 1), q3.narrow(2, D, Rr), o_lat.transpose(0, 1)
         if ops.latent_attention_tiles_supported(q_lat, q_rot, cache):
             # 16-bit models whose sizes fit: (token, head) rows in tiles of 32 on the matrix cores
-            if whole:
-                tables, starts, ctx, longest, splits = batch.block_tables, batch.query_start_loc, batch.context_lens, \
-                    batch.max_query_len, self.key_splits(batch)
+            if part is None:
+                ops.latent_attention_tiles(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.query_start_loc,
+                                           batch.context_lens, batch.max_query_len, self.scale, self.key_splits(batch),
+                                           self.window, gate, sinks)
             else:
                 ql, cl = batch.host_query_lens[s0:s1], batch.host_context_lens[s0:s1]
-                tables, ctx, longest = batch.block_tables[s0:s1], batch.context_lens[s0:s1], max(ql)
-                starts = batch.query_start_loc[s0:s1 + 1] - r0
+                longest = max(ql)
                 splits = self._key_splits(longest, s1 - s0, max(c + n for n, c in zip(ql, cl)))
-            ops.latent_attention_tiles(o_rows, q_lat, q_rot, cache, tables, starts, ctx, longest, self.scale, splits,
-                                       self.window, gate, sinks)
+                ops.latent_attention_tiles(o_rows, q_lat, q_rot, cache, batch.block_tables[s0:s1],
+                                           batch.query_start_loc[s0:s1 + 1] - r0, batch.context_lens[s0:s1], longest,
+                                           self.scale, splits, self.window, gate, sinks)
         else:
-            ops.latent_attention(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.token_seq[r0:r1],
-                                 batch.positions[r0:r1], self.scale, self.window, gate, sinks)
+            rows = slice(None) if part is None else slice(r0, r1)
+            ops.latent_attention(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.token_seq[rows],
+                                 batch.positions[rows], self.scale, self.window, gate, sinks)
         o = torch.bmm(o_lat, self.w_uv_t.data)                                      # [H, T, V]
-        return o.transpose(0, 1).reshape(T, H * V)
+        return o.transpose(0, 1).reshape(T, H * self.value_dim)
 
     @staticmethod
     def get_cache_shape(num_blocks: int, block_size: int, rank: int, rot_dim: int) -> Tuple[int, ...]:
@@ -254,19 +260,18 @@ class LatentKVAttention(nn.Module):
         """q [T, heads * (dim + rot_dim)], head by head [plain | rotated] (rotated in place); kv
         [T, rank + rot_dim] before its norm and rotation (None: the cache already holds this step's rows),
         gate [T, heads] (views with free row strides).  Returns [T, heads * vdim]."""
-        T = q.shape[0]
-        H, D, Rr, V, C = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.rank
         assert (kv is not None) == self.own_latent
         if self.own_latent:
-            ops.latent_rotary_write(q, D + Rr, D, H, kv, self.latent_norm.data, self.eps, cache, batch.positions,
+            D, Rr = self.head_dim, self.rot_dim
+            ops.latent_rotary_write(q, D + Rr, D, self.num_heads, kv, self.latent_norm.data, self.eps, cache, batch.positions,
                                     batch.slot_mapping, self.inv_freq, self.magnitude, self.rot_dims, self.interleaved)
         stretches = None if batch.max_query_len < self.FORMED_MIN_ROWS else self._stretches(batch)
-        if stretches is None or not ops.latent_prompt_supported(q, D, Rr, V, C, cache):
-            return self._attend_latent(q, cache, batch, 0, batch.num_seqs, 0, T, gate)
-        out = torch.empty((T, H * V), dtype=q.dtype, device=q.device)
+        if stretches is None or not ops.latent_prompt_supported(q, self.head_dim, self.rot_dim, self.value_dim, self.rank, cache):
+            return self._attend_latent(q, cache, batch, gate)
+        out = torch.empty((q.shape[0], self.num_heads * self.value_dim), dtype=q.dtype, device=q.device)
         for s0, s1, r0, r1, formed in stretches:
             if formed:
                 self._attend_formed(out, q, cache, batch, s0, s1, r0, r1, gate)
             else:
-                out[r0:r1] = self._attend_latent(q, cache, batch, s0, s1, r0, r1, gate)
+                out[r0:r1] = self._attend_latent(q, cache, batch, gate, (s0, s1, r0, r1))
         return out
