@@ -34,6 +34,7 @@
 // products run on 16x16x4 matrix cores: what the preparation forms and K^^T U in 64 bits, those with S in 32.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "seq_common.h"
 
@@ -260,15 +261,19 @@ __global__ __launch_bounds__(256) void delta_rule_kernel(
   }
 }
 
+constexpr int kStepRows = 4;        // runs of at most this many rows go token by token beside blocks
+
 // Runs of a few rows (decode steps): no staging.  The `split` lanes of a column hold all rows between
-// them, so a token's unit norms are lane sums of what they read for the dot products anyway.
-template <class SI, int R>
+// them, so a token's unit norms are lane sums of what they read for the dot products anyway.  LIMIT: runs of more
+// than kStepRows rows are the block kernels' (a form of its own: the state's loads would wait for the run's length,
+// 129 decode rows of 16 heads of 128 x 128 54.6 us per call, 53.0 without).
+template <class SI, int R, bool LIMIT>
 __global__ __launch_bounds__(256) void delta_rule_step_kernel(
     float* __restrict__ o, DeltaRows<SI> in, const float* __restrict__ a_log,
     const float* __restrict__ dt_bias, float* __restrict__ state,
     const int* __restrict__ query_start_loc, const int* __restrict__ context_lens,
     const int* __restrict__ state_slots, int heads, int kv_heads, int dim, int vdim, int split,
-    int cols, int longest) {
+    int cols) {
   const int h = blockIdx.y, b = blockIdx.z, j0 = blockIdx.x * cols;
   const int g_head = h / (heads / kv_heads);
   const int tid = threadIdx.x;
@@ -276,7 +281,7 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(
   const int j = j0 + jl;
   const bool col = jl < cols && j < vdim;
   const int start = query_start_loc[b], end = query_start_loc[b + 1];
-  if (longest > 0 && end - start > longest) return;        // the block kernels'
+  if (LIMIT && end - start > kStepRows) return;
   float* st = state + (((int64_t)state_slots[b] * heads + h) * vdim + (col ? j : 0)) * dim;
   const bool whole = dim == split * R && (dim & 3) == 0;
   const bool vec = whole && (in.q_stride & 3) == 0 && (in.k_stride & 3) == 0 &&
@@ -367,7 +372,6 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(
 // ---------------------------------------------------------------------------------------------
 // Blocks of 32 rows
 constexpr int kRows = 32;
-constexpr int kStepRows = 4;        // runs of at most this many rows go token by token beside blocks
 constexpr int kMaxBlockDim = 256;
 constexpr int kMat = 36;            // floats per row of a 32 x 32 matrix in LDS
 constexpr int kMatB = 34;           // and of one in 64 bits
@@ -1184,14 +1188,21 @@ int delta_rule_scan(
     auto launch_step = [&](auto kernel) {
       kernel<<<grid, threads, 0, (hipStream_t)stream>>>(scratch, in, a_log, dt_bias, state, query_start_loc,
                                                         context_lens, state_slots, heads, kv_heads, dim, vdim,
-                                                        split, cols, blocks ? kStepRows : 0);
+                                                        split, cols);
     };
-    switch (rows) {
-      case 8: launch_step(delta_rule_step_kernel<SI, 8>); break;
-      case 16: launch_step(delta_rule_step_kernel<SI, 16>); break;
-      case 32: launch_step(delta_rule_step_kernel<SI, 32>); break;
-      default: launch_step(delta_rule_step_kernel<SI, 64>); break;
-    }
+    auto step_of = [&](auto limit) {
+      constexpr bool kLimit = decltype(limit)::value;
+      switch (rows) {
+        case 8: launch_step(delta_rule_step_kernel<SI, 8, kLimit>); break;
+        case 16: launch_step(delta_rule_step_kernel<SI, 16, kLimit>); break;
+        case 32: launch_step(delta_rule_step_kernel<SI, 32, kLimit>); break;
+        default: launch_step(delta_rule_step_kernel<SI, 64, kLimit>); break;
+      }
+    };
+    if (blocks)
+      step_of(std::true_type{});
+    else
+      step_of(std::false_type{});
   }
   auto launch = [&](auto kernel) {
     kernel<<<grid, threads, lds, (hipStream_t)stream>>>(scratch, in, a_log, dt_bias, state, query_start_loc,
