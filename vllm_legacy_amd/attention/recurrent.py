@@ -32,7 +32,7 @@ class GatedLinearRecurrence(nn.Module):
     PIECE_ROWS = int(os.environ.get("VLA_GLA_PIECE_ROWS", "256"))
     SCRATCH_SLOTS = 64      # state slots behind the sequences' own, for the pieces of a step
     # A step goes in chunks of 64 rows (where the sizes allow it) if its longest run has that many and there is enough
-    # for them to do: three short chunks' kernels take 50 us however few the rows.  Heads of 64 x 128, bf16, walked token
+    # for them to do: the three kernels of a few chunks take 50 us however few the rows.  Heads of 64 x 128, bf16, walked token
     # by token / in chunks, us: 16 heads, 1 run of 64 rows 46/50, of 100 52/50, of 128 59/50, of 200 89/51; runs of 65,
     # 40 and 16 46/51; 3 of 80 50/53; 6 of 64 52/56; 16 of 64 113/77; 32 heads, 3 of 64 52/56, of 80 63/59, 6 of 64
     # 109/74.  A single row costs a whole chunk, so many beside one run need a long run (the walk's time is its longest
