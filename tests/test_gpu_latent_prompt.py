@@ -154,6 +154,35 @@ def test_sizes_whose_weights_have_32_bits(sizes, formed):
     assert torch.equal(got, want) != formed
 
 
+@pytest.mark.parametrize("which,size", [("uk", 1.0), ("uk", 3e4), ("uv", 3e3), ("uv", 3e4)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_values_that_leave_the_range(which, size, dtype):
+    """Weights with which a key or a value can be more than float16 holds, where the sums on the latents' side are not:
+    those stay there."""
+    from vllm_legacy_amd.attention.backends.latent_kv import LatentKVAttention
+    H, D, Rr, V, C, n = 2, 32, 16, 32, 64, 150
+    batch, blocks = step([n], [0])
+    attn = LatentKVAttention(H, D, Rr, V, C, 1e-4, 0, 1e4, None, 1e-5, dtype, DEV)
+    w = {"uk": rnd((H * D, C), 1, C**-0.5), "uv": rnd((H * V, C), 2, C**-0.5)}
+    w[which] = w[which] * size
+    attn.set_weights(w["uk"], w["uv"], torch.ones(C))
+    attn.FORMED_MIN_WORK = 0
+    fits = dtype == torch.bfloat16 or size < 1e4
+    assert (attn._stretches(batch) is not None) == fits
+    q, kv = (rnd((n, x), s, 1.0 if s == 6 else 0.25).to(dtype).to(DEV) for x, s in ((H * (D + Rr), 5), (C + Rr, 6)))
+    cache = torch.zeros((blocks, 16, C + Rr), dtype=dtype, device=DEV)
+    got = attn(q, kv, cache, batch).view(n, H, V).double()
+    rows = cache[batch.block_tables[0].long()].view(-1, C + Rr)[:n].double()
+    unseen = torch.ones((n, n), dtype=torch.bool, device=DEV).triu(1)
+    for h in range(H):
+        qh, u = q.view(n, H, D + Rr)[:, h].double(), attn.w_uk.data[h].double()
+        s = (qh[:, :D] @ (rows[:, :C] @ u.t()).t() + qh[:, D:] @ rows[:, C:].t()) * attn.scale
+        want = torch.softmax(s.masked_fill(unseen, float("-inf")), 1) @ (rows[:, :C] @ attn.w_uv_t.data[h].double())
+        live = want.abs().amax(1) < 6e4         # outputs that float16 holds
+        bar = 0.06 if dtype == torch.bfloat16 else 0.06 / 8
+        assert bool(live[20:].all()) and float((got[live, h] - want[live]).abs().max()) <= bar * float(want[live].abs().max())
+
+
 @pytest.mark.parametrize("lens,contexts,most", [([48], [1 << 17], 19968), ([100, 3000, 64, 64], [0, 50000, 9, 900], 4096),
                                                 ([64] * 40, [1000] * 40, 2048), ([64, 64], [0, 0], 64)])
 @pytest.mark.parametrize("window", [0, 1024])

@@ -81,6 +81,7 @@ class LatentKVAttention(nn.Module):
                                  requires_grad=False)
         self.w_uv_t = nn.Parameter(torch.zeros((num_heads, rank, value_dim), dtype=dtype, device=device),
                                    requires_grad=False)
+        self.formed_fits = True
 
     def set_weights(self, uk: torch.Tensor, uv: torch.Tensor, latent_norm: Optional[torch.Tensor] = None,
                     sinks: Optional[torch.Tensor] = None) -> None:
@@ -94,6 +95,10 @@ class LatentKVAttention(nn.Module):
             self.latent_norm.data = latent_norm.float().to(dev).contiguous()
         if self.sinks is not None:
             self.sinks.data = sinks.float().to(dev).contiguous()
+        # No formed key or value may leave the dtype's range, where sums of latents stay in it.  A normed latent's
+        # length is at most sqrt(rank) times the norm's largest weight (another layer's: taken as 8 at most).
+        length = math.sqrt(C) * (float(latent_norm.abs().max()) if self.own_latent else 8.0)
+        self.formed_fits = max(float(w.float().norm(dim=1).max()) for w in (uk, uv)) * length < torch.finfo(self.dtype).max
 
     # workgroups a launch should have before the keys of a row tile stay with one workgroup
     SPLIT_BELOW_WORKGROUPS = 512
@@ -141,7 +146,7 @@ class LatentKVAttention(nn.Module):
         if batch.num_tokens * batch.max_seq_len * each < self.FORMED_MIN_WORK:
             return None                 # most steps: no more than this is asked of them
         least = self.formed_min_rows()
-        if batch.max_query_len < least or not self.scale > 0:
+        if batch.max_query_len < least or not self.scale > 0 or not self.formed_fits:
             return None
         q, ctx = batch.host_query_lens, batch.host_context_lens
         if q is None or ctx is None or torch.cuda.is_current_stream_capturing():

@@ -332,7 +332,8 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
     if (u0 + kKeys <= p_end) bring_keys(u0 + kKeys);
     // A hidden key's weight is 0, which times an infinity or a NaN would not be: a tile that hides keys from some row
     // goes without values that are not finite.  Rows that see such a key are NaN by their scores: a key of the same
-    // latent is not finite either, and it and what it lost to rounding never sum to a number.
+    // latent is not finite either, and it and what it lost to rounding never sum to a number (finite latents give finite
+    // values: the layer looks at its weights for that).
     if (u0 + kKeys - 1 > g_p0 || u0 < g_lo_last) {
 #pragma unroll
       for (int u = 0; u < VI; ++u) {
