@@ -635,6 +635,23 @@ int vla_seq_latent_attention_tiles(void* out, int64_t out_token_stride, int64_t 
                                    void* stream);
 int vla_seq_set_latent_attention_kernel(int mode);
 
+/* The same attention for steps of single rows (decode steps; of a sequence with more, the first row only), rank
+ * 256 or 512 and rot 0 or 64 (vla_seq_latent_decode_supported).  The keys of all sequences are shared out
+ * evenly to `ranges` workgroups per set of heads, from the lengths on the device; vla_seq_latent_decode_ranges gives the
+ * number for sequences of up to max_keys visible keys (any other is right as well).  With more than one, scratch
+ * (16-byte aligned) holds vla_seq_latent_decode_scratch_floats fp32 values.  Query rows, cache rows and strides as
+ * above; the output 8-byte aligned, its strides multiples of 4. */
+int vla_seq_latent_decode_supported(int rank, int rot, int dtype);
+int vla_seq_latent_decode_ranges(int num_seqs, int max_keys, int heads);
+int64_t vla_seq_latent_decode_scratch_floats(int ranges, int heads, int rank);
+int vla_seq_latent_decode(void* out, int64_t out_token_stride, int64_t out_head_stride, const void* q_lat,
+                          int64_t lat_token_stride, int64_t lat_head_stride, const void* q_rot,
+                          int64_t rot_token_stride, int64_t rot_head_stride, const void* cache,
+                          const int* block_tables, int max_blocks, const int* query_start_loc,
+                          const int* context_lens, int num_seqs, int heads, int rank, int rot, int block_size,
+                          int num_blocks, float scale, int ranges, float* scratch, int64_t scratch_floats, int dtype,
+                          int window, const void* gate, int64_t gate_stride, const float* sinks, void* stream);
+
 /* Kernel choice for tests: window attention 0 = per shape, 1 = one wave per (row, head);
  * scan 0 = per shape, 1 = token by token. */
 int vla_seq_set_window_kernel(int mode);

@@ -1,0 +1,125 @@
+"""Latent attention of single rows (csrc/seq_latent_decode.hip) against float64, at the edges of its tiles of 16 keys,
+the rows looked up ahead (1024) and the ranges that all sequences' keys are shared out in."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV, F = "cuda:0", torch.float64
+
+
+def case(lens, heads, rank, rot, block, dtype, window=0, seed=0, slack=0):
+    """A step whose rows see `lens` keys (no window): tensors on the GPU."""
+    g = torch.Generator().manual_seed(seed)
+    B = len(lens)
+    need = [(n + slack + block - 1) // block for n in lens]
+    ids = torch.randperm(sum(need) + 2, generator=g).tolist()
+    tables, at = torch.zeros(B, max(need), dtype=torch.int32), 0
+    for b, n in enumerate(need):
+        tables[b, :n] = torch.tensor(ids[at:at + n], dtype=torch.int32)
+        at += n
+
+    def rnd(*shape, std=1.0):
+        return (std * torch.randn(*shape, generator=g)).to(dtype).to(DEV)
+
+    return dict(cache=rnd(sum(need) + 2, block, rank + rot), tables=tables.to(DEV), scale=0.06,
+                q_lat=rnd(B, heads, rank), q_rot=rnd(B, heads, rot), starts=torch.arange(B + 1, dtype=torch.int32, device=DEV),
+                ctx=torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV), window=window)
+
+
+def run(c, gate=None, sinks=None, out=None, max_keys=None):
+    from vllm_legacy_amd import _seq_ops as ops
+    out = torch.empty_like(c["q_lat"]) if out is None else out
+    assert ops.latent_decode_supported(out, c["q_lat"], c["q_rot"], c["cache"])
+    ops.latent_decode(out, c["q_lat"], c["q_rot"], c["cache"], c["tables"], c["starts"], c["ctx"],
+                      max_keys or int(c["ctx"].max()) + 1, c["scale"], c["window"], gate, sinks)
+    return out
+
+
+def reference(c, gate=None, sinks=None):
+    out = []
+    for b, n in enumerate((c["ctx"] + 1).tolist()):
+        rows = c["cache"].to(F)[c["tables"][b].long()].flatten(0, 1)[max(0, n - c["window"]) if c["window"] else 0:n]
+        q = torch.cat([c["q_lat"][b], c["q_rot"][b]], 1).to(F)
+        s = (q @ rows.t()) * c["scale"]
+        if sinks is not None:
+            s = torch.cat([s, sinks.to(F)[:, None]], 1)
+        p = torch.softmax(s, -1)[:, :rows.shape[0]]
+        o = p @ rows[:, :c["q_lat"].shape[2]]
+        out.append(o if gate is None else o * torch.sigmoid(gate[b].to(F))[:, None])
+    return torch.stack(out)
+
+
+def check(got, want, dtype):
+    # weights and results are rounded to 16 bits: 2^-9 (bfloat16) or 2^-12 of the sums of weights times |value|, which
+    # for n alike weights are up to sqrt(n) times the result; measured 0.002 and 0.0003
+    rel = float((got.to(F) - want).norm() / want.norm())
+    assert rel <= (0.008 if dtype == torch.bfloat16 else 0.001), rel
+    assert not torch.isnan(got).any()
+
+
+LENS = [[1], [15], [16], [17], [31, 32, 33], [63, 1, 64, 65], [1023, 1024, 1025], [3000], [2048, 1, 2, 700, 96],
+        [1 + 13 * i % 190 for i in range(130)], [40] * 600]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens", LENS, ids=lambda x: f"{len(x)}x{max(x)}")
+@pytest.mark.parametrize("rank,rot", [(512, 64), (256, 0)])
+def test_lengths(rank, rot, lens, dtype):
+    c = case(lens, 16, rank, rot, 16, dtype)
+    check(run(c), reference(c), dtype)
+
+
+@pytest.mark.parametrize("rank,rot", [(512, 0), (256, 64)])
+@pytest.mark.parametrize("heads,block,window", [(1, 4, 0), (5, 7, 33), (17, 16, 100), (32, 1, 64), (40, 16, 1)])
+def test_heads_pages_windows_gates_and_sinks(rank, rot, heads, block, window):
+    lens = [200, 5, 33, 64, 129]
+    c = case(lens, heads, rank, rot, block, torch.bfloat16, window)
+    gate = torch.randn(len(lens), heads + 3, device=DEV).to(torch.bfloat16)[:, :heads]
+    sinks = torch.randn(heads, device=DEV)
+    flat = torch.empty(heads, len(lens), rank, dtype=torch.bfloat16, device=DEV).transpose(0, 1)
+    check(run(c, gate, sinks, flat), reference(c, gate, sinks), torch.bfloat16)
+
+
+@pytest.mark.parametrize("ranges_for", [1, 64, 100000])
+def test_any_number_of_ranges(ranges_for):
+    """How many workgroups share the keys is the host's guess; the result does not depend on it."""
+    c = case([500, 31, 1200, 64], 16, 512, 64, 16, torch.bfloat16)
+    check(run(c, max_keys=ranges_for), reference(c), torch.bfloat16)
+
+
+def test_what_lies_behind_the_last_key_does_not_enter():
+    lens = [20, 50, 1000]
+    c = case(lens, 16, 512, 64, 16, torch.bfloat16)
+    want = run(c).clone()
+    for b, n in enumerate(lens):
+        if n % 16:
+            c["cache"][int(c["tables"][b, n // 16]), n % 16:] = math.inf
+    assert torch.equal(run(c), want)
+
+
+def test_replayed_with_other_lengths():
+    c = case([700, 90, 333], 16, 512, 64, 16, torch.bfloat16, slack=2200)
+    out = torch.empty_like(c["q_lat"])
+    run(c, out=out, max_keys=701)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(c, out=out, max_keys=701)
+    for lens in ([700, 90, 333], [1, 2900, 16], [2222, 2223, 2224], [32, 64, 1]):
+        c["ctx"].copy_(torch.tensor([n - 1 for n in lens], dtype=torch.int32))
+        graph.replay()
+        torch.cuda.synchronize()
+        check(out, reference(c), torch.bfloat16)
+
+
+def test_layers_take_it():
+    """A decode step of the layer goes this way and agrees with the kernel for all steps."""
+    from vllm_legacy_amd import _seq_ops as ops
+    c = case([300, 40, 7, 1100], 16, 512, 64, 16, torch.bfloat16)
+    tiles = torch.empty_like(c["q_lat"])
+    ops.latent_attention_tiles(tiles, c["q_lat"], c["q_rot"], c["cache"], c["tables"], c["starts"], c["ctx"], 1, c["scale"], 4)
+    want, got = reference(c), run(c)
+    error = [float((t.to(F) - want).norm() / want.norm()) for t in (tiles, got)]
+    assert error[1] <= 1.1 * error[0], error

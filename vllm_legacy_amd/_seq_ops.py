@@ -1127,6 +1127,50 @@ def latent_attention_tiles(out: torch.Tensor, q_lat: torch.Tensor, q_rot: torch.
             "latent_attention_tiles")
 
 
+def latent_decode_supported(out: torch.Tensor, q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch.Tensor) -> bool:
+    """Whether latent_decode takes these tensors, those of latent_attention_tiles that it supports."""
+    return (bool(_lib.seq_lib().vla_seq_latent_decode_supported(q_lat.shape[2], q_rot.shape[2], _dt(q_lat.dtype))) and
+            cache.shape[0] * cache.shape[1] < 1 << 31 and out.data_ptr() % 8 == 0 and
+            all(out.stride(d) % 4 == 0 or out.shape[d] == 1 for d in (0, 1)))
+
+
+def latent_decode(out: torch.Tensor, q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch.Tensor,
+                  block_tables: torch.Tensor, query_start_loc: torch.Tensor, context_lens: torch.Tensor, max_keys: int,
+                  scale: float, window: int = 0, gate: Optional[torch.Tensor] = None,
+                  sinks: Optional[torch.Tensor] = None) -> None:
+    """latent_attention_tiles for a step of single rows: the keys of all sequences are shared out evenly.  max_keys:
+    about the most that a row sees (decides how many workgroups there are, not what they do)."""
+    _gpu(out, q_lat, q_rot, cache, block_tables, query_start_loc, context_lens, gate, sinks)
+    NB, BS, width = cache.shape
+    T, H, rank = q_lat.shape
+    rot = width - rank
+    B = context_lens.numel()
+    assert sinks is None or (sinks.dtype == torch.float32 and sinks.numel() == H and sinks.is_contiguous())
+    assert gate is None or (gate.dtype == q_lat.dtype and gate.shape[0] == T)
+    assert out.shape == q_lat.shape and q_rot.shape == (T, H, rot) and cache.is_contiguous()
+    assert out.dtype == q_lat.dtype == q_rot.dtype == cache.dtype
+    for t in (out, q_lat, q_rot):
+        assert t.stride(2) == 1 or t.shape[2] == 1
+    for t in (block_tables, query_start_loc, context_lens):
+        assert t.dtype == torch.int32 and t.is_contiguous()
+    assert block_tables.dim() == 2 and block_tables.shape[0] == B and query_start_loc.numel() == B + 1
+
+    def st(t, d):       # a stride that is never used may be anything
+        return t.stride(d) if t.shape[d] > 1 else 0
+
+    L = _lib.seq_lib()
+    ranges = L.vla_seq_latent_decode_ranges(B, int(max_keys), H)
+    need = L.vla_seq_latent_decode_scratch_floats(ranges, H, rank)
+    scratch = torch.empty(need, dtype=torch.float32, device=q_lat.device) if need else None
+    with torch.cuda.device(q_lat.device):
+        seq_check(L.vla_seq_latent_decode(
+            out.data_ptr(), st(out, 0), st(out, 1), q_lat.data_ptr(), st(q_lat, 0), st(q_lat, 1), q_rot.data_ptr(),
+            st(q_rot, 0), st(q_rot, 1), cache.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
+            query_start_loc.data_ptr(), context_lens.data_ptr(), B, H, rank, rot, BS, NB, float(scale), ranges,
+            _p(scratch), need, _dt(q_lat.dtype), int(window), _p(gate), 0 if gate is None else _rows(gate, H),
+            _p(sinks), _stream(q_lat.device)), "latent_decode")
+
+
 def latent_prompt_supported(q: torch.Tensor, dim: int, rot: int, vdim: int, rank: int, cache: torch.Tensor) -> bool:
     """Whether latent_prompt takes these sizes, query rows [T, heads * (dim + rot)] and cache: only where the
     matrix-core latent kernel takes them too, whose weights have 16 bits as latent_prompt's (those of the kernel for all

@@ -238,7 +238,11 @@ class LatentKVAttention(nn.Module):
         q_lat, q_rot, o_rows = q_lat.transpose(0, 1), q3.narrow(2, D, Rr), o_lat.transpose(0, 1)
         if ops.latent_attention_tiles_supported(q_lat, q_rot, cache):
             # 16-bit models whose sizes fit: (token, head) rows in tiles of 32 on the matrix cores
-            if part is None:
+            if part is None and batch.max_query_len == 1 and ops.latent_decode_supported(o_rows, q_lat, q_rot, cache):
+                keys = min(batch.max_seq_len, self.window or batch.max_seq_len)
+                ops.latent_decode(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.query_start_loc,
+                                  batch.context_lens, keys, self.scale, self.window, gate, sinks)
+            elif part is None:
                 ops.latent_attention_tiles(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.query_start_loc,
                                            batch.context_lens, batch.max_query_len, self.scale, self.key_splits(batch),
                                            self.window, gate, sinks)
