@@ -344,7 +344,8 @@ int vla_seq_grouped_glu(void* out, int64_t out_stride, const void* a, int64_t a_
                         int dtype, int num_experts, void* stream);
 
 /* Form of the 16-bit product for tests: 0 = per shape, 1 = one-wave workgroups (decode steps),
- * 2 = runs of tiles per workgroup (prompts), 3 and 4 = the LDS-DMA forms for few and for many rows. */
+ * 2 = runs of tiles per workgroup (prompts), 3 and 4 = the LDS-DMA forms for few and for many rows (5 and 6:
+ * with runs of up to 128 and of up to 256 rows). */
 int vla_seq_set_grouped_linear_form(int mode);
 
 /* out[t] (fp32 [T, width]) = sum_k weights[t, k] * (y[pair_row[t, k]] or, where pair_row is -1,

@@ -700,7 +700,7 @@ def grouped_glu(out: torch.Tensor, a: torch.Tensor, row_token: Optional[torch.Te
 
 def set_grouped_linear_form(mode: int) -> None:
     """0: grouped_linear picks its 16-bit form per shape; 1: one-wave workgroups; 2: runs of tiles; 3, 4: the
-    LDS-DMA forms for few and for many rows."""
+    LDS-DMA forms for few and for many rows (5, 6: with runs of up to 128 and of up to 256 rows)."""
     seq_check(_lib.seq_lib().vla_seq_set_grouped_linear_form(mode), "set_grouped_linear_form")
 
 

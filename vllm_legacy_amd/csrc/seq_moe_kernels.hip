@@ -13,6 +13,8 @@
 // A row's result does not depend on which other rows share its tile or on where the plan put it.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
+#include <type_traits>
 
 #include "seq_common.h"
 
@@ -408,20 +410,35 @@ struct GroupedDma {
   int max_tiles, n_out, k_in, act;
   float limit, alpha, shift;        // the clamped form's, act == kActClamped
   int col_tiles;
-  int64_t groups;                   // workgroups along the rows
 };
 constexpr int kActClamped = 100;
 constexpr int kStep = 64;           // contraction values of a stage: rows of 128 bytes
-constexpr int kRunRows = 4;         // row tiles of a run, at most (a power of two)
 
-__device__ __forceinline__ float glu_apply(float g, float u, const GroupedDma& a) {
-  if (a.act == kActClamped) {
-    const float gc = fminf(g, a.limit), uc = fminf(fmaxf(u, -a.limit), a.limit);
-    return gc / (1.f + expf(-a.alpha * gc)) * (uc + a.shift);
-  }
-  return act_apply(g, a.act) * u;
+// 1 / (1 + exp(-s z)), s z held to both ends of the exponent's range; exp's argument in two numbers
+__device__ __forceinline__ float sigmoid_of(float z, float s) {
+  const float y = __builtin_amdgcn_fmed3f(-s * z, -120.f, 120.f);
+  const float t = 1.44269504f * y, r = fmaf(1.44269504f, y, -t) + 1.92596299e-8f * y;
+  const float e = __builtin_amdgcn_exp2f(t);
+  // the reciprocal of a number near 2^127 would be flushed, so both are held 2^32 apart
+  return __builtin_amdgcn_rcpf(fmaf(fmaf(e, 0.693147181f * r, e), 0x1p-32f, 0x1p-32f)) * 0x1p-32f;
 }
 
+// act(g) * u of four values, the choice of act made once
+__device__ __forceinline__ void glu4(float (&v)[4], const float (&u)[4], const GroupedDma& a) {
+  if (a.act == VLA_ACT_SILU) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = v[k] * sigmoid_of(v[k], 1.f) * u[k];
+  } else if (a.act == kActClamped) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float gc = fminf(v[k], a.limit), uc = fminf(fmaxf(u[k], -a.limit), a.limit);
+      v[k] = gc / (1.f + expf(-a.alpha * gc)) * (uc + a.shift);
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = act_apply(v[k], a.act) * u[k];
+  }
+}
 // 16 bytes per lane from each lane's own address into 1 KB of LDS (no register result)
 __device__ __forceinline__ void moe_dma16(const void* src, uint32_t lds_at) {
   unsigned keep;
@@ -430,6 +447,27 @@ __device__ __forceinline__ void moe_dma16(const void* src, uint32_t lds_at) {
       : "=&s"(keep)
       : "v"(src), "s"(lds_at)
       : "memory");
+}
+
+// the same from a base that the wave shares plus a 32-bit offset, while at < end (no branch that the compiler sees, so
+// what stands around it stays one stretch of instructions)
+__device__ __forceinline__ void moe_dma16(const unsigned char* base, uint32_t off, uint32_t lds_at, int at, int end) {
+  unsigned keep;
+  asm volatile(
+      "s_cmp_lt_i32 %4, %5\n\ts_cbranch_scc0 1f\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0\n1:"
+      : "=&s"(keep)
+      : "v"(off), "s"(base), "s"(lds_at), "s"(at), "s"(end)
+      : "memory", "scc");
+}
+__device__ __forceinline__ void moe_dma16(const unsigned char* src, uint32_t lds_at, int at, int end) {
+  unsigned keep;
+  asm volatile(
+      "s_cmp_lt_i32 %3, %4\n\ts_cbranch_scc0 1f\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0\n1:"
+      : "=&s"(keep)
+      : "v"(src), "s"(lds_at), "s"(at), "s"(end)
+      : "memory", "scc");
 }
 
 // Where a column tile of the few-rows form starts in the contraction.  Rows are a power of two apart in most
@@ -453,163 +491,317 @@ __device__ __forceinline__ void store4(typename SO::T* to, const float (&v)[4], 
   }
 }
 
-// The run of at most kRunRows row tiles of one expert that is number `want` among all such runs: (first tile,
-// count), count 0 behind the last.  Runs start at every kRunRows-th tile from the first of neighbours that have
-// the same expert; every wave scans the tiles' experts for itself.
-__device__ __forceinline__ int2 find_run(const int* __restrict__ tile_expert, int max_tiles, int want) {
-  const int lane = threadIdx.x & 63;
-  int seen = 0, first = 0;                                 // runs before this stretch of 64; its expert's first tile
-  for (int i0 = 0; i0 < max_tiles; i0 += kWave) {
-    const int i = i0 + lane;
-    const int e = i < max_tiles ? tile_expert[i] : -1, before = i > 0 && i < max_tiles ? tile_expert[i - 1] : -1;
-    const uint64_t edges = __ballot(e != before || i == 0);
-    const uint64_t upto = edges & (~0ull >> (63 - lane));
-    const int f = upto ? i0 + 63 - __builtin_clzll(upto) : first;
-    const uint64_t starts = __ballot(e >= 0 && ((i - f) & (kRunRows - 1)) == 0);
-    const int n = __builtin_popcountll(starts);
-    if (want < seen + n) {
-      uint64_t left = starts;
-      for (int k = want - seen; k > 0; --k) left &= left - 1;
-      const int at = __builtin_ctzll(left);
-      const int tile = i0 + at, mine = tile_expert[tile];
-      int count = 1;
-      while (count < kRunRows && tile + count < max_tiles && tile_expert[tile + count] == mine) ++count;
-      return make_int2(tile, count);
-    }
-    seen += n;
-    first = edges ? i0 + 63 - __builtin_clzll(edges) : first;
+// Runs: the tiles of neighbours that have the same expert, split evenly into runs of at most RUN.  The workgroup's eight
+// waves look at 64 tiles each and leave where experts change and where runs start in LDS (one wait for memory); 24 bytes
+// a stretch of 64 tiles.
+struct Runs {
+  const uint64_t* edges;           // [stretches] a tile whose expert is not that of the tile before
+  const uint64_t* starts;          // [stretches] a run's first tile
+  const int* counts;               // [stretches] number of those
+  int stretches, max_tiles;
+  // the last edge at or before tile i, the first one behind it
+  __device__ __forceinline__ int first(int i) const {
+    int s = i >> 6;
+    uint64_t m = edges[s] & (~0ull >> (63 - (i & 63)));
+    while (m == 0) m = edges[--s];                         // tile 0 is one
+    return 64 * s + 63 - __builtin_clzll(m);
   }
-  return make_int2(0, 0);
+  __device__ __forceinline__ int end(int i) const {
+    int s = i >> 6;
+    uint64_t m = (i & 63) == 63 ? 0 : edges[s] & (~0ull << ((i & 63) + 1));
+    while (m == 0 && s + 1 < stretches) m = edges[++s];
+    return m ? 64 * s + __builtin_ctzll(m) : max_tiles;
+  }
+};
+template <int RUN>
+__device__ __forceinline__ int run_size(int tiles) { return (tiles + (tiles + RUN - 1) / RUN - 1) / ((tiles + RUN - 1) / RUN); }
+
+// every wave of the workgroup calls it; the number of runs
+template <int RUN>
+__device__ __forceinline__ int look_up_runs(const int* __restrict__ tile_expert, int max_tiles, unsigned char* smem, Runs& r) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int stretches = (max_tiles + 63) / 64;
+  uint64_t* edges = reinterpret_cast<uint64_t*>(smem);
+  uint64_t* starts = edges + stretches;
+  int* counts = reinterpret_cast<int*>(starts + stretches);
+  r = Runs{edges, starts, counts, stretches, max_tiles};
+  for (int s = w; s < stretches; s += 8) {
+    const int i = 64 * s + lane, at = min(i, max_tiles - 1);
+    const int e = tile_expert[at], before = tile_expert[max(at - 1, 0)];
+    const uint64_t m = __ballot(i < max_tiles && (e != before || i == 0)), used = __ballot(i < max_tiles && e >= 0);
+    if (lane == 0) edges[s] = m, starts[s] = used;
+  }
+  __syncthreads();
+  int total = 0;
+  for (int s = w; s < stretches; s += 8) {
+    const int i = 64 * s + lane;
+    bool start = false;
+    if ((starts[s] >> lane) & 1) {
+      const int f = r.first(i);
+      start = (i - f) % run_size<RUN>(r.end(i) - f) == 0;
+    }
+    const uint64_t m = __ballot(start);
+    if (lane == 0) starts[s] = m, counts[s] = __builtin_popcountll(m);
+  }
+  __syncthreads();
+  for (int s = lane; s < stretches; s += 64) total += counts[s];
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) total += __shfl_xor(total, m, 64);
+  return __builtin_amdgcn_readfirstlane(total);
+}
+// run number `want` (below the number of runs): (first tile, tiles)
+template <int RUN>
+__device__ __forceinline__ int2 run_number(const Runs& r, int want) {
+  int s = 0, n = r.counts[0];
+  while (want >= n) want -= n, n = r.counts[++s];
+  uint64_t m = r.starts[s];
+  for (; want > 0; --want) m &= m - 1;
+  const int tile = 64 * s + __builtin_ctzll(m), f = r.first(tile), end = r.end(tile);
+  return make_int2(tile, min(run_size<RUN>(end - f), end - tile));
 }
 
-// Many rows.  A workgroup is a run of up to 128 rows of one expert by 256 weight rows (GLU: 128 gates and
-// their 128 ups), eight waves of 64 x 64 each; three stages of 48 KB that LDS-DMA fills two steps ahead, one
-// barrier per 64 contraction values, one workgroup per CU.  A stage's row is 128 bytes: its 16-byte pieces
-// are exchanged by the row's number (on the source's side, LDS-DMA writes a row in a row), so the 32 lanes
-// of a fragment read meet all banks.  The launch is cut among the 8 XCDs in contiguous stretches
-// (workgroups go to them round robin), and a stretch goes over up to eight column tiles for each run of rows,
-// so that what runs together shares rows and weights in one L2.  4096 rows of 2048, two of 16 experts of
-// 1408: gate | up and activation 184 us (the LDS form with registers on the way 311 and 17), down 113
-// (189).  A step takes 1.3 us where its products need 0.43; a third of the CUs' time is the last round of
-// workgroups.  128 x 128 tiles with two workgroups per CU and two stages take 190 and 110, four waves
-// of 256 x 64 (less LDS traffic, nothing beside a wave on its SIMD) 304 and 206, column tiles that start
-// at different places of the contraction 190 and 117.
-template <class S, class SO, bool GLU>
+// Many rows.  A workgroup is a run of up to 64 MB rows of one expert by 256 weight rows (GLU: 128 gates and their 128
+// ups), eight waves of 32 MB x 64 each, one workgroup per CU.  LDS-DMA fills a ring of three slots of weights (32 KB for
+// 64 contraction values) and one of two (MB = 4) or three slots of rows; a slot's row is 128 bytes: its 16-byte pieces
+// are exchanged by the row's number (on the source's side, LDS-DMA writes a row in a row), so the 32 lanes of a fragment
+// read meet all banks.  A stage is four phases of 2 MB products, each with the reads of the next phase's fragments and
+// one or two DMA instructions set between them one by one: eight waves that send their DMA together right behind the
+// barrier keep the matrix cores waiting for a thousand cycles, and reads that the compiler moves down to their use make
+// every product wait.  The barrier stands in the middle of the last phase.  The launch's tiles, counted on the device,
+// are cut among the 8 XCDs in contiguous stretches (workgroups go to them round robin), and a stretch goes over up to
+// eight column tiles for each run, so that what runs together shares rows and weights in one L2.
+// 4096 rows of 2048, two of 16 experts of 1408: gate | up and activation 118 us, 800 TFLOP/s (178 with all DMA behind the
+// barrier, reads where they are used and runs that are not split evenly; 105 without DMA), down 87 (107).  A tile of 256
+// rows: runs and first stage 7 us, 32 stages of 1.4 (0.9 for the products), activation and stores 8.
+template <class S, class SO, bool GLU, int MB>
 __global__ __launch_bounds__(512, 2) void grouped_dma_kernel(GroupedDma a) {
-  constexpr int ROWS = 32 * kRunRows, WROWS = 256, STAGE = (ROWS + WROWS) * 128, RING = 3;
+  constexpr int RUN = 2 * MB, AU = 32 * RUN * 128, WU = 256 * 128, RA = MB == 4 ? 2 : 3, RW = 3;
+  constexpr int AI = AU / 8192;                            // DMA instructions of a wave for a stage's rows (weights: 4)
+  constexpr int YOUNG = MB == 4 ? 4 : 6;                   // of them may be on their way when the next stage must be there
   extern __shared__ __align__(16) unsigned char smem[];
-  // stretches of XCDs, then (eight column tiles)(rows)(column tile)
-  const int64_t total = a.groups * a.col_tiles, per = (total + 7) / 8;
-  const int64_t id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if ((int64_t)(blockIdx.x >> 3) >= per || id >= total) return;
-  const int64_t wide = a.groups * 8;
-  const int cb = (int)(id / wide);
-  const int width = min(8, a.col_tiles - 8 * cb);
-  const int64_t rest = id - cb * wide;
-  const int col = 8 * cb + (int)(rest % width);
-  const int n0 = col * (GLU ? 128 : 256);
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hf = lane >> 5, c = lane & 31, wm = w & 1, wn = w >> 1;
   const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
   const int x = hf ^ ((c >> 1) & 7);                       // piece 2 ks + hf stands at (2 ks) ^ x
   const int steps = a.k_in / kStep;
   const bool vec = a.out_stride % 4 == 0 && (uintptr_t)a.out % 16 == 0;
-  // one run per workgroup; those of the last number, which has no run while an expert's tiles are neighbours, take
-  // all that are left
-  for (int64_t want = rest / width;; ++want) {
-    const int2 run = find_run(a.tile_expert, a.max_tiles, (int)want);
-    if (run.y == 0) return;
-    const int e = a.tile_expert[run.x];
-    const int rows = run.y * kTile;
+  [[maybe_unused]] const bool vec8 = a.out_stride % 8 == 0 && (uintptr_t)a.out % 16 == 0;
+  Runs table;
+  const int runs = look_up_runs<RUN>(a.tile_expert, a.max_tiles, smem, table);
+  // stretches of XCDs, then (eight column tiles)(runs)(column tile)
+  const int64_t total = (int64_t)runs * a.col_tiles, per = (total + 7) / 8, wide = (int64_t)runs * 8;
+  for (int64_t slot = blockIdx.x >> 3; slot < per; slot += gridDim.x >> 3) {
+    const int64_t id = (blockIdx.x & 7) * per + slot;
+    if (id >= total) return;
+    if (slot != blockIdx.x >> 3) look_up_runs<RUN>(a.tile_expert, a.max_tiles, smem, table);   // the stages lay over it
+    const int cb = (int)(id / wide);
+    const int width = min(8, a.col_tiles - 8 * cb);
+    const int64_t rest = id - cb * wide;
+    const int n0 = (8 * cb + (int)(rest % width)) * (GLU ? 128 : 256);
+    const int2 run = run_number<RUN>(table, __builtin_amdgcn_readfirstlane((int)(rest / width)));
+    const int run0 = __builtin_amdgcn_readfirstlane(run.x), tiles = __builtin_amdgcn_readfirstlane(run.y);
+    const int e = __builtin_amdgcn_readfirstlane(a.tile_expert[run0]);
+    const int rows = tiles * kTile;
+    __syncthreads();                                       // the table is read
 
-    // wave w brings 16 rows and 32 weight rows, eight per instruction
-    const unsigned char* src_a[2];
-    const unsigned char* src_w[4];
+    // wave w brings 8 AI rows and 32 weight rows, eight per instruction
+    const unsigned char* src_a[AI];
+    uint32_t off_w[4];
     const int64_t weight_rows = (int64_t)(GLU ? 2 : 1) * a.n_out;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int r = 16 * w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
-      const int row = run.x * kTile + min(r, rows - 1);
+    for (int u = 0; u < AI; ++u) {
+      const int r = 8 * AI * w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
+      const int row = run0 * kTile + min(r, rows - 1);
       const int src = a.row_token != nullptr ? max(0, a.row_token[row]) : row;     // padding reads token 0
       src_a[u] = (const unsigned char*)a.a + (int64_t)src * a.a_stride * 2 + 16 * piece;
     }
+    // a wave's 32 weight rows are gates or ups
+    const int first_w = GLU ? 32 * (w & 3) : 32 * w;
+    const unsigned char* base_w =
+        (const unsigned char*)a.weight + ((int64_t)e * weight_rows + (GLU && w >= 4 ? a.n_out : 0) + n0) * a.k_in * 2;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int r = 32 * w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
-      const int n = GLU ? (r < 128 ? min(n0 + r, a.n_out - 1) : a.n_out + min(n0 + r - 128, a.n_out - 1)) : min(n0 + r, a.n_out - 1);
-      src_w[u] = (const unsigned char*)a.weight + ((int64_t)e * weight_rows + n) * a.k_in * 2 + 16 * piece;
+      const int r = first_w + 8 * u + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
+      off_w[u] = (uint32_t)min(r, a.n_out - 1 - n0) * (uint32_t)(2 * a.k_in) + 16 * piece;
     }
-    auto bring = [&](int step, int buf) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) moe_dma16(src_a[u] + step * (2 * kStep), lds0 + buf * STAGE + w * 2048 + 1024 * u);
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        moe_dma16(src_w[u] + step * (2 * kStep), lds0 + buf * STAGE + ROWS * 128 + w * 4096 + 1024 * u);
+    const uint32_t at_a = lds0 + RW * WU + w * (1024 * AI), at_w = lds0 + w * 4096;
+    auto bring_a = [&](int u, int step, int slot) { moe_dma16(src_a[u] + step * (2 * kStep), at_a + slot * AU + 1024 * u, step, steps); };
+    auto bring_w = [&](int u, int step, int slot) {
+      moe_dma16(base_w + step * (2 * kStep), off_w[u], at_w + slot * WU + 1024 * u, step, steps);
     };
-    f32x16 acc[2][2];
+    f32x16 acc[MB][2];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
-    const bool active = 64 * wm < rows;
-    bring(0, 0);
-    if (steps > 1) bring(1, 1);
-    int buf = 0;
-    for (int it = 0; it < steps; ++it) {
-      if (it + 1 < steps)
-        asm volatile("s_waitcnt vmcnt(6)" ::: "memory");      // all but the next stage
-      else
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (it + 2 < steps) bring(it + 2, buf >= 1 ? buf - 1 : RING - 1);
-      const unsigned char* stage = smem + buf * STAGE;
-      buf = buf + 1 < RING ? buf + 1 : 0;
-      if (!active) continue;
-      const unsigned char* a_lds = stage + (64 * wm + c) * 128;
-      const unsigned char* w_lds = stage + ROWS * 128 + ((GLU ? 32 : 64) * wn + c) * 128;
+    // the prologue: as many stages as the rings hold, oldest first
 #pragma unroll
-      for (int ks = 0; ks < kStep / 16; ++ks) {
-        u32x4 av[2], wv[2];
+    for (int st = 0; st < 3; ++st) {
+      if (st < RA)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          av[b] = *reinterpret_cast<const u32x4*>(a_lds + b * 32 * 128 + 16 * ((2 * ks) ^ x));
-          wv[b] = *reinterpret_cast<const u32x4*>(w_lds + b * (GLU ? 128 : 32) * 128 + 16 * ((2 * ks) ^ x));
+        for (int u = 0; u < AI; ++u) bring_a(u, st, st);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) bring_w(u, st, st);
+    }
+    if (steps > 2)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AI + 4 + YOUNG) : "memory");
+    else if (steps > 1)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AI + 4) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    // NB of the wave's row blocks (tiles wm, wm + 2, ... of the run) hold rows
+    auto walk = [&](auto nbv) {
+      constexpr int NB = decltype(nbv)::value;
+      struct Frag {
+        u32x4 v[NB + 2];                                   // two of weights, NB of rows
+      };
+      int sa = 0, sw = 0;
+      const unsigned char* a_lds = smem + RW * WU + (32 * wm + c) * 128;
+      const unsigned char* w_lds = smem + ((GLU ? 32 : 64) * wn + c) * 128;
+      // eight products (2 NB), the reads of the next fragments and DMA instructions between them one by one: left to
+      // itself the compiler moves the reads down to where they are used
+      auto phase = [&](const Frag& f, Frag& next, int ks, auto&& dma) {
+        const unsigned char *wp = w_lds + sw * WU + 16 * ((2 * ks) ^ x), *ap = a_lds + sa * AU + 16 * ((2 * ks) ^ x);
+        constexpr int PER = NB > 1 ? 1 : 2;                // reads ahead of a product
+#pragma unroll
+        for (int i = 0; i < (NB > 0 ? 2 * NB : 4); ++i) {
+          if constexpr (NB > 0) {
+#pragma unroll
+            for (int j = PER * i; j < PER * i + PER; ++j)
+              if (j < NB + 2)
+                next.v[j] = *reinterpret_cast<const u32x4*>(j < 2 ? wp + j * (GLU ? 128 : 32) * 128 : ap + (j - 2) * 64 * 128);
+            __builtin_amdgcn_sched_barrier(0);
+            acc[i >> 1][i & 1] = Mma16<S>::run(f.v[i & 1], f.v[2 + (i >> 1)], acc[i >> 1][i & 1]);
+          }
+          dma(i);
+          __builtin_amdgcn_sched_barrier(0);
         }
+      };
+      constexpr int SPAN = NB > 0 ? 2 * NB : 4;            // places of a phase
+      // the last phase of a stage: half of its products, the change of stages, the other half with the reads of the next
+      // stage's first fragments and the DMA of rows into what is free now
+      auto turn = [&](const Frag& f, Frag& next, int it, int free_a) {
+        const unsigned char *wp = w_lds + sw * WU + 16 * x, *ap = a_lds + sa * AU + 16 * x;
+        constexpr int HALF = SPAN / 2, PER = (NB + 2 + HALF - 1) / HALF, APER = (AI + HALF - 1) / HALF;
+        if constexpr (NB > 0) {
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+          for (int i = 0; i < HALF; ++i) acc[i >> 1][i & 1] = Mma16<S>::run(f.v[i & 1], f.v[2 + (i >> 1)], acc[i >> 1][i & 1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0xc07f);                // lgkmcnt(0): this stage is read
+        // the next stage is there when all but the youngest have come
+        asm volatile("s_cmp_lt_i32 %0, %1\n\ts_cbranch_scc1 1f\n\ts_waitcnt vmcnt(0)\n1:\n\ts_waitcnt vmcnt(%2)" ::"s"(it + 2), "s"(steps),
+                     "n"(YOUNG)
+                     : "memory", "scc");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
 #pragma unroll
-          for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = Mma16<S>::run(wv[nb], av[mb], acc[mb][nb]);
+        for (int i = HALF; i < SPAN; ++i) {
+          if constexpr (NB > 0) {
+#pragma unroll
+            for (int j = PER * (i - HALF); j < PER * (i - HALF) + PER; ++j)
+              if (j < NB + 2)
+                next.v[j] = *reinterpret_cast<const u32x4*>(j < 2 ? wp + j * (GLU ? 128 : 32) * 128 : ap + (j - 2) * 64 * 128);
+            __builtin_amdgcn_sched_barrier(0);
+            acc[i >> 1][i & 1] = Mma16<S>::run(f.v[i & 1], f.v[2 + (i >> 1)], acc[i >> 1][i & 1]);
+          }
+#pragma unroll
+          for (int u = APER * (i - HALF); u < APER * (i - HALF) + APER; ++u)
+            if (u < AI) bring_a(u, it + RA, free_a);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      Frag f0, f1;
+      if constexpr (NB > 0)
+#pragma unroll
+        for (int j = 0; j < NB + 2; ++j)
+          f0.v[j] = *reinterpret_cast<const u32x4*>(j < 2 ? w_lds + j * (GLU ? 128 : 32) * 128 + 16 * x : a_lds + (j - 2) * 64 * 128 + 16 * x);
+      int last_w = 0;                                      // the slot that the stage before freed
+      for (int it = 0; it < steps; ++it) {
+        // W of stage it + 2 in the slot that stage it - 1 left (the first three stages are there already)
+        auto dma_w = [&](int u) {
+          if (u < 4) moe_dma16(base_w + (it + 2) * (2 * kStep), off_w[u], at_w + last_w * WU + 1024 * u, it == 0 ? steps : it + 2, steps);
+        };
+        phase(f0, f1, 1, [&](int i) { if (i == SPAN / 2) dma_w(0); if (i == SPAN - 1) dma_w(1); });
+        phase(f1, f0, 2, [&](int i) { if (i == SPAN / 2) dma_w(2); if (i == SPAN - 1) dma_w(3); });
+        phase(f0, f1, 3, [&](int) {});
+        const int free_a = sa;
+        last_w = sw;
+        sa = sa + 1 < RA ? sa + 1 : 0;
+        sw = sw + 1 < RW ? sw + 1 : 0;
+        // behind the last stage this reads a slot that holds an older one; nothing uses it
+        turn(f1, f0, it, free_a);
       }
+    };
+    const int mine = (tiles - wm + 1) / 2;
+    if (mine == MB)
+      walk(std::integral_constant<int, MB>());
+    else if (MB > 2 && mine == 3)
+      walk(std::integral_constant<int, MB == 4 ? 3 : MB>());
+    else if (mine > 0)
+      walk(std::integral_constant<int, MB / 2>());
+    else
+      walk(std::integral_constant<int, 0>());
+    float scale[MB];
+    bool live[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {                      // all at once: one wait for memory
+      const int row = run0 * kTile + min(64 * mb + 32 * wm + c, rows - 1);
+      live[mb] = a.row_token == nullptr || a.row_token[row] >= 0;
+      scale[mb] = a.row_scale != nullptr ? a.row_scale[row] : 1.f;
     }
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb) {
-      const int r = 64 * wm + 32 * mb + c;
-      if (r >= rows) continue;
-      const int row = run.x * kTile + r;
-      const bool live = a.row_token == nullptr || a.row_token[row] >= 0;
+    for (int mb = 0; mb < MB; ++mb) {
+      const int r = 64 * mb + 32 * wm + c;
+      if (64 * mb + 32 * wm >= rows) continue;             // all of the wave's 32 rows or none
+      const int row = run0 * kTile + r;
       // a padding row leaves what zeros would; its scale was never written
-      const float sc = live ? (a.row_scale != nullptr ? a.row_scale[row] : 1.f) : 0.f;
+      const float sc = live[mb] ? scale[mb] : 0.f;
       typename SO::T* to = (typename SO::T*)a.out + (int64_t)row * a.out_stride;
+      [[maybe_unused]] u32x2 half[4];
 #pragma unroll
       for (int nb = 0; nb < (GLU ? 1 : 2); ++nb)
 #pragma unroll
         for (int i4 = 0; i4 < 4; ++i4) {
           const int n = n0 + (GLU ? 32 * wn : 64 * wn + 32 * nb) + 8 * i4 + 4 * hf;
-          float v[4];
+          float v[4], up[4];
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const float z = live ? acc[mb][nb][4 * i4 + k] * sc : 0.f;
-            if constexpr (GLU)
-              v[k] = glu_apply(z, live ? acc[mb][1][4 * i4 + k] * sc : 0.f, a);
-            else
-              v[k] = act_apply(z, a.act);
+            v[k] = live[mb] ? acc[mb][nb][4 * i4 + k] * sc : 0.f;
+            up[k] = live[mb] ? acc[mb][1][4 * i4 + k] * sc : 0.f;
           }
-          store4<SO>(to + n, v, n, a.n_out, vec);
+          if constexpr (GLU) {
+            glu4(v, up, a);
+          } else if (a.act != VLA_ACT_NONE) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = act_apply(v[k], a.act);
+          }
+          if constexpr (sizeof(typename SO::T) == 2) {
+            half[i4] = u32x2{pack16<SO>(v[0], v[1]), pack16<SO>(v[2], v[3])};
+            if (i4 & 1) {
+              // the two halves of the wave hold four columns of each of two groups of eight; exchanged, a lane has one
+              // group whole: 16 bytes a store
+              const auto lo = __builtin_amdgcn_permlane32_swap(half[i4 - 1][0], half[i4][0], false, false);
+              const auto hi = __builtin_amdgcn_permlane32_swap(half[i4 - 1][1], half[i4][1], false, false);
+              const int n8 = n0 + (GLU ? 32 * wn : 64 * wn + 32 * nb) + 8 * (i4 - 1) + 8 * hf;
+              const u32x4 all = {lo[0], hi[0], lo[1], hi[1]};
+              if (vec8 && n8 + 7 < a.n_out) {
+                *reinterpret_cast<u32x4*>(to + n8) = all;
+              } else {
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                  if (n8 + k < a.n_out) to[n8 + k] = __builtin_bit_cast(typename SO::T, (uint16_t)(all[k >> 1] >> (16 * (k & 1))));
+              }
+            }
+          } else {
+            store4<SO>(to + n, v, n, a.n_out, vec);
+          }
         }
     }
-    if (want + 1 < a.groups) return;
     __syncthreads();                                       // the stages are read
   }
 }
@@ -720,8 +912,7 @@ __global__ __launch_bounds__(256) void grouped_stream_kernel(GroupedDma a) {
     if constexpr (GLU) {
       float up[4];
       sum(1, w, up);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = glu_apply(v[k], up[k], a);
+      glu4(v, up, a);
     } else {
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[k] = act_apply(v[k], a.act);
@@ -730,9 +921,26 @@ __global__ __launch_bounds__(256) void grouped_stream_kernel(GroupedDma a) {
   }
 }
 
+constexpr int kMaxTiles = 1 << 18;   // of a launch for many rows: 24 bytes of LDS for 64 of them
+constexpr int kMaxRowsK = 1 << 22;   // its offsets inside a tile of weights have 32 bits
+
+// Runs of up to 256 rows or of up to 128: what counts is how often the 256 CUs are filled (behind the second time by
+// parts), at 1.55 of the time for a tall run.  An expert has its average of rows and, as they differ, half a run more.
+// us of both products, runs of 128 / 256 rows, 16 experts, top 2, of 1408 x 2048: 1024 tokens 42 + 27 / 44 + 33, 1536
+// 64 + 31 / 55 + 42, 2048 68 + 57 / 86 + 46, 3072 100 + 64 / 99 + 50, 4096 134 + 88 / 118 + 87; 32 experts, top 4, of
+// 1408 x 4096: 512 167 + 93 / 182 + 98, 1024 177 + 126 / 196 + 111, 2048 314 + 181 / 295 + 171.
+bool tall_runs(int max_tiles, int num_experts, int col_tiles) {
+  const double mean = 32.0 * std::max(0, max_tiles - num_experts) / num_experts;
+  auto fills = [&](double rows) {
+    const double n = num_experts * std::max(1.0, mean / rows + 0.5) * col_tiles / 256.0;
+    return n <= 2.0 ? std::ceil(n) : n + 0.5;
+  };
+  return 1.55 * fills(256) < fills(128);
+}
+
 template <class S, class SO, bool GLU>
 int launch_grouped_dma(GroupedDma a, int num_experts, bool few, hipStream_t stream) {
-  if (few && a.max_tiles <= 65535) {
+  if ((few || a.k_in > kMaxRowsK) && a.max_tiles <= 65535) {
     constexpr int lds = 4 * 3 * (kTile + 64) * 128;
     static std::atomic<bool> raised{false};           // LDS limit: raised once per kernel, not per launch
     if (!raised.load(std::memory_order_relaxed)) {
@@ -743,33 +951,52 @@ int launch_grouped_dma(GroupedDma a, int num_experts, bool few, hipStream_t stre
     const int cols = GLU ? 32 : 64;
     grouped_stream_kernel<S, SO, GLU><<<dim3((a.n_out + cols - 1) / cols, a.max_tiles), 256, lds, stream>>>(a);
   } else {
-    constexpr int lds = 3 * (32 * kRunRows + 256) * 128;
-    static std::atomic<bool> raised{false};
-    if (!raised.load(std::memory_order_relaxed)) {
-      VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&grouped_dma_kernel<S, SO, GLU>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-      raised.store(true, std::memory_order_relaxed);
-    }
     const int cols = GLU ? 128 : 256;
     a.col_tiles = (a.n_out + cols - 1) / cols;
-    // where an expert's tiles are neighbours (as moe_plan leaves them) it adds at most one run that is not full, and
-    // the last number has none; tiles in another order are more runs, which the workgroups of that number walk
-    a.groups = a.max_tiles / kRunRows + std::min(num_experts, a.max_tiles) + 1;
-    const int64_t total = a.groups * a.col_tiles;
-    grouped_dma_kernel<S, SO, GLU><<<(unsigned)((total + 7) / 8 * 8), 512, lds, stream>>>(a);
+    auto go = [&](const GroupedDma& d, auto mbv) -> int {
+      constexpr int MB = decltype(mbv)::value, lds = MB == 4 ? 160 * 1024 : 144 * 1024;
+      static std::atomic<bool> raised{false};
+      if (!raised.load(std::memory_order_relaxed)) {
+        VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&grouped_dma_kernel<S, SO, GLU, MB>),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        raised.store(true, std::memory_order_relaxed);
+      }
+      // where an expert's tiles are neighbours (as moe_plan leaves them) it adds at most one run that is not full;
+      // tiles in another order are more runs, which the workgroups walk
+      const int64_t total = (int64_t)(d.max_tiles / (2 * MB) + std::min(num_experts, d.max_tiles)) * d.col_tiles;
+      const int64_t groups = std::min<int64_t>((total + 7) / 8 * 8, 1 << 24);
+      grouped_dma_kernel<S, SO, GLU, MB><<<(unsigned)groups, 512, lds, stream>>>(d);
+      return VLA_OK;
+    };
+    const int form = g_grouped_form.load(std::memory_order_relaxed);
+    const bool tall = form == 5 || form == 6 ? form == 6 : tall_runs(a.max_tiles, num_experts, a.col_tiles);
+    // the kernel's table of runs has room for kMaxTiles
+    for (int t0 = 0; t0 < a.max_tiles; t0 += kMaxTiles) {
+      GroupedDma d = a;
+      const int64_t row = (int64_t)t0 * kTile;
+      d.max_tiles = a.max_tiles - t0 < kMaxTiles ? a.max_tiles - t0 : kMaxTiles;
+      d.tile_expert += t0;
+      d.out = (typename SO::T*)a.out + row * a.out_stride;
+      if (a.row_token != nullptr)
+        d.row_token += row;
+      else
+        d.a = (const typename S::T*)a.a + row * a.a_stride;
+      if (a.row_scale != nullptr) d.row_scale += row;
+      const int rc = tall ? go(d, std::integral_constant<int, 4>()) : go(d, std::integral_constant<int, 2>());
+      if (rc != VLA_OK) return rc;
+    }
   }
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   return VLA_OK;
 }
 
 // Whether a launch is bound by the weights, which in the forms for few rows every tile of 32 rows reads for
-// itself.  The plan leaves room for a tile per expert beside the full ones, so 2.5 tiles per expert are 48
-// rows each (us of the whole block, few / many rows form: 16 experts of 1408 x 2048, top 2: 128 tokens 102 /
-// 107, 256 127 / 149, 384 147 / 151, 512 155 / 154, 1024 215 / 184; 32 experts of 1408 x 4096, top 4: 128
-// 288 / 318, 256 339 / 371, 384 422 / 419, 512 461 / 413).  Without the number of experts: the workgroups
-// of the form for many rows would fill the part.
+// itself.  The plan leaves room for a tile per expert beside the full ones, so 1.5 tiles per expert are 16
+// rows each (us of both products, few / many rows form: 16 experts of 1408 x 2048, top 2: 128 tokens 55 / 50, 256 71 /
+// 52, 512 103 / 59; 32 experts of 1408 x 4096, top 4: 128 225 / 235, 256 284 / 245, 512 415 / 260).  Without the number
+// of experts: the workgroups of the form for many rows would fill the part.
 bool few_tiles(int max_tiles, int weight_rows, int num_experts) {
-  return num_experts > 0 ? 2 * (int64_t)max_tiles <= 5 * (int64_t)num_experts
+  return num_experts > 0 ? 2 * (int64_t)max_tiles <= 3 * (int64_t)num_experts
                          : (int64_t)max_tiles * ((weight_rows + 127) / 128) <= 1024;
 }
 
@@ -917,9 +1144,9 @@ int grouped_linear(void* out, int64_t out_stride, int out_dtype, const void* a,
         // and runs of tiles that share the weight fragments
         const int form = g_grouped_form.load(std::memory_order_relaxed);
         const bool few = form == 0 ? few_tiles(max_tiles, n_out, 0) : form == 1;
-        if (dma_fits(a, a_stride, weight, k_in) && (form == 0 || form == 3 || form == 4)) {
+        if (dma_fits(a, a_stride, weight, k_in) && (form == 0 || form >= 3)) {
           GroupedDma d{out, out_stride, a, a_stride, row_token, weight, tile_expert, row_scale, max_tiles, n_out, k_in, act,
-                       0.f, 0.f, 0.f, 0, 0};
+                       0.f, 0.f, 0.f, 0};
           return launch_grouped_dma<S, SO, false>(d, num_experts > 0 ? num_experts : max_tiles,
                                                   form == 0 ? few_tiles(max_tiles, n_out, num_experts) : form == 3, st);
         }
@@ -968,7 +1195,7 @@ extern "C" int vla_seq_grouped_linear_of(void* out, int64_t out_stride, int out_
 
 extern "C" int vla_seq_grouped_glu_supported(int k_in, int dtype) {
   const int form = g_grouped_form.load(std::memory_order_relaxed);
-  return (dtype == VLA_F16 || dtype == VLA_BF16) && k_in > 0 && k_in % kStep == 0 && (form == 0 || form == 3 || form == 4);
+  return (dtype == VLA_F16 || dtype == VLA_BF16) && k_in > 0 && k_in % kStep == 0 && (form == 0 || form >= 3);
 }
 
 extern "C" int vla_seq_grouped_glu(void* out, int64_t out_stride, const void* a, int64_t a_stride, const int* row_token,
@@ -985,7 +1212,7 @@ extern "C" int vla_seq_grouped_glu(void* out, int64_t out_stride, const void* a,
   auto go = [&](auto s) -> int {
     using S = decltype(s);
     const GroupedDma d{out, out_stride, a, a_stride, row_token, weight, tile_expert, row_scale, max_tiles, n_out, k_in,
-                       clamped ? kActClamped : act, limit, alpha, shift, 0, 0};
+                       clamped ? kActClamped : act, limit, alpha, shift, 0};
     return launch_grouped_dma<S, S, true>(d, num_experts, few, (hipStream_t)stream);
   };
   if (dtype == VLA_BF16) return go(BF16{});
@@ -1012,10 +1239,10 @@ extern "C" int vla_seq_moe_combine(float* out, const float* y, const int* pair_r
 }
 
 // 0: grouped_linear picks its 16-bit form per shape; 1: always one-wave workgroups; 2: always runs of
-// tiles; 3, 4: the LDS-DMA forms for few and for many rows where k_in allows.
+// tiles; 3, 4: the LDS-DMA forms for few and for many rows where k_in allows (5, 6: with runs of 128 and of 256 rows).
 // Tests run all.
 extern "C" int vla_seq_set_grouped_linear_form(int mode) {
-  if (mode < 0 || mode > 4) return VLA_ERR_ARG;
+  if (mode < 0 || mode > 6) return VLA_ERR_ARG;
   g_grouped_form.store(mode, std::memory_order_relaxed);
   return VLA_OK;
 }
