@@ -623,6 +623,16 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, correction: Optional[torch.
     return experts, weights, sg
 
 
+def moe_route_forms_logits(h: torch.Tensor, router: torch.Tensor, shared_gate_weight: Optional[torch.Tensor]) -> bool:
+    """Whether moe_route forms the logits of many tokens itself at least as fast as a matrix product ahead of it
+    (the conditions of csrc/seq_moe_kernels.hip's kernel for 16 tokens a workgroup)."""
+    rows = router.shape[0] + (0 if shared_gate_weight is None else 1)
+    size = h.element_size()
+    return rows <= 64 and h.shape[1] % 32 == 0 and h.stride(1) == 1 and h.data_ptr() % (8 * size) == 0 and \
+        _rows(h, h.shape[1]) % 8 == 0 and router.data_ptr() % 16 == 0 and \
+        (shared_gate_weight is None or shared_gate_weight.data_ptr() % 16 == 0)
+
+
 def moe_plan(experts: torch.Tensor, num_experts: int, weights: Optional[torch.Tensor] = None):
     """-> pair_row int32 [T, top], row_token int32 [rows], tile_expert int32 [tiles]; with weights (fp32
     [T, top]) also row_weight fp32 [rows], the weight of each row's pair (padding rows: anything)."""

@@ -39,21 +39,134 @@ __device__ __forceinline__ float act_apply(float z, int act) {
   }
 }
 
+// The choice of token t by LANES neighbouring lanes of a wave: z [routed (+ 1, the shared gate's)] its logits, group_best
+// and group_open room for `groups` values, all in LDS and these lanes' own; PER * LANES >= routed, LANES >= top.  The
+// wave's lanes come here together; without `live` nothing leaves.
+struct RouteRule {
+  const float* correction;
+  int* experts;
+  float *weights, *shared_gate;
+  int routed, top, score, renormalize, groups, keep_groups;
+  float weight_scale;
+};
+template <int PER, int LANES>
+__device__ __forceinline__ void route_token(int t, bool live, float* z, float* group_best, int* group_open, const RouteRule& a) {
+  const int lane = threadIdx.x & (LANES - 1);
+  const int routed = a.routed, top = a.top, groups = a.groups, keep_groups = a.keep_groups;
+  const float* correction = a.correction;
+  if (a.shared_gate != nullptr && lane == 0 && live) a.shared_gate[t] = 1.f / (1.f + expf(-z[routed]));
+  float s[PER], choice[PER];
+  if (a.score == VLA_SCORE_SIGMOID) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int n = lane + i * LANES;
+      s[i] = n < routed ? 1.f / (1.f + expf(-z[n])) : 0.f;
+    }
+  } else {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int n = lane + i * LANES;
+      s[i] = n < routed ? z[n] : -INFINITY;
+      mx = fmaxf(mx, s[i]);
+    }
+  #pragma unroll
+    for (int m = LANES / 2; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      s[i] = lane + i * LANES < routed ? expf(s[i] - mx) : 0.f;
+      sum += s[i];
+    }
+  #pragma unroll
+    for (int m = LANES / 2; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) s[i] /= sum;
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int n = lane + i * LANES;
+    choice[i] = n < routed ? s[i] + (correction != nullptr ? correction[n] : 0.f) : -INFINITY;
+  }
+  if (keep_groups < groups) {
+    // a group's score is its best choice; only experts of the keep_groups best groups stay
+    const int size = routed / groups;
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (lane + i * LANES < routed) z[lane + i * LANES] = choice[i];
+    wave_sync();
+    for (int g = lane; g < groups; g += LANES) {
+      float best = -INFINITY;
+      for (int n = 0; n < size; ++n) best = fmaxf(best, z[g * size + n]);
+      group_best[g] = best;
+    }
+    wave_sync();
+    for (int g = lane; g < groups; g += LANES) {
+      int ahead = 0;                 // groups that go first: better ones, and equal ones with a lower index
+      for (int o = 0; o < groups; ++o)
+        ahead += group_best[o] > group_best[g] || (group_best[o] == group_best[g] && o < g) ? 1 : 0;
+      group_open[g] = ahead < keep_groups;
+    }
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int n = lane + i * LANES;
+      if (n < routed && !group_open[n / size]) choice[i] = -INFINITY;
+    }
+  }
+  float total = 0.f, mine = 0.f;     // lane k keeps the k-th chosen score
+  int mine_e = 0;
+  for (int k = 0; k < top; ++k) {
+    float best = -INFINITY, best_s = 0.f;
+    int best_n = 0x7fffffff;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int n = lane + i * LANES;
+      if (choice[i] > best) {      // ascending n within a lane: the lowest index wins a tie
+        best = choice[i];
+        best_n = n;
+        best_s = s[i];
+      }
+    }
+#pragma unroll
+    for (int m = LANES / 2; m >= 1; m >>= 1) {
+      const float ob = __shfl_xor(best, m, 64), os = __shfl_xor(best_s, m, 64);
+      const int on = __shfl_xor(best_n, m, 64);
+      if (ob > best || (ob == best && on < best_n)) {
+        best = ob;
+        best_n = on;
+        best_s = os;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (lane + i * LANES == best_n) choice[i] = -INFINITY;
+    total += best_s;
+    if (lane == k) {
+      mine = best_s;
+      mine_e = best_n;
+    }
+  }
+  if (lane < top && live) {
+    a.experts[(int64_t)t * top + lane] = mine_e;
+    a.weights[(int64_t)t * top + lane] = (a.renormalize ? mine / (total + 1e-20f) : mine) * a.weight_scale;
+  }
+}
+
 // One workgroup per token.  The logits come from the caller (a matrix product over many tokens) or
 // are formed here, a router row per wave at a time.
 template <class S>
 __global__ __launch_bounds__(256) void moe_route_kernel(
     const typename S::T* __restrict__ h, int64_t h_stride, const float* __restrict__ router,
     const float* __restrict__ logits, int64_t logits_stride, const float* __restrict__ bias,
-    const float* __restrict__ correction,
-    const float* __restrict__ shared_gate_w, int* __restrict__ experts, float* __restrict__ weights,
-    float* __restrict__ shared_gate, int width, int routed, int top, int score, int renormalize,
-    int groups, int keep_groups, float weight_scale, bool vec) {
+    const float* __restrict__ shared_gate_w, int width, RouteRule rule, bool vec) {
   __shared__ float z[kMaxRouted + 1];
   __shared__ float group_best[kMaxRouted];
   __shared__ int group_open[kMaxRouted];
   const int t = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const bool gated = shared_gate != nullptr;
+  const bool gated = rule.shared_gate != nullptr;
+  const int routed = rule.routed;
   const int rows = routed + (gated ? 1 : 0);
   if (logits != nullptr) {
     for (int n = threadIdx.x; n < rows; n += 256)
@@ -90,103 +203,81 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
     }
   }
   __syncthreads();
-  if (w != 0) return;
-  if (gated && lane == 0) shared_gate[t] = 1.f / (1.f + expf(-z[routed]));
-  constexpr int PER = kMaxRouted / kWave;
-  float s[PER], choice[PER];
-  if (score == VLA_SCORE_SIGMOID) {
+  if (w == 0) route_token<kMaxRouted / kWave, kWave>(t, true, z, group_best, group_open, rule);
+}
+
+// The logits of 16 tokens and the choice, for up to 16 NT router rows (the shared gate's among them): 16x16x4 fp32 MFMAs,
+// the eight waves of a workgroup take every eighth stretch of 32 of the contraction, add up through LDS, and choose for
+// two tokens each.  4096 tokens of 2048, 16 experts: 13 us (rows as fp32, a library product and the
+// choice: 33); 64 tokens 11 (a workgroup per token: 12).
+constexpr int kTileRouted = 64;
+template <class S, int NT>
+__global__ __launch_bounds__(512) void moe_route_tile_kernel(const typename S::T* __restrict__ h, int64_t h_stride,
+                                                             const float* __restrict__ router, const float* __restrict__ bias,
+                                                             const float* __restrict__ shared_gate_w, int num_tokens, int width,
+                                                             RouteRule rule) {
+  constexpr int N = 16 * NT, PITCH = N + 1;
+  __shared__ float part[8][16][PITCH];
+  __shared__ float group_best[16][N];
+  __shared__ int group_open[16][N];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
+  const int t0 = 16 * blockIdx.x;
+  const int rows = rule.routed + (rule.shared_gate != nullptr ? 1 : 0);
+  const typename S::T* hr = h + (int64_t)min(t0 + c, num_tokens - 1) * h_stride + 8 * g;
+  const float* wr[NT];
+  f32x4 acc[NT];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int n = lane + i * kWave;
-      s[i] = n < routed ? 1.f / (1.f + expf(-z[n])) : 0.f;
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = 16 * nt + c;
+    wr[nt] = (n == rule.routed && rows > n ? shared_gate_w : router + (int64_t)min(n, rule.routed - 1) * width) + 8 * g;
+    acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll 8 / NT
+  for (int k = 32 * w; k < width; k += 256) {
+    float x[8];
+    if constexpr (sizeof(typename S::T) == 2) {
+      const u32x4 hv = *reinterpret_cast<const u32x4*>(hr + k);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[2 * e] = lo16<S>(hv[e]);
+        x[2 * e + 1] = hi16<S>(hv[e]);
+      }
+    } else {
+      const f32x4 h0 = *reinterpret_cast<const f32x4*>(hr + k), h1 = *reinterpret_cast<const f32x4*>(hr + k + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = h0[e], x[4 + e] = h1[e];
     }
+    f32x4 wv[NT][2];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      wv[nt][0] = *reinterpret_cast<const f32x4*>(wr[nt] + k);
+      wv[nt][1] = *reinterpret_cast<const f32x4*>(wr[nt] + k + 4);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma4(x[e], wv[nt][e >> 2][e & 3], acc[nt]);
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part[w][4 * g + i][16 * nt + c] = acc[nt][i];
+  __syncthreads();
+  for (int i = tid; i < 16 * N; i += 512) {
+    const int t = i / N, n = i % N;
+    float z = 0.f;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) z += part[o][t][n];
+    if (n < rows) part[0][t][n] = z + (bias != nullptr && n < rule.routed ? bias[n] : 0.f);
+  }
+  __syncthreads();
+  if constexpr (NT <= 2) {                                 // half a wave a token
+    const int t = 2 * w + (lane >> 5);
+    route_token<1, 32>(t0 + t, t0 + t < num_tokens, part[0][t], group_best[t], group_open[t], rule);
   } else {
-    float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int n = lane + i * kWave;
-      s[i] = n < routed ? z[n] : -INFINITY;
-      mx = fmaxf(mx, s[i]);
-    }
-    mx = wave_max(mx);
-    float sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      s[i] = lane + i * kWave < routed ? expf(s[i] - mx) : 0.f;
-      sum += s[i];
-    }
-    sum = wave_sum(sum);
-#pragma unroll
-    for (int i = 0; i < PER; ++i) s[i] /= sum;
-  }
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int n = lane + i * kWave;
-    choice[i] = n < routed ? s[i] + (correction != nullptr ? correction[n] : 0.f) : -INFINITY;
-  }
-  if (keep_groups < groups) {
-    // a group's score is its best choice; only experts of the keep_groups best groups stay
-    const int size = routed / groups;
-    wave_sync();
-#pragma unroll
-    for (int i = 0; i < PER; ++i)
-      if (lane + i * kWave < routed) z[lane + i * kWave] = choice[i];
-    wave_sync();
-    for (int g = lane; g < groups; g += kWave) {
-      float best = -INFINITY;
-      for (int n = 0; n < size; ++n) best = fmaxf(best, z[g * size + n]);
-      group_best[g] = best;
-    }
-    wave_sync();
-    for (int g = lane; g < groups; g += kWave) {
-      int ahead = 0;                 // groups that go first: better ones, and equal ones with a lower index
-      for (int o = 0; o < groups; ++o)
-        ahead += group_best[o] > group_best[g] || (group_best[o] == group_best[g] && o < g) ? 1 : 0;
-      group_open[g] = ahead < keep_groups;
-    }
-    wave_sync();
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int n = lane + i * kWave;
-      if (n < routed && !group_open[n / size]) choice[i] = -INFINITY;
-    }
-  }
-  float total = 0.f, mine = 0.f;     // lane k keeps the k-th chosen score
-  int mine_e = 0;
-  for (int k = 0; k < top; ++k) {
-    float best = -INFINITY, best_s = 0.f;
-    int best_n = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int n = lane + i * kWave;
-      if (choice[i] > best) {      // ascending n within a lane: the lowest index wins a tie
-        best = choice[i];
-        best_n = n;
-        best_s = s[i];
-      }
-    }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-      const float ob = __shfl_xor(best, m, 64), os = __shfl_xor(best_s, m, 64);
-      const int on = __shfl_xor(best_n, m, 64);
-      if (ob > best || (ob == best && on < best_n)) {
-        best = ob;
-        best_n = on;
-        best_s = os;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < PER; ++i)
-      if (lane + i * kWave == best_n) choice[i] = -INFINITY;
-    total += best_s;
-    if (lane == k) {
-      mine = best_s;
-      mine_e = best_n;
-    }
-  }
-  if (lane < top) {
-    experts[(int64_t)t * top + lane] = mine_e;
-    weights[(int64_t)t * top + lane] = (renormalize ? mine / (total + 1e-20f) : mine) * weight_scale;
+    for (int t = 2 * w; t < 2 * w + 2; ++t)
+      route_token<1, 64>(t0 + t, t0 + t < num_tokens, part[0][t], group_best[t], group_open[t], rule);
   }
 }
 
@@ -1064,6 +1155,39 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
   }
 }
 
+// The same four columns at a time, a workgroup 1024 of a token's (out, y and shared_y in 16-byte pieces): 4096 tokens,
+// top 2, 2048 wide 17 us (25 one column at a time), 64 tokens 3 (8).
+template <class S>
+__global__ __launch_bounds__(256) void moe_combine_vec_kernel(
+    float* __restrict__ out, const float* __restrict__ y, const int* __restrict__ pair_row,
+    const float* __restrict__ weights, const typename S::T* __restrict__ h, int64_t h_stride,
+    const float* __restrict__ shared_y, const float* __restrict__ shared_gate, int width, int top) {
+  const int64_t t = blockIdx.x;
+  const int c = 4 * (blockIdx.y * 256 + threadIdx.x);
+  if (c >= width) return;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int k = 0; k < top; ++k) {
+    const int row = pair_row[t * top + k];
+    const float by = weights != nullptr ? weights[t * top + k] : 1.f;
+    f32x4 v;
+    if (row >= 0)
+      v = *reinterpret_cast<const f32x4*>(y + (int64_t)row * width + c);
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = S::to_f32(h[t * h_stride + c + e]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += by * v[e];
+  }
+  if (shared_y != nullptr) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(shared_y + t * width + c);
+    const float by = shared_gate != nullptr ? shared_gate[t] : 1.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += by * v[e];
+  }
+  *reinterpret_cast<f32x4*>(out + t * width + c) = acc;
+}
+
 template <class F>
 int with_io_dtypes(int a, int b, F&& f) {
   return with_dtype(a, [&](auto sa) { return with_dtype(b, [&](auto sb) { return f(sa, sb); }); });
@@ -1095,12 +1219,26 @@ extern "C" int vla_seq_moe_route(const void* h, int64_t h_stride, const float* r
   const int size = dtype == VLA_F32 ? 4 : 2;
   const bool vec = !logits && width % 8 == 0 && (uintptr_t)h % (8 * size) == 0 && h_stride % 8 == 0 &&
                    (uintptr_t)router % 16 == 0 && (uintptr_t)shared_gate_weight % 16 == 0;
+  const RouteRule rule{correction, experts, weights, shared_gate, routed, top, score, renormalize, groups, keep_groups,
+                       weight_scale};
+  const int rows = routed + (gated ? 1 : 0);
   return with_dtype(dtype, [&](auto s) {
     using S = decltype(s);
-    moe_route_kernel<S><<<num_tokens, 256, 0, (hipStream_t)stream>>>(
-        (const typename S::T*)h, h_stride, router, logits, logits_stride, bias, correction,
-        shared_gate_weight, experts, weights, shared_gate, width, routed, top, score, renormalize, groups,
-        keep_groups, weight_scale, vec);
+    if (vec && width % 32 == 0 && rows <= kTileRouted) {
+      auto go = [&](auto nt) {
+        moe_route_tile_kernel<S, decltype(nt)::value><<<(num_tokens + 15) / 16, 512, 0, (hipStream_t)stream>>>(
+            (const typename S::T*)h, h_stride, router, bias, shared_gate_weight, num_tokens, width, rule);
+      };
+      if (rows <= 16)
+        go(std::integral_constant<int, 1>());
+      else if (rows <= 32)
+        go(std::integral_constant<int, 2>());
+      else
+        go(std::integral_constant<int, 4>());
+    } else {
+      moe_route_kernel<S><<<num_tokens, 256, 0, (hipStream_t)stream>>>((const typename S::T*)h, h_stride, router, logits,
+                                                                       logits_stride, bias, shared_gate_weight, width, rule, vec);
+    }
     VLA_SEQ_HIP_CHECK(hipGetLastError());
     return VLA_OK;
   });
@@ -1230,9 +1368,12 @@ extern "C" int vla_seq_moe_combine(float* out, const float* y, const int* pair_r
     return VLA_ERR_ARG;
   return with_dtype(dtype, [&](auto s) {
     using S = decltype(s);
-    moe_combine_kernel<S><<<num_tokens, 256, 0, (hipStream_t)stream>>>(
-        out, y, pair_row, weights, (const typename S::T*)h, h_stride, shared_y, shared_gate, width,
-        top);
+    if (width % 4 == 0 && ((uintptr_t)out | (uintptr_t)y | (uintptr_t)shared_y) % 16 == 0)
+      moe_combine_vec_kernel<S><<<dim3(num_tokens, (width + 1023) / 1024), 256, 0, (hipStream_t)stream>>>(
+          out, y, pair_row, weights, (const typename S::T*)h, h_stride, shared_y, shared_gate, width, top);
+    else
+      moe_combine_kernel<S><<<num_tokens, 256, 0, (hipStream_t)stream>>>(
+          out, y, pair_row, weights, (const typename S::T*)h, h_stride, shared_y, shared_gate, width, top);
     VLA_SEQ_HIP_CHECK(hipGetLastError());
     return VLA_OK;
   });

@@ -14,7 +14,7 @@ optional shared expert runs for every token: plain, multiplied by sigmoid(w_sg .
 (`shared_gated`) of the gated form with a limit of its own and nothing in front.  The output is
 fp32 (the caller norms it and adds it to its stream).
 
-Execution (csrc/seq_moe_kernels.hip): route (the logits of a large step come from one fp32 matrix
+Execution (csrc/seq_moe_kernels.hip): route (the logits of a large step of many experts come from one fp32 matrix
 product) -> plan (pairs grouped by expert into row tiles) ->
 grouped up-projection with the activation fused (rows gathered from the tokens) -> grouped
 down-projection in fp32 -> combine (weighted sum per token in the order of its choices, identity
@@ -36,8 +36,8 @@ def mm_f32(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 class RoutedExperts(nn.Module):
-    # steps with at least this many tokens form the router logits as one matrix product; below,
-    # the routing kernel forms them itself (one launch)
+    # steps with at least this many tokens form the router logits as one matrix product where the routing kernel
+    # has no form for many tokens; below, it forms them itself (one launch)
     ROUTE_PRODUCT_MIN_TOKENS = 256
 
     def __init__(self, width: int, num_experts: int, num_identity: int, top: int, expert_ff: int,
@@ -140,11 +140,11 @@ class RoutedExperts(nn.Module):
         and no identity expert."""
         T = h.shape[0]
         logits = None
-        if T >= self.ROUTE_PRODUCT_MIN_TOKENS:
+        sg_w = None if self.shared_gate is None else self.shared_gate.data
+        if T >= self.ROUTE_PRODUCT_MIN_TOKENS and not ops.moe_route_forms_logits(h, self.router.data, sg_w):
             # many tokens: the router rows (and the shared gate's) as one fp32 matrix product
             logits = torch.mm(h if h.dtype == torch.float32 else h.float(), self.router_rows().t())
-        experts, weights, sg = ops.moe_route(h, self.router.data, self.correction.data,
-                                             None if self.shared_gate is None else self.shared_gate.data, self.top, logits,
+        experts, weights, sg = ops.moe_route(h, self.router.data, self.correction.data, sg_w, self.top, logits,
                                              None if self.router_bias is None else self.router_bias.data,
                                              self.score, self.renormalize, self.groups, self.keep_groups,
                                              self.weight_scale)
