@@ -652,6 +652,18 @@ int vla_seq_latent_decode(void* out, int64_t out_token_stride, int64_t out_head_
                           const int* context_lens, int num_seqs, int heads, int rank, int rot, int block_size,
                           int num_blocks, float scale, int ranges, float* scratch, int64_t scratch_floats, int dtype,
                           int window, const void* gate, int64_t gate_stride, const float* sinks, void* stream);
+/* The same and the heads' up-projection: up[t][h vdim + n] = sum_d out[t, h, d] w[h][d][n], w [heads, rank, vdim] and up
+ * 4-byte aligned, vdim 32, 64, 128 or 256 (vla_seq_latent_decode_up_supported).  out is room for [.., rank] rows whose
+ * contents are not defined afterwards. */
+int vla_seq_latent_decode_up_supported(int vdim);
+int vla_seq_latent_decode_up(void* out, int64_t out_token_stride, int64_t out_head_stride, const void* q_lat,
+                          int64_t lat_token_stride, int64_t lat_head_stride, const void* q_rot,
+                          int64_t rot_token_stride, int64_t rot_head_stride, const void* cache,
+                          const int* block_tables, int max_blocks, const int* query_start_loc,
+                          const int* context_lens, int num_seqs, int heads, int rank, int rot, int block_size,
+                          int num_blocks, float scale, int ranges, float* scratch, int64_t scratch_floats, int dtype,
+                          int window, const void* gate, int64_t gate_stride, const float* sinks, void* stream, const void* w, void* up,
+                             int64_t up_stride, int vdim);
 
 /* Kernel choice for tests: window attention 0 = per shape, 1 = one wave per (row, head);
  * scan 0 = per shape, 1 = token by token. */

@@ -123,3 +123,27 @@ def test_layers_take_it():
     want, got = reference(c), run(c)
     error = [float((t.to(F) - want).norm() / want.norm()) for t in (tiles, got)]
     assert error[1] <= 1.1 * error[0], error
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rank,vdim,heads", [(512, 128, 16), (256, 32, 3), (512, 256, 2), (256, 64, 17)])
+@pytest.mark.parametrize("lens", [[1], [5000], [15, 1, 700], [3000] + [1 + 13 * i % 190 for i in range(15)], [40] * 17, [900] * 33],
+                         ids=lambda x: f"{len(x)}x{max(x)}")
+def test_up_projection(lens, rank, vdim, heads, dtype):
+    """The heads' up-projection in the merge: of the rounded sums, rounded once more."""
+    from vllm_legacy_amd import _seq_ops as ops
+    c = case(lens, heads, rank, 64, 16, dtype)
+    gate = torch.randn(len(lens), heads, device=DEV).to(dtype)
+    w = (torch.randn(heads, rank, vdim, device=DEV) * rank**-0.5).to(dtype)
+    up = torch.full((len(lens), heads * vdim), float("nan"), dtype=dtype, device=DEV)
+    out = torch.empty_like(c["q_lat"])
+    assert ops.latent_decode_up_supported(w)
+    ops.latent_decode(out, c["q_lat"], c["q_rot"], c["cache"], c["tables"], c["starts"], c["ctx"], max(lens), c["scale"], 0,
+                      gate, None, up, w)
+    o = reference(c, gate)
+    want = torch.matmul(o.transpose(0, 1), w.to(F)).transpose(0, 1).reshape(len(lens), -1)
+    check(up, want, dtype)
+    alone = run(c, gate, max_keys=max(lens)).to(F)         # and of what the merge leaves
+    near = torch.matmul(alone.transpose(0, 1), w.to(F)).transpose(0, 1).reshape(len(lens), -1)
+    bound = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    assert float((up.to(F) - near).abs().max()) <= bound * float(near.abs().max()) + 1e-5

@@ -68,6 +68,7 @@ SEQ_EXPORTS = [
     "vla_seq_latent_rotary_write", "vla_seq_latent_attention", "vla_seq_latent_attention_tiles",
     "vla_seq_latent_attention_tiles_supported", "vla_seq_latent_attention_scratch_floats", "vla_seq_set_latent_attention_kernel",
     "vla_seq_latent_decode", "vla_seq_latent_decode_supported", "vla_seq_latent_decode_ranges", "vla_seq_latent_decode_scratch_floats",
+    "vla_seq_latent_decode_up", "vla_seq_latent_decode_up_supported",
     "vla_seq_clamped_glu", "vla_seq_pair_hash_embed",
     "vla_seq_decay_scan", "vla_seq_decay_scan_scratch_floats", "vla_seq_set_decay_scan_kernel",
     "vla_seq_gated_group_rms_norm", "vla_seq_set_short_conv_kernel", "vla_seq_matrix_memory_gates",
@@ -179,12 +180,14 @@ def seq_lib():
         L.vla_seq_latent_attention_scratch_floats.argtypes = [i, i, i, i]
         L.vla_seq_latent_attention_scratch_floats.restype = i64
         L.vla_seq_set_latent_attention_kernel.argtypes = [i]
+        L.vla_seq_latent_decode_up_supported.argtypes = [i]
         L.vla_seq_latent_decode_supported.argtypes = [i, i, i]
         L.vla_seq_latent_decode_ranges.argtypes = [i, i, i]
         L.vla_seq_latent_decode_scratch_floats.argtypes = [i, i, i]
         L.vla_seq_latent_decode_scratch_floats.restype = i64
         L.vla_seq_latent_decode.argtypes = [p, i64, i64, p, i64, i64, p, i64, i64, p, p, i, p, p, i, i, i, i, i, i, f,
                                             i, p, i64, i, i, p, i64, p, p]
+        L.vla_seq_latent_decode_up.argtypes = L.vla_seq_latent_decode.argtypes + [p, p, i64, i]
         L.vla_seq_decay_scan.argtypes = [p, p, i64, p, i64, p, i64, p, i64, p, p, p, p, p, p, p, p, f, f, p, p, p, p,
                                          i, i, i, i, i, i, i, i, i, p, i64, i, p]
         L.vla_seq_decay_scan_scratch_floats.argtypes = [i, i, i, i, i, i, i]

@@ -1144,13 +1144,20 @@ def latent_decode_supported(out: torch.Tensor, q_lat: torch.Tensor, q_rot: torch
             all(out.stride(d) % 4 == 0 or out.shape[d] == 1 for d in (0, 1)))
 
 
+def latent_decode_up_supported(w_up: torch.Tensor) -> bool:
+    """Whether latent_decode takes these up-projections [H, rank, vdim] too."""
+    return w_up.is_contiguous() and bool(_lib.seq_lib().vla_seq_latent_decode_up_supported(w_up.shape[2]))
+
+
 def latent_decode(out: torch.Tensor, q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch.Tensor,
                   block_tables: torch.Tensor, query_start_loc: torch.Tensor, context_lens: torch.Tensor, max_keys: int,
                   scale: float, window: int = 0, gate: Optional[torch.Tensor] = None,
-                  sinks: Optional[torch.Tensor] = None) -> None:
+                  sinks: Optional[torch.Tensor] = None, up: Optional[torch.Tensor] = None,
+                  w_up: Optional[torch.Tensor] = None) -> None:
     """latent_attention_tiles for a step of single rows: the keys of all sequences are shared out evenly.  max_keys:
-    about the most that a row sees (decides how many workgroups there are, not what they do)."""
-    _gpu(out, q_lat, q_rot, cache, block_tables, query_start_loc, context_lens, gate, sinks)
+    about the most that a row sees (decides how many workgroups there are, not what they do).  With up [T, H vdim] and
+    w_up [H, rank, vdim] also up = out w_up head by head (latent_decode_up_supported); out is scratch then."""
+    _gpu(out, q_lat, q_rot, cache, block_tables, query_start_loc, context_lens, gate, sinks, up, w_up)
     NB, BS, width = cache.shape
     T, H, rank = q_lat.shape
     rot = width - rank
@@ -1168,17 +1175,25 @@ def latent_decode(out: torch.Tensor, q_lat: torch.Tensor, q_rot: torch.Tensor, c
     def st(t, d):       # a stride that is never used may be anything
         return t.stride(d) if t.shape[d] > 1 else 0
 
+    if up is not None:
+        assert w_up.shape[:2] == (H, rank) and w_up.is_contiguous() and up.shape == (T, H * w_up.shape[2]) and up.is_contiguous()
+        assert up.dtype == w_up.dtype == q_lat.dtype
     L = _lib.seq_lib()
     ranges = L.vla_seq_latent_decode_ranges(B, int(max_keys), H)
     need = L.vla_seq_latent_decode_scratch_floats(ranges, H, rank)
     scratch = torch.empty(need, dtype=torch.float32, device=q_lat.device) if need else None
     with torch.cuda.device(q_lat.device):
-        seq_check(L.vla_seq_latent_decode(
+        args = (
             out.data_ptr(), st(out, 0), st(out, 1), q_lat.data_ptr(), st(q_lat, 0), st(q_lat, 1), q_rot.data_ptr(),
             st(q_rot, 0), st(q_rot, 1), cache.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
             query_start_loc.data_ptr(), context_lens.data_ptr(), B, H, rank, rot, BS, NB, float(scale), ranges,
             _p(scratch), need, _dt(q_lat.dtype), int(window), _p(gate), 0 if gate is None else _rows(gate, H),
-            _p(sinks), _stream(q_lat.device)), "latent_decode")
+            _p(sinks), _stream(q_lat.device))
+        if up is None:
+            seq_check(L.vla_seq_latent_decode(*args), "latent_decode")
+        else:
+            seq_check(L.vla_seq_latent_decode_up(*args, w_up.data_ptr(), up.data_ptr(), up.stride(0), w_up.shape[2]),
+                      "latent_decode_up")
 
 
 def latent_prompt_supported(q: torch.Tensor, dim: int, rot: int, vdim: int, rank: int, cache: torch.Tensor) -> bool:

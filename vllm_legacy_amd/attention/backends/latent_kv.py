@@ -240,8 +240,13 @@ class LatentKVAttention(nn.Module):
             # 16-bit models whose sizes fit: (token, head) rows in tiles of 32 on the matrix cores
             if part is None and batch.max_query_len == 1 and ops.latent_decode_supported(o_rows, q_lat, q_rot, cache):
                 keys = min(batch.max_seq_len, self.window or batch.max_seq_len)
+                w_uv = self.w_uv_t.data
+                out = torch.empty((T, H * self.value_dim), dtype=q.dtype, device=q.device) \
+                    if ops.latent_decode_up_supported(w_uv) else None
                 ops.latent_decode(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.query_start_loc,
-                                  batch.context_lens, keys, self.scale, self.window, gate, sinks)
+                                  batch.context_lens, keys, self.scale, self.window, gate, sinks, out, w_uv)
+                if out is not None:
+                    return out
             elif part is None:
                 ops.latent_attention_tiles(o_rows, q_lat, q_rot, cache, batch.block_tables, batch.query_start_loc,
                                            batch.context_lens, batch.max_query_len, self.scale, self.key_splits(batch),

@@ -10,7 +10,7 @@
 //   * The keys of all sequences are one line of tiles that the workgroups share out evenly, whatever
 //     the lengths: a range may end inside a sequence and go on in the next.  The lengths are read on the
 //     device, so a captured step may be replayed with others.  A part of a sequence leaves its sums in scratch for
-//     latent_decode_merge_kernel; a sequence that lies within one range is written out at once.
+//     latent_decode_merge_kernel or latent_decode_up_kernel; one that lies within a range is written out at once.
 // Products on 16x16 MFMAs, lane = (g, c) = (lane >> 4, lane & 15), 16 heads to a workgroup:
 //   S^T = K q^T    A = K    lane: key c, dims 32 ks + 8 g .. + 7     (LDS, 16 bytes)
 //                  B = q^T  lane: head c, the same dims              (registers, loaded once a sequence)
@@ -364,15 +364,11 @@ __global__ __launch_bounds__(128 * HS, 2) void latent_decode_kernel(LatentDecode
   }
 }
 
-// out[t, h, d] = sum_s o_s[d] 2^(m_s - M) / sum_s l_s 2^(m_s - M) over the ranges s that a sequence lies in, M the
-// largest m_s.  rank / 4 threads to a head; a sequence that lies within one range is written out already.
-template <class S>
-__global__ __launch_bounds__(128) void latent_decode_merge_kernel(LatentDecode a) {
-  using T = typename S::T;
-  const int lane = threadIdx.x & 63, b = blockIdx.x, row_floats = a.rank + 4;
-  const int per = a.rank / 4, h = blockIdx.y * (128 / per) + threadIdx.x / per, d = 4 * (threadIdx.x % per);
-  int total = 0, start = 0;
-  for (int i = lane; i < a.num_seqs; i += 64) {
+// The first unit of sequence b in the line of all, and a range's share; the same in every lane, which all come here.
+__device__ __forceinline__ void place_of(const LatentDecode& a, int b, int& start, int& share) {
+  int total = 0;
+  start = 0;
+  for (int i = threadIdx.x & 63; i < a.num_seqs; i += 64) {
     const int n = units_of(a, i);
     total += n;
     if (i < b) start += n;
@@ -382,11 +378,14 @@ __global__ __launch_bounds__(128) void latent_decode_merge_kernel(LatentDecode a
     total += __shfl_xor(total, x, 64);
     start += __shfl_xor(start, x, 64);
   }
-  const int units = units_of(a, b), share = share_of(a, total);
-  if (units == 0) return;
-  const int i0 = start / share, i1 = (start + units - 1) / share;
-  if (i0 == i1 || h >= a.heads) return;
-  const int64_t t = a.query_start_loc[b];
+  share = share_of(a, total);
+}
+
+// sum_s o_s[d] 2^(m_s - M) over the ranges s = i0 .. i1, M the largest m_s, of four sums from d + 256 j on each; the
+// result is sum_s l_s 2^(m_s - M)
+template <int NJ>
+__device__ __forceinline__ float merge_parts(const LatentDecode& a, int h, int i0, int i1, int d, f32x4 (&num)[NJ]) {
+  const int lane = threadIdx.x & 63, row_floats = a.rank + 4;
   auto part = [&](int s) {
     const int slot = s == i0 ? 2 * s + 1 : 2 * s;        // its first part is the last of that range
     return a.parts + ((int64_t)slot * a.heads + h) * row_floats;
@@ -394,8 +393,9 @@ __global__ __launch_bounds__(128) void latent_decode_merge_kernel(LatentDecode a
   float big = -INFINITY;
   for (int s = i0 + lane; s <= i1; s += 64) big = fmaxf(big, part(s)[a.rank]);
   big = wave_max(big);
-  f32x4 num = {0.f, 0.f, 0.f, 0.f};
   float den = 0.f;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) num[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int s0 = i0; s0 <= i1; s0 += 64) {
     float f = 0.f, lf = 0.f;
     if (s0 + lane <= i1) {
@@ -405,21 +405,137 @@ __global__ __launch_bounds__(128) void latent_decode_merge_kernel(LatentDecode a
     }
     den += wave_sum(lf);
     const int n = min(64, i1 - s0 + 1);
-    for (int s8 = 0; s8 < n; s8 += 8) {              // eight loads on their way
-      f32x4 v[8];
+    constexpr int AHEAD = 8;
+    for (int s8 = 0; s8 < n; s8 += AHEAD) {              // eight parts on their way
+      f32x4 v[AHEAD][NJ];
 #pragma unroll
-      for (int s = 0; s < 8; ++s) v[s] = *reinterpret_cast<const f32x4*>(part(s0 + min(s8 + s, n - 1)) + d);
+      for (int s = 0; s < AHEAD; ++s)
 #pragma unroll
-      for (int s = 0; s < 8; ++s) {
+        for (int j = 0; j < NJ; ++j) v[s][j] = *reinterpret_cast<const f32x4*>(part(s0 + min(s8 + s, n - 1)) + d + 256 * j);
+#pragma unroll
+      for (int s = 0; s < AHEAD; ++s) {
         const float fs = s8 + s < n ? __shfl(f, s8 + s, 64) : 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) num[e] = s8 + s < n ? num[e] + v[s][e] * fs : num[e];
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) num[j][e] = s8 + s < n ? num[j][e] + v[s][j][e] * fs : num[j][e];
       }
     }
   }
-  const float gv = a.gate != nullptr ? 1.f / (1.f + expf(-S::to_f32(((const T*)a.gate)[t * a.gate_stride + h]))) : 1.f;
-  const u32x2 packed = {pack16<S>(num[0] / den * gv, num[1] / den * gv), pack16<S>(num[2] / den * gv, num[3] / den * gv)};
+  return den;
+}
+template <class S>
+__device__ __forceinline__ float gate_of(const LatentDecode& a, int64_t t, int h) {
+  return a.gate != nullptr ? 1.f / (1.f + expf(-S::to_f32(((const typename S::T*)a.gate)[t * a.gate_stride + h]))) : 1.f;
+}
+
+// out[t, h, d] = the merged sums over the merged weights, times the gate.  rank / 4 threads to a head; a sequence that
+// lies within one range is written out already.
+template <class S>
+__global__ __launch_bounds__(128) void latent_decode_merge_kernel(LatentDecode a) {
+  using T = typename S::T;
+  const int b = blockIdx.x, per = a.rank / 4, h = blockIdx.y * (128 / per) + threadIdx.x / per, d = 4 * (threadIdx.x % per);
+  int start, share;
+  place_of(a, b, start, share);
+  const int units = units_of(a, b), i0 = start / share, i1 = (start + units - 1) / share;
+  if (units == 0 || i0 == i1 || h >= a.heads) return;
+  const int64_t t = a.query_start_loc[b];
+  f32x4 num[1];
+  const float den = merge_parts<1>(a, h, i0, i1, d, num);
+  const float gv = gate_of<S>(a, t, h);
+  const u32x2 packed = {pack16<S>(num[0][0] / den * gv, num[0][1] / den * gv), pack16<S>(num[0][2] / den * gv, num[0][3] / den * gv)};
   *reinterpret_cast<u32x2*>((T*)a.out + t * a.out_token_stride + h * a.out_head_stride + d) = packed;
+}
+
+// The merge and the heads' up-projection in one: up[t, h vdim + n] = sum_d o[t, h, d] w[h, d, n], o rounded to 16 bits as
+// the merge leaves it.  A workgroup is 16 sequences and a head: a wave merges a row (or reads one that is written out
+// already) into LDS, then takes 32 columns and a part of the latent dims.  The weights' rows run along n, where the
+// matrix cores want them along d: a lane loads two columns of eight rows and puts the words together itself.  64
+// sequences of 1 .. 4001 keys, 16 heads, rank 512, vdim 128: 12 us, where the merge, a batched library product and
+// the copy that puts a token's heads side by side took 6, 10 and 4.
+struct LatentUp {
+  void* up;
+  int64_t up_stride;
+  const void* w;                       // [heads, rank, vdim]
+  int vdim;
+};
+template <class S, int NJ>             // rank = 256 NJ
+__global__ __launch_bounds__(1024) void latent_decode_up_kernel(LatentDecode a, LatentUp u) {
+  using T = typename S::T;
+  constexpr int C = 256 * NJ, PITCH = C + 8;
+  __shared__ __align__(16) T o_lds[16 * PITCH];
+  __shared__ float part[16][16][34];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
+  const int b0 = 16 * blockIdx.x, h = blockIdx.y;
+  const int blocks = u.vdim / 32, split = min(16 / blocks, C / 32), nb = w % blocks, ks0 = min(w / blocks, split - 1) * (C / 32 / split);
+  const uint32_t* wr = reinterpret_cast<const uint32_t*>((const T*)u.w + ((int64_t)h * C + 32 * ks0 + 8 * g) * u.vdim + 32 * nb + 2 * c);
+  constexpr int AHEAD = 4;                               // steps whose weights are on their way during the merge
+  const int steps = C / 32 / split;
+  uint32_t x[AHEAD][8];
+#pragma unroll
+  for (int ks = 0; ks < AHEAD; ++ks)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[ks][j] = wr[(int64_t)(32 * min(ks, steps - 1) + j) * (u.vdim / 2)];
+  int start = 0, share = 1;
+  const bool parts = !a.by_sequence && a.ranges > 1;
+  if (parts) place_of(a, b0 + w, start, share);
+  {
+    const int row = w, b = b0 + row;
+    u32x2 packed[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) packed[j] = u32x2{0u, 0u};
+    if (b < a.num_seqs && a.query_start_loc[b + 1] > a.query_start_loc[b]) {
+      const int64_t t = a.query_start_loc[b];
+      const int units = units_of(a, b), i0 = start / share, i1 = (start + units - 1) / share;
+      if (parts && i0 != i1) {
+        f32x4 num[NJ];
+        const float den = merge_parts<NJ>(a, h, i0, i1, 4 * lane, num);
+        const float gv = gate_of<S>(a, t, h);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          packed[j] = u32x2{pack16<S>(num[j][0] / den * gv, num[j][1] / den * gv), pack16<S>(num[j][2] / den * gv, num[j][3] / den * gv)};
+      } else {
+        const T* from = (const T*)a.out + t * a.out_token_stride + h * a.out_head_stride + 4 * lane;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) packed[j] = *reinterpret_cast<const u32x2*>(from + 256 * j);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) *reinterpret_cast<u32x2*>(o_lds + row * PITCH + 256 * j + 4 * lane) = packed[j];
+  }
+  __syncthreads();
+  f32x4 even = {0.f, 0.f, 0.f, 0.f}, odd = {0.f, 0.f, 0.f, 0.f};
+  for (int k8 = 0; k8 < steps; k8 += AHEAD) {
+#pragma unroll
+    for (int ks = 0; ks < AHEAD; ++ks) {
+      if (k8 + ks >= steps) break;
+      const u32x4 ov = *reinterpret_cast<const u32x4*>(o_lds + c * PITCH + 32 * (ks0 + k8 + ks) + 8 * g);
+      u32x4 lo, hi;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        lo[j] = __builtin_amdgcn_perm(x[ks][2 * j + 1], x[ks][2 * j], 0x05040100);
+        hi[j] = __builtin_amdgcn_perm(x[ks][2 * j + 1], x[ks][2 * j], 0x07060302);
+      }
+      even = LdMma<S>::score(ov, lo, even);
+      odd = LdMma<S>::score(ov, hi, odd);
+    }
+    if (k8 + AHEAD < steps) {
+#pragma unroll
+      for (int ks = 0; ks < AHEAD; ++ks)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[ks][j] = wr[(int64_t)(32 * min(k8 + AHEAD + ks, steps - 1) + j) * (u.vdim / 2)];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) part[w][4 * g + i][2 * c] = even[i], part[w][4 * g + i][2 * c + 1] = odd[i];
+  __syncthreads();
+  for (int i = tid; i < 16 * u.vdim / 2; i += 1024) {
+    const int row = i / (u.vdim / 2), n = 2 * (i % (u.vdim / 2)), b = b0 + row;
+    if (b >= a.num_seqs || a.query_start_loc[b + 1] <= a.query_start_loc[b]) continue;
+    float v0 = 0.f, v1 = 0.f;
+    for (int s = 0; s < split; ++s) v0 += part[s * blocks + n / 32][row][n % 32], v1 += part[s * blocks + n / 32][row][n % 32 + 1];
+    *reinterpret_cast<uint32_t*>((T*)u.up + a.query_start_loc[b] * u.up_stride + (int64_t)h * u.vdim + n) = pack16<S>(v0, v1);
+  }
 }
 
 bool latent_decode_sizes(int rank, int rot) {
@@ -429,7 +545,7 @@ bool latent_decode_sizes(int rank, int rot) {
 int head_groups(int heads) { return heads <= 16 ? 1 : (heads + 31) / 32; }
 
 template <class S, int LB, int RB, int HS>
-int launch_latent_decode(const LatentDecode& a, hipStream_t stream) {
+int launch_latent_decode(const LatentDecode& a, const LatentUp* up, hipStream_t stream) {
   constexpr size_t lds = kLdRing * kLdUnit * 128 * (LB + RB) + kLdSlots * 4;
   static std::atomic<bool> allowed{false};         // raised once per kernel, not per launch
   if (lds > 64 * 1024 && !allowed.load(std::memory_order_relaxed)) {
@@ -439,7 +555,10 @@ int launch_latent_decode(const LatentDecode& a, hipStream_t stream) {
   }
   latent_decode_kernel<S, LB, RB, HS><<<dim3(a.ranges, head_groups(a.heads)), 128 * HS, lds, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
-  if (!a.by_sequence && a.ranges > 1) {
+  if (up != nullptr) {
+    latent_decode_up_kernel<S, LB / 4><<<dim3((a.num_seqs + 15) / 16, a.heads), 1024, 0, stream>>>(a, *up);
+    VLA_SEQ_HIP_CHECK(hipGetLastError());
+  } else if (!a.by_sequence && a.ranges > 1) {
     const int heads_per = 128 / (a.rank / 4);
     latent_decode_merge_kernel<S><<<dim3(a.num_seqs, (a.heads + heads_per - 1) / heads_per), 128, 0, stream>>>(a);
     VLA_SEQ_HIP_CHECK(hipGetLastError());
@@ -448,10 +567,10 @@ int launch_latent_decode(const LatentDecode& a, hipStream_t stream) {
 }
 
 template <class S>
-int latent_decode_go(const LatentDecode& a, int rot, hipStream_t stream) {
+int latent_decode_go(const LatentDecode& a, const LatentUp* up, int rot, hipStream_t stream) {
   const bool wide = a.rank == 512, turned = rot == 64;
   const bool two = a.heads > 16;
-#define VLA_LD(L, R) return two ? launch_latent_decode<S, L, R, 2>(a, stream) : launch_latent_decode<S, L, R, 1>(a, stream)
+#define VLA_LD(L, R) return two ? launch_latent_decode<S, L, R, 2>(a, up, stream) : launch_latent_decode<S, L, R, 1>(a, up, stream)
   if (wide && turned) VLA_LD(8, 1);
   if (wide) VLA_LD(8, 0);
   if (turned) VLA_LD(4, 1);
@@ -483,14 +602,15 @@ extern "C" int64_t vla_seq_latent_decode_scratch_floats(int ranges, int heads, i
   return ranges > 1 ? (int64_t)2 * ranges * heads * (rank + 4) : 0;
 }
 
-extern "C" int vla_seq_latent_decode(void* out, int64_t out_token_stride, int64_t out_head_stride, const void* q_lat,
-                                     int64_t lat_token_stride, int64_t lat_head_stride, const void* q_rot,
-                                     int64_t rot_token_stride, int64_t rot_head_stride, const void* cache,
-                                     const int* block_tables, int max_blocks, const int* query_start_loc,
-                                     const int* context_lens, int num_seqs, int heads, int rank, int rot,
-                                     int block_size, int num_blocks, float scale, int ranges, float* scratch,
-                                     int64_t scratch_floats, int dtype, int window, const void* gate,
-                                     int64_t gate_stride, const float* sinks, void* stream) {
+namespace {
+int latent_decode(void* out, int64_t out_token_stride, int64_t out_head_stride, const void* q_lat,
+                  int64_t lat_token_stride, int64_t lat_head_stride, const void* q_rot,
+                  int64_t rot_token_stride, int64_t rot_head_stride, const void* cache,
+                  const int* block_tables, int max_blocks, const int* query_start_loc,
+                  const int* context_lens, int num_seqs, int heads, int rank, int rot,
+                  int block_size, int num_blocks, float scale, int ranges, float* scratch,
+                  int64_t scratch_floats, int dtype, int window, const void* gate,
+                  int64_t gate_stride, const float* sinks, void* stream, const LatentUp* up) {
   if (num_seqs == 0) return VLA_OK;
   if (gate && gate_stride < heads) return VLA_ERR_ARG;
   if (!out || !q_lat || (rot > 0 && !q_rot) || !cache || !block_tables || !query_start_loc || !context_lens ||
@@ -508,6 +628,35 @@ extern "C" int vla_seq_latent_decode(void* out, int64_t out_token_stride, int64_
                        rot_token_stride, rot_head_stride, cache, block_tables, query_start_loc, context_lens, gate,
                        gate_stride, sinks, scratch, max_blocks, num_seqs, heads, rank, block_size, num_blocks, window,
                        ranges > 0 ? ranges : num_seqs, ranges == 0, scale};
-  return dtype == VLA_BF16 ? latent_decode_go<BF16>(a, rot, (hipStream_t)stream)
-                           : latent_decode_go<F16>(a, rot, (hipStream_t)stream);
+  return dtype == VLA_BF16 ? latent_decode_go<BF16>(a, up, rot, (hipStream_t)stream)
+                           : latent_decode_go<F16>(a, up, rot, (hipStream_t)stream);
+}
+}  // namespace
+
+extern "C" int vla_seq_latent_decode(void* out, int64_t out_token_stride, int64_t out_head_stride, const void* q_lat,
+                                     int64_t lat_token_stride, int64_t lat_head_stride, const void* q_rot,
+                                     int64_t rot_token_stride, int64_t rot_head_stride, const void* cache,
+                                     const int* block_tables, int max_blocks, const int* query_start_loc,
+                                     const int* context_lens, int num_seqs, int heads, int rank, int rot,
+                                     int block_size, int num_blocks, float scale, int ranges, float* scratch,
+                                     int64_t scratch_floats, int dtype, int window, const void* gate,
+                                     int64_t gate_stride, const float* sinks, void* stream) {
+  return latent_decode(out, out_token_stride, out_head_stride, q_lat, lat_token_stride, lat_head_stride, q_rot, rot_token_stride, rot_head_stride, cache, block_tables, max_blocks, query_start_loc, context_lens, num_seqs, heads, rank, rot, block_size, num_blocks, scale, ranges, scratch, scratch_floats, dtype, window, gate, gate_stride, sinks, stream, nullptr);
+}
+
+extern "C" int vla_seq_latent_decode_up_supported(int vdim) { return vdim == 32 || vdim == 64 || vdim == 128 || vdim == 256; }
+
+extern "C" int vla_seq_latent_decode_up(void* out, int64_t out_token_stride, int64_t out_head_stride, const void* q_lat,
+                                     int64_t lat_token_stride, int64_t lat_head_stride, const void* q_rot,
+                                     int64_t rot_token_stride, int64_t rot_head_stride, const void* cache,
+                                     const int* block_tables, int max_blocks, const int* query_start_loc,
+                                     const int* context_lens, int num_seqs, int heads, int rank, int rot,
+                                     int block_size, int num_blocks, float scale, int ranges, float* scratch,
+                                     int64_t scratch_floats, int dtype, int window, const void* gate,
+                                     int64_t gate_stride, const float* sinks, void* stream, const void* w, void* up, int64_t up_stride, int vdim) {
+  if (!w || !up || up_stride < (int64_t)heads * vdim || up_stride % 2 || ((uintptr_t)w % 4) || ((uintptr_t)up % 4))
+    return VLA_ERR_ARG;
+  if (!vla_seq_latent_decode_up_supported(vdim)) return VLA_ERR_HEAD_SIZE;
+  const LatentUp to{up, up_stride, w, vdim};
+  return latent_decode(out, out_token_stride, out_head_stride, q_lat, lat_token_stride, lat_head_stride, q_rot, rot_token_stride, rot_head_stride, cache, block_tables, max_blocks, query_start_loc, context_lens, num_seqs, heads, rank, rot, block_size, num_blocks, scale, ranges, scratch, scratch_floats, dtype, window, gate, gate_stride, sinks, stream, &to);
 }
