@@ -16,8 +16,9 @@
 // states after 4096 rows several times as far from 64 bits).
 // All products run on 16x16x4 fp32 matrix cores.  Operands that later kernels read lie in scratch lane for
 // lane.  Bound by memory and the launches: 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB
-// of chunk states and decays; 152 us per call (57 + 23 + 82 under the tracer) where the pieces of 256 rows walked
-// token by token and joined by matrix products took 408.
+// of chunk states and decays; 128 us per call (45 + 23 + 68 under the tracer) where the pieces of 256 rows walked
+// token by token and joined by matrix products took 408.  What a workgroup's 19 and 30 us go to: waits for its rows (5
+// and 7), products (7 and 9), decays (6 and 5), the products inside a block (4), gates and stores (5).
 #include <atomic>
 
 #include "seq_common.h"
@@ -88,6 +89,31 @@ __device__ __forceinline__ f32x4 row4(const typename S::T* p) {
   }
 }
 
+// exp(p) for p <= 0 (NaN passes): 2^n 2^f with the argument's rounding in f.  expf without what other p need; relative
+// error 2.6e-8 (root mean square over -80 .. 0) as expf's.
+__device__ __forceinline__ float exp_of_log(float p) {
+  p = p < -150.f ? -150.f : p;
+  const float n = __builtin_rintf(1.44269504f * p);
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(fmaf(1.92596299e-8f, p, fmaf(1.44269504f, p, -n))), (int)n);
+}
+
+// log1p(x) for 0 <= x <= 1: 2 artanh(s), s = x / (2 + x) <= 1 / 3 in two numbers, by its series up to s^17; relative error
+// 3.6e-8 (log1pf 2.6e-8; states of 4096 rows are off by 1.41e-7 from 64 bits with either) at a quarter of its instructions:
+// the decays were 12 of a workgroup's 25 us, now 5
+__device__ __forceinline__ float log1p_unit(float x) {
+  const float d = 2.f + x, lost = x - (d - 2.f), q = __builtin_amdgcn_rcpf(d), s0 = x * q;
+  const float more = fmaf(-lost, s0, fmaf(-d, s0, x)) * q, s = s0 + more, rest = more - (s - s0), z = s * s;
+  float a = 1.f / 17.f;
+  a = fmaf(a, z, 1.f / 15.f);
+  a = fmaf(a, z, 1.f / 13.f);
+  a = fmaf(a, z, 1.f / 11.f);
+  a = fmaf(a, z, 1.f / 9.f);
+  a = fmaf(a, z, 1.f / 7.f);
+  a = fmaf(a, z, 1.f / 5.f);
+  a = fmaf(a, z, 1.f / 3.f);
+  return 2.f * (s + fmaf(a * z, s, rest));
+}
+
 template <class S>
 __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
   using T = typename S::T;
@@ -108,49 +134,65 @@ __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
   const int RP = (R + 3) / 4 * 4;
   float* mine = a.scratch + ((int64_t)slot * a.heads + h) * chunk_floats(D, V);
 
-  // rows: four threads per row, neighbours read neighbouring values; rows behind the run's end are zeros
+  // rows behind the run's end are zeros
   const int row = tid >> 2, quarter = tid & 3;
   const int64_t t = t0 + min(row, n - 1);
-  const bool live = row < n;
-  const T* kr = (const T*)a.k + t * a.k_stride + (int64_t)h * D;
-  const T* vr = (const T*)a.v + t * a.v_stride + (int64_t)h * V;
+  const int d_mine = tid % D;                // the thread's decay channel and its row of W2, on its way with the rows
+  constexpr int PER = 16 / sizeof(T);
+  const bool w_wide = R % PER == 0 && (uintptr_t)a.w2 % 16 == 0;
+  u32x4 w_row[kMaxRank / PER];
+  float wv[kMaxRank];
+  const T* wr = (const T*)a.w2 + ((int64_t)h * D + d_mine) * R;
+  if (w_wide) {
+#pragma unroll
+    for (int r = 0; r < kMaxRank / PER; ++r)
+      if (PER * r < R) w_row[r] = *reinterpret_cast<const u32x4*>(wr + PER * r);
+  } else {
+#pragma unroll
+    for (int r = 0; r < kMaxRank; ++r) wv[r] = r < R ? S::to_f32(wr[r]) : 0.f;
+  }
+  const float bias = a.bias != nullptr ? a.bias[(int64_t)h * D + d_mine] : 0.f;
 #pragma unroll 4
-  for (int d = 4 * quarter; d < D; d += 16) {
-    f32x4 x = row4<S>(kr + d);
-    if (!live) x = f32x4{0.f, 0.f, 0.f, 0.f};
-    *reinterpret_cast<f32x4*>(k_lds + row * KR + d) = x;
+  for (int i = tid; i < kChunk * D / 4; i += 256) {         // four values a thread, in the order they lie in
+    const int r = i / (D / 4), d = 4 * (i % (D / 4));
+    const f32x4 x = row4<S>((const T*)a.k + (t0 + min(r, n - 1)) * a.k_stride + (int64_t)h * D + d);
+    *reinterpret_cast<f32x4*>(k_lds + r * KR + d) = r < n ? x : f32x4{0.f, 0.f, 0.f, 0.f};
   }
 #pragma unroll 8
-  for (int d = 4 * quarter; d < V; d += 16) {
-    f32x4 x = row4<S>(vr + d);
-    if (!live) x = f32x4{0.f, 0.f, 0.f, 0.f};
-    *reinterpret_cast<f32x4*>(v_lds + row * VR + d) = x;
+  for (int i = tid; i < kChunk * V / 4; i += 256) {
+    const int r = i / (V / 4), d = 4 * (i % (V / 4));
+    const f32x4 x = row4<S>((const T*)a.v + (t0 + min(r, n - 1)) * a.v_stride + (int64_t)h * V + d);
+    *reinterpret_cast<f32x4*>(v_lds + r * VR + d) = r < n ? x : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   for (int r = quarter; r < RP; r += 4)
     y_lds[row * kMaxRank + r] = r < R ? S::to_f32(((const T*)a.y)[t * a.y_stride + r]) : 0.f;
   __syncthreads();
 
   // decays: a thread keeps its channel's row of W2 and walks every (256 / D)-th row
-  for (int d = tid % D, r0 = tid / D; r0 < 256 / D; r0 += 256) {
-    float wv[kMaxRank];
-    const T* wr = (const T*)a.w2 + ((int64_t)h * D + d) * R;
+  if (w_wide) {
 #pragma unroll
-    for (int r = 0; r < kMaxRank; ++r) wv[r] = r < R ? S::to_f32(wr[r]) : 0.f;
-    const float bias = a.bias != nullptr ? a.bias[(int64_t)h * D + d] : 0.f;
-    for (int i = r0; i < kChunk; i += 256 / D) {
-      float z = bias;
-#pragma unroll
-      for (int r4 = 0; r4 < kMaxRank; r4 += 4) {
-        if (r4 >= RP) break;
-        const f32x4 yv = *reinterpret_cast<const f32x4*>(y_lds + i * kMaxRank + r4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) z += wv[r4 + e] * yv[e];
-      }
-      // ln sigmoid(z) = -(max(-z, 0) + log1p(exp(-|z|)))
-      const float ld = -(fmaxf(-z, 0.f) + log1pf(expf(-fabsf(z)))) * a.inv_tau;
-      a_lds[i * D + d] = i < n ? ld : 0.f;
-      mine[i * D + d] = i < n ? ld : 0.f;
+    for (int r = 0; r < kMaxRank; ++r) {
+      if (r >= R)
+        wv[r] = 0.f;
+      else if constexpr (sizeof(T) == 2)
+        wv[r] = r & 1 ? hi16<S>(w_row[r / PER][r % PER / 2]) : lo16<S>(w_row[r / PER][r % PER / 2]);
+      else
+        wv[r] = __builtin_bit_cast(float, (uint32_t)w_row[r / PER][r % PER]);
     }
+  }
+  for (int i = tid / D; i < kChunk; i += 256 / D) {
+    float z = bias;
+#pragma unroll
+    for (int r4 = 0; r4 < kMaxRank; r4 += 4) {
+      if (r4 >= RP) break;
+      const f32x4 yv = *reinterpret_cast<const f32x4*>(y_lds + i * kMaxRank + r4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z += wv[r4 + e] * yv[e];
+    }
+    // ln sigmoid(z) = -(max(-z, 0) + log1p(exp(-|z|)))
+    const float ld = -(fmaxf(-z, 0.f) + log1p_unit(exp_of_log(-fabsf(z)))) * a.inv_tau;
+    a_lds[i * D + d_mine] = i < n ? ld : 0.f;
+    mine[i * D + d_mine] = i < n ? ld : 0.f;
   }
   __syncthreads();
 
@@ -163,7 +205,7 @@ __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
     float p = 0.f;
 #pragma unroll
     for (int i = kBlock - 1; i >= 0; --i) {
-      k_lds[(kBlock * seg + i) * KR + d] *= expf(p);
+      k_lds[(kBlock * seg + i) * KR + d] *= exp_of_log(p);
       p += av[i];
     }
     tot[seg * D + d] = p;
@@ -171,29 +213,33 @@ __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
   __syncthreads();
   for (int d = tid; d < D; d += 256) {
     const float t3 = tot[3 * D + d], t2 = tot[2 * D + d] + t3, t1 = tot[D + d] + t2;
-    mine[kChunk * D + d] = expf(tot[d] + t1);
+    mine[kChunk * D + d] = exp_of_log(tot[d] + t1);
     // from here on: the decay over the blocks behind each
-    tot[d] = expf(t1);
-    tot[D + d] = expf(t2);
-    tot[2 * D + d] = expf(t3);
+    tot[d] = exp_of_log(t1);
+    tot[D + d] = exp_of_log(t2);
+    tot[2 * D + d] = exp_of_log(t3);
     tot[3 * D + d] = 1.f;
   }
   __syncthreads();
   float* r_out = mine + kChunk * D + D;
   const int dt_n = D / 16, vt_n = V / 16;
-  for (int tile = w; tile < dt_n * vt_n; tile += 4) {
-    const int dt = tile / vt_n, vt = tile - dt * vt_n;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const int pairs = (vt_n + 1) / 2;            // two value tiles share the reads of the keys
+  for (int item = w; item < dt_n * pairs; item += 4) {
+    const int dt = item / pairs, vt = 2 * (item - dt * pairs), vt2 = min(vt + 1, vt_n - 1);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = acc;
 #pragma unroll
     for (int seg = 0; seg < 4; ++seg) {
       const float m = tot[seg * D + 16 * dt + c];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int j = kBlock * seg + 4 * g + e;
-        acc = mfma4(k_lds[j * KR + 16 * dt + c] * m, v_lds[j * VR + 16 * vt + c], acc);
+        const float kj = k_lds[j * KR + 16 * dt + c] * m;
+        acc = mfma4(kj, v_lds[j * VR + 16 * vt + c], acc);
+        acc2 = mfma4(kj, v_lds[j * VR + 16 * vt2 + c], acc2);
       }
     }
-    *reinterpret_cast<f32x4*>(r_out + ((int64_t)tile * 64 + lane) * 4) = acc;
+    *reinterpret_cast<f32x4*>(r_out + ((int64_t)(dt * vt_n + vt) * 64 + lane) * 4) = acc;
+    if (vt2 != vt) *reinterpret_cast<f32x4*>(r_out + ((int64_t)(dt * vt_n + vt2) * 64 + lane) * 4) = acc2;
   }
 }
 
@@ -287,7 +333,7 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
       }
       *reinterpret_cast<f32x4*>(q_lds + row * KR + d) = qv[x];
       *reinterpret_cast<f32x4*>(k_lds + row * KR + d) = kv[x];
-      *reinterpret_cast<f32x4*>(a_lds + row * D + d) = f32x4{expf(av[x][0]), expf(av[x][1]), expf(av[x][2]), expf(av[x][3])};
+      *reinterpret_cast<f32x4*>(a_lds + row * D + d) = f32x4{exp_of_log(av[x][0]), exp_of_log(av[x][1]), exp_of_log(av[x][2]), exp_of_log(av[x][3])};
     }
   }
   __syncthreads();
@@ -327,13 +373,13 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
 #pragma unroll
     for (int i = 0; i < kBlock; ++i) {
       p += av[i];
-      q_lds[(kBlock * seg + i) * KR + d] *= expf(p);
+      q_lds[(kBlock * seg + i) * KR + d] *= exp_of_log(p);
     }
     tot[seg * D + d] = p;
     p = 0.f;
 #pragma unroll
     for (int i = kBlock - 1; i >= 0; --i) {
-      k_lds[(kBlock * seg + i) * KR + d] *= expf(p);
+      k_lds[(kBlock * seg + i) * KR + d] *= exp_of_log(p);
       p += av[i];
     }
   }
@@ -352,7 +398,7 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
       const f32x4 tv = *reinterpret_cast<const f32x4*>(tot + o * D + 16 * x + 4 * g);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        acc = mfma4(qv[e] * expf(before[x][e]), kv[e], acc);
+        acc = mfma4(qv[e] * exp_of_log(before[x][e]), kv[e], acc);
         before[x][e] += tv[e];
       }
     }
@@ -376,13 +422,33 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
     }
   const bool some_bad = __syncthreads_or(odd);
 
+  // Results leave through LDS, eight neighbouring columns of a row to a lane, where the rows of gates and results allow
+  // it (16-bit types).  Gates and norm weights are there ahead of the stores: a load behind a store that may write the same
+  // place waits for it.
+  const bool wide = sizeof(T) == 2 && a.gate_stride % 8 == 0 && a.out_stride % 8 == 0 &&
+                    (uintptr_t)a.gate % 16 == 0 && (uintptr_t)a.out % 16 == 0;
+  constexpr int PIECES = 4;                                // 16 rows of 16 pieces over 64 lanes
+  u32x4 gates[PIECES];
+  float norm[8];
+  const int row_of = lane >> 3, col_of = 8 * (lane & 7);   // of half the columns: rows row_of and row_of + 8
+#pragma unroll
+  for (int vt = 0; vt < 8; ++vt)
+    if (vt < vt_n) norm[vt] = a.norm_weight[16 * vt + c];
+  if (wide) {
+#pragma unroll
+    for (int u = 0; u < PIECES; ++u) {
+      const int i = min(kBlock * w + row_of + 8 * (u & 1), n - 1), col = 64 * (u >> 1) + col_of;
+      if (col < V) gates[u] = *reinterpret_cast<const u32x4*>((const T*)a.gate + (int64_t)(t0 + i) * a.gate_stride + (int64_t)h * V + col);
+    }
+  }
+
   f32x4 acc[8];
   f32x4 qs[DT];
 #pragma unroll
   for (int x = 0; x < DT; ++x) {
     qs[x] = *reinterpret_cast<const f32x4*>(q_lds + (kBlock * w + c) * KR + 16 * x + 4 * g);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) qs[x][e] *= expf(before[x][e]);
+    for (int e = 0; e < 4; ++e) qs[x][e] *= exp_of_log(before[x][e]);
   }
   float ss[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -423,19 +489,54 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
   group_sums(ss[0], ss[1], 16);
   group_sums(ss[2], ss[3], 16);
   // lane: column 16 vt + c of rows 16 w + 4 g .. + 3
+  float inv[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) inv[e] = a.out_scale / sqrtf(ss[e] / (float)V + a.eps);
+  if constexpr (sizeof(T) == 2) {
+    if (wide) {
+      float* own = a_mat + kBlock * w * kAMat;             // the wave's rows of A, which it alone reads and has read
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        if (64 * half >= V) break;
+        wave_sync();
+#pragma unroll
+        for (int vt = 4 * half; vt < 4 * half + 4; ++vt)
+          if (vt < vt_n)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) own[(4 * g + e) * kAMat + 16 * (vt - 4 * half) + c] = acc[vt][e] * inv[e] * norm[vt];
+        wave_sync();
+#pragma unroll
+        for (int r8 = 0; r8 < 2; ++r8) {
+          const int r = row_of + 8 * r8, i = kBlock * w + r, col = 64 * half + col_of;
+          if (i >= n || col >= V) continue;
+          const f32x4 x0 = *reinterpret_cast<const f32x4*>(own + r * kAMat + col_of), x1 = *reinterpret_cast<const f32x4*>(own + r * kAMat + col_of + 4);
+          const u32x4 gw = gates[2 * half + r8];
+          u32x4 res;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float g0 = lo16<S>(gw[k]), g1 = hi16<S>(gw[k]);
+            const float y0 = 2 * k < 4 ? x0[2 * k & 3] : x1[2 * k & 3], y1 = 2 * k < 4 ? x0[(2 * k + 1) & 3] : x1[(2 * k + 1) & 3];
+            res[k] = pack16<S>(y0 * (g0 / (1.f + expf(-g0))), y1 * (g1 / (1.f + expf(-g1))));
+          }
+          *reinterpret_cast<u32x4*>((T*)a.out + (int64_t)(t0 + i) * a.out_stride + (int64_t)h * V + col) = res;
+        }
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int i = kBlock * w + 4 * g + e;
     if (i >= n) continue;
-    const float inv = a.out_scale / sqrtf(ss[e] / (float)V + a.eps);
     const T* gr = (const T*)a.gate + (int64_t)(t0 + i) * a.gate_stride + (int64_t)h * V + c;
     T* to = (T*)a.out + (int64_t)(t0 + i) * a.out_stride + (int64_t)h * V + c;
+    float gt[8];
 #pragma unroll
     for (int vt = 0; vt < 8; ++vt)
-      if (vt < vt_n) {
-        const float gt = S::to_f32(gr[16 * vt]);
-        to[16 * vt] = S::from_f32(acc[vt][e] * inv * a.norm_weight[16 * vt + c] * (gt / (1.f + expf(-gt))));
-      }
+      if (vt < vt_n) gt[vt] = S::to_f32(gr[16 * vt]);
+#pragma unroll
+    for (int vt = 0; vt < 8; ++vt)
+      if (vt < vt_n) to[16 * vt] = S::from_f32(acc[vt][e] * inv[e] * norm[vt] * (gt[vt] / (1.f + expf(-gt[vt]))));
   }
 }
 
