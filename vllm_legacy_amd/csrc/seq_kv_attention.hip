@@ -596,11 +596,11 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
   auto look_up = [&](int u0) {
     const int j = key_of(min(u0 + tid, total - 1));    // behind the end: the last key again, masked
     const int nb = shifts ? j >> shift : j / block_size;
-    const int blk = table[nb];
-    return Place{(unsigned)blk < (unsigned)num_blocks ? blk : 0, j - nb * block_size};
+    return Place{table[nb], j - nb * block_size};      // not looked at yet: that would wait for it, and for the DMA
   };
   auto store_row = [&](Place p, int buf) {
-    const long long row = ((long long)p.blk * block_size + p.at) * kv_heads + g;
+    const int blk = (unsigned)p.blk < (unsigned)num_blocks ? p.blk : 0;
+    const long long row = ((long long)blk * block_size + p.at) * kv_heads + g;
     rows_lds[buf][0][tid] = row * (2 * D);
     rows_lds[buf][1][tid] = row * (2 * v_row);
   };
@@ -706,15 +706,32 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) st[kb][i] *= scale2;
     }
-    // every key of the tile visible to every row of the wave: no masks
-    if (kept_tile || j0 + kKeys - 1 > p0 || nq != kTile || j0 < lo_last) {
+    // Masks, only where some key of the tile is hidden from some row of the wave; rows behind the run's end (c >= nq)
+    // may see anything, nobody writes them.  A tile of 64 consecutive keys compares its 32 numbers, known when it is
+    // compiled, with one limit a lane; tiles with kept tokens work out every key.
+    if (kept_tile || j0 < keep_first) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int j = key_of(u0 + 32 * kb + (i & 3) + 8 * (i >> 2) + 4 * hf);
-          st[kb][i] = c < nq && j <= pq && (j >= lo_q || j < keep_first) ? st[kb][i] : -INFINITY;
+          st[kb][i] = j <= pq && (j >= lo_q || j < keep_first) ? st[kb][i] : -INFINITY;
         }
+    } else {
+      if (j0 + kKeys - 1 > p0) {
+        const int last = pq - j0 - 4 * hf;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) st[kb][i] = 32 * kb + (i & 3) + 8 * (i >> 2) <= last ? st[kb][i] : -INFINITY;
+      }
+      if (j0 < lo_last) {
+        const int least = lo_q - j0 - 4 * hf;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) st[kb][i] = 32 * kb + (i & 3) + 8 * (i >> 2) >= least ? st[kb][i] : -INFINITY;
+      }
     }
     float mt = -INFINITY;
 #pragma unroll
