@@ -273,6 +273,16 @@ int vla_seq_kv_attention_tiles(void* out, int64_t out_stride, const void* q, int
                                int block_size, int num_blocks, int window, float scale, int dtype,
                                int keep_first, float softcap, int chunk, const float* sinks,
                                void* stream);
+/* The same for a step of num_rows rows in all (sequences of different lengths launch no more than they need). */
+int vla_seq_kv_attention_tiles_of(void* out, int64_t out_stride, const void* q, int64_t q_stride,
+                                  const void* gate, int64_t gate_stride, const void* key_cache,
+                                  const void* value_cache, const int* block_tables, int max_blocks,
+                                  const int* query_start_loc, const int* context_lens,
+                                  const float* out_inv_freq, int interleaved, int num_seqs,
+                                  int max_query_len, int64_t num_rows, int heads, int kv_heads, int dim, int vdim,
+                                  int block_size, int num_blocks, int window, float scale, int dtype,
+                                  int keep_first, float softcap, int chunk, const float* sinks,
+                                  void* stream);
 int vla_seq_set_kv_attention_kernel(int mode);
 
 /* ---- element-wise gated recurrence (minGRU) ---------------------------------------------------- */

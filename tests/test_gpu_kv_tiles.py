@@ -1,7 +1,8 @@
 """Runs of query rows on the LDS-DMA tile kernel: every key and value size class it exchanges differently, groups of
 1 to 4 heads, pages of 1, 4 and 16 tokens, runs around its tiles of 32 rows and 64 keys, windows, chunks, kept
 first tokens, caps, sinks, gates, values that turn back, scales of either sign, outputs at odd addresses, both
-with the keys shared out to two groups of waves and (many sequences) with one -- against the same attention in
+with the keys shared out to two groups of waves and (many sequences) with one, with tiles found by their rank (up to
+256 sequences, one to four registers a lane) and by the grid (more) -- against the same attention in
 float64 and the bound of the single rows' test: 1 % of the largest value in bfloat16, an eighth in float16."""
 import pytest
 import torch
@@ -24,7 +25,7 @@ CASES = [
 
 @pytest.mark.parametrize("case", CASES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("copies", [1, 600])
+@pytest.mark.parametrize("copies", [1, 60, 600])
 def test_runs_of_rows(case, dtype, copies):
     from vllm_legacy_amd import _seq_ops as ops
     H, G, D, V, bs, runs, opt = case

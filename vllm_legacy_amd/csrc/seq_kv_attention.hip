@@ -22,6 +22,7 @@
 // tile is 64 keys: lane j scores key j against the query held in LDS, the wave reduces max / sum
 // (online softmax across tiles), then lane d accumulates sum_j p_j v_j[d] with coalesced reads.
 #include <atomic>
+#include <type_traits>
 
 #include "seq_common.h"
 
@@ -443,18 +444,20 @@ __device__ __forceinline__ void turn_back(f32x16 (&o)[VB], int hf, float p,
 // max / sum (base 2) and the accumulators are fp32; a weight enters the second product rounded to
 // the model dtype.
 //
-// Bound by the products and the softmax between them (about 30 vector cycles per score), so the tiles
+// Bound by the vector port and the chain from the scores over their maximum to the second product: a wave alone takes
+// 3000 cycles for a tile (1024 of products, 1200 of vector instructions), two that share a SIMD 4500 for one each.  Tiles
 // come in by LDS-DMA: no staging registers, no waits before the stores to LDS, one barrier per tile, two
-// tiles in LDS (64 KB at most and 2 KB of the rows' places: two workgroups share a CU and one's softmax runs under
+// tiles in LDS (64 KB at most and the rows' places: two workgroups share a CU and one's softmax runs under
 // the other's products).  A DMA instruction writes 64 lanes x 16 bytes in a row, so rows cannot be padded: 16-byte
 // pieces of a key row and 64-byte units of a value row are exchanged by the row's number on the source's
-// side, so that the lanes of a read fall into different banks.  What only some calls need (a cap, masks)
-// is a loop of its own behind one branch.  Workgroups go out longest walk first over all sequences, and those
-// of a (sequence, head) share an XCD's L2 when their number is a multiple of 8.  Where the workgroups are few,
+// side, so that the lanes of a read fall into different banks.  The next tile's DMA goes out between the first products
+// (sent at once it holds a wave up for 700 cycles), weights are formed between the second ones, and accumulators are
+// scaled only when a maximum has moved by more than kLag.  What is the same for all lanes is told to the compiler, or every
+// choice of a mask or a scale copies the 32 scores.  Workgroups go out longest walk first over all sequences,
+// groups of heads next to each other: each XCD's L2 holds few heads' keys.  Where the workgroups are few,
 // each has two groups of four waves (KG = 2) that take every other tile and join their sums at the end.  Four
-// prompts of up to 2047 rows, 16 heads on 4 of 128: 102 us, against 172 with tiles staged through registers
-// into padded rows.  A wave alone takes 2.6 us per tile, 0.45 of them products: what is left is the chain
-// from the scores over their maximum and the exponentials to the second product.
+// prompts of up to 2047 rows, 16 heads on 4 of 128: 62 us (104 with DMA in a burst, masks for all tiles of a run's last
+// rows and a grid as long as the longest prompt for each; 172 with tiles staged through registers into padded rows).
 template <class S>
 struct Mfma16;
 template <>
@@ -473,6 +476,7 @@ struct Mfma16<F16> {
 };
 
 constexpr int kKeys = 64;     // keys per staged tile
+constexpr float kLag = 8.f;   // how far a row's scores (base 2) may lie above its running maximum
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef s16x4 __attribute__((address_space(3))) * lds_s16x4;
 
@@ -496,14 +500,99 @@ __device__ __forceinline__ int value_exchange(int r) {
   return VB == 4 ? r & 3 : VB == 2 ? (r >> 1) & 1 : 0;
 }
 
-// 16 bytes per lane from each lane's own address into 1 KB of LDS (no register result)
-__device__ __forceinline__ void tile_dma16(const void* src, uint32_t lds_at) {
+// 16 bytes per lane from each lane's own address into 1 KB of LDS (no register result), where `go`: a branch that the
+// compiler does not see, so that the products around it stay one block
+__device__ __forceinline__ void tile_dma16(const void* src, uint32_t lds_at, int go) {
   unsigned keep;
   asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+      "s_cmp_lg_u32 %3, 0\n\ts_cbranch_scc0 1f\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0\n1:"
       : "=&s"(keep)
-      : "v"(src), "s"(lds_at)
-      : "memory");
+      : "v"(src), "s"(lds_at), "s"(__builtin_amdgcn_readfirstlane(go))
+      : "memory", "scc");
+}
+
+// the larger of a lane's value and that of the lane 32 further on
+__device__ __forceinline__ float max_halves(float v) {
+  const uint32_t x = __builtin_bit_cast(uint32_t, v);
+  const auto both = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)both[0]), __builtin_bit_cast(float, (uint32_t)both[1]));
+}
+
+// the sum over a wave, in every lane
+__device__ __forceinline__ int wave_total(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);      // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);     // row_bcast 15 to rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);     // row_bcast 31 to rows 2 and 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// The `rank`-th of all tiles of 2^shift rows of a step's sequences, counted from those that walk the most keys (a
+// tile's level: how many tiles of keys lie ahead of its last row).  Every wave finds it for itself: a search over
+// the levels for the one whose tiles hold the rank, with the sequences in the lanes' registers.  Launching one
+// workgroup per tile of the longest sequence for every sequence instead left empty ones between the real ones:
+// workgroups go to the shader engines of an XCD in turn, an engine that is full holds all others up, and half the
+// chip stood idle for 40 of 98 us with four prompts of 2047, 1265, 483 and 1748 rows.  The search takes about 2 us
+// of a workgroup.
+constexpr int kRankedChunks = 4;
+constexpr int kRankedSeqs = kRankedChunks * kWave;
+__device__ __forceinline__ bool ranked_tile(int rank, int num_seqs, const int* __restrict__ query_start_loc,
+                                            const int* __restrict__ context_lens, int shift, int& seq, int& tile) {
+  const int lane = threadIdx.x & 63, chunks = (num_seqs + kWave - 1) / kWave;
+  int first[kRankedChunks], end[kRankedChunks];       // the levels of a sequence's tiles
+  int top = 0, all = 0;
+#pragma unroll
+  for (int k = 0; k < kRankedChunks; ++k) {
+    first[k] = end[k] = 0;
+    if (k < chunks) {
+      const int s = k * kWave + lane;
+      if (s < num_seqs) {
+        first[k] = context_lens[s] >> shift;
+        end[k] = first[k] + ((max(query_start_loc[s + 1] - query_start_loc[s], 0) + (1 << shift) - 1) >> shift);
+      }
+      all += end[k] - first[k];
+      top = max(top, end[k]);
+    }
+  }
+  if (wave_total(all) <= rank) return false;
+#pragma unroll
+  for (int x = 1; x < kWave; x <<= 1) top = max(top, __shfl_xor(top, x, 64));
+  auto at_least = [&](int level) {                     // tiles of this level and above
+    int n = 0;
+#pragma unroll
+    for (int k = 0; k < kRankedChunks; ++k)
+      if (k < chunks) n += max(end[k] - max(first[k], level), 0);
+    return wave_total(n);
+  };
+  int lo = 0, hi = __builtin_amdgcn_readfirstlane(top), above = 0;      // at_least(lo) > rank >= at_least(hi) = above
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1, n = at_least(mid);
+    if (n > rank) {
+      lo = mid;
+    } else {
+      hi = mid;
+      above = n;
+    }
+  }
+  int left = rank - above;
+#pragma unroll
+  for (int k = 0; k < kRankedChunks; ++k)
+    if (k < chunks && left >= 0) {
+      const bool here = first[k] <= lo && lo < end[k];
+      const uint64_t mask = __ballot(here);
+      const int n = __popcll(mask);
+      if (left < n) {
+        const uint64_t which = __ballot(here && __popcll(mask & ((1ull << lane) - 1)) == left);
+        const int l = __ffsll((unsigned long long)which) - 1;
+        seq = k * kWave + l;
+        tile = lo - __builtin_amdgcn_readlane(first[k], l);
+      }
+      left -= n;
+    }
+  return true;
 }
 
 template <class S, int DB, int VB, int KG>
@@ -515,7 +604,7 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
     const int* __restrict__ context_lens, const float* __restrict__ out_inv_freq, int interleaved,
     int heads, int kv_heads, int head_groups, int block_size, int num_blocks, int window, float scale, int head_waves,
     int keep_first, float softcap, int chunk, const float* __restrict__ sinks, int v_row, int v_first,
-    int last_tile) {
+    int last_tile, int ranked_seqs, int first_rank) {
   using T = typename S::T;
   using M = Mfma16<S>;
   constexpr int D = 32 * DB, VD = 32 * VB;
@@ -527,12 +616,17 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
   constexpr int KMASK = DB == 4 ? 15 : DB == 2 ? 7 : 3, KSHIFT = DB == 4 ? 0 : DB == 2 ? 1 : 2;
   // two tiles for every group of waves: one is read while the next lands
   __shared__ __align__(16) unsigned char all_tiles[KG * 2 * STAGE];
-  __shared__ long long all_rows[KG][2][2][kKeys];      // first byte of each key and value row of a tile
-  const int b = blockIdx.x / head_groups, yb = blockIdx.x - b * head_groups;
+  __shared__ uint32_t all_rows[KG][2][kKeys];          // the cache row (slot) of each key of a tile
+  const int yb = blockIdx.x % head_groups;
   const int row_blocks = 4 / head_waves;              // blocks of 32 query rows per workgroup
   const int tile_rows = kTile * row_blocks;
   // the last tiles of a run have the most keys to walk: they are dispatched first
-  const int tile_x = last_tile - (int)blockIdx.y;
+  int b = blockIdx.x / head_groups, tile_x = last_tile - (int)blockIdx.y;
+  if (ranked_seqs > 0) {
+    if (!ranked_tile(first_rank + b, ranked_seqs, query_start_loc, context_lens, __builtin_ctz(tile_rows), b, tile_x)) return;
+    b = __builtin_amdgcn_readfirstlane(b);
+    tile_x = __builtin_amdgcn_readfirstlane(tile_x);
+  }
   const int t_first = query_start_loc[b] + tile_rows * tile_x;
   const int n_tile = min(tile_rows, query_start_loc[b + 1] - t_first);
   if (n_tile <= 0) return;
@@ -552,84 +646,82 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
   const int p_first = context_lens[b] + tile_rows * tile_x, p_last = p_first + n_tile - 1;
   const int p0 = p_first + kTile * rb;                // this wave's first position
   const int pq = p0 + c;
-  const int j_lo = first_key(p_first, window, chunk);
+  // (the compiler does not see that a remainder is the same for all lanes, and would take every branch on it for one
+  // that is not)
+  const int j_lo = __builtin_amdgcn_readfirstlane(first_key(p_first, window, chunk));
   const int lo_q = first_key(pq, window, chunk);      // this lane's row's first key
-  const int lo_first = first_key(p0, window, chunk);  // of the wave's first row and of its last
-  const int lo_last = first_key(p0 + kTile - 1, window, chunk);
+  // of the wave's first row and of its last
+  const int lo_first = __builtin_amdgcn_readfirstlane(first_key(p0, window, chunk));
+  const int lo_last = __builtin_amdgcn_readfirstlane(first_key(p0 + kTile - 1, window, chunk));
   // the keys this workgroup walks, through one index: the kept first tokens that lie ahead of the
   // first row's window, then the window's first key to the last row
   const int nk = min(keep_first, j_lo);
   const int total = nk + p_last - j_lo + 1;
   auto key_of = [&](int u) { return u < nk ? u : u - nk + j_lo; };
+  // in that index, a row sees u <= last and (u >= least or u < kept); the same for the wave's rows together
+  const int kept = nk == j_lo ? keep_first : nk;
+  const int last_q = pq + nk - j_lo, least_q = lo_q + nk - j_lo;
+  const int last_first = p0 + nk - j_lo, last_last = last_first + nq - 1;
+  const int least_first = lo_first + nk - j_lo, least_last = lo_last + nk - j_lo;
   const int* table = block_tables + (int64_t)b * max_blocks;
   const float scale2 = scale * 1.4426950408889634f;   // scores in base 2
   const float cap2 = softcap * 1.4426950408889634f, cap_arg = softcap > 0.f ? 2.f * 1.4426950408889634f / softcap : 0.f;
   // a positive scale is left to the exponent's fused product; otherwise scores are scaled before the maximum
   const bool late = softcap <= 0.f && scale2 > 0.f;
-  const float factor = late ? scale2 : 1.f;
 
-  u32x4 qf[D / 16];
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (active && c < nq)
-      v = *reinterpret_cast<const u32x4*>(q + (int64_t)(t0 + c) * q_stride + (int64_t)h * D + 16 * ks + 8 * hf);
-    qf[ks] = v;
-  }
   f32x16 o[VB];
 #pragma unroll
   for (int n = 0; n < VB; ++n)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[n][i] = 0.f;
-  float m = -INFINITY, l = 0.f;
+  float m = -INFINITY, top = 0.f, l = 0.f;            // top: m, and 0 where nothing was seen yet
   if (sinks != nullptr && active && kg == 0) {     // the denominator's first term, counted in one lane half
-    m = sinks[h] * 1.4426950408889634f;
+    top = m = sinks[h] * 1.4426950408889634f;
     l = hf == 0 ? 1.f : 0.f;
   }
 
-  // threads 0 .. 63 look the rows of a tile up: the block id is read one step before it is used
+  // the first wave looks the rows of a tile up: the block id is read one step before it is used
   const bool shifts = (block_size & (block_size - 1)) == 0;
   const int shift = __builtin_ctz(block_size);
   struct Place {
     int blk, at;
   };
   auto look_up = [&](int u0) {
-    const int j = key_of(min(u0 + tid, total - 1));    // behind the end: the last key again, masked
+    const int j = key_of(min(u0 + lane, total - 1));   // behind the end: the last key again, masked
     const int nb = shifts ? j >> shift : j / block_size;
     return Place{table[nb], j - nb * block_size};      // not looked at yet: that would wait for it, and for the DMA
   };
   auto store_row = [&](Place p, int buf) {
     const int blk = (unsigned)p.blk < (unsigned)num_blocks ? p.blk : 0;
-    const long long row = ((long long)blk * block_size + p.at) * kv_heads + g;
-    rows_lds[buf][0][tid] = row * (2 * D);
-    rows_lds[buf][1][tid] = row * (2 * v_row);
+    rows_lds[buf][lane] = (uint32_t)blk * (uint32_t)block_size + (uint32_t)p.at;      // a card holds fewer than 2^32 rows
   };
   // what this lane brings in: the row of a tile, and the piece of it that stands at the lane's place
-  int row_k[DB], at_k[DB], row_v[VB], at_v[VB];
+  constexpr int kPieces = DB + VB;                     // DMA instructions of a wave
+  int row_of[kPieces];
+  const unsigned char* from[kPieces];                  // where the piece of cache row 0 lies
 #pragma unroll
   for (int u = 0; u < DB; ++u) {
     const int at = (w * DB + u) * 64 + lane, r = at / (KB / 16), p = at % (KB / 16);
-    row_k[u] = r;
-    at_k[u] = 16 * ((p & ~KMASK) | ((p ^ (r >> KSHIFT)) & KMASK));
+    row_of[u] = r;
+    from[u] = (const unsigned char*)key_cache + (size_t)g * KB + 16 * ((p & ~KMASK) | ((p ^ (r >> KSHIFT)) & KMASK));
   }
 #pragma unroll
   for (int u = 0; u < VB; ++u) {
     const int at = (w * VB + u) * 64 + lane, r = at / (VBYTES / 16), p = at % (VBYTES / 16);
-    row_v[u] = r;
-    at_v[u] = 2 * v_first + 16 * ((((p >> 2) ^ value_exchange<VB>(r)) << 2) | (p & 3));
+    row_of[DB + u] = r;
+    from[DB + u] = (const unsigned char*)value_cache + (size_t)g * (2 * v_row) + 2 * v_first +
+                   16 * ((((p >> 2) ^ value_exchange<VB>(r)) << 2) | (p & 3));
   }
+  const uint32_t key_row = (uint32_t)kv_heads * KB, value_row = (uint32_t)kv_heads * 2 * v_row;
   const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)tiles;
-  auto bring = [&](int buf) {                          // the tile whose rows are in rows_lds[buf] into buffer buf
-    const uint32_t to = lds0 + buf * STAGE;
-    const unsigned char *sk[DB], *sv[VB];              // all of them first: one wait for LDS
+  uint32_t slot[kPieces];
+  auto slots_of = [&](int buf) {                       // the rows of the tile that is brought in next
 #pragma unroll
-    for (int u = 0; u < DB; ++u) sk[u] = (const unsigned char*)key_cache + (rows_lds[buf][0][row_k[u]] + at_k[u]);
-#pragma unroll
-    for (int u = 0; u < VB; ++u) sv[u] = (const unsigned char*)value_cache + (rows_lds[buf][1][row_v[u]] + at_v[u]);
-#pragma unroll
-    for (int u = 0; u < DB; ++u) tile_dma16(sk[u], to + (w * DB + u) * 1024);
-#pragma unroll
-    for (int u = 0; u < VB; ++u) tile_dma16(sv[u], to + KTILE + (w * VB + u) * 1024);
+    for (int i = 0; i < kPieces; ++i) slot[i] = DB == VB && i >= DB ? slot[i - DB] : rows_lds[buf][row_of[i]];
+  };
+  auto bring = [&](int i, int buf, int go) {           // piece i of that tile into buffer buf
+    const uint32_t to = lds0 + buf * STAGE + (i < DB ? (w * DB + i) * 1024 : KTILE + (w * VB + i - DB) * 1024);
+    tile_dma16(from[i] + (uint64_t)slot[i] * (i < DB ? key_row : value_row), to, go);
   };
   // where this lane reads: the exchanged piece of its key row, and the unit of its value rows
   const int kx = (hf ^ (c >> KSHIFT)) & KMASK;         // piece 2 ks + hf stands at 2 ks ^ kx within its group
@@ -639,17 +731,38 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
   const int vat = vr * VBYTES + 32 * (c >> 4) + 8 * (i16 & 3);
 
   // One barrier per tile.  Behind it in step `it`: tile `it` is in its buffer, the rows of tile it + 1 are in
-  // rows_lds[(it + 1) & 1], and threads 0 .. 63 hold the block ids of tile it + 2.
-  Place next = {0, 0};
-  if (tid < kKeys) {
+  // rows_lds[(it + 1) & 1], and the first wave holds the block ids of tile it + 2.
+  // (the first three ids are asked for together, ahead of the query rows: nothing waits for more than it needs)
+  Place next = {0, 0}, first = {0, 0}, second = {0, 0};
+  if (w == 0) {
     const int u = kg * kKeys;
-    store_row(look_up(u), 0);
-    store_row(look_up(u + kStep), 1);
+    first = look_up(u);
+    second = look_up(u + kStep);
     next = look_up(u + 2 * kStep);
   }
+  __builtin_amdgcn_sched_barrier(0);
+  u32x4 qf[D / 16];
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) {
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (active && c < nq)
+      v = *reinterpret_cast<const u32x4*>(q + (int64_t)(t0 + c) * q_stride + (int64_t)h * D + 16 * ks + 8 * hf);
+    qf[ks] = v;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (w == 0) {
+    store_row(first, 0);
+    store_row(second, 1);
+  }
   __syncthreads();
-  if (kg * kKeys < total) bring(0);
+  slots_of(0);
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) bring(i, 0, kg * kKeys < total);
   const int steps = (total + kStep - 1) / kStep;
+  // the loop once for scores that go to the exponent as they are and once for the others: both in one cost the
+  // first 32 moves a step
+  auto walk = [&](auto scaled_late) {
+  constexpr bool kLate = decltype(scaled_late)::value;
   for (int it = 0; it < steps; ++it) {
     const int u0 = it * kStep + kg * kKeys;
     // the builtin and not asm: the compiler then knows that the query rows have arrived, and does not wait for
@@ -657,130 +770,144 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
     __builtin_amdgcn_s_waitcnt(0x0f70);                // vmcnt(0)
     asm volatile("" ::: "memory");
     __syncthreads();
-    // ahead of the next DMA, whose end the use of a loaded block id would otherwise wait for
-    // (rows of tile `it` were read ahead of the barrier)
-    if (tid < kKeys) store_row(next, it & 1);
-    if (u0 + kStep < total) bring((it + 1) & 1);
-    if (tid < kKeys) next = look_up(u0 + 3 * kStep);
+    const int more = __builtin_amdgcn_readfirstlane(u0 + kStep < total), into = (it + 1) & 1;
+    slots_of(into);
     const unsigned char* k_lds = tiles + (it & 1) * STAGE;
     const unsigned char* v_lds = k_lds + KTILE;
-    // a tile with kept tokens ahead of the window concerns every row; of the others, a tile whose
-    // keys lie past this wave's last row, or before its first row's window (and are not kept ones),
-    // is none of its business
-    const bool kept_tile = u0 < nk;
-    const int j0 = u0 - nk + j_lo;            // the tile's first key when it holds window keys only
-    if (!active || u0 >= total || !(kept_tile || (j0 <= p0 + nq - 1 && !(j0 + kKeys - 1 < lo_first && j0 >= keep_first)))) continue;
+    // a tile that no row of this wave sees is none of its business
+    const bool concerned = active && u0 < total && u0 <= last_last && (u0 < kept || u0 + kKeys > least_first);
     f32x16 st[2];
+    if (concerned) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) st[kb][i] = 0.f;
-    // keys are read two steps ahead of their products, which the compiler would not do by itself
-    auto key_at = [&](int ks, int kb) {
-      const int slot = ((2 * ks) & ~KMASK) | (((2 * ks) & KMASK) ^ kx);
-      return *reinterpret_cast<const u32x4*>(k_lds + (32 * kb + c) * KB + 16 * slot);
-    };
-    u32x4 ka[3][2];
+        for (int i = 0; i < 16; ++i) st[kb][i] = 0.f;
+      // keys are read two steps ahead of their products, which the compiler would not do by itself, and the next
+      // tile's DMA goes out between the products: a burst of it holds a wave up for longer than half of them take
+      auto key_at = [&](int ks, int kb) {
+        const int piece = ((2 * ks) & ~KMASK) | (((2 * ks) & KMASK) ^ kx);
+        return *reinterpret_cast<const u32x4*>(k_lds + (32 * kb + c) * KB + 16 * piece);
+      };
+      u32x4 ka[3][2];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
+      for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) ka[ks][kb] = key_at(ks, kb);
+        for (int kb = 0; kb < 2; ++kb) ka[ks][kb] = key_at(ks, kb);
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      if (ks + 2 < D / 16) {
+      for (int ks = 0; ks < 2 * DB; ++ks) {
+        if (ks + 2 < 2 * DB) {
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) ka[(ks + 2) % 3][kb] = key_at(ks + 2, kb);
+          for (int kb = 0; kb < 2; ++kb) ka[(ks + 2) % 3][kb] = key_at(ks + 2, kb);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) st[kb] = M::run(ka[ks % 3][kb], qf[ks], st[kb]);
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i)
+          if (i * (2 * DB) / kPieces == ks) bring(i, into, more);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
+    } else {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) st[kb] = M::run(ka[ks % 3][kb], qf[ks], st[kb]);
+      for (int i = 0; i < kPieces; ++i) bring(i, into, more);
     }
-    if (softcap > 0.f) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) st[kb][i] = cap_score_fast(st[kb][i] * scale, cap2, cap_arg);
-    } else if (!late) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) st[kb][i] *= scale2;
+    if (w == 0) {
+      store_row(next, it & 1);                         // (the rows of tile `it` were read ahead of the barrier)
+      next = look_up(u0 + 3 * kStep);
     }
-    // Masks, only where some key of the tile is hidden from some row of the wave; rows behind the run's end (c >= nq)
-    // may see anything, nobody writes them.  A tile of 64 consecutive keys compares its 32 numbers, known when it is
-    // compiled, with one limit a lane; tiles with kept tokens work out every key.
-    if (kept_tile || j0 < keep_first) {
+    if (!concerned) continue;
+    // Values: a transposing read of the row-major tile.  A group of 16 lanes reads 4 keys x 16 dims, 8 bytes per
+    // lane (key i16 >> 2, dims 4 (i16 & 3) .. + 3), and every lane receives the four keys of dim i16 of the group.
+    u32x4 va[2][VB];
+    auto value_at = [&](int s4, int n) {               // keys 16 s4 .. + 15, dims 32 n ..
+      const unsigned char* at = v_lds + vat + 16 * s4 * VBYTES + 64 * (n ^ vf);
+      const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)at));
+      const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 8 * VBYTES)));
+      return u32x4{lo[0], lo[1], hi[0], hi[1]};
+    };
+#pragma unroll
+    for (int n = 0; n < VB; ++n) va[0][n] = value_at(0, n);
+    if constexpr (!kLate) {
+      if (softcap > 0.f) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) st[kb][i] = cap_score_fast(st[kb][i] * scale, cap2, cap_arg);
+      } else {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) st[kb][i] *= scale2;
+      }
+    }
+    // Masks, only where some key of the tile is hidden from some row of the wave, against numbers that are known when
+    // it is compiled; rows behind the run's end (c >= nq) may see anything, nobody writes them.
+    if (u0 + kKeys - 1 > last_first || (u0 < least_last && u0 + kKeys > kept)) {
+      const int last = last_q - u0 - 4 * hf, least = least_q - u0 - 4 * hf, held = kept - u0 - 4 * hf;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int j = key_of(u0 + 32 * kb + (i & 3) + 8 * (i >> 2) + 4 * hf);
-          st[kb][i] = j <= pq && (j >= lo_q || j < keep_first) ? st[kb][i] : -INFINITY;
+          const int e = 32 * kb + (i & 3) + 8 * (i >> 2);
+          st[kb][i] = e <= last && (e >= least || e < held) ? st[kb][i] : -INFINITY;
         }
-    } else {
-      if (j0 + kKeys - 1 > p0) {
-        const int last = pq - j0 - 4 * hf;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) st[kb][i] = 32 * kb + (i & 3) + 8 * (i >> 2) <= last ? st[kb][i] : -INFINITY;
-      }
-      if (j0 < lo_last) {
-        const int least = lo_q - j0 - 4 * hf;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) st[kb][i] = 32 * kb + (i & 3) + 8 * (i >> 2) >= least ? st[kb][i] : -INFINITY;
-      }
     }
-    float mt = -INFINITY;
+    float mts[2] = {-INFINITY, -INFINITY};             // chains of their own
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int i = 0; i < 16; ++i)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mt = fmaxf(mt, st[kb][i]);
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64)) * factor;
-    const float m_new = fmaxf(m, mt);
-    const float shift = m_new == -INFINITY ? 0.f : m_new;  // nothing seen yet: every weight is 2^-inf
-    const float corr = __builtin_amdgcn_exp2f(m - shift);
-    float psum = 0.f;
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kb][i], factor, -shift));
-        st[kb][i] = pv;
-        psum += pv;
-      }
-    l = l * corr + psum;            // this lane's keys; the partner's half is added at the end
-    if (__any(m_new != m)) {        // the running max of some row moved
+      for (int kb = 0; kb < 2; ++kb) mts[kb] = fmaxf(mts[kb], st[kb][i]);
+    const float mt = max_halves(fmaxf(mts[0], mts[1])) * (kLate ? scale2 : 1.f);
+    // The running maximum follows only where a row is more than kLag above it: weights stay below 2^kLag, which
+    // neither a 16-bit weight's rounding nor a sum in 32 bits feels, and most tiles leave the accumulators alone.
+    if (__any(mt > m + kLag)) {
+      const float m_new = fmaxf(m, mt);
+      top = m_new == -INFINITY ? 0.f : m_new;          // nothing seen yet: every weight is 2^-inf
+      const float corr = __builtin_amdgcn_exp2f(m - top);
+      l *= corr;
 #pragma unroll
       for (int n = 0; n < VB; ++n)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[n][i] *= corr;
+      m = m_new;
     }
-    m = m_new;
+    // weights 8 s4 .. + 7 of this lane; the partner's half of the sum is added at the end
+    auto weight2 = [&](int s4, int e) {
+      const float a0 = st[s4 >> 1][8 * (s4 & 1) + 2 * e];
+      const float b0 = st[s4 >> 1][8 * (s4 & 1) + 2 * e + 1];
+      const float a = __builtin_amdgcn_exp2f(kLate ? __builtin_fmaf(a0, scale2, -top) : a0 - top);
+      const float b = __builtin_amdgcn_exp2f(kLate ? __builtin_fmaf(b0, scale2, -top) : b0 - top);
+      l += a;
+      l += b;
+      return pack2<S>(a, b);
+    };
+    u32x4 pb[2];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int e = 0; e < 4; ++e) pb[0][e] = weight2(0, e);
+    // the next 16 keys' weights are formed between the products of these
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        u32x4 pb;
+    for (int s4 = 0; s4 < 4; ++s4) {
+      if (s4 < 3) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) pb[e] = pack2<S>(st[kb][8 * s2 + 2 * e], st[kb][8 * s2 + 2 * e + 1]);
-        // transposing read of the row-major tile: a group of 16 lanes reads 4 keys x 16 dims, 8
-        // bytes per lane (key i16 >> 2, dims 4 (i16 & 3) .. + 3), and every lane receives the four
-        // keys of dim i16 of the group
-        const unsigned char* src = v_lds + vat + (32 * kb + 16 * s2) * VBYTES;
-#pragma unroll
-        for (int n = 0; n < VB; ++n) {
-          const unsigned char* at = src + 64 * (n ^ vf);
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)at);
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 8 * VBYTES));
-          const u32x2 lo2 = __builtin_bit_cast(u32x2, lo), hi2 = __builtin_bit_cast(u32x2, hi);
-          const u32x4 a = {lo2[0], lo2[1], hi2[0], hi2[1]};
-          o[n] = M::run(a, pb, o[n]);
-        }
+        for (int n = 0; n < VB; ++n) va[(s4 + 1) & 1][n] = value_at(s4 + 1, n);
       }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < VB; ++n) {
+        o[n] = M::run(va[s4 & 1][n], pb[s4 & 1], o[n]);
+        if (s4 < 3) {
+#pragma unroll
+          for (int e = 4 * n / VB; e < 4 * (n + 1) / VB; ++e) pb[(s4 + 1) & 1][e] = weight2(s4 + 1, e);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
   }
+  };
+  if (late)
+    walk(std::true_type{});
+  else
+    walk(std::false_type{});
   if constexpr (KG == 2) {
     // the second group hands its sums over: registers lie lane for lane in the tiles' place
     __syncthreads();
@@ -1471,27 +1598,47 @@ int launch_heads_one(dim3 grid, hipStream_t stream, typename S::T* out, int64_t 
   return VLA_OK;
 }
 
+struct TileGrid {
+  int64_t tiles;        // ranked: at most this many tiles of rows; otherwise those of the longest sequence
+  int num_seqs, head_groups, key_groups;
+};
+
 template <class S, int DB, int VB>
-int launch_tiles_one(dim3 grid, hipStream_t stream, typename S::T* out, int64_t out_stride,
+int launch_tiles_one(TileGrid to, hipStream_t stream, typename S::T* out, int64_t out_stride,
                      const typename S::T* q, int64_t q_stride, const typename S::T* gate,
                      int64_t gate_stride, const typename S::T* key_cache,
                      const typename S::T* value_cache, const int* block_tables, int max_blocks,
                      const int* qsl, const int* ctx, const float* out_inv_freq, int interleaved,
                      int heads, int kv_heads, int block_size, int num_blocks, int window,
                      float scale, int head_waves, int keep_first, float softcap, int chunk,
-                     const float* sinks, int key_groups, int v_row, int v_first) {
+                     const float* sinks, int v_row, int v_first) {
+  auto go = [&](dim3 grid, int b0, int last_tile, int ranked_seqs, int first_rank) -> int {
+    auto* kernel = to.key_groups == 2 ? &kv_attention_tile_kernel<S, DB, VB, 2> : &kv_attention_tile_kernel<S, DB, VB, 1>;
+    kernel<<<grid, 256 * to.key_groups, 0, stream>>>(
+        out, out_stride, q, q_stride, gate, gate_stride, key_cache, value_cache, block_tables + (int64_t)b0 * max_blocks,
+        max_blocks, qsl + b0, ctx + b0, out_inv_freq, interleaved, heads, kv_heads, to.head_groups, block_size, num_blocks,
+        window, scale, head_waves, keep_first, softcap, chunk, sinks, v_row, v_first, last_tile, ranked_seqs, first_rank);
+    VLA_SEQ_HIP_CHECK(hipGetLastError());
+    return VLA_OK;
+  };
+  // a launch counts its threads in 32 bits: more than 16.7 million groups of heads go in several launches
+  const int64_t most = std::max(1, 0xffffff / (to.head_groups * to.key_groups));
+  if (to.num_seqs <= kRankedSeqs) {
+    for (int64_t r = 0; r < to.tiles; r += most) {
+      const int rc = go(dim3(to.head_groups * (unsigned)std::min(most, to.tiles - r)), 0, 0, to.num_seqs, (int)r);
+      if (rc != VLA_OK) return rc;
+    }
+    return VLA_OK;
+  }
   // grid: (sequences x groups of heads, row tiles); more tiles than a grid's second side takes go in several
   // launches, the last rows first
   constexpr int kSide = 65535;
-  for (int left = grid.y; left > 0; left -= kSide) {
-    const dim3 part(grid.x, left < kSide ? left : kSide);
-    auto* kernel = key_groups == 2 ? &kv_attention_tile_kernel<S, DB, VB, 2> : &kv_attention_tile_kernel<S, DB, VB, 1>;
-    kernel<<<part, 256 * key_groups, 0, stream>>>(
-        out, out_stride, q, q_stride, gate, gate_stride, key_cache, value_cache, block_tables,
-        max_blocks, qsl, ctx, out_inv_freq, interleaved, heads, kv_heads, (int)grid.z, block_size, num_blocks,
-        window, scale, head_waves, keep_first, softcap, chunk, sinks, v_row, v_first, left - 1);
-    VLA_SEQ_HIP_CHECK(hipGetLastError());
-  }
+  for (int64_t b0 = 0; b0 < to.num_seqs; b0 += most)
+    for (int left = (int)to.tiles; left > 0; left -= kSide) {
+      const dim3 grid(to.head_groups * (unsigned)std::min(most, to.num_seqs - b0), std::min(left, kSide));
+      const int rc = go(grid, (int)b0, left - 1, 0, 0);
+      if (rc != VLA_OK) return rc;
+    }
   return VLA_OK;
 }
 
@@ -1744,11 +1891,24 @@ extern "C" int vla_seq_kv_attention_tiles(
     int interleaved, int num_seqs, int max_query_len, int heads, int kv_heads, int dim, int vdim,
     int block_size, int num_blocks, int window, float scale, int dtype, int keep_first,
     float softcap, int chunk, const float* sinks, void* stream) {
+  return vla_seq_kv_attention_tiles_of(out, out_stride, q, q_stride, gate, gate_stride, key_cache, value_cache, block_tables,
+                                       max_blocks, query_start_loc, context_lens, out_inv_freq, interleaved, num_seqs,
+                                       max_query_len, (int64_t)num_seqs * max_query_len, heads, kv_heads, dim, vdim, block_size,
+                                       num_blocks, window, scale, dtype, keep_first, softcap, chunk, sinks, stream);
+}
+
+extern "C" int vla_seq_kv_attention_tiles_of(
+    void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* gate,
+    int64_t gate_stride, const void* key_cache, const void* value_cache, const int* block_tables,
+    int max_blocks, const int* query_start_loc, const int* context_lens, const float* out_inv_freq,
+    int interleaved, int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads, int dim, int vdim,
+    int block_size, int num_blocks, int window, float scale, int dtype, int keep_first,
+    float softcap, int chunk, const float* sinks, void* stream) {
   if (num_seqs == 0 || max_query_len == 0) return VLA_OK;
   if (keep_first < 0 || !(softcap >= 0.f)) return VLA_ERR_ARG;
   if (window <= 0 && chunk <= 0) keep_first = 0;
   if (!out || !q || !key_cache || !value_cache || !block_tables || !query_start_loc || !context_lens ||
-      num_seqs < 0 || num_seqs > 65535 || max_query_len < 0 || heads <= 0 || kv_heads <= 0 ||
+      num_seqs < 0 || num_seqs > 65535 || max_query_len < 0 || num_rows < 0 || heads <= 0 || kv_heads <= 0 ||
       heads % kv_heads != 0 || block_size <= 0 || num_blocks <= 0 || max_blocks <= 0 ||
       out_stride < (int64_t)heads * vdim || q_stride < (int64_t)heads * dim ||
       (gate && gate_stride < heads))
@@ -1767,29 +1927,21 @@ extern "C" int vla_seq_kv_attention_tiles(
   const int head_waves = group >= 3 ? 4 : group;      // waves of a workgroup that are heads
   const int tile_rows = kTile * (4 / head_waves);
   const int head_groups = kv_heads * ((group + head_waves - 1) / head_waves);
-  // (the launch counts every sequence as long as the longest: a prompt beside many single rows keeps one group)
-  // few workgroups share their keys out to two groups of four waves: of 2047 rows, 16 heads on 4 of 128, one run
-  // (256 workgroups) takes 68 us instead of 88, two take 76 instead of 100; four fill the chip with independent
-  // ones (116 instead of 138: two workgroups of a CU do not wait for each other)
-  const int64_t workgroups = (int64_t)head_groups * num_seqs * ((max_query_len + tile_rows - 1) / tile_rows);
-  const int key_groups = workgroups <= 512 ? 2 : 1;
-  // a launch counts its threads in 32 bits: more than 16.7 million groups of heads go in several launches
-  const int most = std::max(1, 0xffffff / head_groups);
+  // few workgroups share their keys out to two groups of four waves, one workgroup a CU: of 16 heads on 4 of 128, a run
+  // of 2047 rows (256 workgroups) takes 41 us instead of 49, runs of 2047 and 1265 45 instead of 55, of 4096 rows (512) 95
+  // instead of 109; 700 workgroups fill the chip with independent ones (62 instead of 73 us)
+  const int64_t of_longest = (max_query_len + tile_rows - 1) / tile_rows;
+  const int64_t tiles = std::min(num_seqs * of_longest, num_rows / tile_rows + num_seqs);     // of all sequences, at most
+  const int key_groups = head_groups * tiles <= 512 ? 2 : 1;
+  const TileGrid to{num_seqs <= kRankedSeqs ? tiles : of_longest, num_seqs, head_groups, key_groups};
   auto go = [&](auto tag) {
     using S = decltype(tag);
     using T = typename S::T;
     return by_value_slices(vdim, [&](int vb, int v_first) -> int {
-      for (int b0 = 0; b0 < num_seqs; b0 += most) {
-        const dim3 grid(head_groups * std::min(most, num_seqs - b0), (max_query_len + tile_rows - 1) / tile_rows, head_groups);
-        const int rc = launch_tiles<S>(
-                             dim / 32, vb, grid, (hipStream_t)stream, (T*)out, out_stride, (const T*)q, q_stride,
-                             (const T*)gate, gate_stride, (const T*)key_cache, (const T*)value_cache,
-                             block_tables + (int64_t)b0 * max_blocks, max_blocks, query_start_loc + b0, context_lens + b0, out_inv_freq,
-                             interleaved, heads, kv_heads, block_size, num_blocks, window, scale,
-                             head_waves, keep_first, softcap, chunk, sinks, key_groups, vdim, v_first);
-        if (rc != VLA_OK) return rc;
-      }
-      return VLA_OK;
+      return launch_tiles<S>(dim / 32, vb, to, (hipStream_t)stream, (T*)out, out_stride, (const T*)q, q_stride,
+                             (const T*)gate, gate_stride, (const T*)key_cache, (const T*)value_cache, block_tables,
+                             max_blocks, query_start_loc, context_lens, out_inv_freq, interleaved, heads, kv_heads,
+                             block_size, num_blocks, window, scale, head_waves, keep_first, softcap, chunk, sinks, vdim, v_first);
     });
   };
   return dtype == VLA_BF16 ? go(BF16{}) : go(F16{});
