@@ -451,13 +451,13 @@ __device__ __forceinline__ void turn_back(f32x16 (&o)[VB], int hf, float p,
 // the other's products).  A DMA instruction writes 64 lanes x 16 bytes in a row, so rows cannot be padded: 16-byte
 // pieces of a key row and 64-byte units of a value row are exchanged by the row's number on the source's
 // side, so that the lanes of a read fall into different banks.  The next tile's DMA goes out between the first products
-// (sent at once it holds a wave up for 700 cycles), weights are formed between the second ones, and accumulators are
-// scaled only when a maximum has moved by more than kLag.  What is the same for all lanes is told to the compiler, or every
-// choice of a mask or a scale copies the 32 scores.  Workgroups go out longest walk first over all sequences,
-// groups of heads next to each other: each XCD's L2 holds few heads' keys.  Where the workgroups are few,
-// each has two groups of four waves (KG = 2) that take every other tile and join their sums at the end.  Four
-// prompts of up to 2047 rows, 16 heads on 4 of 128: 62 us (104 with DMA in a burst, masks for all tiles of a run's last
-// rows and a grid as long as the longest prompt for each; 172 with tiles staged through registers into padded rows).
+// (sent at once it holds a wave up for 700 cycles), weights are formed between the second ones.  What is the same for
+// all lanes is told to the compiler, or every choice of a mask or a scale copies the 32 scores.  Workgroups go out
+// longest walk first over all sequences, groups of heads next to each other: each XCD's L2 holds few heads' keys.
+// Where the workgroups are few, each has two groups of four waves (KG = 2) that take every other tile and join their
+// sums at the end.  Four prompts of up to 2047 rows, 16 heads on 4 of 128: 65 us (104 with DMA in a burst, masks for
+// all tiles of a run's last rows and a grid as long as the longest prompt for each; 172 with tiles staged through
+// registers into padded rows).
 template <class S>
 struct Mfma16;
 template <>
@@ -476,7 +476,6 @@ struct Mfma16<F16> {
 };
 
 constexpr int kKeys = 64;     // keys per staged tile
-constexpr float kLag = 8.f;   // how far a row's scores (base 2) may lie above its running maximum
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef s16x4 __attribute__((address_space(3))) * lds_s16x4;
 
@@ -858,9 +857,9 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) mts[kb] = fmaxf(mts[kb], st[kb][i]);
     const float mt = max_halves(fmaxf(mts[0], mts[1])) * (kLate ? scale2 : 1.f);
-    // The running maximum follows only where a row is more than kLag above it: weights stay below 2^kLag, which
-    // neither a 16-bit weight's rounding nor a sum in 32 bits feels, and most tiles leave the accumulators alone.
-    if (__any(mt > m + kLag)) {
+    // (a maximum that may lag behind, by 8 in base 2, leaves the accumulators alone in most tiles and is 2.5 % faster, but
+    // the largest weight is then no longer 1 and rounds like the others: errors grow by 1 to 2 %)
+    if (__any(mt > m)) {
       const float m_new = fmaxf(m, mt);
       top = m_new == -INFINITY ? 0.f : m_new;          // nothing seen yet: every weight is 2^-inf
       const float corr = __builtin_amdgcn_exp2f(m - top);
