@@ -219,6 +219,22 @@ def test_rows_that_do_not_see_one_that_is_not_finite(row, window, value):
     assert torch.equal(got[~sees], clean[~sees]) and not got[sees].isfinite().any()
 
 
+@pytest.mark.parametrize("seqs", [1, 40, 65, 130, 256, 257, 300])
+@pytest.mark.parametrize("window", [0, 90])
+def test_one_group_of_waves_and_two(seqs, window):
+    """Many workgroups have one group of waves and find their tiles by their rank (up to 256 sequences) or by the grid;
+    a small workspace makes few of them, which share a tile's keys out to two groups: one rounding of an output."""
+    lens, contexts = [129 + 11 * (i % 13) for i in range(seqs)], [7 * (i % 9) for i in range(seqs)]
+    sizes = (4, 128, 64, 128, 128)
+    attn, batch, q, kv, gate, cache = layer_and_step(lens, contexts, sizes, window)
+    assert (4 * ((sum(lens) + sum(contexts)) // 128 + seqs) > 512) == (seqs > 40)
+    want = attn(q.clone(), kv, cache.clone(), batch, gate)
+    attn.FORMED_WORKSPACE = 2048 * 2 * (128 + 64 + 4 * 384)
+    got = attn(q.clone(), kv, cache.clone(), batch, gate)
+    assert float((got - want).abs().max()) <= 0.008 * float(want.abs().max())
+    assert float(want.abs().max()) > 0.1 and bool(want.isfinite().all())
+
+
 def test_lengths_that_are_not_the_hosts():
     """Rows of a sequence that grew on the device are NaN, not what memory held; a captured step takes the latent
     kernel, which follows the device."""

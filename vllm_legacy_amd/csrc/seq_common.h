@@ -120,6 +120,105 @@ __device__ __forceinline__ f32x4 load4(const typename S::T* row, int d, int dim,
   return r;
 }
 
+// 16 bytes per lane from each lane's own address into 1 KB of LDS (no register result), where `go`: a branch that the
+// compiler does not see, so that the products around it stay one block
+__device__ __forceinline__ void tile_dma16(const void* src, uint32_t lds_at, int go) {
+  unsigned keep;
+  asm volatile(
+      "s_cmp_lg_u32 %3, 0\n\ts_cbranch_scc0 1f\n\ts_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0\n1:"
+      : "=&s"(keep)
+      : "v"(src), "s"(lds_at), "s"(__builtin_amdgcn_readfirstlane(go))
+      : "memory", "scc");
+}
+
+// the larger of a lane's value and that of the lane 32 further on
+__device__ __forceinline__ float max_halves(float v) {
+  const uint32_t x = __builtin_bit_cast(uint32_t, v);
+  const auto both = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)both[0]), __builtin_bit_cast(float, (uint32_t)both[1]));
+}
+
+// the sum over a wave, in every lane
+__device__ __forceinline__ int wave_total(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);      // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);     // row_bcast 15 to rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);     // row_bcast 31 to rows 2 and 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// The `rank`-th of all tiles of 2^shift rows of a step's sequences, counted from those that walk the most keys (a
+// tile's level: how many tiles of keys lie ahead of its last row).  Every wave finds it for itself: a search over
+// the levels for the one whose tiles hold the rank, with the sequences in the lanes' registers.  Launching one
+// workgroup per tile of the longest sequence for every sequence instead left empty ones between the real ones:
+// workgroups go to the shader engines of an XCD in turn, an engine that is full holds all others up, and half the
+// chip stood idle for 40 of 98 us with four prompts of 2047, 1265, 483 and 1748 rows.  The search takes about 2 us
+// of a workgroup.  Returns the number of tiles; seq and tile are set
+// where the rank is below it.
+constexpr int kRankedChunks = 4;
+constexpr int kRankedSeqs = kRankedChunks * kWave;
+__device__ __forceinline__ int ranked_tile(int rank, int num_seqs, const int* __restrict__ query_start_loc,
+                                            const int* __restrict__ context_lens, int shift, int& seq, int& tile) {
+  const int lane = threadIdx.x & 63, chunks = (num_seqs + kWave - 1) / kWave;
+  int first[kRankedChunks], end[kRankedChunks];       // the levels of a sequence's tiles
+  int top = 0, all = 0;
+#pragma unroll
+  for (int k = 0; k < kRankedChunks; ++k) {
+    first[k] = end[k] = 0;
+    if (k < chunks) {
+      const int s = k * kWave + lane;
+      if (s < num_seqs) {
+        first[k] = context_lens[s] >> shift;
+        end[k] = first[k] + ((max(query_start_loc[s + 1] - query_start_loc[s], 0) + (1 << shift) - 1) >> shift);
+      }
+      all += end[k] - first[k];
+      top = max(top, end[k]);
+    }
+  }
+  all = wave_total(all);
+  if (all <= rank) return all;
+#pragma unroll
+  for (int x = 1; x < kWave; x <<= 1) top = max(top, __shfl_xor(top, x, 64));
+  auto at_least = [&](int level) {                     // tiles of this level and above
+    int n = 0;
+#pragma unroll
+    for (int k = 0; k < kRankedChunks; ++k)
+      if (k < chunks) n += max(end[k] - max(first[k], level), 0);
+    return wave_total(n);
+  };
+  int lo = 0, hi = __builtin_amdgcn_readfirstlane(top), above = 0;      // at_least(lo) > rank >= at_least(hi) = above
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1, n = at_least(mid);
+    if (n > rank) {
+      lo = mid;
+    } else {
+      hi = mid;
+      above = n;
+    }
+  }
+  int left = rank - above;
+#pragma unroll
+  for (int k = 0; k < kRankedChunks; ++k)
+    if (k < chunks && left >= 0) {
+      const bool here = first[k] <= lo && lo < end[k];
+      const uint64_t mask = __ballot(here);
+      const int n = __popcll(mask);
+      if (left < n) {
+        const uint64_t which = __ballot(here && __popcll(mask & ((1ull << lane) - 1)) == left);
+        const int l = __ffsll((unsigned long long)which) - 1;
+        seq = k * kWave + l;
+        tile = lo - __builtin_amdgcn_readlane(first[k], l);
+      }
+      left -= n;
+    }
+  seq = __builtin_amdgcn_readfirstlane(seq);
+  tile = __builtin_amdgcn_readfirstlane(tile);
+  return all;
+}
+
 __device__ __forceinline__ bool finite(float x) { return fabsf(x) <= 3.402823466e38f; }
 
 __device__ __forceinline__ float softplusf(float z) { return z > 20.f ? z : log1pf(expf(z)); }

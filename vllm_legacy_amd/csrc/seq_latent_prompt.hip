@@ -5,7 +5,7 @@
 // queries of the run.  A run of rows therefore gathers its visible cache rows into one place
 // (latent_gather_kernel), the caller multiplies them with the two up-projections, and
 // latent_prompt_kernel below is plain causal attention with keys [formed (dim) | shared rotated part
-// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 184 us (470 TFLOP/s; 650
+// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 148 us (580 TFLOP/s; 810
 // with the remainders' product) where latent_attention_tile_kernel takes 1685, plus 9 us to gather and 60 for the
 // three products (the products on the query's side that they replace take 46).
 //
@@ -13,7 +13,7 @@
 // side, which is the same for all keys of a row and mostly cancels in the softmax; a key's rounding is its own.
 // Outputs' error against 64 bits, this / one 16-bit number / the latent kernel, bf16, 1e-3: independent latents
 // 2.5 / 2.8 / 2.8, with scores four times as large 2.4 / 3.8 / 3.6 (float16: an eighth of each).  One number
-// per key takes 136 us, and 189 instead of 257 for the whole layer.
+// per key took 136 us when two took 184.
 //
 // The rows of sequence b are its keys from first_b = max(0, context - window + 1) (0 without a window) to
 // its last new row; sequences follow each other, so a sequence's place is the sum of the counts before
@@ -26,9 +26,16 @@
 // Tiles come in by LDS-DMA, keys and values in turn (one tile of each in LDS: 56 KB), without staging registers.  A DMA
 // instruction writes 64 lanes x 16 bytes in a row, so rows cannot be padded; 16-byte pieces (values:
 // 64-byte ones) are exchanged within a row by the row's number instead, on the source's side, so that
-// the lanes of a read fall into different banks.  Two workgroups share a CU: one's softmax (about 30
-// vector cycles per score) runs under the other's products.  Workgroups of one head are 8 apart or a
-// multiple of it when heads are a multiple of 8, so they share an XCD's L2 for that head's keys.
+// the lanes of a read fall into different banks.  DMA goes out between the products, a value tile's between the first
+// ones and a key tile's ahead of and between the second ones, and weights are formed between those (184 us and bursts
+// behind the barriers before).
+//
+// Workgroups go out longest walk first over all sequences (ranked_tile), heads next to each other.  Up to 512 of
+// them have two groups of four waves, a CU each, that take every other tile and join their sums at the end: with
+// one group, two workgroups to a CU, all 512 of a run of 4096 rows are on the chip at once and the ones with 64 tiles
+// stay alone on their CUs (168 us; 2048 rows 72 instead of 60).  A wave alone takes 4400 cycles for a tile, 1800 of
+// products; two on a SIMD 6300 for one each, at 1.6 GHz, where the card holds its power.  Taken back: the second group
+// half a step behind the first (with two tiles of values: 157), raised priority for the first product (162).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -42,7 +49,9 @@ namespace {
 constexpr int kKeys = 64;           // keys of a tile
 constexpr int kRowsPerWave = 32;
 constexpr int kWaves = 4;
-constexpr int kRowsPerGroup = kRowsPerWave * kWaves;
+constexpr int kRowsPerGroup = kRowsPerWave * kWaves, kGroupShift = 7;
+static_assert(kRowsPerGroup == 1 << kGroupShift, "tiles of rows are ranked by their level");
+constexpr int kEarly = 4;           // a wave's DMA instructions for the next keys ahead of the softmax
 constexpr int kGatherRows = 32;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef s16x4 __attribute__((address_space(3))) * lds_s16x4;
@@ -131,25 +140,16 @@ struct LatentPrompt {
   const float* sinks;
   float* carry;                 // one sequence whose keys come in ranges: [T, heads, VD + 4], null otherwise
   int heads, dim, rot, vdim, rank, window, num_rows, row_tiles;
+  int ranked_seqs, tiles;       // ranked_seqs > 0: tiles are found by their rank, `tiles` of them are launched
   int key_first, key_total;     // the range's first key and all keys of the sequence
   float scale;
 };
 
-// 16 bytes per lane from each lane's own address into 1 KB of LDS (no register result)
-__device__ __forceinline__ void dma16(const void* src, uint32_t lds_at) {
-  unsigned keep;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-      : "=&s"(keep)
-      : "v"(src), "s"(lds_at)
-      : "memory");
-}
-
 // for pieces of LDS rows behind a row's end
 __device__ const u32x4 kNothing = {0u, 0u, 0u, 0u};
 
-template <class S, int DB, int VB, int LB>
-__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
+template <class S, int DB, int VB, int LB, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void latent_prompt_kernel(LatentPrompt a) {
   using T = typename S::T;
   using M = Mma<S>;
   constexpr int DQ = 32 * DB, VD = 32 * VB, LD = 32 * LB;
@@ -159,13 +159,18 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
   // a key row is a whole number of 256 bytes (all 64 banks), or half of one more: which pieces change place
   constexpr int KMASK = KB % 256 == 0 ? 15 : 7, KSHIFT = KB % 256 == 0 ? 0 : 1;
   constexpr int RMASK = RB % 256 == 0 ? 15 : 7, RSHIFT = RB % 256 == 0 ? 0 : 1;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int h = blockIdx.x, b = blockIdx.z;
+  constexpr int kStep = kKeys * KG;                        // keys of a step: a tile for every group of four waves
+  extern __shared__ __align__(16) unsigned char all_tiles[];
+  const int h = blockIdx.x % a.heads;
+  auto one_tile = [&](int b, int tile) __attribute__((always_inline)) {
   const int run = a.query_start_loc[b + 1] - a.query_start_loc[b];
-  const int tile = a.row_tiles - 1 - (int)blockIdx.y;       // the longest walks first
   const int r0 = tile * kRowsPerGroup;
   if (r0 >= run) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));        // what follows from it is not kept over the loop around a tile
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);     // group of waves
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane((tid & 255) >> 6);
+  unsigned char* smem = all_tiles + kg * (KTILE + RTILE + VTILE);
   const int hf = lane >> 5, c = lane & 31;
   const bool ranged = a.carry != nullptr, last_range = !ranged || a.key_first + a.num_rows == a.key_total;
   const int ctx = a.context_lens[b], first = first_formed(ctx, a.window) + (ranged ? a.key_first : 0);
@@ -207,12 +212,12 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
     for (int i = 0; i < 16; ++i) o[n][i] = 0.f;
   const float scale2 = a.scale * 1.4426950408889634f;      // scores in base 2; scale > 0
   float m = -INFINITY, l = 0.f;
-  if (a.sinks != nullptr) {                                // the denominator's first term, counted in one lane half
+  if (a.sinks != nullptr && kg == 0) {                     // the denominator's first term, counted in one lane half
     m = a.sinks[h] * 1.4426950408889634f;
     l = hf == 0 ? 1.f : 0.f;
   }
   float* carry = a.carry + ((int64_t)(t0 + c) * a.heads + h) * (VD + 4);
-  if (ranged && a.key_first > 0 && c < nq) {               // where the range before this one ended
+  if (ranged && a.key_first > 0 && c < nq && kg == 0) {               // where the range before this one ended
     m = carry[0];
     l = carry[1 + hf];
 #pragma unroll
@@ -227,12 +232,13 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
 
   // What this lane brings in: piece `at` of a tile in LDS is row at / pieces; which 16 bytes of the row
   // stand there follows from the exchange.  Pieces past the end of a key are zeros; those past a value's repeat its
-  // first ones, for columns nobody writes.
-  const unsigned char *src_k[KI], *src_r[RI], *src_v[VI];
-  int row_k[KI], row_r[RI], row_v[VI];
-  unsigned step_k[KI], step_r[RI];
-  const unsigned key_row = (unsigned)a.heads * a.dim * 2, value_row = (unsigned)a.heads * a.vdim * 2;
-  const unsigned lat_row = (unsigned)(a.rank + a.rot) * 2;
+  // first ones, for columns nobody writes.  The first KI pieces are the keys', the next RI what rounding took.
+  constexpr int kKeyPieces = KI + RI;
+  const unsigned char* from_k[kKeyPieces];                  // where the piece of the first tile lies
+  int row_k[kKeyPieces];
+  int step_k[kKeyPieces];
+  const int key_row = a.heads * a.dim * 2, value_row = a.heads * a.vdim * 2;
+  const int lat_row = (a.rank + a.rot) * 2;
   const int64_t first_key = (int64_t)base * key_row + (int64_t)h * a.dim * 2;
 #pragma unroll
   for (int u = 0; u < KI; ++u) {
@@ -240,44 +246,36 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
     const int piece = (s & ~KMASK) | ((s ^ (r >> KSHIFT)) & KMASK);
     const int d = 8 * piece;
     row_k[u] = r;
-    src_k[u] = d < a.dim ? (const unsigned char*)a.keys + first_key + 2 * d
-                         : (const unsigned char*)a.rows + (int64_t)base * lat_row + (a.rank + d - a.dim) * 2;
-    step_k[u] = d < a.dim ? key_row : lat_row;
-    if (d >= width) {
-      src_k[u] = (const unsigned char*)&kNothing;
-      step_k[u] = 0;
-    }
+    step_k[u] = d < a.dim ? key_row : d < width ? lat_row : 0;
+    from_k[u] = d < a.dim   ? (const unsigned char*)a.keys + first_key + 2 * d
+                : d < width ? (const unsigned char*)a.rows + (int64_t)base * lat_row + (a.rank + d - a.dim) * 2
+                            : (const unsigned char*)&kNothing;
+    from_k[u] += (int64_t)r * step_k[u];
   }
 #pragma unroll
   for (int u = 0; u < RI; ++u) {
     const int at = ((w * RI + u) * 1024 + 16 * lane) / 16, r = at / (RB / 16), s = at % (RB / 16);
     const int piece = (s & ~RMASK) | ((s ^ (r >> RSHIFT)) & RMASK);
     const int d = 8 * piece;
-    row_r[u] = r;
-    src_r[u] = d < a.dim ? (const unsigned char*)a.keys_rest + first_key + 2 * d : (const unsigned char*)&kNothing;
-    step_r[u] = d < a.dim ? key_row : 0;
+    row_k[KI + u] = r;
+    step_k[KI + u] = d < a.dim ? key_row : 0;
+    from_k[KI + u] = d < a.dim ? (const unsigned char*)a.keys_rest + first_key + 2 * d : (const unsigned char*)&kNothing;
+    from_k[KI + u] += (int64_t)r * step_k[KI + u];
   }
-#pragma unroll
-  for (int u = 0; u < VI; ++u) {
-    const int at = ((w * VI + u) * 1024 + 16 * lane) / 16, r = at / (VBYTES / 16), s = at % (VBYTES / 16);
-    const int f = VB == 4 ? r & 3 : (r >> 1) & (VB - 1);
-    const int d = 8 * ((((s >> 2) ^ f) << 2) | (s & 3));
-    row_v[u] = r;
-    src_v[u] = (const unsigned char*)a.values + (int64_t)base * value_row + ((int64_t)h * a.vdim + (d < a.vdim ? d : 0)) * 2;
-  }
+  // (a value row's pieces come in at the same places for every instruction, kValueRows rows further on)
+  constexpr int kValueRows = 1024 / VBYTES;
+  const int row_v = w * VI * kValueRows + lane / (VBYTES / 16), unit_v = VB == 4 ? row_v & 3 : (row_v >> 1) & (VB - 1);
+  const int sv = lane % (VBYTES / 16), dv = 8 * ((((sv >> 2) ^ unit_v) << 2) | (sv & 3));
+  const unsigned char* from_v = (const unsigned char*)a.values + (int64_t)(base + row_v) * value_row +
+                                ((int64_t)h * a.vdim + (dv < a.vdim ? dv : 0)) * 2;
   const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
-  auto bring_keys = [&](int u0) {
-#pragma unroll
-    for (int u = 0; u < KI; ++u)
-      dma16(src_k[u] + (uint64_t)(unsigned)min(u0 + row_k[u], n_keys - 1) * step_k[u], lds0 + (w * KI + u) * 1024);
-#pragma unroll
-    for (int u = 0; u < RI; ++u)
-      dma16(src_r[u] + (uint64_t)(unsigned)min(u0 + row_r[u], n_keys - 1) * step_r[u], lds0 + KTILE + (w * RI + u) * 1024);
+  // piece i of the tile that begins with key u0; behind the end the last key again
+  auto bring_key = [&](int i, int u0, int go) {
+    tile_dma16(from_k[i] + (int64_t)min(u0, n_keys - 1 - row_k[i]) * step_k[i],
+               lds0 + (i < KI ? (w * KI + i) * 1024 : KTILE + (w * RI + i - KI) * 1024), go);
   };
-  auto bring_values = [&](int u0) {
-#pragma unroll
-    for (int u = 0; u < VI; ++u)
-      dma16(src_v[u] + (uint64_t)(unsigned)min(u0 + row_v[u], n_keys - 1) * value_row, lds0 + KTILE + RTILE + (w * VI + u) * 1024);
+  auto bring_value = [&](int i, int u0, int go) {
+    tile_dma16(from_v + (int64_t)min(u0 + i * kValueRows, n_keys - 1 - row_v) * value_row, lds0 + KTILE + RTILE + (w * VI + i) * 1024, go);
   };
   // where this lane reads: the exchanged piece of its key row, and the unit of its value rows
   const int kx = (hf ^ ((c >> KSHIFT) & KMASK)) & KMASK;   // piece 2 ks + hf stands at 2 ks ^ kx within its group
@@ -299,42 +297,57 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
     asm volatile("" ::: "memory");
     __syncthreads();
   };
-  int u0 = g_first & ~(kKeys - 1);
-  if (u0 <= p_end) bring_keys(u0);
-  for (; u0 <= p_end; u0 += kKeys) {
+  int u0 = (g_first & ~(kKeys - 1)) + kg * kKeys;
+  float top = m == -INFINITY ? 0.f : m;                    // m, and 0 where nothing was seen yet
+  if (u0 <= p_end)
+#pragma unroll
+    for (int i = 0; i < kKeyPieces; ++i) bring_key(i, u0, 1);
+  for (; u0 - kg * kKeys <= p_end; u0 += kStep) {
     landed();
-    bring_values(u0);
-    const bool concerned = nq > 0 && u0 <= p0 + nq - 1 && u0 + kKeys > lo_first;     // some key of it concerns this wave
+    const bool concerned = nq > 0 && u0 <= p_end && u0 <= p0 + nq - 1 && u0 + kKeys > lo_first;     // some key of it concerns this wave
     f32x16 st[2];
     if (concerned) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) st[kb][i] = 0.f;
+      // keys are read two steps ahead of their products, and the values' DMA goes out between the products
+      constexpr int kSteps = (DQ + LD) / 16;
+      auto key_at = [&](int ks, int kb) {
+        const int k = ks < DQ / 16 ? ks : ks - DQ / 16;
+        const int slot = ks < DQ / 16 ? ((2 * k) & ~KMASK) | (((2 * k) & KMASK) ^ kx) : ((2 * k) & ~RMASK) | (((2 * k) & RMASK) ^ rx);
+        return *reinterpret_cast<const u32x4*>((ks < DQ / 16 ? k_lds + (32 * kb + c) * KB : r_lds + (32 * kb + c) * RB) + 16 * slot);
+      };
+      u32x4 ka[3][2];
 #pragma unroll
-      for (int ks = 0; ks < DQ / 16; ++ks)
+      for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-          const int slot = ((2 * ks) & ~KMASK) | (((2 * ks) & KMASK) ^ kx);
-          const u32x4 ka = *reinterpret_cast<const u32x4*>(k_lds + (32 * kb + c) * KB + 16 * slot);
-          st[kb] = M::run(ka, qf[ks], st[kb]);
+        for (int kb = 0; kb < 2; ++kb) ka[ks][kb] = key_at(ks, kb);
+#pragma unroll
+      for (int ks = 0; ks < kSteps; ++ks) {
+        if (ks + 2 < kSteps) {
+#pragma unroll
+          for (int kb = 0; kb < 2; ++kb) ka[(ks + 2) % 3][kb] = key_at(ks + 2, kb);
         }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ks = 0; ks < LD / 16; ++ks)
+        for (int kb = 0; kb < 2; ++kb) st[kb] = M::run(ka[ks % 3][kb], qf[ks < DQ / 16 ? ks : ks - DQ / 16], st[kb]);
+        if (ks < VI) bring_value(ks, u0, 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-          const int slot = ((2 * ks) & ~RMASK) | (((2 * ks) & RMASK) ^ rx);
-          const u32x4 ra = *reinterpret_cast<const u32x4*>(r_lds + (32 * kb + c) * RB + 16 * slot);
-          st[kb] = M::run(ra, qf[ks], st[kb]);
-        }
+      for (int i = 0; i < VI; ++i) bring_value(i, u0, u0 <= p_end);
     }
     landed();
-    if (u0 + kKeys <= p_end) bring_keys(u0 + kKeys);
+    const int more = u0 + kStep <= p_end;
+#pragma unroll
+    for (int i = 0; i < kEarly; ++i) bring_key(i, u0 + kStep, more);
     // A hidden key's weight is 0, which times an infinity or a NaN would not be: a tile that hides keys from some row
     // goes without values that are not finite.  Rows that see such a key are NaN by their scores: a key of the same
     // latent is not finite either, and it and what it lost to rounding never sum to a number (finite latents give finite
     // values: the layer looks at its weights for that).
-    if (u0 + kKeys - 1 > g_p0 || u0 < g_lo_last) {
+    if (u0 + (KG - kg) * kKeys - 1 > g_p0 || u0 - kg * kKeys < g_lo_last) {      // (the same for both groups: a barrier)
 #pragma unroll
       for (int u = 0; u < VI; ++u) {
         u32x4* at = reinterpret_cast<u32x4*>(smem + KTILE + RTILE + (w * VI + u) * 1024 + 16 * lane);
@@ -350,61 +363,104 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
       }
       __syncthreads();
     }
-    if (!concerned) continue;
-    // every key of the tile visible to every row of the wave: no masks
-    if (!(u0 + kKeys - 1 <= p0 && u0 >= lo_last && nq == kRowsPerWave)) {
+    if (!concerned) {
+#pragma unroll
+      for (int i = kEarly; i < kKeyPieces; ++i) bring_key(i, u0 + kStep, more);
+      continue;
+    }
+    // Values: transposing reads, the first 16 keys' under the softmax
+    u32x4 va[VB];
+    auto value_at = [&](int s4, int n) {                   // keys 16 s4 .. + 15, dims 32 n ..
+      // 8 rows further on the exchange is the same for four units; for two it is too (8 / 2 even)
+      const unsigned char* at = v_lds + vat + 16 * s4 * VBYTES + 64 * (n ^ vf);
+      const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)at));
+      const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 8 * VBYTES)));
+      return u32x4{lo[0], lo[1], hi[0], hi[1]};
+    };
+#pragma unroll
+    for (int n = 0; n < VB; ++n) va[n] = value_at(0, n);
+    // masks only where some key of the tile is hidden from some row of the wave; nobody writes the rows behind the run's end
+    if (u0 + kKeys - 1 > p0 || u0 < lo_last) {
+      const int least = lo_q - u0 - 4 * hf;
+      const uint32_t seen = max(pq - lo_q + 1, 0);        // (rows ahead of a range of keys see none)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int j = u0 + 32 * kb + (i & 3) + 8 * (i >> 2) + 4 * hf;
-          st[kb][i] = c < nq && j <= pq && j >= lo_q ? st[kb][i] : -INFINITY;
-        }
+        for (int i = 0; i < 16; ++i)
+          st[kb][i] = (uint32_t)(32 * kb + (i & 3) + 8 * (i >> 2) - least) < seen ? st[kb][i] : -INFINITY;
     }
-    float mt = -INFINITY;
+    float mts[2] = {-INFINITY, -INFINITY};                 // chains of their own
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int i = 0; i < 16; ++i)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mt = fmaxf(mt, st[kb][i]);
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64)) * scale2;
-    const float m_new = fmaxf(m, mt);
-    const float shift = m_new == -INFINITY ? 0.f : m_new;  // nothing seen yet: every weight is 2^-inf
-    const float corr = __builtin_amdgcn_exp2f(m - shift);
-    float psum = 0.f;
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kb][i], scale2, -shift));
-        st[kb][i] = pv;
-        psum += pv;
-      }
-    l = l * corr + psum;                                   // this lane's keys; the partner's half is added at the end
-    if (__any(m_new != m)) {                               // the running maximum of some row moved
+      for (int kb = 0; kb < 2; ++kb) mts[kb] = fmaxf(mts[kb], st[kb][i]);
+    const float mt = max_halves(fmaxf(mts[0], mts[1])) * scale2;
+    // (a maximum that may lag behind, by 8 in base 2, leaves the accumulators alone in most tiles and is 2.5 % faster, but
+    // the largest weight is then no longer 1 and rounds like the others: errors grow by 1 to 2 %)
+    if (__any(mt > m)) {
+      const float m_new = fmaxf(m, mt);
+      top = m_new == -INFINITY ? 0.f : m_new;              // nothing seen yet: every weight is 2^-inf
+      const float corr = __builtin_amdgcn_exp2f(m - top);
+      l *= corr;
 #pragma unroll
       for (int n = 0; n < VB; ++n)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[n][i] *= corr;
+      m = m_new;
     }
-    m = m_new;
+    // weights 8 s4 .. + 7 of this lane; the partner's half of the sum is added at the end
+    auto weight2 = [&](int s4, int e) {
+      const float a0 = st[s4 >> 1][8 * (s4 & 1) + 2 * e], b0 = st[s4 >> 1][8 * (s4 & 1) + 2 * e + 1];
+      const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(a0, scale2, -top));
+      const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(b0, scale2, -top));
+      l += x;
+      l += y;
+      return M::pack2(x, y);
+    };
+    u32x4 pb[2];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int e = 0; e < 4; ++e) pb[0][e] = weight2(0, e);
+    // the next 16 keys' weights are formed, and the next tile's keys sent for, between the products of these
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        u32x4 pb;
+    for (int s4 = 0; s4 < 4; ++s4) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) pb[e] = M::pack2(st[kb][8 * s2 + 2 * e], st[kb][8 * s2 + 2 * e + 1]);
-        const unsigned char* src = v_lds + vat + (32 * kb + 16 * s2) * VBYTES;
+      for (int n = 0; n < VB; ++n) {
+        o[n] = M::run(va[n], pb[s4 & 1], o[n]);
+        if (s4 < 3) {
+          va[n] = value_at(s4 + 1, n);
 #pragma unroll
-        for (int n = 0; n < VB; ++n) {
-          const unsigned char* at = src + 64 * (n ^ vf);
-          // 8 rows further on the exchange is the same for four units; for two it is too (8 / 2 even)
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)at);
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 8 * VBYTES));
-          const u32x2 lo2 = __builtin_bit_cast(u32x2, lo), hi2 = __builtin_bit_cast(u32x2, hi);
-          o[n] = M::run(u32x4{lo2[0], lo2[1], hi2[0], hi2[1]}, pb, o[n]);
+          for (int e = 4 * n / VB; e < 4 * (n + 1) / VB; ++e) pb[(s4 + 1) & 1][e] = weight2(s4 + 1, e);
         }
+#pragma unroll
+        for (int i = kEarly; i < kKeyPieces; ++i)
+          if ((i - kEarly) * 2 * VB / (kKeyPieces - kEarly) == s4 * VB + n) bring_key(i, u0 + kStep, more);
+        __builtin_amdgcn_sched_barrier(0);
       }
+    }
+  }
+  if constexpr (KG == 2) {
+    // the second group hands its sums over: registers lie lane for lane in the tiles' place
+    __syncthreads();
+    float* part = reinterpret_cast<float*>(all_tiles) + w * (VB * 16 + 2) * kWave + lane;
+    if (kg == 1) {
+      part[0] = m;
+      part[kWave] = l;
+#pragma unroll
+      for (int n = 0; n < VB; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[(2 + 16 * n + i) * kWave] = o[n][i];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m2 = part[0], m_new = fmaxf(m, m2);
+    const float shift = m_new == -INFINITY ? 0.f : m_new;
+    const float f = __builtin_amdgcn_exp2f(m - shift), f2 = __builtin_amdgcn_exp2f(m2 - shift);
+    l = l * f + part[kWave] * f2;
+#pragma unroll
+    for (int n = 0; n < VB; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[n][i] = o[n][i] * f + part[(2 + 16 * n + i) * kWave] * f2;
+    m = m_new;
   }
   if (!last_range) {
     if (c >= nq) return;
@@ -430,20 +486,41 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPrompt a) {
         *reinterpret_cast<u32x2*>(orow + d) =
             u32x2{M::pack2(o[n][i] * inv, o[n][i + 1] * inv), M::pack2(o[n][i + 2] * inv, o[n][i + 3] * inv)};
     }
+  };
+  // (a second tile only where the sequences are longer than the host's lengths say)
+  int rank = a.ranked_seqs > 0 ? blockIdx.x / a.heads : 0, all = 1;
+  for (;;) {
+    int b = blockIdx.z, tile = a.row_tiles - 1 - (int)blockIdx.y;       // the longest walks first
+    if (a.ranked_seqs > 0) {
+      all = ranked_tile(rank, a.ranked_seqs, a.query_start_loc, a.context_lens, kGroupShift, b, tile);
+      if (rank >= all) return;
+    }
+    one_tile(b, tile);
+    rank += a.tiles;
+    if (rank >= all) return;
+    __syncthreads();
+  }
 }
 
-template <class S, int DB, int VB, int LB>
-int launch_latent_prompt(const LatentPrompt& a, dim3 grid, hipStream_t stream) {
-  constexpr size_t lds = kKeys * 64 * (DB + VB + LB);
+template <class S, int DB, int VB, int LB, int KG>
+int launch_latent_prompt_groups(const LatentPrompt& a, dim3 grid, hipStream_t stream) {
+  constexpr size_t tiles = kKeys * 64 * (DB + VB + LB) * KG, sums = KG == 2 ? sizeof(float) * kWaves * (VB * 16 + 2) * kWave : 0;
+  constexpr size_t lds = tiles > sums ? tiles : sums;
+  static_assert(lds <= 160 * 1024, "two groups' tiles fit a CU's LDS");
   static std::atomic<bool> raised{false};           // LDS limit: raised once per kernel, not per launch
   if (lds > 64 * 1024 && !raised.load(std::memory_order_relaxed)) {
-    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_prompt_kernel<S, DB, VB, LB>),
+    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_prompt_kernel<S, DB, VB, LB, KG>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     raised.store(true, std::memory_order_relaxed);
   }
-  latent_prompt_kernel<S, DB, VB, LB><<<grid, 256, lds, stream>>>(a);
+  latent_prompt_kernel<S, DB, VB, LB, KG><<<grid, 256 * KG, lds, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   return VLA_OK;
+}
+template <class S, int DB, int VB, int LB>
+int launch_latent_prompt(const LatentPrompt& a, dim3 grid, int key_groups, hipStream_t stream) {
+  return key_groups == 2 ? launch_latent_prompt_groups<S, DB, VB, LB, 2>(a, grid, stream)
+                         : launch_latent_prompt_groups<S, DB, VB, LB, 1>(a, grid, stream);
 }
 
 bool prompt_sizes(int dim, int rot, int vdim, int rank) {
@@ -531,14 +608,20 @@ extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* 
   a.row_tiles = (max_query_len + kRowsPerGroup - 1) / kRowsPerGroup;
   a.scale = scale;
   if (a.row_tiles > 65535) return VLA_ERR_ARG;
-  const dim3 grid(heads, a.row_tiles, num_seqs);
+  // every query row is a gathered row, too (a range's launch: one sequence)
+  const int64_t tiles = std::min((int64_t)num_seqs * a.row_tiles, carry ? (int64_t)a.row_tiles : (int64_t)num_rows / kRowsPerGroup + num_seqs);
+  const bool ranked = num_seqs <= kRankedSeqs && tiles * heads <= 0xffffff;
+  a.ranked_seqs = ranked ? num_seqs : 0;
+  a.tiles = ranked ? (int)tiles : 1;
+  const int key_groups = tiles * heads <= 512 ? 2 : 1;
+  const dim3 grid = ranked ? dim3((unsigned)(heads * tiles)) : dim3(heads, a.row_tiles, num_seqs);
   auto go = [&](auto s) -> int {
     using S = decltype(s);
     auto with_values = [&](auto vb) -> int {
       constexpr int VB = decltype(vb)::value;
-      if (dim > 128) return launch_latent_prompt<S, 6, VB, 6>(a, grid, (hipStream_t)stream);
-      return dim + rot > 128 ? launch_latent_prompt<S, 6, VB, 4>(a, grid, (hipStream_t)stream)
-                             : launch_latent_prompt<S, 4, VB, 4>(a, grid, (hipStream_t)stream);
+      if (dim > 128) return launch_latent_prompt<S, 6, VB, 6>(a, grid, key_groups, (hipStream_t)stream);
+      return dim + rot > 128 ? launch_latent_prompt<S, 6, VB, 4>(a, grid, key_groups, (hipStream_t)stream)
+                             : launch_latent_prompt<S, 4, VB, 4>(a, grid, key_groups, (hipStream_t)stream);
     };
     return vdim <= 64 ? with_values(std::integral_constant<int, 2>{}) : with_values(std::integral_constant<int, 4>{});
   };
