@@ -394,10 +394,11 @@ struct DeltaBlocks {
 
 // A block's operands lie in scratch as the walk's waves take them, lane for lane: [16 x 16 tile][lane][4].
 // (Lanes side by side in memory matter: with lanes 64 bytes apart the walk below took 192 us.)
-// Floats of a block's scratch: W | Q~ | K^ (each 32 x DP) | G_31 and a place for stores nobody wants
-// (padded to 4) | A (its three lower 16 x 16 tiles) | T V (32 x VP) | from which row on a column is not finite (VP)
+// Floats of a block's scratch: W | Q~ | K^ (each 32 x DP) | a place for stores nobody wants (padded to 4) | A (its
+// three lower 16 x 16 tiles, and G_31 as the fourth of every lane) | T V (32 x VP) | from which row on a column is not
+// finite (VP)
 __host__ __device__ __forceinline__ int64_t delta_block_floats(int dp, int vp) {
-  return (int64_t)3 * kRows * dp + 4 + 3 * 256 + kRows * vp + vp;
+  return (int64_t)3 * kRows * dp + 4 + 4 * 256 + kRows * vp + vp;
 }
 
 // Which sequence and block a block slot is: sequence b's blocks are slots start_b / 32 + b + 0, 1, ...
@@ -457,12 +458,13 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
   float* w_out = out;                                      // [DP / 16][2][lane][4]: row c, head row 4 g + e
   float* q_out = w_out + kRows * DP;                       // the same
   float* k_out = q_out + kRows * DP;                       // [DP / 16][2][lane][4]: head row pc (below), row 4 g + e
-  float* g_out = k_out + kRows * DP;
-  float* a_out = g_out + 4;                                // [3 tiles][wave][lane]
-  float* u_out = a_out + 3 * 256;                          // [vb][2][lane][4]: column c, row 4 g + e
+  float* a_out = k_out + kRows * DP + 4;                   // [wave][lane][three tiles, G_31]
+  float* u_out = a_out + 4 * 256;                          // [vb][2][lane][4]: column c, row 4 g + e
   const int row = tid >> 3, eighth = tid & 7;              // 8 neighbouring lanes share a row
 
-  // a wave's columns of v, rows 4 g .. and 16 + 4 g ..: the first two tiles are asked for at the start
+  // a wave's columns of v, rows 4 g .. and 16 + 4 g ..: the first two tiles are asked for at the start.  What lies behind
+  // the run or the columns is left out where the values are used: chosen here, each load would be waited for behind a
+  // branch of its own.
   auto fetch_v = [&](float (&to)[2][4], int vt) {
     const int col = 16 * vt + c;
     const float* vr = a.in.v + (int64_t)h * V + min(col, V - 1);
@@ -471,8 +473,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int j = 16 * it + 4 * g + e;
-        const float got = vr[(int64_t)(t0 + min(j, n - 1)) * a.in.v_stride];
-        to[it][e] = j < n && col < V ? got : 0.f;
+        to[it][e] = vr[(int64_t)(t0 + min(j, n - 1)) * a.in.v_stride];
       }
   };
 
@@ -648,10 +649,9 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
         }
       } else {
         // A as the walk's waves take it: wave c & 3 meets contraction index 4 (c >> 2) + (c & 3)
-        float v[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = i0 + 4 * g + e >= j ? (float)got[e] : 0.f;
-        *reinterpret_cast<f32x4*>(a_out + (kind * 4 + (c & 3)) * 64 + ((c >> 2) << 4) + 4 * g) = f32x4{v[0], v[1], v[2], v[3]};
+        for (int e = 0; e < 4; ++e)
+          a_out[((c & 3) * 64 + ((c >> 2) << 4) + 4 * g + e) * 4 + kind] = i0 + 4 * g + e >= j ? (float)got[e] : 0.f;
       }
     }
   }
@@ -696,7 +696,8 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
 #pragma unroll
     for (int e = 0; e < 4; ++e) t_mat[(at + 4 * g + e) * kMatT + c] = x[e];
   } else {
-    if (tid == 128) g_out[0] = l_mat[(kRows - 1) * kMat + kRows];
+    const float g_last = l_mat[(kRows - 1) * kMat + kRows];
+    for (int i = tid - 128; i < 256; i += 128) a_out[4 * i + 3] = g_last;
     for (int i = tid - 128; i < DP * (kRows / 4); i += 128) {
       const int d = 16 * (i >> 7) + 4 * (i & 3) + ((i >> 2) & 3), j = 4 * ((i >> 4) & 7);    // i: tile, half, lane (row pc)
       const f32x4 lv = *reinterpret_cast<const f32x4*>(l_mat + (kRows - 1) * kMat + j);
@@ -772,11 +773,15 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
 #pragma unroll
     for (int it = 0; it < 2; ++it)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+      for (int e = 0; e < 4; ++e) {
+        const int j = 16 * it + 4 * g + e;
+        asm volatile("" : "+v"(v_a[it][e]));
+        v_a[it][e] = j < n && 16 * vt + c < V ? v_a[it][e] : 0.f;
         if (!finite(v_a[it][e])) {
-          from = min(from, 16 * it + 4 * g + e);
+          from = min(from, j);
           v_a[it][e] = 0.f;
         }
+      }
     if (__any(from < kRows)) {
       from = min(from, __shfl_xor(from, 16, 64));
       from = min(from, __shfl_xor(from, 32, 64));
@@ -805,12 +810,22 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
   }
 }
 
-// What bounds it: a wave has 35 matrix-core instructions of 32 cycles per block and 16 of 64 (1.1 us of 128 x 128) in a
-// chain product -> LDS -> barrier -> LDS -> product, one wave per SIMD and nobody to fill its waits: the
-// loads are a block ahead, the product for the outputs stands where the exchange of U is on its way.
-// Two prompts of 2999 and 1854 tokens, 16 heads of 128 x 128 (94 blocks in a row), under the tracer: the walk 212 us,
-// 2.3 us per block; the prepare kernel 124 (101 with every product in 32 bits and no look at what is not finite), the
-// norms 20 and the step kernel's empty launch 5; a call 333, where the token-by-token walk of the same prompts takes 1079.
+// a value that is the same for all lanes, where a choice by it should be no branch
+__device__ __forceinline__ int lane_value(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// What bounds it: a wave has 35 matrix-core instructions of 32 cycles per block and 16 of 64 (2140 of about 3300 cycles
+// of 128 x 128) in a chain product -> LDS -> barrier -> LDS -> product, one wave per SIMD and nobody to fill its
+// waits.  So the next block's loads go out between the products (56 KB per block and workgroup: sent at once they held a
+// wave up for 1250 cycles), the product for the outputs stands where the exchange of U is on its way, and the
+// state of 16 rows and the block before's outputs are formed under the 64-bit products.  No value of a block may be
+// copied from turn to turn (its load would be waited for right there), and the first block's loads keep the order of
+// the loop's, which waits for what both orders have in common.
+// Two prompts of 2999 and 1854 tokens, 16 heads of 128 x 128 (94 blocks in a row), under the tracer: the walk 178 us, 1.9
+// us per block (212 with the loads at once and choices by branches), the prepare kernel 92, the norms 20 and the
+// step kernel's empty launch 5; a call 267 (333), where the token-by-token walk of the same prompts takes 1079.
 // What a block adds to the state is summed in 64 bits: in 32 a call is 32 us less and states are 1.2 times as far
 // from 64 bits as token by token where keys share a part three times as large as the rest (1.0).
 template <int DX>
@@ -841,47 +856,51 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
   }
   const int blocks = (run + kRows - 1) / kRows;
   struct Block {
-    f32x4 wv[DX][2], qv[DX][2], kv[DX][2], u[2];
-    float av[3], g_last, from;
+    f32x4 wv[DX][2], qv[DX][2], kv[DX][2], u[2], av;
+    float from;
   };
-  const int at_x = w * DX * 2 * 256 + 4 * lane, at_a = w * 64 + lane, at_u = blockIdx.y * 2 * 256 + 4 * lane;
-  auto fetch = [&](Block& f, const float* p) {
-#pragma unroll
-    for (int x = 0; x < DX; ++x)
-#pragma unroll
-      for (int it = 0; it < 2; ++it) {
-        const float* px = p + at_x + (2 * x + it) * 256;
-        f.wv[x][it] = *reinterpret_cast<const f32x4*>(px);
-        f.qv[x][it] = *reinterpret_cast<const f32x4*>(px + kRows * DP);
-        f.kv[x][it] = *reinterpret_cast<const f32x4*>(px + 2 * kRows * DP);
-      }
+  const int at_x = w * DX * 2 * 256 + 4 * lane, at_a = 4 * (w * 64 + lane), at_u = blockIdx.y * 2 * 256 + 4 * lane;
+  // piece j of a block, in the order that the walk wants them: W, Q~, T V, K^, A and the rest
+  constexpr int kHalves = 2 * DX, kPieces = 3 * kHalves + 4, kFirst = 2 * kHalves;
+  auto fetch = [&](Block& f, const float* p, int j) __attribute__((always_inline)) {
     const float* pa = p + 3 * kRows * DP;
-    f.g_last = pa[0];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) f.av[i] = pa[4 + at_a + 256 * i];
-#pragma unroll
-    for (int it = 0; it < 2; ++it) f.u[it] = *reinterpret_cast<const f32x4*>(pa + 4 + 3 * 256 + at_u + 256 * it);
-    f.from = pa[4 + 3 * 256 + kRows * vp + col];
+    const int x = (j % kHalves) >> 1, it = j & 1;
+    if (j < kHalves)
+      f.wv[x][it] = *reinterpret_cast<const f32x4*>(p + at_x + 256 * j);
+    else if (j < kFirst)
+      f.qv[x][it] = *reinterpret_cast<const f32x4*>(p + kRows * DP + at_x + 256 * (j - kHalves));
+    else if (j < kFirst + 2)
+      f.u[it] = *reinterpret_cast<const f32x4*>(pa + 4 + 4 * 256 + at_u + 256 * it);
+    else if (j < kFirst + 2 + kHalves)
+      f.kv[((j - 2) % kHalves) >> 1][it] = *reinterpret_cast<const f32x4*>(p + 2 * kRows * DP + at_x + 256 * (j - 2 - kFirst));
+    else if (j == kPieces - 2)
+      f.av = *reinterpret_cast<const f32x4*>(pa + 4 + at_a);
+    else
+      f.from = pa[4 + 4 * 256 + kRows * vp + col];
   };
   // wave w finishes rows 16 it + 4 g + w of a block's outputs; what has no place goes to the block's pad
   const int64_t row_step = (int64_t)a.heads * V;
   float* o_at = a.o + ((int64_t)(t_begin + 4 * g + w) * a.heads + h) * V + (col < V ? col : 0);
-  float* nowhere = a.scratch + ((int64_t)(t_begin / kRows + b) * a.heads + h) * per + 3 * kRows * DP + 1;
+  float* nowhere = a.scratch + ((int64_t)(t_begin / kRows + b) * a.heads + h) * per + 3 * kRows * DP;
   // column c is NaN from its first row on that is not finite, as the state that a walk reads it with
   const float row_w = (float)(4 * g + w);
-  float from = (float)kRows;                               // of the block to finish
-  auto finish = [&](int i) {
-    const int buf = i & 1;
+  const unsigned rows_here = col < V ? run : 0;
+  auto finish_read = [&](int i, float (&o)[2][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int it = 0; it < 2; ++it)
+#pragma unroll
+      for (int ow = 0; ow < 4; ++ow) o[it][ow] = o_part[i & 1][ow][it][w][lane];
+  };
+  auto finish = [&](int i, const float (&o)[2][4], float from) __attribute__((always_inline)) {
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
-      const float o = (o_part[buf][0][it][w][lane] + o_part[buf][1][it][w][lane]) +
-                      (o_part[buf][2][it][w][lane] + o_part[buf][3][it][w][lane]);
-      const bool live = i * kRows + 16 * it + 4 * g + w < run && col < V;
-      *(live ? o_at + 16 * it * row_step : nowhere) = row_w + 16.f * it < from ? o : NAN;
+      const float sum = (o[it][0] + o[it][1]) + (o[it][2] + o[it][3]);
+      const bool live = (unsigned)(i * kRows + 16 * it + 4 * g + w) < rows_here;      // (block -1 has none)
+      *(live ? o_at + (i * kRows + 16 * it) * row_step : nowhere) = row_w + 16.f * it < from ? sum : NAN;
     }
-    o_at += kRows * row_step;
   };
-  auto advance = [&](const Block& f, int i) {
+  const int own = lane_value(w);
+  auto advance = [&](const Block& f, Block& next, const float* next_at, int i) __attribute__((always_inline)) {
     const int buf = i & 1;
     // sums in several parts: half the roundings in a row
     constexpr int kParts = DX > 1 ? 2 : 1;
@@ -895,7 +914,11 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int it = 0; it < 2; ++it) xu[it][x % kParts] = mfma4(f.wv[x][it][e], s[x][e], xu[it][x % kParts]);
+        for (int it = 0; it < 2; ++it) {
+          xu[it][x % kParts] = mfma4(f.wv[x][it][e], s[x][e], xu[it][x % kParts]);
+          if (it == 0 && e % 2 == 0) fetch(next, next_at, 2 * x + e / 2);
+          __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
 #pragma unroll
@@ -915,8 +938,13 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int it = 0; it < 2; ++it) xo[it][x % kParts] = mfma4(f.qv[x][it][e], s[x][e], xo[it][x % kParts]);
-    if (i > 0) finish(i - 1);
+        for (int it = 0; it < 2; ++it) {
+          xo[it][x % kParts] = mfma4(f.qv[x][it][e], s[x][e], xo[it][x % kParts]);
+          if (it == 0 && e % 2 == 0) fetch(next, next_at, kHalves + 2 * x + e / 2);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    float done[2][4];
+    finish_read(i - 1, done);                              // (ahead of the first block: what nobody wants)
     __builtin_amdgcn_sched_barrier(0);
     f32x4 u[2];
 #pragma unroll
@@ -924,26 +952,22 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         u[it][e] = f.u[it][e] - ((p[it][0][e] + p[it][1][e]) + (p[it][2][e] + p[it][3][e]));
-    // what the block adds is summed by itself, in 64 bits: one rounding of the state per block
-    f64x4 ds[DX];
-#pragma unroll
-    for (int x = 0; x < DX; ++x) ds[x] = f64x4{0., 0., 0., 0.};
-#pragma unroll
-    for (int it = 0; it < 2; ++it)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int x = 0; x < DX; ++x) ds[x] = mfma4_f64((double)f.kv[x][it][e], (double)u[it][e], ds[x]);
     // A U: the wave takes contraction index 4 g + w, so that the sum over waves is the whole product.  A row's product
     // with the rows behind it is 0 times their U: those that are not finite stay out.
-    float u0 = w == 0 ? u[0][0] : w == 1 ? u[0][1] : w == 2 ? u[0][2] : u[0][3];
-    float u1 = w == 0 ? u[1][0] : w == 1 ? u[1][1] : w == 2 ? u[1][2] : u[1][3];
-    u0 = row_w < f.from ? u0 : 0.f;
-    u1 = row_w + 16.f < f.from ? u1 : 0.f;
-    from = f.from;
-    xo[0][0] = mfma4(f.av[0], u0, xo[0][0]);
-    xo[1][0] = mfma4(f.av[1], u0, xo[1][0]);
-    xo[1][0] = mfma4(f.av[2], u1, xo[1][0]);
+    float us[2];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(u[it][e]));       // (chosen, not worked out again behind branches)
+      const float even = own & 2 ? u[it][2] : u[it][0], odd = own & 2 ? u[it][3] : u[it][1];
+      us[it] = own & 1 ? odd : even;
+    }
+    const float u0 = row_w < f.from ? us[0] : 0.f, u1 = row_w + 16.f < f.from ? us[1] : 0.f;
+    f32x4 av = f.av;
+    asm volatile("" : "+v"(av));                            // (whole: a part by itself would be copied from block to block)
+    xo[0][0] = mfma4(av[0], u0, xo[0][0]);
+    xo[1][0] = mfma4(av[1], u0, xo[1][0]);
+    xo[1][0] = mfma4(av[2], u1, xo[1][0]);
 #pragma unroll
     for (int it = 0; it < 2; ++it)
 #pragma unroll
@@ -951,25 +975,50 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
         if constexpr (kParts > 1) xo[it][0][e] += xo[it][1][e];
         o_part[buf][w][it][e][lane] = xo[it][0][e];
       }
+    // What the block adds is summed by itself, in 64 bits: one rounding of the state per block.  One 16 rows after the
+    // other, so that a state is formed under the next one's products, as are the outputs of the block before.
+    f64x4 ds[DX];
 #pragma unroll
-    for (int x = 0; x < DX; ++x)
+    for (int x = 0; x < DX; ++x) {
+      ds[x] = f64x4{0., 0., 0., 0.};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[x][e] = (float)((double)f.g_last * (double)s[x][e] + ds[x][e]);
+      for (int it = 0; it < 2; ++it)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          ds[x] = mfma4_f64((double)f.kv[x][it][e], (double)u[it][e], ds[x]);
+          constexpr int kLeft = kPieces - kFirst, kProducts = 8 * DX;
+          const int at = 8 * x + 4 * it + e;
+          if (at == kProducts / 2 - 1) finish(i - 1, done, next.from);     // (next has the block before in its place)
+#pragma unroll
+          for (int j = 0; j < kLeft; ++j)
+            if (j * kProducts / kLeft == at) fetch(next, next_at, kFirst + j);
+          if (x > 0 && it == 0) s[x - 1][e] = (float)((double)av[3] * (double)s[x - 1][e] + ds[x - 1][e]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[DX - 1][e] = (float)((double)av[3] * (double)s[DX - 1][e] + ds[DX - 1][e]);
   };
   // two blocks in turn, so that one is asked for while the other is worked on
   Block f0, f1;
-  fetch(f0, base);
-  for (int i = 0; i < blocks; i += 2) {
-    fetch(f1, base + (int64_t)min(i + 1, blocks - 1) * step);
-    __builtin_amdgcn_sched_barrier(0);
-    advance(f0, i);
-    if (i + 1 >= blocks) break;
-    fetch(f0, base + (int64_t)min(i + 2, blocks - 1) * step);
-    __builtin_amdgcn_sched_barrier(0);
-    advance(f1, i + 1);
+#pragma unroll
+  for (int j = 0; j < kPieces; ++j) {
+    fetch(f0, base, j);
+    __builtin_amdgcn_sched_barrier(0);                     // (the loop waits for the order that it finds here, too)
   }
+  const float* at = base;
+  for (int i = 0; i < blocks; i += 2) {
+    at += i + 1 < blocks ? step : 0;
+    advance(f0, f1, at, i);
+    if (i + 1 >= blocks) break;
+    at += i + 2 < blocks ? step : 0;
+    advance(f1, f0, at, i + 1);
+  }
+  const float from = at[3 * kRows * DP + 4 + 4 * 256 + kRows * vp + col];      // (f0's would be copied, and waited for, in each turn)
   __syncthreads();
-  finish(blocks - 1);
+  float done[2][4];
+  finish_read(blocks - 1, done);
+  finish(blocks - 1, done, from);
   if (col < V) {
 #pragma unroll
     for (int x = 0; x < DX; ++x) {
@@ -1063,7 +1112,7 @@ std::atomic<int> g_delta_kernel{0};
 
 // Blocks pay from about a block's rows on (us on the GPU, calls back to back, 16 heads of 128, token by token / in
 // blocks: one run of 33 rows 21 / 23, 48 rows 24 / 23, 100 rows 43 / 28; six runs of 64 rows 55 / 44; 32 runs of 33
-// rows 140 / 114, of 64 217 / 129; one of 33 beside 31 single rows 50 / 41).  Their scratch is 68 KB per block and head of 128 x 128;
+// rows 140 / 114, of 64 217 / 129; one of 33 beside 31 single rows 50 / 41).  Their scratch is 69 KB per block and head of 128 x 128;
 // a step that would want more than 4 GiB of it walks token by token.
 constexpr int kBlockMinRows = 33;
 
@@ -1073,8 +1122,9 @@ int64_t delta_out_floats(int num_tokens, int heads, int vdim) {
 
 bool wants_blocks(int mode, int num_tokens, int num_seqs, int max_query_len, int heads, int dim, int vdim) {
   if (mode != 0 || dim > kMaxBlockDim || max_query_len < kBlockMinRows || (vdim + 15) / 16 > 65535) return false;
+  // (G_31's places are not counted)
   return delta_block_slots(num_tokens, num_seqs) * heads *
-             delta_block_floats((dim + 63) / 64 * 64, (vdim + 15) / 16 * 16) <= ((int64_t)1 << 30);
+             (delta_block_floats((dim + 63) / 64 * 64, (vdim + 15) / 16 * 16) - 256) <= ((int64_t)1 << 30);
 }
 
 int pow2_at_least(int n) {
