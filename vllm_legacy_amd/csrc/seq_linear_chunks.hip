@@ -16,10 +16,13 @@
 // states after 4096 rows several times as far from 64 bits).
 // All products run on 16x16x4 fp32 matrix cores.  Operands that later kernels read lie in scratch lane for
 // lane.  Bound by memory and the launches: 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB
-// of chunk states and decays; 130 us per call (45 + 23 + 68 under the tracer) where the pieces of 256 rows walked
-// token by token and joined by matrix products took 408.  What a workgroup's 19 and 30 us go to: waits for its rows (5
-// and 7), products (7 and 9), decays (6 and 5), the products inside a block (4), gates and stores (5).
+// of chunk states and decays; 123 us per call (42 + 23 + 66 under the tracer) where the pieces of 256 rows walked
+// token by token and joined by matrix products took 408.  What a workgroup's 19 and 29 us go to: waits for its rows
+// (4 and 5), products (7 and 9), decays (6 and 5), the products inside a block (4), gates and stores (5).  Rows are
+// asked for together and made numbers afterwards, start states a tile of columns ahead (130 us where values and W2
+// were each waited for behind a condition of their own, and keys, values and y in turn).
 #include <atomic>
+#include <type_traits>
 
 #include "seq_common.h"
 
@@ -78,15 +81,24 @@ __device__ __forceinline__ bool find_chunk(const GlaChunks& a, int slot, int& b,
   return chunk >= 0 && chunk * kChunk < a.query_start_loc[b + 1] - a.query_start_loc[b];
 }
 
-// four values of a row, aligned for one access
+// Four values of a row, aligned for one access, as they lie there and as numbers.  (Two steps: where loads stand behind
+// conditions, one that is made a number at once is waited for before the next is asked for.)
+template <class S>
+using Four = std::conditional_t<sizeof(typename S::T) == 2, u32x2, f32x4>;
+template <class S>
+__device__ __forceinline__ Four<S> fetch4(const typename S::T* p) {
+  return *reinterpret_cast<const Four<S>*>(p);
+}
+template <class S>
+__device__ __forceinline__ f32x4 numbers(Four<S> x) {
+  if constexpr (sizeof(typename S::T) == 2)
+    return f32x4{lo16<S>(x[0]), hi16<S>(x[0]), lo16<S>(x[1]), hi16<S>(x[1])};
+  else
+    return x;
+}
 template <class S>
 __device__ __forceinline__ f32x4 row4(const typename S::T* p) {
-  if constexpr (sizeof(typename S::T) == 2) {
-    const u32x2 x = *reinterpret_cast<const u32x2*>(p);
-    return f32x4{lo16<S>(x[0]), hi16<S>(x[0]), lo16<S>(x[1]), hi16<S>(x[1])};
-  } else {
-    return *reinterpret_cast<const f32x4*>(p);
-  }
+  return numbers<S>(fetch4<S>(p));
 }
 
 // exp(p) for p <= 0 (NaN passes): 2^n 2^f with the argument's rounding in f.  expf without what other p need, the same
@@ -119,11 +131,12 @@ __device__ __forceinline__ float log_sigmoid(float z) {
   return -(t + (lost_lo + fmaf(a * y, s, more)));
 }
 
-template <class S>
+template <class S, int DT>          // DT: dim / 16
 __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
   using T = typename S::T;
   extern __shared__ __align__(16) float lds[];
-  const int D = a.dim, V = a.vdim, R = a.rank, KR = D + 4, VR = V + 4;
+  constexpr int D = 16 * DT, KR = D + 4;
+  const int V = a.vdim, R = a.rank, VR = V + 4;
   float* k_lds = lds;                       // [64][KR]
   float* a_lds = k_lds + kChunk * KR;       // [64][D]
   float* v_lds = a_lds + kChunk * D;        // [64][VR]
@@ -139,7 +152,7 @@ __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
   const int RP = (R + 3) / 4 * 4;
   float* mine = a.scratch + ((int64_t)slot * a.heads + h) * chunk_floats(D, V);
 
-  // rows behind the run's end are zeros
+  // rows behind the run's end are zeros; every load is on its way before the first is waited for
   const int row = tid >> 2, quarter = tid & 3;
   const int64_t t = t0 + min(row, n - 1);
   const int d_mine = tid % D;                // the thread's decay channel and its row of W2, on its way with the rows
@@ -150,27 +163,47 @@ __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
   const T* wr = (const T*)a.w2 + ((int64_t)h * D + d_mine) * R;
   if (w_wide) {
 #pragma unroll
-    for (int r = 0; r < kMaxRank / PER; ++r)
-      if (PER * r < R) w_row[r] = *reinterpret_cast<const u32x4*>(wr + PER * r);
+    for (int r = 0; r < kMaxRank / PER; ++r) w_row[r] = *reinterpret_cast<const u32x4*>(wr + min(PER * r, R - PER));
   } else {
+    T raw[kMaxRank];
 #pragma unroll
-    for (int r = 0; r < kMaxRank; ++r) wv[r] = r < R ? S::to_f32(wr[r]) : 0.f;
+    for (int r = 0; r < kMaxRank; ++r) raw[r] = wr[min(r, R - 1)];
+#pragma unroll
+    for (int r = 0; r < kMaxRank; ++r) wv[r] = r < R ? S::to_f32(raw[r]) : 0.f;
   }
   const float bias = a.bias != nullptr ? a.bias[(int64_t)h * D + d_mine] : 0.f;
-#pragma unroll 4
-  for (int i = tid; i < kChunk * D / 4; i += 256) {         // four values a thread, in the order they lie in
-    const int r = i / (D / 4), d = 4 * (i % (D / 4));
-    const f32x4 x = row4<S>((const T*)a.k + (t0 + min(r, n - 1)) * a.k_stride + (int64_t)h * D + d);
-    *reinterpret_cast<f32x4*>(k_lds + r * KR + d) = r < n ? x : f32x4{0.f, 0.f, 0.f, 0.f};
+  T ys[kMaxRank / 4];
+#pragma unroll
+  for (int u = 0; u < kMaxRank / 4; ++u) ys[u] = ((const T*)a.y)[t * a.y_stride + min(quarter + 4 * u, R - 1)];
+  // four values a thread, in the order they lie in: D / 16 and V / 16 of them, whole for all threads
+  constexpr int kMost = 8;
+  Four<S> ks[DT], vs[kMost];
+  const int per_row = V / 4, inverse = (65536 + per_row - 1) / per_row;      // (i * inverse) >> 16 is i / per_row below 2048
+#pragma unroll
+  for (int u = 0; u < DT; ++u) {
+    const int i = tid + 256 * u, r = i / (D / 4), d = 4 * (i % (D / 4));
+    ks[u] = fetch4<S>((const T*)a.k + (t0 + min(r, n - 1)) * a.k_stride + (int64_t)h * D + d);
   }
-#pragma unroll 8
-  for (int i = tid; i < kChunk * V / 4; i += 256) {
-    const int r = i / (V / 4), d = 4 * (i % (V / 4));
-    const f32x4 x = row4<S>((const T*)a.v + (t0 + min(r, n - 1)) * a.v_stride + (int64_t)h * V + d);
-    *reinterpret_cast<f32x4*>(v_lds + r * VR + d) = r < n ? x : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < kMost; ++u) {
+    const int i = tid + 256 * min(u, V / 16 - 1), r = (i * inverse) >> 16, d = 4 * (i - r * per_row);
+    vs[u] = fetch4<S>((const T*)a.v + (t0 + min(r, n - 1)) * a.v_stride + (int64_t)h * V + d);
   }
-  for (int r = quarter; r < RP; r += 4)
-    y_lds[row * kMaxRank + r] = r < R ? S::to_f32(((const T*)a.y)[t * a.y_stride + r]) : 0.f;
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < kMaxRank / 4; ++u)
+    if (4 * u < RP) y_lds[row * kMaxRank + quarter + 4 * u] = quarter + 4 * u < R ? S::to_f32(ys[u]) : 0.f;
+#pragma unroll
+  for (int u = 0; u < DT; ++u) {
+    const int i = tid + 256 * u, r = i / (D / 4), d = 4 * (i % (D / 4));
+    *reinterpret_cast<f32x4*>(k_lds + r * KR + d) = r < n ? numbers<S>(ks[u]) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int u = 0; u < kMost; ++u)
+    if (16 * u < V) {
+      const int i = tid + 256 * u, r = (i * inverse) >> 16, d = 4 * (i - r * per_row);
+      *reinterpret_cast<f32x4*>(v_lds + r * VR + d) = r < n ? numbers<S>(vs[u]) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
   __syncthreads();
 
   // decays: a thread keeps its channel's row of W2 and walks every (256 / D)-th row
@@ -410,19 +443,26 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
     for (int e = 0; e < 4; ++e) a_mat[(kBlock * w + 4 * g + e) * kAMat + kBlock * o + c] = acc[e];
   }
   // the values take the keys' and the decays' place
-  f32x4 held[8];
+  Four<S> held[8];
 #pragma unroll
   for (int x = 0; x < 8; ++x)
-    if (4 * quarter + 16 * x < V) held[x] = row4<S>(vr + 4 * quarter + 16 * x);
+    if (16 * x < V) held[x] = fetch4<S>(vr + 4 * quarter + 16 * x);
+  // the start state of a tile of columns is asked for a tile ahead
+  f32x4 sv[2][DT];
+  auto fetch_state = [&](int vt) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < DT; ++x) sv[vt & 1][x] = *reinterpret_cast<const f32x4*>(s_in + ((int64_t)(x * vt_n + vt) * 64 + lane) * 4);
+  };
+  fetch_state(0);
   __syncthreads();
   bool odd = false;
 #pragma unroll
   for (int x = 0; x < 8; ++x)
-    if (4 * quarter + 16 * x < V) {
-      if (!live) held[x] = f32x4{0.f, 0.f, 0.f, 0.f};
-      *reinterpret_cast<f32x4*>(v_lds + row * VR + 4 * quarter + 16 * x) = held[x];
+    if (16 * x < V) {
+      const f32x4 put = live ? numbers<S>(held[x]) : f32x4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<f32x4*>(v_lds + row * VR + 4 * quarter + 16 * x) = put;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) odd |= !finite(held[x][e]);
+      for (int e = 0; e < 4; ++e) odd |= !finite(put[e]);
     }
   const bool some_bad = __syncthreads_or(odd);
 
@@ -459,9 +499,7 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
   for (int vt = 0; vt < 8; ++vt) {
     acc[vt] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (vt < vt_n) {
-      f32x4 sv[DT];
-#pragma unroll
-      for (int x = 0; x < DT; ++x) sv[x] = *reinterpret_cast<const f32x4*>(s_in + ((int64_t)(x * vt_n + vt) * 64 + lane) * 4);
+      if (vt + 1 < vt_n) fetch_state(vt + 1);
       for (int o = 0; o < w; ++o) {
         const f32x4 am = *reinterpret_cast<const f32x4*>(a_mat + (kBlock * w + c) * kAMat + kBlock * o + 4 * g);
 #pragma unroll
@@ -483,7 +521,7 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
 #pragma unroll
       for (int x = 0; x < DT; ++x)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[vt] = mfma4(qs[x][e], sv[x][e], acc[vt]);
+        for (int e = 0; e < 4; ++e) acc[vt] = mfma4(qs[x][e], sv[vt & 1][x][e], acc[vt]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[vt][e] = 4 * g + e < bad ? acc[vt][e] : NAN;
 #pragma unroll
@@ -560,13 +598,19 @@ int raise_lds(K kernel, size_t lds, std::atomic<size_t>& allowed) {
 }
 
 template <class S, int DT>
-int launch_out(const GlaChunks& a, dim3 grid, hipStream_t stream) {
+int launch_chunks(const GlaChunks& a, dim3 grid, hipStream_t stream) {
   constexpr int D = 16 * DT;
+  static std::atomic<size_t> allowed{64 * 1024}, allowed_out{64 * 1024};   // raised once per kernel, not per launch
+  const size_t lds = sizeof(float) * ((size_t)kChunk * (D + 4 + D + a.vdim + 4 + kMaxRank) + 4 * D);
+  if (const int rc = raise_lds(&gla_chunk_state_kernel<S, DT>, lds, allowed)) return rc;
+  gla_chunk_state_kernel<S, DT><<<grid, 256, lds, stream>>>(a);
+  VLA_SEQ_HIP_CHECK(hipGetLastError());
+  gla_chunk_scan_kernel<<<dim3(a.heads, (D * a.vdim / 4 + 255) / 256, a.num_seqs), 256, 0, stream>>>(a);
+  VLA_SEQ_HIP_CHECK(hipGetLastError());
   const size_t keys = (size_t)kChunk * (D + 4 + D), values = (size_t)kChunk * (a.vdim + 4);
-  const size_t lds = sizeof(float) * ((size_t)kChunk * (D + 4) + kChunk * kAMat + 4 * D + (keys > values ? keys : values));
-  static std::atomic<size_t> allowed{64 * 1024};   // raised once per kernel, not per launch
-  if (const int rc = raise_lds(&gla_chunk_out_kernel<S, DT>, lds, allowed)) return rc;
-  gla_chunk_out_kernel<S, DT><<<grid, 256, lds, stream>>>(a);
+  const size_t lds_out = sizeof(float) * ((size_t)kChunk * (D + 4) + kChunk * kAMat + 4 * D + (keys > values ? keys : values));
+  if (const int rc = raise_lds(&gla_chunk_out_kernel<S, DT>, lds_out, allowed_out)) return rc;
+  gla_chunk_out_kernel<S, DT><<<grid, 256, lds_out, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   return VLA_OK;
 }
@@ -614,20 +658,13 @@ extern "C" int vla_seq_gla_chunks(void* out, int64_t out_stride, const void* q, 
                     rank, q_scale, inv_tau, eps, out_scale};
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)chunk_slots(num_tokens, num_seqs), heads);
-  const size_t lds = sizeof(float) * ((size_t)kChunk * (dim + 4 + dim + vdim + 4 + kMaxRank) + 4 * dim);
   return with_dtype(dtype, [&](auto s) -> int {
     using S = decltype(s);
-    static std::atomic<size_t> allowed{64 * 1024};   // raised once per kernel, not per launch
-    if (const int rc = raise_lds(&gla_chunk_state_kernel<S>, lds, allowed)) return rc;
-    gla_chunk_state_kernel<S><<<grid, 256, lds, st>>>(a);
-    VLA_SEQ_HIP_CHECK(hipGetLastError());
-    gla_chunk_scan_kernel<<<dim3(heads, (dim * vdim / 4 + 255) / 256, num_seqs), 256, 0, st>>>(a);
-    VLA_SEQ_HIP_CHECK(hipGetLastError());
     switch (dim / 16) {
-      case 1: return launch_out<S, 1>(a, grid, st);
-      case 2: return launch_out<S, 2>(a, grid, st);
-      case 4: return launch_out<S, 4>(a, grid, st);
-      default: return launch_out<S, 8>(a, grid, st);
+      case 1: return launch_chunks<S, 1>(a, grid, st);
+      case 2: return launch_chunks<S, 2>(a, grid, st);
+      case 4: return launch_chunks<S, 4>(a, grid, st);
+      default: return launch_chunks<S, 8>(a, grid, st);
     }
   });
 }
