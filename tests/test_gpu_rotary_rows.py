@@ -1,0 +1,50 @@
+"""Rotary rows written 16 bytes at a time against the kernel that takes any address: the same rows one element further on
+go there.  Both form the same products and round once, so results are the same bits (float16: the compiler has a sum
+rounded at once in one kernel and by way of 32 bits in the other, one unit in the last place where it lies half way): pairs side by side and in halves,
+heads that turn in part, more pieces than a wave fetches ahead, rows that no cache takes, and tokens around the
+sizes of a workgroup."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def shifted(t, by):
+    """The same rows in a wider tensor, `by` elements behind its start."""
+    wide = torch.zeros(t.shape[0], t.shape[1] + 16, dtype=t.dtype, device=DEV)
+    wide[:, by:by + t.shape[1]] = t
+    return wide[:, by:by + t.shape[1]]
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("T,heads,kv_heads,dim,vdim,rot", [
+    (1, 1, 1, 16, 8, 16), (5, 16, 4, 128, 128, 128), (1023, 16, 4, 128, 128, 64), (1024, 4, 4, 64, 128, 64),
+    (1029, 32, 8, 128, 128, 128), (7, 72, 24, 128, 72, 96), (6, 6, 3, 48, 40, 48), (3, 8, 8, 256, 256, 256),
+    (3, 5, 1, 264, 24, 16), (70, 3, 3, 8 + 16, 8, 16), (2, 256, 16, 128, 64, 128), (2, 260, 4, 128, 64, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_same_bits_as_rows_anywhere(interleaved, T, heads, kv_heads, dim, vdim, rot, dtype):
+    from vllm_legacy_amd import _seq_ops as ops
+    g = torch.Generator(device=DEV).manual_seed(T + heads)
+    q, k, v = (torch.randn(T, n, generator=g, device=DEV).to(dtype) for n in (heads * dim, kv_heads * dim, kv_heads * vdim))
+    blocks, size = T // 16 + 2, 16
+    slots = torch.randperm(blocks * size, generator=g, device=DEV)[:T].contiguous()
+    slots[T // 2] = -1 if T > 1 else slots[0]
+    if T > 2:
+        slots[T // 3] = blocks * size
+    positions = torch.randint(0, 40000, (T, ), generator=g, device=DEV)
+    freq = 10000.0**(-torch.arange(0, rot, 2, device=DEV, dtype=torch.float32) / rot)
+    got = []
+    for by in (8, 1):
+        mine = [shifted(t, by) for t in (q, k, v)]
+        caches = [torch.full((blocks, size, kv_heads, n), 7.0, dtype=dtype, device=DEV) for n in (dim, vdim)]
+        ops.rotary_kv_write(*mine, *caches, positions, slots, freq, None, heads, rot, interleaved)
+        got.append([mine[0].clone()] + caches)
+        assert torch.equal(mine[1], k) and torch.equal(mine[2], v)
+    for a, b in zip(*got):
+        if dtype == torch.bfloat16:
+            assert torch.equal(a, b)
+        else:       # a unit: 2^-10 of the value, 2^-24 below 2^-14
+            a, b = a.double(), b.double()
+            assert bool(((a - b).abs() <= 2.0**-10 * b.abs() + 2.0**-24).all()) and float((a != b).double().mean()) < 1e-3
+    assert not torch.equal(got[0][0], q) and bool((got[0][1] == 7.0).any())
