@@ -1,4 +1,4 @@
-"""Rotary rows written 16 bytes at a time against the kernel that takes any address: the same rows one element further on
+"""Rotary and latent rows written 16 bytes at a time against the kernel that takes any address: the same rows one element further on
 go there.  Both form the same products and round once, so results are the same bits (float16: the compiler has a sum
 rounded at once in one kernel and by way of 32 bits in the other, one unit in the last place where it lies half way): pairs side by side and in halves,
 heads that turn in part, more pieces than a wave fetches ahead, rows that no cache takes, and tokens around the
@@ -48,3 +48,35 @@ def test_same_bits_as_rows_anywhere(interleaved, T, heads, kv_heads, dim, vdim, 
             a, b = a.double(), b.double()
             assert bool(((a - b).abs() <= 2.0**-10 * b.abs() + 2.0**-24).all()) and float((a != b).double().mean()) < 1e-3
     assert not torch.equal(got[0][0], q) and bool((got[0][1] == 7.0).any())
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("T,heads,rank,rot,rot_dims,head,first", [
+    (1, 1, 8, 16, 16, 16, 0), (5, 16, 512, 64, 64, 192, 128), (1025, 16, 256, 64, 32, 128, 64), (7, 3, 520, 0, 0, 64, 8),
+    (6, 40, 1024, 128, 128, 128, 0), (3, 5, 72, 272, 256, 280, 8), (1024, 4, 512, 64, 64, 64, 0), (9, 2, 504, 24, 16, 40, 8)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_latent_rows_as_rows_anywhere(interleaved, T, heads, rank, rot, rot_dims, head, first, dtype):
+    """The latent's norm adds its squares in another order: relative differences of some 2^-22 ahead of one rounding."""
+    from vllm_legacy_amd import _seq_ops as ops
+    g = torch.Generator(device=DEV).manual_seed(T + heads)
+    q, kv = (torch.randn(T, n, generator=g, device=DEV).to(dtype) for n in (heads * head, rank + rot))
+    weight = torch.rand(rank, generator=g, device=DEV) + 0.5
+    blocks, size = T // 16 + 2, 16
+    slots = torch.randperm(blocks * size, generator=g, device=DEV)[:T].contiguous()
+    if T > 2:
+        slots[T // 2], slots[T // 3] = -1, blocks * size
+    positions = torch.randint(0, 40000, (T, ), generator=g, device=DEV)
+    freq = 10000.0**(-torch.arange(0, rot_dims, 2, device=DEV, dtype=torch.float32) / max(rot_dims, 1)) if rot_dims else None
+    got = []
+    for by in (8, 1):
+        rows, lat = shifted(q, by), shifted(kv, by)
+        cache = torch.full((blocks, size, rank + rot), 7.0, dtype=dtype, device=DEV)
+        ops.latent_rotary_write(rows, head, first, heads, lat, weight, 1e-5, cache, positions, slots, freq, 0.9, rot_dims,
+                                interleaved)
+        assert torch.equal(lat, kv)
+        got.append((rows.clone().double(), cache.double()))
+    unit = 2.0**-7 if dtype == torch.bfloat16 else 2.0**-10
+    for a, b in zip(*got):
+        assert bool(((a - b).abs() <= unit * b.abs() + 2.0**-24).all()) and float((a != b).double().mean()) < 2e-3
+    assert rot_dims == 0 or not torch.equal(got[0][0], q.double())
+    assert bool((got[0][1] == 7.0).any()) and not bool((got[0][1] == 7.0).all())

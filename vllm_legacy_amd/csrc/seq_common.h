@@ -53,6 +53,46 @@ __device__ __forceinline__ uint32_t pack16(float lo, float hi) {
          ((uint32_t)__builtin_bit_cast(uint16_t, S::from_f32(hi)) << 16);
 }
 
+// (which product is fused is said here, so that every kernel rounds alike)
+__device__ __forceinline__ void turn_by(float& a, float& b, float2 sc) {
+  const float a2 = fmaf(a, sc.y, -(b * sc.x));
+  b = fmaf(b, sc.y, a * sc.x);
+  a = a2;
+}
+
+// i / d for i < 2048 with inverse = 65536 / d rounded up, d <= 32
+__device__ __forceinline__ int quotient(int i, int inverse) { return (i * inverse) >> 16; }
+
+// Eight neighbouring pairs of a head, as two pieces of 16 bytes: pairs side by side, or the same places of the two pieces.
+struct TurnPieces {
+  u32x4 x, y;
+};
+template <class S>
+__device__ __forceinline__ TurnPieces turn_eight(TurnPieces in, const float2* sines, int interleaved) {
+  TurnPieces out;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const u32x4 two = *reinterpret_cast<const u32x4*>(sines + 2 * e);
+    const float2 s0 = {__builtin_bit_cast(float, (uint32_t)two[0]), __builtin_bit_cast(float, (uint32_t)two[1])};
+    const float2 s1 = {__builtin_bit_cast(float, (uint32_t)two[2]), __builtin_bit_cast(float, (uint32_t)two[3])};
+    const uint32_t wx = interleaved ? (e < 2 ? in.x[2 * e & 3] : in.y[2 * e & 3]) : in.x[e];
+    const uint32_t wy = interleaved ? (e < 2 ? in.x[(2 * e + 1) & 3] : in.y[(2 * e + 1) & 3]) : in.y[e];
+    float a0 = lo16<S>(wx), b0 = interleaved ? hi16<S>(wx) : lo16<S>(wy);
+    float a1 = interleaved ? lo16<S>(wy) : hi16<S>(wx), b1 = hi16<S>(wy);
+    turn_by(a0, b0, s0);
+    turn_by(a1, b1, s1);
+    const uint32_t u0 = pack16<S>(a0, interleaved ? b0 : a1), u1 = pack16<S>(interleaved ? a1 : b0, b1);
+    if (interleaved) {
+      (e < 2 ? out.x : out.y)[2 * e & 3] = u0;
+      (e < 2 ? out.x : out.y)[(2 * e + 1) & 3] = u1;
+    } else {
+      out.x[e] = u0;
+      out.y[e] = u1;
+    }
+  }
+  return out;
+}
+
 // sum over a workgroup of up to 1024 threads; red holds 16 floats; every thread gets the sum
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);

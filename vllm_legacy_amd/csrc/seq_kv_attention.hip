@@ -42,13 +42,6 @@ __device__ __forceinline__ void turn(float& a, float& b, float angle) {
   b = b * c + a * s;
   a = a2;
 }
-// (which product is fused is said here, so that every kernel rounds alike)
-__device__ __forceinline__ void turn_by(float& a, float& b, float2 sc) {
-  const float a2 = fmaf(a, sc.y, -(b * sc.x));
-  b = fmaf(b, sc.y, a * sc.x);
-  a = a2;
-}
-
 // cap * tanh(s / cap): libm's tanh in the fp32 kernel, one exponential and one reciprocal in the
 // matrix-core kernels (absolute error of a few 1e-7 times cap)
 __device__ __forceinline__ float cap_score(float s, float cap) { return cap * tanhf(s / cap); }
@@ -251,9 +244,6 @@ struct RotaryRows {
   int num_tokens, heads, kv_heads, dim, vdim, rot_dims, interleaved;
 };
 
-// i / d for i < 2048 with inverse = 65536 / d rounded up, d <= 32
-__device__ __forceinline__ int quotient(int i, int inverse) { return (i * inverse) >> 16; }
-
 bool rows_fit(const RotaryRows& a) {
   const int eighth = a.rot_dims / 16;    // pieces of pairs of a head
   const uintptr_t at = (uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.key_cache | (uintptr_t)a.value_cache;
@@ -288,44 +278,20 @@ __global__ __launch_bounds__(64 * kTurnWaves) void rotary_kv_rows_kernel(RotaryR
     j = i - h * eighth;
     return h * a.dim + (a.interleaved ? 16 : 8) * j;
   };
-  struct Pieces {
-    u32x4 x, y;
-  };
   auto fetch = [&](const T* row, int i) {
     int j;
     const T* at = row + where(i, j);
-    return Pieces{*reinterpret_cast<const u32x4*>(at), *reinterpret_cast<const u32x4*>(at + second)};
+    return TurnPieces{*reinterpret_cast<const u32x4*>(at), *reinterpret_cast<const u32x4*>(at + second)};
   };
-  auto turn_into = [&](T* row, int i, Pieces in) {
+  auto turn_into = [&](T* row, int i, TurnPieces in) {
     int j;
     T* at = row + where(i, j);
-    Pieces out;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      // pairs: neighbours, or the same places of the two pieces
-      const u32x4 two = *reinterpret_cast<const u32x4*>(&sines[w][8 * j + 2 * e]);
-      const float2 s0 = {__builtin_bit_cast(float, (uint32_t)two[0]), __builtin_bit_cast(float, (uint32_t)two[1])};
-      const float2 s1 = {__builtin_bit_cast(float, (uint32_t)two[2]), __builtin_bit_cast(float, (uint32_t)two[3])};
-      const uint32_t wx = a.interleaved ? (e < 2 ? in.x[2 * e & 3] : in.y[2 * e & 3]) : in.x[e];
-      const uint32_t wy = a.interleaved ? (e < 2 ? in.x[(2 * e + 1) & 3] : in.y[(2 * e + 1) & 3]) : in.y[e];
-      float a0 = lo16<S>(wx), b0 = a.interleaved ? hi16<S>(wx) : lo16<S>(wy);
-      float a1 = a.interleaved ? lo16<S>(wy) : hi16<S>(wx), b1 = hi16<S>(wy);
-      turn_by(a0, b0, s0);
-      turn_by(a1, b1, s1);
-      const uint32_t u0 = pack16<S>(a0, a.interleaved ? b0 : a1), u1 = pack16<S>(a.interleaved ? a1 : b0, b1);
-      if (a.interleaved) {
-        (e < 2 ? out.x : out.y)[2 * e & 3] = u0;
-        (e < 2 ? out.x : out.y)[(2 * e + 1) & 3] = u1;
-      } else {
-        out.x[e] = u0;
-        out.y[e] = u1;
-      }
-    }
+    const TurnPieces out = turn_eight<S>(in, &sines[w][8 * j], a.interleaved);
     *reinterpret_cast<u32x4*>(at) = out.x;
     *reinterpret_cast<u32x4*>(at + second) = out.y;
   };
   constexpr int QU = 4, VU = 2;
-  Pieces qp[QU], kp;
+  TurnPieces qp[QU], kp;
   u32x4 vp[VU];
 #pragma unroll
   for (int u = 0; u < QU; ++u)
