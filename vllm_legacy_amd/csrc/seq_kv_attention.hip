@@ -678,8 +678,9 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
     for (int i = 0; i < 16; ++i) o[n][i] = 0.f;
   float m = -INFINITY, top = 0.f, l = 0.f;            // top: m, and 0 where nothing was seen yet
   if (sinks != nullptr && active && kg == 0) {     // the denominator's first term, counted in one lane half
-    top = m = sinks[h] * 1.4426950408889634f;
-    l = hf == 0 ? 1.f : 0.f;
+    m = sinks[h] * 1.4426950408889634f;
+    top = m == -INFINITY ? 0.f : m;                   // (a sink that counts for nothing, also where base 2 overflows)
+    l = hf == 0 ? __builtin_amdgcn_exp2f(m - top) : 0.f;       // 1, 0 or, for an infinite one, NaN
   }
 
   // the first wave looks the rows of a tile up: the block id is read one step before it is used

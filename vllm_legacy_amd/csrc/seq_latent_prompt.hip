@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256 * KG, 2) void latent_prompt_kernel(LatentPrompt
   float m = -INFINITY, l = 0.f;
   if (a.sinks != nullptr && kg == 0) {                     // the denominator's first term, counted in one lane half
     m = a.sinks[h] * 1.4426950408889634f;
-    l = hf == 0 ? 1.f : 0.f;
+    l = hf == 0 ? __builtin_amdgcn_exp2f(m - (m == -INFINITY ? 0.f : m)) : 0.f;      // 1, 0 or, for an infinite one, NaN
   }
   float* carry = a.carry + ((int64_t)(t0 + c) * a.heads + h) * (VD + 4);
   if (ranged && a.key_first > 0 && c < nq && kg == 0) {               // where the range before this one ended
