@@ -255,6 +255,25 @@ def test_lengths_that_are_not_the_hosts():
     assert inside is None
 
 
+@pytest.mark.parametrize("seqs,fit", [(4, 2), (4, 0), (70, 66), (200, 130), (300, 290)])
+@pytest.mark.parametrize("window", [0, 400])
+def test_sequences_that_rows_were_not_gathered_for(seqs, fit, window):
+    """From the first sequence on that grew on the device all rows are NaN, those ahead of it what they are without; there
+    are more tiles of rows than the host's lengths have."""
+    from dataclasses import replace
+    lens, contexts = [40 + 37 * (i % 4) for i in range(seqs)], [90 + 11 * (i % 5) for i in range(seqs)]
+    grown = contexts[:fit] + [c + 200 for c in contexts[fit:]]
+    attn, batch, q, kv, gate, cache = layer_and_step(lens, grown, (2, 64, 0, 64, 64), window)
+    want = attn(q.clone(), kv, cache.clone(), batch, gate)
+    got = attn(q.clone(), kv, cache.clone(), replace(batch, host_context_lens=contexts), gate)
+    # (the first one may still find room among the rows of those behind it)
+    ends = [sum(n + c for n, c in zip(lens[:b + 1], grown)) for b in range(seqs)]
+    held = sum(1 for e in ends if e <= sum(lens) + sum(contexts))
+    rows = sum(lens[:held])
+    assert fit <= held < seqs and bool(want.isfinite().all())
+    assert torch.equal(got[:rows], want[:rows]) and bool(got[rows:].isnan().all())
+
+
 @pytest.mark.parametrize("workspace", [1 << 28, 1 << 22])
 def test_a_portion_of_a_long_context(workspace):
     """A hundred thousand cached tokens, all at once and in ranges, beside the latent kernel."""

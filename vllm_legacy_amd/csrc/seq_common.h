@@ -179,47 +179,81 @@ __device__ __forceinline__ float max_halves(float v) {
   return fmaxf(__builtin_bit_cast(float, (uint32_t)both[0]), __builtin_bit_cast(float, (uint32_t)both[1]));
 }
 
-// the sum over a wave, in every lane
-__device__ __forceinline__ int wave_total(int v) {
+// the sums over a wave's first 1, 2, .. lanes, each in its last lane
+__device__ __forceinline__ int wave_sums(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);      // row_shr 1, 2, 4, 8
   v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
   v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
   v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
   v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);     // row_bcast 15 to rows 1 and 3
   v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);     // row_bcast 31 to rows 2 and 3
-  return __builtin_amdgcn_readlane(v, 63);
+  return v;
 }
+
+// the sum over a wave, in every lane
+__device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_sums(v), 63); }
+
+// the first row of a sequence's cache that its new rows see
+__device__ __forceinline__ int first_formed(int context, int window) { return window > 0 ? max(0, context - window + 1) : 0; }
 
 // The `rank`-th of all tiles of 2^shift rows of a step's sequences, counted from those that walk the most keys (a
 // tile's level: how many tiles of keys lie ahead of its last row).  Every wave finds it for itself: a search over
 // the levels for the one whose tiles hold the rank, with the sequences in the lanes' registers.  Launching one
 // workgroup per tile of the longest sequence for every sequence instead left empty ones between the real ones:
 // workgroups go to the shader engines of an XCD in turn, an engine that is full holds all others up, and half the
-// chip stood idle for 40 of 98 us with four prompts of 2047, 1265, 483 and 1748 rows.  The search takes about 2 us
-// of a workgroup.  Returns the number of tiles; seq and tile are set
-// where the rank is below it.
+// chip stood idle for 40 of 98 us with four prompts of 2047, 1265, 483 and 1748 rows.  A sequence has at most `most` tiles,
+// so that the caller's bound on all of them holds whatever the lengths on the device are.
+// kGathered: a sequence's rows context .. and the keys ahead of them that its window sees lie one behind the other among
+// num_rows gathered ones (`before` of them ahead of it); those that do not end there have no tiles, nor have those
+// behind them (`fitting` sequences do).
 constexpr int kRankedChunks = 4;
 constexpr int kRankedSeqs = kRankedChunks * kWave;
-__device__ __forceinline__ int ranked_tile(int rank, int num_seqs, const int* __restrict__ query_start_loc,
-                                            const int* __restrict__ context_lens, int shift, int& seq, int& tile) {
+struct RankedTile {
+  int all, fitting;                                    // the tiles there are; below, where the rank is one of them:
+  int seq, tile;
+  int first_row, rows, context, before;                // the sequence's first row, its rows and what lies ahead of them
+};
+template <bool kGathered>
+__device__ __forceinline__ RankedTile ranked_tile(int rank, int num_seqs, const int* __restrict__ query_start_loc,
+                                                  const int* __restrict__ context_lens, int shift, int most,
+                                                  int window = 0, int num_rows = 0) {
   const int lane = threadIdx.x & 63, chunks = (num_seqs + kWave - 1) / kWave;
+  int begin[kRankedChunks], rows[kRankedChunks], context[kRankedChunks], before[kRankedChunks];
   int first[kRankedChunks], end[kRankedChunks];       // the levels of a sequence's tiles
-  int top = 0, all = 0;
+  RankedTile r = {0, num_seqs, 0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int k = 0; k < kRankedChunks; ++k) {
-    first[k] = end[k] = 0;
+    begin[k] = rows[k] = context[k] = 0;
+    const int s = k * kWave + lane;
+    if (k < chunks && s < num_seqs) {
+      begin[k] = query_start_loc[s];
+      rows[k] = query_start_loc[s + 1];
+      context[k] = context_lens[s];
+    }
+  }
+  int top = 0, behind = 0;
+  if constexpr (kGathered) r.fitting = 0;
+#pragma unroll
+  for (int k = 0; k < kRankedChunks; ++k) {
+    before[k] = first[k] = end[k] = 0;
     if (k < chunks) {
-      const int s = k * kWave + lane;
-      if (s < num_seqs) {
-        first[k] = context_lens[s] >> shift;
-        end[k] = first[k] + ((max(query_start_loc[s + 1] - query_start_loc[s], 0) + (1 << shift) - 1) >> shift);
+      rows[k] -= begin[k];
+      first[k] = context[k] >> shift;
+      end[k] = first[k] + min((max(rows[k], 0) + (1 << shift) - 1) >> shift, most);
+      if constexpr (kGathered) {
+        const int keys = context[k] + rows[k] - first_formed(context[k], window), sums = wave_sums(keys);
+        before[k] = behind + sums - keys;
+        const bool fits = behind + sums <= num_rows;
+        if (!fits) end[k] = first[k];
+        r.fitting += __popcll(__ballot(fits && k * kWave + lane < num_seqs));
+        behind += __builtin_amdgcn_readlane(sums, 63);
       }
-      all += end[k] - first[k];
+      r.all += end[k] - first[k];
       top = max(top, end[k]);
     }
   }
-  all = wave_total(all);
-  if (all <= rank) return all;
+  r.all = wave_total(r.all);
+  if (r.all <= rank) return r;
 #pragma unroll
   for (int x = 1; x < kWave; x <<= 1) top = max(top, __shfl_xor(top, x, 64));
   auto at_least = [&](int level) {                     // tiles of this level and above
@@ -249,14 +283,18 @@ __device__ __forceinline__ int ranked_tile(int rank, int num_seqs, const int* __
       if (left < n) {
         const uint64_t which = __ballot(here && __popcll(mask & ((1ull << lane) - 1)) == left);
         const int l = __ffsll((unsigned long long)which) - 1;
-        seq = k * kWave + l;
-        tile = lo - __builtin_amdgcn_readlane(first[k], l);
+        r.seq = k * kWave + l;
+        r.tile = lo - __builtin_amdgcn_readlane(first[k], l);
+        r.first_row = __builtin_amdgcn_readlane(begin[k], l);
+        r.rows = __builtin_amdgcn_readlane(rows[k], l);
+        r.context = __builtin_amdgcn_readlane(context[k], l);
+        r.before = __builtin_amdgcn_readlane(before[k], l);
       }
       left -= n;
     }
-  seq = __builtin_amdgcn_readfirstlane(seq);
-  tile = __builtin_amdgcn_readfirstlane(tile);
-  return all;
+  // (the compiler does not see that these are the same for all lanes)
+  for (int* x : {&r.seq, &r.tile, &r.first_row, &r.rows, &r.context, &r.before}) *x = __builtin_amdgcn_readfirstlane(*x);
+  return r;
 }
 
 __device__ __forceinline__ bool finite(float x) { return fabsf(x) <= 3.402823466e38f; }

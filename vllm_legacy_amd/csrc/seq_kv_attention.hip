@@ -627,7 +627,10 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
   int b = blockIdx.x / head_groups, tile_x = last_tile - (int)blockIdx.y;
   if (ranked_seqs > 0) {
     const int rank = first_rank + b;
-    if (ranked_tile(rank, ranked_seqs, query_start_loc, context_lens, __builtin_ctz(tile_rows), b, tile_x) <= rank) return;
+    const RankedTile found = ranked_tile<false>(rank, ranked_seqs, query_start_loc, context_lens, __builtin_ctz(tile_rows), 0x7fffff);
+    if (rank >= found.all) return;
+    b = found.seq;
+    tile_x = found.tile;
   }
   const int t_first = query_start_loc[b] + tile_rows * tile_x;
   const int n_tile = min(tile_rows, query_start_loc[b + 1] - t_first);

@@ -86,8 +86,6 @@ __device__ __forceinline__ uint32_t odd_halves(uint32_t x) {
   return ((x & kLow) == kLow ? 0xffffu : 0u) | ((x & kHigh) == kHigh ? 0xffff0000u : 0u);
 }
 
-__device__ __forceinline__ int first_formed(int context, int window) { return window > 0 ? max(0, context - window + 1) : 0; }
-
 // where sequence b's rows begin among all gathered rows (one wave; every lane gets it)
 __device__ __forceinline__ int gathered_before(const int* __restrict__ query_start_loc,
                                                const int* __restrict__ context_lens, int b, int window) {
@@ -140,7 +138,7 @@ struct LatentPrompt {
   const float* sinks;
   float* carry;                 // one sequence whose keys come in ranges: [T, heads, VD + 4], null otherwise
   int heads, dim, rot, vdim, rank, window, num_rows, row_tiles;
-  int ranked_seqs, tiles;       // ranked_seqs > 0: tiles are found by their rank, `tiles` of them are launched
+  int ranked_seqs, tiles;       // ranked_seqs > 0: tiles are found by their rank among at most `tiles`
   int key_first, key_total;     // the range's first key and all keys of the sequence
   float scale;
 };
@@ -162,30 +160,51 @@ __global__ __launch_bounds__(256 * KG, 2) void latent_prompt_kernel(LatentPrompt
   constexpr int kStep = kKeys * KG;                        // keys of a step: a tile for every group of four waves
   extern __shared__ __align__(16) unsigned char all_tiles[];
   const int h = blockIdx.x % a.heads;
-  auto one_tile = [&](int b, int tile) __attribute__((always_inline)) {
-  const int run = a.query_start_loc[b + 1] - a.query_start_loc[b];
+  const bool ranged = a.carry != nullptr, last_range = !ranged || a.key_first + a.num_rows == a.key_total;
+  int b = blockIdx.z, tile = a.row_tiles - 1 - (int)blockIdx.y;       // the longest walks first
+  int t_first, run, ctx, base;
+  if (a.ranked_seqs > 0) {
+    const int rank = blockIdx.x / a.heads;
+    const RankedTile found = ranked_tile<true>(rank, a.ranked_seqs, a.query_start_loc, a.context_lens, kGroupShift, a.row_tiles,
+                                               a.window, ranged ? 0x7fffffff : a.num_rows);
+    // the host gathered for other lengths than the device has: no answer for those behind, and none that looks like one
+    for (int i = rank; i < (a.ranked_seqs - found.fitting) * a.row_tiles; i += a.tiles) {
+      const int s = found.fitting + i / a.row_tiles, r = kRowsPerGroup * (i % a.row_tiles);
+      const int n = min(kRowsPerGroup, a.query_start_loc[s + 1] - a.query_start_loc[s] - r);
+      T* row = (T*)a.out + (int64_t)(a.query_start_loc[s] + r) * a.out_stride + (int64_t)h * a.vdim;
+      for (int e = threadIdx.x; e < n * a.vdim; e += 256 * KG) row[e / a.vdim * a.out_stride + e % a.vdim] = S::from_f32(NAN);
+    }
+    if (rank >= found.all) return;
+    tile = found.tile;
+    t_first = found.first_row;
+    run = found.rows;
+    ctx = found.context;
+    base = found.before;
+  } else {
+    t_first = a.query_start_loc[b];
+    run = a.query_start_loc[b + 1] - t_first;
+    ctx = a.context_lens[b];
+    base = ranged ? 0 : gathered_before(a.query_start_loc, a.context_lens, b, a.window);
+  }
   const int r0 = tile * kRowsPerGroup;
   if (r0 >= run) return;
-  int tid = threadIdx.x;
-  asm volatile("" : "+v"(tid));        // what follows from it is not kept over the loop around a tile
+  const int tid = threadIdx.x;
   const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);     // group of waves
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane((tid & 255) >> 6);
   unsigned char* smem = all_tiles + kg * (KTILE + RTILE + VTILE);
   const int hf = lane >> 5, c = lane & 31;
-  const bool ranged = a.carry != nullptr, last_range = !ranged || a.key_first + a.num_rows == a.key_total;
-  const int ctx = a.context_lens[b], first = first_formed(ctx, a.window) + (ranged ? a.key_first : 0);
-  const int base = ranged ? 0 : gathered_before(a.query_start_loc, a.context_lens, b, a.window);
+  const int first = first_formed(ctx, a.window) + (ranged ? a.key_first : 0);
   const int n_rows = min(kRowsPerGroup, run - r0);         // rows of this workgroup
   const int nq = min(kRowsPerWave, n_rows - kRowsPerWave * w);               // and of this wave (<= 0: none)
-  const int t0 = a.query_start_loc[b] + r0 + kRowsPerWave * w;
+  const int t0 = t_first + r0 + kRowsPerWave * w;
   // positions, counted from the first gathered key
   const int p0 = ctx + r0 + kRowsPerWave * w - first, pq = p0 + c;
   const int n_keys = min(ctx + run - first, a.num_rows);
   const int p_end = min(ctx + r0 + n_rows - 1 - first, n_keys - 1);
-  T* orow = (T*)a.out + (int64_t)(t0 + c) * a.out_stride + (int64_t)h * a.vdim + 4 * hf;
   if (ranged ? ctx + run - first != a.key_total - a.key_first : base + ctx + run - first > a.num_rows) {
-    // the host gathered for other lengths than the device has: no answer, and none that looks like one
+    // other lengths again
     const uint32_t nan2 = M::pack2(NAN, NAN);
+    T* orow = (T*)a.out + (int64_t)(t0 + c) * a.out_stride + (int64_t)h * a.vdim + 4 * hf;
     for (int d = 0; c < nq && d + 4 * hf < a.vdim; d += 8) *reinterpret_cast<u32x2*>(orow + d) = u32x2{nan2, nan2};
     return;
   }
@@ -216,8 +235,8 @@ __global__ __launch_bounds__(256 * KG, 2) void latent_prompt_kernel(LatentPrompt
     m = a.sinks[h] * 1.4426950408889634f;
     l = hf == 0 ? __builtin_amdgcn_exp2f(m - (m == -INFINITY ? 0.f : m)) : 0.f;      // 1, 0 or, for an infinite one, NaN
   }
-  float* carry = a.carry + ((int64_t)(t0 + c) * a.heads + h) * (VD + 4);
   if (ranged && a.key_first > 0 && c < nq && kg == 0) {               // where the range before this one ended
+    const float* carry = a.carry + ((int64_t)(t0 + c) * a.heads + h) * (VD + 4);
     m = carry[0];
     l = carry[1 + hf];
 #pragma unroll
@@ -462,44 +481,36 @@ __global__ __launch_bounds__(256 * KG, 2) void latent_prompt_kernel(LatentPrompt
       for (int i = 0; i < 16; ++i) o[n][i] = o[n][i] * f + part[(2 + 16 * n + i) * kWave] * f2;
     m = m_new;
   }
+  // (this lane's row and half again: what follows from them would be kept through the loop, which has no registers left)
+  int me = threadIdx.x;
+  asm volatile("" : "+v"(me));
+  const int row = t0 + (me & 31), half = (me >> 5) & 1;
   if (!last_range) {
-    if (c >= nq) return;
-    if (hf == 0) carry[0] = m;
-    carry[1 + hf] = l;
+    if (row >= t0 + nq) return;
+    float* carry = a.carry + ((int64_t)row * a.heads + h) * (VD + 4);
+    if (half == 0) carry[0] = m;
+    carry[1 + half] = l;
 #pragma unroll
     for (int n = 0; n < VB; ++n)
 #pragma unroll
       for (int i = 0; i < 16; i += 4)
-        *reinterpret_cast<f32x4*>(carry + 4 + 32 * n + 8 * (i >> 2) + 4 * hf) = f32x4{o[n][i], o[n][i + 1], o[n][i + 2], o[n][i + 3]};
+        *reinterpret_cast<f32x4*>(carry + 4 + 32 * n + 8 * (i >> 2) + 4 * half) = f32x4{o[n][i], o[n][i + 1], o[n][i + 2], o[n][i + 3]};
     return;
   }
   l += __shfl_xor(l, 32, 64);
-  if (c >= nq) return;
+  if (row >= t0 + nq) return;
+  T* orow = (T*)a.out + (int64_t)row * a.out_stride + (int64_t)h * a.vdim + 4 * half;
   float inv = 1.f / l;
-  if (a.gate != nullptr) inv /= 1.f + expf(-S::to_f32(((const T*)a.gate)[(int64_t)(t0 + c) * a.gate_stride + h]));
+  if (a.gate != nullptr) inv /= 1.f + expf(-S::to_f32(((const T*)a.gate)[(int64_t)row * a.gate_stride + h]));
 #pragma unroll
   for (int n = 0; n < VB; ++n)
 #pragma unroll
     for (int i = 0; i < 16; i += 4) {
       const int d = 32 * n + 8 * (i >> 2);
-      if (d + 4 * hf < a.vdim)
+      if (d + 4 * half < a.vdim)
         *reinterpret_cast<u32x2*>(orow + d) =
             u32x2{M::pack2(o[n][i] * inv, o[n][i + 1] * inv), M::pack2(o[n][i + 2] * inv, o[n][i + 3] * inv)};
     }
-  };
-  // (a second tile only where the sequences are longer than the host's lengths say)
-  int rank = a.ranked_seqs > 0 ? blockIdx.x / a.heads : 0, all = 1;
-  for (;;) {
-    int b = blockIdx.z, tile = a.row_tiles - 1 - (int)blockIdx.y;       // the longest walks first
-    if (a.ranked_seqs > 0) {
-      all = ranked_tile(rank, a.ranked_seqs, a.query_start_loc, a.context_lens, kGroupShift, b, tile);
-      if (rank >= all) return;
-    }
-    one_tile(b, tile);
-    rank += a.tiles;
-    if (rank >= all) return;
-    __syncthreads();
-  }
 }
 
 template <class S, int DB, int VB, int LB, int KG>
@@ -608,7 +619,8 @@ extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* 
   a.row_tiles = (max_query_len + kRowsPerGroup - 1) / kRowsPerGroup;
   a.scale = scale;
   if (a.row_tiles > 65535) return VLA_ERR_ARG;
-  // every query row is a gathered row, too (a range's launch: one sequence)
+  // Every query row is a gathered row, too (a range's launch: one sequence).  The bound holds whatever the lengths on the
+  // device are: sequences have at most row_tiles tiles, and only those whose rows were gathered have any.
   const int64_t tiles = std::min((int64_t)num_seqs * a.row_tiles, carry ? (int64_t)a.row_tiles : (int64_t)num_rows / kRowsPerGroup + num_seqs);
   const bool ranked = num_seqs <= kRankedSeqs && tiles * heads <= 0xffffff;
   a.ranked_seqs = ranked ? num_seqs : 0;
