@@ -193,6 +193,17 @@ __device__ __forceinline__ int wave_sums(int v) {
 // the sum over a wave, in every lane
 __device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_sums(v), 63); }
 
+// the largest of a wave's values, none of them negative, in every lane
+__device__ __forceinline__ int wave_most(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // the first row of a sequence's cache that its new rows see
 __device__ __forceinline__ int first_formed(int context, int window) { return window > 0 ? max(0, context - window + 1) : 0; }
 
@@ -221,6 +232,15 @@ __device__ __forceinline__ RankedTile ranked_tile(int rank, int num_seqs, const 
   int begin[kRankedChunks], rows[kRankedChunks], context[kRankedChunks], before[kRankedChunks];
   int first[kRankedChunks], end[kRankedChunks];       // the levels of a sequence's tiles
   RankedTile r = {0, num_seqs, 0, 0, 0, 0, 0, 0};
+  if (num_seqs == 1) {                                 // its last tile is the first
+    r.first_row = query_start_loc[0];
+    r.rows = query_start_loc[1] - r.first_row;
+    r.context = context_lens[0];
+    r.all = min((max(r.rows, 0) + (1 << shift) - 1) >> shift, most);
+    if (kGathered && r.context + r.rows - first_formed(r.context, window) > num_rows) r.all = r.fitting = 0;
+    r.tile = r.all - 1 - rank;
+    return r;
+  }
 #pragma unroll
   for (int k = 0; k < kRankedChunks; ++k) {
     begin[k] = rows[k] = context[k] = 0;
@@ -254,8 +274,6 @@ __device__ __forceinline__ RankedTile ranked_tile(int rank, int num_seqs, const 
   }
   r.all = wave_total(r.all);
   if (r.all <= rank) return r;
-#pragma unroll
-  for (int x = 1; x < kWave; x <<= 1) top = max(top, __shfl_xor(top, x, 64));
   auto at_least = [&](int level) {                     // tiles of this level and above
     int n = 0;
 #pragma unroll
@@ -263,7 +281,7 @@ __device__ __forceinline__ RankedTile ranked_tile(int rank, int num_seqs, const 
       if (k < chunks) n += max(end[k] - max(first[k], level), 0);
     return wave_total(n);
   };
-  int lo = 0, hi = __builtin_amdgcn_readfirstlane(top), above = 0;      // at_least(lo) > rank >= at_least(hi) = above
+  int lo = 0, hi = wave_most(top), above = 0;      // at_least(lo) > rank >= at_least(hi) = above
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1, n = at_least(mid);
     if (n > rank) {

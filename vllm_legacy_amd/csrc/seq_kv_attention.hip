@@ -625,15 +625,23 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
   const int tile_rows = kTile * row_blocks;
   // the last tiles of a run have the most keys to walk: they are dispatched first
   int b = blockIdx.x / head_groups, tile_x = last_tile - (int)blockIdx.y;
+  int first_row, run, context;
   if (ranked_seqs > 0) {
     const int rank = first_rank + b;
-    const RankedTile found = ranked_tile<false>(rank, ranked_seqs, query_start_loc, context_lens, __builtin_ctz(tile_rows), 0x7fffff);
+    const RankedTile found = ranked_tile<false>(rank, ranked_seqs, query_start_loc, context_lens, __builtin_ctz(tile_rows), last_tile + 1);
     if (rank >= found.all) return;
     b = found.seq;
     tile_x = found.tile;
+    first_row = found.first_row;
+    run = found.rows;
+    context = found.context;
+  } else {
+    first_row = query_start_loc[b];
+    run = query_start_loc[b + 1] - first_row;
+    context = context_lens[b];
   }
-  const int t_first = query_start_loc[b] + tile_rows * tile_x;
-  const int n_tile = min(tile_rows, query_start_loc[b + 1] - t_first);
+  const int t_first = first_row + tile_rows * tile_x;
+  const int n_tile = min(tile_rows, run - tile_rows * tile_x);
   if (n_tile <= 0) return;
   const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);      // group of waves
   const int tid = threadIdx.x & 255, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -648,7 +656,7 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
   const int t0 = t_first + kTile * rb;
   const int nq = min(kTile, n_tile - kTile * rb);     // <= 0: no rows for this wave
   const bool active = h < g * group + group && nq > 0;
-  const int p_first = context_lens[b] + tile_rows * tile_x, p_last = p_first + n_tile - 1;
+  const int p_first = context + tile_rows * tile_x, p_last = p_first + n_tile - 1;
   const int p0 = p_first + kTile * rb;                // this wave's first position
   const int pq = p0 + c;
   // (the compiler does not see that a remainder is the same for all lanes, and would take every branch on it for one
@@ -1605,7 +1613,8 @@ int launch_heads_one(dim3 grid, hipStream_t stream, typename S::T* out, int64_t 
 }
 
 struct TileGrid {
-  int64_t tiles;        // ranked: at most this many tiles of rows; otherwise those of the longest sequence
+  int64_t tiles;        // at most this many tiles of rows, of all sequences
+  int of_longest;       // and of one
   int num_seqs, head_groups, key_groups;
 };
 
@@ -1631,7 +1640,7 @@ int launch_tiles_one(TileGrid to, hipStream_t stream, typename S::T* out, int64_
   const int64_t most = std::max(1, 0xffffff / (to.head_groups * to.key_groups));
   if (to.num_seqs <= kRankedSeqs) {
     for (int64_t r = 0; r < to.tiles; r += most) {
-      const int rc = go(dim3(to.head_groups * (unsigned)std::min(most, to.tiles - r)), 0, 0, to.num_seqs, (int)r);
+      const int rc = go(dim3(to.head_groups * (unsigned)std::min(most, to.tiles - r)), 0, to.of_longest - 1, to.num_seqs, (int)r);
       if (rc != VLA_OK) return rc;
     }
     return VLA_OK;
@@ -1640,7 +1649,7 @@ int launch_tiles_one(TileGrid to, hipStream_t stream, typename S::T* out, int64_
   // launches, the last rows first
   constexpr int kSide = 65535;
   for (int64_t b0 = 0; b0 < to.num_seqs; b0 += most)
-    for (int left = (int)to.tiles; left > 0; left -= kSide) {
+    for (int left = to.of_longest; left > 0; left -= kSide) {
       const dim3 grid(to.head_groups * (unsigned)std::min(most, to.num_seqs - b0), std::min(left, kSide));
       const int rc = go(grid, (int)b0, left - 1, 0, 0);
       if (rc != VLA_OK) return rc;
@@ -1950,7 +1959,7 @@ extern "C" int vla_seq_kv_attention_tiles_of(
   const int64_t of_longest = (max_query_len + tile_rows - 1) / tile_rows;
   const int64_t tiles = std::min(num_seqs * of_longest, num_rows / tile_rows + num_seqs);     // of all sequences, at most
   const int key_groups = head_groups * tiles <= 512 ? 2 : 1;
-  const TileGrid to{num_seqs <= kRankedSeqs ? tiles : of_longest, num_seqs, head_groups, key_groups};
+  const TileGrid to{tiles, (int)of_longest, num_seqs, head_groups, key_groups};
   auto go = [&](auto tag) {
     using S = decltype(tag);
     using T = typename S::T;
