@@ -260,7 +260,7 @@ int vla_seq_kv_attention_shared(void* out, int64_t out_stride, const void* q, in
  * the matrix cores: rows query_start_loc[b] .. query_start_loc[b + 1] - 1 of sequence b sit at
  * positions context_lens[b] ...  dim must be a multiple of 32 up to 128, vdim one up to 512 (values of
  * more than 128 dims in slices, a launch each; up to 128 with out_inv_freq)
- * (vla_seq_kv_attention_tiles_supported; turned: with out_inv_freq); query rows and cache rows must be 8-byte aligned.
+ * (vla_seq_kv_attention_tiles_supported; turned: with out_inv_freq); query rows and cache rows must be 16-byte aligned.
  * vla_seq_kv_attention takes single rows of such shapes to the matrix cores by itself;
  * vla_seq_set_kv_attention_kernel(1) keeps both off them (tests run both), 0 is the default. */
 int vla_seq_kv_attention_tiles_supported(int dim, int vdim, int turned, int dtype);
@@ -273,7 +273,12 @@ int vla_seq_kv_attention_tiles(void* out, int64_t out_stride, const void* q, int
                                int block_size, int num_blocks, int window, float scale, int dtype,
                                int keep_first, float softcap, int chunk, const float* sinks,
                                void* stream);
-/* The same for a step of num_rows rows in all (sequences of different lengths launch no more than they need). */
+/* The same for a step of num_rows rows in all (sequences of different lengths launch no more than they need).
+ * vla_seq_kv_attention_tiles_form: how it does: 1 or 2 groups of waves share a workgroup's keys (a group rounds its
+ * weights against a maximum of its own, so a row's bits may depend on the step that it is in), and 4 more where tiles of
+ * rows are found by their rank and not by the grid. */
+int vla_seq_kv_attention_tiles_form(int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads,
+                                    int max_blocks, int block_size, int window, int keep_first, int chunk);
 int vla_seq_kv_attention_tiles_of(void* out, int64_t out_stride, const void* q, int64_t q_stride,
                                   const void* gate, int64_t gate_stride, const void* key_cache,
                                   const void* value_cache, const int* block_tables, int max_blocks,
@@ -448,7 +453,10 @@ int vla_seq_gla_chunks(void* out, int64_t out_stride, const void* q, int64_t q_s
  * 64) of its key_total visible ones on, whole tiles of 64 except at the end, and carry, fp32 [T, heads, 68 or
  * (vdim above 64) 132], 16-byte aligned, in which a call leaves what the next goes on from.  The call with
  * key_first 0 starts, the one that ends at key_total writes out.  All keys at once: 0, 0 and null.
- * Rows of a sequence whose lengths on the device are not those that rows were gathered for are NaN. */
+ * Rows of a sequence whose lengths on the device are not those that rows were gathered for are NaN.
+ * vla_seq_latent_prompt_form: how it does (ranged: with a carry), as vla_seq_kv_attention_tiles_form. */
+int vla_seq_latent_prompt_form(int num_rows, int num_seqs, int max_query_len, int heads, int dim, int rot, int vdim,
+                               int ranged);
 int vla_seq_latent_prompt_supported(int dim, int rot, int vdim, int rank, int dtype);
 int vla_seq_latent_gather(void* rows, int num_rows, const void* cache, const int* block_tables,
                           int max_blocks, const int* query_start_loc, const int* context_lens, int num_seqs,

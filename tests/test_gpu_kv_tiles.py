@@ -1,8 +1,7 @@
 """Runs of query rows on the LDS-DMA tile kernel: every key and value size class it exchanges differently, groups of
 1 to 4 heads, pages of 1, 4 and 16 tokens, runs around its tiles of 32 rows and 64 keys, windows, chunks, kept
-first tokens, caps, sinks, gates, values that turn back, scales of either sign, outputs at odd addresses, both
-with the keys shared out to two groups of waves and (many sequences) with one, with tiles found by their rank (up to
-256 sequences, one to four registers a lane) and by the grid (more) -- against the same attention in
+first tokens, caps, sinks, gates, values that turn back, scales of either sign, outputs at odd addresses, one to 1200
+sequences of nearly equal lengths (uneven ones in every way that a step is shared out: test_gpu_uneven_prompts.py) -- against the same attention in
 float64 and the bound of the single rows' test: 1 % of the largest value in bfloat16, an eighth in float16."""
 import pytest
 import torch

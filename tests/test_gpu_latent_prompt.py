@@ -220,19 +220,22 @@ def test_rows_that_do_not_see_one_that_is_not_finite(row, window, value):
 
 
 @pytest.mark.parametrize("seqs", [1, 40, 65, 130, 256, 257, 300])
-@pytest.mark.parametrize("window", [0, 90])
+@pytest.mark.parametrize("window", [0, 600])
 def test_one_group_of_waves_and_two(seqs, window):
     """Many workgroups have one group of waves and find their tiles by their rank (up to 256 sequences) or by the grid;
     a small workspace makes few of them, which share a tile's keys out to two groups: one rounding of an output."""
-    lens, contexts = [129 + 11 * (i % 13) for i in range(seqs)], [7 * (i % 9) for i in range(seqs)]
+    from vllm_legacy_amd import _lib
+    lens, contexts = [129 + 11 * (i % 13) for i in range(seqs)], [420 + 7 * (i % 9) for i in range(seqs)]
     sizes = (4, 128, 64, 128, 128)
     attn, batch, q, kv, gate, cache = layer_and_step(lens, contexts, sizes, window)
-    assert (4 * ((sum(lens) + sum(contexts)) // 128 + seqs) > 512) == (seqs > 40)
+    form = lambda n, c: _lib.seq_lib().vla_seq_latent_prompt_form(sum(n) + sum(c), len(n), max(n), 4, 128, 64, 128, 0)
+    assert form(lens, contexts) == (1 if seqs > 256 else 5 if seqs > 30 else 6) and form(lens[:3], contexts[:3]) == 6
     want = attn(q.clone(), kv, cache.clone(), batch, gate)
     attn.FORMED_WORKSPACE = 2048 * 2 * (128 + 64 + 4 * 384)
     got = attn(q.clone(), kv, cache.clone(), batch, gate)
     assert float((got - want).abs().max()) <= 0.008 * float(want.abs().max())
     assert float(want.abs().max()) > 0.1 and bool(want.isfinite().all())
+    assert torch.equal(got, want) == (seqs == 1)
 
 
 def test_lengths_that_are_not_the_hosts():

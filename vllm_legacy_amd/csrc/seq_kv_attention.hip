@@ -636,6 +636,11 @@ __global__ __launch_bounds__(256 * KG, 2) void kv_attention_tile_kernel(
     run = found.rows;
     context = found.context;
   } else {
+    if (ranked_seqs < 0) {                            // in the order of the rows
+      const int at = first_rank + b;
+      b = at / (last_tile + 1);
+      tile_x = last_tile - (at - b * (last_tile + 1));
+    }
     first_row = query_start_loc[b];
     run = query_start_loc[b + 1] - first_row;
     context = context_lens[b];
@@ -1615,8 +1620,47 @@ int launch_heads_one(dim3 grid, hipStream_t stream, typename S::T* out, int64_t 
 struct TileGrid {
   int64_t tiles;        // at most this many tiles of rows, of all sequences
   int of_longest;       // and of one
-  int num_seqs, head_groups, key_groups;
+  int num_seqs, head_waves, head_groups, key_groups;
+  bool ranked;          // a tile is found by its rank, not by the grid
+  bool in_order;        // the grid goes through the rows in order, not through the last tiles of all sequences first
 };
+
+// num_rows rows in all, walks of at most `keys` keys.
+// Two groups of four waves, one workgroup a CU, share a workgroup's keys where there are few workgroups: of 16 heads on 4
+// of 128, a run of 2047 rows (256 of them) takes 44 us instead of 52, one of 4096 (512) 103 instead of 114, 16 of 96 to
+// 256 rows behind up to 3000 keys (436) 63 instead of 76; 700 fill the chip with independent ones (62 instead of 73).
+// Between one and two workgroups a CU it needs walks of some length: 40 runs of up to 100 rows 22 us with two groups, 14 with
+// one; behind 300 keys 27 and 21; a run of 256 rows beside 60 of 20 19 and 14.
+// By their rank, so that none is empty and the longest walks go out first: not where no workgroup is empty and the walks are
+// short: the search is a wait for memory more, 256 runs of 33 rows take 42 us with it and 39 without, 128 of 64 48
+// and 39; (one sequence does without in any case).
+// In the order of the rows where all runs are the same whole tiles: tiles of the same number lie at the same distance from
+// each other and meet in the same memory channels (128 runs of 64 rows 26 us, last tiles first 47; 64 of 128 28 and 43; of
+// 60 rows 28 and 27, which is why other runs keep that order).
+TileGrid tile_grid(int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads, int64_t keys) {
+  TileGrid to;
+  const int group = heads / kv_heads;
+  to.num_seqs = num_seqs;
+  to.head_waves = group >= 3 ? 4 : group;      // waves of a workgroup that are heads
+  const int tile_rows = kTile * (4 / to.head_waves);
+  to.head_groups = kv_heads * ((group + to.head_waves - 1) / to.head_waves);
+  to.of_longest = (max_query_len + tile_rows - 1) / tile_rows;
+  const int64_t all = (int64_t)num_seqs * to.of_longest;
+  to.tiles = std::min(all, num_rows / tile_rows + num_seqs);
+  const int64_t workgroups = to.head_groups * to.tiles;
+  to.key_groups = workgroups <= 256 || (workgroups <= 512 && keys > 512) ? 2 : 1;
+  to.in_order = keys <= 128 && max_query_len % tile_rows == 0 && num_rows == (int64_t)num_seqs * max_query_len;
+  to.ranked = num_seqs <= kRankedSeqs && !to.in_order && !(to.tiles == all && keys <= 256);
+  return to;
+}
+
+// the most keys that a workgroup's rows walk
+int64_t walked_keys(int max_blocks, int block_size, int window, int keep_first, int chunk) {
+  int64_t keys = (int64_t)max_blocks * block_size;
+  if (window > 0) keys = std::min(keys, (int64_t)window + 4 * kTile + keep_first);
+  if (chunk > 0) keys = std::min(keys, (int64_t)chunk + 4 * kTile + keep_first);
+  return keys;
+}
 
 template <class S, int DB, int VB>
 int launch_tiles_one(TileGrid to, hipStream_t stream, typename S::T* out, int64_t out_stride,
@@ -1625,22 +1669,23 @@ int launch_tiles_one(TileGrid to, hipStream_t stream, typename S::T* out, int64_
                      const typename S::T* value_cache, const int* block_tables, int max_blocks,
                      const int* qsl, const int* ctx, const float* out_inv_freq, int interleaved,
                      int heads, int kv_heads, int block_size, int num_blocks, int window,
-                     float scale, int head_waves, int keep_first, float softcap, int chunk,
+                     float scale, int keep_first, float softcap, int chunk,
                      const float* sinks, int v_row, int v_first) {
   auto go = [&](dim3 grid, int b0, int last_tile, int ranked_seqs, int first_rank) -> int {
     auto* kernel = to.key_groups == 2 ? &kv_attention_tile_kernel<S, DB, VB, 2> : &kv_attention_tile_kernel<S, DB, VB, 1>;
     kernel<<<grid, 256 * to.key_groups, 0, stream>>>(
         out, out_stride, q, q_stride, gate, gate_stride, key_cache, value_cache, block_tables + (int64_t)b0 * max_blocks,
         max_blocks, qsl + b0, ctx + b0, out_inv_freq, interleaved, heads, kv_heads, to.head_groups, block_size, num_blocks,
-        window, scale, head_waves, keep_first, softcap, chunk, sinks, v_row, v_first, last_tile, ranked_seqs, first_rank);
+        window, scale, to.head_waves, keep_first, softcap, chunk, sinks, v_row, v_first, last_tile, ranked_seqs, first_rank);
     VLA_SEQ_HIP_CHECK(hipGetLastError());
     return VLA_OK;
   };
   // a launch counts its threads in 32 bits: more than 16.7 million groups of heads go in several launches
   const int64_t most = std::max(1, 0xffffff / (to.head_groups * to.key_groups));
-  if (to.num_seqs <= kRankedSeqs) {
+  if (to.ranked || to.in_order) {
     for (int64_t r = 0; r < to.tiles; r += most) {
-      const int rc = go(dim3(to.head_groups * (unsigned)std::min(most, to.tiles - r)), 0, to.of_longest - 1, to.num_seqs, (int)r);
+      const int rc = go(dim3(to.head_groups * (unsigned)std::min(most, to.tiles - r)), 0, to.of_longest - 1,
+                        to.ranked ? to.num_seqs : -1, (int)r);
       if (rc != VLA_OK) return rc;
     }
     return VLA_OK;
@@ -1910,6 +1955,16 @@ extern "C" int vla_seq_kv_attention_tiles_supported(int dim, int vdim, int turne
          g_kv_kernel.load(std::memory_order_relaxed) == 0;
 }
 
+extern "C" int vla_seq_kv_attention_tiles_form(int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads,
+                                               int max_blocks, int block_size, int window, int keep_first, int chunk) {
+  if (num_seqs <= 0 || max_query_len <= 0 || num_rows < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 ||
+      max_blocks <= 0 || block_size <= 0)
+    return 0;
+  const TileGrid to = tile_grid(num_seqs, max_query_len, num_rows, heads, kv_heads,
+                                walked_keys(max_blocks, block_size, window, window > 0 || chunk > 0 ? keep_first : 0, chunk));
+  return to.key_groups + (to.ranked ? 4 : 0);
+}
+
 extern "C" int vla_seq_kv_attention_tiles(
     void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* gate,
     int64_t gate_stride, const void* key_cache, const void* value_cache, const int* block_tables,
@@ -1949,17 +2004,8 @@ extern "C" int vla_seq_kv_attention_tiles_of(
   if (((uintptr_t)q % 16) || ((q_stride * 2) % 16) || ((uintptr_t)key_cache % 16) ||
       ((uintptr_t)value_cache % 16))
     return VLA_ERR_ARG;
-  const int group = heads / kv_heads;
-  const int head_waves = group >= 3 ? 4 : group;      // waves of a workgroup that are heads
-  const int tile_rows = kTile * (4 / head_waves);
-  const int head_groups = kv_heads * ((group + head_waves - 1) / head_waves);
-  // few workgroups share their keys out to two groups of four waves, one workgroup a CU: of 16 heads on 4 of 128, a run
-  // of 2047 rows (256 workgroups) takes 41 us instead of 49, runs of 2047 and 1265 45 instead of 55, of 4096 rows (512) 95
-  // instead of 109; 700 workgroups fill the chip with independent ones (62 instead of 73 us)
-  const int64_t of_longest = (max_query_len + tile_rows - 1) / tile_rows;
-  const int64_t tiles = std::min(num_seqs * of_longest, num_rows / tile_rows + num_seqs);     // of all sequences, at most
-  const int key_groups = head_groups * tiles <= 512 ? 2 : 1;
-  const TileGrid to{tiles, (int)of_longest, num_seqs, head_groups, key_groups};
+  const TileGrid to = tile_grid(num_seqs, max_query_len, num_rows, heads, kv_heads,
+                                walked_keys(max_blocks, block_size, window, keep_first, chunk));
   auto go = [&](auto tag) {
     using S = decltype(tag);
     using T = typename S::T;
@@ -1967,7 +2013,7 @@ extern "C" int vla_seq_kv_attention_tiles_of(
       return launch_tiles<S>(dim / 32, vb, to, (hipStream_t)stream, (T*)out, out_stride, (const T*)q, q_stride,
                              (const T*)gate, gate_stride, (const T*)key_cache, (const T*)value_cache, block_tables,
                              max_blocks, query_start_loc, context_lens, out_inv_freq, interleaved, heads, kv_heads,
-                             block_size, num_blocks, window, scale, head_waves, keep_first, softcap, chunk, sinks, vdim, v_first);
+                             block_size, num_blocks, window, scale, keep_first, softcap, chunk, sinks, vdim, v_first);
     });
   };
   return dtype == VLA_BF16 ? go(BF16{}) : go(F16{});

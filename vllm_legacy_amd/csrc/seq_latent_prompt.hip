@@ -30,10 +30,12 @@
 // ones and a key tile's ahead of and between the second ones, and weights are formed between those (184 us and bursts
 // behind the barriers before).
 //
-// Workgroups go out longest walk first over all sequences (ranked_tile), heads next to each other.  Up to 512 of
-// them have two groups of four waves, a CU each, that take every other tile and join their sums at the end: with
+// Workgroups go out longest walk first over all sequences (ranked_tile), heads next to each other.  Few of
+// them (prompt_form) have two groups of four waves, a CU each, that take every other tile and join their sums at the end: with
 // one group, two workgroups to a CU, all 512 of a run of 4096 rows are on the chip at once and the ones with 64 tiles
-// stay alone on their CUs (168 us; 2048 rows 72 instead of 60).  A wave alone takes 4400 cycles for a tile, 1800 of
+// stay alone on their CUs (165 us instead of 150; 2048 rows 70 instead of 59).  Each group rounds its weights to 16 bits against
+// a maximum of its own: a row's bits differ by one rounding between steps of one form and the other (errors against 64 bits
+// do not).  A wave alone takes 4400 cycles for a tile, 1800 of
 // products; two on a SIMD 6300 for one each, at 1.6 GHz, where the card holds its power.  Taken back: the second group
 // half a step behind the first (with two tiles of values: 157), raised priority for the first product (162).
 #include <algorithm>
@@ -534,6 +536,32 @@ int launch_latent_prompt(const LatentPrompt& a, dim3 grid, int key_groups, hipSt
                          : launch_latent_prompt_groups<S, DB, VB, LB, 1>(a, grid, stream);
 }
 
+// How many tiles of rows there are at most, how many groups of waves share a workgroup's keys, and whether a tile is found
+// by its rank.  Every query row is a gathered row, too (a range's launch: one sequence).  The bound holds whatever the
+// lengths on the device are: sequences have at most row_tiles tiles, and only those whose rows were gathered have any.
+// Two groups where a CU has one workgroup and the walks are long enough for two (16 heads of 128 + 64, values of 128: one
+// run of 512 rows 22 us with two groups, 23 with one; 16 of 128 behind 300 keys 29 and 28; 128 rows behind 2000 60 and 71;
+// four heads of 64 + 32 and 64: 12 runs of 50 to 500 rows 16 and 18, 16 of 128 10 and 9.5), or where long runs have walks
+// of all lengths (one of 4096 rows 152 and 165, two of 2048 78 and 83, three of 1024 behind 1000 95 and 88, 32 of 33 18
+// and 10, eight of 512 42 and 31, 16 of 256 behind 2000 202 and 150).  The bound may be a few workgroups too high.
+// Not by their rank where no workgroup is empty and the walks are short, as key / value prompts: 256 runs of 33 rows 72
+// and 67 us, 128 of 128 101 and 98.
+struct PromptForm {
+  int64_t tiles;
+  int key_groups;
+  bool ranked;
+};
+PromptForm prompt_form(int num_rows, int num_seqs, int max_query_len, int heads, int dim, int rot, int vdim, bool ranged) {
+  const int64_t row_tiles = ((int64_t)max_query_len + kRowsPerGroup - 1) / kRowsPerGroup, all = num_seqs * row_tiles;
+  PromptForm form;
+  form.tiles = std::min(all, ranged ? row_tiles : (int64_t)num_rows / kRowsPerGroup + num_seqs);
+  const int64_t workgroups = form.tiles * heads, keys = num_rows / num_seqs;
+  const bool wide = dim + rot > 128 || vdim > 64;
+  form.key_groups = (workgroups <= 288 && keys >= (wide ? 512 : 129)) || (workgroups <= 512 && max_query_len > 1024) ? 2 : 1;
+  form.ranked = num_seqs <= kRankedSeqs && workgroups <= 0xffffff && !(form.tiles == all && num_seqs > 1 && keys <= 256);
+  return form;
+}
+
 bool prompt_sizes(int dim, int rot, int vdim, int rank) {
   return dim > 0 && dim % 8 == 0 && rot >= 0 && rot % 8 == 0 && vdim > 0 && vdim % 8 == 0 && rank > 0 && rank % 8 == 0 &&
          dim + rot <= 192 && vdim <= 128;
@@ -566,6 +594,13 @@ extern "C" int vla_seq_latent_gather(void* rows, int num_rows, const void* cache
       num_blocks, window, num_rows, key_first);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   return VLA_OK;
+}
+
+extern "C" int vla_seq_latent_prompt_form(int num_rows, int num_seqs, int max_query_len, int heads, int dim, int rot, int vdim,
+                                         int ranged) {
+  if (num_rows <= 0 || num_seqs <= 0 || max_query_len <= 0 || heads <= 0) return 0;
+  const PromptForm form = prompt_form(num_rows, num_seqs, max_query_len, heads, dim, rot, vdim, ranged != 0);
+  return form.key_groups + (form.ranked ? 4 : 0);
 }
 
 extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* q, int64_t q_stride,
@@ -619,14 +654,11 @@ extern "C" int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* 
   a.row_tiles = (max_query_len + kRowsPerGroup - 1) / kRowsPerGroup;
   a.scale = scale;
   if (a.row_tiles > 65535) return VLA_ERR_ARG;
-  // Every query row is a gathered row, too (a range's launch: one sequence).  The bound holds whatever the lengths on the
-  // device are: sequences have at most row_tiles tiles, and only those whose rows were gathered have any.
-  const int64_t tiles = std::min((int64_t)num_seqs * a.row_tiles, carry ? (int64_t)a.row_tiles : (int64_t)num_rows / kRowsPerGroup + num_seqs);
-  const bool ranked = num_seqs <= kRankedSeqs && tiles * heads <= 0xffffff;
-  a.ranked_seqs = ranked ? num_seqs : 0;
-  a.tiles = ranked ? (int)tiles : 1;
-  const int key_groups = tiles * heads <= 512 ? 2 : 1;
-  const dim3 grid = ranked ? dim3((unsigned)(heads * tiles)) : dim3(heads, a.row_tiles, num_seqs);
+  const PromptForm form = prompt_form(num_rows, num_seqs, max_query_len, heads, dim, rot, vdim, carry != nullptr);
+  a.ranked_seqs = form.ranked ? num_seqs : 0;
+  a.tiles = form.ranked ? (int)form.tiles : 1;
+  const int key_groups = form.key_groups;
+  const dim3 grid = form.ranked ? dim3((unsigned)(heads * form.tiles)) : dim3(heads, a.row_tiles, num_seqs);
   auto go = [&](auto s) -> int {
     using S = decltype(s);
     auto with_values = [&](auto vb) -> int {
