@@ -213,7 +213,12 @@ int vla_seq_pair_hash_embed(float* out, const void* table, const void* pair_tabl
  * the root) and multiplied by these weights before it is rotated; with head_norm every head is
  * divided by its own root mean square over dim instead, and null weights mean 1.  v_other (null: none; rows of
  * kv_heads * vdim values, not together with value_inv_freq): the cached value is
- * (1 - v_blend[0]) v + v_blend[0] v_other, v_blend one fp32 number on the device. */
+ * (1 - v_blend[0]) v + v_blend[0] v_other, v_blend one fp32 number on the device.
+ * vla_seq_rotary_kv_write_form: 1 where rows like these (no norms, no blend, values as they are) are written in pieces of
+ * 16 bytes, a wave per token. */
+int vla_seq_rotary_kv_write_form(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                                 int64_t v_stride, const void* key_cache, const void* value_cache, int heads,
+                                 int kv_heads, int dim, int vdim, int rot_dims, int dtype);
 int vla_seq_rotary_kv_write(void* q, int64_t q_stride, const void* k, int64_t k_stride,
                             const void* v, int64_t v_stride, void* key_cache, void* value_cache,
                             const int64_t* positions, const int64_t* slot_mapping,
@@ -618,7 +623,11 @@ int vla_seq_rglru_scan(void* out, int64_t out_stride, int out_dtype, const float
  * (2i, 2i + 1) when interleaved, (i, i + rot_dims / 2) otherwise, turn by positions[t] * inv_freq[i],
  * sine and cosine times `magnitude`) and
  * writes the rows [kv[:rank] / sqrt(mean^2 + eps) * norm_weight | kv[rank:] rotated the same way].
- * slot_mapping < 0 skips the cache. */
+ * slot_mapping < 0 skips the cache.
+ * vla_seq_latent_rotary_write_form: 1 where rows like these are written in pieces of 16 bytes, a wave per token. */
+int vla_seq_latent_rotary_write_form(const void* q, int64_t q_stride, int q_head_stride, int q_first, const void* kv,
+                                     int64_t kv_stride, const float* norm_weight, const void* cache, int num_tokens,
+                                     int heads, int rank, int rot, int rot_dims, int dtype);
 int vla_seq_latent_rotary_write(void* q, int64_t q_stride, int q_head_stride, int q_first,
                                 const void* kv, int64_t kv_stride, const float* norm_weight,
                                 float eps, void* cache, const int64_t* positions,

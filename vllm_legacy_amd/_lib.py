@@ -57,7 +57,7 @@ SEQ_EXPORTS = [
     "vla_seq_window_attention_tiles_supported", "vla_seq_set_scan_kernel",
     "vla_seq_gla_piece_prefix", "vla_seq_gla_combine_states",
     "vla_seq_residual_norms", "vla_seq_causal_conv", "vla_seq_concat_cast", "vla_seq_gated_act",
-    "vla_seq_rotary_kv_write", "vla_seq_kv_attention", "vla_seq_mingru_scratch_floats",
+    "vla_seq_rotary_kv_write", "vla_seq_rotary_kv_write_form", "vla_seq_kv_attention", "vla_seq_mingru_scratch_floats",
     "vla_seq_mingru_scan", "vla_seq_moe_route", "vla_seq_moe_route_form", "vla_seq_set_moe_route_form", "vla_seq_moe_tile_rows", "vla_seq_moe_plan",
     "vla_seq_grouped_linear", "vla_seq_moe_combine", "vla_seq_kv_attention_tiles_supported",
     "vla_seq_kv_attention_tiles", "vla_seq_kv_attention_tiles_of", "vla_seq_kv_attention_tiles_form", "vla_seq_set_kv_attention_kernel", "vla_seq_set_grouped_linear_form",
@@ -65,7 +65,7 @@ SEQ_EXPORTS = [
     "vla_seq_embed_scaled", "vla_seq_softcap", "vla_seq_kv_attention_shared", "vla_seq_kv_attention_scratch_floats", "vla_seq_grouped_linear_of", "vla_seq_grouped_glu", "vla_seq_grouped_glu_supported", "vla_seq_grouped_form", "vla_seq_gla_chunks", "vla_seq_gla_chunks_scratch_floats", "vla_seq_latent_gather", "vla_seq_latent_prompt", "vla_seq_latent_prompt_form", "vla_seq_latent_prompt_supported",
     "vla_seq_delta_rule_scan", "vla_seq_delta_rule_scan_blocks", "vla_seq_delta_rule_block_scratch_floats",
     "vla_seq_delta_rule_scratch_floats", "vla_seq_set_delta_kernel", "vla_seq_rglru_scan",
-    "vla_seq_latent_rotary_write", "vla_seq_latent_attention", "vla_seq_latent_attention_tiles",
+    "vla_seq_latent_rotary_write", "vla_seq_latent_rotary_write_form", "vla_seq_latent_attention", "vla_seq_latent_attention_tiles",
     "vla_seq_latent_attention_tiles_supported", "vla_seq_latent_attention_scratch_floats", "vla_seq_set_latent_attention_kernel",
     "vla_seq_latent_decode", "vla_seq_latent_decode_supported", "vla_seq_latent_decode_ranges", "vla_seq_latent_decode_scratch_floats",
     "vla_seq_latent_decode_up", "vla_seq_latent_decode_up_supported",
@@ -130,6 +130,8 @@ def seq_lib():
         L.vla_seq_kv_attention_tiles_of.argtypes = [p, i64, p, i64, p, i64, p, p, p, i, p, p, p, i, i, i, i64,
                                                     i, i, i, i, i, i, i, f, i, i, f, i, p, p]
         L.vla_seq_kv_attention_tiles_form.argtypes = [i, i, i64, i, i, i, i, i, i, i]
+        L.vla_seq_rotary_kv_write_form.argtypes = [p, i64, p, i64, p, i64, p, p, i, i, i, i, i, i]
+        L.vla_seq_latent_rotary_write_form.argtypes = [p, i64, i, i, p, i64, p, p, i, i, i, i, i, i]
         L.vla_seq_latent_prompt_form.argtypes = [i, i, i, i, i, i, i, i]
         L.vla_seq_set_kv_attention_kernel.argtypes = [i]
         L.vla_seq_set_grouped_linear_form.argtypes = [i]

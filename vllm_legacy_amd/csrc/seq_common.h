@@ -53,7 +53,8 @@ __device__ __forceinline__ uint32_t pack16(float lo, float hi) {
          ((uint32_t)__builtin_bit_cast(uint16_t, S::from_f32(hi)) << 16);
 }
 
-// (which product is fused is said here, so that every kernel rounds alike)
+// (which product is fused is said here, so that the sums in 32 bits are the same in every kernel; a float16 result may still be
+// rounded from them at once in one kernel and by way of 32 bits in another)
 __device__ __forceinline__ void turn_by(float& a, float& b, float2 sc) {
   const float a2 = fmaf(a, sc.y, -(b * sc.x));
   b = fmaf(b, sc.y, a * sc.x);

@@ -1759,6 +1759,14 @@ int by_value_slices(int vdim, F&& f) {
 using namespace vla;
 using namespace vla::seq;
 
+extern "C" int vla_seq_rotary_kv_write_form(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                                            int64_t v_stride, const void* key_cache, const void* value_cache, int heads,
+                                            int kv_heads, int dim, int vdim, int rot_dims, int dtype) {
+  if (dtype != VLA_BF16 && dtype != VLA_F16) return 0;
+  return rows_fit(RotaryRows{(void*)q, q_stride, k, k_stride, v, v_stride, (void*)key_cache, (void*)value_cache, nullptr, nullptr,
+                             nullptr, 0, 0, heads, kv_heads, dim, vdim, rot_dims, 0});
+}
+
 extern "C" int vla_seq_rotary_kv_write(void* q, int64_t q_stride, const void* k, int64_t k_stride,
                                        const void* v, int64_t v_stride, void* key_cache,
                                        void* value_cache, const int64_t* positions,
