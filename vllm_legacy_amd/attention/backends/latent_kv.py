@@ -124,17 +124,18 @@ class LatentKVAttention(nn.Module):
 
     # Multiply-adds of a step on the latent kernel (a fifth of a matrix product's rate) from which the other way's
     # seven launches more are paid back.  Rows x keys before them, 16 heads of 128 + 64, rank 512, latent / formed us
-    # per call: 128 x 2000 (4.6e9) 118 / 160, 192 x 2000 (7.0e9) 183 / 154, four of 384 x 0 (5.1e9) 137 / 140.
+    # per call: 128 x 2000 (4.6e9) 118 / 147, 192 x 2000 (7.0e9) 179 / 133, four of 384 x 0 (5.1e9) 132 / 141, one of 768
+    # x 0 (5.1e9) 161 / 138, 1024 x 0 (9.1e9) 159 / 138.  (The launches take the host 138 us, whatever the sizes.)
     FORMED_MIN_WORK = 6e9
     # Rows of a run at least: forming a key's numbers costs as much for few rows as for many.  Sixteen of 64 rows x
-    # 1000 268 / 349, of 96 389 / 346; four of 64 x 2000 176 / 243, of 96 282 / 238.
+    # 1000 266 / 338, of 96 389 / 328; four of 64 x 2000 174 / 212, of 96 282 / 208; one of 96 x 4000 162 / 175.
     FORMED_MIN_ROWS = 96
 
     def formed_min_rows(self) -> int:
         """Rows from which a run's keys and values are worth forming.  A (query, key) pair of a head costs the
         latent kernel 2 rank + rot multiply-adds at a fifth of a matrix product's rate (less where the rank is small),
         the formed one dim + rot + vdim at about half of it; forming costs rank (dim + vdim) per key at the full rate.
-        (A rank of 64 beside heads of 128 + 64: 2048 rows 190 / 160 us, 4096 585 / 249.)"""
+        (A rank of 64 beside heads of 128 + 64: 1024 rows 98 / 140 us, 2048 167 / 141, 4096 535 / 186.)"""
         C, D, R, V = self.rank, self.head_dim, self.rot_dim, self.value_dim
         gain = 5 * (2 * C + R) - 2 * (D + R + V)
         return max(self.FORMED_MIN_ROWS, -(-C * (D + V) // gain)) if gain > 0 else 1 << 30

@@ -826,7 +826,7 @@ __device__ __forceinline__ int lane_value(int v) {
 // Two prompts of 2999 and 1854 tokens, 16 heads of 128 x 128 (94 blocks in a row), under the tracer: the walk 178 us, 1.9
 // us per block (212 with the loads at once and choices by branches), the prepare kernel 92, the norms 20 and the
 // step kernel's empty launch 5; a call 267 (333), where the token-by-token walk of the same prompts takes 1079.
-// What a block adds to the state is summed in 64 bits: in 32 a call is 32 us less and states are 1.2 times as far
+// What a block adds to the state is summed in 64 bits: in 32 a call is 20 us less and states are 1.2 times as far
 // from 64 bits as token by token where keys share a part three times as large as the rest (1.0).
 template <int DX>
 __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(DeltaBlocks a) {
@@ -1113,7 +1113,8 @@ std::atomic<int> g_delta_kernel{0};
 // Blocks pay from about a block's rows on (us on the GPU, calls back to back, 16 heads of 128, token by token / in
 // blocks: one run of 33 rows 21 / 23, 48 rows 24 / 23, 100 rows 43 / 28; six runs of 64 rows 55 / 44; 32 runs of 33
 // rows 140 / 114, of 64 217 / 129; one of 33 beside 31 single rows 50 / 41).  Their scratch is 69 KB per block and head of 128 x 128;
-// a step that would want more than 4 GiB of it walks token by token.
+// a step that would want more than 4 GiB of it walks token by token.  (The 1 KB of a block and head where G_31 lies is not
+// counted, so that the line lies where it did before: steps of up to 4.06 GiB at 128 x 128, 4.14 at 64 x 16, go in blocks.)
 constexpr int kBlockMinRows = 33;
 
 int64_t delta_out_floats(int num_tokens, int heads, int vdim) {
@@ -1122,7 +1123,6 @@ int64_t delta_out_floats(int num_tokens, int heads, int vdim) {
 
 bool wants_blocks(int mode, int num_tokens, int num_seqs, int max_query_len, int heads, int dim, int vdim) {
   if (mode != 0 || dim > kMaxBlockDim || max_query_len < kBlockMinRows || (vdim + 15) / 16 > 65535) return false;
-  // (G_31's places are not counted)
   return delta_block_slots(num_tokens, num_seqs) * heads *
              (delta_block_floats((dim + 63) / 64 * 64, (vdim + 15) / 16 * 16) - 256) <= ((int64_t)1 << 30);
 }
