@@ -5,7 +5,7 @@
 // queries of the run.  A run of rows therefore gathers its visible cache rows into one place
 // (latent_gather_kernel), the caller multiplies them with the two up-projections, and
 // latent_prompt_kernel below is plain causal attention with keys [formed (dim) | shared rotated part
-// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 148 us (580 TFLOP/s; 810
+// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 137 us under the tracer (630 TFLOP/s; 880
 // with the remainders' product) where latent_attention_tile_kernel takes 1685, plus 9 us to gather and 60 for the
 // three products (the products on the query's side that they replace take 46).
 //
@@ -35,7 +35,7 @@
 // one group, two workgroups to a CU, all 512 of a run of 4096 rows are on the chip at once and the ones with 64 tiles
 // stay alone on their CUs (165 us instead of 150; 2048 rows 70 instead of 59).  Each group rounds its weights to 16 bits against
 // a maximum of its own: a row's bits differ by one rounding between steps of one form and the other (errors against 64 bits
-// do not).  A wave alone takes 4400 cycles for a tile, 1800 of
+// are the same).  A wave alone takes 4400 cycles for a tile, 1800 of
 // products; two on a SIMD 6300 for one each, at 1.6 GHz, where the card holds its power.  Taken back: the second group
 // half a step behind the first (with two tiles of values: 157), raised priority for the first product (162).
 #include <algorithm>
