@@ -281,8 +281,8 @@ int vla_seq_kv_attention_tiles(void* out, int64_t out_stride, const void* q, int
 /* The same for a step of num_rows rows in all (sequences of different lengths launch no more than they need).
  * vla_seq_kv_attention_tiles_form: how it does: 1 or 2 groups of waves share a workgroup's keys (a group rounds its
  * weights against a maximum of its own, so a row's bits may depend on the step that it is in), and 4 more where tiles of
- * rows are found by their rank and not by the grid. */
-int vla_seq_kv_attention_tiles_form(int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads,
+ * rows are found by their rank and not by the grid, 8 where the grid goes through the rows in order. */
+int vla_seq_kv_attention_tiles_form(int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads, int dim,
                                     int max_blocks, int block_size, int window, int keep_first, int chunk);
 int vla_seq_kv_attention_tiles_of(void* out, int64_t out_stride, const void* q, int64_t q_stride,
                                   const void* gate, int64_t gate_stride, const void* key_cache,

@@ -10,7 +10,7 @@ import torch
 from tests.test_gpu_kv_decode import DEV, rnd
 
 pytestmark = pytest.mark.gpu
-ONE, TWO, RANKED = 1, 2, 4
+ONE, TWO, RANKED, IN_ORDER = 1, 2, 4, 8
 
 
 def ragged(count, longest, context, seed=0):
@@ -26,7 +26,8 @@ def ragged(count, longest, context, seed=0):
     (16, 4, ragged(250, 40, 90, 6), 0, ONE + RANKED), (16, 4, [(1300, 0), (129, 40), (700, 0), (2100, 0), (64, 8)], 0, ONE + RANKED),
     (8, 8, ragged(300, 130, 90, 7), 0, ONE), (4, 1, ragged(260, 32, 700, 8), 0, TWO),
     (16, 4, ragged(100, 32, 60, 9), 0, ONE), (16, 4, [(64, 0)] * 40, 0, ONE), (16, 4, [(32, 40), (32, 0), (32, 96)], 0, TWO),
-    (2, 2, [(64, c % 60) for c in range(270)], 0, ONE)])
+    (2, 2, [(64, c % 60) for c in range(270)], 0, ONE), (64, 16, [(64, 0)] * 40, 0, ONE + IN_ORDER),
+    (64, 16, [(32, 40), (32, 0), (32, 96)], 0, TWO + IN_ORDER), (64, 16, [(32, c % 60) for c in range(270)], 0, ONE + IN_ORDER)])
 def test_all_rows(heads, kv_heads, runs, window, form):
     from vllm_legacy_amd import _lib
     from vllm_legacy_amd import _seq_ops as ops
@@ -39,7 +40,7 @@ def test_all_rows(heads, kv_heads, runs, window, form):
         tables[b, :len(own)] = own
     q = rnd((T, heads * D), 4).to(torch.bfloat16)
     starts = torch.tensor([0] + [n for n, _ in runs]).cumsum(0)
-    assert _lib.seq_lib().vla_seq_kv_attention_tiles_form(len(runs), longest, T, heads, kv_heads, max(need), bs, window, 0, 0) == form
+    assert _lib.seq_lib().vla_seq_kv_attention_tiles_form(len(runs), longest, T, heads, kv_heads, D, max(need), bs, window, 0, 0) == form
     out = torch.full((T + 1, heads * D), 7.0, dtype=torch.bfloat16, device=DEV)
     ops.kv_attention_tiles(out[:T], q.to(DEV), None, kc.to(DEV), vc.to(DEV), tables.to(DEV), starts.int().to(DEV),
                            torch.tensor([c for _, c in runs], dtype=torch.int32, device=DEV), longest, None, False, heads, window, D**-0.5)
@@ -58,10 +59,10 @@ def test_all_rows(heads, kv_heads, runs, window, form):
 
 @pytest.mark.parametrize("sizes,runs,window,form", [
     ((2, 128, 64, 128, 64), [(700, 0)], 0, TWO + RANKED), ((2, 128, 64, 128, 64), ragged(9, 300, 2000, 1), 700, TWO + RANKED),
-    ((4, 64, 32, 64, 32), ragged(30, 200, 200, 2), 0, TWO), ((4, 64, 32, 64, 32), ragged(30, 200, 700, 2), 0, TWO + RANKED), ((1, 32, 16, 40, 32), ragged(200, 60, 500, 3), 0, TWO + RANKED),
-    ((1, 32, 16, 40, 32), ragged(270, 60, 400, 4), 0, TWO), ((2, 136, 56, 128, 32), [(1030, 40)] + ragged(20, 200, 30, 5), 0, TWO + RANKED),
+    ((4, 64, 32, 64, 32), ragged(30, 128, 200, 2), 0, TWO), ((4, 64, 32, 64, 32), ragged(30, 200, 700, 2), 0, TWO + RANKED), ((1, 32, 16, 40, 32), ragged(200, 60, 500, 3), 0, TWO + RANKED),
+    ((1, 32, 16, 40, 32), [(1030, 40)] + ragged(260, 30, 20, 4), 0, TWO), ((2, 136, 56, 128, 32), [(1030, 40)] + ragged(20, 200, 30, 5), 0, TWO + RANKED),
     ((2, 128, 64, 128, 64), [(130, 0), (100, 20)], 0, ONE + RANKED), ((8, 128, 64, 72, 64), ragged(80, 250, 500, 6), 300, ONE + RANKED),
-    ((3, 64, 0, 64, 32), ragged(256, 200, 60, 7), 0, ONE), ((3, 64, 0, 64, 32), ragged(240, 200, 500, 8), 0, ONE + RANKED),
+    ((3, 64, 0, 64, 32), ragged(256, 120, 60, 7), 0, ONE), ((3, 64, 0, 64, 32), ragged(240, 200, 500, 8), 0, ONE + RANKED),
     ((8, 64, 16, 128, 32), ragged(300, 150, 90, 9), 70, ONE)])
 def test_latent_prompts(sizes, runs, window, form):
     """Keys in two parts and values as given."""

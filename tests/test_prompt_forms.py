@@ -2,12 +2,12 @@
 where both sides were timed: one or two groups of waves to a workgroup, tiles found by their rank or by the grid."""
 import pytest
 
-ONE, TWO, RANKED = 1, 2, 4
+ONE, TWO, RANKED, IN_ORDER = 1, 2, 4, 8
 
 
 def kv(seqs, longest, rows, heads, kv_heads, keys, window=0, keep=0, chunk=0):
     from vllm_legacy_amd import _lib
-    return _lib.seq_lib().vla_seq_kv_attention_tiles_form(seqs, longest, rows, heads, kv_heads, (keys + 15) // 16, 16, window, keep, chunk)
+    return _lib.seq_lib().vla_seq_kv_attention_tiles_form(seqs, longest, rows, heads, kv_heads, 128, (keys + 15) // 16, 16, window, keep, chunk)
 
 
 @pytest.mark.parametrize("args,want", [
@@ -22,8 +22,8 @@ def kv(seqs, longest, rows, heads, kv_heads, keys, window=0, keep=0, chunk=0):
     ((4, 2047, 5543, 16, 4, 2047), ONE + RANKED),
     # no search where no workgroup is empty and walks are short: 39 us and 42, 42 and 45
     ((256, 33, 256 * 33, 16, 4, 33), ONE), ((256, 64, 11000, 16, 4, 64), ONE), ((256, 64, 11000, 16, 4, 600), ONE + RANKED),
-    # the same whole tiles: 26 us in order, 47 last tiles first
-    ((128, 64, 128 * 64, 16, 4, 64), ONE),
+    # the same whole tiles: 26 us in order, 47 last tiles first; smaller rows: 46 and 42
+    ((128, 64, 128 * 64, 16, 4, 64), ONE + IN_ORDER), ((400, 128, 400 * 128, 8, 1, 128), ONE),
     # more sequences than a wave's registers hold
     ((257, 33, 257 * 33, 16, 4, 1000), ONE), ((300, 20, 3000, 4, 1, 1000), TWO)])
 def test_key_value_prompts(args, want):
@@ -41,6 +41,8 @@ def latent(rows, seqs, longest, heads, dim, rot, vdim, ranged=0):
     ((2128, 1, 128, 16, 128, 64, 128), TWO + RANKED), ((512, 1, 512, 16, 128, 64, 128), TWO + RANKED),
     # narrow heads: 16 and 18
     ((2800, 12, 500, 4, 64, 32, 64), TWO + RANKED),
+    # two to a CU: 20 us with one group, 25 with two
+    ((70 * 331, 70, 100, 4, 64, 32, 64), ONE + RANKED),
     # 10 us with one group, 18 with two; 22 and 31, 31 and 42, 52 and 63, 150 and 202, 88 and 95, 12 and 14
     ((32 * 33, 32, 33, 16, 128, 64, 128), ONE), ((32 * 128, 32, 128, 16, 128, 64, 128), ONE),
     ((8 * 512, 8, 512, 16, 128, 64, 128), ONE + RANKED), ((20 * 728, 20, 128, 16, 128, 64, 128), ONE + RANKED),
@@ -48,7 +50,7 @@ def latent(rows, seqs, longest, heads, dim, rot, vdim, ranged=0):
     ((128, 1, 128, 16, 128, 64, 128), ONE + RANKED),
     # by the grid: 67 us, 72 by rank; 98 and 101; of different lengths by rank
     ((256 * 33, 256, 33, 16, 128, 64, 128), ONE), ((128 * 128, 128, 128, 16, 128, 64, 128), ONE),
-    ((128 * 100, 128, 300, 16, 128, 64, 128), ONE + RANKED), ((257 * 300, 257, 300, 16, 128, 64, 128), ONE),
+    ((128 * 100, 128, 300, 16, 128, 64, 128), ONE + RANKED), ((200 + 60 * 210, 61, 200, 16, 128, 64, 128), ONE + RANKED), ((257 * 300, 257, 300, 16, 128, 64, 128), ONE),
     # a range of one sequence's keys: its rows are not among them
     ((64, 1, 4096, 16, 128, 64, 128, 1), TWO + RANKED), ((64, 1, 128, 16, 128, 64, 128, 1), ONE + RANKED)])
 def test_latent_prompts(args, want):

@@ -129,7 +129,7 @@ def seq_lib():
                                                  i, i, i, i, i, i, i, f, i, i, f, i, p, p]
         L.vla_seq_kv_attention_tiles_of.argtypes = [p, i64, p, i64, p, i64, p, p, p, i, p, p, p, i, i, i, i64,
                                                     i, i, i, i, i, i, i, f, i, i, f, i, p, p]
-        L.vla_seq_kv_attention_tiles_form.argtypes = [i, i, i64, i, i, i, i, i, i, i]
+        L.vla_seq_kv_attention_tiles_form.argtypes = [i, i, i64, i, i, i, i, i, i, i, i]
         L.vla_seq_rotary_kv_write_form.argtypes = [p, i64, p, i64, p, i64, p, p, i, i, i, i, i, i]
         L.vla_seq_latent_rotary_write_form.argtypes = [p, i64, i, i, p, i64, p, p, i, i, i, i, i, i]
         L.vla_seq_latent_prompt_form.argtypes = [i, i, i, i, i, i, i, i]

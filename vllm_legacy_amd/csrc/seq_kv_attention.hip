@@ -1634,10 +1634,10 @@ struct TileGrid {
 // By their rank, so that none is empty and the longest walks go out first: not where no workgroup is empty and the walks are
 // short: the search is a wait for memory more, 256 runs of 33 rows take 42 us with it and 39 without, 128 of 64 48
 // and 39; (one sequence does without in any case).
-// In the order of the rows where all runs are the same whole tiles: tiles of the same number lie at the same distance from
-// each other and meet in the same memory channels (128 runs of 64 rows 26 us, last tiles first 47; 64 of 128 28 and 43; of
-// 60 rows 28 and 27, which is why other runs keep that order).
-TileGrid tile_grid(int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads, int64_t keys) {
+// In the order of the rows where all runs are the same whole tiles of rows of 4 KB or more: tiles of the same number lie at the
+// same distance from each other and meet in the same memory channels (128 runs of 64 rows 26 us, last tiles first 47; 64
+// of 128 28 and 43).  Others keep that order: of 60 rows 28 and 27, 400 runs of 128 rows of 8 heads of 64 46 and 42.
+TileGrid tile_grid(int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads, int dim, int64_t keys) {
   TileGrid to;
   const int group = heads / kv_heads;
   to.num_seqs = num_seqs;
@@ -1649,7 +1649,8 @@ TileGrid tile_grid(int num_seqs, int max_query_len, int64_t num_rows, int heads,
   to.tiles = std::min(all, num_rows / tile_rows + num_seqs);
   const int64_t workgroups = to.head_groups * to.tiles;
   to.key_groups = workgroups <= 256 || (workgroups <= 512 && keys > 512) ? 2 : 1;
-  to.in_order = keys <= 128 && max_query_len % tile_rows == 0 && num_rows == (int64_t)num_seqs * max_query_len;
+  to.in_order = keys <= 128 && (int64_t)heads * dim >= 2048 && max_query_len % tile_rows == 0 &&
+                num_rows == (int64_t)num_seqs * max_query_len;
   to.ranked = num_seqs <= kRankedSeqs && !to.in_order && !(to.tiles == all && keys <= 256);
   return to;
 }
@@ -1963,14 +1964,14 @@ extern "C" int vla_seq_kv_attention_tiles_supported(int dim, int vdim, int turne
          g_kv_kernel.load(std::memory_order_relaxed) == 0;
 }
 
-extern "C" int vla_seq_kv_attention_tiles_form(int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads,
+extern "C" int vla_seq_kv_attention_tiles_form(int num_seqs, int max_query_len, int64_t num_rows, int heads, int kv_heads, int dim,
                                                int max_blocks, int block_size, int window, int keep_first, int chunk) {
   if (num_seqs <= 0 || max_query_len <= 0 || num_rows < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 ||
-      max_blocks <= 0 || block_size <= 0)
+      dim <= 0 || max_blocks <= 0 || block_size <= 0)
     return 0;
-  const TileGrid to = tile_grid(num_seqs, max_query_len, num_rows, heads, kv_heads,
+  const TileGrid to = tile_grid(num_seqs, max_query_len, num_rows, heads, kv_heads, dim,
                                 walked_keys(max_blocks, block_size, window, window > 0 || chunk > 0 ? keep_first : 0, chunk));
-  return to.key_groups + (to.ranked ? 4 : 0);
+  return to.key_groups + (to.ranked ? 4 : 0) + (to.in_order ? 8 : 0);
 }
 
 extern "C" int vla_seq_kv_attention_tiles(
@@ -2012,7 +2013,7 @@ extern "C" int vla_seq_kv_attention_tiles_of(
   if (((uintptr_t)q % 16) || ((q_stride * 2) % 16) || ((uintptr_t)key_cache % 16) ||
       ((uintptr_t)value_cache % 16))
     return VLA_ERR_ARG;
-  const TileGrid to = tile_grid(num_seqs, max_query_len, num_rows, heads, kv_heads,
+  const TileGrid to = tile_grid(num_seqs, max_query_len, num_rows, heads, kv_heads, dim,
                                 walked_keys(max_blocks, block_size, window, keep_first, chunk));
   auto go = [&](auto tag) {
     using S = decltype(tag);

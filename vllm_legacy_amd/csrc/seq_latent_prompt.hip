@@ -543,9 +543,11 @@ int launch_latent_prompt(const LatentPrompt& a, dim3 grid, int key_groups, hipSt
 // run of 512 rows 22 us with two groups, 23 with one; 16 of 128 behind 300 keys 29 and 28; 128 rows behind 2000 60 and 71;
 // four heads of 64 + 32 and 64: 12 runs of 50 to 500 rows 16 and 18, 16 of 128 10 and 9.5), or where long runs have walks
 // of all lengths (one of 4096 rows 152 and 165, two of 2048 78 and 83, three of 1024 behind 1000 95 and 88, 32 of 33 18
-// and 10, eight of 512 42 and 31, 16 of 256 behind 2000 202 and 150).  The bound may be a few workgroups too high.
-// Not by their rank where no workgroup is empty and the walks are short, as key / value prompts: 256 runs of 33 rows 72
-// and 67 us, 128 of 128 101 and 98.
+// and 10, eight of 512 42 and 31, 16 of 256 behind 2000 202 and 150; 280 workgroups of 4 narrow heads, 10 runs of 100 and 60
+// of 20 behind 300, 25 and 20).
+// Not by their rank where a sequence is a tile and the walks are short, as key / value prompts: 256 runs of 33 rows 72
+// and 67 us, 128 of 128 101 and 98 (but one of 200 beside 60 of 10 behind 200 keys 44 and 54: the bound, which counts keys for
+// rows, does not show that workgroups are empty).
 struct PromptForm {
   int64_t tiles;
   int key_groups;
@@ -557,8 +559,8 @@ PromptForm prompt_form(int num_rows, int num_seqs, int max_query_len, int heads,
   form.tiles = std::min(all, ranged ? row_tiles : (int64_t)num_rows / kRowsPerGroup + num_seqs);
   const int64_t workgroups = form.tiles * heads, keys = num_rows / num_seqs;
   const bool wide = dim + rot > 128 || vdim > 64;
-  form.key_groups = (workgroups <= 288 && keys >= (wide ? 512 : 129)) || (workgroups <= 512 && max_query_len > 1024) ? 2 : 1;
-  form.ranked = num_seqs <= kRankedSeqs && workgroups <= 0xffffff && !(form.tiles == all && num_seqs > 1 && keys <= 256);
+  form.key_groups = (workgroups <= 256 && keys >= (wide ? 512 : 129)) || (workgroups <= 512 && max_query_len > 1024) ? 2 : 1;
+  form.ranked = num_seqs <= kRankedSeqs && workgroups <= 0xffffff && !(row_tiles == 1 && num_seqs > 1 && keys <= 256);
   return form;
 }
 
