@@ -183,3 +183,35 @@ def test_steps_that_go_in_chunks(H, lens, chunks, monkeypatch):
         outs.append(out)
     assert len(went) == int(chunks)
     assert float((outs[0] - outs[1]).abs().max()) <= 6e-5 * float(outs[1].abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gates_of_any_size(dtype):
+    """Gates at and beyond where exp(-gate) leaves fp32, in whole 16-byte pieces of a row: a result is its gate's silu times what
+    the same row gives with a gate that silu leaves as it is (40), to one rounding of each."""
+    from vllm_legacy_amd.attention.batch import SequenceBatch
+    from vllm_legacy_amd.attention.recurrent import GatedLinearRecurrence
+    H, D, V, rank, n = 2, 64, 128, 16, 100
+    layer = GatedLinearRecurrence(H, D, V, 5.0, 1e-5)
+    layer.CHUNK_ALONE_ROWS = 0
+    g = torch.Generator().manual_seed(7)
+    wide = torch.randn(n, 2 * H * D + H * V + rank, generator=g).to(dtype).to(DEV)
+    q, k, v, y = wide.split([H * D, H * D, H * V, rank], 1)
+    w2, bias, norm = torch.randn(H * D, rank, generator=g).to(dtype).to(DEV), torch.ones(H * D, device=DEV), torch.ones(V, device=DEV)
+    b = SequenceBatch.build([n], [0], [[0] * 64], [0], 16, DEV)
+    values = torch.tensor([-120.0, -95.0, -88.5, -87.5, -86.5, -20.0, -0.5, 0.0, 0.5, 20.0, 88.5, 300.0, float("inf")])
+
+    def out(gate):
+        got = torch.empty(n, H * V, device=DEV, dtype=dtype)
+        layer(got, q, k, v, gate, y, w2, bias, norm, torch.zeros(1, H, D, V, device=DEV), b)
+        return got.double().cpu()
+
+    gate = values[torch.arange(n * H * V) % len(values)].view(n, H * V).to(dtype)
+    plain = out(torch.full_like(gate, 40.0).to(DEV)) / 40
+    gd = gate.double()
+    want = plain * torch.where(gd.isinf(), gd, gd / (1 + torch.exp(-gd)))
+    got, finite = out(gate.to(DEV)), want.isfinite() & (want.abs() < torch.finfo(dtype).max / 2)
+    small = torch.finfo(dtype).tiny * 2          # below, a result may be rounded to a coarser step or to nothing
+    eps = 2.0**-7 if dtype == torch.bfloat16 else 2.0**-10
+    assert bool(((got - want).abs() <= eps * want.abs() + small)[finite].all())
+    assert bool((got == want)[want.isinf()].all())

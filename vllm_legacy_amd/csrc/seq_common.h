@@ -318,6 +318,40 @@ __device__ __forceinline__ RankedTile ranked_tile(int rank, int num_seqs, const 
 
 __device__ __forceinline__ bool finite(float x) { return fabsf(x) <= 3.402823466e38f; }
 
+// z / (1 + exp(-z)).  exp(-z) = 2^n 2^f with the argument's rounding in f; the quotient is the hardware reciprocal's product
+// and what that leaves over, divided once more.  Error against 64 bits as that of expf and a division: 3.84e-8 (root mean
+// square over -20 .. 20), 1.85e-7 at most.
+template <int N>
+__device__ __forceinline__ void silu(float (&v)[N]) {
+#pragma clang fp contract(off)
+  float top = 0.f;                                         // NaN aside, which both ways hand on
+#pragma unroll
+  for (int k = 0; k < N; ++k) top = fmaxf(top, fabsf(v[k]));
+  if (__any(top >= 87.f)) {
+    // exp(-z) beyond what the reciprocal takes, where the sum is exp(-z) alone: 2^64 of it, and the rest from the quotient's
+    // exponent.  And infinity, whose remainder is not a number.
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const float y = __builtin_amdgcn_fmed3f(-v[k], -100.f, 400.f), t = 1.44269504f * y, n = __builtin_rintf(t);
+      const float x = __builtin_amdgcn_exp2f((t - n) + fmaf(1.92596299e-8f, y, fmaf(1.44269504f, y, -t)));
+      const bool far = v[k] < -87.f;
+      const float d = far ? __builtin_amdgcn_ldexpf(x, 64) : 1.f + __builtin_amdgcn_ldexpf(x, (int)n);
+      const float r = __builtin_amdgcn_rcpf(d), q = v[k] * r, w = fmaf(fmaf(-d, q, v[k]), r, q);
+      v[k] = far ? __builtin_amdgcn_ldexpf(w, 64 - (int)n) : v[k] == INFINITY ? v[k] : w;
+    }
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    // n in the low bits of a sum with 1.5 2^23, from where it is added to the exponent
+    const float t = -1.44269504f * v[k], at = t + 12582912.f, n = at - 12582912.f;
+    const float x = __builtin_amdgcn_exp2f((t - n) + fmaf(-1.92596299e-8f, v[k], fmaf(-1.44269504f, v[k], -t)));
+    const float d = 1.f + __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) + (__builtin_bit_cast(uint32_t, at) << 23));
+    const float r = __builtin_amdgcn_rcpf(d), q = v[k] * r;
+    v[k] = fmaf(fmaf(-d, q, v[k]), r, q);
+  }
+}
+
 __device__ __forceinline__ float softplusf(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 
 }  // namespace seq

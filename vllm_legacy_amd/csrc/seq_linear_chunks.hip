@@ -14,13 +14,14 @@
 // logarithms over just those rows: nothing is divided and no sums are subtracted, so a decay of 0 beside decays of
 // 1 is exact, and decays near 1 keep the precision of their logarithms (multiplied row by row they left the
 // states after 4096 rows several times as far from 64 bits).
-// All products run on 16x16x4 fp32 matrix cores.  Operands that later kernels read lie in scratch lane for
-// lane.  Bound by memory and the launches: 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB
-// of chunk states and decays; 123 us per call (42 + 23 + 66 under the tracer) where the pieces of 256 rows walked
-// token by token and joined by matrix products took 408.  What a workgroup's 19 and 29 us go to: waits for its rows
-// (4 and 5), products (7 and 9), decays (6 and 5), the products inside a block (4), gates and stores (5).  Rows are
-// asked for together and made numbers afterwards, start states a tile of columns ahead (130 us where values and W2
-// were each waited for behind a condition of their own, and keys, values and y in turn).
+// All products run on 16x16x4 fp32 matrix cores.  Operands that later kernels read lie in scratch lane for lane.
+// 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB of chunk states and decays: 97 us per call (31 + 23 + 52
+// under the tracer; pieces of 256 rows walked token by token and joined by matrix products took 408).  Four workgroups share a
+// CU, so that all 1024 of that step are there at once: 16-bit rows stay 16-bit in LDS (39 of 40 KB), a thread holds a channel's
+// logarithms of a block in registers, A lies where its queries lay and the values where the keys were (two workgroups per CU
+// and two rounds of them, with rows as 32-bit numbers beside a copy of the decays: 123 us, 42 + 23 + 66).  What bounds the
+// first and last kernel now are vector instructions (three fifths of their cycles; exponentials and logarithms most of them)
+// and products (three tenths); the scan is a copy of the states, 67 MB in 23 us.
 #include <atomic>
 #include <type_traits>
 
@@ -105,7 +106,7 @@ __device__ __forceinline__ f32x4 row4(const typename S::T* p) {
 // error: 2.62e-8 root mean square over -87 .. 0, 8.4e-8 at most.
 __device__ __forceinline__ float exp_of_log(float p) {
 #pragma clang fp contract(off)
-  p = p < -150.f ? -150.f : p;
+  p = __builtin_elementwise_maximum(p, -150.f);
   const float t = 1.44269504f * p, n = __builtin_rintf(t);
   return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - n) + fmaf(1.92596299e-8f, p, fmaf(1.44269504f, p, -t))), (int)n);
 }
@@ -131,17 +132,48 @@ __device__ __forceinline__ float log_sigmoid(float z) {
   return -(t + (lost_lo + fmaf(a * y, s, more)));
 }
 
+// Values of a chunk in LDS, as they lie in memory: rows of V elements and some, so that rows 4 apart start 16 banks apart.
+template <class S>
+__host__ __device__ __forceinline__ int value_row(int vdim) {
+  return (vdim + 31) / 32 * 32 + (sizeof(typename S::T) == 2 ? 8 : 4);
+}
+
+// Tiles of 16 value columns come in pairs that share a read: lane c has columns 2 c and 2 c + 1 of 32, the first for the one
+// tile and the second for the other.  The last of an odd number of tiles stands alone and has column c.
+struct TilePair {
+  int at;          // where lane c reads its two values of a row
+  bool alone, second;
+  __device__ __forceinline__ TilePair(int pair, int tiles, int c)
+      : at(2 * pair + 1 < tiles ? 32 * pair + 2 * c : 32 * pair + (c & ~1)), alone(2 * pair + 1 >= tiles), second(alone && (c & 1)) {}
+  template <class S>
+  __device__ __forceinline__ void read(const typename S::T* row, float& x, float& y) const {
+    if constexpr (sizeof(typename S::T) == 2) {
+      const uint32_t two = *reinterpret_cast<const uint32_t*>(row + at);
+      x = lo16<S>(two);
+      y = hi16<S>(two);
+    } else {
+      const float2 two = *reinterpret_cast<const float2*>(row + at);
+      x = two.x;
+      y = two.y;
+    }
+    x = second ? y : x;
+  }
+};
+__device__ __forceinline__ int tile_column(int tile, int tiles, int c) {
+  return (tile | 1) < tiles ? 32 * (tile >> 1) + 2 * c + (tile & 1) : 16 * tile + c;
+}
+
 template <class S, int DT>          // DT: dim / 16
-__global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
+__global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2) void gla_chunk_state_kernel(GlaChunks a) {
   using T = typename S::T;
   extern __shared__ __align__(16) float lds[];
-  constexpr int D = 16 * DT, KR = D + 4;
-  const int V = a.vdim, R = a.rank, VR = V + 4;
+  constexpr int D = 16 * DT, KR = D + 4, ITEMS = (4 * D + 255) / 256;
+  const int V = a.vdim, R = a.rank, VR = value_row<S>(V);
+  const int RP = (R + 3) / 4 * 4;
   float* k_lds = lds;                       // [64][KR]
-  float* a_lds = k_lds + kChunk * KR;       // [64][D]
-  float* v_lds = a_lds + kChunk * D;        // [64][VR]
-  float* y_lds = v_lds + kChunk * VR;       // [64][R padded to 4]
-  float* tot = y_lds + kChunk * kMaxRank;   // [4][D]: a block's sum of logarithms
+  float* tot = k_lds + kChunk * KR;         // [4][D]: a block's sum of logarithms
+  float* y_lds = tot + 4 * D;               // [64][RP]
+  T* v_lds = (T*)(y_lds + kChunk * RP);     // [64][VR]
   const int slot = blockIdx.x, h = blockIdx.y;
   int b, chunk;
   if (!find_chunk(a, slot, b, chunk)) return;
@@ -149,18 +181,18 @@ __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
   const int t0 = a.query_start_loc[b] + chunk * kChunk, n = min(kChunk, run - chunk * kChunk);
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c = lane & 15;
-  const int RP = (R + 3) / 4 * 4;
   float* mine = a.scratch + ((int64_t)slot * a.heads + h) * chunk_floats(D, V);
 
   // rows behind the run's end are zeros; every load is on its way before the first is waited for
-  const int row = tid >> 2, quarter = tid & 3;
-  const int64_t t = t0 + min(row, n - 1);
-  const int d_mine = tid % D;                // the thread's decay channel and its row of W2, on its way with the rows
+  const int d = tid % D;                     // a thread has a channel's 16 rows of a block (two blocks with 128 channels)
+  auto block_of = [&](int u) __attribute__((always_inline)) {
+    return D >= 64 ? __builtin_amdgcn_readfirstlane((tid + 256 * u) / D) : min(tid / D, 3);
+  };
   constexpr int PER = 16 / sizeof(T);
   const bool w_wide = R % PER == 0 && (uintptr_t)a.w2 % 16 == 0;
   u32x4 w_row[kMaxRank / PER];
   float wv[kMaxRank];
-  const T* wr = (const T*)a.w2 + ((int64_t)h * D + d_mine) * R;
+  const T* wr = (const T*)a.w2 + ((int64_t)h * D + d) * R;
   if (w_wide) {
 #pragma unroll
     for (int r = 0; r < kMaxRank / PER; ++r) w_row[r] = *reinterpret_cast<const u32x4*>(wr + min(PER * r, R - PER));
@@ -171,42 +203,34 @@ __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
 #pragma unroll
     for (int r = 0; r < kMaxRank; ++r) wv[r] = r < R ? S::to_f32(raw[r]) : 0.f;
   }
-  const float bias = a.bias != nullptr ? a.bias[(int64_t)h * D + d_mine] : 0.f;
+  const float bias = a.bias != nullptr ? a.bias[(int64_t)h * D + d] : 0.f;
+  const int row = tid >> 2, quarter = tid & 3;
+  const int64_t t = t0 + min(row, n - 1);
   T ys[kMaxRank / 4];
 #pragma unroll
   for (int u = 0; u < kMaxRank / 4; ++u) ys[u] = ((const T*)a.y)[t * a.y_stride + min(quarter + 4 * u, R - 1)];
-  // four values a thread, in the order they lie in: D / 16 and V / 16 of them, whole for all threads
+  T ks[ITEMS][kBlock];
+#pragma unroll
+  for (int u = 0; u < ITEMS; ++u)
+#pragma unroll
+    for (int i = 0; i < kBlock; ++i)
+      ks[u][i] = ((const T*)a.k + (t0 + min(kBlock * block_of(u) + i, n - 1)) * a.k_stride + (int64_t)h * D)[d];
+  // four values a thread, in the order they lie in: V / 16 of them, whole for all threads
   constexpr int kMost = 8;
-  Four<S> ks[DT], vs[kMost];
+  Four<S> vs[kMost];
   const int per_row = V / 4, inverse = (65536 + per_row - 1) / per_row;      // (i * inverse) >> 16 is i / per_row below 2048
 #pragma unroll
-  for (int u = 0; u < DT; ++u) {
-    const int i = tid + 256 * u, r = i / (D / 4), d = 4 * (i % (D / 4));
-    ks[u] = fetch4<S>((const T*)a.k + (t0 + min(r, n - 1)) * a.k_stride + (int64_t)h * D + d);
-  }
-#pragma unroll
   for (int u = 0; u < kMost; ++u) {
-    const int i = tid + 256 * min(u, V / 16 - 1), r = (i * inverse) >> 16, d = 4 * (i - r * per_row);
-    vs[u] = fetch4<S>((const T*)a.v + (t0 + min(r, n - 1)) * a.v_stride + (int64_t)h * V + d);
+    const int i = tid + 256 * min(u, V / 16 - 1), r = (i * inverse) >> 16, at = 4 * (i - r * per_row);
+    vs[u] = fetch4<S>((const T*)a.v + (t0 + min(r, n - 1)) * a.v_stride + (int64_t)h * V + at);
   }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int u = 0; u < kMaxRank / 4; ++u)
-    if (4 * u < RP) y_lds[row * kMaxRank + quarter + 4 * u] = quarter + 4 * u < R ? S::to_f32(ys[u]) : 0.f;
-#pragma unroll
-  for (int u = 0; u < DT; ++u) {
-    const int i = tid + 256 * u, r = i / (D / 4), d = 4 * (i % (D / 4));
-    *reinterpret_cast<f32x4*>(k_lds + r * KR + d) = r < n ? numbers<S>(ks[u]) : f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-#pragma unroll
-  for (int u = 0; u < kMost; ++u)
-    if (16 * u < V) {
-      const int i = tid + 256 * u, r = (i * inverse) >> 16, d = 4 * (i - r * per_row);
-      *reinterpret_cast<f32x4*>(v_lds + r * VR + d) = r < n ? numbers<S>(vs[u]) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    if (4 * u < RP) y_lds[row * RP + quarter + 4 * u] = quarter + 4 * u < R ? S::to_f32(ys[u]) : 0.f;
   __syncthreads();
 
-  // decays: a thread keeps its channel's row of W2 and walks every (256 / D)-th row
+  // decays, and keys times the decays behind them in their block
   if (w_wide) {
 #pragma unroll
     for (int r = 0; r < kMaxRank; ++r) {
@@ -218,123 +242,127 @@ __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunks a) {
         wv[r] = __builtin_bit_cast(float, (uint32_t)w_row[r / PER][r % PER]);
     }
   }
-  for (int i = tid / D; i < kChunk; i += 256 / D) {
-    float z = bias;
+#pragma unroll
+  for (int u = 0; u < ITEMS; ++u) {
+    const int r0 = kBlock * block_of(u);
+    const bool act = D >= 64 || tid < 4 * D;
+    float av[kBlock];
+#pragma unroll
+    for (int i = 0; i < kBlock; ++i) av[i] = bias;
 #pragma unroll
     for (int r4 = 0; r4 < kMaxRank; r4 += 4) {
       if (r4 >= RP) break;
-      const f32x4 yv = *reinterpret_cast<const f32x4*>(y_lds + i * kMaxRank + r4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) z += wv[r4 + e] * yv[e];
+      for (int i = 0; i < kBlock; ++i) {
+        const f32x4 yv = *reinterpret_cast<const f32x4*>(y_lds + (r0 + i) * RP + r4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) av[i] += wv[r4 + e] * yv[e];
+      }
     }
-    const float ld = log_sigmoid(z) * a.inv_tau;
-    a_lds[i * D + d_mine] = i < n ? ld : 0.f;
-    mine[i * D + d_mine] = i < n ? ld : 0.f;
-  }
-  __syncthreads();
-
-  // keys times the decays behind them: inside a block of 16 rows first, then the later blocks' products
-  for (int item = tid; item < 4 * D; item += 256) {
-    const int seg = item / D, d = item - seg * D;
-    float av[kBlock];
-#pragma unroll
-    for (int i = 0; i < kBlock; ++i) av[i] = a_lds[(kBlock * seg + i) * D + d];
     float p = 0.f;
 #pragma unroll
     for (int i = kBlock - 1; i >= 0; --i) {
-      k_lds[(kBlock * seg + i) * KR + d] *= exp_of_log(p);
+      av[i] = r0 + i < n ? log_sigmoid(av[i]) * a.inv_tau : 0.f;
+      if (act) {
+        mine[(r0 + i) * D + d] = av[i];
+        k_lds[(r0 + i) * KR + d] = r0 + i < n ? S::to_f32(ks[u][i]) * exp_of_log(p) : 0.f;
+      }
       p += av[i];
     }
-    tot[seg * D + d] = p;
+    if (act) tot[(r0 / kBlock) * D + d] = p;
   }
-  __syncthreads();
-  for (int d = tid; d < D; d += 256) {
-    const float t3 = tot[3 * D + d], t2 = tot[2 * D + d] + t3, t1 = tot[D + d] + t2;
-    mine[kChunk * D + d] = exp_of_log(tot[d] + t1);
-    // from here on: the decay over the blocks behind each
-    tot[d] = exp_of_log(t1);
-    tot[D + d] = exp_of_log(t2);
-    tot[2 * D + d] = exp_of_log(t3);
-    tot[3 * D + d] = 1.f;
-  }
+#pragma unroll
+  for (int u = 0; u < kMost; ++u)
+    if (16 * u < V) {
+      const int i = tid + 256 * u, r = (i * inverse) >> 16, at = 4 * (i - r * per_row);
+      *reinterpret_cast<Four<S>*>(v_lds + r * VR + at) = r < n ? vs[u] : Four<S>{};
+    }
   __syncthreads();
   float* r_out = mine + kChunk * D + D;
-  const int dt_n = D / 16, vt_n = V / 16;
-  const int pairs = (vt_n + 1) / 2;            // two value tiles share the reads of the keys
-  for (int item = w; item < dt_n * pairs; item += 4) {
-    const int dt = item / pairs, vt = 2 * (item - dt * pairs), vt2 = min(vt + 1, vt_n - 1);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = acc;
+  const int vt_n = V / 16, pairs = (vt_n + 1) / 2;
+  constexpr int SHARE = DT >= 4 ? 1 : 4 / DT;              // waves that share the keys' 16 channels
+  for (int dt = w / SHARE; dt < DT; dt += 4 / SHARE) {
+    // the decay over the blocks behind each
+    const int ch = 16 * dt + c;
+    const float t3 = tot[3 * D + ch], t2 = tot[2 * D + ch] + t3, t1 = tot[D + ch] + t2;
+    const float m[4] = {exp_of_log(t1), exp_of_log(t2), exp_of_log(t3), 1.f};
+    if (w % SHARE == 0 && g == 0) mine[kChunk * D + ch] = exp_of_log(tot[ch] + t1);
+    float kj[kBlock];
 #pragma unroll
-    for (int seg = 0; seg < 4; ++seg) {
-      const float m = tot[seg * D + 16 * dt + c];
+    for (int x = 0; x < kBlock; ++x) kj[x] = k_lds[(kBlock * (x >> 2) + 4 * g + (x & 3)) * KR + ch] * m[x >> 2];
+    for (int pair = w % SHARE; pair < pairs; pair += SHARE) {
+      const TilePair tp(pair, vt_n, c);
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = acc;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int j = kBlock * seg + 4 * g + e;
-        const float kj = k_lds[j * KR + 16 * dt + c] * m;
-        acc = mfma4(kj, v_lds[j * VR + 16 * vt + c], acc);
-        acc2 = mfma4(kj, v_lds[j * VR + 16 * vt2 + c], acc2);
+      for (int x = 0; x < kBlock; ++x) {
+        float v0, v1;
+        tp.read<S>(v_lds + (kBlock * (x >> 2) + 4 * g + (x & 3)) * VR, v0, v1);
+        acc = mfma4(kj[x], v0, acc);
+        acc2 = mfma4(kj[x], v1, acc2);
       }
+      float* to = r_out + ((int64_t)(dt * vt_n + 2 * pair) * 64 + lane) * 4;
+      *reinterpret_cast<f32x4*>(to) = acc;
+      if (!tp.alone) *reinterpret_cast<f32x4*>(to + 256) = acc2;
     }
-    *reinterpret_cast<f32x4*>(r_out + ((int64_t)(dt * vt_n + vt) * 64 + lane) * 4) = acc;
-    if (vt2 != vt) *reinterpret_cast<f32x4*>(r_out + ((int64_t)(dt * vt_n + vt2) * 64 + lane) * 4) = acc2;
   }
 }
 
-// one thread: four neighbouring channels of a value column, over the run's chunks
+// one thread: two neighbouring channels of a value column, over the run's chunks
 __global__ __launch_bounds__(256) void gla_chunk_scan_kernel(GlaChunks a) {
   const int D = a.dim, V = a.vdim, vt_n = V / 16;
   const int h = blockIdx.x, b = blockIdx.z;
-  const int item = blockIdx.y * 256 + threadIdx.x;         // tile, lane
-  if (item >= D * V / 4) return;
+  const int item = blockIdx.y * 256 + threadIdx.x;         // tile, lane, which two of its four channels
+  if (item >= D * V / 2) return;
   const int begin = a.query_start_loc[b], run = a.query_start_loc[b + 1] - begin;
   if (run <= 0) return;
-  const int tile = item >> 6, lane = item & 63, g = lane >> 4, c = lane & 15;
-  const int d = 16 * (tile / vt_n) + 4 * g, v = 16 * (tile % vt_n) + c;
+  const int tile = item >> 7, lane = (item >> 1) & 63, g = lane >> 4, c = lane & 15;
+  const int d = 16 * (tile / vt_n) + 4 * g + 2 * (item & 1), v = tile_column(tile % vt_n, vt_n, c);
   float* st = a.state + (((int64_t)a.state_slots[b] * a.heads + h) * D + d) * V + v;
-  f32x4 s = {0.f, 0.f, 0.f, 0.f};
-  if (a.context_lens[b] > 0)
-    s = f32x4{st[0], st[V], st[2 * V], st[3 * V]};
+  f32x2 s = {0.f, 0.f};
+  if (a.context_lens[b] > 0) s = f32x2{st[0], st[V]};
   const int chunks = (run + kChunk - 1) / kChunk;
   const int64_t per = chunk_floats(D, V), step = a.heads * per;
   float* p = a.scratch + ((int64_t)(begin / kChunk + b) * a.heads + h) * per + kChunk * D;
-  constexpr int AHEAD = 8;
-  f32x4 rv[AHEAD], gv[AHEAD];
+  constexpr int AHEAD = 16;
+  f32x2 rv[AHEAD], gv[AHEAD];
 #pragma unroll
   for (int u = 0; u < AHEAD; ++u) {
     const float* at = p + min(u, chunks - 1) * step;
-    gv[u] = *reinterpret_cast<const f32x4*>(at + d);
-    rv[u] = *reinterpret_cast<const f32x4*>(at + D + 4 * item);
+    gv[u] = *reinterpret_cast<const f32x2*>(at + d);
+    rv[u] = *reinterpret_cast<const f32x2*>(at + D + 2 * item);
   }
   for (int i = 0; i < chunks; i += AHEAD) {
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) {
       if (i + u < chunks) {
-        *reinterpret_cast<f32x4*>(p + (i + u) * step + D + 4 * item) = s;    // the chunk's start state
+        *reinterpret_cast<f32x2*>(p + (i + u) * step + D + 2 * item) = s;    // the chunk's start state
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] = gv[u][e] * s[e] + rv[u][e];
+        for (int e = 0; e < 2; ++e) s[e] = gv[u][e] * s[e] + rv[u][e];
         const float* at = p + min(i + u + AHEAD, chunks - 1) * step;
         // (behind the end this is a place already overwritten, and what it gives is not used)
-        gv[u] = *reinterpret_cast<const f32x4*>(at + d);
-        rv[u] = *reinterpret_cast<const f32x4*>(at + D + 4 * item);
+        gv[u] = *reinterpret_cast<const f32x2*>(at + d);
+        rv[u] = *reinterpret_cast<const f32x2*>(at + D + 2 * item);
       }
     }
   }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) st[e * V] = s[e];
+  st[0] = s[0];
+  st[V] = s[1];
+}
+
+// r *= d in the wave's first n lanes, of which all run: four instructions fewer than a choice of the factor
+__device__ __forceinline__ void times_in_lanes_below(int n, f32x4& r, f32x4 d) {
+  asm("s_bfm_b64 exec, %8, 0\n\tv_mul_f32 %0, %0, %4\n\tv_mul_f32 %1, %1, %5\n\tv_mul_f32 %2, %2, %6\n\t"
+      "v_mul_f32 %3, %3, %7\n\ts_mov_b64 exec, -1"
+      : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3])
+      : "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "s"(n));
 }
 
 template <class S, int DT>          // DT: dim / 16
-__global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
+__global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2) void gla_chunk_out_kernel(GlaChunks a) {
   using T = typename S::T;
   extern __shared__ __align__(16) float lds[];
-  constexpr int D = 16 * DT, KR = D + 4;
-  const int V = a.vdim, VR = V + 4, vt_n = V / 16;
-  float* q_lds = lds;                                      // [64][KR]
-  float* a_mat = q_lds + kChunk * KR;                      // [64][kAMat]
-  float* tot = a_mat + kChunk * kAMat;                     // [4][D]
-  float* k_lds = tot + 4 * D;                              // [64][KR], later v [64][VR] from here on
-  float* a_lds = k_lds + kChunk * KR;                      // [64][D]
-  float* v_lds = k_lds;
+  constexpr int D = 16 * DT, KR = D + 4, QR = KR > kAMat ? KR : kAMat, ITEMS = (D + 63) / 64;
+  const int V = a.vdim, VR = value_row<S>(V), vt_n = V / 16;
   const int slot = blockIdx.x, h = blockIdx.y;
   int b, chunk;
   if (!find_chunk(a, slot, b, chunk)) return;
@@ -342,84 +370,112 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
   const int t0 = a.query_start_loc[b] + chunk * kChunk, n = min(kChunk, run - chunk * kChunk);
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c = lane & 15;
+  // A wave has a block's 16 rows of queries and then, in their place, of A; keys and values are everyone's.
+  float* q_own = lds + kBlock * w * QR;                    // [16][QR]
+  float* a_own = q_own;                                    // [16][kAMat]
+  float* tot = lds + kChunk * QR;                          // [4][D]
+  float* decay_own = tot + 4 * D + kBlock * kBlock * w;    // [16][16]
+  float* k_lds = tot + 4 * D + kChunk * kBlock;            // [64][KR], then the values
+  T* v_lds = (T*)k_lds;                                    // [64][VR]
   const float* mine = a.scratch + ((int64_t)slot * a.heads + h) * chunk_floats(D, V);
   const float* s_in = mine + kChunk * D + D;
 
-  const int row = tid >> 2, quarter = tid & 3;
+  const int row = tid >> 2, quarter = tid & 3;             // the wave's rows again
   const int64_t t = t0 + min(row, n - 1);
   const bool live = row < n;
   const T* qr = (const T*)a.q + t * a.q_stride + (int64_t)h * D;
   const T* kr = (const T*)a.k + t * a.k_stride + (int64_t)h * D;
   const T* vr = (const T*)a.v + t * a.v_stride + (int64_t)h * V;
-  {
-    f32x4 qv[DT], kv[DT], av[DT];
+  Four<S> q_raw[DT], k_raw[DT], held[8];
+  f32x4 av[DT];
+  float down[ITEMS][kBlock];                               // a channel's logarithms in the wave's rows
 #pragma unroll
-    for (int x = 0; x < DT; ++x) {
-      const int d = 4 * quarter + 16 * x;
-      qv[x] = row4<S>(qr + d);
-      kv[x] = row4<S>(kr + d);
-      av[x] = *reinterpret_cast<const f32x4*>(mine + row * D + d);
-    }
-#pragma unroll
-    for (int x = 0; x < DT; ++x) {
-      const int d = 4 * quarter + 16 * x;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        qv[x][e] = live ? qv[x][e] * a.q_scale : 0.f;
-        if (!live) kv[x][e] = 0.f;
-      }
-      *reinterpret_cast<f32x4*>(q_lds + row * KR + d) = qv[x];
-      *reinterpret_cast<f32x4*>(k_lds + row * KR + d) = kv[x];
-      *reinterpret_cast<f32x4*>(a_lds + row * D + d) = f32x4{exp_of_log(av[x][0]), exp_of_log(av[x][1]), exp_of_log(av[x][2]), exp_of_log(av[x][3])};
-    }
+  for (int x = 0; x < DT; ++x) {
+    q_raw[x] = fetch4<S>(qr + 4 * quarter + 16 * x);
+    k_raw[x] = fetch4<S>(kr + 4 * quarter + 16 * x);
+    av[x] = *reinterpret_cast<const f32x4*>(mine + row * D + 4 * quarter + 16 * x);
   }
-  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < ITEMS; ++u)
+#pragma unroll
+    for (int i = 0; i < kBlock; ++i) down[u][i] = mine[(kBlock * w + i) * D + (lane + 64 * u) % D];
+#pragma unroll
+  for (int x = 0; x < 8; ++x) held[x] = fetch4<S>(vr + 4 * quarter + 16 * min(x, vt_n - 1));
+  const float norm_mine = a.norm_weight[min(tid, V - 1)];
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 kv[DT];
+#pragma unroll
+  for (int x = 0; x < DT; ++x) {
+    const int at = 4 * quarter + 16 * x;
+    f32x4 qv = numbers<S>(q_raw[x]);
+    kv[x] = numbers<S>(k_raw[x]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      qv[e] = live ? qv[e] * a.q_scale : 0.f;
+      if (!live) kv[x][e] = 0.f;
+    }
+    *reinterpret_cast<f32x4*>(q_own + (lane >> 2) * QR + at) = qv;
+    *reinterpret_cast<f32x4*>(k_lds + row * KR + at) = kv[x];
+  }
 
-  // A inside the wave's block of 16 rows: lane (j, part) decays a quarter of k_j's channels row by row
-  {
-    const int j = lane >> 2, part = lane & 3, r0 = kBlock * w;
-    f32x4 r[DT];
+  // A inside the block: lane (j, part) decays a quarter of k_j's channels row by row, 16 channels at a time
+  const int j = lane >> 2, part = lane & 3;
+  float dot[kBlock];
 #pragma unroll
-    for (int x = 0; x < DT; ++x) r[x] = *reinterpret_cast<const f32x4*>(k_lds + (r0 + j) * KR + 4 * part + 16 * x);
-#pragma unroll 4
+  for (int i = 0; i < kBlock; ++i) dot[i] = 0.f;
+#pragma unroll
+  for (int x = 0; x < DT; ++x) {
+    wave_sync();
+    *reinterpret_cast<f32x4*>(decay_own + j * kBlock + 4 * part) =
+        f32x4{exp_of_log(av[x][0]), exp_of_log(av[x][1]), exp_of_log(av[x][2]), exp_of_log(av[x][3])};
+    wave_sync();
+    f32x4 r = kv[x];
+#pragma unroll
     for (int i = 0; i < kBlock; ++i) {
-      float dot = 0.f, none = 0.f;
+      const f32x4 dv = *reinterpret_cast<const f32x4*>(decay_own + i * kBlock + 4 * part);
+      const f32x4 qv = *reinterpret_cast<const f32x4*>(q_own + i * QR + 4 * part + 16 * x);
+      if (i > 0) times_in_lanes_below(4 * i, r, dv);       // j < i
 #pragma unroll
-      for (int x = 0; x < DT; ++x) {
-        const f32x4 av = *reinterpret_cast<const f32x4*>(a_lds + (r0 + i) * D + 4 * part + 16 * x);
-        const f32x4 qv = *reinterpret_cast<const f32x4*>(q_lds + (r0 + i) * KR + 4 * part + 16 * x);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          r[x][e] *= i > j ? av[e] : 1.f;
-          dot += qv[e] * r[x][e];
-        }
-      }
-      group_sums(dot, none, 4);
-      if (part == 0) a_mat[(r0 + i) * kAMat + r0 + j] = i >= j ? dot : 0.f;
+      for (int e = 0; e < 4; ++e) dot[i] += qv[e] * r[e];
     }
   }
-  __syncthreads();
+  float inside[4];                                         // of rows part, part + 4, ..
+#pragma unroll
+  for (int i = 0; i < kBlock; i += 2) group_sums(dot[i], dot[i + 1], 4);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const float x = part & 2 ? (part & 1 ? dot[4 * u + 3] : dot[4 * u + 2]) : (part & 1 ? dot[4 * u + 1] : dot[4 * u]);
+    inside[u] = 4 * u + part >= j ? x : 0.f;
+  }
 
   // queries times the decays from their block's start, keys times those to their block's end
-  for (int item = tid; item < 4 * D; item += 256) {
-    const int seg = item / D, d = item - seg * D;
-    float av[kBlock];
+  wave_sync();
 #pragma unroll
-    for (int i = 0; i < kBlock; ++i) av[i] = mine[(kBlock * seg + i) * D + d];
-    float p = 0.f;
+  for (int u = 0; u < ITEMS; ++u) {
+    const int ch = lane + 64 * u;
+    if (ch < D) {
+      float p = 0.f;
 #pragma unroll
-    for (int i = 0; i < kBlock; ++i) {
-      p += av[i];
-      q_lds[(kBlock * seg + i) * KR + d] *= exp_of_log(p);
-    }
-    tot[seg * D + d] = p;
-    p = 0.f;
+      for (int i = 0; i < kBlock; ++i) {
+        p += down[u][i];
+        q_own[i * QR + ch] *= exp_of_log(p);
+      }
+      tot[w * D + ch] = p;
+      p = 0.f;
 #pragma unroll
-    for (int i = kBlock - 1; i >= 0; --i) {
-      k_lds[(kBlock * seg + i) * KR + d] *= exp_of_log(p);
-      p += av[i];
+      for (int i = kBlock - 1; i >= 0; --i) {
+        k_lds[(kBlock * w + i) * KR + ch] *= exp_of_log(p);
+        p += down[u][i];
+      }
     }
   }
+  wave_sync();
+  f32x4 qs[DT];
+#pragma unroll
+  for (int x = 0; x < DT; ++x) qs[x] = *reinterpret_cast<const f32x4*>(q_own + c * QR + 16 * x + 4 * g);
+  wave_sync();
+#pragma unroll
+  for (int u = 0; u < 4; ++u) a_own[(4 * u + part) * kAMat + kBlock * w + j] = inside[u];
   __syncthreads();
 
   // the wave's rows against the blocks before them, and the product over those blocks for the start state
@@ -430,23 +486,23 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int x = 0; x < DT; ++x) {
-      const f32x4 qv = *reinterpret_cast<const f32x4*>(q_lds + (kBlock * w + c) * KR + 16 * x + 4 * g);
       const f32x4 kv = *reinterpret_cast<const f32x4*>(k_lds + (kBlock * o + c) * KR + 16 * x + 4 * g);
       const f32x4 tv = *reinterpret_cast<const f32x4*>(tot + o * D + 16 * x + 4 * g);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        acc = mfma4(qv[e] * exp_of_log(before[x][e]), kv[e], acc);
+        acc = mfma4(o == w - 1 ? qs[x][e] : qs[x][e] * exp_of_log(before[x][e]), kv[e], acc);
         before[x][e] += tv[e];
       }
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) a_mat[(kBlock * w + 4 * g + e) * kAMat + kBlock * o + c] = acc[e];
+    for (int e = 0; e < 4; ++e) a_own[(4 * g + e) * kAMat + kBlock * o + c] = acc[e];
   }
-  // the values take the keys' and the decays' place
-  Four<S> held[8];
+  if (w > 0) {
 #pragma unroll
-  for (int x = 0; x < 8; ++x)
-    if (16 * x < V) held[x] = fetch4<S>(vr + 4 * quarter + 16 * x);
+    for (int x = 0; x < DT; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qs[x][e] *= exp_of_log(before[x][e]);
+  }
   // the start state of a tile of columns is asked for a tile ahead
   f32x4 sv[2][DT];
   auto fetch_state = [&](int vt) __attribute__((always_inline)) {
@@ -454,15 +510,19 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
     for (int x = 0; x < DT; ++x) sv[vt & 1][x] = *reinterpret_cast<const f32x4*>(s_in + ((int64_t)(x * vt_n + vt) * 64 + lane) * 4);
   };
   fetch_state(0);
+  // the values take the keys' place, the norm's weights that of the decays inside the blocks
+  float* norm = tot + 4 * D;
+  if (tid < V) norm[tid] = norm_mine;
   __syncthreads();
   bool odd = false;
 #pragma unroll
   for (int x = 0; x < 8; ++x)
     if (16 * x < V) {
-      const f32x4 put = live ? numbers<S>(held[x]) : f32x4{0.f, 0.f, 0.f, 0.f};
-      *reinterpret_cast<f32x4*>(v_lds + row * VR + 4 * quarter + 16 * x) = put;
+      const Four<S> put = live ? held[x] : Four<S>{};
+      *reinterpret_cast<Four<S>*>(v_lds + row * VR + 4 * quarter + 16 * x) = put;
+      const f32x4 num = numbers<S>(put);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) odd |= !finite(put[e]);
+      for (int e = 0; e < 4; ++e) odd |= !finite(num[e]);
     }
   const bool some_bad = __syncthreads_or(odd);
 
@@ -473,11 +533,7 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
                     (uintptr_t)a.gate % 16 == 0 && (uintptr_t)a.out % 16 == 0;
   constexpr int PIECES = 4;                                // 16 rows of 16 pieces over 64 lanes
   u32x4 gates[PIECES];
-  float norm[8];
   const int row_of = lane >> 3, col_of = 8 * (lane & 7);   // of half the columns: rows row_of and row_of + 8
-#pragma unroll
-  for (int vt = 0; vt < 8; ++vt)
-    if (vt < vt_n) norm[vt] = a.norm_weight[16 * vt + c];
   if (wide) {
 #pragma unroll
     for (int u = 0; u < PIECES; ++u) {
@@ -487,56 +543,83 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
   }
 
   f32x4 acc[8];
-  f32x4 qs[DT];
-#pragma unroll
-  for (int x = 0; x < DT; ++x) {
-    qs[x] = *reinterpret_cast<const f32x4*>(q_lds + (kBlock * w + c) * KR + 16 * x + 4 * g);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) qs[x][e] *= exp_of_log(before[x][e]);
-  }
   float ss[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int vt = 0; vt < 8; ++vt) {
-    acc[vt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (vt < vt_n) {
-      if (vt + 1 < vt_n) fetch_state(vt + 1);
+  for (int pair = 0; pair < 4; ++pair) {
+    acc[2 * pair] = acc[2 * pair + 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (2 * pair < vt_n) {
+      const TilePair tp(pair, vt_n, c);
+      auto two = [&](int at, float& x, float& y) __attribute__((always_inline)) { tp.read<S>(v_lds + at * VR, x, y); };
       for (int o = 0; o < w; ++o) {
-        const f32x4 am = *reinterpret_cast<const f32x4*>(a_mat + (kBlock * w + c) * kAMat + kBlock * o + 4 * g);
+        const f32x4 am = *reinterpret_cast<const f32x4*>(a_own + c * kAMat + kBlock * o + 4 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[vt] = mfma4(am[e], v_lds[(kBlock * o + 4 * g + e) * VR + 16 * vt + c], acc[vt]);
+        for (int e = 0; e < 4; ++e) {
+          float v0, v1;
+          two(kBlock * o + 4 * g + e, v0, v1);
+          acc[2 * pair] = mfma4(am[e], v0, acc[2 * pair]);
+          acc[2 * pair + 1] = mfma4(am[e], v1, acc[2 * pair + 1]);
+        }
       }
       // A row's product with the rows behind it is 0 times their values, which must be finite for that; and a column
       // in which one was not stays so, as it does in the state of a walk.
-      int bad = kBlock;                                    // the block's first such row in column c
+      int bad[2] = {kBlock, kBlock};                       // the block's first such row in the lane's columns
       if (some_bad) {
-        for (int j = kBlock * (w + 1) - 1; j >= 0; --j)
-          if (!finite(v_lds[j * VR + 16 * vt + c])) bad = max(j - kBlock * w, 0);
+        for (int i = kBlock * (w + 1) - 1; i >= 0; --i) {
+          float v0, v1;
+          two(i, v0, v1);
+          if (!finite(v0)) bad[0] = max(i - kBlock * w, 0);
+          if (!finite(v1)) bad[1] = max(i - kBlock * w, 0);
+        }
       }
-      const f32x4 am = *reinterpret_cast<const f32x4*>(a_mat + (kBlock * w + c) * kAMat + kBlock * w + 4 * g);
-      f32x4 vv;
+      const f32x4 am = *reinterpret_cast<const f32x4*>(a_own + c * kAMat + kBlock * w + 4 * g);
+      f32x4 v0, v1;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) vv[e] = v_lds[(kBlock * w + 4 * g + e) * VR + 16 * vt + c];
+      for (int e = 0; e < 4; ++e) {
+        float x, y;
+        two(kBlock * w + 4 * g + e, x, y);
+        v0[e] = x;
+        v1[e] = y;
+      }
+      if (some_bad) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[vt] = mfma4(am[e], 4 * g + e < bad ? vv[e] : 0.f, acc[vt]);
+        for (int e = 0; e < 4; ++e) {
+          v0[e] = 4 * g + e < bad[0] ? v0[e] : 0.f;
+          v1[e] = 4 * g + e < bad[1] ? v1[e] : 0.f;
+        }
+      }
 #pragma unroll
-      for (int x = 0; x < DT; ++x)
+      for (int e = 0; e < 4; ++e) {
+        acc[2 * pair] = mfma4(am[e], v0[e], acc[2 * pair]);
+        acc[2 * pair + 1] = mfma4(am[e], v1[e], acc[2 * pair + 1]);
+      }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[vt] = mfma4(qs[x][e], sv[vt & 1][x][e], acc[vt]);
+      for (int half = 0; half < 2; ++half) {
+        const int vt = 2 * pair + half;
+        if (vt < vt_n) {
+          if (vt + 1 < vt_n) fetch_state(vt + 1);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[vt][e] = 4 * g + e < bad ? acc[vt][e] : NAN;
+          for (int x = 0; x < DT; ++x)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) ss[e] += acc[vt][e] * acc[vt][e];
+            for (int e = 0; e < 4; ++e) acc[vt] = mfma4(qs[x][e], sv[half][x][e], acc[vt]);
+          if (some_bad) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[vt][e] = 4 * g + e < bad[half] ? acc[vt][e] : NAN;
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ss[e] += acc[vt][e] * acc[vt][e];
+        }
+      }
     }
   }
   group_sums(ss[0], ss[1], 16);
   group_sums(ss[2], ss[3], 16);
-  // lane: column 16 vt + c of rows 16 w + 4 g .. + 3
+  // lane: its columns of rows 16 w + 4 g .. + 3
   float inv[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) inv[e] = a.out_scale / sqrtf(ss[e] / (float)V + a.eps);
   if constexpr (sizeof(T) == 2) {
     if (wide) {
-      float* own = a_mat + kBlock * w * kAMat;             // the wave's rows of A, which it alone reads and has read
+      float* own = a_own;                                  // the wave's rows of A, which it alone reads and has read
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         if (64 * half >= V) break;
@@ -545,7 +628,7 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
         for (int vt = 4 * half; vt < 4 * half + 4; ++vt)
           if (vt < vt_n)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) own[(4 * g + e) * kAMat + 16 * (vt - 4 * half) + c] = acc[vt][e] * inv[e] * norm[vt];
+            for (int e = 0; e < 4; ++e) own[(4 * g + e) * kAMat + tile_column(vt, vt_n, c) - 64 * half] = acc[vt][e] * inv[e] * norm[tile_column(vt, vt_n, c)];
         wave_sync();
 #pragma unroll
         for (int r8 = 0; r8 < 2; ++r8) {
@@ -553,12 +636,18 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
           if (i >= n || col >= V) continue;
           const f32x4 x0 = *reinterpret_cast<const f32x4*>(own + r * kAMat + col_of), x1 = *reinterpret_cast<const f32x4*>(own + r * kAMat + col_of + 4);
           const u32x4 gw = gates[2 * half + r8];
+          float gv[8];
           u32x4 res;
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const float g0 = lo16<S>(gw[k]), g1 = hi16<S>(gw[k]);
+            gv[2 * k] = lo16<S>(gw[k]);
+            gv[2 * k + 1] = hi16<S>(gw[k]);
+          }
+          silu(gv);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
             const float y0 = 2 * k < 4 ? x0[2 * k & 3] : x1[2 * k & 3], y1 = 2 * k < 4 ? x0[(2 * k + 1) & 3] : x1[(2 * k + 1) & 3];
-            res[k] = pack16<S>(y0 * (g0 / (1.f + expf(-g0))), y1 * (g1 / (1.f + expf(-g1))));
+            res[k] = pack16<S>(y0 * gv[2 * k], y1 * gv[2 * k + 1]);
           }
           *reinterpret_cast<u32x4*>((T*)a.out + (int64_t)(t0 + i) * a.out_stride + (int64_t)h * V + col) = res;
         }
@@ -570,15 +659,15 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(GlaChunks a) {
   for (int e = 0; e < 4; ++e) {
     const int i = kBlock * w + 4 * g + e;
     if (i >= n) continue;
-    const T* gr = (const T*)a.gate + (int64_t)(t0 + i) * a.gate_stride + (int64_t)h * V + c;
-    T* to = (T*)a.out + (int64_t)(t0 + i) * a.out_stride + (int64_t)h * V + c;
+    const T* gr = (const T*)a.gate + (int64_t)(t0 + i) * a.gate_stride + (int64_t)h * V;
+    T* to = (T*)a.out + (int64_t)(t0 + i) * a.out_stride + (int64_t)h * V;
     float gt[8];
 #pragma unroll
     for (int vt = 0; vt < 8; ++vt)
-      if (vt < vt_n) gt[vt] = S::to_f32(gr[16 * vt]);
+      if (vt < vt_n) gt[vt] = S::to_f32(gr[tile_column(vt, vt_n, c)]);
 #pragma unroll
     for (int vt = 0; vt < 8; ++vt)
-      if (vt < vt_n) to[16 * vt] = S::from_f32(acc[vt][e] * inv[e] * norm[vt] * (gt[vt] / (1.f + expf(-gt[vt]))));
+      if (vt < vt_n) to[tile_column(vt, vt_n, c)] = S::from_f32(acc[vt][e] * inv[e] * norm[tile_column(vt, vt_n, c)] * (gt[vt] / (1.f + expf(-gt[vt]))));
   }
 }
 
@@ -601,14 +690,15 @@ template <class S, int DT>
 int launch_chunks(const GlaChunks& a, dim3 grid, hipStream_t stream) {
   constexpr int D = 16 * DT;
   static std::atomic<size_t> allowed{64 * 1024}, allowed_out{64 * 1024};   // raised once per kernel, not per launch
-  const size_t lds = sizeof(float) * ((size_t)kChunk * (D + 4 + D + a.vdim + 4 + kMaxRank) + 4 * D);
+  const size_t values = sizeof(typename S::T) * (size_t)kChunk * value_row<S>(a.vdim);
+  const size_t lds = sizeof(float) * ((size_t)kChunk * (D + 4 + (a.rank + 3) / 4 * 4) + 4 * D) + values;
   if (const int rc = raise_lds(&gla_chunk_state_kernel<S, DT>, lds, allowed)) return rc;
   gla_chunk_state_kernel<S, DT><<<grid, 256, lds, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
-  gla_chunk_scan_kernel<<<dim3(a.heads, (D * a.vdim / 4 + 255) / 256, a.num_seqs), 256, 0, stream>>>(a);
+  gla_chunk_scan_kernel<<<dim3(a.heads, (D * a.vdim / 2 + 255) / 256, a.num_seqs), 256, 0, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
-  const size_t keys = (size_t)kChunk * (D + 4 + D), values = (size_t)kChunk * (a.vdim + 4);
-  const size_t lds_out = sizeof(float) * ((size_t)kChunk * (D + 4) + kChunk * kAMat + 4 * D + (keys > values ? keys : values));
+  const size_t keys = sizeof(float) * (size_t)kChunk * (D + 4);
+  const size_t lds_out = sizeof(float) * ((size_t)kChunk * (D + 4 > kAMat ? D + 4 : kAMat) + 4 * D + kChunk * kBlock) + (keys > values ? keys : values);
   if (const int rc = raise_lds(&gla_chunk_out_kernel<S, DT>, lds_out, allowed_out)) return rc;
   gla_chunk_out_kernel<S, DT><<<grid, 256, lds_out, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
