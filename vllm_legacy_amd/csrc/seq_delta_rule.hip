@@ -416,11 +416,14 @@ __device__ __forceinline__ bool find_delta_block(const DeltaBlocks& a, int slot,
   return block >= 0 && block * kRows < a.query_start_loc[b + 1] - a.query_start_loc[b];
 }
 
-// LDS of the prepare kernel: keys and queries, then the waves' partial products, whose place the
-// 32 x 32 matrices take, then L (column 32: G), decays, betas, what makes keys and queries unit rows, and
+// LDS of the prepare kernel: keys, then queries, whose place the waves' partial products take and then the
+// 32 x 32 matrices, then L (column 32: G), decays, betas, what makes keys and queries unit rows, and
 // which rows are not finite
+__host__ __device__ constexpr int delta_prepare_shared_floats(int dp) {
+  return kRows * (dp + 4) > 4 * 6 * 256 ? kRows * (dp + 4) : 4 * 6 * 256;
+}
 __host__ __device__ constexpr size_t delta_prepare_lds_floats(int dp) {
-  return (size_t)2 * kRows * (dp + 4) + 4 * 6 * 256 + kRows * kMat + 6 * kRows;
+  return (size_t)kRows * (dp + 4) + delta_prepare_shared_floats(dp) + kRows * kMat + 6 * kRows;
 }
 
 // one 16x16x4 matrix-core step in 64 bits: operands as mfma4's, lane (g, c) ends with column c, rows g + 4 i
@@ -429,17 +432,20 @@ __device__ __forceinline__ f64x4 mfma4_f64(double a, double b, f64x4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// Bound by 64-bit matrix-core instructions (four tenths of its cycles), as many vector ones and the waits between them: a
+// workgroup by itself takes 13 us.  Heads of 128: 47 KB of LDS and 168 registers, so that three workgroups share a CU
+// (two with the partial products beside the queries: 90 us instead of 78 for 153 blocks of 16 heads).
 template <int DX>
-__global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kernel(DeltaBlocks a) {
+__global__ __launch_bounds__(256, DX <= 2 ? 3 : 1) void delta_block_prepare_kernel(DeltaBlocks a) {
   constexpr int DP = 64 * DX, RS = DP + 4;
   extern __shared__ __align__(16) float lds[];
   float* k_lds = lds;                                      // [32][RS]
   float* q_lds = k_lds + kRows * RS;                       // [32][RS]
-  float* part = q_lds + kRows * RS;                        // [4 waves][6 tiles][64 lanes][4]
+  float* part = q_lds;                                     // [4 waves][6 tiles][64 lanes][4]
   double* b_mat = reinterpret_cast<double*>(part);         // B, strictly lower
   double* t_mat = b_mat + kRows * kMatB;                   // the 16 x 16 blocks on the diagonal of (I + B)^-1
   double* p_mat = t_mat + 2 * 16 * kMatT;                  // [4 waves]: one between two products
-  float* l_mat = part + 4 * 6 * 256;                       // [32][kMat]
+  float* l_mat = part + delta_prepare_shared_floats(DP);   // [32][kMat]
   float* g_lds = l_mat + kRows * kMat;                     // [32]
   float* beta_lds = g_lds + kRows;                         // [32]
   float* ks_lds = beta_lds + kRows;                        // [32]
@@ -599,6 +605,7 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_prepare_kern
         acc[5] = mfma4_f64(q1d, k1d, acc[5]);
       }
     }
+    __syncthreads();                                       // the sums take the queries' place
     // [tile][lane of mfma4's result][4]
 #pragma unroll
     for (int i = 0; i < 6; ++i)
@@ -824,8 +831,8 @@ __device__ __forceinline__ int lane_value(int v) {
 // copied from turn to turn (its load would be waited for right there), and the first block's loads keep the order of
 // the loop's, which waits for what both orders have in common.
 // Two prompts of 2999 and 1854 tokens, 16 heads of 128 x 128 (94 blocks in a row), under the tracer: the walk 178 us, 1.9
-// us per block (212 with the loads at once and choices by branches), the prepare kernel 92, the norms 20 and the
-// step kernel's empty launch 5; a call 267 (333), where the token-by-token walk of the same prompts takes 1079.
+// us per block (212 with the loads at once and choices by branches), the prepare kernel 78, the norms 20 and the
+// step kernel's empty launch 5; a call 251 (333), where the token-by-token walk of the same prompts takes 1079.
 // What a block adds to the state is summed in 64 bits: in 32 a call is 20 us less and states are 1.2 times as far
 // from 64 bits as token by token where keys share a part three times as large as the rest (1.0).
 template <int DX>
