@@ -450,9 +450,11 @@ int vla_seq_gla_chunks(void* out, int64_t out_stride, const void* q, int64_t q_s
  * without a window, to its last new row) behind those of the sequences before it: rows [num_rows, width].
  * max_seq_rows: the most rows of one sequence.
  * key_first > 0 (one sequence): from its visible row key_first on.
+ * vla_seq_latent_form: keys [num_rows, heads * dim] and values [num_rows, heads * vdim] = the first `rank` numbers of rows
+ * [num_rows, row_width] times w_uk [heads * dim, rank] transposed and w_uv [heads, rank, vdim], summed in fp32; keys_rest (as
+ * keys): what rounding to 16 bits took from the keys.  rank: a multiple of 32.  All pointers 16-byte aligned.
  * vla_seq_latent_prompt: out [T, heads * vdim] from q [T, heads * (dim + rot)] (a head's row: plain | rotated),
- * keys [num_rows, heads * dim] and values [num_rows, heads * vdim] that the caller formed from the gathered
- * latents, keys_rest (as keys) what rounding to 16 bits took from the keys (scores are of their sum), and the
+ * the formed keys, keys_rest and values (scores are of keys and keys_rest together), and the
  * gathered rows themselves for the rotated parts behind them.
  * One sequence's keys may come in ranges, one call after the other: num_rows rows from row key_first (a multiple of
  * 64) of its key_total visible ones on, whole tiles of 64 except at the end, and carry, fp32 [T, heads, 68 or
@@ -467,6 +469,9 @@ int vla_seq_latent_gather(void* rows, int num_rows, const void* cache, const int
                           int max_blocks, const int* query_start_loc, const int* context_lens, int num_seqs,
                           int max_seq_rows, int width, int block_size, int num_blocks, int window, int key_first,
                           int dtype, void* stream);
+int vla_seq_latent_form(void* keys, void* keys_rest, void* values, const void* rows, int num_rows, int row_width,
+                        const void* w_uk, const void* w_uv, int heads, int dim, int vdim, int rank, int dtype,
+                        void* stream);
 int vla_seq_latent_prompt(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* keys,
                           const void* keys_rest, const void* values, const void* rows, int num_rows, const int* query_start_loc,
                           const int* context_lens, int num_seqs, int max_query_len, int heads, int dim,

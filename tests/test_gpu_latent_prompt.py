@@ -288,3 +288,41 @@ def test_a_portion_of_a_long_context(workspace):
     want = attn(q.clone(), kv, cache.clone(), replace(batch, host_query_lens=None), gate)
     for rows in (slice(0, 70), slice(70, 120)):
         assert float((got[rows] - want[rows]).abs().max()) <= 0.03 * float(want[rows].abs().max())
+
+
+@pytest.mark.parametrize("rows", [1, 255, 257, 600])
+@pytest.mark.parametrize("sizes", [(1, 8, 16, 8, 32), (3, 40, 0, 72, 64), (2, 128, 64, 128, 96), (5, 136, 16, 120, 128), (16, 128, 64, 64, 512)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_formed_keys_and_values(rows, sizes, dtype):
+    """Around tiles of 256 rows and 128 columns, one to sixteen stages of the rank, heads that share a tile or part of one,
+    weights at odd addresses: a key and what it lost together to 2 roundings of 16 bits and the sum's own (2^-24 of the
+    terms' sum, by their number), a key or value alone to one."""
+    from vllm_legacy_amd import _seq_ops as ops
+    H, D, Rr, V, C = sizes
+    x = rnd((rows, C + Rr), 1).to(dtype).to(DEV)
+    w_uk, w_uv = (rnd((H * D * C + 1, ), 2, C**-0.5).to(dtype).to(DEV), rnd((H * C * V + 1, ), 3, C**-0.5).to(dtype).to(DEV))
+    eps = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    tiny = 2.0**-24 if dtype == torch.float16 else 0.0      # what a remainder below the least normal number keeps
+    for off in (0, 1):
+        uk, uv = w_uk[off:off + H * D * C].view(H, D, C), w_uv[off:off + H * C * V].view(H, C, V)
+        keys, rest, values = ops.latent_form(x, uk, uv)
+        lat = x[:, :C].double().cpu()
+        for got, left, w in ((keys, rest, uk.double().cpu().reshape(H * D, C).t()),
+                             (values, None, uv.double().cpu().transpose(0, 1).reshape(C, H * V))):
+            want, terms = lat @ w, lat.abs() @ w.abs()
+            got = got.double().cpu()
+            bar = eps * want.abs() + C * 2.0**-24 * terms + tiny
+            assert bool(((got - want).abs() <= bar).all())
+            if left is not None:
+                assert bool(((got + left.double().cpu() - want).abs() <= 2 * eps * eps * want.abs() + C * 2.0**-24 * terms + tiny).all())
+
+
+def test_which_steps_are_formed():
+    """Short runs behind few keys, and steps of both kinds only where there is enough for two ways."""
+    from vllm_legacy_amd.attention.backends.latent_kv import LatentKVAttention
+    attn = LatentKVAttention(16, 128, 64, 128, 512, 192**-0.5, 64, 1e4, None, 1e-5, torch.bfloat16, DEV)
+    for lens, contexts, want in (([33], [0], [True]), ([31], [0], None), ([33], [300], None), ([48], [300], [True]), ([60], [2000], None),
+                                 ([96], [4000], [True]), ([64, 20], [0, 0], None), ([64, 60], [0, 2000], None),
+                                 ([1000, 20], [0, 0], [True, False])):
+        got = attn._stretches(step(lens, contexts)[0])
+        assert (got and [s[4] for s in got]) == want, (lens, contexts)

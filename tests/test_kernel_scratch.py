@@ -38,7 +38,7 @@ def kernels_of_object(elf):
     return {}
 
 
-@pytest.mark.parametrize("kernel,instances", [("latent_prompt_kernel", 24), ("kv_attention_tile_kernel", 64)])
+@pytest.mark.parametrize("kernel,instances", [("latent_prompt_kernel", 24), ("latent_form_kernel", 2), ("kv_attention_tile_kernel", 64)])
 def test_nothing_is_kept_in_memory(kernel, instances):
     from vllm_legacy_amd import _lib
     if not os.path.exists(_lib.SEQ_LIB_PATH):

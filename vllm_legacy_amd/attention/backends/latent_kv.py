@@ -82,6 +82,8 @@ class LatentKVAttention(nn.Module):
         self.w_uv_t = nn.Parameter(torch.zeros((num_heads, rank, value_dim), dtype=dtype, device=device),
                                    requires_grad=False)
         self.formed_fits = True
+        gain = 5 * (2 * rank + rot_dim) - 2 * (head_dim + rot_dim + value_dim)      # (formed_min_rows)
+        self.least_rows = -(-rank * (head_dim + value_dim) // gain) if gain > 0 else 1 << 30
 
     def set_weights(self, uk: torch.Tensor, uv: torch.Tensor, latent_norm: Optional[torch.Tensor] = None,
                     sinks: Optional[torch.Tensor] = None) -> None:
@@ -122,46 +124,64 @@ class LatentKVAttention(nn.Module):
     # the longest stretches of sequences a step is cut into; one that alternates more often stays whole
     MAX_STRETCHES = 4
 
-    # Multiply-adds of a step on the latent kernel (a fifth of a matrix product's rate) from which the other way's
-    # seven launches more are paid back.  Rows x keys before them, 16 heads of 128 + 64, rank 512, latent / formed us
-    # per call: 128 x 2000 (4.6e9) 118 / 147, 192 x 2000 (7.0e9) 179 / 133, four of 384 x 0 (5.1e9) 132 / 141, one of 768
-    # x 0 (5.1e9) 161 / 138, 1024 x 0 (9.1e9) 159 / 138.  (The launches take the host 138 us, whatever the sizes.)
-    FORMED_MIN_WORK = 6e9
-    # Rows of a run at least: forming a key's numbers costs as much for few rows as for many.  Sixteen of 64 rows x
-    # 1000 266 / 338, of 96 389 / 328; four of 64 x 2000 174 / 212, of 96 282 / 208; one of 96 x 4000 162 / 175.
+    # Multiply-adds of a step on the latent kernel (a fifth of a matrix product's rate) from which the other way, which
+    # gathers and forms keys first, is the faster one.  Rows x keys before them, 16 heads of 128 + 64, rank 512, latent / formed
+    # us on the GPU: one of 33 x 0 (1e7) 38 / 30, 64 x 0 (4e7) 40 / 30, 256 x 0 (6e8) 69 / 41, 400 x 0 89 / 45.  (Python and
+    # launches take the host 98 and 78 us.)  A step that goes both ways pays for both: so many times the work.
+    FORMED_MIN_WORK = 9e6
+    FORMED_MIXED_WORK = 700
+    # Rows of a run at least: forming a key's numbers costs as much for few rows as for many, and one tile of rows walks
+    # all keys by itself where the latent kernel shares them out.  One row more for so many keys ahead of them, no more than
+    # FORMED_MIN_ROWS, and that many in a step that goes both ways.  33 rows x 300 68 / 42, x 1000 70 / 61, x 2000 79 / 84, thirty
+    # of x 300 85 / 43 and x 1000 333 / 376; 48 x 1500 107 / 86, x 4000 113 / 138, thirty of x 2000 666 / 690; 64 x 1000
+    # 73 / 63, x 2000 77 / 91; 96 x 500 74 / 51, x 4000 158 / 138.
+    FORMED_FEW_ROWS = 32
+    FORMED_KEYS_PER_ROW = 64
     FORMED_MIN_ROWS = 96
 
-    def formed_min_rows(self) -> int:
-        """Rows from which a run's keys and values are worth forming.  A (query, key) pair of a head costs the
-        latent kernel 2 rank + rot multiply-adds at a fifth of a matrix product's rate (less where the rank is small),
-        the formed one dim + rot + vdim at about half of it; forming costs rank (dim + vdim) per key at the full rate.
-        (A rank of 64 beside heads of 128 + 64: 1024 rows 98 / 140 us, 2048 167 / 141, 4096 535 / 186.)"""
-        C, D, R, V = self.rank, self.head_dim, self.rot_dim, self.value_dim
-        gain = 5 * (2 * C + R) - 2 * (D + R + V)
-        return max(self.FORMED_MIN_ROWS, -(-C * (D + V) // gain)) if gain > 0 else 1 << 30
+    def formed_min_rows(self, context: Optional[int] = None) -> int:
+        """Rows from which a run's keys and values are worth forming, behind `context` keys (None: any number).  A (query,
+        key) pair of a head costs the latent kernel 2 rank + rot multiply-adds at a fifth of a matrix product's rate (less
+        where the rank is small), the formed one dim + rot + vdim at about half of it; forming costs rank (dim + vdim) per
+        key at the full rate.  (A rank of 64 beside heads of 128 + 64: 1024 rows 98 / 140 us, 2048 167 / 141, 4096 535 / 186,
+        with three products of a library for the forming.)"""
+        least = self.FORMED_MIN_ROWS
+        if context is not None:
+            least = min(least, self.FORMED_FEW_ROWS + min(context, self.window or context) // self.FORMED_KEYS_PER_ROW)
+        return max(least, self.least_rows)
 
     def _stretches(self, batch: SequenceBatch):
         """[[first sequence, one behind the last, first row, one behind the last, formed]]: neighbours that go
         the same way; None when the whole step takes the latent kernel."""
         each = self.num_heads * (2 * self.rank + self.rot_dim)          # multiply-adds of a (query, key) pair
-        if batch.num_tokens * batch.max_seq_len * each < self.FORMED_MIN_WORK:
+        most = batch.num_tokens * batch.max_seq_len * each
+        if most < self.FORMED_MIN_WORK or batch.max_query_len < self.FORMED_FEW_ROWS:
             return None                 # most steps: no more than this is asked of them
-        least = self.formed_min_rows()
-        if batch.max_query_len < least or not self.scale > 0 or not self.formed_fits:
-            return None
         q, ctx = batch.host_query_lens, batch.host_context_lens
-        if q is None or ctx is None or torch.cuda.is_current_stream_capturing():
+        if q is None or ctx is None:
+            return None
+        work, short = self.FORMED_MIN_WORK, min(q)
+        if short >= self.FORMED_FEW_ROWS and short >= self.least_rows and (
+                short >= self.formed_min_rows(max(ctx)) or all(n >= self.formed_min_rows(c) for n, c in zip(q, ctx))):
+            least = 0                   # all of them
+        else:
+            least, work = self.formed_min_rows(), work * self.FORMED_MIXED_WORK
+            if most < work:
+                return None
+        if not self.scale > 0 or not self.formed_fits or torch.cuda.is_current_stream_capturing():
             return None                 # a captured step is replayed with other lengths than the host's
-        out, row, pairs = [], 0, 0
+        out, row = [], 0
+        pairs = 0
         for b, (n, c) in enumerate(zip(q, ctx)):
-            if n >= least:
+            formed = n >= least
+            if formed:
                 pairs += n * min(c, self.window or c) + (n * (n + 1) // 2 if not self.window else n * min(n, self.window))
-            if out and out[-1][4] == (n >= least):
+            if out and out[-1][4] == formed:
                 out[-1][1], out[-1][3] = b + 1, row + n
             else:
-                out.append([b, b + 1, row, row + n, n >= least])
+                out.append([b, b + 1, row, row + n, formed])
             row += n
-        if pairs * each < self.FORMED_MIN_WORK:
+        if pairs * each < work:
             return None
         return out if len(out) <= self.MAX_STRETCHES else None
 
@@ -198,8 +218,6 @@ class LatentKVAttention(nn.Module):
         H, D, Rr, V, C = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.rank
         ql, cl = batch.host_query_lens[s0:s1], batch.host_context_lens[s0:s1]
         sinks = None if self.sinks is None else self.sinks.data
-        w_uk = self.w_uk.data.reshape(H * D, C).t()
-        w_uv = self.w_uv_t.data.transpose(0, 1).reshape(C, H * V)
         carry = None
         for b0, b1, k0, count, total in self._formed_parts(ql, cl, self.formed_keys(q.element_size())):
             if k0 == 0:
@@ -213,16 +231,13 @@ class LatentKVAttention(nn.Module):
             rows = torch.empty((count, C + Rr), dtype=q.dtype, device=q.device)
             longest = count if b1 == b0 + 1 else max(c + n for n, c in zip(ql[b0:b1], cl[b0:b1]))
             ops.latent_gather(rows, cache, tables, starts, ctx, longest, self.window, k0)
-            latents = rows[:, :C]
             # A key's rounding is its own, where that of a query on the latents' side is the same for all keys and
             # mostly cancels in the softmax: the keys keep what they lose.
-            keys = torch.mm(latents, w_uk)
-            keys_rest = torch.addmm(keys, latents, w_uk, beta=-1)
-            values = torch.mm(latents, w_uv)
+            keys, keys_rest, values = ops.latent_form(rows, self.w_uk.data, self.w_uv_t.data)
             ops.latent_prompt(out[t0:t1], q[t0:t1], keys, keys_rest, values, rows, starts, ctx, max(ql[b0:b1]), H, D, Rr, V,
                               self.scale, self.window, None if gate is None else gate[t0:t1], sinks, k0,
                               total if carry is not None else 0, carry)
-            del rows, latents, keys, keys_rest, values          # the next part's take their place
+            del rows, keys, keys_rest, values          # the next part's take their place
 
     def _attend_latent(self, q, cache, batch: SequenceBatch, gate, part=None) -> torch.Tensor:
         """The step, or of part (s0, s1, r0, r1) sequences s0 .. s1 - 1 (rows r0 .. r1 - 1), on the cached latents ->
@@ -280,7 +295,7 @@ class LatentKVAttention(nn.Module):
             D, Rr = self.head_dim, self.rot_dim
             ops.latent_rotary_write(q, D + Rr, D, self.num_heads, kv, self.latent_norm.data, self.eps, cache, batch.positions,
                                     batch.slot_mapping, self.inv_freq, self.magnitude, self.rot_dims, self.interleaved)
-        stretches = None if batch.max_query_len < self.FORMED_MIN_ROWS else self._stretches(batch)
+        stretches = None if batch.max_query_len < self.FORMED_FEW_ROWS else self._stretches(batch)
         if stretches is None or not ops.latent_prompt_supported(q, self.head_dim, self.rot_dim, self.value_dim, self.rank, cache):
             return self._attend_latent(q, cache, batch, gate)
         out = torch.empty((q.shape[0], self.num_heads * self.value_dim), dtype=q.dtype, device=q.device)

@@ -3,11 +3,11 @@
 // Scoring the cached latent itself costs a head 2 rank + rot numbers per (query, key) pair; a head's own
 // key and value cost dim + rot + vdim, and forming them rank (dim + vdim) per key and head, once for all
 // queries of the run.  A run of rows therefore gathers its visible cache rows into one place
-// (latent_gather_kernel), the caller multiplies them with the two up-projections, and
+// (latent_gather_kernel), latent_form_kernel multiplies them with the two up-projections, and
 // latent_prompt_kernel below is plain causal attention with keys [formed (dim) | shared rotated part
 // (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 137 us under the tracer (630 TFLOP/s; 880
-// with the remainders' product) where latent_attention_tile_kernel takes 1685, plus 9 us to gather and 60 for the
-// three products (the products on the query's side that they replace take 46).
+// with the remainders' product) where latent_attention_tile_kernel takes 1685, plus 5 us to gather (9 with 32 rows to a
+// workgroup instead of 8) and 31 to form keys and values (the products on the query's side that they replace take 46).
 //
 // Keys come as two 16-bit numbers, the rounded one and what rounding took.  The latent kernel rounds the query's
 // side, which is the same for all keys of a row and mostly cancels in the softmax; a key's rounding is its own.
@@ -54,7 +54,7 @@ constexpr int kWaves = 4;
 constexpr int kRowsPerGroup = kRowsPerWave * kWaves, kGroupShift = 7;
 static_assert(kRowsPerGroup == 1 << kGroupShift, "tiles of rows are ranked by their level");
 constexpr int kEarly = 4;           // a wave's DMA instructions for the next keys ahead of the softmax
-constexpr int kGatherRows = 32;
+constexpr int kGatherRows = 8;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef s16x4 __attribute__((address_space(3))) * lds_s16x4;
 
@@ -122,6 +122,164 @@ __global__ __launch_bounds__(256) void latent_gather_kernel(
       rows[(int64_t)(base + r0 + r) * pieces + v] = cache[((int64_t)blk * block_size + j % block_size) * pieces + v];
     }
   }
+}
+
+// Every head's keys, in two numbers each, and values of the gathered rows: [num_rows, rank] times W_uk^T [rank, heads * dim]
+// and W_uv [rank, heads * vdim] in one launch.  A workgroup has 256 rows and 128 columns of keys or of values, a wave 128 rows
+// and 64 columns; products on 32x32x16 MFMAs with the weights as the rows, so that a lane ends with neighbouring columns of
+// one row.  Stages of 32 numbers of the rank come by LDS-DMA into a ring of three (72 KB: two workgroups to a CU, one's
+// results leave under the other's products), 16-byte pieces (values' weights, which lie with a head's columns
+// as rows and are read transposing: 64-byte ones) exchanged by the row's number.  A key's remainder comes from the sum in the
+// registers.  4096 rows of rank 512 and 16 heads of 128 + 128: 31 us, 550 TFLOP/s, bound by LDS (a stage is 72 KB of it read
+// and written in 1150 cycles of the two workgroups, beside 1024 of products) and by the 50 MB of results at the end; a
+// library's product per operand and a third for what the first lost, with a copy of the keys ahead of it and one of the
+// values' weights, were 70.
+constexpr int kFormRows = 256, kFormCols = 128, kFormStep = 32;
+constexpr int kFormLatents = kFormRows * kFormStep * 2, kFormStage = kFormLatents + kFormCols * kFormStep * 2;
+struct LatentForm {
+  void* keys;
+  void* keys_rest;
+  void* values;
+  const void* rows;             // [num_rows, row_width]: latents of `rank` and something behind them
+  const void* w_uk;             // [heads * dim, rank]
+  const void* w_uv;             // [heads, rank, vdim]
+  int num_rows, row_width, heads, dim, vdim, rank;
+  int key_tiles, tiles;         // column tiles: of keys, and all
+};
+
+template <class S>
+__global__ __launch_bounds__(256, 2) void latent_form_kernel(LatentForm a) {
+  using T = typename S::T;
+  using M = Mma<S>;
+  extern __shared__ __align__(16) unsigned char smem[];
+  // an XCD's workgroups (every eighth) share an eighth of the column tiles, whose weights stay in its L2
+  const int share = (a.tiles + 7) / 8, id = blockIdx.x >> 3;
+  const int tile = (blockIdx.x & 7) + 8 * (id % share), m0 = id / share * kFormRows;
+  if (tile >= a.tiles) return;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hf = lane >> 5, c = lane & 31, wm = w & 1, wn = w >> 1;
+  const int steps = a.rank / kFormStep;
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  const unsigned char* src[6];                             // four pieces of latents, two of weights
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int r = 16 * (4 * w + u) + (lane >> 2), piece = (lane & 3) ^ ((r >> 2) & 3);
+    src[u] = (const unsigned char*)a.rows + ((int64_t)min(m0 + r, a.num_rows - 1) * a.row_width + 8 * piece) * 2;
+  }
+  auto form = [&](auto is_key) __attribute__((always_inline)) {
+    constexpr bool KEY = decltype(is_key)::value;
+    const int n_all = KEY ? a.heads * a.dim : a.heads * a.vdim;
+    const int n0 = kFormCols * (KEY ? tile : tile - a.key_tiles);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int i = 2 * w + u;
+      if constexpr (KEY) {
+        const int r = 16 * i + (lane >> 2), piece = (lane & 3) ^ ((r >> 2) & 3);
+        src[4 + u] = (const unsigned char*)a.w_uk + ((int64_t)min(n0 + r, n_all - 1) * a.rank + 8 * piece) * 2;
+      } else {
+        const int k = 4 * i + (lane >> 4), s = lane & 15;
+        const int n = min(n0 + 32 * ((s >> 2) ^ (k & 3)) + 8 * (s & 3), n_all - 8), h = n / a.vdim;
+        src[4 + u] = (const unsigned char*)a.w_uv + (((int64_t)h * a.rank + k) * a.vdim + (n - h * a.vdim)) * 2;
+      }
+    }
+    const int w_step = KEY ? 2 * kFormStep : 2 * kFormStep * a.vdim;
+    auto bring = [&](int u, int step, int slot, int go) {
+      tile_dma16(src[u] + (int64_t)step * (u < 4 ? 2 * kFormStep : w_step),
+                 lds0 + slot * kFormStage + (u < 4 ? (4 * w + u) * 1024 : kFormLatents + (2 * w + u - 4) * 1024), go);
+    };
+    f32x16 acc[4][2];
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
+#pragma unroll
+    for (int u = 0; u < 6; ++u) bring(u, 0, 0, 1);
+#pragma unroll
+    for (int u = 0; u < 6; ++u) bring(u, 1, 1, steps > 1);
+    const int swap = (c >> 2) & 3, i16 = c & 15;
+    // fragment i of 16 numbers of the rank: two of weights, then four of rows
+    auto read = [&](const unsigned char* at, int ks, int i) {
+      if (i >= 2) return *reinterpret_cast<const u32x4*>(at + (128 * wm + 32 * (i - 2) + c) * 64 + 16 * ((2 * ks + hf) ^ swap));
+      if constexpr (KEY) {
+        return *reinterpret_cast<const u32x4*>(at + kFormLatents + (64 * wn + 32 * i + c) * 64 + 16 * ((2 * ks + hf) ^ swap));
+      } else {
+        const unsigned char* p = at + kFormLatents + (16 * ks + 8 * hf + (i16 >> 2)) * (2 * kFormCols) +
+                                 64 * ((2 * wn + i) ^ (i16 >> 2)) + 32 * (c >> 4) + 8 * (i16 & 3);
+        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)p));
+        const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(p + 4 * 2 * kFormCols)));
+        return u32x4{lo[0], lo[1], hi[0], hi[1]};
+      }
+    };
+    int slot = 0;
+    for (int it = 0; it < steps; ++it) {
+      // this stage has come (of the younger one's six pieces none need have), and the stage before it is read
+      if (it + 1 < steps)
+        __builtin_amdgcn_s_waitcnt(0x0076);                // vmcnt(6), lgkmcnt(0)
+      else
+        __builtin_amdgcn_s_waitcnt(0x0070);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const unsigned char* at = smem + slot * kFormStage;
+      const int free_slot = slot == 0 ? 2 : slot - 1;
+      u32x4 f[2][6];
+#pragma unroll
+      for (int i = 0; i < 6; ++i) f[0][i] = read(at, 0, i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if (ks == 0 && i < 6) f[1][i] = read(at, 1, i);
+          acc[i >> 1][i & 1] = M::run(f[ks][i & 1], f[ks][2 + (i >> 1)], acc[i >> 1][i & 1]);
+          if (ks == 0 && i >= 2) bring(i - 2, it + 2, free_slot, it + 2 < steps);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      slot = slot == 2 ? 0 : slot + 1;
+    }
+    // eight neighbouring columns a lane: of two groups of eight, the lower half of the wave has the first
+    const int n = n0 + 64 * wn + 8 * hf;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+      const int row = m0 + 128 * wm + 32 * mb + c;
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          u32x4 put, rest;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            uint32_t hi[2], lo[2];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+              const float x = acc[mb][nb][8 * j + 4 * g + 2 * e], y = acc[mb][nb][8 * j + 4 * g + 2 * e + 1];
+              hi[g] = M::pack2(x, y);
+              if constexpr (KEY) lo[g] = M::pack2(x - lo16<S>(hi[g]), y - hi16<S>(hi[g]));
+            }
+            const auto both = __builtin_amdgcn_permlane32_swap(hi[0], hi[1], false, false);
+            put[e] = both[0];
+            put[2 + e] = both[1];
+            if constexpr (KEY) {
+              const auto left = __builtin_amdgcn_permlane32_swap(lo[0], lo[1], false, false);
+              rest[e] = left[0];
+              rest[2 + e] = left[1];
+            }
+          }
+          const int col = n + 32 * nb + 16 * j;
+          if (row < a.num_rows && col < n_all) {
+            const int64_t to = (int64_t)row * n_all + col;
+            *reinterpret_cast<u32x4*>((T*)(KEY ? a.keys : a.values) + to) = put;
+            if constexpr (KEY) *reinterpret_cast<u32x4*>((T*)a.keys_rest + to) = rest;
+          }
+        }
+    }
+  };
+  if (tile < a.key_tiles)
+    form(std::true_type{});
+  else
+    form(std::false_type{});
 }
 
 struct LatentPrompt {
@@ -596,6 +754,49 @@ extern "C" int vla_seq_latent_gather(void* rows, int num_rows, const void* cache
       num_blocks, window, num_rows, key_first);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   return VLA_OK;
+}
+
+extern "C" int vla_seq_latent_form(void* keys, void* keys_rest, void* values, const void* rows, int num_rows, int row_width,
+                                  const void* w_uk, const void* w_uv, int heads, int dim, int vdim, int rank, int dtype,
+                                  void* stream) {
+  if (num_rows == 0) return VLA_OK;
+  if (!keys || !keys_rest || !values || !rows || !w_uk || !w_uv || num_rows < 0 || heads <= 0 || dim <= 0 || vdim <= 0 ||
+      rank <= 0 || row_width < rank || (int64_t)heads * dim > 0x3fffffff || (int64_t)heads * vdim > 0x3fffffff)
+    return VLA_ERR_ARG;
+  if (dtype != VLA_F16 && dtype != VLA_BF16) return VLA_ERR_DTYPE;
+  if (dim % 8 || vdim % 8 || rank % kFormStep || row_width % 8) return VLA_ERR_HEAD_SIZE;
+  for (const void* p : {(const void*)keys, (const void*)keys_rest, (const void*)values, rows, w_uk, w_uv})
+    if ((uintptr_t)p % 16) return VLA_ERR_ARG;
+  LatentForm a;
+  a.keys = keys;
+  a.keys_rest = keys_rest;
+  a.values = values;
+  a.rows = rows;
+  a.w_uk = w_uk;
+  a.w_uv = w_uv;
+  a.num_rows = num_rows;
+  a.row_width = row_width;
+  a.heads = heads;
+  a.dim = dim;
+  a.vdim = vdim;
+  a.rank = rank;
+  a.key_tiles = (heads * dim + kFormCols - 1) / kFormCols;
+  a.tiles = a.key_tiles + (heads * vdim + kFormCols - 1) / kFormCols;
+  const int64_t groups = ((int64_t)a.tiles + 7) / 8 * 8 * ((num_rows + (int64_t)kFormRows - 1) / kFormRows);
+  if (groups > 0xffffff) return VLA_ERR_ARG;
+  auto go = [&](auto s) -> int {
+    using S = decltype(s);
+    static std::atomic<bool> raised{false};           // LDS limit: raised once per kernel, not per launch
+    if (!raised.load(std::memory_order_relaxed)) {
+      VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_form_kernel<S>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, 3 * kFormStage));
+      raised.store(true, std::memory_order_relaxed);
+    }
+    latent_form_kernel<S><<<(unsigned)groups, 256, 3 * kFormStage, (hipStream_t)stream>>>(a);
+    VLA_SEQ_HIP_CHECK(hipGetLastError());
+    return VLA_OK;
+  };
+  return dtype == VLA_BF16 ? go(BF16{}) : go(F16{});
 }
 
 extern "C" int vla_seq_latent_prompt_form(int num_rows, int num_seqs, int max_query_len, int heads, int dim, int rot, int vdim,
