@@ -29,7 +29,7 @@ def _dt(t: torch.Tensor) -> int:
 
 
 def _stream(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)     # (0.2 us; by way of a Stream object 3)
 
 
 def _ptr(t) -> Optional[int]:
