@@ -467,3 +467,32 @@ def test_grouped_mid_row_blocks(ops, counts, tail, gather):
         start += c
     if not gather:
         assert not got[start:].any()
+
+
+# Launches of more than one round of 256 workgroups whose last tiles are cut into K slices (2, 3, 4 or 8 of them):
+# a last row and column tile partly outside the matrix, 64-deep groups, the GPTQ zero convention; against fp32
+# products of the dequantised weights, to one rounding and the sums' own error (2^-24 of the terms, K of them).
+@pytest.mark.parametrize("kind,m,k,n,group,slices", [("awq", 1930, 4096, 4104, 128, 8), ("awq", 2784, 14336, 4096, 128, 2),
+                                                     ("gptq", 300, 4096, 28672, 128, 2), ("awq", 1025, 4096, 8200, 64, 4),
+                                                     ("gptq", 2400, 6144, 4120, 64, 3)])
+def test_last_tiles_in_slices(ops, kind, m, k, n, group, slices):
+    from vllm_legacy_amd import _lib
+    tiles = -(-n // 256) * -(-m // 128)
+    assert _lib.lib().vla_q4_gemm_workspace_bytes(m, n, k, group) == slices * (tiles % 256) * 128 * 256 * 4
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    x = (torch.rand(m, k, generator=g, device="cuda") * 2 - 1).half()
+    qw = torch.randint(-2**31, 2**31 - 1, (k // 8, n), generator=g, device="cuda", dtype=torch.int32)
+    qz = torch.randint(-2**31, 2**31 - 1, (k // group, n // 8), generator=g, device="cuda", dtype=torch.int32)
+    sc = ((torch.rand(k // group, n, generator=g, device="cuda") + 0.5) * 1e-2).half()
+    got = ops.q4_gemm_packed(x, qw, qz, sc, 1 if kind == "gptq" else 0)
+    part = ops.q4_gemm_packed_partial(x, qw, qz, sc, 1 if kind == "gptq" else 0)
+    assert torch.equal(part, got)                # (finished, too: no slabs for a consumer)
+    # the nibble of k 8 r + e; zeros are packed plainly, eight columns a word
+    nibble = [0, 4, 1, 5, 2, 6, 3, 7]
+    cols = torch.unique(torch.cat([torch.arange(0, n, 37, device="cuda"), torch.arange(n - 40, n, device="cuda")]))
+    q = torch.stack([(qw[:, cols] >> (4 * o)) & 15 for o in nibble], 1).reshape(k, -1)
+    z = (qz[:, cols // 8] >> (4 * (cols % 8))[None].int()) & 15
+    w = ((q - z.repeat_interleave(group, 0) - (1 if kind == "gptq" else 0)).half() *
+         sc[:, cols].repeat_interleave(group, 0)).float()
+    want, terms = x.float() @ w, x.float().abs() @ w.abs()
+    assert bool(((got[:, cols].float() - want).abs() <= 2.0**-11 * want.abs() + k * 2.0**-24 * terms).all())

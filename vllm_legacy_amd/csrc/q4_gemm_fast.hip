@@ -1028,11 +1028,20 @@ struct Q4Dma2 {
   static_assert(BYTES >= 4 * 128 * 64 * 4, "the K parts' sums meet in the ring's memory");
 };
 
-template <int ZOFF, bool SPLIT, int STAGES, int D>
+// TAIL: the tiles behind the last whole round of 256 workgroups, which would leave most of the chip
+// idle for a round, are cut into K slices: workgroups tail.first .. are (tile, slice), their sums
+// go to fp32 slabs [slice][tile][128][256] that q4_tail_reduce_kernel adds up.
+struct Q4Tail {
+  int first = 0, tiles = 0, slices = 0;      // slices: 0 without a tail
+  float* slabs = nullptr;
+};
+
+template <int ZOFF, bool SPLIT, int STAGES, int D, bool TAIL = false>
 __global__ __launch_bounds__(512) void q4_gemm_dma2_kernel(
     const _Float16* __restrict__ x, const uint32_t* __restrict__ qw,
     const uint32_t* __restrict__ qz, const _Float16* __restrict__ scales, void* __restrict__ outp,
-    int m, int n, int k, int group_size, int k_per_split) {
+    int m, int n, int k, int group_size, int k_per_split, Q4Tail tail) {
+  static_assert(!TAIL || !SPLIT, "whole tiles and slices of the last ones");
   using L = Q4Dma2<STAGES>;
   constexpr int MT = 4, NT = 2;
   static_assert(D >= 1 && STAGES >= D + 1 && STAGES <= 3 && L::PER_TILE * (D - 1) < 64, "ring depth");
@@ -1045,9 +1054,19 @@ __global__ __launch_bounds__(512) void q4_gemm_dma2_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wn = wave & 3, wk = wave >> 2;                 // column wave, K part
   const int h = lane >> 5, c = lane & 31;
-  const int n0 = blockIdx.x * 256, m0 = blockIdx.y * 128;
-  const int k_part = k_per_split / 2;                      // the host keeps this whole groups
-  const int k_begin = blockIdx.z * k_per_split + wk * k_part;
+  int tile_x = blockIdx.x, tile_y = blockIdx.y, slice = blockIdx.z, k_slice = k_per_split;
+  const bool sliced = TAIL && (int)blockIdx.x >= tail.first;
+  if constexpr (TAIL) {
+    const int cols = (n + 255) >> 8, behind = (int)blockIdx.x - tail.first;
+    const int tile = sliced ? tail.first + behind / tail.slices : (int)blockIdx.x;
+    slice = sliced ? behind % tail.slices : 0;
+    k_slice = sliced ? k / tail.slices : k;
+    tile_y = tile / cols;
+    tile_x = tile - tile_y * cols;
+  }
+  const int n0 = tile_x * 256, m0 = tile_y * 128;
+  const int k_part = k_slice / 2;                          // the host keeps this whole groups
+  const int k_begin = slice * k_slice + wk * k_part;
   const int nsteps = k_part / TK;                          // the same for both parts
   if (nsteps <= 0) return;
   const int wcol0 = n0 + 64 * wn;                          // first column of this wave
@@ -1288,6 +1307,14 @@ __global__ __launch_bounds__(512) void q4_gemm_dma2_kernel(
       for (int a = 0; a < MT; ++a)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[g][a][i] += red[((g * MT + a) * 16 + i) * 64];
+  }
+  if constexpr (TAIL) {
+    if (sliced) {
+      const int64_t at = ((int64_t)slice * tail.tiles + ((int)blockIdx.x - tail.first) / tail.slices) * 128;
+#pragma unroll
+      for (int g = 0; g < NT; ++g) store_tile<true, MT>(acc[g], tail.slabs, c, 128, 64 * wn + 32 * g + 4 * h, 256, at);
+      return;
+    }
   }
 #pragma unroll
   for (int g = 0; g < NT; ++g)
@@ -1582,6 +1609,19 @@ __global__ __launch_bounds__(256) void q4_splitk_reduce_kernel(const float* __re
   *reinterpret_cast<u32x2*>(out + i) = o;
 }
 
+// out = fp16(sum over slices) of a product's last tiles (Q4Tail); 4 columns per thread
+__global__ __launch_bounds__(256) void q4_tail_reduce_kernel(Q4Tail tail, _Float16* __restrict__ out, int m, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x, tile = i >> 13, r = (i >> 6) & 127, c = 4 * (i & 63);
+  const int cols = (n + 255) >> 8, ty = (tail.first + tile) / cols, tx = tail.first + tile - ty * cols;
+  const int row = 128 * ty + r, col = 256 * tx + c;
+  if (row >= m || col >= n) return;
+  const float* at = tail.slabs + (int64_t)i * 4;
+  f32x4 s = *reinterpret_cast<const f32x4*>(at);
+  for (int p = 1; p < tail.slices; ++p) s += *reinterpret_cast<const f32x4*>(at + (int64_t)p * tail.tiles * (128 * 256));
+  const f16x2 lo = {(_Float16)s[0], (_Float16)s[1]}, hi = {(_Float16)s[2], (_Float16)s[3]};
+  *reinterpret_cast<u32x2*>(out + (int64_t)row * n + col) = u32x2{as_u32(lo), as_u32(hi)};
+}
+
 // AWQ [K][N/8] (8 columns per word, nibble P[i] = column 8j+i, P = {0,4,1,5,2,6,3,7}) ->
 // k-packed pair order [K/8][N]; one thread per output word
 __global__ __launch_bounds__(256) void awq_repack_weight_kernel(const uint32_t* __restrict__ qweight,
@@ -1814,12 +1854,12 @@ static hipError_t launch_dma(dim3 grid, hipStream_t s, const _Float16* x, const 
   return hipSuccess;
 }
 
-template <int Z, bool SP, int ST, int D>
+template <int Z, bool SP, int ST, int D, bool TAIL = false>
 static hipError_t launch_dma2(dim3 grid, hipStream_t s, const _Float16* x, const uint32_t* qw,
                               const uint32_t* qz, const _Float16* sc, void* dst, int m, int n, int k,
-                              int group, int kps) {
+                              int group, int kps, const Q4Tail& tail = Q4Tail()) {
   using L = Q4Dma2<ST>;
-  auto fn = q4_gemm_dma2_kernel<Z, SP, ST, D>;
+  auto fn = q4_gemm_dma2_kernel<Z, SP, ST, D, TAIL>;
   static std::atomic<uint64_t> ready{0};
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -1830,7 +1870,7 @@ static hipError_t launch_dma2(dim3 grid, hipStream_t s, const _Float16* x, const
     if (e != hipSuccess) return e;
     ready.fetch_or(1ull << (dev & 63), std::memory_order_release);
   }
-  hipLaunchKernelGGL(fn, grid, dim3(512), L::BYTES, s, x, qw, qz, sc, dst, m, n, k, group, kps);
+  hipLaunchKernelGGL(fn, grid, dim3(512), L::BYTES, s, x, qw, qz, sc, dst, m, n, k, group, kps, tail);
   return hipSuccess;
 }
 
@@ -1854,6 +1894,29 @@ static hipError_t launch_dma_kp(dim3 grid, hipStream_t s, const _Float16* x, con
   return hipSuccess;
 }
 
+// The K slices of a product's tiles behind the last whole round of 256 workgroups (one to a CU): as many as
+// the round has room for, at most 8, in whole groups and at least four K steps to each of a workgroup's two
+// parts.  Only where a round lasts: what is saved, (1 - 1 / slices) of a round of 16 us per 1024 of K, must
+// be worth the slabs and their reduction (8 .. 12 us).
+static Q4Tail pick_tail(int m, int n, int k, int group, const Q4Shape& shape) {
+  Q4Tail t;
+  if (group % TK || shape.mt != 4 || shape.nw != 8 || shape.splits != 1 || k % (2 * group) || k / (2 * TK) < 16 ||
+      (int64_t)m * k >= (1ll << 30) || (int64_t)n * 32 >= (1ll << 30))
+    return t;
+  const int64_t tiles = (int64_t)((n + 255) / 256) * ((m + 127) / 128);
+  const int rest = (int)(tiles % 256);
+  if (tiles < 256 || tiles > (1 << 24) || rest == 0) return t;
+  for (int s = 8; s >= 2; --s)
+    if (rest * s <= 256 && k % (s * 2 * group) == 0 && k / (s * 2 * TK) >= 4 && k - k / s >= 2048) {
+      t.first = (int)tiles - rest;
+      t.tiles = rest;
+      t.slices = s;
+      break;
+    }
+  return t;
+}
+static int64_t tail_bytes(const Q4Tail& t) { return (int64_t)t.slices * t.tiles * 128 * 256 * 4; }
+
 extern "C" int vla_set_q4_row_block_kernel(int mode) {
   return q4_mid_set_mode(mode) ? VLA_ERR_ARG : VLA_OK;
 }
@@ -1862,10 +1925,16 @@ extern "C" int64_t vla_q4_gemm_workspace_bytes(int m, int n, int k, int group) {
   if (m <= 0 || n <= 0 || k <= 0 || group <= 0) return 0;
   int sk_nwv = 0, sk_splits = 0, sk_cs = 0;
   int md_splits = 0;
-  const int s = q4_skinny_shape(m, n, k, group, &sk_nwv, &sk_splits, &sk_cs)
-                    ? sk_splits
-                    : q4_mid_shape(m, n, k, group, &md_splits) ? md_splits
-                                                               : pick_shape(m, n, k, group).splits;
+  int s;
+  if (q4_skinny_shape(m, n, k, group, &sk_nwv, &sk_splits, &sk_cs)) {
+    s = sk_splits;
+  } else if (q4_mid_shape(m, n, k, group, &md_splits)) {
+    s = md_splits;
+  } else {
+    const Q4Shape shape = pick_shape(m, n, k, group);
+    s = shape.splits;
+    if (s == 1) return tail_bytes(pick_tail(m, n, k, group, shape));
+  }
   return s > 1 ? (int64_t)s * m * n * 4 : 0;
 }
 
@@ -1942,6 +2011,19 @@ static int q4_gemm_run(const void* x, const int32_t* qweight, const int32_t* qze
   const int kps = k / splits;
   void* dst = splits > 1 ? workspace : out;
   const bool parts_ok = kps % (2 * (group > TK ? group : TK)) == 0;   // two K parts of whole groups
+  Q4Tail tail = pick_tail(m, n, k, group, shape);
+  if (tail.slices && dma_env < 0 && workspace && workspace_bytes >= tail_bytes(tail) && (uintptr_t)workspace % 16 == 0) {
+    tail.slabs = (float*)workspace;
+    const dim3 tgrid((unsigned)(tail.first + tail.tiles * tail.slices));
+    auto go = [&](auto z) {
+      return launch_dma2<decltype(z)::value, false, 3, 2, true>(tgrid, s, (const _Float16*)x, (const uint32_t*)qweight, (const uint32_t*)qzeros,
+                                                                (const _Float16*)scales, out, m, n, k, group, k, tail);
+    };
+    VLA_HIP_CHECK((zero_offset == 0 ? go(std::integral_constant<int, 0>()) : go(std::integral_constant<int, 1>())));
+    hipLaunchKernelGGL(q4_tail_reduce_kernel, dim3((unsigned)tail.tiles * 32), dim3(256), 0, s, tail, (_Float16*)out, m, n);
+    VLA_HIP_CHECK(hipGetLastError());
+    return VLA_OK;
+  }
   if (dma_env < 0) dma_stages = (splits == 1 && shape.nw == 8 && parts_ok && kps / (2 * TK) >= 16) ? 23 : 3;
   if (dma_stages == 23 && !(shape.nw == 8 && parts_ok)) dma_stages = 3;
 #define VLA_Q4_ARGS                                                                            \
