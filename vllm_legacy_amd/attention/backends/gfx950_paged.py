@@ -215,13 +215,13 @@ class Gfx950PagedAttentionImpl(AttentionImpl):
                     raise NotImplementedError(
                         f"prefix prefill: dtype {query.dtype}, head size {self.head_size}, "
                         f"block size {block_size} has no gfx950 kernel")
-                output[:n_pre] = PagedAttention.forward_prefix(
+                PagedAttention.forward_prefix(
                     query[:n_pre], key[:n_pre], value[:n_pre], key_cache, value_cache,
                     bt.to(torch.int32), prefill_meta.query_start_loc.to(torch.int32),
                     prefill_meta.seq_lens_tensor.to(torch.int32),
                     prefill_meta.context_lens_tensor.to(torch.int32),
                     int(prefill_meta.max_query_len), self._alibi(query.device),
-                    self.sliding_window, self.kv_cache_dtype, kv_scale, self.scale)
+                    self.sliding_window, self.kv_cache_dtype, kv_scale, self.scale, out=output[:n_pre])
             elif ops.prefill_attention_supported(query.dtype, self.head_size):
                 # HIP flash-style kernel over the packed prompt tokens; seq_start_loc is the
                 # cumulative prompt length table the reference's metadata carries
@@ -247,11 +247,11 @@ class Gfx950PagedAttentionImpl(AttentionImpl):
                 tp_rank=bsp.tp_rank, blocksparse_local_blocks=bsp.local_blocks,
                 blocksparse_vert_stride=bsp.vert_stride, blocksparse_block_size=bsp.block_size,
                 blocksparse_head_sliding_step=bsp.head_sliding_step)
-            output[n_pre:] = PagedAttention.forward_decode(
+            PagedAttention.forward_decode(
                 query[n_pre:], key_cache, value_cache, decode_meta.block_tables,
                 decode_meta.seq_lens_tensor, decode_meta.max_decode_seq_len, self.kv_cache_dtype,
                 self.num_kv_heads, self.scale, self._alibi(query.device), kv_scale,
-                seq_order=decode_meta.decode_seq_order, **sparse)
+                seq_order=decode_meta.decode_seq_order, out=output[n_pre:], **sparse)
         return output.view(num_tokens, hidden)
 
 

@@ -73,8 +73,10 @@ class PagedAttention:
                        blocksparse_local_blocks: int = 0, blocksparse_vert_stride: int = 0,
                        blocksparse_block_size: int = 64,
                        blocksparse_head_sliding_step: int = 0,
-                       seq_order: Optional[torch.Tensor] = None) -> torch.Tensor:
-        output = torch.empty_like(query)
+                       seq_order: Optional[torch.Tensor] = None,
+                       out: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """out: where the result goes, a part of the caller's tensor for instance."""
+        output = torch.empty_like(query) if out is None else out
         block_size = value_cache.shape[3]
         num_seqs, num_heads, head_size = query.shape
         if PagedAttention.use_v1(max_seq_len, num_seqs, num_heads, num_kv_heads):
@@ -106,12 +108,14 @@ class PagedAttention:
                        seq_lens_tensor: torch.Tensor, context_lens: torch.Tensor,
                        max_query_len: int, alibi_slopes: Optional[torch.Tensor],
                        sliding_window: Optional[int], kv_cache_dtype: str = "auto",
-                       kv_scale: float = 1.0, scale: Optional[float] = None) -> torch.Tensor:
+                       kv_scale: float = 1.0, scale: Optional[float] = None,
+                       out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Prompt attention over a cached prefix (vllm/attention/ops/paged_attn.py:185-216).
         The reference's kernel fixes the softmax scale at head_size ** -0.5
         (vllm/attention/ops/prefix_prefill.py:707) and reads a byte cache without its scale;
-        `scale`, `kv_cache_dtype` and `kv_scale` let the caller pass the layer's own values."""
-        output = torch.empty_like(query)
+        `scale`, `kv_cache_dtype` and `kv_scale` let the caller pass the layer's own values.
+        out: where the result goes, a part of the caller's tensor for instance."""
+        output = torch.empty_like(query) if out is None else out
         head_size = query.shape[-1]
         ops.prefix_prefill_attention(
             output, query, key, value, key_cache, value_cache, block_tables, query_start_loc,
