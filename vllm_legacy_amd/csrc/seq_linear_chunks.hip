@@ -14,14 +14,16 @@
 // logarithms over just those rows: nothing is divided and no sums are subtracted, so a decay of 0 beside decays of
 // 1 is exact, and decays near 1 keep the precision of their logarithms (multiplied row by row they left the
 // states after 4096 rows several times as far from 64 bits).
-// All products run on 16x16x4 fp32 matrix cores.  Operands that later kernels read lie in scratch lane for lane.
-// 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB of chunk states and decays: 97 us per call (31 + 23 + 52
+// Products run on 16x16x4 fp32 matrix cores, those with values of bfloat16 on its own (ThreeParts below).  Operands that
+// later kernels read lie in scratch lane for lane.
+// 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB of chunk states and decays: 83 us per call (22 + 23 + 45
 // under the tracer; pieces of 256 rows walked token by token and joined by matrix products took 408).  Four workgroups share a
 // CU, so that all 1024 of that step are there at once: 16-bit rows stay 16-bit in LDS (39 of 40 KB), a thread holds a channel's
 // logarithms of a block in registers, A lies where its queries lay and the values where the keys were (two workgroups per CU
-// and two rounds of them, with rows as 32-bit numbers beside a copy of the decays: 123 us, 42 + 23 + 66).  What bounds the
-// first and last kernel now are vector instructions (three fifths of their cycles; exponentials and logarithms most of them)
-// and products (three tenths); the scan is a copy of the states, 67 MB in 23 us.
+// and two rounds of them, with rows as 32-bit numbers beside a copy of the decays: 123 us, 42 + 23 + 66; with all products on
+// the fp32 instructions 97, 31 + 23 + 52).  What bounds the first and last kernel now are vector instructions (more than half
+// of their cycles; exponentials and logarithms most of them), in the last also the fp32 products with the start states (a
+// fourth); the scan is a copy of the states, 67 MB in 23 us.
 #include <atomic>
 #include <type_traits>
 
@@ -60,6 +62,7 @@ struct GlaChunks {
   const int* state_slots;
   int num_seqs, heads, dim, vdim, rank;
   float q_scale, inv_tau, eps, out_scale;
+  bool paired;                  // how tiles of columns lie in scratch: paired_column, or one after the other
 };
 
 // floats of a chunk and head: logarithms of the decays [64][dim] | G [dim] | R, then the start state [dim / 16][vdim / 16][lane][4]
@@ -159,8 +162,62 @@ struct TilePair {
     x = second ? y : x;
   }
 };
-__device__ __forceinline__ int tile_column(int tile, int tiles, int c) {
+__device__ __forceinline__ int paired_column(int tile, int tiles, int c) {
   return (tile | 1) < tiles ? 32 * (tile >> 1) + 2 * c + (tile & 1) : 16 * tile + c;
+}
+
+// Products with values of bfloat16 run on its matrix cores, 32 rows at a time: a 32-bit factor is three bfloat16 numbers whose
+// sum it is (8 of its 24 bits each), the value is one, every product is exact and sums are fp32 as those of the fp32
+// instructions, which take five times as long (eight of 32 cycles where these take three of 16) and hold up vector
+// instructions meanwhile.  Values come in by transposing reads: lane c has column c of a tile, rows 4 g .. 4 g + 3 of two
+// blocks of 16.
+template <class S>
+constexpr bool kSplit = std::is_same<S, BF16>::value;
+template <class S>
+__device__ __forceinline__ int tile_column(int tile, int tiles, int c) {
+  return kSplit<S> ? 16 * tile + c : paired_column(tile, tiles, c);
+}
+typedef short gla_s16x4 __attribute__((ext_vector_type(4)));
+typedef gla_s16x4 __attribute__((address_space(3))) * gla_lds_s16x4;
+struct ThreeParts {
+  u32x4 part[3];                                           // the largest first
+};
+__device__ __forceinline__ ThreeParts three_parts(f32x4 x, f32x4 y) {
+  float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]}, most = 0.f;
+  ThreeParts t;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      t.part[p][e] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, v[2 * e + 1]), __builtin_bit_cast(uint32_t, v[2 * e]), 0x07060302u);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if (p == 0) most = fmaxf(most, fabsf(v[e]));
+      v[e] -= __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[e]) & 0xffff0000u);
+    }
+  }
+  if (__any(most == INFINITY)) {                           // an infinity has no rest
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t w = t.part[0][e], keep = ((w & 0x7fffu) == 0x7f80u ? 0u : 0xffffu) | ((w & 0x7fff0000u) == 0x7f800000u ? 0u : 0xffff0000u);
+      t.part[1][e] &= keep;
+      t.part[2][e] &= keep;
+    }
+  }
+  return t;
+}
+// values of lane c's column, at `rows` (the lane's row of a block and its place in it) and 16 rows further on
+__device__ __forceinline__ u32x4 two_blocks(const void* rows, int pitch) {
+  const char* at = (const char*)rows;
+  const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((gla_lds_s16x4)(at)));
+  const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((gla_lds_s16x4)(at + 16 * pitch)));
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+__device__ __forceinline__ f32x4 mfma_parts(const ThreeParts& a, u32x4 b, f32x4 c) {
+#pragma unroll
+  for (int p = 2; p >= 0; --p)
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a.part[p]), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  return c;
 }
 
 template <class S, int DT>          // DT: dim / 16
@@ -290,6 +347,20 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
     float kj[kBlock];
 #pragma unroll
     for (int x = 0; x < kBlock; ++x) kj[x] = k_lds[(kBlock * (x >> 2) + 4 * g + (x & 3)) * KR + ch] * m[x >> 2];
+    if constexpr (kSplit<S>) {
+      ThreeParts kp[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+        kp[x] = three_parts(f32x4{kj[8 * x], kj[8 * x + 1], kj[8 * x + 2], kj[8 * x + 3]}, f32x4{kj[8 * x + 4], kj[8 * x + 5], kj[8 * x + 6], kj[8 * x + 7]});
+      const T* at = v_lds + (4 * g + (c >> 2)) * VR + 4 * (c & 3);
+      for (int vt = w % SHARE; vt < vt_n; vt += SHARE) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int x = 0; x < 2; ++x) acc = mfma_parts(kp[x], two_blocks(at + 32 * x * VR + 16 * vt, 2 * VR), acc);
+        *reinterpret_cast<f32x4*>(r_out + ((int64_t)(dt * vt_n + vt) * 64 + lane) * 4) = acc;
+      }
+      continue;
+    }
     for (int pair = w % SHARE; pair < pairs; pair += SHARE) {
       const TilePair tp(pair, vt_n, c);
       f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = acc;
@@ -316,7 +387,7 @@ __global__ __launch_bounds__(256) void gla_chunk_scan_kernel(GlaChunks a) {
   const int begin = a.query_start_loc[b], run = a.query_start_loc[b + 1] - begin;
   if (run <= 0) return;
   const int tile = item >> 7, lane = (item >> 1) & 63, g = lane >> 4, c = lane & 15;
-  const int d = 16 * (tile / vt_n) + 4 * g + 2 * (item & 1), v = tile_column(tile % vt_n, vt_n, c);
+  const int d = 16 * (tile / vt_n) + 4 * g + 2 * (item & 1), v = a.paired ? paired_column(tile % vt_n, vt_n, c) : 16 * (tile % vt_n) + c;
   float* st = a.state + (((int64_t)a.state_slots[b] * a.heads + h) * D + d) * V + v;
   f32x2 s = {0.f, 0.f};
   if (a.context_lens[b] > 0) s = f32x2{st[0], st[V]};
@@ -544,6 +615,61 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
 
   f32x4 acc[8];
   float ss[4] = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (kSplit<S>) {
+    // the wave's rows of A over one or two pairs of blocks; zeros behind its own block, which the values there meet
+    const bool two = w >= 2;
+    ThreeParts ap[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      const f32x4 a0 = *reinterpret_cast<const f32x4*>(a_own + c * kAMat + 32 * x + 4 * g), a1 = *reinterpret_cast<const f32x4*>(a_own + c * kAMat + 32 * x + 16 + 4 * g);
+      if (x == 0 || two) ap[x] = three_parts(2 * x <= w ? a0 : zero, 2 * x + 1 <= w ? a1 : zero);
+    }
+    const T* at = v_lds + (4 * g + (c >> 2)) * VR + 4 * (c & 3);
+    // (behind all of these where registers are for four workgroups a CU; for two, tile by tile)
+    auto with_state = [&](int vt) __attribute__((always_inline)) {
+      if (vt + 1 < vt_n) fetch_state(vt + 1);
+#pragma unroll
+      for (int x = 0; x < DT; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[vt] = mfma4(qs[x][e], sv[vt & 1][x][e], acc[vt]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss[e] += acc[vt][e] * acc[vt][e];
+    };
+#pragma unroll
+    for (int vt = 0; vt < 8; ++vt) {
+      acc[vt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (vt < vt_n) {
+        u32x4 v0 = two_blocks(at + 16 * vt, 2 * VR), v1 = v0;
+        if (two) v1 = two_blocks(at + 32 * VR + 16 * vt, 2 * VR);
+        // A row's product with the rows behind it is 0 times their values, which must be finite for that; and a column
+        // in which one was not stays so, as it does in the state of a walk.
+        int bad = kBlock;                                  // the block's first such row in the lane's column
+        if (some_bad) {
+          for (int i = kBlock * (w + 1) - 1; i >= 0; --i)
+            if (!finite(S::to_f32(v_lds[i * VR + 16 * vt + c]))) bad = max(i - kBlock * w, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            auto keep = [](uint32_t x) { return ((x & 0x7f80u) == 0x7f80u ? 0u : 0xffffu) | ((x & 0x7f800000u) == 0x7f800000u ? 0u : 0xffff0000u); };
+            v0[e] &= keep(v0[e]);
+            v1[e] &= keep(v1[e]);
+          }
+        }
+        acc[vt] = mfma_parts(ap[0], v0, acc[vt]);
+        if (two) acc[vt] = mfma_parts(ap[1], v1, acc[vt]);
+        if (some_bad) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[vt][e] = 4 * g + e < bad ? acc[vt][e] : NAN;
+        }
+        if constexpr (DT > 4) with_state(vt);
+      }
+    }
+    if constexpr (DT <= 4) {
+#pragma unroll
+      for (int vt = 0; vt < 8; ++vt)
+        if (vt < vt_n) with_state(vt);
+    }
+  } else {
 #pragma unroll
   for (int pair = 0; pair < 4; ++pair) {
     acc[2 * pair] = acc[2 * pair + 1] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -611,6 +737,7 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
       }
     }
   }
+  }
   group_sums(ss[0], ss[1], 16);
   group_sums(ss[2], ss[3], 16);
   // lane: its columns of rows 16 w + 4 g .. + 3
@@ -628,7 +755,7 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
         for (int vt = 4 * half; vt < 4 * half + 4; ++vt)
           if (vt < vt_n)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) own[(4 * g + e) * kAMat + tile_column(vt, vt_n, c) - 64 * half] = acc[vt][e] * inv[e] * norm[tile_column(vt, vt_n, c)];
+            for (int e = 0; e < 4; ++e) own[(4 * g + e) * kAMat + tile_column<S>(vt, vt_n, c) - 64 * half] = acc[vt][e] * inv[e] * norm[tile_column<S>(vt, vt_n, c)];
         wave_sync();
 #pragma unroll
         for (int r8 = 0; r8 < 2; ++r8) {
@@ -664,10 +791,10 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
     float gt[8];
 #pragma unroll
     for (int vt = 0; vt < 8; ++vt)
-      if (vt < vt_n) gt[vt] = S::to_f32(gr[tile_column(vt, vt_n, c)]);
+      if (vt < vt_n) gt[vt] = S::to_f32(gr[tile_column<S>(vt, vt_n, c)]);
 #pragma unroll
     for (int vt = 0; vt < 8; ++vt)
-      if (vt < vt_n) to[tile_column(vt, vt_n, c)] = S::from_f32(acc[vt][e] * inv[e] * norm[tile_column(vt, vt_n, c)] * (gt[vt] / (1.f + expf(-gt[vt]))));
+      if (vt < vt_n) to[tile_column<S>(vt, vt_n, c)] = S::from_f32(acc[vt][e] * inv[e] * norm[tile_column<S>(vt, vt_n, c)] * (gt[vt] / (1.f + expf(-gt[vt]))));
   }
 }
 
@@ -745,7 +872,7 @@ extern "C" int vla_seq_gla_chunks(void* out, int64_t out_stride, const void* q, 
   if (q_stride % 4 || k_stride % 4 || v_stride % 4) return VLA_ERR_ARG;
   const GlaChunks a{out, out_stride, q, q_stride, k, k_stride, v, v_stride, gate, gate_stride, y, y_stride, w2, bias,
                     norm_weight, state, scratch, query_start_loc, context_lens, state_slots, num_seqs, heads, dim, vdim,
-                    rank, q_scale, inv_tau, eps, out_scale};
+                    rank, q_scale, inv_tau, eps, out_scale, dtype != VLA_BF16};
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)chunk_slots(num_tokens, num_seqs), heads);
   return with_dtype(dtype, [&](auto s) -> int {
