@@ -223,6 +223,14 @@ def test_up_projection(lens, rank, vdim, heads, dtype):
     assert float((up.to(F) - near).abs().max()) <= bound * float(near.abs().max()) + 1e-5
 
 
+@pytest.mark.parametrize("rank,vdim,heads", [(512, 128, 16), (256, 64, 17)])
+@pytest.mark.parametrize("lens", [[400] * 137, [9000] + [1 + 29 * i % 411 for i in range(128)]], ids=["even", "uneven"])
+def test_up_projection_of_many_sequences(lens, rank, vdim, heads):
+    """Sixteen sequences to a workgroup, where eight would be more workgroups than CUs: two to five parts of each, and seventy of one."""
+    assert (len(lens) + 7) // 8 * heads > 256
+    test_up_projection(lens, rank, vdim, heads, torch.bfloat16)
+
+
 @pytest.mark.parametrize("window,sinks", [(0, True), (100, False), (70, True)])
 @pytest.mark.parametrize("lens", [[33, 190, 64, 5], [3000, 33, 700, 64, 5]], ids=["whole", "shared"])
 def test_up_projection_with_windows_sinks_and_sequences_without_a_row(lens, window, sinks):

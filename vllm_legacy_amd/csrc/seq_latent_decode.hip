@@ -393,35 +393,45 @@ __device__ __forceinline__ void place_of(const LatentDecode& a, int b, int& star
 
 // sum_s o_s[d] 2^(m_s - M) over the ranges s = i0 .. i1, M the largest m_s, of four sums from d + 256 j on each; the
 // result is sum_s l_s 2^(m_s - M)
-template <int NJ>
+// EARLY: the first eight parts are asked for with their maxima, where there are registers for that.
+template <int NJ, bool EARLY>
 __device__ __forceinline__ float merge_parts(const LatentDecode& a, int h, int i0, int i1, int d, f32x4 (&num)[NJ]) {
   const int lane = threadIdx.x & 63, row_floats = a.rank + 4;
   auto part = [&](int s) {
     const int slot = s == i0 ? 2 * s + 1 : 2 * s;        // its first part is the last of that range
     return a.parts + ((int64_t)slot * a.heads + h) * row_floats;
   };
-  float big = -INFINITY;
-  for (int s = i0 + lane; s <= i1; s += 64) big = fmaxf(big, part(s)[a.rank]);
+  constexpr int AHEAD = EARLY ? 8 : 4;                   // (where workgroups are many, sequences have few parts)
+  f32x4 v[AHEAD][NJ];
+  auto fetch = [&](int s0, int n, int s8) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) v[s][j] = *reinterpret_cast<const f32x4*>(part(s0 + min(s8 + s, n - 1)) + d + 256 * j);
+  };
+  float ms = 0.f, ls = 0.f, big = -INFINITY;
+  if (EARLY) {
+    const int at = min(i0 + lane, i1);
+    ms = part(at)[a.rank];
+    ls = part(at)[a.rank + 1];
+    fetch(i0, min(64, i1 - i0 + 1), 0);
+    big = i0 + lane <= i1 ? ms : -INFINITY;
+  }
+  for (int s = i0 + (EARLY ? 64 : 0) + lane; s <= i1; s += 64) big = fmaxf(big, part(s)[a.rank]);
   big = wave_max(big);
   float den = 0.f;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) num[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int s0 = i0; s0 <= i1; s0 += 64) {
-    float f = 0.f, lf = 0.f;
-    if (s0 + lane <= i1) {
-      const float ms = part(s0 + lane)[a.rank];
-      f = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - big);
-      lf = part(s0 + lane)[a.rank + 1] * f;
-    }
-    den += wave_sum(lf);
     const int n = min(64, i1 - s0 + 1);
-    constexpr int AHEAD = 8;
-    for (int s8 = 0; s8 < n; s8 += AHEAD) {              // eight parts on their way
-      f32x4 v[AHEAD][NJ];
-#pragma unroll
-      for (int s = 0; s < AHEAD; ++s)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) v[s][j] = *reinterpret_cast<const f32x4*>(part(s0 + min(s8 + s, n - 1)) + d + 256 * j);
+    if (!EARLY || s0 > i0) {
+      ms = part(min(s0 + lane, i1))[a.rank];
+      ls = part(min(s0 + lane, i1))[a.rank + 1];
+    }
+    const float f = lane >= n || ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - big);
+    den += wave_sum(lane < n ? ls * f : 0.f);
+    for (int s8 = 0; s8 < n; s8 += AHEAD) {              // several parts on their way
+      if (!EARLY || s8 > 0 || s0 > i0) fetch(s0, n, s8);
 #pragma unroll
       for (int s = 0; s < AHEAD; ++s) {
         const float fs = s8 + s < n ? __shfl(f, s8 + s, 64) : 0.f;
@@ -451,17 +461,17 @@ __global__ __launch_bounds__(128) void latent_decode_merge_kernel(LatentDecode a
   if (units == 0 || i0 == i1 || h >= a.heads) return;
   const int64_t t = a.query_start_loc[b];
   f32x4 num[1];
-  const float den = merge_parts<1>(a, h, i0, i1, d, num);
+  const float den = merge_parts<1, true>(a, h, i0, i1, d, num);
   const float gv = gate_of<S>(a, t, h);
   const u32x2 packed = {pack16<S>(num[0][0] / den * gv, num[0][1] / den * gv), pack16<S>(num[0][2] / den * gv, num[0][3] / den * gv)};
   *reinterpret_cast<u32x2*>((T*)a.out + t * a.out_token_stride + h * a.out_head_stride + d) = packed;
 }
 
 // The merge and the heads' up-projection in one: up[t, h vdim + n] = sum_d o[t, h, d] w[h, d, n], o rounded to 16 bits as
-// the merge leaves it.  A workgroup is 16 sequences and a head: a wave merges a row (or reads one that is written out
+// the merge leaves it.  A workgroup is 8 or 16 sequences and a head: a wave merges a row (or reads one that is written out
 // already) into LDS, then takes 32 columns and a part of the latent dims.  The weights' rows run along n, where the
 // matrix cores want them along d: a lane loads two columns of eight rows and puts the words together itself.  64
-// sequences of 1 .. 4001 keys, 16 heads, rank 512, vdim 128: 12 us, where the merge, a batched library product and
+// sequences of 1 .. 4001 keys, 16 heads, rank 512, vdim 128: 10 us, where the merge, a batched library product and
 // the copy that puts a token's heads side by side took 6, 10 and 4.
 struct LatentUp {
   void* up;
@@ -469,15 +479,15 @@ struct LatentUp {
   const void* w;                       // [heads, rank, vdim]
   int vdim;
 };
-template <class S, int NJ>             // rank = 256 NJ
-__global__ __launch_bounds__(1024) void latent_decode_up_kernel(LatentDecode a, LatentUp u) {
+template <class S, int NJ, int ROWS>   // rank = 256 NJ
+__global__ __launch_bounds__(64 * ROWS) void latent_decode_up_kernel(LatentDecode a, LatentUp u) {
   using T = typename S::T;
   constexpr int C = 256 * NJ, PITCH = C + 8;
-  __shared__ __align__(16) T o_lds[16 * PITCH];
-  __shared__ float part[16][16][34];
+  __shared__ __align__(16) T o_lds[ROWS * PITCH];
+  __shared__ float part[ROWS][ROWS][34];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
-  const int b0 = 16 * blockIdx.x, h = blockIdx.y;
-  const int blocks = u.vdim / 32, split = min(16 / blocks, C / 32), nb = w % blocks, ks0 = min(w / blocks, split - 1) * (C / 32 / split);
+  const int b0 = ROWS * blockIdx.x, h = blockIdx.y;
+  const int blocks = u.vdim / 32, split = min(ROWS / blocks, C / 32), nb = w % blocks, ks0 = min(w / blocks, split - 1) * (C / 32 / split);
   const uint32_t* wr = reinterpret_cast<const uint32_t*>((const T*)u.w + ((int64_t)h * C + 32 * ks0 + 8 * g) * u.vdim + 32 * nb + 2 * c);
   constexpr int AHEAD = 4;                               // steps whose weights are on their way during the merge
   const int steps = C / 32 / split;
@@ -499,7 +509,7 @@ __global__ __launch_bounds__(1024) void latent_decode_up_kernel(LatentDecode a, 
       const int units = units_of(a, b), i0 = start / share, i1 = (start + units - 1) / share;
       if (parts && i0 != i1) {
         f32x4 num[NJ];
-        const float den = merge_parts<NJ>(a, h, i0, i1, 4 * lane, num);
+        const float den = merge_parts<NJ, ROWS == 8>(a, h, i0, i1, 4 * lane, num);
         const float gv = gate_of<S>(a, t, h);
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
@@ -519,7 +529,7 @@ __global__ __launch_bounds__(1024) void latent_decode_up_kernel(LatentDecode a, 
 #pragma unroll
     for (int ks = 0; ks < AHEAD; ++ks) {
       if (k8 + ks >= steps) break;
-      const u32x4 ov = *reinterpret_cast<const u32x4*>(o_lds + c * PITCH + 32 * (ks0 + k8 + ks) + 8 * g);
+      const u32x4 ov = *reinterpret_cast<const u32x4*>(o_lds + c % ROWS * PITCH + 32 * (ks0 + k8 + ks) + 8 * g);
       u32x4 lo, hi;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -537,9 +547,10 @@ __global__ __launch_bounds__(1024) void latent_decode_up_kernel(LatentDecode a, 
     }
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) part[w][4 * g + i][2 * c] = even[i], part[w][4 * g + i][2 * c + 1] = odd[i];
+  for (int i = 0; i < 4; ++i)
+    if (4 * g + i < ROWS) part[w][4 * g + i][2 * c] = even[i], part[w][4 * g + i][2 * c + 1] = odd[i];
   __syncthreads();
-  for (int i = tid; i < 16 * u.vdim / 2; i += 1024) {
+  for (int i = tid; i < ROWS * u.vdim / 2; i += 64 * ROWS) {
     const int row = i / (u.vdim / 2), n = 2 * (i % (u.vdim / 2)), b = b0 + row;
     if (b >= a.num_seqs || a.query_start_loc[b + 1] <= a.query_start_loc[b]) continue;
     float v0 = 0.f, v1 = 0.f;
@@ -566,7 +577,13 @@ int launch_latent_decode(const LatentDecode& a, const LatentUp* up, hipStream_t 
   latent_decode_kernel<S, LB, RB, HS><<<dim3(a.ranges, head_groups(a.heads)), 128 * HS, lds, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   if (up != nullptr) {
-    latent_decode_up_kernel<S, LB / 4><<<dim3((a.num_seqs + 15) / 16, a.heads), 1024, 0, stream>>>(a, *up);
+    // Eight sequences to a workgroup while that leaves one for each CU at most: more of them, and registers for the first parts
+    // ahead of their maxima (16 heads: 64 of 1 .. 4001 keys 9.8 us instead of 11.9, of 4000 10.4 and 13.4, one of 4000 10.7 and
+    // 11.7); sixteen beyond, where weights would be read twice as often (256 of 1000 11.9, with eight 17.1; 1024 of 100 19 and 31).
+    if ((int64_t)((a.num_seqs + 7) / 8) * a.heads <= 256)
+      latent_decode_up_kernel<S, LB / 4, 8><<<dim3((a.num_seqs + 7) / 8, a.heads), 512, 0, stream>>>(a, *up);
+    else
+      latent_decode_up_kernel<S, LB / 4, 16><<<dim3((a.num_seqs + 15) / 16, a.heads), 1024, 0, stream>>>(a, *up);
     VLA_SEQ_HIP_CHECK(hipGetLastError());
   } else if (!a.by_sequence && a.ranges > 1) {
     const int heads_per = 128 / (a.rank / 4);
