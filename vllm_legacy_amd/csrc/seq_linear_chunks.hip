@@ -422,10 +422,10 @@ __global__ __launch_bounds__(256) void gla_chunk_scan_kernel(GlaChunks a) {
 
 // r *= d in the wave's first n lanes, of which all run: four instructions fewer than a choice of the factor
 __device__ __forceinline__ void times_in_lanes_below(int n, f32x4& r, f32x4 d) {
-  asm("s_bfm_b64 exec, %8, 0\n\tv_mul_f32 %0, %0, %4\n\tv_mul_f32 %1, %1, %5\n\tv_mul_f32 %2, %2, %6\n\t"
-      "v_mul_f32 %3, %3, %7\n\ts_mov_b64 exec, -1"
-      : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3])
-      : "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "s"(n));
+  asm volatile("s_bfm_b64 exec, %8, 0\n\tv_mul_f32 %0, %0, %4\n\tv_mul_f32 %1, %1, %5\n\tv_mul_f32 %2, %2, %6\n\t"
+               "v_mul_f32 %3, %3, %7\n\ts_mov_b64 exec, -1"
+               : "+&v"(r[0]), "+&v"(r[1]), "+&v"(r[2]), "+&v"(r[3])
+               : "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "s"(n));
 }
 
 template <class S, int DT>          // DT: dim / 16
