@@ -161,6 +161,43 @@ def test_rows_ahead_of_one_that_is_not_finite(what, value, row, dtype):
     assert torch.equal(state[0].isfinite(), S.isfinite())
 
 
+@pytest.mark.parametrize("row", [0, 15, 16, 63, 64, 100, 129])
+@pytest.mark.parametrize("D,V", [(16, 16), (32, 48), (64, 128), (128, 112)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_states_of_infinite_values(dtype, D, V, row):
+    """A state that a walk in float64 leaves infinite is so, with its sign, not NaN; keys of 0 and values of both signs are
+    NaN there and here; the other columns are, bit for bit, what they are without such values."""
+    from vllm_legacy_amd.attention.batch import SequenceBatch
+    from vllm_legacy_amd.attention.recurrent import GatedLinearRecurrence
+    H, rank, n, g = 2, 3, 130, torch.Generator().manual_seed(row + D)
+    layer = GatedLinearRecurrence(H, D, V, 5.0, 1e-5)
+    layer.CHUNK_ALONE_ROWS = 0
+    q, k, v, gate, y, w2 = (torch.randn(*shape, generator=g).to(dtype) for shape in [(n, H * D)] * 2 + [(n, H * V)] * 2 + [
+        (n, rank), (H * D, rank)])
+    bias = torch.randn(H * D, generator=g) + 2
+    k[row, 2] = 0.0
+    b = SequenceBatch.build([n], [0], [[0] * 64], [0], 16, DEV)
+
+    def go(v):
+        state = torch.zeros(1, H, D, V, device=DEV)
+        layer(torch.empty(n, H * V, device=DEV, dtype=dtype), q.to(DEV), k.to(DEV), v.to(DEV), gate.to(DEV), y.to(DEV), w2.to(DEV),
+              bias.to(DEV), torch.ones(V, device=DEV), state, b)
+        return state[0].cpu().double()
+
+    clean = go(v)
+    v[row, 1], v[row, 5], v[row, 7] = float("inf"), float("-inf"), float("nan")
+    v[row, 9], v[(row + 70) % n, 9] = float("inf"), float("-inf")
+    got = go(v)
+    a = torch.exp(R.log_decay(y.to(R.F), w2.to(R.F), bias.to(R.F), 5.0)).view(-1, H, D)
+    S = torch.zeros(H, D, V, dtype=R.F)
+    for t in range(n):
+        S = a[t][:, :, None] * S + k[t].to(R.F).view(H, D, 1) * v[t].to(R.F).view(H, 1, V)
+    assert int(S.isinf().sum()) > 2 * (D - 1) and int(S.isnan().sum()) > D
+    assert torch.equal(got.isnan(), S.isnan())
+    assert torch.equal(got[S.isinf()], S[S.isinf()])
+    assert torch.equal(got[S.isfinite()], clean[S.isfinite()])
+
+
 @pytest.mark.parametrize("H,lens,chunks", [(2, [99], False), (2, [100], True), (2, [100] + [1] * 6, False), (70, [64, 35], False),
                                            (70, [64, 36], True), (70, [63, 63], False)])
 def test_steps_that_go_in_chunks(H, lens, chunks, monkeypatch):

@@ -100,10 +100,6 @@ __device__ __forceinline__ f32x4 numbers(Four<S> x) {
   else
     return x;
 }
-template <class S>
-__device__ __forceinline__ f32x4 row4(const typename S::T* p) {
-  return numbers<S>(fetch4<S>(p));
-}
 
 // exp(p) for p <= 0 (NaN passes): 2^n 2^f with the argument's rounding in f.  expf without what other p need, the same
 // error: 2.62e-8 root mean square over -87 .. 0, 8.4e-8 at most.
@@ -169,14 +165,16 @@ __device__ __forceinline__ int paired_column(int tile, int tiles, int c) {
 // Products with values of bfloat16 run on its matrix cores, 32 rows at a time: a 32-bit factor is three bfloat16 numbers whose
 // sum it is (8 of its 24 bits each), the value is one, every product is exact and sums are fp32 as those of the fp32
 // instructions, which take five times as long (eight of 32 cycles where these take three of 16) and hold up vector
-// instructions meanwhile.  Values come in by transposing reads: lane c has column c of a tile, rows 4 g .. 4 g + 3 of two
-// blocks of 16.
+// instructions meanwhile.  An infinite value meets a factor's first part only: the others are often 0, and 0 times it is not
+// a number where the factor times it is infinite.  Values come in by transposing reads: lane c has column c of a tile, rows
+// 4 g .. 4 g + 3 of two blocks of 16.
 template <class S>
 constexpr bool kSplit = std::is_same<S, BF16>::value;
 template <class S>
 __device__ __forceinline__ int tile_column(int tile, int tiles, int c) {
   return kSplit<S> ? 16 * tile + c : paired_column(tile, tiles, c);
 }
+typedef unsigned short gla_u16x2 __attribute__((ext_vector_type(2)));
 typedef short gla_s16x4 __attribute__((ext_vector_type(4)));
 typedef gla_s16x4 __attribute__((address_space(3))) * gla_lds_s16x4;
 struct ThreeParts {
@@ -213,10 +211,18 @@ __device__ __forceinline__ u32x4 two_blocks(const void* rows, int pitch) {
   const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((gla_lds_s16x4)(at + 16 * pitch)));
   return u32x4{lo[0], lo[1], hi[0], hi[1]};
 }
-__device__ __forceinline__ f32x4 mfma_parts(const ThreeParts& a, u32x4 b, f32x4 c) {
+// bfloat16 numbers, those that are not finite as 0
+__device__ __forceinline__ u32x4 finite_only(u32x4 v) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    v[e] &= ((v[e] & 0x7f80u) == 0x7f80u ? 0u : 0xffffu) | ((v[e] & 0x7f800000u) == 0x7f800000u ? 0u : 0xffff0000u);
+  return v;
+}
+// rest: what the second and third parts meet
+__device__ __forceinline__ f32x4 mfma_parts(const ThreeParts& a, u32x4 b, u32x4 rest, f32x4 c) {
 #pragma unroll
   for (int p = 2; p >= 0; --p)
-    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a.part[p]), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a.part[p]), __builtin_bit_cast(bf16x8, p ? rest : b), c, 0, 0, 0);
   return c;
 }
 
@@ -230,7 +236,8 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
   float* k_lds = lds;                       // [64][KR]
   float* tot = k_lds + kChunk * KR;         // [4][D]: a block's sum of logarithms
   float* y_lds = tot + 4 * D;               // [64][RP]
-  T* v_lds = (T*)(y_lds + kChunk * RP);     // [64][VR]
+  int* odd_lds = (int*)(y_lds + kChunk * RP);                // [4]: a wave has met a value that is not finite
+  T* v_lds = (T*)(odd_lds + 4);             // [64][VR]
   const int slot = blockIdx.x, h = blockIdx.y;
   int b, chunk;
   if (!find_chunk(a, slot, b, chunk)) return;
@@ -334,9 +341,20 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
       const int i = tid + 256 * u, r = (i * inverse) >> 16, at = 4 * (i - r * per_row);
       *reinterpret_cast<Four<S>*>(v_lds + r * VR + at) = r < n ? vs[u] : Four<S>{};
     }
+  if constexpr (kSplit<S>) {
+    gla_u16x2 most = {0, 0};
+#pragma unroll
+    for (int u = 0; u < kMost; ++u)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) most = __builtin_elementwise_max(most, __builtin_bit_cast(gla_u16x2, vs[u][e] & 0x7fff7fffu));
+    const bool odd = __any(max(most[0], most[1]) >= 0x7f80);
+    if (lane == 0) odd_lds[w] = odd;
+  }
   __syncthreads();
   float* r_out = mine + kChunk * D + D;
   const int vt_n = V / 16, pairs = (vt_n + 1) / 2;
+  bool some_odd = false;
+  if constexpr (kSplit<S>) some_odd = __builtin_amdgcn_readfirstlane(odd_lds[0] | odd_lds[1] | odd_lds[2] | odd_lds[3]);
   constexpr int SHARE = DT >= 4 ? 1 : 4 / DT;              // waves that share the keys' 16 channels
   for (int dt = w / SHARE; dt < DT; dt += 4 / SHARE) {
     // the decay over the blocks behind each
@@ -356,7 +374,12 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
       for (int vt = w % SHARE; vt < vt_n; vt += SHARE) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int x = 0; x < 2; ++x) acc = mfma_parts(kp[x], two_blocks(at + 32 * x * VR + 16 * vt, 2 * VR), acc);
+        for (int x = 0; x < 2; ++x) {
+          const u32x4 v = two_blocks(at + 32 * x * VR + 16 * vt, 2 * VR);
+          u32x4 rest = v;
+          if (some_odd) rest = finite_only(v);
+          acc = mfma_parts(kp[x], v, rest, acc);
+        }
         *reinterpret_cast<f32x4*>(r_out + ((int64_t)(dt * vt_n + vt) * 64 + lane) * 4) = acc;
       }
       continue;
@@ -648,15 +671,11 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
         if (some_bad) {
           for (int i = kBlock * (w + 1) - 1; i >= 0; --i)
             if (!finite(S::to_f32(v_lds[i * VR + 16 * vt + c]))) bad = max(i - kBlock * w, 0);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            auto keep = [](uint32_t x) { return ((x & 0x7f80u) == 0x7f80u ? 0u : 0xffffu) | ((x & 0x7f800000u) == 0x7f800000u ? 0u : 0xffff0000u); };
-            v0[e] &= keep(v0[e]);
-            v1[e] &= keep(v1[e]);
-          }
+          v0 = finite_only(v0);
+          v1 = finite_only(v1);
         }
-        acc[vt] = mfma_parts(ap[0], v0, acc[vt]);
-        if (two) acc[vt] = mfma_parts(ap[1], v1, acc[vt]);
+        acc[vt] = mfma_parts(ap[0], v0, v0, acc[vt]);
+        if (two) acc[vt] = mfma_parts(ap[1], v1, v1, acc[vt]);
         if (some_bad) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[vt][e] = 4 * g + e < bad ? acc[vt][e] : NAN;
@@ -818,7 +837,7 @@ int launch_chunks(const GlaChunks& a, dim3 grid, hipStream_t stream) {
   constexpr int D = 16 * DT;
   static std::atomic<size_t> allowed{64 * 1024}, allowed_out{64 * 1024};   // raised once per kernel, not per launch
   const size_t values = sizeof(typename S::T) * (size_t)kChunk * value_row<S>(a.vdim);
-  const size_t lds = sizeof(float) * ((size_t)kChunk * (D + 4 + (a.rank + 3) / 4 * 4) + 4 * D) + values;
+  const size_t lds = sizeof(float) * ((size_t)kChunk * (D + 4 + (a.rank + 3) / 4 * 4) + 4 * D + 4) + values;
   if (const int rc = raise_lds(&gla_chunk_state_kernel<S, DT>, lds, allowed)) return rc;
   gla_chunk_state_kernel<S, DT><<<grid, 256, lds, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
