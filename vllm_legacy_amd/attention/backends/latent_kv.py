@@ -112,9 +112,12 @@ class LatentKVAttention(nn.Module):
         keys."""
         return self._key_splits(batch.max_query_len, batch.num_seqs, batch.max_seq_len)
 
-    def _key_splits(self, max_query_len: int, num_seqs: int, keys: int) -> int:
+    def _row_tiles(self, max_query_len: int, num_seqs: int) -> int:
         heads_per = min(self.num_heads, 32)
-        tiles = -(-max_query_len // (32 // heads_per)) * -(-self.num_heads // heads_per) * num_seqs
+        return -(-max_query_len // (32 // heads_per)) * -(-self.num_heads // heads_per) * num_seqs
+
+    def _key_splits(self, max_query_len: int, num_seqs: int, keys: int) -> int:
+        tiles = self._row_tiles(max_query_len, num_seqs)
         if tiles >= self.SPLIT_BELOW_WORKGROUPS:
             return 1
         if self.window:
@@ -124,66 +127,76 @@ class LatentKVAttention(nn.Module):
     # the longest stretches of sequences a step is cut into; one that alternates more often stays whole
     MAX_STRETCHES = 4
 
-    # Multiply-adds of a step on the latent kernel (a fifth of a matrix product's rate) from which the other way, which
-    # gathers and forms keys first, is the faster one.  Rows x keys before them, 16 heads of 128 + 64, rank 512, latent / formed
-    # us on the GPU: one of 33 x 0 (1e7) 38 / 30, 64 x 0 (4e7) 40 / 30, 256 x 0 (6e8) 69 / 41, 400 x 0 89 / 45.  (Python and
-    # launches take the host 98 and 78 us.)  A step that goes both ways pays for both: so many times the work.
-    FORMED_MIN_WORK = 9e6
-    FORMED_MIXED_WORK = 700
-    # Rows of a run at least: forming a key's numbers costs as much for few rows as for many, and one tile of rows walks
-    # all keys by itself where the latent kernel shares them out.  One row more for so many keys ahead of them, no more than
-    # FORMED_MIN_ROWS, and that many in a step that goes both ways.  33 rows x 300 68 / 42, x 1000 70 / 61, x 2000 79 / 84, thirty
-    # of x 300 85 / 43 and x 1000 333 / 376; 48 x 1500 107 / 86, x 4000 113 / 138, thirty of x 2000 666 / 690; 64 x 1000
-    # 73 / 63, x 2000 77 / 91; 96 x 500 74 / 51, x 4000 158 / 138.
-    FORMED_FEW_ROWS = 32
-    FORMED_KEYS_PER_ROW = 64
+    # Multiply-adds of a step's long runs on the latent kernel from which those runs go formed whatever else is in the step.
+    FORMED_MIN_WORK = 6e9
+    # Their rows at least: forming a key's numbers costs as much for few rows as for many.
     FORMED_MIN_ROWS = 96
+    # A step below that with so much work, in which every run has so many rows, goes formed as a whole where that is clearly
+    # the faster way.
+    FORMED_LEAST_WORK = 9e6
+    FORMED_FEW_ROWS = 32
+    FORMED_CLEARLY = 1.2
 
-    def formed_min_rows(self, context: Optional[int] = None) -> int:
-        """Rows from which a run's keys and values are worth forming, behind `context` keys (None: any number).  A (query,
-        key) pair of a head costs the latent kernel 2 rank + rot multiply-adds at a fifth of a matrix product's rate (less
-        where the rank is small), the formed one dim + rot + vdim at about half of it; forming costs rank (dim + vdim) per
-        key at the full rate.  (A rank of 64 beside heads of 128 + 64: 1024 rows 98 / 140 us, 2048 167 / 141, 4096 535 / 186,
-        with three products of a library for the forming.)"""
-        least = self.FORMED_MIN_ROWS
-        if context is not None:
-            least = min(least, self.FORMED_FEW_ROWS + min(context, self.window or context) // self.FORMED_KEYS_PER_ROW)
-        return max(least, self.least_rows)
+    def formed_min_rows(self) -> int:
+        """Rows from which a run's keys and values are worth forming.  A (query, key) pair of a head costs the
+        latent kernel 2 rank + rot multiply-adds at a fifth of a matrix product's rate (less where the rank is small),
+        the formed one dim + rot + vdim at about half of it; forming costs rank (dim + vdim) per key at the full rate."""
+        return max(self.FORMED_MIN_ROWS, self.least_rows)
+
+    def formed_is_faster(self, lens, contexts) -> bool:
+        """Both ways' time on the GPU for sequences of `lens` rows behind `contexts` keys, in us, as measured over 1 to 128
+        heads of 32 to 128, ranks of 64 to 512, 1 to 30 sequences of 33 to 512 rows behind 0 to 8000 keys (859 steps;
+        rms errors of 14 and 9 %).  Latent: launches, a merge where keys are shared out, the products, and the longest
+        chain of key tiles in a row.  Formed: launches, the walk of the longest sequence's keys by one workgroup per
+        128 rows and head, forming, products and the gathered rows; one part of the workspace after the other.  With
+        the margin none of those steps is slower than on the latent kernel.  Latent / formed, 16 heads of 128 + 64, rank
+        512: 33 rows x 300 keys 67 / 40, x 1000 68 / 57, x 2000 77 / 80, thirty of x 300 127 / 112 and x 1000 334 / 350;
+        48 x 1500 73 / 71; 64 x 1000 69 / 59, x 2000 74 / 88; 96 x 500 72 / 48, x 2500 109 / 105; four of 48 x 2000
+        177 / 121.  Rank 64, 96 x 1500 48 / 63, 1024 x 0 90 / 55.  One or two heads, whose few workgroups the sums are
+        furthest off for, stay (one head, 128 x 1500 63 / 71, x 5000 66 / 152).  Of 439 steps of uneven lengths over these
+        ranges the three that were slower, by 3 to 17 %, were of such layers."""
+        H, D, R, V, C = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.rank
+        w = self.window
+        seen = [c + n if not w else min(c, w) + n for n, c in zip(lens, contexts)]
+        pairs = sum(n * (k - n) + (n * (n + 1) // 2 if not w else n * min(n, w)) for n, k in zip(lens, seen)) * H
+        if H <= 2 or pairs * (2 * C + R) < self.FORMED_LEAST_WORK:
+            return False
+        longest, total = max(seen), sum(seen)
+        tiles = self._row_tiles(max(lens), len(lens))
+        splits = self._key_splits(max(lens), len(lens), max(c + n for n, c in zip(lens, contexts)))
+        rounds, share = -(-tiles * splits // self.SPLIT_BELOW_WORKGROUPS), -(-longest // splits)
+        latent = 33 + 5 * (splits > 1) + 10e-9 * pairs * (2 * C + R) + rounds * share * (0.023 + 0.064 / 512 * C)
+        most, parts, walk = self.formed_keys(2), 1, longest
+        if total > most:
+            held = self._formed_parts(lens, contexts, most)
+            parts, walk = len(held), sum(count if b1 == b0 + 1 else max(seen[b0:b1]) for b0, b1, _, count, _ in held)
+        formed = 27 * parts + walk * (0.015 + 0.0057 / 128 * D) + 1.6e-9 * pairs * (2 * D + R + V) + \
+            total * (2.2e-9 * H * (D + V) * (C + 128) + 2.2e-6 * (C + R))
+        return self.FORMED_CLEARLY * formed < latent
 
     def _stretches(self, batch: SequenceBatch):
         """[[first sequence, one behind the last, first row, one behind the last, formed]]: neighbours that go
         the same way; None when the whole step takes the latent kernel."""
-        each = self.num_heads * (2 * self.rank + self.rot_dim)          # multiply-adds of a (query, key) pair
-        most = batch.num_tokens * batch.max_seq_len * each
-        if most < self.FORMED_MIN_WORK or batch.max_query_len < self.FORMED_FEW_ROWS:
-            return None                 # most steps: no more than this is asked of them
         q, ctx = batch.host_query_lens, batch.host_context_lens
-        if q is None or ctx is None:
-            return None
-        work, short = self.FORMED_MIN_WORK, min(q)
-        if short >= self.FORMED_FEW_ROWS and short >= self.least_rows and (
-                short >= self.formed_min_rows(max(ctx)) or all(n >= self.formed_min_rows(c) for n, c in zip(q, ctx))):
-            least = 0                   # all of them
-        else:
-            least, work = self.formed_min_rows(), work * self.FORMED_MIXED_WORK
-            if most < work:
-                return None
-        if not self.scale > 0 or not self.formed_fits or torch.cuda.is_current_stream_capturing():
+        if q is None or ctx is None or not self.scale > 0 or not self.formed_fits or torch.cuda.is_current_stream_capturing():
             return None                 # a captured step is replayed with other lengths than the host's
-        out, row = [], 0
-        pairs = 0
-        for b, (n, c) in enumerate(zip(q, ctx)):
-            formed = n >= least
-            if formed:
-                pairs += n * min(c, self.window or c) + (n * (n + 1) // 2 if not self.window else n * min(n, self.window))
-            if out and out[-1][4] == formed:
-                out[-1][1], out[-1][3] = b + 1, row + n
-            else:
-                out.append([b, b + 1, row, row + n, formed])
-            row += n
-        if pairs * each < work:
-            return None
-        return out if len(out) <= self.MAX_STRETCHES else None
+        each = self.num_heads * (2 * self.rank + self.rot_dim)          # multiply-adds of a (query, key) pair
+        least = self.formed_min_rows()
+        if batch.max_query_len >= least and batch.num_tokens * batch.max_seq_len * each >= self.FORMED_MIN_WORK:
+            out, row, pairs = [], 0, 0
+            for b, (n, c) in enumerate(zip(q, ctx)):
+                if n >= least:
+                    pairs += n * min(c, self.window or c) + (n * (n + 1) // 2 if not self.window else n * min(n, self.window))
+                if out and out[-1][4] == (n >= least):
+                    out[-1][1], out[-1][3] = b + 1, row + n
+                else:
+                    out.append([b, b + 1, row, row + n, n >= least])
+                row += n
+            if pairs * each >= self.FORMED_MIN_WORK:
+                return out if len(out) <= self.MAX_STRETCHES else None
+        if min(q) >= max(self.FORMED_FEW_ROWS, self.least_rows) and self.formed_is_faster(q, ctx):
+            return [[0, len(q), 0, batch.num_tokens, True]]
+        return None
 
     # bytes of gathered rows and formed keys and values at a time: 20 thousand keys of 16 heads of 128 + 128
     FORMED_WORKSPACE = 1 << 28
