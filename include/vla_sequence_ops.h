@@ -452,7 +452,9 @@ int vla_seq_gla_chunks(void* out, int64_t out_stride, const void* q, int64_t q_s
  * key_first > 0 (one sequence): from its visible row key_first on.
  * vla_seq_latent_form: keys [num_rows, heads * dim] and values [num_rows, heads * vdim] = the first `rank` numbers of rows
  * [num_rows, row_width] times w_uk [heads * dim, rank] transposed and w_uv [heads, rank, vdim], summed in fp32; keys_rest (as
- * keys): what rounding to 16 bits took from the keys.  rank: a multiple of 32.  All pointers 16-byte aligned.
+ * keys): what rounding to 16 bits took from the keys.  16-bit types, dim, vdim and row_width (at least rank) multiples of 8,
+ * rank one of 32, which vla_seq_latent_form_supported asks for; all pointers 16-byte aligned.  (vla_seq_latent_prompt takes
+ * keys and values however they were formed.)
  * vla_seq_latent_prompt: out [T, heads * vdim] from q [T, heads * (dim + rot)] (a head's row: plain | rotated),
  * the formed keys, keys_rest and values (scores are of keys and keys_rest together), and the
  * gathered rows themselves for the rotated parts behind them.
@@ -469,6 +471,7 @@ int vla_seq_latent_gather(void* rows, int num_rows, const void* cache, const int
                           int max_blocks, const int* query_start_loc, const int* context_lens, int num_seqs,
                           int max_seq_rows, int width, int block_size, int num_blocks, int window, int key_first,
                           int dtype, void* stream);
+int vla_seq_latent_form_supported(int dim, int vdim, int rank, int row_width, int dtype);
 int vla_seq_latent_form(void* keys, void* keys_rest, void* values, const void* rows, int num_rows, int row_width,
                         const void* w_uk, const void* w_uv, int heads, int dim, int vdim, int rank, int dtype,
                         void* stream);

@@ -122,3 +122,19 @@ def test_up_projections_at_odd_addresses_are_not_taken():
     assert ops.latent_decode_up_supported(flat[2:].view(2, 256, 64))
     assert not ops.latent_decode_up_supported(flat[1:-1].view(2, 256, 64))
     assert not ops.latent_decode_up_supported(flat[:-2].view(2, 64, 256).transpose(1, 2))
+
+
+@pytest.mark.parametrize("dim,vdim,rank,width", [(128, 128, 512, 576), (8, 8, 32, 32), (128, 64, 40, 48), (64, 64, 16, 32), (12, 64, 32, 32),
+                                                 (64, 68, 32, 64), (64, 64, 32, 36), (64, 64, 64, 32)])
+def test_what_forms_latent_keys(dim, vdim, rank, width):
+    """The query says no exactly where the forming entry refuses the sizes (ahead of any use of a pointer), also where the
+    prompts' kernel itself would take what another program has formed (rank 40, 16)."""
+    from vllm_legacy_amd import _lib
+    L = _lib.seq_lib()
+    fits = dim % 8 == 0 and vdim % 8 == 0 and rank % 32 == 0 and width % 8 == 0 and width >= rank
+    for dtype in (_lib.F16, _lib.BF16):
+        assert bool(L.vla_seq_latent_form_supported(dim, vdim, rank, width, dtype)) == fits
+    assert not L.vla_seq_latent_form_supported(dim, vdim, rank, width, _lib.F32)
+    if not fits:
+        assert L.vla_seq_latent_form(*[256] * 4, 1, width, 256, 256, 1, dim, vdim, rank, _lib.F16, None) != 0
+        assert (rank % 32 == 0) or L.vla_seq_latent_prompt_supported(dim, 0, vdim, rank, _lib.F16)

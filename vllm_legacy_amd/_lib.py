@@ -62,7 +62,7 @@ SEQ_EXPORTS = [
     "vla_seq_grouped_linear", "vla_seq_moe_combine", "vla_seq_kv_attention_tiles_supported",
     "vla_seq_kv_attention_tiles", "vla_seq_kv_attention_tiles_of", "vla_seq_kv_attention_tiles_form", "vla_seq_set_kv_attention_kernel", "vla_seq_set_grouped_linear_form",
     "vla_seq_post_norm", "vla_seq_rms_norm_rows", "vla_seq_short_conv", "vla_seq_gated_act_lookup",
-    "vla_seq_embed_scaled", "vla_seq_softcap", "vla_seq_kv_attention_shared", "vla_seq_kv_attention_scratch_floats", "vla_seq_grouped_linear_of", "vla_seq_grouped_glu", "vla_seq_grouped_glu_supported", "vla_seq_grouped_form", "vla_seq_gla_chunks", "vla_seq_gla_chunks_scratch_floats", "vla_seq_latent_gather", "vla_seq_latent_form", "vla_seq_latent_prompt", "vla_seq_latent_prompt_form", "vla_seq_latent_prompt_supported",
+    "vla_seq_embed_scaled", "vla_seq_softcap", "vla_seq_kv_attention_shared", "vla_seq_kv_attention_scratch_floats", "vla_seq_grouped_linear_of", "vla_seq_grouped_glu", "vla_seq_grouped_glu_supported", "vla_seq_grouped_form", "vla_seq_gla_chunks", "vla_seq_gla_chunks_scratch_floats", "vla_seq_latent_gather", "vla_seq_latent_form", "vla_seq_latent_form_supported", "vla_seq_latent_prompt", "vla_seq_latent_prompt_form", "vla_seq_latent_prompt_supported",
     "vla_seq_delta_rule_scan", "vla_seq_delta_rule_scan_blocks", "vla_seq_delta_rule_block_scratch_floats",
     "vla_seq_delta_rule_scratch_floats", "vla_seq_set_delta_kernel", "vla_seq_rglru_scan",
     "vla_seq_latent_rotary_write", "vla_seq_latent_rotary_write_form", "vla_seq_latent_attention", "vla_seq_latent_attention_tiles",
@@ -163,6 +163,7 @@ def seq_lib():
                                          i, i, i, f, f, f, f, p, i64, i, p]
         L.vla_seq_latent_prompt_supported.argtypes = [i, i, i, i, i]
         L.vla_seq_latent_gather.argtypes = [p, i, p, p, i, p, p, i, i, i, i, i, i, i, i, p]
+        L.vla_seq_latent_form_supported.argtypes = [i, i, i, i, i]
         L.vla_seq_latent_form.argtypes = [p, p, p, p, i, i, p, p, i, i, i, i, i, p]
         L.vla_seq_latent_prompt.argtypes = [p, i64, p, i64, p, p, p, p, i, p, p, i, i, i, i, i, i, i, f, i, p, i64, p, i, i, p, i, p]
         L.vla_seq_delta_rule_scan_blocks.argtypes = L.vla_seq_delta_rule_scan.argtypes[:-1] + [i64, p]

@@ -756,6 +756,11 @@ extern "C" int vla_seq_latent_gather(void* rows, int num_rows, const void* cache
   return VLA_OK;
 }
 
+extern "C" int vla_seq_latent_form_supported(int dim, int vdim, int rank, int row_width, int dtype) {
+  return (dtype == VLA_F16 || dtype == VLA_BF16) && dim > 0 && dim % 8 == 0 && vdim > 0 && vdim % 8 == 0 && rank > 0 &&
+         rank % kFormStep == 0 && row_width >= rank && row_width % 8 == 0;
+}
+
 extern "C" int vla_seq_latent_form(void* keys, void* keys_rest, void* values, const void* rows, int num_rows, int row_width,
                                   const void* w_uk, const void* w_uv, int heads, int dim, int vdim, int rank, int dtype,
                                   void* stream) {
@@ -764,7 +769,7 @@ extern "C" int vla_seq_latent_form(void* keys, void* keys_rest, void* values, co
       rank <= 0 || row_width < rank || (int64_t)heads * dim > 0x3fffffff || (int64_t)heads * vdim > 0x3fffffff)
     return VLA_ERR_ARG;
   if (dtype != VLA_F16 && dtype != VLA_BF16) return VLA_ERR_DTYPE;
-  if (dim % 8 || vdim % 8 || rank % kFormStep || row_width % 8) return VLA_ERR_HEAD_SIZE;
+  if (!vla_seq_latent_form_supported(dim, vdim, rank, row_width, dtype)) return VLA_ERR_HEAD_SIZE;
   for (const void* p : {(const void*)keys, (const void*)keys_rest, (const void*)values, rows, w_uk, w_uv})
     if ((uintptr_t)p % 16) return VLA_ERR_ARG;
   LatentForm a;
