@@ -127,6 +127,52 @@ def test_copy_blocks_many_layers(ops):
     ops.copy_blocks([], [], torch.zeros((0, 2), dtype=torch.int64, device="cuda"))  # no-op
 
 
+@pytest.mark.parametrize("device", ["cuda", "cuda:0", torch.device("cuda"), torch.device("cuda", 0), 0])
+def test_caches_that_name_their_device_their_own_way(ops, device):
+    """A cache object that is not a tensor: its device without an index, as text or as a number."""
+
+    class Cache:
+        is_cuda = True
+
+        def __init__(self, t):
+            self.t, self.device = t, device
+
+        def __getitem__(self, i):
+            return self.t[i]
+
+        def data_ptr(self):
+            return self.t.data_ptr()
+
+        def element_size(self):
+            return self.t.element_size()
+
+    k, v = (torch.randn(6, 2, 16, 16, device="cuda") for _ in range(2))
+    want = [t.clone() for t in (k, v)]
+    for t in want:
+        t[4] = t[1]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ops.copy_blocks([Cache(k)], [Cache(v)], torch.tensor([[1, 4]], device="cuda"))
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(k, want[0]) and torch.equal(v, want[1])
+
+
+@pytest.mark.parametrize("missing", [False, True])
+def test_stream_handles(missing, monkeypatch):
+    """The current stream's, whatever the form of the device and whether or not torch has its short way."""
+    from vllm_legacy_amd import _device
+    if missing:
+        monkeypatch.setattr(_device, "_raw_stream", None)
+    side = torch.cuda.Stream()
+    for stream in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(stream):
+            for device in ("cuda", torch.device("cuda"), torch.device("cuda", 0), 0, None):
+                assert _device.stream_handle(device) == stream.cuda_stream
+    with pytest.raises(Exception):
+        _device.stream_handle(torch.device("cpu"))
+
+
 @pytest.mark.parametrize("direction", [("cuda", "cpu"), ("cuda", "cuda"), ("cpu", "cuda")])
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("kv_fp8", [False, True])

@@ -16,6 +16,7 @@ from typing import List, Optional
 import torch
 
 from . import _lib
+from ._device import stream_handle as _stream
 from ._lib import check
 
 _DTYPE = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
@@ -26,10 +27,6 @@ def _dt(t: torch.Tensor) -> int:
         return _DTYPE[t.dtype]
     except KeyError:
         raise RuntimeError(f"Unsupported input type of kv cache: {t.dtype}") from None
-
-
-def _stream(device) -> int:
-    return torch._C._cuda_getCurrentRawStream(device.index)     # (0.2 us; by way of a Stream object 3)
 
 
 def _ptr(t) -> Optional[int]:
