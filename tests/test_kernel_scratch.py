@@ -38,11 +38,16 @@ def kernels_of_object(elf):
     return {}
 
 
-@pytest.mark.parametrize("kernel,instances", [("latent_prompt_kernel", 24), ("latent_form_kernel", 2), ("kv_attention_tile_kernel", 64)])
+@pytest.mark.parametrize("kernel,instances", [
+    ("latent_prompt_kernel", 24), ("latent_form_kernel", 2), ("kv_attention_tile_kernel", 64), ("gla_chunk_state_kernel", 12),
+    ("gla_chunk_out_kernel", 12), ("delta_block_prepare_kernel", 4), ("delta_block_walk_kernel", 4), ("latent_decode_up_kernel", 8),
+    ("16moe_route_kernel", 6), ("q4_gemm_dma2_kernelILi0ELb0ELi3ELi2ELb1E", 1), ("q4_gemm_dma2_kernelILi1ELb0ELi3ELi2ELb1E", 1)])
 def test_nothing_is_kept_in_memory(kernel, instances):
+    """(The int4 products: those whose last tiles are cut into slices.)"""
     from vllm_legacy_amd import _lib
-    if not os.path.exists(_lib.SEQ_LIB_PATH):
+    path = _lib.LIB_PATH if kernel.startswith("q4") else _lib.SEQ_LIB_PATH
+    if not os.path.exists(path):
         pytest.skip("not built")
-    kept = {k: v for k, v in kernels_of(_lib.SEQ_LIB_PATH).items() if kernel in k}
+    kept = {k: v for k, v in kernels_of(path).items() if kernel in k}
     assert len(kept) == instances, sorted(kept)
     assert not any(kept.values()), {k: v for k, v in kept.items() if v}
