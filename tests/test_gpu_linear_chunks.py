@@ -67,6 +67,14 @@ def test_results_eight_columns_at_a_time(shape, lens, ctx, dtype):
     run(*shape, lens, ctx, dtype)
 
 
+@pytest.mark.parametrize("lens,ctx", [([128, 129], [1, 0]), ([320, 321], [0, 2]), ([512, 513], [0, 0]), ([640, 641, 1], [3, 0, 0]),
+                                      ([960, 64, 1025], [0, 1, 1])])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_runs_of_as_many_chunks_as_are_on_their_way(lens, ctx, dtype):
+    """2, 5, 8 and 10 chunks and one more, whole groups of eight and the rest of one."""
+    run(1, 32, 48, 5, lens, ctx, dtype)
+
+
 def test_decays_are_as_exact_as_with_the_library(monkeypatch):
     """ln sigmoid(z) of one chunk (where the kernels leave it for each other) against float64: an error, root mean square,
     of no more than that of fp32 exp and log1p (3.3e-8), but for 5 % for the sample."""

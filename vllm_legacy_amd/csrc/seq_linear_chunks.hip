@@ -16,14 +16,14 @@
 // states after 4096 rows several times as far from 64 bits).
 // Products run on 16x16x4 fp32 matrix cores, those with values of bfloat16 on its own (ThreeParts below).  Operands that
 // later kernels read lie in scratch lane for lane.
-// 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB of chunk states and decays: 83 us per call (22 + 23 + 45
+// 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB of chunk states and decays: 74 us per call (21 + 13 + 43
 // under the tracer; pieces of 256 rows walked token by token and joined by matrix products took 408).  Four workgroups share a
 // CU, so that all 1024 of that step are there at once: 16-bit rows stay 16-bit in LDS (39 of 40 KB), a thread holds a channel's
 // logarithms of a block in registers, A lies where its queries lay and the values where the keys were (two workgroups per CU
 // and two rounds of them, with rows as 32-bit numbers beside a copy of the decays: 123 us, 42 + 23 + 66; with all products on
 // the fp32 instructions 97, 31 + 23 + 52).  What bounds the first and last kernel now are vector instructions (more than half
 // of their cycles; exponentials and logarithms most of them), in the last also the fp32 products with the start states (a
-// fourth); the scan is a copy of the states, 67 MB in 23 us.
+// fourth); the scan is a copy of the states, 34 MB in and out in 13 us.
 #include <atomic>
 #include <type_traits>
 
@@ -417,28 +417,46 @@ __global__ __launch_bounds__(256) void gla_chunk_scan_kernel(GlaChunks a) {
   const int chunks = (run + kChunk - 1) / kChunk;
   const int64_t per = chunk_floats(D, V), step = a.heads * per;
   float* p = a.scratch + ((int64_t)(begin / kChunk + b) * a.heads + h) * per + kChunk * D;
-  constexpr int AHEAD = 16;
-  f32x2 rv[AHEAD], gv[AHEAD];
+  // `ahead` chunks on their way; whole: no more than those, and nothing is asked for behind them.  Whole groups of chunks
+  // have no conditions between them, behind which a wait is for everything on its way (64 chunks 23 us instead of 13).
+  auto walk = [&](auto ahead, auto whole) __attribute__((always_inline)) {
+    constexpr int AHEAD = decltype(ahead)::value;
+    f32x2 rv[AHEAD], gv[AHEAD];
+    auto fetch = [&](int u, int i) __attribute__((always_inline)) {
+      const float* at = p + min(i, chunks - 1) * step;
+      gv[u] = *reinterpret_cast<const f32x2*>(at + d);
+      rv[u] = *reinterpret_cast<const f32x2*>(at + D + 2 * item);
+    };
+    auto pass = [&](int u, int i) __attribute__((always_inline)) {
+      *reinterpret_cast<f32x2*>(p + i * step + D + 2 * item) = s;            // the chunk's start state
 #pragma unroll
-  for (int u = 0; u < AHEAD; ++u) {
-    const float* at = p + min(u, chunks - 1) * step;
-    gv[u] = *reinterpret_cast<const f32x2*>(at + d);
-    rv[u] = *reinterpret_cast<const f32x2*>(at + D + 2 * item);
-  }
-  for (int i = 0; i < chunks; i += AHEAD) {
+      for (int e = 0; e < 2; ++e) s[e] = gv[u][e] * s[e] + rv[u][e];
+    };
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-      if (i + u < chunks) {
-        *reinterpret_cast<f32x2*>(p + (i + u) * step + D + 2 * item) = s;    // the chunk's start state
+    for (int u = 0; u < AHEAD; ++u) fetch(u, u);
+    int i = 0;
+    if constexpr (!decltype(whole)::value)
+      for (; i + AHEAD <= chunks; i += AHEAD)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) s[e] = gv[u][e] * s[e] + rv[u][e];
-        const float* at = p + min(i + u + AHEAD, chunks - 1) * step;
-        // (behind the end this is a place already overwritten, and what it gives is not used)
-        gv[u] = *reinterpret_cast<const f32x2*>(at + d);
-        rv[u] = *reinterpret_cast<const f32x2*>(at + D + 2 * item);
-      }
-    }
-  }
+        for (int u = 0; u < AHEAD; ++u) {
+          pass(u, i + u);
+          fetch(u, i + u + AHEAD);       // (behind the end a place already overwritten, whose numbers are not used)
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (i + u < chunks) pass(u, i + u);
+  };
+  // Short runs ask for what they have: 16 runs of one chunk (16 heads of 64 x 128) 9 us, and 24 asking for sixteen chunks each.
+  using std::integral_constant;
+  if (chunks <= 2)
+    walk(integral_constant<int, 2>(), std::true_type());
+  else if (chunks <= 5)
+    walk(integral_constant<int, 5>(), std::true_type());
+  else if (chunks <= 10)
+    walk(integral_constant<int, 10>(), std::true_type());
+  else
+    walk(integral_constant<int, 8>(), std::false_type());
   st[0] = s[0];
   st[V] = s[1];
 }
