@@ -68,7 +68,7 @@ def test_results_eight_columns_at_a_time(shape, lens, ctx, dtype):
 
 
 @pytest.mark.parametrize("lens,ctx", [([128, 129], [1, 0]), ([320, 321], [0, 2]), ([512, 513], [0, 0]), ([640, 641, 1], [3, 0, 0]),
-                                      ([960, 64, 1025], [0, 1, 1])])
+                                      ([960, 64, 1000], [0, 1, 1])])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_runs_of_as_many_chunks_as_are_on_their_way(lens, ctx, dtype):
     """2, 5, 8 and 10 chunks and one more, whole groups of eight and the rest of one."""
