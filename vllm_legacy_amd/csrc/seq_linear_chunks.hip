@@ -238,6 +238,7 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
   float* y_lds = tot + 4 * D;               // [64][RP]
   int* odd_lds = (int*)(y_lds + kChunk * RP);                // [4]: a wave has met a value that is not finite
   T* v_lds = (T*)(odd_lds + 4);             // [64][VR]
+  float* a_lds = (float*)(v_lds + kChunk * VR);              // [64][D]: logarithms, heads of less than 64 channels
   const int slot = blockIdx.x, h = blockIdx.y;
   int b, chunk;
   if (!find_chunk(a, slot, b, chunk)) return;
@@ -306,29 +307,52 @@ __global__ __launch_bounds__(256, DT <= 4 && sizeof(typename S::T) == 2 ? 4 : 2)
         wv[r] = __builtin_bit_cast(float, (uint32_t)w_row[r / PER][r % PER]);
     }
   }
+  // logarithms of rows first, first + step, ..
+  auto logarithms = [&](auto& av, int first, int step) __attribute__((always_inline)) {
+    constexpr int N = sizeof(av) / sizeof(av[0]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) av[i] = bias;
+#pragma unroll
+    for (int r4 = 0; r4 < kMaxRank; r4 += 4) {
+      if (r4 >= RP) break;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const f32x4 yv = *reinterpret_cast<const f32x4*>(y_lds + (first + step * i) * RP + r4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) av[i] += wv[r4 + e] * yv[e];
+      }
+    }
+#pragma unroll
+    for (int i = N - 1; i >= 0; --i) av[i] = first + step * i < n ? log_sigmoid(av[i]) * a.inv_tau : 0.f;
+  };
+  if constexpr (D < 64) {
+    // Fewer channels' blocks than threads: their logarithms are everyone's (16 rows by a thread of each block: a workgroup of
+    // 16 channels takes 2.3 us more).
+    float av[D / 4];
+    logarithms(av, tid / D, 256 / D);
+#pragma unroll
+    for (int i = 0; i < D / 4; ++i) {
+      const int at = (tid / D + 256 / D * i) * D + d;
+      a_lds[at] = mine[at] = av[i];
+    }
+    __syncthreads();
+  }
 #pragma unroll
   for (int u = 0; u < ITEMS; ++u) {
     const int r0 = kBlock * block_of(u);
     const bool act = D >= 64 || tid < 4 * D;
     float av[kBlock];
+    if constexpr (D >= 64) {
+      logarithms(av, r0, 1);
+    } else {
 #pragma unroll
-    for (int i = 0; i < kBlock; ++i) av[i] = bias;
-#pragma unroll
-    for (int r4 = 0; r4 < kMaxRank; r4 += 4) {
-      if (r4 >= RP) break;
-#pragma unroll
-      for (int i = 0; i < kBlock; ++i) {
-        const f32x4 yv = *reinterpret_cast<const f32x4*>(y_lds + (r0 + i) * RP + r4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) av[i] += wv[r4 + e] * yv[e];
-      }
+      for (int i = 0; i < kBlock; ++i) av[i] = a_lds[(r0 + i) * D + d];
     }
     float p = 0.f;
 #pragma unroll
     for (int i = kBlock - 1; i >= 0; --i) {
-      av[i] = r0 + i < n ? log_sigmoid(av[i]) * a.inv_tau : 0.f;
       if (act) {
-        mine[(r0 + i) * D + d] = av[i];
+        if (D >= 64) mine[(r0 + i) * D + d] = av[i];
         k_lds[(r0 + i) * KR + d] = r0 + i < n ? S::to_f32(ks[u][i]) * exp_of_log(p) : 0.f;
       }
       p += av[i];
@@ -855,7 +879,7 @@ int launch_chunks(const GlaChunks& a, dim3 grid, hipStream_t stream) {
   constexpr int D = 16 * DT;
   static std::atomic<size_t> allowed{64 * 1024}, allowed_out{64 * 1024};   // raised once per kernel, not per launch
   const size_t values = sizeof(typename S::T) * (size_t)kChunk * value_row<S>(a.vdim);
-  const size_t lds = sizeof(float) * ((size_t)kChunk * (D + 4 + (a.rank + 3) / 4 * 4) + 4 * D + 4) + values;
+  const size_t lds = sizeof(float) * ((size_t)kChunk * (D + 4 + (a.rank + 3) / 4 * 4 + (D < 64 ? D : 0)) + 4 * D + 4) + values;
   if (const int rc = raise_lds(&gla_chunk_state_kernel<S, DT>, lds, allowed)) return rc;
   gla_chunk_state_kernel<S, DT><<<grid, 256, lds, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
