@@ -29,6 +29,25 @@ inline int with_dtype(int dtype, F&& f) {
   }
 }
 
+// LDS of a launch of so many workgroups: where they are fewer than the CUs have room for, as much as leaves room for a CU's
+// share of them.  Workgroups go where there is room: four to some CUs while others have none.  Linear recurrence, us with and
+// without: 8 runs of 200 rows, 16 heads of 64 x 128, float16 (512 workgroups, room for 1024) 18 + 29 and 22 + 36; 4096 rows of
+// 4 heads of 128 x 128, float32 (256, room for 512) 24 + 38 and 28 + 49.
+constexpr int64_t kLdsOfCu = 160 * 1024, kLdsGrain = 1280;
+inline size_t spread_lds(size_t lds, int64_t workgroups) {
+  const int64_t share = (workgroups + 255) / 256;
+  if (share > 8) return lds;
+  const size_t least = kLdsOfCu / (share + 1) / kLdsGrain * kLdsGrain + kLdsGrain;      // share + 1 of it are more than there is
+  return lds > least ? lds : least;
+}
+// Pieces of up to `rows` new rows of num_seqs sequences, of which the host knows the sum of the lengths, in slots
+// start_b / rows + b + 0, 1, ..: no more than (tokens + seqs (rows - 1)) / rows have rows.  Where the slots are even in
+// number, those without may all be one XCD's, and the others' CUs have more than their share: then all count.
+inline int64_t pieces_at_most(int num_tokens, int num_seqs, int rows) {
+  const int64_t slots = (int64_t)num_tokens / rows + num_seqs;
+  return slots % 2 ? (num_tokens + (int64_t)num_seqs * (rows - 1)) / rows : slots;
+}
+
 // Orders one wave's LDS traffic: what its lanes wrote before is visible to what they read after.
 // (The hardware keeps a wave's LDS instructions in order; the fences keep the compiler from
 // moving accesses of different types across the point.)

@@ -1042,12 +1042,16 @@ __global__ __launch_bounds__(256, DX <= 2 ? 2 : 1) void delta_block_walk_kernel(
 }
 
 template <int DX>
-int launch_delta_blocks(const DeltaBlocks& a, int64_t slots, hipStream_t stream) {
-  constexpr size_t lds = delta_prepare_lds_floats(64 * DX) * sizeof(float);
+int launch_delta_blocks(const DeltaBlocks& a, int num_tokens, int64_t slots, hipStream_t stream) {
+  // Heads of more than 192: as if lengths were even, since no more than two share a CU and a second round of a few costs no
+  // more than uneven shares do (4 heads of 256, 16 runs of 100 rows 23 us, with two to some CUs 31).
+  const int64_t even = (int64_t)a.num_seqs * ((num_tokens + (int64_t)a.num_seqs * kRows - 1) / ((int64_t)a.num_seqs * kRows));
+  const size_t lds = spread_lds(delta_prepare_lds_floats(64 * DX) * sizeof(float),
+                                (DX > 3 ? even : pieces_at_most(num_tokens, a.num_seqs, kRows)) * a.heads);
   static std::atomic<bool> raised{false};           // LDS limit: raised once per kernel, not per launch
   if (lds > 64 * 1024 && !raised.load(std::memory_order_relaxed)) {
     VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_block_prepare_kernel<DX>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
     raised.store(true, std::memory_order_relaxed);
   }
   delta_block_prepare_kernel<DX><<<dim3((unsigned)slots, a.heads), 256, lds, stream>>>(a);
@@ -1234,10 +1238,10 @@ int delta_rule_scan(
       return VLA_ERR_ARG;
     int rc = VLA_OK;
     switch ((dim + 63) / 64) {
-      case 1: rc = launch_delta_blocks<1>(a, slots, (hipStream_t)stream); break;
-      case 2: rc = launch_delta_blocks<2>(a, slots, (hipStream_t)stream); break;
-      case 3: rc = launch_delta_blocks<3>(a, slots, (hipStream_t)stream); break;
-      default: rc = launch_delta_blocks<4>(a, slots, (hipStream_t)stream); break;
+      case 1: rc = launch_delta_blocks<1>(a, num_tokens, slots, (hipStream_t)stream); break;
+      case 2: rc = launch_delta_blocks<2>(a, num_tokens, slots, (hipStream_t)stream); break;
+      case 3: rc = launch_delta_blocks<3>(a, num_tokens, slots, (hipStream_t)stream); break;
+      default: rc = launch_delta_blocks<4>(a, num_tokens, slots, (hipStream_t)stream); break;
     }
     if (rc != VLA_OK) return rc;
   }

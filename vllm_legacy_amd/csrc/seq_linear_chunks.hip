@@ -866,28 +866,29 @@ bool chunk_sizes(int dim, int vdim, int rank) {
 int64_t chunk_slots(int num_tokens, int num_seqs) { return (int64_t)num_tokens / kChunk + num_seqs; }
 
 template <class K>
-int raise_lds(K kernel, size_t lds, std::atomic<size_t>& allowed) {
-  if (lds > allowed.load(std::memory_order_relaxed)) {
-    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    allowed.store(lds, std::memory_order_relaxed);
+int raise_lds(K kernel, size_t lds, std::atomic<bool>& raised) {
+  if (lds > 64 * 1024 && !raised.load(std::memory_order_relaxed)) {     // once per kernel, to what any launch may ask for
+    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
+    raised.store(true, std::memory_order_relaxed);
   }
   return VLA_OK;
 }
 
 template <class S, int DT>
-int launch_chunks(const GlaChunks& a, dim3 grid, hipStream_t stream) {
+int launch_chunks(const GlaChunks& a, int num_tokens, dim3 grid, hipStream_t stream) {
   constexpr int D = 16 * DT;
-  static std::atomic<size_t> allowed{64 * 1024}, allowed_out{64 * 1024};   // raised once per kernel, not per launch
+  static std::atomic<bool> raised{false}, raised_out{false};
+  auto spread = [&](size_t lds) { return spread_lds(lds, pieces_at_most(num_tokens, a.num_seqs, kChunk) * a.heads); };
   const size_t values = sizeof(typename S::T) * (size_t)kChunk * value_row<S>(a.vdim);
-  const size_t lds = sizeof(float) * ((size_t)kChunk * (D + 4 + (a.rank + 3) / 4 * 4 + (D < 64 ? D : 0)) + 4 * D + 4) + values;
-  if (const int rc = raise_lds(&gla_chunk_state_kernel<S, DT>, lds, allowed)) return rc;
+  const size_t lds = spread(sizeof(float) * ((size_t)kChunk * (D + 4 + (a.rank + 3) / 4 * 4 + (D < 64 ? D : 0)) + 4 * D + 4) + values);
+  if (const int rc = raise_lds(&gla_chunk_state_kernel<S, DT>, lds, raised)) return rc;
   gla_chunk_state_kernel<S, DT><<<grid, 256, lds, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   gla_chunk_scan_kernel<<<dim3(a.heads, (D * a.vdim / 2 + 255) / 256, a.num_seqs), 256, 0, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   const size_t keys = sizeof(float) * (size_t)kChunk * (D + 4);
-  const size_t lds_out = sizeof(float) * ((size_t)kChunk * (D + 4 > kAMat ? D + 4 : kAMat) + 4 * D + kChunk * kBlock) + (keys > values ? keys : values);
-  if (const int rc = raise_lds(&gla_chunk_out_kernel<S, DT>, lds_out, allowed_out)) return rc;
+  const size_t lds_out = spread(sizeof(float) * ((size_t)kChunk * (D + 4 > kAMat ? D + 4 : kAMat) + 4 * D + kChunk * kBlock) + (keys > values ? keys : values));
+  if (const int rc = raise_lds(&gla_chunk_out_kernel<S, DT>, lds_out, raised_out)) return rc;
   gla_chunk_out_kernel<S, DT><<<grid, 256, lds_out, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   return VLA_OK;
@@ -939,10 +940,10 @@ extern "C" int vla_seq_gla_chunks(void* out, int64_t out_stride, const void* q, 
   return with_dtype(dtype, [&](auto s) -> int {
     using S = decltype(s);
     switch (dim / 16) {
-      case 1: return launch_chunks<S, 1>(a, grid, st);
-      case 2: return launch_chunks<S, 2>(a, grid, st);
-      case 4: return launch_chunks<S, 4>(a, grid, st);
-      default: return launch_chunks<S, 8>(a, grid, st);
+      case 1: return launch_chunks<S, 1>(a, num_tokens, grid, st);
+      case 2: return launch_chunks<S, 2>(a, num_tokens, grid, st);
+      case 4: return launch_chunks<S, 4>(a, num_tokens, grid, st);
+      default: return launch_chunks<S, 8>(a, num_tokens, grid, st);
     }
   });
 }
