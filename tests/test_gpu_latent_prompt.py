@@ -323,10 +323,11 @@ def test_which_steps_are_formed():
     from vllm_legacy_amd.attention.backends.latent_kv import LatentKVAttention
     for H, C, lens, contexts, want in ((16, 512, [33], [0], [True]), (16, 512, [31], [0], None), (16, 512, [33], [300], [True]),
                                        (16, 512, [48], [300], [True]), (16, 512, [60], [2000], None), (16, 512, [64], [2000], None),
-                                       (16, 512, [33] * 30, [300] * 30, None), (16, 512, [64] * 30, [300] * 30, [True]),
-                                       (16, 512, [96], [2500], None), (16, 512, [96], [4000], [True]), (16, 512, [48] * 4, [2000] * 4, [True]),
+                                       (16, 512, [33] * 30, [1000] * 30, None), (16, 512, [64] * 30, [300] * 30, [True]),
+                                       (16, 512, [54] * 3, [1240] * 3, [True]), (16, 512, [96], [4000], [True]), (16, 512, [48] * 4, [2000] * 4, [True]),
                                        (16, 512, [64, 20], [0, 0], None), (16, 512, [64, 60], [0, 2000], None),
-                                       (16, 512, [1000, 20], [0, 0], [True, False]), (16, 64, [96], [1500], None),
+                                       (16, 512, [1000, 20], [0, 0], [True, False]), (16, 512, [1000, 40], [0, 40], [True]),
+                                       (16, 512, [1000, 33], [0, 4000], [True, False]), (16, 64, [96], [1500], None),
                                        (16, 64, [1024], [0], [True]), (1, 512, [128], [1500], None), (4, 512, [128], [2500], None), (1, 512, [512], [0], None)):
         attn = LatentKVAttention(H, 128, 64, 128, C, 192**-0.5, 64, 1e4, None, 1e-5, torch.bfloat16, DEV)
         got = attn._stretches(step(lens, contexts)[0])

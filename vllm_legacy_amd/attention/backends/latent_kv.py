@@ -84,6 +84,18 @@ class LatentKVAttention(nn.Module):
         self.formed_fits = True
         gain = 5 * (2 * rank + rot_dim) - 2 * (head_dim + rot_dim + value_dim)      # (formed_min_rows)
         self.least_rows = -(-rank * (head_dim + value_dim) // gain) if gain > 0 else 1 << 30
+        self.few_rows = max(self.FORMED_FEW_ROWS, self.least_rows) if num_heads > 2 else 1 << 30
+        self.tile_rows, self.tile_sets = 32 // min(num_heads, 32), -(-num_heads // min(num_heads, 32))
+        # (formed_is_faster: us a (query, key) pair and a key of a CU's walk on the latent kernel; the keys of a part; us a key of
+        # the longest walk, a pair and a key of them all, formed)
+        self.costs = (2.1e-9 * num_heads * (2 * rank + rot_dim), 0.0155 + 0.0912 / 512 * rank, self.formed_keys(2),
+                      0.0158 + 0.0046 / 128 * head_dim, 1.75e-9 * num_heads * (2 * head_dim + rot_dim + value_dim),
+                      2.44e-9 * num_heads * (head_dim + value_dim) * (rank + 128) + 1.17e-6 * (rank + rot_dim))
+        # keys behind which runs of FORMED_MIN_ROWS go formed, however many there are: nothing more is asked of most steps
+        self.near_keys, rows = self.FORMED_NEAR_KEYS, max(self.FORMED_MIN_ROWS, self.least_rows)
+        while self.near_keys < 2400 and rows < 1024 and all(
+                self.formed_is_faster([rows] * n, [2 * self.near_keys] * n) for n in (1, 4, 32)):
+            self.near_keys *= 2
 
     def set_weights(self, uk: torch.Tensor, uv: torch.Tensor, latent_norm: Optional[torch.Tensor] = None,
                     sinks: Optional[torch.Tensor] = None) -> None:
@@ -112,12 +124,8 @@ class LatentKVAttention(nn.Module):
         keys."""
         return self._key_splits(batch.max_query_len, batch.num_seqs, batch.max_seq_len)
 
-    def _row_tiles(self, max_query_len: int, num_seqs: int) -> int:
-        heads_per = min(self.num_heads, 32)
-        return -(-max_query_len // (32 // heads_per)) * -(-self.num_heads // heads_per) * num_seqs
-
     def _key_splits(self, max_query_len: int, num_seqs: int, keys: int) -> int:
-        tiles = self._row_tiles(max_query_len, num_seqs)
+        tiles = -(-max_query_len // self.tile_rows) * self.tile_sets * num_seqs
         if tiles >= self.SPLIT_BELOW_WORKGROUPS:
             return 1
         if self.window:
@@ -131,11 +139,10 @@ class LatentKVAttention(nn.Module):
     FORMED_MIN_WORK = 6e9
     # Their rows at least: forming a key's numbers costs as much for few rows as for many.
     FORMED_MIN_ROWS = 96
-    # A step below that with so much work, in which every run has so many rows, goes formed as a whole where that is clearly
-    # the faster way.
-    FORMED_LEAST_WORK = 9e6
+    # Runs of so many rows go formed too, all of a step's, where that is the faster way: behind so few keys it always is (of 382
+    # measured steps), behind more formed_is_faster says so.
     FORMED_FEW_ROWS = 32
-    FORMED_CLEARLY = 1.2
+    FORMED_NEAR_KEYS = 300
 
     def formed_min_rows(self) -> int:
         """Rows from which a run's keys and values are worth forming.  A (query, key) pair of a head costs the
@@ -144,35 +151,40 @@ class LatentKVAttention(nn.Module):
         return max(self.FORMED_MIN_ROWS, self.least_rows)
 
     def formed_is_faster(self, lens, contexts) -> bool:
-        """Both ways' time on the GPU for sequences of `lens` rows behind `contexts` keys, in us, as measured over 1 to 128
-        heads of 32 to 128, ranks of 64 to 512, 1 to 30 sequences of 33 to 512 rows behind 0 to 8000 keys (859 steps;
-        rms errors of 14 and 9 %).  Latent: launches, a merge where keys are shared out, the products, and the longest
-        chain of key tiles in a row.  Formed: launches, the walk of the longest sequence's keys by one workgroup per
-        128 rows and head, forming, products and the gathered rows; one part of the workspace after the other.  With
-        the margin none of those steps is slower than on the latent kernel.  Latent / formed, 16 heads of 128 + 64, rank
-        512: 33 rows x 300 keys 67 / 40, x 1000 68 / 57, x 2000 77 / 80, thirty of x 300 127 / 112 and x 1000 334 / 350;
-        48 x 1500 73 / 71; 64 x 1000 69 / 59, x 2000 74 / 88; 96 x 500 72 / 48, x 2500 109 / 105; four of 48 x 2000
-        177 / 121.  Rank 64, 96 x 1500 48 / 63, 1024 x 0 90 / 55.  One or two heads, whose few workgroups the sums are
-        furthest off for, stay (one head, 128 x 1500 63 / 71, x 5000 66 / 152).  Of 439 steps of uneven lengths over these
-        ranges the three that were slower, by 3 to 17 %, were of such layers."""
-        H, D, R, V, C = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.rank
-        w = self.window
-        seen = [c + n if not w else min(c, w) + n for n, c in zip(lens, contexts)]
-        pairs = sum(n * (k - n) + (n * (n + 1) // 2 if not w else n * min(n, w)) for n, k in zip(lens, seen)) * H
-        if H <= 2 or pairs * (2 * C + R) < self.FORMED_LEAST_WORK:
-            return False
-        longest, total = max(seen), sum(seen)
-        tiles = self._row_tiles(max(lens), len(lens))
-        splits = self._key_splits(max(lens), len(lens), max(c + n for n, c in zip(lens, contexts)))
-        rounds, share = -(-tiles * splits // self.SPLIT_BELOW_WORKGROUPS), -(-longest // splits)
-        latent = 33 + 5 * (splits > 1) + 10e-9 * pairs * (2 * C + R) + rounds * share * (0.023 + 0.064 / 512 * C)
-        most, parts, walk = self.formed_keys(2), 1, longest
-        if total > most:
-            held = self._formed_parts(lens, contexts, most)
-            parts, walk = len(held), sum(count if b1 == b0 + 1 else max(seen[b0:b1]) for b0, b1, _, count, _ in held)
-        formed = 27 * parts + walk * (0.015 + 0.0057 / 128 * D) + 1.6e-9 * pairs * (2 * D + R + V) + \
-            total * (2.2e-9 * H * (D + V) * (C + 128) + 2.2e-6 * (C + R))
-        return self.FORMED_CLEARLY * formed < latent
+        """Both ways' time on the GPU for sequences of `lens` rows behind `contexts` keys, in us, as measured over 4 to 128
+        heads of 32 to 128, ranks of 64 to 512, 1 to 30 sequences of 33 to 512 rows behind 0 to 8000 keys (750 steps;
+        rms errors of 12 and 9 %).  Latent: launches, a merge where keys are shared out, the products, and the keys that
+        a CU's workgroups walk (between the most that one may have and its share).  Formed: launches, the walk of the longest
+        sequence's keys by one workgroup per 128 rows and head, forming, products and the gathered rows; one part of the
+        workspace after the other.  Of those steps four are slower than on the latent kernel, by 2 to 10 %, of 439 of uneven lengths none; the
+        host's part is less (65 us of Python and launches, 90).  Latent / formed, 16 heads of 128 + 64, rank 512: 33 rows
+        x 300 keys 67 / 40, x 1000 68 / 57, x 2000 77 / 80, thirty of x 300 127 / 112 and x 1000 334 / 350; 48 x 1500 73 / 71;
+        64 x 1000 69 / 59, x 2000 74 / 88; 96 x 500 72 / 48, x 2500 109 / 105; three of 54 x 1240 117 / 79, four of 48 x 2000
+        177 / 121.  Rank 64, 96 x 1500 48 / 63, 1024 x 0 90 / 55.  One or two heads, whose few workgroups the sums are furthest
+        off for, stay (one head, 128 x 1500 63 / 71, x 5000 66 / 152)."""
+        w, rows_of_tile, tile_sets = self.window, self.tile_rows, self.tile_sets
+        pairs = total = walked = longest = most_rows = 0
+        for n, c in zip(lens, contexts):
+            k = (min(c, w) if w else c) + n
+            pairs += n * (k - n) + (n * (n + 1) // 2 if not w else n * min(n, w))
+            total += k
+            walked += -(-n // rows_of_tile) * k
+            if k > longest:
+                longest = k
+            if n > most_rows:
+                most_rows = n
+        splits = self._key_splits(most_rows, len(lens), longest)
+        share, walked = -(-longest // splits), walked * tile_sets
+        most = -(-sum(-(-n // rows_of_tile) * -(-((min(c, w) if w else c) + n) // share) for n, c in zip(lens, contexts)) *
+                 tile_sets // 256) * share
+        of_pair, of_key, room, of_walk, of_formed_pair, of_formed_key = self.costs
+        latent = 33.4 + 5.5 * (splits > 1) + of_pair * pairs + (most + max(share, walked / 256)) / 2 * of_key
+        parts, walk = 1, longest
+        if total > room:
+            held = self._formed_parts(lens, contexts, room)
+            parts, walk = len(held), sum(count if b1 == b0 + 1 else max((min(c, w) if w else c) + n for n, c in zip(
+                lens[b0:b1], contexts[b0:b1])) for b0, b1, _, count, _ in held)
+        return 26.5 * parts + walk * of_walk + of_formed_pair * pairs + total * of_formed_key < latent
 
     def _stretches(self, batch: SequenceBatch):
         """[[first sequence, one behind the last, first row, one behind the last, formed]]: neighbours that go
@@ -180,9 +192,13 @@ class LatentKVAttention(nn.Module):
         q, ctx = batch.host_query_lens, batch.host_context_lens
         if q is None or ctx is None or not self.scale > 0 or not self.formed_fits or torch.cuda.is_current_stream_capturing():
             return None                 # a captured step is replayed with other lengths than the host's
+        short = min(q)
+        whole = short >= self.few_rows
+        if whole and max(ctx) <= (self.near_keys if short >= self.formed_min_rows() else self.FORMED_NEAR_KEYS):
+            return [[0, len(q), 0, batch.num_tokens, True]]
         each = self.num_heads * (2 * self.rank + self.rot_dim)          # multiply-adds of a (query, key) pair
-        least = self.formed_min_rows()
-        if batch.max_query_len >= least and batch.num_tokens * batch.max_seq_len * each >= self.FORMED_MIN_WORK:
+        if batch.num_tokens * batch.max_seq_len * each >= self.FORMED_MIN_WORK and batch.max_query_len >= self.FORMED_MIN_ROWS:
+            least = self.formed_min_rows()
             out, row, pairs = [], 0, 0
             for b, (n, c) in enumerate(zip(q, ctx)):
                 if n >= least:
@@ -193,8 +209,12 @@ class LatentKVAttention(nn.Module):
                     out.append([b, b + 1, row, row + n, n >= least])
                 row += n
             if pairs * each >= self.FORMED_MIN_WORK:
+                if len(out) > 1 and whole:
+                    few = [(n, c) for n, c in zip(q, ctx) if n < least]
+                    if self.formed_is_faster([n for n, _ in few], [c for _, c in few]):
+                        return [[0, len(q), 0, row, True]]
                 return out if len(out) <= self.MAX_STRETCHES else None
-        if min(q) >= max(self.FORMED_FEW_ROWS, self.least_rows) and self.formed_is_faster(q, ctx):
+        if whole and self.formed_is_faster(q, ctx):
             return [[0, len(q), 0, batch.num_tokens, True]]
         return None
 
