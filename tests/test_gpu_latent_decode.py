@@ -231,6 +231,13 @@ def test_up_projection_of_many_sequences(lens, rank, vdim, heads):
     test_up_projection(lens, rank, vdim, heads, torch.bfloat16)
 
 
+@pytest.mark.parametrize("rank,vdim,heads,lens", [(512, 256, 17, [400] * 70), (512, 256, 2, [500] * 65), (512, 256, 9, [90] * 70),
+                                                  (256, 256, 5, [90] * 20), (256, 128, 5, [90] * 20), (512, 64, 3, [90] * 40)])
+def test_up_projection_on_both_sides_of_the_rule(rank, vdim, heads, lens):
+    """Sixteen and eight sequences to a workgroup by the columns, the latent dims and whether there are parts."""
+    test_up_projection(lens, rank, vdim, heads, torch.bfloat16)
+
+
 @pytest.mark.parametrize("window,sinks", [(0, True), (100, False), (70, True)])
 @pytest.mark.parametrize("lens", [[33, 190, 64, 5], [3000, 33, 700, 64, 5]], ids=["whole", "shared"])
 def test_up_projection_with_windows_sinks_and_sequences_without_a_row(lens, window, sinks):

@@ -580,7 +580,13 @@ int launch_latent_decode(const LatentDecode& a, const LatentUp* up, hipStream_t 
     // Eight sequences to a workgroup while that leaves one for each CU at most: more of them, and registers for the first parts
     // ahead of their maxima (16 heads: 64 of 1 .. 4001 keys 9.8 us instead of 11.9, of 4000 10.4 and 13.4, one of 4000 10.7 and
     // 11.7); sixteen beyond, where weights would be read twice as often (256 of 1000 11.9, with eight 17.1; 1024 of 100 19 and 31).
-    if ((int64_t)((a.num_seqs + 7) / 8) * a.heads <= 256)
+    // Half the waves also take twice the steps each, which only merging outweighs where they are more than are asked for ahead:
+    // with eight and with sixteen, whole sequences of 100 keys, rank 512, vdim 128 7.2 and 5.1 (32 heads, 64 sequences), 256 13.2
+    // and 8.0 (128 heads, 16); vdim 64 the call of 64 sequences of 16 heads 13.9 and 14.8 (rank 256).  In parts, vdim 256, the call
+    // of 32 heads, 16 sequences of 4000, 46.1 and 53.1, of 64 of 1 .. 1000 46.5 and 45.7.
+    const int64_t eights = (int64_t)((a.num_seqs + 7) / 8) * a.heads;
+    const bool whole = a.by_sequence || a.ranges <= 1;
+    if (whole ? eights <= 256 && a.rank * up->vdim <= 512 * 64 : eights <= (up->vdim <= 128 ? 256 : 128))
       latent_decode_up_kernel<S, LB / 4, 8><<<dim3((a.num_seqs + 7) / 8, a.heads), 512, 0, stream>>>(a, *up);
     else
       latent_decode_up_kernel<S, LB / 4, 16><<<dim3((a.num_seqs + 15) / 16, a.heads), 1024, 0, stream>>>(a, *up);
