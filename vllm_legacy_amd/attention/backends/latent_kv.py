@@ -91,10 +91,10 @@ class LatentKVAttention(nn.Module):
         self.costs = (2.1e-9 * num_heads * (2 * rank + rot_dim), 0.0155 + 0.0912 / 512 * rank, self.formed_keys(2),
                       0.0158 + 0.0046 / 128 * head_dim, 1.75e-9 * num_heads * (2 * head_dim + rot_dim + value_dim),
                       2.44e-9 * num_heads * (head_dim + value_dim) * (rank + 128) + 1.17e-6 * (rank + rot_dim))
-        # keys behind which runs of FORMED_MIN_ROWS go formed, however many there are: nothing more is asked of most steps
+        # keys behind which runs of FORMED_MIN_ROWS go formed (one or four of them): nothing more is asked of most steps
         self.near_keys, rows = self.FORMED_NEAR_KEYS, max(self.FORMED_MIN_ROWS, self.least_rows)
         while self.near_keys < 2400 and rows < 1024 and all(
-                self.formed_is_faster([rows] * n, [2 * self.near_keys] * n) for n in (1, 4, 32)):
+                self.formed_is_faster([rows] * n, [2 * self.near_keys] * n) for n in (1, 4)):
             self.near_keys *= 2
 
     def set_weights(self, uk: torch.Tensor, uv: torch.Tensor, latent_norm: Optional[torch.Tensor] = None,
