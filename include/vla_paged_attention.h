@@ -256,8 +256,10 @@ int vla_awq_repack(const int32_t* qweight, const int32_t* qzeros, int32_t* out_q
 
 /* The dequant-GEMM behind awq_gemm / gptq_gemm for k-packed weights (gptq_shuffle'd GPTQ with
  * zero_offset 1, vla_awq_repack'ed AWQ with zero_offset 0): out[m, n] fp16 = x[m, k] fp16 . W.
- * workspace (nullable): device scratch of vla_q4_gemm_workspace_bytes() bytes for split-K
- * partial sums; without it the contraction is not split. k % 64 == 0, group % 32 == 0. */
+ * workspace (nullable): device scratch of vla_q4_gemm_workspace_bytes() bytes, 16-byte aligned, for
+ * split-K partial sums: of the whole product, or, where a product is not split, of its tiles behind the
+ * last whole round of workgroups (up to 32 MiB); without it the contraction is not split.
+ * k % 64 == 0, group % 32 == 0. */
 int64_t vla_q4_gemm_workspace_bytes(int m, int n, int k, int group);
 int vla_q4_gemm_packed(const void* x, const int32_t* qweight, const int32_t* qzeros,
                        const void* scales, void* out, int m, int n, int k, int group,

@@ -1897,7 +1897,9 @@ static hipError_t launch_dma_kp(dim3 grid, hipStream_t s, const _Float16* x, con
 // The K slices of a product's tiles behind the last whole round of 256 workgroups (one to a CU): as many as
 // the round has room for, at most 8, in whole groups and at least four K steps to each of a workgroup's two
 // parts.  Only where a round lasts: what is saved, (1 - 1 / slices) of a round of 16 us per 1024 of K, must
-// be worth the slabs and their reduction (8 .. 12 us).
+// be worth the slabs and their reduction (5 us and more).  43 products of 256 .. 5700 rows and K of 4096 ..
+// 28672 drawn at random, with and without: 1.003 (4509 x 8192 x 57344, 4138 us) to 1.43 times as fast (1103 x
+// 28672 x 8192, 476 us), none slower; errors against 64 bits the same in five digits.
 static Q4Tail pick_tail(int m, int n, int k, int group, const Q4Shape& shape) {
   Q4Tail t;
   if (group % TK || shape.mt != 4 || shape.nw != 8 || shape.splits != 1 || k % (2 * group) || k / (2 * TK) < 16 ||

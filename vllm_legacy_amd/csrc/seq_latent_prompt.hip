@@ -5,9 +5,10 @@
 // queries of the run.  A run of rows therefore gathers its visible cache rows into one place
 // (latent_gather_kernel), latent_form_kernel multiplies them with the two up-projections, and
 // latent_prompt_kernel below is plain causal attention with keys [formed (dim) | shared rotated part
-// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 137 us under the tracer (630 TFLOP/s; 880
-// with the remainders' product) where latent_attention_tile_kernel takes 1685, plus 5 us to gather (9 with 32 rows to a
-// workgroup instead of 8) and 31 to form keys and values (the products on the query's side that they replace take 46).
+// (rot)] and values of vdim.  4096 rows of 16 heads (128 + 64, values of 128, rank 512): 143 us under the tracer on average
+// (139 to 172 from box to box; 600 TFLOP/s, 840 with the remainders' product) where latent_attention_tile_kernel takes 1685,
+// plus 5 us to gather (9 with 32 rows to a workgroup instead of 8) and 31 to form keys and values (the products on the query's
+// side that they replace take 46).
 //
 // Keys come as two 16-bit numbers, the rounded one and what rounding took.  The latent kernel rounds the query's
 // side, which is the same for all keys of a row and mostly cancels in the softmax; a key's rounding is its own.
@@ -35,9 +36,9 @@
 // one group, two workgroups to a CU, all 512 of a run of 4096 rows are on the chip at once and the ones with 64 tiles
 // stay alone on their CUs (165 us instead of 150; 2048 rows 70 instead of 59).  Each group rounds its weights to 16 bits against
 // a maximum of its own: a row's bits differ by one rounding between steps of one form and the other (errors against 64 bits
-// are the same).  A wave alone takes 4400 cycles for a tile, 1800 of
-// products; two on a SIMD 6300 for one each, at 1.6 GHz, where the card holds its power.  Taken back: the second group
-// half a step behind the first (with two tiles of values: 157), raised priority for the first product (162).
+// are the same).  Counted: matrix cores 45 %, vector instructions 38 % of a CU's busy cycles, at 2.07 GHz; within a wave a
+// tile's scores, maximum, weights and second product are a chain.  Taken back: the second group half a step behind the first
+// (with two tiles of values: 157), raised priority for the first product (162).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -130,10 +131,10 @@ __global__ __launch_bounds__(256) void latent_gather_kernel(
 // one row.  Stages of 32 numbers of the rank come by LDS-DMA into a ring of three (72 KB: two workgroups to a CU, one's
 // results leave under the other's products), 16-byte pieces (values' weights, which lie with a head's columns
 // as rows and are read transposing: 64-byte ones) exchanged by the row's number.  A key's remainder comes from the sum in the
-// registers.  4096 rows of rank 512 and 16 heads of 128 + 128: 31 us, 550 TFLOP/s, bound by LDS (a stage is 72 KB of it read
-// and written in 1150 cycles of the two workgroups, beside 1024 of products) and by the 50 MB of results at the end; a
-// library's product per operand and a third for what the first lost, with a copy of the keys ahead of it and one of the
-// values' weights, were 70.
+// registers.  4096 rows of rank 512 and 16 heads of 128 + 128: 31 us, 550 TFLOP/s; a library's product per operand and a third
+// for what the first lost, with a copy of the keys ahead of it and one of the values' weights, were 70.  Counted: matrix
+// cores are at work in 34 % of a CU's busy cycles, vector instructions in 22 %, LDS reads in 13 %: all 512 workgroups are there at
+// once, wait for their first stages together and write 50 MB of results together at the end.
 constexpr int kFormRows = 256, kFormCols = 128, kFormStep = 32;
 constexpr int kFormLatents = kFormRows * kFormStep * 2, kFormStage = kFormLatents + kFormCols * kFormStep * 2;
 struct LatentForm {

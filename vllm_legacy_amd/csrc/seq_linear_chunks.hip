@@ -16,14 +16,14 @@
 // states after 4096 rows several times as far from 64 bits).
 // Products run on 16x16x4 fp32 matrix cores, those with values of bfloat16 on its own (ThreeParts below).  Operands that
 // later kernels read lie in scratch lane for lane.
-// 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB of chunk states and decays: 74 us per call (21 + 13 + 43
+// 4096 rows of 16 heads of 64 x 128 are 68 MB in and out and 100 MB of chunk states and decays: 74 us per call (23 + 13 + 44
 // under the tracer; pieces of 256 rows walked token by token and joined by matrix products took 408).  Four workgroups share a
 // CU, so that all 1024 of that step are there at once: 16-bit rows stay 16-bit in LDS (39 of 40 KB), a thread holds a channel's
 // logarithms of a block in registers, A lies where its queries lay and the values where the keys were (two workgroups per CU
 // and two rounds of them, with rows as 32-bit numbers beside a copy of the decays: 123 us, 42 + 23 + 66; with all products on
-// the fp32 instructions 97, 31 + 23 + 52).  What bounds the first and last kernel now are vector instructions (more than half
-// of their cycles; exponentials and logarithms most of them), in the last also the fp32 products with the start states (a
-// fourth); the scan is a copy of the states, 34 MB in and out in 13 us.
+// the fp32 instructions 97, 31 + 23 + 52).  What bounds the first and last kernel now are vector instructions (84 and 60 % of
+// a CU's busy cycles, counted; exponentials and logarithms most of them), in the last also matrix cores (24 %, most of it the
+// fp32 products with the start states); the scan is a copy of the states, 34 MB in and out in 13 us.
 #include <atomic>
 #include <type_traits>
 
