@@ -1,6 +1,8 @@
 // Shared by the sources of libvla_seq_gfx950.so: dtype dispatch, block reductions, error slot.
 #pragma once
 
+#include <atomic>
+
 #include "../../include/vla_sequence_ops.h"
 #include "vla_common.h"
 
@@ -39,6 +41,19 @@ inline size_t spread_lds(size_t lds, int64_t workgroups) {
   if (share > 8) return lds;
   const size_t least = kLdsOfCu / (share + 1) / kLdsGrain * kLdsGrain + kLdsGrain;      // share + 1 of it are more than there is
   return lds > least ? lds : least;
+}
+// A kernel's LDS limit, raised once on each device that launches it, to what any launch may ask for.
+template <class K>
+inline int raise_lds(K kernel, size_t lds, std::atomic<uint64_t>& raised) {
+  if (lds <= 64 * 1024) return VLA_OK;
+  int dev = 0;
+  VLA_SEQ_HIP_CHECK(hipGetDevice(&dev));
+  const uint64_t bit = 1ull << (dev & 63);
+  if (!(raised.load(std::memory_order_relaxed) & bit)) {
+    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
+    raised.fetch_or(bit, std::memory_order_relaxed);
+  }
+  return VLA_OK;
 }
 // Pieces of up to `rows` new rows of num_seqs sequences, of which the host knows the sum of the lengths, in slots
 // start_b / rows + b + 0, 1, ..: no more than (tokens + seqs (rows - 1)) / rows have rows.  Where the slots are even in

@@ -1049,12 +1049,8 @@ int launch_delta_blocks(const DeltaBlocks& a, int num_tokens, int64_t slots, hip
   const int64_t even = (int64_t)a.num_seqs * ((num_tokens + (int64_t)a.num_seqs * kRows - 1) / ((int64_t)a.num_seqs * kRows));
   const size_t lds = spread_lds(delta_prepare_lds_floats(64 * DX) * sizeof(float),
                                 (DX > 3 ? even : pieces_at_most(num_tokens, a.num_seqs, kRows)) * a.heads);
-  static std::atomic<bool> raised{false};           // LDS limit: raised once per kernel, not per launch
-  if (lds > 64 * 1024 && !raised.load(std::memory_order_relaxed)) {
-    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_block_prepare_kernel<DX>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
-    raised.store(true, std::memory_order_relaxed);
-  }
+  static std::atomic<uint64_t> raised{0};
+  if (const int rc = raise_lds(&delta_block_prepare_kernel<DX>, lds, raised)) return rc;
   delta_block_prepare_kernel<DX><<<dim3((unsigned)slots, a.heads), 256, lds, stream>>>(a);
   VLA_SEQ_HIP_CHECK(hipGetLastError());
   delta_block_walk_kernel<DX><<<dim3(a.heads, (a.vdim + 15) / 16, a.num_seqs), 256, 0, stream>>>(a);

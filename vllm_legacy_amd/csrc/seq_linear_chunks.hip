@@ -865,19 +865,10 @@ bool chunk_sizes(int dim, int vdim, int rank) {
 }
 int64_t chunk_slots(int num_tokens, int num_seqs) { return (int64_t)num_tokens / kChunk + num_seqs; }
 
-template <class K>
-int raise_lds(K kernel, size_t lds, std::atomic<bool>& raised) {
-  if (lds > 64 * 1024 && !raised.load(std::memory_order_relaxed)) {     // once per kernel, to what any launch may ask for
-    VLA_SEQ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
-    raised.store(true, std::memory_order_relaxed);
-  }
-  return VLA_OK;
-}
-
 template <class S, int DT>
 int launch_chunks(const GlaChunks& a, int num_tokens, dim3 grid, hipStream_t stream) {
   constexpr int D = 16 * DT;
-  static std::atomic<bool> raised{false}, raised_out{false};
+  static std::atomic<uint64_t> raised{0}, raised_out{0};
   auto spread = [&](size_t lds) { return spread_lds(lds, pieces_at_most(num_tokens, a.num_seqs, kChunk) * a.heads); };
   const size_t values = sizeof(typename S::T) * (size_t)kChunk * value_row<S>(a.vdim);
   const size_t lds = spread(sizeof(float) * ((size_t)kChunk * (D + 4 + (a.rank + 3) / 4 * 4 + (D < 64 ? D : 0)) + 4 * D + 4) + values);
