@@ -831,8 +831,8 @@ __device__ __forceinline__ int lane_value(int v) {
 // copied from turn to turn (its load would be waited for right there), and the first block's loads keep the order of
 // the loop's, which waits for what both orders have in common.
 // Two prompts of 2999 and 1854 tokens, 16 heads of 128 x 128 (94 blocks in a row), under the tracer, which lets no launch
-// begin before the one ahead of it has ended: the walk 175 us, 1.9 us per block (212 with the loads at once and choices by
-// branches), the prepare kernel 78, the norms 20 and the step kernel's empty launch 5; a call, whose launches overlap,
+// begin before the one ahead of it has ended: the walk 179 us, 1.9 us per block (212 with the loads at once and choices by
+// branches), the prepare kernel 79, the norms 20 and the step kernel's empty launch 5; a call, whose launches overlap,
 // 251 (333), where the token-by-token walk of the same prompts takes 1079.
 // What a block adds to the state is summed in 64 bits: in 32 a call is 20 us less and states are 1.2 times as far
 // from 64 bits as token by token where keys share a part three times as large as the rest (1.0).
